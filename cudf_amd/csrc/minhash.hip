@@ -277,70 +277,22 @@ __device__ __forceinline__ void process_section(const uint8_t* row, int64_t n, i
   using H = HashTraits<T>;
   if (static_cast<int64_t>(width) * 4 <= kHalo) {
     // usual case: a window (<= 4*width bytes) fits the halo staged behind every tile
-    uint32_t const halo = static_cast<uint32_t>(width) * 4u;
     forget_hashes(lds, lane);  // (the wave barrier after the first tile's staging comes before the first look)
     for (int64_t base = s_begin; base < s_end; base += kTile) {
       uint32_t const cnt = static_cast<uint32_t>(min(static_cast<int64_t>(kTile), s_end - base));
-      uint32_t const len = static_cast<uint32_t>(min(n - base, static_cast<int64_t>(cnt + halo)));
-      bool all_ascii;
-      uint32_t const mis = stage_bytes(row, base, len, lds.bytes, lane, &all_ascii);
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      uint32_t count = 0;  // compacted hashes so far (wave-uniform)
-      // In a tile of one-byte characters of a row of at least `width` bytes every window is `width` bytes long: the
-      // hash then runs with a length that the compiler knows to be the same in every lane (its loops over the
-      // blocks and the tail become scalar branches instead of masked ones).
-      bool const plain         = all_ascii && n >= static_cast<int64_t>(width);
-      uint32_t const width_all = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(width));
-      if (plain) {
-        for (uint32_t q = 0; q < cnt; q += kWave) {
-          uint32_t const p = q + lane;
-          bool valid = p < cnt && n - (base + p) >= static_cast<int64_t>(width_all);
-          T hv       = 0;
-          if (valid) {
-            WordSrc const src{lds.bytes, mis + p};
-            hv = H::hash(src, width_all, seed);
-            hv = hv < 1 ? T{1} : hv;  // minhash.cu:141
-          }
-          valid             = valid && !seen_lately(lds, hv);
-          uint64_t const vm = ballot64(valid);
-          if (valid) lds.hashes[count + lanes_below(vm)] = hv;
+      uint32_t count     = 0;  // compacted hashes so far (wave-uniform)
+      auto const hash    = [seed](WordSrc const& src, uint32_t len) {
+        T const hv = H::hash(src, len, seed);
+        return hv < 1 ? T{1} : hv;  // minhash.cu:141
+      };
+      hash_tile_windows<T>(row, n, base, cnt, width, lds.bytes, lds.chars, lane, hash, [&](auto const& valid, auto const& hv) {
+        for (auto const& h : hv) {
+          bool const fresh  = valid[&h - hv] && !seen_lately(lds, h);
+          uint64_t const vm = ballot64(fresh);
+          if (fresh) lds.hashes[count + lanes_below(vm)] = h;
           count += static_cast<uint32_t>(__builtin_popcountll(vm));
         }
-      } else {
-        // A tile with longer characters: all of them are found at once, and where they follow one another without a gap
-        // a lane takes a character, not a byte, and reads its window's length from the list of characters instead of
-        // walking.  (A row shorter than `width` comes here too, whatever its bytes.)
-        CharMap map;
-        map.exact = false;
-        if (!all_ascii) map.build(lds.bytes, mis, len, cnt, base + len == n, lds.chars, lane);
-        uint32_t const items = map.exact ? map.windows : cnt;  // characters, or byte positions
-        for (uint32_t q = 0; q < items; q += kWave) {
-          uint32_t const item = q + lane;
-          bool valid          = false;
-          T hv                = 0;
-          if (item < items) {
-            uint32_t p = item, hlen;
-            if (map.exact) {
-              valid = map.window(item, len, base == 0, width, lds.chars, &p, &hlen);
-            } else {
-              int64_t const gpos = base + p;
-              WordSrc const at{lds.bytes, mis + p};
-              valid = window_at(at, row + gpos, n - gpos, len - p, gpos == 0, all_ascii, width, &hlen);
-            }
-            if (valid) {
-              WordSrc const src{lds.bytes, mis + p};
-              hv = H::hash(src, hlen, seed);
-              hv = hv < 1 ? T{1} : hv;  // minhash.cu:141
-            }
-          }
-          valid             = valid && !seen_lately(lds, hv);
-          uint64_t const vm = ballot64(valid);
-          if (valid) lds.hashes[count + lanes_below(vm)] = hv;
-          count += static_cast<uint32_t>(__builtin_popcountll(vm));
-        }
-      }
+      });
       fold_hashes<T, K, Tail>(lds.hashes, count, a, b, m, lane, pk, tail);
     }
   } else {
@@ -780,7 +732,7 @@ struct AlignedSrc {
 };
 
 constexpr uint32_t kNgramStageBytes = 4096;                             // longest stretch of chars hashed out of LDS
-constexpr uint32_t kNgramStageWords = (kNgramStageBytes + 4 + 28) / 4;  // + misalignment, + over-read of the hash tail
+constexpr uint32_t kNgramStageWords = (kNgramStageBytes + 16 + 32) / 4;  // + misalignment, + whole blocks and over-read of the hash tail
 
 // One workgroup per (group of consecutive rows, parameter chunk), as in minhash_rows_kernel: a row of up to
 // kNgramSoloPositions positions is done by one wavefront alone, 64 positions a trip (wavefront w takes the rows w, w + 4, .. of the group,
@@ -801,7 +753,7 @@ __global__ void __launch_bounds__(kThreads) minhash_ngrams_kernel(ListView in, i
   // the chars of the elements a wavefront is hashing (32-bit hash only: measured 13 % faster there, 9 % slower for the
   // 64-bit hash, whose 16-byte steps cost more to assemble out of LDS than they save)
   constexpr bool kStageRuns = sizeof(T) == 4;
-  __shared__ uint32_t run_bytes[kWaves][kStageRuns ? kNgramStageWords : 1];
+  __shared__ alignas(16) uint32_t run_bytes[kWaves][kStageRuns ? kNgramStageWords : 1];
   __shared__ uint32_t next_row;
 
   int const group_rows = solo_per_wave > 0 ? solo_per_wave * kWaves : 1;

@@ -54,9 +54,10 @@ struct BoundedSrc {
   }
 };
 
-// Hash of window bytes [0, len) of `src`.
+// Hash of window bytes [0, len) of `src` before its final mix.  The mix is a bijection that keeps 0, so where hashes are
+// only compared with one another and with 0 this does as well.
 template <typename Src>
-__device__ __forceinline__ uint32_t murmur3_x86_32(Src const& src, uint32_t len, uint32_t seed)
+__device__ __forceinline__ uint32_t murmur3_x86_32_unmixed(Src const& src, uint32_t len, uint32_t seed)
 {
   uint32_t const c1 = 0xcc9e2d51u, c2 = 0x1b873593u;
   uint32_t h1           = seed;
@@ -78,7 +79,13 @@ __device__ __forceinline__ uint32_t murmur3_x86_32(Src const& src, uint32_t len,
     k1 *= c2;
     h1 ^= k1;
   }
-  h1 ^= len;
+  return h1 ^ len;
+}
+
+template <typename Src>
+__device__ __forceinline__ uint32_t murmur3_x86_32(Src const& src, uint32_t len, uint32_t seed)
+{
+  uint32_t h1 = murmur3_x86_32_unmixed(src, len, seed);
   h1 ^= h1 >> 16;
   h1 *= 0x85ebca6bu;
   h1 ^= h1 >> 13;

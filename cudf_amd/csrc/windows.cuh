@@ -1,5 +1,5 @@
 // Character windows of a row, shared by minhash and jaccard_index: a wavefront stages a tile of row bytes
-// in LDS with aligned dword loads and decides, per byte position, whether a `width`-character window
+// in LDS with aligned 16-byte loads and decides, per byte position, whether a `width`-character window
 // starts there and how many bytes it spans
 // (cpp/src/text/minhash.cu:120-133, cpp/src/text/jaccard.cu:268-277, cpp/include/cudf/strings/string_view.cuh:67-80).
 #pragma once
@@ -13,7 +13,7 @@ constexpr int kWaves     = 4;                  // wavefronts per workgroup
 constexpr int kThreads   = kWaves * kWave;     // 256
 constexpr int kTile      = 256;                // window starts per wavefront tile
 constexpr int kHalo      = 128;                // bytes staged past the tile (windows up to 32 4-byte chars)
-constexpr int kTileWords = (kTile + kHalo + 4 + 24) / 4;  // +4 misalignment, +24 over-read of the hash tail
+constexpr int kTileWords = (kTile + kHalo + 16 + 32) / 4;  // +16 misalignment, +32 for whole blocks and the over-read of the hash tail
 constexpr int kSpan      = 16384;              // bytes of a row handled by one workgroup
 
 // Windows repeat (text repeats its words: a tenth of the windows of a tile, a third within 4 KB of ordinary text), and a
@@ -25,32 +25,29 @@ constexpr int recent_entries() { return 256; }  // (512 costs the kernels a work
 
 template <typename T>
 struct WaveLds {
-  uint32_t bytes[kTileWords];
+  alignas(16) uint32_t bytes[kTileWords];
   alignas(16) T hashes[kTile + 4];
   alignas(16) T recent[recent_entries<T>()];
-  uint32_t chars[kTile + kHalo];  // the characters that start in the staged bytes, in order: start | end << 16 (see CharMap)
+  uint16_t chars[kTile + kHalo];  // the characters that start in the staged bytes, in order: start | bytes << 9 (see CharMap)
 };
 
-// Stage row bytes [base, base+len) into dst; returns the byte offset of `base` inside it.
-// Only aligned dwords that overlap the range are read.  *all_ascii: no byte of the range
-// has its top bit set (wave-uniform).
+// Stage row bytes [base, base+len) into dst (16-byte aligned); returns the byte offset of `base` inside it.
+// Only aligned 16-byte blocks that overlap the range are read (a lane a block: one load and one LDS write for a tile).
+// *all_ascii: no byte of these blocks has its top bit set (wave-uniform); a byte beyond ASCII next to the range costs
+// the caller its shorter way and nothing else.
 __device__ __forceinline__ uint32_t stage_bytes(const uint8_t* row, int64_t base, uint32_t len, uint32_t* dst, int lane, bool* all_ascii)
 {
   const uint8_t* g   = row + base;
-  uint32_t const mis = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(g) & 3u);
-  const uint32_t* ap = reinterpret_cast<const uint32_t*>(g - mis);
-  uint32_t const end = mis + len;  // exclusive byte offset inside dst
-  uint32_t const nw  = (end + 3u) >> 2;
+  uint32_t const mis = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(g) & 15u);
+  const uint4* ap    = reinterpret_cast<const uint4*>(g - mis);
+  uint32_t const nb  = (mis + len + 15u) >> 4;
   uint32_t hibits    = 0;
-  for (uint32_t i = lane; i < nw; i += kWave) {
-    uint32_t const v = ap[i];
-    dst[i]           = v;
-    uint32_t keep    = 0xffffffffu;
-    if (i == 0) keep <<= 8 * mis;                                    // bytes before the range
-    if (4 * i + 4 > end) keep &= (1u << (8 * (end - 4 * i))) - 1u;    // bytes after the range
-    hibits |= v & keep & 0x80808080u;
+  for (uint32_t i = lane; i < nb; i += kWave) {
+    uint4 const v                     = ap[i];
+    reinterpret_cast<uint4*>(dst)[i]  = v;
+    hibits |= v.x | v.y | v.z | v.w;
   }
-  *all_ascii = ballot64(hibits != 0) == 0;
+  *all_ascii = ballot64((hibits & 0x80808080u) != 0) == 0;
   return mis;
 }
 
@@ -58,10 +55,13 @@ __device__ __forceinline__ uint32_t stage_bytes(const uint8_t* row, int64_t base
 // ASCII.  The reference walks from every window start byte by byte, adding up what each first byte of a character
 // says of its length until `width` characters are counted (cpp/include/cudf/strings/string_view.cuh:67-80).  Where
 // every character of the staged bytes ends exactly where the next one starts, that sum is the distance from the start
-// of character k to the end of character k + width - 1: the characters are listed in LDS (start | end << 16, in
+// of character k to the end of character k + width - 1: the characters are listed in LDS (start | bytes << 9, in
 // order), a lane takes a character instead of a byte position, and a window costs two reads of the list.  Other tiles
 // (stray continuation bytes, first bytes that promise more than follows) keep the walk.
+static_assert(kTile + kHalo <= 512, "a character's start takes nine bits of its record");
 struct CharMap {
+  static __device__ __forceinline__ uint32_t start_of(uint32_t c) { return c & 0x1FFu; }
+  static __device__ __forceinline__ uint32_t end_of(uint32_t c) { return (c & 0x1FFu) + (c >> 9); }
   uint32_t count;    // characters that start in the staged bytes
   uint32_t windows;  // of them, in the tile's window starts (the first `cnt` staged bytes)
   bool exact;        // the list gives every window of the tile its length
@@ -69,7 +69,7 @@ struct CharMap {
 
   // staged: the tile's bytes in LDS, its first byte at byte offset `mis`; len of them are the row's, the first cnt are
   // window starts; chars: the list (room for a character per staged byte).
-  __device__ __forceinline__ void build(const uint32_t* staged, uint32_t mis, uint32_t len, uint32_t cnt, bool reaches_row_end, uint32_t* chars,
+  __device__ __forceinline__ void build(const uint32_t* staged, uint32_t mis, uint32_t len, uint32_t cnt, bool reaches_row_end, uint16_t* chars,
                                         int lane)
   {
     const uint8_t* const sb = reinterpret_cast<const uint8_t*>(staged) + mis;
@@ -81,7 +81,7 @@ struct CharMap {
       uint32_t const b     = pos < len ? sb[pos] : 0x80u;
       bool const start     = !is_utf8_continuation(b);
       uint64_t const found = ballot64(start);
-      if (start) chars[count + lanes_below(found)] = pos | ((pos + static_cast<uint32_t>(bytes_in_utf8_byte(b))) << 16);
+      if (start) chars[count + lanes_below(found)] = static_cast<uint16_t>(pos | (static_cast<uint32_t>(bytes_in_utf8_byte(b)) << 9));
       count += static_cast<uint32_t>(__builtin_popcountll(found));
       if (base < cnt) windows += static_cast<uint32_t>(__builtin_popcountll(ballot64(start && pos < cnt)));
     }
@@ -92,27 +92,27 @@ struct CharMap {
     bool broken = false;
     for (uint32_t k0 = 0; k0 < count; k0 += kWave) {
       uint32_t const k = k0 + static_cast<uint32_t>(lane);
-      if (k >= 1 && k < count) broken = broken || (chars[k - 1] >> 16) != (chars[k] & 0xFFFFu);
+      if (k >= 1 && k < count) broken = broken || end_of(chars[k - 1]) != start_of(chars[k]);
     }
     // the last one: ends with the row, or, when the row goes on, begins in the last four staged bytes (then every window
     // start of the tile, at least 4 * width bytes before the end of the staged bytes, has its `width` characters listed)
     bool tail = false;
     if (count > 0) {
       uint32_t const last = chars[count - 1];
-      tail                = reaches_row_end ? (last >> 16) == len : len - (last & 0xFFFFu) <= 4u;
+      tail                = reaches_row_end ? end_of(last) == len : len - start_of(last) <= 4u;
     }
     exact = tail && ballot64(broken) == 0;
   }
 
   // The window that begins with character k (k < windows): whether it counts, where it starts and its bytes.
   // row_start: staged byte 0 is the row's first byte.
-  __device__ __forceinline__ bool window(uint32_t k, uint32_t len, bool row_start, int32_t width, const uint32_t* chars, uint32_t* pos,
+  __device__ __forceinline__ bool window(uint32_t k, uint32_t len, bool row_start, int32_t width, const uint16_t* chars, uint32_t* pos,
                                          uint32_t* hlen) const
   {
-    uint32_t const first = chars[k] & 0xFFFFu;
+    uint32_t const first = start_of(chars[k]);
     *pos                 = first;
     if (k + static_cast<uint32_t>(width) <= count) {
-      *hlen = (chars[k + static_cast<uint32_t>(width) - 1u] >> 16) - first;
+      *hlen = end_of(chars[k + static_cast<uint32_t>(width) - 1u]) - first;
       return true;
     }
     // fewer than `width` characters are left (the staged bytes reach the end of the row): only the row's first position counts
@@ -160,6 +160,73 @@ __device__ __forceinline__ bool window_at(Src const& src, const uint8_t* g, int6
   // a malformed trailing lead byte may declare more bytes than the row holds: clamp to the row
   *hlen = static_cast<uint32_t>(min(static_cast<int64_t>(bytes), remaining));
   return first || left <= 0;
+}
+
+// The windows that start in [base, base + cnt) of a row of n bytes (cnt <= kTile, 4 * width <= kHalo): `hash(src, bytes)`
+// of each goes to `sink(valid, hash)`, which every lane of the wavefront calls together, with arrays of one window per
+// lane or of two (two chains of LDS reads and multiplies in flight instead of one).  `bytes` and `chars` are the
+// wavefront's own LDS.
+template <typename T, typename Hash, typename Sink>
+__device__ __forceinline__ void hash_tile_windows(const uint8_t* row, int64_t n, int64_t base, uint32_t cnt, int32_t width, uint32_t* bytes,
+                                                  uint16_t* chars, int lane, Hash const& hash, Sink&& sink)
+{
+  uint32_t const halo = static_cast<uint32_t>(width) * 4u;
+  uint32_t const len  = static_cast<uint32_t>(min(n - base, static_cast<int64_t>(cnt + halo)));
+  bool all_ascii;
+  uint32_t const mis = stage_bytes(row, base, len, bytes, lane, &all_ascii);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  // In a tile of one-byte characters of a row of at least `width` bytes every window is `width` bytes long: the
+  // hash then runs with a length that the compiler knows to be the same in every lane (its loops over the
+  // blocks and the tail become scalar branches instead of masked ones).
+  bool const plain         = all_ascii && n >= static_cast<int64_t>(width);
+  uint32_t const width_all = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(width));
+  if (plain) {
+    // (len and width fit 32 bits, and the last window of the row ends with it)
+    uint32_t const starts = min(cnt, len - min(len, width_all - 1u));
+    uint32_t q = 0;
+    for (; q + kWave < starts; q += 2 * kWave) {
+      // (a lane beyond the last window hashes the bytes of that one: no branch)
+      uint32_t const p      = q + lane;
+      bool const valid[2]   = {true, p + kWave < starts};
+      T const hv[2]         = {hash(WordSrc{bytes, mis + p}, width_all), hash(WordSrc{bytes, mis + min(p + kWave, starts - 1u)}, width_all)};
+      sink(valid, hv);
+    }
+    if (q < starts) {
+      uint32_t const p    = q + lane;
+      bool const valid[1] = {p < starts};
+      T const hv[1]       = {hash(WordSrc{bytes, mis + min(p, starts - 1u)}, width_all)};
+      sink(valid, hv);
+    }
+  } else {
+    // A tile with longer characters: all of them are found at once, and where they follow one another without a gap
+    // a lane takes a character, not a byte, and reads its window's length from the list of characters instead of
+    // walking.  (A row shorter than `width` comes here too, whatever its bytes.)
+    CharMap map;
+    map.exact = false;
+    if (!all_ascii) map.build(bytes, mis, len, cnt, base + len == n, chars, lane);
+    uint32_t const items = map.exact ? map.windows : cnt;  // characters, or byte positions
+    for (uint32_t q = 0; q < items; q += kWave) {
+      uint32_t const item = q + lane;
+      bool valid[1]       = {false};
+      T hv[1]             = {0};
+      if (item < items) {
+        uint32_t p = item, hlen;
+        if (map.exact) {
+          valid[0] = map.window(item, len, base == 0, width, chars, &p, &hlen);
+        } else {
+          int64_t const gpos = base + p;
+          WordSrc const at{bytes, mis + p};
+          valid[0] = window_at(at, row + gpos, n - gpos, len - p, gpos == 0, all_ascii, width, &hlen);
+        }
+        if (valid[0]) hv[0] = hash(WordSrc{bytes, mis + p}, hlen);
+      }
+      sink(valid, hv);
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
 }  // namespace nvtext_amd
