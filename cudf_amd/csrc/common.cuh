@@ -480,6 +480,9 @@ void device_exclusive_scan(F f, int64_t n, OutT* out, uint64_t* temp, hipStream_
   hipLaunchKernelGGL(HIP_KERNEL_NAME(scan_apply_kernel<F, OutT>), dim3(static_cast<unsigned>(tiles)), dim3(kScanThreads), 0, stream, f, n, temp, out);
 }
 
+// Compute units of the current device (read once per device).
+int device_cus();
+
 // ------------------------------------------------------------------ scalars for the host
 // A few KB of pinned host memory that kernels write and the host reads once the stream is synchronised (a copy of a
 // few bytes into ordinary host memory goes through a staging buffer and costs ten microseconds and more): eight 64-bit

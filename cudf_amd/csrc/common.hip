@@ -3,6 +3,7 @@
 // C-ABI utilities (version, last error, result release).
 #include "common.cuh"
 
+#include <atomic>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -154,6 +155,20 @@ __global__ void read_two_offsets_kernel(const void* offsets, int is64, int64_t f
   dst[threadIdx.x] = static_cast<uint64_t>(is64 ? static_cast<const int64_t*>(offsets)[i] : static_cast<int64_t>(static_cast<const int32_t*>(offsets)[i]));
 }
 }  // namespace
+
+int device_cus()
+{
+  constexpr int kMost = 64;
+  static std::atomic<int> known[kMost] = {};
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= kMost) return 256;
+  int cus = known[device].load(std::memory_order_relaxed);
+  if (cus == 0) {
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus <= 0) cus = 256;
+    known[device].store(cus, std::memory_order_relaxed);
+  }
+  return cus;
+}
 
 uint64_t* host_scalars()
 {

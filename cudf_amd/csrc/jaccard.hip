@@ -597,9 +597,7 @@ nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* inpu
   ColView const v1 = make_view(*input1);
   ColView const v2 = make_view(*input2);
   float* const values = static_cast<float*>(out->data);
-  int device = 0, cus = 256;
-  (void)hipGetDevice(&device);
-  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
+  int const cus       = device_cus();
   {
     ProfileScope ps("jaccard_wave_kernel", stream);
     int per_group = kThreads;

@@ -10,10 +10,9 @@
 //   * it then switches to lanes <-> parameters: every lane keeps K (a, b) pairs and
 //     K running minima in registers and streams the tile's hashes through LDS
 //     broadcast reads, so the inner loop is v_mad_u64_u32 + v_min only;
-//   * a workgroup takes four rows: a row of up to 1 KiB belongs to one wavefront alone; the 4
-//     wavefronts split the first 16 KiB of a longer row and combine in LDS (plain store); the
-//     rest of a still longer row is covered by extra workgroups that merge with atomic min, so
-//     no output pre-initialisation is needed;
+//   * a wavefront does a row alone, or a part of it: rows are cut into parts of at most 4 KiB (of
+//     fewer bytes in a column too small to give every wavefront of the device one of that size),
+//     and the parts of a row meet in the result with an atomic minimum;
 //   * in a tile with characters of more than one byte the wavefront lists the characters first,
 //     so that a lane takes a character and reads its window's length instead of walking to it;
 //     hashes that the wavefront has folded lately are dropped (a minimum does not mind).
@@ -28,12 +27,12 @@
 #include <mutex>
 #include <type_traits>
 
-// Scratch of nvtext_amd_minhash_preallocated, the entry point that allocates nothing: the extra-span counts of the
-// rows (rows + 1 values) and behind them the tile sums of the scans.  Every device holds its own copy of the array
+// Scratch of nvtext_amd_minhash_preallocated, the entry point that allocates nothing: the part counts of the
+// rows (rows + 1 values) and behind them the tile sums of the scans and the counter of the parts.  Every device holds its own copy of the array
 // for as long as the library is loaded (4.2 MB).
 constexpr int32_t kPreallocatedMaxRows = NVTEXT_AMD_MINHASH_PREALLOCATED_MAX_ROWS;
 constexpr size_t kScratchPrefixBytes   = (static_cast<size_t>(kPreallocatedMaxRows) + 1 + 63) / 64 * 64 * sizeof(uint32_t);
-constexpr size_t kScratchScanBytes     = (static_cast<size_t>(kPreallocatedMaxRows) / nvtext_amd::kScanTile + 2) * sizeof(uint64_t);
+constexpr size_t kScratchScanBytes     = (static_cast<size_t>(kPreallocatedMaxRows) / nvtext_amd::kScanTile + 3) * sizeof(uint64_t);
 static __device__ __align__(256) unsigned char scratch[kScratchPrefixBytes + kScratchScanBytes];
 
 namespace nvtext_amd {
@@ -331,26 +330,54 @@ __device__ __forceinline__ void load_params(const T* pa, const T* pb, int32_t P,
   }
 }
 
-// One workgroup per (group of consecutive rows, parameter chunk).  A row of up to kSoloBytes (kSoloBytesMany when a
-// wavefront takes several) is done by one wavefront alone (wavefront w takes the rows w, w + 4, .. of the group, `solo_per_wave` of them: nothing to combine, the minima go
-// from the registers to the result); a longer row is shared by the four wavefronts, which split its first kSpan bytes
-// and combine through LDS, one such row after the other.  The groups lie along x and, beyond kMaxRowBlocks of them,
-// along z.
-// Rows differ in length, and a workgroup lasts as long as its slowest wavefront: with one short row per wavefront the
-// others waited for the longest of four (8 M rows of about 500 bytes: 88 ms; four rows per wavefront 80 ms, sixteen
-// 77 ms).  More rows per workgroup mean fewer workgroups, and a column of few rows needs them all to fill the device
-// and to even out its end: the host asks for as many rows per wavefront (a power of two, at most kMaxSoloPerWave) as
-// leave at least kMinRowGroups groups.
-constexpr int64_t kSoloBytes      = 1024;   // with one row to a wavefront
-constexpr int64_t kSoloBytesMany  = 4096;   // with several: their sum evens out, and a row done alone needs no barrier (2 M rows of 2 KB: 2 % faster than 1024)
-constexpr int kMaxSoloPerWave     = 16;
-constexpr int32_t kMinRowGroups   = 16384;  // sixteen times the workgroups that 256 CUs hold at four apiece
-inline int solo_rows_per_wave(int32_t rows)
+// How the rows are shared out.  In a column of at least kManyRows rows a wavefront does the rows of up to kPartBytes
+// bytes alone, several in turn (minhash_rows_kernel), and the longer ones are cut into parts; in a column of fewer rows
+// every row is cut into parts (minhash_parts_kernel), so that the device is full whatever the rows' lengths: 999
+// documents of 2 KB (256 parameters) with a workgroup each, and another launch for what lay beyond their first 16 KB,
+// took 282 us for 23 us of arithmetic, most of it spent on the longest document; 42 us in parts.  20,011 rows of 16 KB
+// (uint64, 128 parameters) 9.0 -> 7.4 ms, the long rows of 400,000 documents of 2 KB 9.7 -> 9.2 ms.
+// A workgroup lasts as long as its slowest wavefront, and rows differ in length: with one row per wavefront the others
+// waited for the longest of four (8 M rows of about 500 bytes: 88 ms; four rows per wavefront 80 ms, sixteen 77 ms).
+// More rows per workgroup mean fewer workgroups, and the column needs them all to fill the device and to even out its
+// end: the host asks for as many rows per wavefront (a power of two, at most kMaxRowsPerWave) as leave at least
+// kMinRowGroups groups.
+constexpr int32_t kManyRows     = 131072;
+constexpr int64_t kPartBytes    = 4096;
+constexpr int64_t kMinPartBytes = 256;     // a tile: less would be staged for its halo
+constexpr int kMaxRowsPerWave   = 16;
+constexpr int32_t kMinRowGroups = 16384;  // sixteen times the workgroups that 256 CUs hold at four apiece
+inline int rows_per_wave(int32_t rows)
 {
-  int spw = 1;
-  while (spw < kMaxSoloPerWave && rows / (2 * spw * kWaves) >= kMinRowGroups) spw *= 2;
-  return spw;
+  int rpw = 1;
+  while (rpw < kMaxRowsPerWave && rows / (2 * rpw * kWaves) >= kMinRowGroups) rpw *= 2;
+  return rpw;
 }
+
+// The parts of every row: none for a null row and for the rows that minhash_rows_kernel does, one for an empty row (its
+// zeros have to be written).
+struct RowParts {
+  ColView col;
+  int32_t waves;      // wavefronts that the device holds
+  int64_t row_bytes;  // rows of at most this many bytes are done by minhash_rows_kernel; -1: none is
+  // Bytes of a part: kPartBytes where that leaves every wavefront four parts and more, else a quarter of what each has to
+  // do, in columns of less than a kilobyte per wavefront all of it (a second round of parts would be longer than the
+  // imbalance it removes).
+  __device__ __forceinline__ int64_t part_bytes() const
+  {
+    if (row_bytes >= 0) return kPartBytes;
+    int64_t const share = (col.off(col.size) - col.off(0)) / waves;
+    int64_t const bytes = ((share < 1024 ? share : share / 4) + kWave) / kWave * kWave;
+    return min(max(bytes, kMinPartBytes), kPartBytes);
+  }
+  __device__ __forceinline__ uint64_t operator()(int64_t i) const
+  {
+    if (!col.valid(i)) return 0;
+    int64_t const n = col.off(i + 1) - col.off(i);
+    if (n <= row_bytes) return 0;
+    int64_t const bytes = part_bytes();
+    return n == 0 ? 1 : static_cast<uint64_t>((n + bytes - 1) / bytes);
+  }
+};
 
 // The tail of a launch with TAIL: the P - 64 K parameters (1..32) beyond the K full sets of the one chunk.
 template <typename T, int K, bool TAIL>
@@ -377,19 +404,24 @@ struct TailOf<T, K, true> {
   static __device__ __forceinline__ T value(type const& t) { return t.m[0]; }
 };
 
+// Wavefronts per SIMD that the registers are held to.
+template <typename T>
+constexpr int minhash_waves() { return sizeof(T) == 4 ? 7 : 4; }
+
+// One workgroup per (group of consecutive rows, parameter chunk): its wavefronts take the group's rows of up to kPartBytes
+// bytes one at a time from a counter in LDS, so that the four are done together whatever the rows' lengths; the minima
+// go from the registers to the result.  The groups lie along x and, beyond kMaxRowBlocks of them, along z.
 template <typename T, int K, bool TAIL>
-__global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 7 : 4) minhash_rows_kernel(ColView col, T seed, const T* __restrict__ pa, const T* __restrict__ pb, int32_t P,
-                                                                int32_t width, const int32_t* __restrict__ out_offsets, T* __restrict__ out,
-                                                                int solo_per_wave)
+__global__ void __launch_bounds__(kThreads, minhash_waves<T>()) minhash_rows_kernel(ColView col, T seed, const T* __restrict__ pa, const T* __restrict__ pb,
+                                                                int32_t P, int32_t width, const int32_t* __restrict__ out_offsets, T* __restrict__ out,
+                                                                int per_wave)
 {
   using TailT = TailOf<T, K, TAIL>;
   constexpr int kSets = K + (TAIL ? 1 : 0);
   __shared__ WaveLds<T> lds[kWaves];
-  __shared__ T red[kWaves][kSets * kWave];
   __shared__ uint32_t next_row;
 
-  int const group_rows     = solo_per_wave * kWaves;
-  int64_t const solo_bytes = solo_per_wave > 1 ? kSoloBytesMany : kSoloBytes;
+  int const group_rows = per_wave * kWaves;
   int64_t const r0     = (static_cast<int64_t>(blockIdx.z) * gridDim.x + blockIdx.x) * group_rows;
   if (r0 >= col.size) return;
   int const lane           = lane_id();
@@ -405,122 +437,105 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 7 : 4) minhash_rows
   int const rows_here = static_cast<int>(min(static_cast<int64_t>(group_rows), col.size - r0));
   if (threadIdx.x == 0) next_row = 0;
   __syncthreads();
-
-  // First the short rows of the group: a wavefront takes the next one whenever it is done with one (a counter in LDS),
-  // so that the four are done with their short rows at about the same time whatever the rows' lengths.  Then, from
-  // `together` = 0 on, its part of the rows that are too long for that, one after the other.
-  int together = -1;
   for (;;) {
-    int i;
-    if (together < 0) {
-      int t = 0;
-      if (lane == 0) t = static_cast<int>(atomicAdd(&next_row, 1u));
-      i = __builtin_amdgcn_readfirstlane(t);  // (the same in every lane: what depends on it stays scalar)
-      if (i >= rows_here) {
-        together = 0;
-        continue;
-      }
-    } else {
-      if (together >= rows_here) break;
-      i = together++;
-    }
-    bool const solo = together < 0;
+    int t = 0;
+    if (lane == 0) t = static_cast<int>(atomicAdd(&next_row, 1u));
+    int const i = __builtin_amdgcn_readfirstlane(t);  // (the same in every lane: what depends on it stays scalar)
+    if (i >= rows_here) break;
     if (!col.valid(r0 + i)) continue;
     int64_t const o = col.off(r0 + i);
     int64_t const n = col.off(r0 + i + 1) - o;
-    if (solo != (n <= solo_bytes)) continue;
+    if (n > kPartBytes) continue;
 #pragma unroll
     for (int k = 0; k < K; ++k) m[k] = std::numeric_limits<T>::max();
     TailT::reset(tail);
-    int64_t sb = 0, se = n;
-    if (!solo) {
-      int64_t const span = min(n, static_cast<int64_t>(kSpan));
-      int64_t sec        = (span + kWaves - 1) / kWaves;
-      sec                = (sec + kWave - 1) / kWave * kWave;
-      sb                 = min(span, wave * sec);
-      se                 = min(span, sb + sec);
-    }
-    if (sb < se) process_section<T, K>(col.chars + o, n, sb, se, seed, width, a, b, m, lds[wave], lane, pk, tail);
+    if (n > 0) process_section<T, K>(col.chars + o, n, 0, n, seed, width, a, b, m, lds[wave], lane, pk, tail);
     if (K == 1) m[0] = pk.combine(m[0]);
     TailT::finish(tail);
     T* const dst = out + static_cast<int64_t>(out_offsets[r0 + i]) + chunk_base;
-    if (solo) {
-      // nothing to combine: the minima go from the registers to the result; an empty row is zeros (minhash.cu:318)
+    // an empty row is zeros (minhash.cu:318)
 #pragma unroll
-      for (int k = 0; k < K; ++k) {
-        int32_t const j = lane + kWave * k;  // (with fewer than 64 parameters the first lanes hold one each, in order)
-        if (j < in_chunk) dst[j] = n > 0 ? m[k] : T{0};
-      }
-      if (TAIL && K * kWave + lane < in_chunk) dst[K * kWave + lane] = n > 0 ? TailT::value(tail) : T{0};
-    } else {
-      __syncthreads();  // (the row before has been read out of red)
-#pragma unroll
-      for (int k = 0; k < K; ++k) red[wave][k * kWave + lane] = m[k];
-      if (TAIL) red[wave][K * kWave + lane] = TailT::value(tail);
-      __syncthreads();
-      for (int j = threadIdx.x; j < in_chunk; j += kThreads) {
-        T v = red[0][j];
-#pragma unroll
-        for (int w = 1; w < kWaves; ++w) v = min(v, red[w][j]);
-        dst[j] = v;
-      }
+    for (int k = 0; k < K; ++k) {
+      int32_t const j = lane + kWave * k;  // (with fewer than 64 parameters the first lanes hold one each, in order)
+      if (j < in_chunk) dst[j] = n > 0 ? m[k] : T{0};
     }
+    if (TAIL && K * kWave + lane < in_chunk) dst[K * kWave + lane] = n > 0 ? TailT::value(tail) : T{0};
   }
 }
 
-// Extra parts of rows longer than kSpan: task t covers bytes [part*kSpan, (part+1)*kSpan) of its row.
-// extra_prefix[r] = number of extra parts in rows < r (rows+1 entries).
-// (uint32: held to the registers of six wavefronts per SIMD, which left to itself the compiler exceeds with four and
-// five sets of parameters: the reference's 260-parameter shapes 3 to 5 % faster; uint64 gains nothing from it.)
+// Parts of rows, a wavefront each: part t is one of the row r with prefix[r] <= t < prefix[r + 1].  A row of one part is
+// stored, the parts of the others meet with an atomic minimum (their slots hold the largest value before).  With more
+// than eight parts for every wavefront they are handed out by a counter, else by place (a counter answers about 150 M
+// requests a second: seven thousand wavefronts asking at once would wait 50 us).  The chunks of parameters come one
+// after the other in the same count.
 template <typename T, int K, bool TAIL>
-__global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 6 : 1) minhash_extra_kernel(ColView col, T seed, const T* __restrict__ pa, const T* __restrict__ pb, int32_t P,
-                                                                 int32_t width, const int32_t* __restrict__ out_offsets,
-                                                                 const uint32_t* __restrict__ extra_prefix, T* __restrict__ out)
+__global__ void __launch_bounds__(kThreads, minhash_waves<T>()) minhash_parts_kernel(RowParts parts, T seed, const T* __restrict__ pa, const T* __restrict__ pb,
+                                                                int32_t P, int32_t width, int32_t chunks, const int32_t* __restrict__ out_offsets,
+                                                                const uint32_t* __restrict__ prefix, unsigned long long* __restrict__ counter,
+                                                                T* __restrict__ out)
 {
   using TailT = TailOf<T, K, TAIL>;
   constexpr int kSets = K + (TAIL ? 1 : 0);
   __shared__ WaveLds<T> lds[kWaves];
-  __shared__ T red[kWaves][kSets * kWave];
-  uint32_t const total     = extra_prefix[col.size];
-  int32_t const chunk_base = blockIdx.y * (K * kWave);
-  int32_t const in_chunk   = min(kSets * kWave, P - chunk_base);
-  int const lane           = lane_id();
-  int const wave           = threadIdx.x / kWave;
-  Packing const pk         = K == 1 ? packing_for(P) : Packing{kWave, 1};
-  for (uint32_t t = blockIdx.x; t < total; t += gridDim.x) {
-    // last row r with extra_prefix[r] <= t
-    int64_t lo = 0, hi = col.size;
-    while (hi - lo > 1) {
-      int64_t const mid = (lo + hi) >> 1;
-      if (extra_prefix[mid] <= t) lo = mid; else hi = mid;
+  ColView const& col    = parts.col;
+  uint32_t const total  = prefix[col.size];
+  uint64_t const tasks  = static_cast<uint64_t>(total) * static_cast<uint32_t>(chunks);
+  int64_t const bytes   = parts.part_bytes();
+  int const lane        = lane_id();
+  int const wave        = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
+  uint64_t const nwaves = static_cast<uint64_t>(gridDim.x) * kWaves;
+  Packing const pk      = K == 1 ? packing_for(P) : Packing{kWave, 1};
+  T a[K], b[K], m[K];
+  typename TailT::type tail;
+  uint32_t chunk = 0;
+  load_params<T, K>(pa, pb, P, 0, pk.param_lane(lane), a, b, m);
+  TailT::load(tail, pa, pb, P, lane);
+  for (uint64_t task = static_cast<uint64_t>(blockIdx.x) * kWaves + wave; task < tasks;) {
+    uint32_t const t = static_cast<uint32_t>(task - static_cast<uint64_t>(chunk) * total);
+    if (t >= total) {  // the next chunk of parameters
+      ++chunk;
+      load_params<T, K>(pa, pb, P, static_cast<int32_t>(chunk) * (K * kWave), pk.param_lane(lane), a, b, m);
+      continue;
     }
-    int64_t const r    = lo;
-    int64_t const part = static_cast<int64_t>(t - extra_prefix[r]) + 1;
-    int64_t const o    = col.off(r);
-    int64_t const n    = col.off(r + 1) - o;
-    T a[K], b[K], m[K];
-    load_params<T, K>(pa, pb, P, chunk_base, pk.param_lane(lane), a, b, m);
-    typename TailT::type tail;
-    TailT::load(tail, pa, pb, P, lane);
-    int64_t const pb0  = part * kSpan;
-    int64_t const pe0  = min(n, pb0 + kSpan);
-    int64_t const sec  = kSpan / kWaves;
-    int64_t const sb   = min(pe0, pb0 + wave * sec);
-    int64_t const se   = min(pe0, sb + sec);
+    int32_t const chunk_base = static_cast<int32_t>(chunk) * (K * kWave);
+    int32_t const in_chunk   = min(kSets * kWave, P - chunk_base);
+    // the last row r with prefix[r] <= t, 64 of them looked at in one step
+    int64_t r = 0, end = col.size;
+    while (end - r > 1) {
+      int64_t const step = (end - r + kWave - 1) / kWave;
+      int64_t const at   = r + lane * step;
+      int const below    = __builtin_popcountll(ballot64(at < end && prefix[min(at, end - 1)] <= t));
+      r += (below - 1) * step;
+      end = min(end, r + step);
+    }
+    int64_t const o   = col.off(r);
+    int64_t const n   = col.off(r + 1) - o;
+    int64_t const sb  = static_cast<int64_t>(t - prefix[r]) * bytes;
+    int64_t const se  = min(n, sb + bytes);
+    bool const shared = n > bytes;
+#pragma unroll
+    for (int k = 0; k < K; ++k) m[k] = std::numeric_limits<T>::max();
+    TailT::reset(tail);
     if (sb < se) process_section<T, K>(col.chars + o, n, sb, se, seed, width, a, b, m, lds[wave], lane, pk, tail);
     if (K == 1) m[0] = pk.combine(m[0]);
     TailT::finish(tail);
-    __syncthreads();
+    T* const dst = out + static_cast<int64_t>(out_offsets[r]) + chunk_base;
+    auto const put = [&](int32_t j, T v) {
+      if (j >= in_chunk) return;
+      if (!shared)
+        dst[j] = n > 0 ? v : T{0};  // an empty row is zeros (minhash.cu:318)
+      else if (v != std::numeric_limits<T>::max())
+        atomicMin(&dst[j], v);
+    };
 #pragma unroll
-    for (int k = 0; k < K; ++k) red[wave][k * kWave + lane] = m[k];
-    if (TAIL) red[wave][K * kWave + lane] = TailT::value(tail);
-    __syncthreads();
-    T* dst = out + static_cast<int64_t>(out_offsets[r]) + chunk_base;
-    for (int j = threadIdx.x; j < in_chunk; j += kThreads) {
-      T v = red[0][j];
-#pragma unroll
-      for (int w = 1; w < kWaves; ++w) v = min(v, red[w][j]);
-      if (v != std::numeric_limits<T>::max()) atomicMin(&dst[j], v);
+    for (int k = 0; k < K; ++k) put(lane + kWave * k, m[k]);
+    if (TAIL) put(K * kWave + lane, TailT::value(tail));
+    if (tasks <= 8 * nwaves) {
+      task += nwaves;
+    } else {
+      unsigned long long next = 0;
+      if (lane == 0) next = atomicAdd(counter, 1ull);
+      task = nwaves + wave_bcast64(next, 0);
     }
   }
 }
@@ -531,16 +546,6 @@ struct ValidTimesP {
   __device__ uint64_t operator()(int64_t i) const { return col.valid(i) ? static_cast<uint64_t>(P) : 0; }
 };
 
-struct ExtraParts {
-  ColView col;
-  __device__ uint64_t operator()(int64_t i) const
-  {
-    if (!col.valid(i)) return 0;
-    int64_t const n = col.off(i + 1) - col.off(i);
-    return n > kSpan ? static_cast<uint64_t>((n + kSpan - 1) / kSpan - 1) : 0;
-  }
-};
-
 __global__ void uniform_offsets_kernel(int32_t* out, int32_t rows, int32_t P)
 {
   int64_t const i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -549,26 +554,89 @@ __global__ void uniform_offsets_kernel(int32_t* out, int32_t rows, int32_t P)
 
 constexpr int32_t kMaxRowBlocks = 1 << 15;  // groups along x (a launch of 4 M rows, 64 to a group, has two layers along z: the tests reach them)
 
-template <typename T, int K, bool TAIL>
-void launch_kernels(const ColView& v, T seed, const T* a, const T* b, int32_t P, int32_t width, const int32_t* offsets,
-                    const uint32_t* extra_prefix, T* child, hipStream_t stream)
+// The largest value into the slots of the rows that are done in several parts, and 0 into the counter of the parts: a
+// wavefront looks at 64 rows and fills those of them one after the other.
+template <typename T>
+__global__ void __launch_bounds__(kThreads) minhash_clear_kernel(RowParts parts, int32_t P, const int32_t* __restrict__ out_offsets,
+                                                                 unsigned long long* __restrict__ counter, T* __restrict__ out)
 {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *counter = 0;
+  int const lane  = lane_id();
+  int64_t const r = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  bool const many = r < parts.col.size && parts(r) > 1;
+  int64_t const o = many ? out_offsets[r] : 0;
+  for (uint64_t todo = ballot64(many); todo != 0; todo &= todo - 1) {
+    T* const dst = out + static_cast<int64_t>(wave_bcast64(static_cast<uint64_t>(o), __builtin_ctzll(todo)));
+    for (int32_t j = lane; j < P; j += kWave) dst[j] = std::numeric_limits<T>::max();
+  }
+}
+
+// Everything that comes before the hashing of a column of few rows, in one launch: workgroup 0 counts the parts of the
+// rows (and finds the rows' places in the result where some are null), the others write the places where none is and
+// fill the result.
+constexpr int32_t kPlanRows = kScanSmallTiles * kScanTile;
+template <typename T>
+__global__ void __launch_bounds__(kScanThreads) minhash_plan_kernel(RowParts parts, int32_t P, int32_t* __restrict__ out_offsets,
+                                                                    uint32_t* __restrict__ prefix, unsigned long long* __restrict__ counter,
+                                                                    T* __restrict__ out, int64_t out_size)
+{
+  int32_t const rows = parts.col.size;
+  if (blockIdx.x > 0) {
+    int64_t const first  = static_cast<int64_t>(blockIdx.x - 1) * kScanThreads + threadIdx.x;
+    int64_t const stride = static_cast<int64_t>(gridDim.x - 1) * kScanThreads;
+    if (!parts.col.use_mask)
+      for (int64_t i = first; i <= rows; i += stride) out_offsets[i] = static_cast<int32_t>(i * P);
+    for (int64_t i = first; i < out_size; i += stride) out[i] = std::numeric_limits<T>::max();
+    return;
+  }
+  __shared__ uint64_t lds[kScanThreads / kWave + 1];
+  uint64_t carry = 0;  // parts in the low half, valid rows in the high half
+  for (int32_t tile = 0; tile < rows; tile += kScanTile) {
+    int32_t const base = tile + static_cast<int32_t>(threadIdx.x) * kScanItems;
+    uint64_t vals[kScanItems], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+      bool const in = base + k < rows;
+      vals[k]       = in ? parts(base + k) | (static_cast<uint64_t>(parts.col.valid(base + k)) << 32) : 0;
+      sum += vals[k];
+    }
+    uint64_t total;
+    uint64_t run = block_exclusive_scan64<kScanThreads>(sum, lds, &total) + carry;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+      if (base + k < rows) {
+        prefix[base + k] = static_cast<uint32_t>(run);
+        if (parts.col.use_mask) out_offsets[base + k] = static_cast<int32_t>(run >> 32) * P;
+      }
+      run += vals[k];
+    }
+    carry += total;
+  }
+  if (threadIdx.x == 0) {
+    *counter     = 0;
+    prefix[rows] = static_cast<uint32_t>(carry);
+    if (parts.col.use_mask) out_offsets[rows] = static_cast<int32_t>(carry >> 32) * P;
+  }
+}
+
+template <typename T, int K, bool TAIL>
+void launch_kernels(RowParts const& parts, T seed, const T* a, const T* b, int32_t P, int32_t width, const int32_t* offsets,
+                    const uint32_t* prefix, unsigned long long* counter, T* child, hipStream_t stream)
+{
+  ColView const& v     = parts.col;
   int32_t const chunks = TAIL ? 1 : (P + K * kWave - 1) / (K * kWave);
-  int const solo_per_wave = solo_rows_per_wave(v.size);
-  int32_t const groups    = (v.size + solo_per_wave * kWaves - 1) / (solo_per_wave * kWaves);
-  dim3 grid(static_cast<unsigned>(std::min(groups, kMaxRowBlocks)), static_cast<unsigned>(chunks),
-            static_cast<unsigned>((groups + kMaxRowBlocks - 1) / kMaxRowBlocks));
-  {
+  if (v.size >= kManyRows) {
+    int const per_wave   = rows_per_wave(v.size);
+    int32_t const groups = (v.size + per_wave * kWaves - 1) / (per_wave * kWaves);
+    dim3 grid(static_cast<unsigned>(std::min(groups, kMaxRowBlocks)), static_cast<unsigned>(chunks),
+              static_cast<unsigned>((groups + kMaxRowBlocks - 1) / kMaxRowBlocks));
     ProfileScope ps("minhash_rows_kernel", stream);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_rows_kernel<T, K, TAIL>), grid, dim3(kThreads), 0, stream, v, seed, a, b, P, width, offsets, child,
-                       solo_per_wave);
+                       per_wave);
   }
-  dim3 grid2(4096, static_cast<unsigned>(chunks));
-  {
-    ProfileScope ps("minhash_extra_kernel", stream);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_extra_kernel<T, K, TAIL>), grid2, dim3(kThreads), 0, stream, v, seed, a, b, P, width, offsets,
-                       extra_prefix, child);
-  }
+  ProfileScope ps("minhash_parts_kernel", stream);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_parts_kernel<T, K, TAIL>), dim3(static_cast<unsigned>(parts.waves / kWaves)), dim3(kThreads), 0, stream, parts,
+                     seed, a, b, P, width, chunks, offsets, prefix, counter, child);
 }
 
 // How the parameters are shared out: chunks of K sets of 64 (every chunk hashes the windows again, and a lane without
@@ -594,32 +662,43 @@ inline Sharing sharing_for(int32_t P)
   return best;
 }
 
-// The launches of one minhash call: the row offsets of the result, the number of extra workgroup-spans of every
-// row, then the two hashing kernels.  extra_prefix holds rows + 1 values, scan_tmp scan_temp_bytes(rows) bytes.
+// The launches of one minhash call: the row offsets of the result and the parts of every row, then the hashing kernels.
+// prefix holds rows + 1 values, scan_tmp scan_temp_bytes(rows) bytes and one 64-bit counter behind them.
 template <typename T>
 void run_minhash(const ColView& v, T seed, const T* a, const T* b, int32_t P, int32_t width, int32_t* offsets, T* child, int64_t child_size,
-                 uint32_t* extra_prefix, uint64_t* scan_tmp, hipStream_t stream)
+                 uint32_t* prefix, uint64_t* scan_tmp, hipStream_t stream)
 {
   int32_t const rows = v.size;
-  if (v.use_mask) {
-    device_exclusive_scan(ValidTimesP{v, P}, static_cast<int64_t>(rows), offsets, scan_tmp, stream);
+  RowParts const parts{v, device_cus() * 4 * minhash_waves<T>(), rows >= kManyRows ? kPartBytes : -1};
+  auto* const counter = reinterpret_cast<unsigned long long*>(scan_tmp) + scan_temp_bytes(rows) / sizeof(uint64_t);
+  if (rows <= kPlanRows) {
+    int64_t const most    = std::max<int64_t>(child_size, rows + 1);
+    unsigned const groups = static_cast<unsigned>(std::min<int64_t>((most + 4 * kScanThreads - 1) / (4 * kScanThreads), 1024));
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_plan_kernel<T>), dim3(1 + groups), dim3(kScanThreads), 0, stream, parts, P, offsets, prefix, counter, child,
+                       child_size);
   } else {
-    hipLaunchKernelGGL(uniform_offsets_kernel, dim3((rows + 1 + 255) / 256), dim3(256), 0, stream, offsets, rows, P);
+    if (v.use_mask) {
+      device_exclusive_scan(ValidTimesP{v, P}, static_cast<int64_t>(rows), offsets, scan_tmp, stream);
+    } else {
+      hipLaunchKernelGGL(uniform_offsets_kernel, dim3((rows + 1 + 255) / 256), dim3(256), 0, stream, offsets, rows, P);
+    }
+    device_exclusive_scan(parts, static_cast<int64_t>(rows), prefix, scan_tmp, stream);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_clear_kernel<T>), dim3((rows + kThreads - 1) / kThreads), dim3(kThreads), 0, stream, parts, P, offsets, counter,
+                       child);
   }
-  device_exclusive_scan(ExtraParts{v}, static_cast<int64_t>(rows), extra_prefix, scan_tmp, stream);
 
   if (child_size > 0) {
     Sharing const sh = sharing_for(P);
     switch (sh.k * 2 + (sh.tail ? 1 : 0)) {
-      case 10: launch_kernels<T, 5, false>(v, seed, a, b, P, width, offsets, extra_prefix, child, stream); break;
-      case 9: launch_kernels<T, 4, true>(v, seed, a, b, P, width, offsets, extra_prefix, child, stream); break;
-      case 8: launch_kernels<T, 4, false>(v, seed, a, b, P, width, offsets, extra_prefix, child, stream); break;
-      case 7: launch_kernels<T, 3, true>(v, seed, a, b, P, width, offsets, extra_prefix, child, stream); break;
-      case 6: launch_kernels<T, 3, false>(v, seed, a, b, P, width, offsets, extra_prefix, child, stream); break;
-      case 5: launch_kernels<T, 2, true>(v, seed, a, b, P, width, offsets, extra_prefix, child, stream); break;
-      case 4: launch_kernels<T, 2, false>(v, seed, a, b, P, width, offsets, extra_prefix, child, stream); break;
-      case 3: launch_kernels<T, 1, true>(v, seed, a, b, P, width, offsets, extra_prefix, child, stream); break;
-      default: launch_kernels<T, 1, false>(v, seed, a, b, P, width, offsets, extra_prefix, child, stream); break;
+      case 10: launch_kernels<T, 5, false>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
+      case 9: launch_kernels<T, 4, true>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
+      case 8: launch_kernels<T, 4, false>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
+      case 7: launch_kernels<T, 3, true>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
+      case 6: launch_kernels<T, 3, false>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
+      case 5: launch_kernels<T, 2, true>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
+      case 4: launch_kernels<T, 2, false>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
+      case 3: launch_kernels<T, 1, true>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
+      default: launch_kernels<T, 1, false>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
     }
   }
 }
@@ -676,14 +755,14 @@ nvtext_amd_status minhash_impl(const nvtext_amd_strings_column* input, T seed, c
   }
 
   ColView const v = make_view(*input);
-  Temp scan_tmp(mr, scan_temp_bytes(rows));
-  Temp extra(mr, static_cast<size_t>(rows + 1) * sizeof(uint32_t));
-  if (!scan_tmp.ok() || !extra.ok()) {
+  size_t const temp_bytes[2] = {scan_temp_bytes(rows) + sizeof(uint64_t), static_cast<size_t>(rows + 1) * sizeof(uint32_t)};
+  TempParts<2> const temp(mr, temp_bytes);
+  if (!temp.ok()) {
     nvtext_amd_list_column_free(out, stream_, mr_);
     return fail(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");
   }
-  run_minhash<T>(v, seed, a, b, P, width, out->offsets, static_cast<T*>(out->child), out->child_size, extra.as<uint32_t>(),
-                 scan_tmp.as<uint64_t>(), stream);
+  run_minhash<T>(v, seed, a, b, P, width, out->offsets, static_cast<T*>(out->child), out->child_size, temp.part<uint32_t>(1),
+                 temp.part<uint64_t>(0), stream);
   NVTEXT_HIP_TRY_OR(hipGetLastError(), nvtext_amd_list_column_free(out, stream_, mr_));
   return NVTEXT_AMD_SUCCESS;
 }
@@ -874,7 +953,7 @@ void launch_ngrams(const ListView& v, int32_t ngrams, T seed, const T* a, const 
                    hipStream_t stream)
 {
   int32_t const chunks    = (P + K * kWave - 1) / (K * kWave);
-  int const solo_per_wave = v.size >= 131072 ? solo_rows_per_wave(v.size) : 0;
+  int const solo_per_wave = v.size >= kManyRows ? rows_per_wave(v.size) : 0;
   int32_t const group     = solo_per_wave > 0 ? solo_per_wave * kWaves : 1;
   int32_t const groups    = (v.size + group - 1) / group;
   dim3 grid(static_cast<unsigned>(std::min(groups, kMaxRowBlocks)), static_cast<unsigned>(chunks),
@@ -1025,13 +1104,13 @@ nvtext_amd_status nvtext_amd_minhash_preallocated(const nvtext_amd_strings_colum
   unsigned char* base = nullptr;
   nvtext_amd_status const st = scratch_of_current_device(&base);
   if (st != NVTEXT_AMD_SUCCESS) return st;
-  uint32_t* const extra_prefix = reinterpret_cast<uint32_t*>(base);
-  uint64_t* const scan_tmp     = reinterpret_cast<uint64_t*>(base + kScratchPrefixBytes);
+  uint32_t* const prefix   = reinterpret_cast<uint32_t*>(base);
+  uint64_t* const scan_tmp = reinterpret_cast<uint64_t*>(base + kScratchPrefixBytes);
 
   if (input->null_mask) launch_copy_bitmask(out_null_mask, input->null_mask, input->offset, rows, stream);
   ColView const v = make_view(*input);
   // every value of the scratch that the kernels read is written earlier in this same call: nothing to clear
-  run_minhash<uint32_t>(v, seed, a, b, P, width, out_offsets, out_child, child_size, extra_prefix, scan_tmp, stream);
+  run_minhash<uint32_t>(v, seed, a, b, P, width, out_offsets, out_child, child_size, prefix, scan_tmp, stream);
   NVTEXT_HIP_TRY(hipGetLastError());
   return NVTEXT_AMD_SUCCESS;
 }

@@ -14,7 +14,6 @@ constexpr int kThreads   = kWaves * kWave;     // 256
 constexpr int kTile      = 256;                // window starts per wavefront tile
 constexpr int kHalo      = 128;                // bytes staged past the tile (windows up to 32 4-byte chars)
 constexpr int kTileWords = (kTile + kHalo + 16 + 32) / 4;  // +16 misalignment, +32 for whole blocks and the over-read of the hash tail
-constexpr int kSpan      = 16384;              // bytes of a row handled by one workgroup
 
 // Windows repeat (text repeats its words: a tenth of the windows of a tile, a third within 4 KB of ordinary text), and a
 // hash that has been folded once changes no minimum when it is folded again.  Every wavefront keeps the hashes it

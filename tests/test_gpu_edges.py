@@ -46,3 +46,51 @@ def test_jaccard_pair_sizes(nv, orc, width):
     h1, h2 = (HostStringsColumn.from_pylist([t.decode() for t in rows]) for rows in (left, right))
     got, exp = nv.jaccard_index(dev(nv, h1), dev(nv, h2), width).to_host(), orc.jaccard_index(h1, h2, width, nthreads=8)
     assert np.array_equal(got.values.view(np.uint32), exp.values.view(np.uint32))
+
+
+def mixed_rows(rng, lens, nulls=()):
+    """Rows of these lengths as a column; the rows named in `nulls` are null (and empty)."""
+    lens = np.array(lens, np.int64)
+    lens[list(nulls)] = 0
+    offsets = np.concatenate([[0], np.cumsum(lens)])
+    chars = rng.choice(np.frombuffer(b"abcdefgh ", np.uint8), int(offsets[-1]))
+    mask = None
+    if nulls:
+        bits = np.ones((len(lens) + 31) // 32 * 32, np.uint8)
+        bits[len(lens):] = 0
+        bits[list(nulls)] = 0
+        mask = np.packbits(bits, bitorder="little").view(np.uint32)
+    return HostStringsColumn(chars, offsets.astype(np.int32), mask, len(lens), 0, len(nulls))
+
+
+def params(rng, count, bits):
+    dtype = np.uint32 if bits == 32 else np.uint64
+    return rng.integers(1, 2**bits, count, dtype=np.uint64).astype(dtype), rng.integers(0, 2**bits, count, dtype=np.uint64).astype(dtype)
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("count", [1, 33, 64, 128, 260, 700])
+def test_minhash_parts_of_rows(nv, orc, bits, count):
+    """Rows one byte around one part and several, parts of 256 bytes (little text) and of 4096 (8 MB and more), the
+    parameters in one chunk and in several, null and empty rows between them."""
+    rng = np.random.default_rng(count)
+    edges = [0, 1, 4, 5, 63, 64, 65, 255, 256, 257, 511, 513, 4095, 4096, 4097, 8192, 8193, 20_000]
+    call, ref = (nv.minhash, orc.minhash) if bits == 32 else (nv.minhash64, orc.minhash64)
+    a, b = params(rng, count, bits)
+    for more in ([], [3_000_000] * 11 if count == 64 else []):
+        host = mixed_rows(rng, edges + more + [0] + edges[::-1], nulls=(2, 20 + len(more)))
+        assert call(dev(nv, host), 5, a, b, 5).to_host().equals(ref(host, 5, a, b, 5, nthreads=8))
+
+
+@pytest.mark.parametrize("rows", [8192, 8193, 131_071, 131_072])
+@pytest.mark.parametrize("nulls", [False, True])
+def test_minhash_row_counts(nv, orc, rows, nulls):
+    """Around the row counts at which the plan takes several launches and at which short rows are done in groups."""
+    rng = np.random.default_rng(rows)
+    lens = rng.integers(0, 12, rows)
+    lens[[0, 7, rows // 2, rows - 1]] = [4097, 4096, 30_000, 9000]
+    host = mixed_rows(rng, lens, nulls=(1, rows // 3, rows - 2) if nulls else ())
+    a, b = params(rng, 3, 32)
+    assert nv.minhash(dev(nv, host), 5, a, b, 4).to_host().equals(orc.minhash(host, 5, a, b, 4, nthreads=8))
+    a, b = params(rng, 3, 64)
+    assert nv.minhash64(dev(nv, host), 5, a, b, 4).to_host().equals(orc.minhash64(host, 5, a, b, 4, nthreads=8))
