@@ -733,9 +733,9 @@ struct ShortWord {
   // trip waits twice: 18 % slower, the scattered reads cost more than the waits they save; settling pieces that need
   // no lookup several to a trip, also with their openings coming from LDS: fewer trips, each slower by more, and the
   // registers it takes cost wavefronts per SIMD, which this loop needs: 1.03 ms with 8 of them, 1.07 with 6, 1.28 with 4.)
-  template <typename Emit>
-  __device__ __forceinline__ void step(VocabTable const& t, const int32_t* first_ids, const uint16_t* l3, const int32_t* pair, const uint4* trim,
-                                       Emit&& emit)
+  // (next: the opening of the next piece, once the piece before it has been dropped)
+  template <typename Next, typename Emit>
+  __device__ __forceinline__ void step(VocabTable const& t, const uint4* trim, Next&& next, Emit&& emit)
   {
     uint32_t const kind = count ? 1u : 0u;
     cand &= (lens << 2) | 3u;
@@ -783,7 +783,7 @@ struct ShortWord {
     cand  = longer_left | (cand & 3u);
     if (hit && !done) {
       advance(len);  // next piece: the rest of the word (381-395)
-      open_piece(t, 1, request_next(t, first_ids, l3, pair));
+      open_piece(t, 1, next());
     }
   }
 };
@@ -859,7 +859,13 @@ struct TileArgs {
   uint32_t* queue_size;    // entries reserved so far
   uint32_t* counter;       // next range to hand out
   uint32_t* overflow;      // set when a range has more words than range_cap
+  // one launch for all (INLINE): the most bytes it is for, and what it leaves in place of the counters and flags
+  int64_t most_bytes;
+  uint32_t* first_row_out; // as range_first_row
+  uint32_t* range_notes;   // per range: kNoteSpill, kNoteAgain
 };
+constexpr uint32_t kNoteSpill = 1u;  // more words than range_cap, or more of them not in the vocabulary than queue_cap
+constexpr uint32_t kNoteAgain = 2u;  // a word of more tokens than a queue record keeps
 
 // The flag words of a tokenize call (indices of 32-bit words; what is asked for with atomics has a 128-byte line of its own):
 constexpr uint32_t kCounterGroups = 8;
@@ -971,9 +977,25 @@ __global__ void range_first_row_kernel(ColView col, int64_t first_offset, uint32
 // drop the words past each row's limit; list the words (word k pairs start k with end k); look all of them up (lanes
 // <-> words, one probe each) and write their slots; give every row that starts in the tile the number of words of the
 // range before it.
-template <int TILE, bool IS64, bool LIMIT>
-__global__ void __launch_bounds__(kTokThreads, 6) wordpiece_word_kernel(TileArgs a)
+// INLINE (a small column, where the launches and the waits for one another would be most of the call): a range is one
+// tile; where the bytes lie and which rows the range has the wavefront finds out itself, from the offsets; and it
+// tokenizes the words that are not in the vocabulary itself, lanes <-> words, into the range's own part of the queue
+// (queue_cap records), where the other way leaves the out-of-vocabulary pass to put its results.
+template <int TILE, bool IS64, bool LIMIT, bool INLINE>
+__global__ void __launch_bounds__(kTokThreads, INLINE ? 4 : 6) wordpiece_word_kernel(TileArgs a)
 {
+  if constexpr (INLINE) {
+    int64_t const first_offset = a.col.off(0), bytes = a.col.off(a.col.size) - first_offset;
+    if (bytes <= 0 || bytes > a.most_bytes) return;
+    const uint8_t* const first_byte = a.col.chars + first_offset;
+    a.first_offset = first_offset;
+    a.cbeg         = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(first_byte) & 15u);
+    a.abase        = reinterpret_cast<const uint4*>(first_byte - a.cbeg);
+    a.cend         = a.cbeg + bytes;
+    a.ntiles       = (a.cend + TILE - 1) / TILE;
+    a.nranges      = static_cast<uint32_t>(a.ntiles);
+    a.range_tiles  = 1;
+  }
   constexpr int kBlocks       = TILE / 16;
   constexpr int kSubs         = kBlocks / kWave;
   constexpr uint32_t kWordCap = TileLds<TILE>::kWordCap;
@@ -1000,19 +1022,52 @@ __global__ void __launch_bounds__(kTokThreads, 6) wordpiece_word_kernel(TileArgs
   const uint8_t* const lds_byte = reinterpret_cast<const uint8_t*>(lds.bytes);
   uint16_t* const word16        = reinterpret_cast<uint16_t*>(lds.word);
   uint32_t q_pos = 0, q_lim = 0;  // this wavefront's reserved queue entries [q_pos, q_lim)
+  uint32_t inline_range = 0;
 
   uint32_t const my_number = blockIdx.x * kTokWaves + threadIdx.x / kWave;
   for (bool first = true;; first = false) {
-    uint32_t const range = next_unit(a.counter, first, my_number, lane);
+    uint32_t range;
+    if constexpr (INLINE) {
+      range = first ? static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(my_number))) : inline_range + gridDim.x * kTokWaves;
+      inline_range = range;
+    } else {
+      range = next_unit(a.counter, first, my_number, lane);
+    }
     if (range >= a.nranges) break;
     int64_t t           = static_cast<int64_t>(range) * a.range_tiles;
     int64_t const t_end = min(t + a.range_tiles, a.ntiles);
-    uint32_t r_cur      = a.range_first_row[range];
+    uint32_t r_cur;
+    if constexpr (INLINE) {
+      // the first row that starts at or after the tile's first byte, 64 rows looked at in one step
+      uint32_t lo = 0, hi = rows;  // the answer lies in [lo, hi]
+      while (lo < hi) {
+        uint32_t const step = (hi - lo + kWave - 1) / kWave;
+        uint32_t const at   = lo + step * static_cast<uint32_t>(lane);
+        bool const before   = at < hi && coord(at) < t * TILE;
+        uint32_t const n    = static_cast<uint32_t>(__builtin_popcountll(ballot64(before)));
+        if (n == 0) break;  // (lo)
+        hi = min(hi, lo + n * step);
+        lo = lo + (n - 1) * step + 1;
+      }
+      r_cur = lo;
+      if (lane == 0) {
+        a.first_row_out[range] = r_cur;
+        if (range + 1 == a.nranges) a.first_row_out[a.nranges] = rows;
+      }
+    } else {
+      r_cur = a.range_first_row[range];
+    }
     uint32_t cursor     = 0;  // words of this range so far
     uint32_t known      = 0;  // of them, in the vocabulary (or too long: one unknown token each)
+    uint32_t oov_tokens = 0;  // INLINE: tokens of the others, my lane's
     uint32_t open_left  = 0;  // words the row that runs into the tile may still have (with a word limit)
     uint32_t* const region = a.arena + static_cast<int64_t>(range) * a.range_cap;
     bool spill             = false;
+    bool again             = false;  // INLINE: a word of more tokens than its record keeps
+    if constexpr (INLINE) {
+      q_pos = range * a.queue_cap;
+      q_lim = q_pos + a.queue_cap;
+    }
     if (LIMIT && r_cur > 0) {
       uint32_t const ro  = r_cur - 1;
       int64_t const c0   = coord(ro), c1 = coord(ro + 1);
@@ -1299,7 +1354,9 @@ __global__ void __launch_bounds__(kTokThreads, 6) wordpiece_word_kernel(TileArgs
           uint32_t value       = too_long ? static_cast<uint32_t>(table.unk_id) : static_cast<uint32_t>(id);
           uint64_t const mm    = ballot64(defer != 0);
           uint32_t const nm    = static_cast<uint32_t>(__builtin_popcountll(mm));
-          if (listed + nm > room && !have_fresh) {
+          if constexpr (INLINE) {
+            if (listed + nm > room) spill = true;
+          } else if (listed + nm > room && !have_fresh) {
             if (lane == 0) fresh = atomicAdd(a.queue_size, kQueueChunk);
             fresh      = wave_bcast(fresh, 0);
             have_fresh = true;
@@ -1328,7 +1385,40 @@ __global__ void __launch_bounds__(kTokThreads, 6) wordpiece_word_kernel(TileArgs
             uint4 const keep = trim[min(wl, 16u)];
             int64_t const at = tb + s;
             uint32_t const q = queue_place(c);
-            if (q < a.queue_cap) {
+            if constexpr (INLINE) {
+              int32_t tok[kOovKeep];
+              auto const keep_token = [&](uint32_t j, int32_t id) {
+#pragma unroll
+                for (int i = 0; i < kOovKeep; ++i)
+                  if (j == static_cast<uint32_t>(i)) tok[i] = id;
+              };
+              uint32_t count;
+              if (wl <= 16) {
+                head[0] &= keep.x;
+                head[1] &= keep.y;
+                head[2] &= keep.z;
+                head[3] &= keep.w;
+                const int32_t* const first_ids = table.short_ids + 2 * 65536;
+                ShortWord sw;
+                sw.begin(table, first_ids, head, wl, defer == 1u, false);
+                while (!sw.done) sw.step(table, trim, [&] { return sw.request(table, first_ids, 1u, 0u); }, keep_token);
+                count = sw.count;
+              } else {
+                count = tokenize_oov_word(table, tw, wl, keep_token);
+              }
+              oov_tokens += count;
+              if (count > kOovKeep) again = true;
+              if (c < room) {
+                uint4* const dst = reinterpret_cast<uint4*>(a.queue + q);
+                if (count <= kOovKeep) {
+                  dst[0] = make_uint4(static_cast<uint32_t>(tok[0]), static_cast<uint32_t>(tok[1]), static_cast<uint32_t>(tok[2]), static_cast<uint32_t>(tok[3]));
+                  dst[1] = make_uint4(static_cast<uint32_t>(tok[4]), static_cast<uint32_t>(tok[5]), static_cast<uint32_t>(tok[6]), count);
+                } else {  // (as the out-of-vocabulary pass leaves it)
+                  dst[0] = make_uint4(0u, 0u, 0u, static_cast<uint32_t>(static_cast<uint64_t>(at) >> 32));
+                  dst[1] = make_uint4(wl | (defer == 2u ? kUnprobed : 0u), range, static_cast<uint32_t>(at), count);
+                }
+              }
+            } else if (q < a.queue_cap) {
               uint4* const dst = reinterpret_cast<uint4*>(a.queue + q);
               store_stream(dst, make_uint4(head[0] & keep.x, head[1] & keep.y, head[2] & keep.z, head[3] & keep.w));
               store_stream(dst + 1, make_uint4(wl | (defer == 2u ? kUnprobed : 0u), range, static_cast<uint32_t>(at),
@@ -1336,7 +1426,9 @@ __global__ void __launch_bounds__(kTokThreads, 6) wordpiece_word_kernel(TileArgs
             }
           }
         }
-        if (listed > room) {
+        if (INLINE) {
+          q_pos += min(listed, room);
+        } else if (listed > room) {
           q_pos = fresh + (listed - room);
           q_lim = fresh + kQueueChunk;
         } else {
@@ -1347,12 +1439,20 @@ __global__ void __launch_bounds__(kTokThreads, 6) wordpiece_word_kernel(TileArgs
         if (w_hi == nw) break;
       }
     }
+    if constexpr (INLINE) {
+      known += wave_bcast(wave_inclusive_scan(oov_tokens), kWave - 1);
+      again = ballot64(again) != 0;
+    }
     if (lane == 0) {
       a.range_words[range]  = cursor;
       a.range_tokens[range] = known;
-      if (spill) *a.overflow = 1u;
+      if (INLINE)
+        a.range_notes[range] = (spill ? kNoteSpill : 0u) | (again ? kNoteAgain : 0u);
+      else if (spill)
+        *a.overflow = 1u;
     }
   }
+  if (INLINE) return;
   // the reserved entries that no word took
   for (uint32_t q = q_pos + lane; q < q_lim; q += kWave)
     if (q < a.queue_cap) a.queue[q].len_flags = 0;
@@ -1543,7 +1643,7 @@ __global__ void __launch_bounds__(kOovThreads, 8) wordpiece_oov_kernel(VocabTabl
       if (drained && ballot64(busy) == 0) break;
       continue;
     }
-    if (busy && !sw.done) sw.step(table, first_ids, letters3, pair_ids, trim, keep_token);
+    if (busy && !sw.done) sw.step(table, trim, [&] { return sw.request_next(table, first_ids, letters3, pair_ids); }, keep_token);
   }
   add_together(acc_count != 0);
 }
@@ -1773,11 +1873,24 @@ __global__ void __launch_bounds__(kRareThreads) wordpiece_retokenize_kernel(Voca
 // looked up whole.  It runs on the offsets alone, before the host knows where the bytes begin, and leaves the view's
 // first and last offset for the host as well: the call synchronises once for both.
 constexpr int kSampleWindows = 512;
+// A column that is put on the stream whole before its size is known (see nvtext_amd_wordpiece_tokenize).  One launch that
+// does everything per tile beats the three passes up to about 50 MB of text (16 MB of the benchmark's rows 125 against
+// 245 us, 32 MB 211 against 286, 48 MB 300 against 319, 60 MB 359 against 337), after which the passes' better use of the
+// lanes tells; it stops at 32 MB for its temporaries, six bytes per byte that the column might have.
+constexpr int32_t kSmallRows     = 131072;
+constexpr int64_t kSmallRowBytes = 4096;
+constexpr int64_t kSmallLeast    = 256 << 10;
+constexpr int64_t kSmallBytes    = 32 << 20;
+constexpr int kSmallTile         = 1024;
+constexpr uint32_t kSmallSlots   = kSmallTile / 2 + 8;  // words of a tile: one letter and a space each (rows of one letter go the other way)
+constexpr unsigned kSmallGrid    = 2048;                // workgroups at most: a wavefront then takes several tiles
+constexpr uint32_t kSmallQueue   = kSmallTile / 8;  // words of a tile that are not in the vocabulary (one in 37 bytes on the benchmark's rows)
 constexpr int kSampleBytes   = 512;
 constexpr int kSampleTail    = 208;  // bytes staged past a window: a word that starts in it ends there, or is kMaxWord bytes or more
 static_assert(3 * kSampleWindows <= kHostSampleWords, "a window's three counts fit the pinned words");
 
-__global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, VocabTable table, uint64_t* __restrict__ first_last,
+// (skip_bytes: a column of at most so many bytes is not sampled)
+__global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, VocabTable table, int64_t skip_bytes, uint64_t* __restrict__ first_last,
                                                                uint32_t* __restrict__ counts)
 {
   __shared__ uint32_t staged[(kSampleBytes + kSampleTail + 8) / 4 + 4];  // byte 4 + x of it: byte x of the window; byte 3: the one before
@@ -1788,6 +1901,7 @@ __global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, Vo
     first_last[1] = static_cast<uint64_t>(last);
   }
   int64_t const span    = last - first;
+  if (span <= skip_bytes) return;
   int64_t const windows = min(static_cast<int64_t>(kSampleWindows), (span + kSampleBytes - 1) / kSampleBytes);
   uint32_t words = 0, queued = 0, bytes = 0;
   if (static_cast<int64_t>(blockIdx.x) < windows) {
@@ -1841,6 +1955,50 @@ __global__ void publish_state_kernel(const uint64_t* __restrict__ total, const u
   if (threadIdx.x == 0) dst[0] = *total;
   if (threadIdx.x == 1) dst[1] = flags[kFlagOverflow];
   if (threadIdx.x == 2) dst[2] = flags[kFlagQueueSize];
+}
+
+// The same, and the places of the ranges' tokens, after the one launch for a small column: one workgroup.  dst[0] = the
+// number of tokens, dst[1] = the ranges' notes together.
+constexpr int kFinishThreads = 1024;
+__global__ void __launch_bounds__(kFinishThreads) wordpiece_finish_kernel(TileArgs a, int tile, int64_t* __restrict__ bases, uint32_t* __restrict__ again_count,
+                                                                          uint64_t* __restrict__ dst)
+{
+  __shared__ uint64_t lds[kFinishThreads / kWave + 1];
+  __shared__ uint32_t all_notes;
+  int64_t const first_offset = a.col.off(0), bytes = a.col.off(a.col.size) - first_offset;
+  if (bytes <= 0 || bytes > a.most_bytes) return;
+  int64_t const cbeg   = static_cast<int64_t>(reinterpret_cast<uintptr_t>(a.col.chars + first_offset) & 15u);
+  uint32_t const n     = static_cast<uint32_t>((cbeg + bytes + tile - 1) / tile);
+  uint32_t notes = 0;
+  uint64_t carry = 0;
+  if (threadIdx.x == 0) all_notes = 0;
+  constexpr uint32_t kEach = 4;
+  for (uint32_t base = 0; base < n; base += kEach * kFinishThreads) {
+    uint32_t const i = base + kEach * threadIdx.x;
+    uint64_t v[kEach], sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kEach; ++k) {
+      v[k] = i + k < n ? a.range_tokens[i + k] : 0;
+      if (i + k < n) notes |= a.range_notes[i + k];
+      sum += v[k];
+    }
+    uint64_t total;
+    uint64_t run = carry + block_exclusive_scan64<kFinishThreads>(sum, lds, &total);
+#pragma unroll
+    for (uint32_t k = 0; k < kEach; ++k) {
+      if (i + k < n) bases[i + k] = static_cast<int64_t>(run);
+      run += v[k];
+    }
+    carry += total;
+  }
+  __syncthreads();
+  if (notes) atomicOr(&all_notes, notes);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    *again_count = 0;
+    dst[0]       = carry;
+    dst[1]       = all_notes;
+  }
 }
 
 struct RangeTokensOf {
@@ -2278,14 +2436,94 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   uint64_t* const scalars = host_scalars();  // pinned words that kernels write for the host (nullptr: copy instead)
   bool const sampling     = g_sizing_sample.load(std::memory_order_relaxed) != 0;
   double sample_words = 0, sample_queued = 0, sample_bytes = 0;  // what the sample found (nothing without the pinned words)
+  bool const is64  = input->offsets_is_int64 != 0;
+  bool const limit = max_words_per_row > 0;
+  // A column of few rows is probably small, and then the call is launches and waits more than work: everything up to the
+  // number of tokens is put on the stream at once, for a column of up to kSmallRowBytes bytes a row and kSmallBytes in all,
+  // before the host knows how many bytes there are.  Where there are more, these kernels leave at once, the sample that
+  // follows them does what it does for a large column, and the call goes on from there.
+  // (29 rows of 180 bytes: 87 us in eleven launches with two waits, 43 us in four with one; 32,768 rows of 120 bytes
+  // 145 -> 60 us)
+  bool const small = scalars && sampling && rows <= kSmallRows && g_forced_range_tiles.load(std::memory_order_relaxed) == 0;
+  int64_t const small_bytes = small ? std::min(std::max(static_cast<int64_t>(rows) * kSmallRowBytes, kSmallLeast), kSmallBytes) : 0;
+  uint32_t const small_ranges = static_cast<uint32_t>(small_bytes / kSmallTile + 1);
+  size_t const small_temp_bytes[8] = {static_cast<size_t>(small_ranges) * kSmallSlots * sizeof(uint32_t),
+                                      (static_cast<size_t>(small_ranges) + 1) * sizeof(uint32_t),
+                                      static_cast<size_t>(small_ranges) * sizeof(uint32_t),
+                                      static_cast<size_t>(small_ranges) * sizeof(uint32_t),
+                                      static_cast<size_t>(small_ranges) * sizeof(uint32_t),
+                                      (static_cast<size_t>(small_ranges) + 1) * sizeof(int64_t),
+                                      (static_cast<size_t>(small_ranges) * kSmallQueue + 1) * sizeof(uint32_t),
+                                      static_cast<size_t>(small_ranges) * kSmallQueue * sizeof(OovEntry)};
+  bool tried = false;
+  if (small) {
+    TempParts<8> const temps(mr, small_temp_bytes);
+    if (temps.ok()) {
+      tried = true;
+      TileArgs args{};
+      args.col           = v;
+      args.table         = vocabulary->table;
+      args.max_words     = max_words_per_row;
+      args.range_cap     = kSmallSlots;
+      args.arena         = temps.part<uint32_t>(0);
+      args.first_row_out = temps.part<uint32_t>(1);
+      args.range_words   = temps.part<uint32_t>(2);
+      args.range_tokens  = temps.part<uint32_t>(3);
+      args.range_notes   = temps.part<uint32_t>(4);
+      args.offsets_out   = out->offsets;
+      args.queue         = temps.part<OovEntry>(7);
+      args.queue_cap     = kSmallQueue;
+      args.most_bytes    = small_bytes;
+      int64_t* const bases        = temps.part<int64_t>(5);
+      uint32_t* const again_count = temps.part<uint32_t>(6);
+      void (*const kernel)(TileArgs) = is64 ? (limit ? wordpiece_word_kernel<kSmallTile, true, true, true> : wordpiece_word_kernel<kSmallTile, true, false, true>)
+                                            : (limit ? wordpiece_word_kernel<kSmallTile, false, true, true> : wordpiece_word_kernel<kSmallTile, false, false, true>);
+      {
+        ProfileScope ps("wordpiece_word_kernel (small column)", stream);
+        hipLaunchKernelGGL(kernel, dim3(std::min((small_ranges + kTokWaves - 1) / kTokWaves, kSmallGrid)), dim3(kTokThreads), 0, stream, args);
+      }
+      hipLaunchKernelGGL(wordpiece_finish_kernel, dim3(1), dim3(kFinishThreads), 0, stream, args, kSmallTile, bases, again_count, scalars + 2);
+      hipLaunchKernelGGL(wordpiece_sample_kernel, dim3(kSampleWindows), dim3(kWave), 0, stream, v, vocabulary->table, small_bytes, scalars,
+                         reinterpret_cast<uint32_t*>(scalars + 8));
+      hipError_t e = hipGetLastError();
+      if (e == hipSuccess) e = hipStreamSynchronize(stream);
+      if (e != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
+      first_offset = static_cast<int64_t>(scalars[0]);
+      last_offset  = static_cast<int64_t>(scalars[1]);
+      if (last_offset > first_offset && last_offset - first_offset <= small_bytes && (scalars[3] & kNoteSpill) == 0) {
+        uint64_t const total = scalars[2];
+        out->child_size      = static_cast<int64_t>(total);
+        out->child_bytes     = static_cast<size_t>(total) * sizeof(int32_t);
+        if (total) {
+          out->child = mr.allocate(out->child_bytes);
+          if (!out->child) return give_up(NVTEXT_AMD_ALLOC_FAILED, "child allocation failed");
+        }
+        const uint8_t* const first_byte = v.chars + first_offset;
+        uint32_t const cbeg             = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(first_byte) & 15u);
+        uint32_t const nranges          = static_cast<uint32_t>((cbeg + (last_offset - first_offset) + kSmallTile - 1) / kSmallTile);
+        ProfileScope ps("wordpiece_emit_kernel", stream);
+        hipLaunchKernelGGL(wordpiece_emit_kernel, dim3((nranges + kTokWaves - 1) / kTokWaves), dim3(kTokThreads), 0, stream, nranges, args.arena, kSmallSlots,
+                           args.range_words, bases, args.first_row_out, args.queue, out->offsets, static_cast<int32_t*>(out->child), again_count + 1,
+                           again_count);
+        if (scalars[3] & kNoteAgain)
+          hipLaunchKernelGGL(wordpiece_retokenize_kernel, dim3(64), dim3(kRareThreads), 0, stream, vocabulary->table,
+                             reinterpret_cast<const uint4*>(first_byte - cbeg), args.queue, again_count + 1, again_count, static_cast<int32_t*>(out->child));
+        if (hipGetLastError() != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, "kernel launch failed");
+        return NVTEXT_AMD_SUCCESS;
+      }
+    }  // (no room for the temporaries of the largest column that it might be: as for a large column)
+  }
+  bool const have_sample = tried && last_offset - first_offset > small_bytes;
   if (scalars) {
     uint32_t* const counts = reinterpret_cast<uint32_t*>(scalars + 8);
-    if (sampling)
-      hipLaunchKernelGGL(wordpiece_sample_kernel, dim3(kSampleWindows), dim3(kWave), 0, stream, v, vocabulary->table, scalars, counts);
+    if (have_sample) {
+      // (the two offsets as well)
+    } else if (sampling)
+      hipLaunchKernelGGL(wordpiece_sample_kernel, dim3(kSampleWindows), dim3(kWave), 0, stream, v, vocabulary->table, int64_t{-1}, scalars, counts);
     else
       launch_read_two_offsets(input->offsets, input->offsets_is_int64 != 0, input->offset, static_cast<int64_t>(input->offset) + rows, scalars, stream);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(stream);
+    if (e == hipSuccess && !have_sample) e = hipStreamSynchronize(stream);
     if (e != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
     first_offset = static_cast<int64_t>(scalars[0]);
     last_offset  = static_cast<int64_t>(scalars[1]);
@@ -2340,10 +2578,8 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     }
     return static_cast<int64_t>(per_cu) * cus;
   };
-  bool const is64  = input->offsets_is_int64 != 0;
-  bool const limit = max_words_per_row > 0;
-  void (*const word_kernel)(TileArgs) = is64 ? (limit ? wordpiece_word_kernel<kTile, true, true> : wordpiece_word_kernel<kTile, true, false>)
-                                             : (limit ? wordpiece_word_kernel<kTile, false, true> : wordpiece_word_kernel<kTile, false, false>);
+  void (*const word_kernel)(TileArgs) = is64 ? (limit ? wordpiece_word_kernel<kTile, true, true, false> : wordpiece_word_kernel<kTile, true, false, false>)
+                                             : (limit ? wordpiece_word_kernel<kTile, false, true, false> : wordpiece_word_kernel<kTile, false, false, false>);
   int64_t const word_resident = resident(reinterpret_cast<const void*>(word_kernel), kTokThreads, (is64 ? 2 : 0) + (limit ? 1 : 0));
   // A range is what a wavefront works through by itself, one tile after the other: kRangeTiles tiles when that still
   // leaves every wavefront of the word pass eight ranges or more (the last ones then end close together), fewer in a

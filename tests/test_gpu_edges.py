@@ -94,3 +94,54 @@ def test_minhash_row_counts(nv, orc, rows, nulls):
     assert nv.minhash(dev(nv, host), 5, a, b, 4).to_host().equals(orc.minhash(host, 5, a, b, 4, nthreads=8))
     a, b = params(rng, 3, 64)
     assert nv.minhash64(dev(nv, host), 5, a, b, 4).to_host().equals(orc.minhash64(host, 5, a, b, 4, nthreads=8))
+
+
+def words_column(rng, lens, vocabulary, oov):
+    """Rows of about these many bytes: words of the vocabulary, and `oov` of them random letters."""
+    stems = [w for w in vocabulary if not w.startswith("##") and not w.startswith("[")]
+    rows = []
+    for n in lens:
+        parts, size = [], 0
+        while size < n:
+            w = stems[int(rng.integers(0, len(stems)))] if rng.random() >= oov else "".join(rng.choice(list("abcdefgxyz"), int(rng.integers(1, 26))))
+            parts.append(w)
+            size += len(w) + 1
+        rows.append(" ".join(parts)[:n])
+    return HostStringsColumn.from_pylist(rows)
+
+
+LETTERS = list("abcdefghijklmnopqrstuvwxyz")
+VOCABULARY = ["[PAD]", "[UNK]"] + LETTERS[:20] + ["##" + c for c in LETTERS[:20]] + ["hello", "world", "data", "frame", "##ing", "##ed", "abc", "##abc", "internationalization",
+                                                                                      "naïve", "漢", "##漢"]
+
+
+@pytest.mark.parametrize("limit", [0, 1, 9])
+@pytest.mark.parametrize("oov", [0.0, 0.2, 1.0])
+def test_tokenize_small_columns(nv, orc, limit, oov):
+    """Columns that are tokenized in one launch: rows around the 1024-byte tiles and across several of them, words of more
+    than sixteen bytes and of more than seven tokens, every word unknown (too many for a tile's records: the passes of a
+    large column then), one-letter words and rows, a view."""
+    rng = np.random.default_rng(int(10 * oov) + limit)
+    hv = HostStringsColumn.from_pylist(VOCABULARY)
+    vocabulary, reference = nv.WordPieceVocabulary(dev(nv, hv)), orc.Vocabulary(hv)
+    columns = [words_column(rng, [1], VOCABULARY, oov), words_column(rng, [1023, 1, 1024, 0, 1025, 2047, 5000, 3, 16, 17], VOCABULARY, oov),
+               words_column(rng, list(rng.integers(0, 90, 3000)), VOCABULARY, oov),
+               HostStringsColumn.from_pylist(["a b c d e " * 300, "漢 naïve 漢漢漢漢漢漢漢漢 " * 50, "x" * 199 + " " + "y" * 200 + " " + "a" * 40] + ["a"] * 2000)]
+    for host in columns:
+        d = dev(nv, host)
+        assert nv.wordpiece_tokenize(d, vocabulary, limit).to_host().equals(orc.wordpiece_tokenize(host, reference, limit))
+        if host.size > 8:
+            view = host.slice(3, host.size - 2)
+            assert nv.wordpiece_tokenize(d.slice(3, host.size - 2, 0), vocabulary, limit).to_host().equals(orc.wordpiece_tokenize(view, reference, limit))
+
+
+@pytest.mark.parametrize("rows, each", [(4, 65_537), (4, 65_535), (131_072, 10), (131_073, 10), (9000, 3800)])
+def test_tokenize_where_small_columns_end(nv, orc, rows, each):
+    """Around the bytes (256 KiB; 32 MiB) and the rows up to which a column is put on the stream before its size is known."""
+    rng = np.random.default_rng(rows)
+    hv = HostStringsColumn.from_pylist(VOCABULARY)
+    vocabulary, reference = nv.WordPieceVocabulary(dev(nv, hv)), orc.Vocabulary(hv)
+    text = words_column(rng, [rows * each], VOCABULARY, 0.1)
+    offsets = np.linspace(0, rows * each, rows + 1).astype(np.int32)
+    host = HostStringsColumn(text.chars, offsets, None, rows, 0, 0)
+    assert nv.wordpiece_tokenize(dev(nv, host), vocabulary, 50).to_host().equals(orc.wordpiece_tokenize(host, reference, 50, nthreads=8))
