@@ -165,7 +165,8 @@ struct TempParts {
     for (int i = 0; i < N; ++i) sum += (bytes[i] + 255) & ~static_cast<size_t>(255);
     return sum;
   }
-  TempParts(Mr m, const size_t (&bytes)[N]) : whole(m, total(bytes))
+  // (wanted: false for no allocation at all)
+  TempParts(Mr m, const size_t (&bytes)[N], bool wanted = true) : whole(m, wanted ? total(bytes) : 0)
   {
     at[0] = 0;
     for (int i = 0; i < N; ++i) at[i + 1] = at[i] + ((bytes[i] + 255) & ~static_cast<size_t>(255));
@@ -491,6 +492,8 @@ int device_cus();
 constexpr size_t kHostSampleWords = 3 * 512;
 constexpr size_t kHostScalarBytes = 8 * sizeof(uint64_t) + kHostSampleWords * sizeof(uint32_t);
 uint64_t* host_scalars();
+// *dst = *src
+void launch_publish(const uint64_t* src, uint64_t* dst, hipStream_t stream);
 // dst[0] = offsets[first_index], dst[1] = offsets[last_index] (offsets of 32 or 64 bits)
 void launch_read_two_offsets(const void* offsets, int is64, int64_t first_index, int64_t last_index, uint64_t* dst, hipStream_t stream);
 

@@ -187,6 +187,15 @@ uint64_t* host_scalars()
   return slot.p;
 }
 
+namespace {
+__global__ void publish_kernel(const uint64_t* __restrict__ src, uint64_t* __restrict__ dst) { *dst = *src; }
+}  // namespace
+
+void launch_publish(const uint64_t* src, uint64_t* dst, hipStream_t stream)
+{
+  hipLaunchKernelGGL(publish_kernel, dim3(1), dim3(1), 0, stream, src, dst);
+}
+
 void launch_read_two_offsets(const void* offsets, int is64, int64_t first_index, int64_t last_index, uint64_t* dst, hipStream_t stream)
 {
   hipLaunchKernelGGL(read_two_offsets_kernel, dim3(1), dim3(2), 0, stream, offsets, is64, first_index, last_index, dst);

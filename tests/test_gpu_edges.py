@@ -145,3 +145,27 @@ def test_tokenize_where_small_columns_end(nv, orc, rows, each):
     offsets = np.linspace(0, rows * each, rows + 1).astype(np.int32)
     host = HostStringsColumn(text.chars, offsets, None, rows, 0, 0)
     assert nv.wordpiece_tokenize(dev(nv, host), vocabulary, 50).to_host().equals(orc.wordpiece_tokenize(host, reference, 50, nthreads=8))
+
+
+@pytest.mark.parametrize("rows, each", [(1, 1), (3, 2047), (3, 2048), (61, 300), (4, 65_535), (4, 65_537), (131_072, 9), (131_073, 9), (30_000, 2300)])
+def test_normalize_where_small_columns_end(nv, rows, each):
+    """Tiles of 2048 bytes and their remainders, and the bytes (256 KiB; 64 MiB) and rows up to which a column is worked on
+    before its size is known; a view of it too."""
+    from oracle import normalize_py
+    rng = np.random.default_rng(rows)
+    text = "Héllo Wörld, [CLS] naïve 漢字! ΑΒΓ don't [sep] plain words and more plain words of text "
+    chars = np.frombuffer((text * (rows * each // len(text) + 1)).encode(), np.uint8).copy()
+    cuts = np.sort(rng.integers(0, chars.size, rows - 1)) if rows > 1 else np.zeros(0, np.int64)
+    while True:  # whole characters
+        inside = (cuts > 0) & ((chars[np.minimum(cuts, chars.size - 1)] & 0xC0) == 0x80)
+        if not inside.any():
+            break
+        cuts[inside] -= 1
+    host = HostStringsColumn(chars, np.concatenate([[0], cuts, [chars.size]]).astype(np.int32), None, rows, 0, 0)
+    special = HostStringsColumn.from_pylist(["[CLS]", "[SEP]"])
+    normalizer = nv.CharacterNormalizer(True, dev(nv, special))
+    d = dev(nv, host)
+    for lo, hi in ((0, rows), (1, rows - 1)) if rows > 4 else ((0, rows),):
+        got = nv.normalize_characters(d.slice(lo, hi, 0), normalizer).to_host()
+        exp = normalize_py.normalize_characters_native(host.slice(lo, hi), True, [b"[CLS]", b"[SEP]"], nthreads=8)
+        assert np.array_equal(got.chars, exp.chars) and np.array_equal(got.offsets, exp.offsets)
