@@ -20,6 +20,7 @@
 // Null rows get no output slot (the reference drops them with purge_nonempty_nulls,
 // minhash.cu:626-628), empty rows are all zeros (minhash.cu:318).
 #include "common.cuh"
+#include "filter64.cuh"
 #include "murmur.cuh"
 #include "windows.cuh"
 
@@ -48,7 +49,7 @@ struct HashTraits<uint32_t> {
     return murmur3_x86_32(src, len, seed);
   }
   // Permutation (minhash.cu:350-351) in uint32 arithmetic: the product and sum wrap mod 2^32, after
-  // which "% (2^61-1)" and "& max" change nothing: (hv * a + b), see Fold<uint32_t>.
+  // which "% (2^61-1)" and "& max" change nothing: (hv * a + b), see Fold.
 };
 template <>
 struct HashTraits<uint64_t> {
@@ -57,58 +58,8 @@ struct HashTraits<uint64_t> {
   {
     return murmur3_x64_128_lo(src, len, seed);  // minhash.cu:138: first word of the 128-bit hash
   }
-  // Permutation (minhash.cu:350-351): ((hv*a + b) mod 2^64) % (2^61-1), see Fold<uint64_t>.
+  // Permutation (minhash.cu:350-351): ((hv*a + b) mod 2^64) % (2^61-1), see filter64.cuh.
 };
-
-// ((h * a + b) mod 2^64) folded once mod 2^61 - 1, that is (x & p) + (x >> 61) for the 64-bit x: at most p + 7; for two
-// hashes and one (a, b).  x = h.lo * a.lo + b is one 64-bit multiply-add; the two cross products, of which only the low
-// dwords count, are two more, chained (h.lo * a.hi, then h.hi * a.lo added to it), and their sum goes to the high dword
-// of x with a plain 32-bit add, which issues in half the cycles of a multiply or of a three-operand add (left to itself
-// the compiler makes them two multiplies and a three-operand add).  The fold is a shift and a mask of that dword and
-// one more multiply-add (q * 1 + x) for the carry.  Eight instructions per hash, none that only moves a value.  The
-// chained pairs of the two hashes stand interleaved in one block of assembly, so that neither waits for its own first
-// half; everything else is left to the compiler, which puts an idle cycle between instructions it cannot see into.
-__device__ __forceinline__ void permute_fold_u64_pair(uint64_t h0, uint64_t h1, uint64_t a, uint64_t b, uint32_t one, uint64_t* y0,
-                                                      uint64_t* y1)
-{
-  uint32_t const al = static_cast<uint32_t>(a), ah = static_cast<uint32_t>(a >> 32);
-  uint32_t const l0 = static_cast<uint32_t>(h0), u0 = static_cast<uint32_t>(h0 >> 32);
-  uint32_t const l1 = static_cast<uint32_t>(h1), u1 = static_cast<uint32_t>(h1 >> 32);
-  uint64_t c0, c1;
-  asm("v_mad_u64_u32 %0, vcc, %2, %6, 0\n\t"
-      "v_mad_u64_u32 %1, vcc, %4, %6, 0\n\t"
-      "v_mad_u64_u32 %0, vcc, %3, %7, %0\n\t"
-      "v_mad_u64_u32 %1, vcc, %5, %7, %1"
-      : "=&v"(c0), "=&v"(c1)
-      : "v"(l0), "v"(u0), "v"(l1), "v"(u1), "v"(ah), "v"(al)
-      : "vcc");
-  uint64_t const x0 = static_cast<uint64_t>(l0) * al + b;
-  uint64_t const x1 = static_cast<uint64_t>(l1) * al + b;
-  uint32_t xh0      = static_cast<uint32_t>(x0 >> 32) + static_cast<uint32_t>(c0);
-  uint32_t xh1      = static_cast<uint32_t>(x1 >> 32) + static_cast<uint32_t>(c1);
-  uint32_t const q0 = xh0 >> 29, q1 = xh1 >> 29;
-  xh0 &= 0x1FFFFFFFu;
-  xh1 &= 0x1FFFFFFFu;
-  *y0 = static_cast<uint64_t>(q0) * one + ((static_cast<uint64_t>(xh0) << 32) | static_cast<uint32_t>(x0));
-  *y1 = static_cast<uint64_t>(q1) * one + ((static_cast<uint64_t>(xh1) << 32) | static_cast<uint32_t>(x1));
-}
-
-// min of two values below 2^62 in one instruction: such bit patterns are non-negative finite doubles
-// (or denormals, which this code object keeps: float_denorm_mode_16_64 = 3), and those order like the
-// integers.  An operand that is all ones (the "no hash yet" start value, a NaN pattern) loses to the other.
-__device__ __forceinline__ uint64_t min_below_2_62(uint64_t m, uint64_t y)
-{
-  uint64_t r;
-  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(m), "v"(y));
-  return r;
-}
-
-// Folds the compacted hashes first, first + 1, .. of every `stride` (the count padded to a multiple of the stride)
-// into m[K]; lanes <-> parameters.  A wavefront whose lanes all hold different parameters folds every hash
-// (first 0, stride = the hashes of one trip); with few parameters the lanes form groups that hold the same
-// parameters and fold every other trip each (see Packing).
-template <typename T, int K>
-struct Fold;
 
 // How the lanes of a wavefront share the work when there are at most 32 parameters: `groups` sets of `ppad` lanes
 // (both powers of two, groups <= 16), lane l holding parameter l % ppad and folding the trips l / ppad,
@@ -138,119 +89,287 @@ __host__ __device__ inline Packing packing_for(int32_t P)
   return Packing{ppad, kWave / ppad};
 }
 
+// Folds the compacted hashes first, first + 1, .. of every `stride` (the count padded to a multiple of the stride)
+// into m[K]; lanes <-> parameters.  A wavefront whose lanes all hold different parameters folds every hash
+// (first 0, stride = the hashes of one trip); with few parameters the lanes form groups that hold the same
+// parameters and fold every other trip each (see Packing).
+constexpr uint32_t kFoldTrip = 4;
 template <int K>
-struct Fold<uint32_t, K> {
-  static constexpr uint32_t kPerTrip = 4;
-  static __device__ __forceinline__ void run(const uint32_t* hashes, uint32_t padded, uint32_t first, uint32_t stride,
-                                             const uint32_t (&a)[K], const uint32_t (&b)[K], uint32_t (&m)[K])
-  {
-    for (uint32_t i = first; i < padded; i += stride) {
-      uint32_t const h0 = hashes[i], h1 = hashes[i + 1], h2 = hashes[i + 2], h3 = hashes[i + 3];
+__device__ __forceinline__ void fold32(const uint32_t* hashes, uint32_t padded, uint32_t first, uint32_t stride, const uint32_t (&a)[K],
+                                       const uint32_t (&b)[K], uint32_t (&m)[K])
+{
+  for (uint32_t i = first; i < padded; i += stride) {
+    uint32_t const h0 = hashes[i], h1 = hashes[i + 1], h2 = hashes[i + 2], h3 = hashes[i + 3];
 #pragma unroll
-      for (int k = 0; k < K; ++k) {
-        // one v_mad_u64_u32 per product, one v_min3_u32 per two products
-        uint32_t const r0 = h0 * a[k] + b[k];
-        uint32_t const r1 = h1 * a[k] + b[k];
-        uint32_t const r2 = h2 * a[k] + b[k];
-        uint32_t const r3 = h3 * a[k] + b[k];
-        m[k]              = min(min(m[k], r0), r1);
-        m[k]              = min(min(m[k], r2), r3);
-      }
+    for (int k = 0; k < K; ++k) {
+      // one v_mad_u64_u32 per product, one v_min3_u32 per two products
+      uint32_t const r0 = h0 * a[k] + b[k];
+      uint32_t const r1 = h1 * a[k] + b[k];
+      uint32_t const r2 = h2 * a[k] + b[k];
+      uint32_t const r3 = h3 * a[k] + b[k];
+      m[k]              = min(min(m[k], r0), r1);
+      m[k]              = min(min(m[k], r2), r3);
     }
   }
-};
+}
 
-template <int K>
-struct Fold<uint64_t, K> {
-  static constexpr uint64_t p = (1ull << 61) - 1;
-  // x mod p for x < 2^64: x = q*2^61 + r with q <= 7, so y = r + q <= p + 7.
-  static __device__ __forceinline__ uint64_t fold_once(uint64_t x) { return (x & p) + (x >> 61); }
-
-  // hashes per trip: four (with two, and two and more sets of parameters, the loop issued 3 to 5 % less: fewer
-  // independent products between a trip's LDS read and its dependent minima)
-  static constexpr uint32_t kPerTrip = 4;
-  static __device__ __forceinline__ void run(const uint64_t* hashes, uint32_t padded, uint32_t first, uint32_t stride,
-                                             const uint64_t (&a)[K], const uint64_t (&b)[K], uint64_t (&m)[K])
-  {
-    // Fast pass: the final "subtract p if y >= p" is left out.  y >= p needs the top dword of y to be
-    // at least 0x1FFFFFFF (one chance in 2^29 per product), which is tracked with a running maximum;
-    // if it ever happens the tile is folded again exactly.  Unreduced values are >= p, above every
-    // reduced value, so they can never displace a correct minimum.
-    uint32_t top = 0;
-    uint32_t one;  // the number 1 where the compiler does not see it: q * one + x stays one multiply-add
-    asm("s_mov_b32 %0, 1" : "=s"(one));
-    for (uint32_t i = first; i < padded; i += stride) {
-      uint64_t h[kPerTrip];
-#pragma unroll
-      for (uint32_t j = 0; j < kPerTrip; ++j) h[j] = hashes[i + j];
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-#pragma unroll
-        for (uint32_t j = 0; j < kPerTrip; j += 2) {
-          uint64_t y0, y1;
-          permute_fold_u64_pair(h[j], h[j + 1], a[k], b[k], one, &y0, &y1);
-          top               = max(max(top, static_cast<uint32_t>(y0 >> 32)), static_cast<uint32_t>(y1 >> 32));
-          m[k]              = min_below_2_62(min_below_2_62(m[k], y0), y1);
-        }
-      }
-    }
-    if (ballot64(top >= 0x1FFFFFFFu) != 0) {
-      // every lane folds every hash here: a minimum does not mind the hashes of the other sets
-      for (uint32_t i = 0; i < padded; ++i) {
-        uint64_t const h = hashes[i];
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-          uint64_t const y = fold_once(h * a[k] + b[k]);
-          m[k]             = min(m[k], y >= p ? y - p : y);
-        }
-      }
-    }
-  }
-};
-
-// The parameters beyond the last full set of 64, when there are at most 32 of them: one more (a, b) pair per lane,
-// shared out over sets of lanes as Packing describes, so that they cost the fold a share of a full set (4 parameters
-// beyond 256: a sixteenth) instead of a whole one.
+// What the kernels are given of the parameters.
 template <typename T>
-struct TailParams {
-  T a[1], b[1], m[1];
-  Packing pk;
+struct Params {
+  const T* a;
+  const T* b;
+  int32_t count;
+  const filter64::Group* groups;  // 64-bit hashes only: the same, laid out for the matrix cores
 };
-struct NoTail {};
 
-template <typename T, int K, typename Tail = NoTail>
-__device__ __forceinline__ void fold_hashes(T* hashes, uint32_t count, const T (&a)[K], const T (&b)[K], T (&m)[K], int lane, Packing pk, Tail& tail)
-{
-  constexpr bool kHasTail = !std::is_same<Tail, NoTail>::value;
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  if (count == 0) return;
-  // a duplicate never changes a minimum
-  uint32_t stride = K > 1 ? Fold<T, K>::kPerTrip : pk.stride(Fold<T, K>::kPerTrip);  // a power of two, at most 64
-  if constexpr (kHasTail) stride = max(stride, tail.pk.stride(Fold<T, 1>::kPerTrip));
-  uint32_t const padded = (count + stride - 1u) & ~(stride - 1u);
-  if (lane < static_cast<int>(padded - count)) hashes[count + lane] = hashes[0];
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  // the usual case keeps the loop counter out of the vector registers
-  if (K > 1 || pk.groups == 1)
-    Fold<T, K>::run(hashes, padded, 0u, Fold<T, K>::kPerTrip, a, b, m);
-  else
-    Fold<T, K>::run(hashes, padded, pk.first(lane, Fold<T, K>::kPerTrip), pk.stride(Fold<T, K>::kPerTrip), a, b, m);
-  if constexpr (kHasTail)
-    Fold<T, 1>::run(hashes, padded, tail.pk.first(lane, Fold<T, 1>::kPerTrip), tail.pk.stride(Fold<T, 1>::kPerTrip), tail.a, tail.b, tail.m);
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-template <typename T, int K>
-__device__ __forceinline__ void fold_hashes(T* hashes, uint32_t count, const T (&a)[K], const T (&b)[K], T (&m)[K], int lane,
-                                            Packing pk = Packing{kWave, 1})
-{
-  NoTail none;
-  fold_hashes<T, K, NoTail>(hashes, count, a, b, m, lane, pk, none);
-}
+// The minima of a row (or of a part of one) over the parameters of a chunk, by one wavefront: load() the chunk, reset(),
+// fold() hashes out of LDS as often as needed, finish(), each(put) calls put(j, minimum) for the parameters.
+
+// uint32: K sets of 64 parameters, a lane has one of each set; with TAIL the parameters beyond the last full set, when
+// there are at most 32 of them, are one more (a, b) pair per lane, shared out over sets of lanes as Packing describes, so
+// that they cost the fold a share of a full set (4 parameters beyond 256: a sixteenth) instead of a whole one.
+template <int K, bool TAIL>
+struct Minima32 {
+  using T = uint32_t;
+  struct Lds {};
+  static constexpr int kParams = K * kWave;                       // of a chunk
+  static constexpr int kSlots  = (K + (TAIL ? 1 : 0)) * kWave;    // (with TAIL there is one chunk)
+  static constexpr int kSimdWaves = 7;                             // wavefronts per SIMD that the registers are held to
+  T a[K], b[K], m[K];
+  T tail_a[1], tail_b[1], tail_m[1];
+  Packing pk, tail_pk;
+  int lane;
+
+  __device__ __forceinline__ Minima32(Lds*, int lane_) : lane(lane_) {}
+  __device__ __forceinline__ void load(Params<T> const& p, int32_t chunk)
+  {
+    pk = K == 1 ? packing_for(p.count) : Packing{kWave, 1};
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      int32_t const j = chunk * kParams + pk.param_lane(lane) + kWave * k;
+      a[k]            = j < p.count ? p.a[j] : T{0};
+      b[k]            = j < p.count ? p.b[j] : T{0};
+    }
+    if (TAIL) {
+      tail_pk         = packing_for(p.count - kParams);
+      int32_t const j = kParams + tail_pk.param_lane(lane);
+      tail_a[0]       = j < p.count ? p.a[j] : T{0};
+      tail_b[0]       = j < p.count ? p.b[j] : T{0};
+    }
+  }
+  __device__ __forceinline__ void reset()
+  {
+#pragma unroll
+    for (int k = 0; k < K; ++k) m[k] = std::numeric_limits<T>::max();
+    tail_m[0] = std::numeric_limits<T>::max();
+  }
+  // hashes: `count` of them, and room for 63 more
+  __device__ __forceinline__ void fold(T* hashes, uint32_t count)
+  {
+    wave_lds_fence();
+    if (count == 0) return;
+    // a duplicate never changes a minimum
+    uint32_t stride = K > 1 ? kFoldTrip : pk.stride(kFoldTrip);  // a power of two, at most 64
+    if (TAIL) stride = max(stride, tail_pk.stride(kFoldTrip));
+    uint32_t const padded = (count + stride - 1u) & ~(stride - 1u);
+    if (lane < static_cast<int>(padded - count)) hashes[count + lane] = hashes[0];
+    wave_lds_fence();
+    // the usual case keeps the loop counter out of the vector registers
+    if (K > 1 || pk.groups == 1)
+      fold32<K>(hashes, padded, 0u, kFoldTrip, a, b, m);
+    else
+      fold32<K>(hashes, padded, pk.first(lane, kFoldTrip), pk.stride(kFoldTrip), a, b, m);
+    if (TAIL) fold32<1>(hashes, padded, tail_pk.first(lane, kFoldTrip), tail_pk.stride(kFoldTrip), tail_a, tail_b, tail_m);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  __device__ __forceinline__ void finish()
+  {
+    if (K == 1) m[0] = pk.combine(m[0]);
+    if (TAIL) tail_m[0] = tail_pk.combine(tail_m[0]);  // every set of lanes then holds the minima
+  }
+  template <typename Put>
+  __device__ __forceinline__ void each(Put const& put) const
+  {
+    // (with fewer than 64 parameters the first lanes hold one each, in order)
+#pragma unroll
+    for (int k = 0; k < K; ++k) put(lane + kWave * k, m[k]);
+    if (TAIL) put(kParams + lane, tail_m[0]);
+  }
+};
+
+// uint64: G groups of 32 parameters, each product to 17 bits by the matrix cores (see filter64.cuh), 32 hashes at a time.
+// A lane has a parameter of every group and half of the hashes.  Of the hashes that lie in LDS (`fold`) it finds the
+// least fraction, whose hash it is, and the second least: two matrix instructions, 16 shifts that put the fractions in
+// order with a number below them and 23 minima, medians and maxima for 1,024 products, without a branch.  Per row and
+// group it keeps the least fraction so far and its hash (`best`, `best_hash`: not computed exactly until it has to be)
+// and the largest fraction that can still belong to the minimum (`limit`).  A fraction that is less than the best by
+// more than the slack takes its place; of two within the slack of each other one is computed exactly, and so is one
+// below the slack, which may have come round from the top; where the second least is not above the limit either, all of
+// the lane's hashes are (one parameter in fifty of 256 hashes).
+template <int G>
+struct Minima64 {
+  using T = uint64_t;
+  static constexpr int kParams    = G * filter64::kGroup;
+  static constexpr int kSlots     = kParams;
+  static constexpr int kSimdWaves = G <= 2 ? 4 : 3;  // (four with three groups and more: registers are spilled)
+  struct Lds {
+    unsigned long long exact[kParams];  // the least value computed exactly, of every parameter
+    T hash[2 * kWave];                  // what is waiting to be computed exactly: the hash
+    uint8_t param[2 * kWave];           // and the parameter
+  };
+  uint32_t pieces[G][2][6];
+  uint32_t slack[G], limit[G], best[G];
+  T best_hash[G];
+  int scale[2];
+  uint32_t waiting;
+  Params<T> params;
+  int32_t base;  // first parameter of the chunk
+  Lds* lds;
+  int lane;
+
+  __device__ __forceinline__ Minima64(Lds* lds_, int lane_) : lds(lds_), lane(lane_)
+  {
+    scale[0] = filter64::scale_of(0, lane);
+    scale[1] = filter64::scale_of(1, lane);
+  }
+  __device__ __forceinline__ void load(Params<T> const& p, int32_t chunk)
+  {
+    params             = p;
+    base               = chunk * kParams;
+    int32_t const last = (p.count - 1) / filter64::kGroup;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      filter64::Group const& from = p.groups[min(chunk * G + g, last)];
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int d = 0; d < 6; ++d) pieces[g][k][d] = from.pieces[k][d][lane];
+      slack[g] = from.slack[lane % filter64::kGroup] << filter64::kKeyShift;
+    }
+  }
+  __device__ __forceinline__ void reset()
+  {
+    waiting = 0;
+#pragma unroll
+    for (int g = 0; g < G; ++g) limit[g] = best[g] = filter64::kNoKey;
+    for (int j = lane; j < kParams; j += kWave) lds->exact[j] = ~0ull;
+  }
+
+  __device__ __forceinline__ void compute(int at, T h)
+  {
+    int32_t const j            = min(base + at, params.count - 1);
+    unsigned long long const v = filter64::exact(h, params.a[j], params.b[j]);
+    if (v < lds->exact[at]) atomicMin(&lds->exact[at], v);
+  }
+  // Computes the first 64 of those waiting, or all of them.
+  __device__ __forceinline__ void compute_waiting()
+  {
+    wave_lds_fence();
+    if (static_cast<uint32_t>(lane) < waiting) compute(lds->param[lane], lds->hash[lane]);
+    if (waiting > kWave) {
+      T const h       = lds->hash[kWave + lane];
+      uint8_t const j = lds->param[kWave + lane];
+      wave_lds_fence();
+      lds->hash[lane]  = h;
+      lds->param[lane] = j;
+      waiting -= kWave;
+    } else {
+      waiting = 0;
+    }
+  }
+  __device__ __forceinline__ void wait(bool yes, int g, T h)
+  {
+    uint64_t const who = ballot64(yes);
+    if (who == 0) return;
+    if (yes) {
+      uint32_t const at = waiting + lanes_below(who);
+      lds->hash[at]     = h;
+      lds->param[at]    = static_cast<uint8_t>(g * filter64::kGroup + lane % filter64::kGroup);
+    }
+    waiting += static_cast<uint32_t>(__builtin_popcountll(who));
+    if (waiting >= kWave) compute_waiting();
+  }
+
+  // The least and the second least key of a group's products with the hashes: what becomes of them.
+  __device__ __forceinline__ void settle(int g, uint32_t least, uint32_t second, const T* hashes, uint32_t count)
+  {
+    bool const certain = least >= slack[g];
+    if (certain) limit[g] = min(limit[g], add_saturating(filter64::key_ceiling(least), slack[g]));
+    limit[g]      = min_of_halves(limit[g]);
+    bool const in = least <= limit[g];
+    if (ballot64(in) == 0) return;
+    T const h         = hashes[(least >> 4 & 0x7FFu) * 32u + filter64::hash_of_sum(least & 15u, lane)];
+    bool const better = certain && least < best[g];
+    bool const near   = best[g] != filter64::kNoKey && add_saturating(least, slack[g]) >= best[g] && h != best_hash[g];
+    wait(in && (!certain || near), g, certain && better ? best_hash[g] : h);
+    if (in && better) {
+      best[g]      = least;
+      best_hash[g] = h;
+    }
+    for (uint64_t todo = ballot64(second <= limit[g]); todo != 0; todo &= todo - 1) {
+      int const who    = static_cast<int>(__builtin_ctzll(todo));
+      uint32_t const n = (count + 31u) / 32u * 16u;  // hashes that the lane has
+      int at           = g * filter64::kGroup + who % filter64::kGroup;
+      asm("" : "+v"(at));  // (an address that the compiler knows to be the same in every lane: it builds a loop over the lanes)
+      for (uint32_t i = lane; i < n; i += kWave) compute(at, hashes[(i >> 4) * 32u + filter64::hash_of_sum(i & 15u, who)]);
+    }
+  }
+
+  // hashes: `count` of them (at most 2^11 blocks of 32), and room up to the next multiple of 32
+  __device__ __forceinline__ void fold(T* hashes, uint32_t count)
+  {
+    wave_lds_fence();
+    if (count == 0) return;
+    // the last block is filled up with different ones: with equal ones a least fraction would be the second least too
+    uint32_t const rest = (0u - count) & 31u;
+    if (static_cast<uint32_t>(lane) < rest) hashes[count + lane] = hashes[count > 32u ? static_cast<uint32_t>(lane) : static_cast<uint32_t>(lane) % count];
+    wave_lds_fence();
+    filter64::Sums start;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) start[r] = 6.0f;
+    asm("" : "+v"(start));  // (one set of registers, not one filled anew for every block)
+    uint32_t least[G], second[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) least[g] = second[g] = filter64::kNoKey;
+    for (uint32_t block = 0; block < count; block += 32u) {
+      filter64::V8 const digits = filter64::digits_of(hashes[block + static_cast<uint32_t>(lane % 32)]);
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        filter64::Sums const sums = filter64::sums_of(digits, pieces[g][0], pieces[g][1], scale[0], scale[1], start);
+        uint32_t key[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) key[r] = (__float_as_uint(sums[r]) << filter64::kKeyShift) | static_cast<uint32_t>(r);
+        uint32_t one = min(key[0], key[1]), two = max(key[0], key[1]);
+#pragma unroll
+        for (int r = 2; r < 16; r += 2) {
+          two = min(two, median(one, key[r], key[r + 1]));
+          one = min(min(one, key[r]), key[r + 1]);
+        }
+        one |= block >> 1;  // (16 times the number of the block)
+        second[g] = min(min(second[g], two), max(least[g], one));
+        least[g]  = min(least[g], one);
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) settle(g, least[g], second[g], hashes, count);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  __device__ __forceinline__ void finish()
+  {
+#pragma unroll
+    for (int g = 0; g < G; ++g) wait(best[g] <= limit[g] && best[g] != filter64::kNoKey, g, best_hash[g]);
+    if (waiting > 0) compute_waiting();
+    wave_lds_fence();
+  }
+  template <typename Put>
+  __device__ __forceinline__ void each(Put const& put) const
+  {
+    for (int j = lane; j < kParams; j += kWave) put(j, static_cast<T>(lds->exact[j]));
+    __builtin_amdgcn_wave_barrier();
+  }
+};
 
 // Whether the wavefront has met this hash lately (it is noted either way).  Called by the lanes that have a hash.
 template <typename T>
@@ -268,10 +387,10 @@ __device__ __forceinline__ void forget_hashes(WaveLds<T>& lds, int lane)
 }
 
 // Processes the window starts [s_begin, s_end) of one row with one wavefront and folds the
-// permuted hashes into m[K].  Lane l owns parameters chunk_base + l + 64*k.
-template <typename T, int K, typename Tail>
+// permuted hashes into the minima.
+template <typename Minima, typename T>
 __device__ __forceinline__ void process_section(const uint8_t* row, int64_t n, int64_t s_begin, int64_t s_end, T seed, int32_t width,
-                                                const T (&a)[K], const T (&b)[K], T (&m)[K], WaveLds<T>& lds, int lane, Packing pk, Tail& tail)
+                                                Minima& minima, WaveLds<T>& lds, int lane)
 {
   using H = HashTraits<T>;
   if (static_cast<int64_t>(width) * 4 <= kHalo) {
@@ -292,7 +411,7 @@ __device__ __forceinline__ void process_section(const uint8_t* row, int64_t n, i
           count += static_cast<uint32_t>(__builtin_popcountll(vm));
         }
       });
-      fold_hashes<T, K, Tail>(lds.hashes, count, a, b, m, lane, pk, tail);
+      minima.fold(lds.hashes, count);
     }
   } else {
     // very wide windows: 64 starts at a time, bytes read straight from global memory
@@ -313,20 +432,8 @@ __device__ __forceinline__ void process_section(const uint8_t* row, int64_t n, i
       }
       uint64_t const vm = ballot64(valid);
       if (valid) lds.hashes[lanes_below(vm)] = hv;
-      fold_hashes<T, K, Tail>(lds.hashes, static_cast<uint32_t>(__builtin_popcountll(vm)), a, b, m, lane, pk, tail);
+      minima.fold(lds.hashes, static_cast<uint32_t>(__builtin_popcountll(vm)));
     }
-  }
-}
-
-template <typename T, int K>
-__device__ __forceinline__ void load_params(const T* pa, const T* pb, int32_t P, int32_t chunk_base, int lane, T (&a)[K], T (&b)[K], T (&m)[K])
-{
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    int32_t const j = chunk_base + lane + kWave * k;
-    a[k]            = j < P ? pa[j] : T{0};
-    b[k]            = j < P ? pb[j] : T{0};
-    m[k]            = std::numeric_limits<T>::max();
   }
 }
 
@@ -379,46 +486,16 @@ struct RowParts {
   }
 };
 
-// The tail of a launch with TAIL: the P - 64 K parameters (1..32) beyond the K full sets of the one chunk.
-template <typename T, int K, bool TAIL>
-struct TailOf {
-  using type = NoTail;
-  static __device__ __forceinline__ void load(type&, const T*, const T*, int32_t, int) {}
-  static __device__ __forceinline__ void reset(type&) {}
-  static __device__ __forceinline__ void finish(type&) {}
-  static __device__ __forceinline__ T value(type const&) { return T{0}; }
-};
-template <typename T, int K>
-struct TailOf<T, K, true> {
-  using type = TailParams<T>;
-  static __device__ __forceinline__ void load(type& t, const T* pa, const T* pb, int32_t P, int lane)
-  {
-    t.pk            = packing_for(P - K * kWave);
-    int32_t const j = K * kWave + t.pk.param_lane(lane);
-    t.a[0]          = j < P ? pa[j] : T{0};
-    t.b[0]          = j < P ? pb[j] : T{0};
-    t.m[0]          = std::numeric_limits<T>::max();
-  }
-  static __device__ __forceinline__ void reset(type& t) { t.m[0] = std::numeric_limits<T>::max(); }
-  static __device__ __forceinline__ void finish(type& t) { t.m[0] = t.pk.combine(t.m[0]); }  // every set of lanes then holds the minima
-  static __device__ __forceinline__ T value(type const& t) { return t.m[0]; }
-};
-
-// Wavefronts per SIMD that the registers are held to.
-template <typename T>
-constexpr int minhash_waves() { return sizeof(T) == 4 ? 7 : 4; }
-
 // One workgroup per (group of consecutive rows, parameter chunk): its wavefronts take the group's rows of up to kPartBytes
 // bytes one at a time from a counter in LDS, so that the four are done together whatever the rows' lengths; the minima
 // go from the registers to the result.  The groups lie along x and, beyond kMaxRowBlocks of them, along z.
-template <typename T, int K, bool TAIL>
-__global__ void __launch_bounds__(kThreads, minhash_waves<T>()) minhash_rows_kernel(ColView col, T seed, const T* __restrict__ pa, const T* __restrict__ pb,
-                                                                int32_t P, int32_t width, const int32_t* __restrict__ out_offsets, T* __restrict__ out,
-                                                                int per_wave)
+template <typename Minima, typename T = typename Minima::T>
+__global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_rows_kernel(ColView col, T seed, Params<T> params, int32_t width,
+                                                                                   const int32_t* __restrict__ out_offsets, T* __restrict__ out,
+                                                                                   int per_wave)
 {
-  using TailT = TailOf<T, K, TAIL>;
-  constexpr int kSets = K + (TAIL ? 1 : 0);
   __shared__ WaveLds<T> lds[kWaves];
+  __shared__ typename Minima::Lds minima_lds[kWaves];
   __shared__ uint32_t next_row;
 
   int const group_rows = per_wave * kWaves;
@@ -426,13 +503,10 @@ __global__ void __launch_bounds__(kThreads, minhash_waves<T>()) minhash_rows_ker
   if (r0 >= col.size) return;
   int const lane           = lane_id();
   int const wave           = threadIdx.x / kWave;
-  int32_t const chunk_base = blockIdx.y * (K * kWave);  // (with TAIL there is one chunk)
-  int32_t const in_chunk   = min(kSets * kWave, P - chunk_base);
-  Packing const pk         = K == 1 ? packing_for(P) : Packing{kWave, 1};
-  T a[K], b[K], m[K];
-  load_params<T, K>(pa, pb, P, chunk_base, pk.param_lane(lane), a, b, m);
-  typename TailT::type tail;
-  TailT::load(tail, pa, pb, P, lane);
+  int32_t const chunk_base = blockIdx.y * Minima::kParams;
+  int32_t const in_chunk   = min(Minima::kSlots, params.count - chunk_base);
+  Minima minima(&minima_lds[wave], lane);
+  minima.load(params, blockIdx.y);
 
   int const rows_here = static_cast<int>(min(static_cast<int64_t>(group_rows), col.size - r0));
   if (threadIdx.x == 0) next_row = 0;
@@ -446,20 +520,13 @@ __global__ void __launch_bounds__(kThreads, minhash_waves<T>()) minhash_rows_ker
     int64_t const o = col.off(r0 + i);
     int64_t const n = col.off(r0 + i + 1) - o;
     if (n > kPartBytes) continue;
-#pragma unroll
-    for (int k = 0; k < K; ++k) m[k] = std::numeric_limits<T>::max();
-    TailT::reset(tail);
-    if (n > 0) process_section<T, K>(col.chars + o, n, 0, n, seed, width, a, b, m, lds[wave], lane, pk, tail);
-    if (K == 1) m[0] = pk.combine(m[0]);
-    TailT::finish(tail);
+    minima.reset();
+    if (n > 0) process_section(col.chars + o, n, 0, n, seed, width, minima, lds[wave], lane);
+    minima.finish();
     T* const dst = out + static_cast<int64_t>(out_offsets[r0 + i]) + chunk_base;
-    // an empty row is zeros (minhash.cu:318)
-#pragma unroll
-    for (int k = 0; k < K; ++k) {
-      int32_t const j = lane + kWave * k;  // (with fewer than 64 parameters the first lanes hold one each, in order)
-      if (j < in_chunk) dst[j] = n > 0 ? m[k] : T{0};
-    }
-    if (TAIL && K * kWave + lane < in_chunk) dst[K * kWave + lane] = n > 0 ? TailT::value(tail) : T{0};
+    minima.each([&](int32_t j, T v) {
+      if (j < in_chunk) dst[j] = n > 0 ? v : T{0};  // an empty row is zeros (minhash.cu:318)
+    });
   }
 }
 
@@ -468,15 +535,14 @@ __global__ void __launch_bounds__(kThreads, minhash_waves<T>()) minhash_rows_ker
 // than eight parts for every wavefront they are handed out by a counter, else by place (a counter answers about 150 M
 // requests a second: seven thousand wavefronts asking at once would wait 50 us).  The chunks of parameters come one
 // after the other in the same count.
-template <typename T, int K, bool TAIL>
-__global__ void __launch_bounds__(kThreads, minhash_waves<T>()) minhash_parts_kernel(RowParts parts, T seed, const T* __restrict__ pa, const T* __restrict__ pb,
-                                                                int32_t P, int32_t width, int32_t chunks, const int32_t* __restrict__ out_offsets,
-                                                                const uint32_t* __restrict__ prefix, unsigned long long* __restrict__ counter,
-                                                                T* __restrict__ out)
+template <typename Minima, typename T = typename Minima::T>
+__global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_parts_kernel(RowParts parts, T seed, Params<T> params, int32_t width,
+                                                                                    int32_t chunks, const int32_t* __restrict__ out_offsets,
+                                                                                    const uint32_t* __restrict__ prefix,
+                                                                                    unsigned long long* __restrict__ counter, T* __restrict__ out)
 {
-  using TailT = TailOf<T, K, TAIL>;
-  constexpr int kSets = K + (TAIL ? 1 : 0);
   __shared__ WaveLds<T> lds[kWaves];
+  __shared__ typename Minima::Lds minima_lds[kWaves];
   ColView const& col    = parts.col;
   uint32_t const total  = prefix[col.size];
   uint64_t const tasks  = static_cast<uint64_t>(total) * static_cast<uint32_t>(chunks);
@@ -484,21 +550,18 @@ __global__ void __launch_bounds__(kThreads, minhash_waves<T>()) minhash_parts_ke
   int const lane        = lane_id();
   int const wave        = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
   uint64_t const nwaves = static_cast<uint64_t>(gridDim.x) * kWaves;
-  Packing const pk      = K == 1 ? packing_for(P) : Packing{kWave, 1};
-  T a[K], b[K], m[K];
-  typename TailT::type tail;
-  uint32_t chunk = 0;
-  load_params<T, K>(pa, pb, P, 0, pk.param_lane(lane), a, b, m);
-  TailT::load(tail, pa, pb, P, lane);
+  uint32_t chunk        = 0;
+  Minima minima(&minima_lds[wave], lane);
+  minima.load(params, 0);
   for (uint64_t task = static_cast<uint64_t>(blockIdx.x) * kWaves + wave; task < tasks;) {
     uint32_t const t = static_cast<uint32_t>(task - static_cast<uint64_t>(chunk) * total);
     if (t >= total) {  // the next chunk of parameters
       ++chunk;
-      load_params<T, K>(pa, pb, P, static_cast<int32_t>(chunk) * (K * kWave), pk.param_lane(lane), a, b, m);
+      minima.load(params, static_cast<int32_t>(chunk));
       continue;
     }
-    int32_t const chunk_base = static_cast<int32_t>(chunk) * (K * kWave);
-    int32_t const in_chunk   = min(kSets * kWave, P - chunk_base);
+    int32_t const chunk_base = static_cast<int32_t>(chunk) * Minima::kParams;
+    int32_t const in_chunk   = min(Minima::kSlots, params.count - chunk_base);
     // the last row r with prefix[r] <= t, 64 of them looked at in one step
     int64_t r = 0, end = col.size;
     while (end - r > 1) {
@@ -513,23 +576,17 @@ __global__ void __launch_bounds__(kThreads, minhash_waves<T>()) minhash_parts_ke
     int64_t const sb  = static_cast<int64_t>(t - prefix[r]) * bytes;
     int64_t const se  = min(n, sb + bytes);
     bool const shared = n > bytes;
-#pragma unroll
-    for (int k = 0; k < K; ++k) m[k] = std::numeric_limits<T>::max();
-    TailT::reset(tail);
-    if (sb < se) process_section<T, K>(col.chars + o, n, sb, se, seed, width, a, b, m, lds[wave], lane, pk, tail);
-    if (K == 1) m[0] = pk.combine(m[0]);
-    TailT::finish(tail);
+    minima.reset();
+    if (sb < se) process_section(col.chars + o, n, sb, se, seed, width, minima, lds[wave], lane);
+    minima.finish();
     T* const dst = out + static_cast<int64_t>(out_offsets[r]) + chunk_base;
-    auto const put = [&](int32_t j, T v) {
+    minima.each([&](int32_t j, T v) {
       if (j >= in_chunk) return;
       if (!shared)
         dst[j] = n > 0 ? v : T{0};  // an empty row is zeros (minhash.cu:318)
       else if (v != std::numeric_limits<T>::max())
         atomicMin(&dst[j], v);
-    };
-#pragma unroll
-    for (int k = 0; k < K; ++k) put(lane + kWave * k, m[k]);
-    if (TAIL) put(K * kWave + lane, TailT::value(tail));
+    });
     if (tasks <= 8 * nwaves) {
       task += nwaves;
     } else {
@@ -571,19 +628,34 @@ __global__ void __launch_bounds__(kThreads) minhash_clear_kernel(RowParts parts,
   }
 }
 
+// The parameters of 64-bit hashes, laid out for the matrix cores.
+constexpr int groups_of(int32_t P) { return (P + filter64::kGroup - 1) / filter64::kGroup; }
+__global__ void __launch_bounds__(kWave) minhash64_prepare_kernel(const uint64_t* a, const uint64_t* b, int32_t P, filter64::Group* groups)
+{
+  filter64::prepare_group(a, b, P, static_cast<int32_t>(blockIdx.x), &groups[blockIdx.x], lane_id());
+}
+
 // Everything that comes before the hashing of a column of few rows, in one launch: workgroup 0 counts the parts of the
 // rows (and finds the rows' places in the result where some are null), the others write the places where none is and
-// fill the result.
+// fill the result; the wavefronts of the workgroups from `fillers` + 1 on lay out the parameters of 64-bit hashes.
 constexpr int32_t kPlanRows = kScanSmallTiles * kScanTile;
 template <typename T>
-__global__ void __launch_bounds__(kScanThreads) minhash_plan_kernel(RowParts parts, int32_t P, int32_t* __restrict__ out_offsets,
-                                                                    uint32_t* __restrict__ prefix, unsigned long long* __restrict__ counter,
-                                                                    T* __restrict__ out, int64_t out_size)
+__global__ void __launch_bounds__(kScanThreads) minhash_plan_kernel(RowParts parts, Params<T> params, filter64::Group* groups, unsigned fillers,
+                                                                    int32_t* __restrict__ out_offsets, uint32_t* __restrict__ prefix,
+                                                                    unsigned long long* __restrict__ counter, T* __restrict__ out, int64_t out_size)
 {
   int32_t const rows = parts.col.size;
+  int32_t const P    = params.count;
+  if constexpr (sizeof(T) == 8) {
+    if (blockIdx.x > fillers) {
+      int32_t const group = static_cast<int32_t>((blockIdx.x - fillers - 1) * (kScanThreads / kWave) + threadIdx.x / kWave);
+      if (group < groups_of(P)) filter64::prepare_group(params.a, params.b, P, group, &groups[group], lane_id());
+      return;
+    }
+  }
   if (blockIdx.x > 0) {
     int64_t const first  = static_cast<int64_t>(blockIdx.x - 1) * kScanThreads + threadIdx.x;
-    int64_t const stride = static_cast<int64_t>(gridDim.x - 1) * kScanThreads;
+    int64_t const stride = static_cast<int64_t>(fillers) * kScanThreads;
     if (!parts.col.use_mask)
       for (int64_t i = first; i <= rows; i += stride) out_offsets[i] = static_cast<int32_t>(i * P);
     for (int64_t i = first; i < out_size; i += stride) out[i] = std::numeric_limits<T>::max();
@@ -619,27 +691,25 @@ __global__ void __launch_bounds__(kScanThreads) minhash_plan_kernel(RowParts par
   }
 }
 
-template <typename T, int K, bool TAIL>
-void launch_kernels(RowParts const& parts, T seed, const T* a, const T* b, int32_t P, int32_t width, const int32_t* offsets,
+template <typename Minima, typename T = typename Minima::T>
+void launch_kernels(RowParts const& parts, T seed, Params<T> const& params, int32_t chunks, int32_t width, const int32_t* offsets,
                     const uint32_t* prefix, unsigned long long* counter, T* child, hipStream_t stream)
 {
-  ColView const& v     = parts.col;
-  int32_t const chunks = TAIL ? 1 : (P + K * kWave - 1) / (K * kWave);
+  ColView const& v = parts.col;
   if (v.size >= kManyRows) {
     int const per_wave   = rows_per_wave(v.size);
     int32_t const groups = (v.size + per_wave * kWaves - 1) / (per_wave * kWaves);
     dim3 grid(static_cast<unsigned>(std::min(groups, kMaxRowBlocks)), static_cast<unsigned>(chunks),
               static_cast<unsigned>((groups + kMaxRowBlocks - 1) / kMaxRowBlocks));
     ProfileScope ps("minhash_rows_kernel", stream);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_rows_kernel<T, K, TAIL>), grid, dim3(kThreads), 0, stream, v, seed, a, b, P, width, offsets, child,
-                       per_wave);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_rows_kernel<Minima>), grid, dim3(kThreads), 0, stream, v, seed, params, width, offsets, child, per_wave);
   }
   ProfileScope ps("minhash_parts_kernel", stream);
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_parts_kernel<T, K, TAIL>), dim3(static_cast<unsigned>(parts.waves / kWaves)), dim3(kThreads), 0, stream, parts,
-                     seed, a, b, P, width, chunks, offsets, prefix, counter, child);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_parts_kernel<Minima>), dim3(static_cast<unsigned>(parts.waves / kWaves)), dim3(kThreads), 0, stream, parts,
+                     seed, params, width, chunks, offsets, prefix, counter, child);
 }
 
-// How the parameters are shared out: chunks of K sets of 64 (every chunk hashes the windows again, and a lane without
+// How the parameters of 32-bit hashes are shared out: chunks of K sets of 64 (every chunk hashes the windows again, and a lane without
 // a parameter still folds), or, for 65 to 288 parameters of which at most 32 lie beyond the last full set, one chunk of
 // K full sets and a tail that costs the fold the share `lanes of a tail set / 64` of a set.  Costs in 64ths of a set.
 struct Sharing {
@@ -662,44 +732,77 @@ inline Sharing sharing_for(int32_t P)
   return best;
 }
 
+// Calls launch(which, chunks) for the minima that serve P parameters, which::type, and the chunks of parameters they take.
+template <typename M>
+struct Which {
+  using type = M;
+};
+template <typename T, typename Launch>
+void with_minima(int32_t P, Launch const& launch)
+{
+  if constexpr (sizeof(T) == 8) {
+    // as few chunks as four groups each allow (every chunk hashes the windows again), of equal size
+    int const groups     = groups_of(P);
+    int32_t const chunks = (groups + 3) / 4;
+    switch ((groups + chunks - 1) / chunks) {
+      case 1: launch(Which<Minima64<1>>{}, chunks); break;
+      case 2: launch(Which<Minima64<2>>{}, chunks); break;
+      case 3: launch(Which<Minima64<3>>{}, chunks); break;
+      default: launch(Which<Minima64<4>>{}, chunks); break;
+    }
+  } else {
+    Sharing const sh     = sharing_for(P);
+    int32_t const chunks = sh.tail ? 1 : (P + sh.k * kWave - 1) / (sh.k * kWave);
+    switch (sh.k * 2 + (sh.tail ? 1 : 0)) {
+      case 10: launch(Which<Minima32<5, false>>{}, chunks); break;
+      case 9: launch(Which<Minima32<4, true>>{}, chunks); break;
+      case 8: launch(Which<Minima32<4, false>>{}, chunks); break;
+      case 7: launch(Which<Minima32<3, true>>{}, chunks); break;
+      case 6: launch(Which<Minima32<3, false>>{}, chunks); break;
+      case 5: launch(Which<Minima32<2, true>>{}, chunks); break;
+      case 4: launch(Which<Minima32<2, false>>{}, chunks); break;
+      case 3: launch(Which<Minima32<1, true>>{}, chunks); break;
+      default: launch(Which<Minima32<1, false>>{}, chunks); break;
+    }
+  }
+}
+
 // The launches of one minhash call: the row offsets of the result and the parts of every row, then the hashing kernels.
-// prefix holds rows + 1 values, scan_tmp scan_temp_bytes(rows) bytes and one 64-bit counter behind them.
+// prefix holds rows + 1 values, scan_tmp scan_temp_bytes(rows) bytes and one 64-bit counter behind them; laid_out (64-bit
+// hashes) groups_of(P).
 template <typename T>
 void run_minhash(const ColView& v, T seed, const T* a, const T* b, int32_t P, int32_t width, int32_t* offsets, T* child, int64_t child_size,
-                 uint32_t* prefix, uint64_t* scan_tmp, hipStream_t stream)
+                 uint32_t* prefix, uint64_t* scan_tmp, filter64::Group* laid_out, hipStream_t stream)
 {
   int32_t const rows = v.size;
-  RowParts const parts{v, device_cus() * 4 * minhash_waves<T>(), rows >= kManyRows ? kPartBytes : -1};
+  int simd_waves = 0;
+  with_minima<T>(P, [&](auto which, int32_t) { simd_waves = decltype(which)::type::kSimdWaves; });
+  RowParts const parts{v, device_cus() * 4 * simd_waves, rows >= kManyRows ? kPartBytes : -1};
+  Params<T> const params{a, b, P, laid_out};
   auto* const counter = reinterpret_cast<unsigned long long*>(scan_tmp) + scan_temp_bytes(rows) / sizeof(uint64_t);
   if (rows <= kPlanRows) {
     int64_t const most    = std::max<int64_t>(child_size, rows + 1);
-    unsigned const groups = static_cast<unsigned>(std::min<int64_t>((most + 4 * kScanThreads - 1) / (4 * kScanThreads), 1024));
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_plan_kernel<T>), dim3(1 + groups), dim3(kScanThreads), 0, stream, parts, P, offsets, prefix, counter, child,
-                       child_size);
+    unsigned const fillers = static_cast<unsigned>(std::min<int64_t>((most + 4 * kScanThreads - 1) / (4 * kScanThreads), 1024));
+    unsigned const layers  = sizeof(T) == 8 ? static_cast<unsigned>((groups_of(P) + kScanThreads / kWave - 1) / (kScanThreads / kWave)) : 0u;
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_plan_kernel<T>), dim3(1 + fillers + layers), dim3(kScanThreads), 0, stream, parts, params, laid_out,
+                       fillers, offsets, prefix, counter, child, child_size);
   } else {
     if (v.use_mask) {
       device_exclusive_scan(ValidTimesP{v, P}, static_cast<int64_t>(rows), offsets, scan_tmp, stream);
     } else {
       hipLaunchKernelGGL(uniform_offsets_kernel, dim3((rows + 1 + 255) / 256), dim3(256), 0, stream, offsets, rows, P);
     }
+    if constexpr (sizeof(T) == 8)
+      hipLaunchKernelGGL(minhash64_prepare_kernel, dim3(static_cast<unsigned>(groups_of(P))), dim3(kWave), 0, stream, a, b, P, laid_out);
     device_exclusive_scan(parts, static_cast<int64_t>(rows), prefix, scan_tmp, stream);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_clear_kernel<T>), dim3((rows + kThreads - 1) / kThreads), dim3(kThreads), 0, stream, parts, P, offsets, counter,
                        child);
   }
 
   if (child_size > 0) {
-    Sharing const sh = sharing_for(P);
-    switch (sh.k * 2 + (sh.tail ? 1 : 0)) {
-      case 10: launch_kernels<T, 5, false>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
-      case 9: launch_kernels<T, 4, true>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
-      case 8: launch_kernels<T, 4, false>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
-      case 7: launch_kernels<T, 3, true>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
-      case 6: launch_kernels<T, 3, false>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
-      case 5: launch_kernels<T, 2, true>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
-      case 4: launch_kernels<T, 2, false>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
-      case 3: launch_kernels<T, 1, true>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
-      default: launch_kernels<T, 1, false>(parts, seed, a, b, P, width, offsets, prefix, counter, child, stream); break;
-    }
+    with_minima<T>(P, [&](auto which, int32_t chunks) {
+      launch_kernels<typename decltype(which)::type>(parts, seed, params, chunks, width, offsets, prefix, counter, child, stream);
+    });
   }
 }
 
@@ -755,14 +858,15 @@ nvtext_amd_status minhash_impl(const nvtext_amd_strings_column* input, T seed, c
   }
 
   ColView const v = make_view(*input);
-  size_t const temp_bytes[2] = {scan_temp_bytes(rows) + sizeof(uint64_t), static_cast<size_t>(rows + 1) * sizeof(uint32_t)};
-  TempParts<2> const temp(mr, temp_bytes);
+  size_t const temp_bytes[3] = {scan_temp_bytes(rows) + sizeof(uint64_t), static_cast<size_t>(rows + 1) * sizeof(uint32_t),
+                                sizeof(T) == 8 ? static_cast<size_t>(groups_of(P)) * sizeof(filter64::Group) : 0};
+  TempParts<3> const temp(mr, temp_bytes);
   if (!temp.ok()) {
     nvtext_amd_list_column_free(out, stream_, mr_);
     return fail(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");
   }
   run_minhash<T>(v, seed, a, b, P, width, out->offsets, static_cast<T*>(out->child), out->child_size, temp.part<uint32_t>(1),
-                 temp.part<uint64_t>(0), stream);
+                 temp.part<uint64_t>(0), temp.part<filter64::Group>(2), stream);
   NVTEXT_HIP_TRY_OR(hipGetLastError(), nvtext_amd_list_column_free(out, stream_, mr_));
   return NVTEXT_AMD_SUCCESS;
 }
@@ -821,14 +925,15 @@ constexpr uint32_t kNgramStageWords = (kNgramStageBytes + 16 + 32) / 4;  // + mi
 // (solo_per_wave 0): it needs its workgroups to fill the device and to even out its end (20,000 rows of 3,000 elements:
 // four rows to a workgroup were 8 % slower).
 constexpr int64_t kNgramSoloPositions = 2048;
-template <typename T, int K>
-__global__ void __launch_bounds__(kThreads) minhash_ngrams_kernel(ListView in, int32_t ngrams, T seed, const T* __restrict__ pa,
-                                                                  const T* __restrict__ pb, int32_t P, const int32_t* __restrict__ out_offsets,
-                                                                  T* __restrict__ out, int solo_per_wave)
+template <typename Minima, typename T = typename Minima::T>
+__global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 6 : Minima::kSimdWaves) minhash_ngrams_kernel(ListView in, int32_t ngrams, T seed, Params<T> params,
+                                                                                     const int32_t* __restrict__ out_offsets, T* __restrict__ out,
+                                                                                     int solo_per_wave)
 {
   using H = HashTraits<T>;
   __shared__ alignas(16) T hashes[kWaves][2 * kWave];  // 64 hashes a trip, padded to the stride of the fold (at most 64 more)
-  __shared__ T red[kWaves][K * kWave];
+  __shared__ typename Minima::Lds minima_lds[kWaves];
+  __shared__ T red[kWaves][Minima::kSlots];
   // the chars of the elements a wavefront is hashing (32-bit hash only: measured 13 % faster there, 9 % slower for the
   // 64-bit hash, whose 16-byte steps cost more to assemble out of LDS than they save)
   constexpr bool kStageRuns = sizeof(T) == 4;
@@ -839,12 +944,12 @@ __global__ void __launch_bounds__(kThreads) minhash_ngrams_kernel(ListView in, i
   int64_t const r0     = (static_cast<int64_t>(blockIdx.z) * gridDim.x + blockIdx.x) * group_rows;  // groups along x, then z
   if (r0 >= in.size) return;
   int64_t const solo_positions = solo_per_wave > 0 ? kNgramSoloPositions : -1;
-  int32_t const chunk_base     = blockIdx.y * (K * kWave);
-  int32_t const in_chunk       = min(K * kWave, P - chunk_base);
+  int32_t const chunk_base     = blockIdx.y * Minima::kParams;
+  int32_t const in_chunk       = min(Minima::kSlots, params.count - chunk_base);
   int const lane               = lane_id();
   int const wave               = threadIdx.x / kWave;
-  T a[K], b[K], m[K];
-  load_params<T, K>(pa, pb, P, chunk_base, lane, a, b, m);
+  Minima minima(&minima_lds[wave], lane);
+  minima.load(params, blockIdx.y);
 
   int const rows_here = static_cast<int>(min(static_cast<int64_t>(group_rows), in.size - r0));
   if (threadIdx.x == 0) next_row = 0;
@@ -873,8 +978,7 @@ __global__ void __launch_bounds__(kThreads) minhash_ngrams_kernel(ListView in, i
     // minhash.cu:311-314 with width = ngrams: the positions that the permutation looks at
     int64_t const positions = max(static_cast<int64_t>(1), n - ngrams + 1);
     if (solo != (positions <= solo_positions)) continue;
-#pragma unroll
-    for (int k = 0; k < K; ++k) m[k] = std::numeric_limits<T>::max();
+    minima.reset();
     if (n > 0) {
       int64_t const trip = solo ? kWave : kWaves * kWave;
       for (int64_t base = solo ? 0 : static_cast<int64_t>(wave) * kWave; base < positions; base += trip) {
@@ -916,21 +1020,19 @@ __global__ void __launch_bounds__(kThreads) minhash_ngrams_kernel(ListView in, i
         if (valid) hv = hv < 1 ? T{1} : hv;  // 237
         uint64_t const vm = ballot64(valid);
         if (valid) hashes[wave][lanes_below(vm)] = hv;
-        fold_hashes<T, K>(hashes[wave], static_cast<uint32_t>(__builtin_popcountll(vm)), a, b, m, lane);
+        minima.fold(hashes[wave], static_cast<uint32_t>(__builtin_popcountll(vm)));
       }
     }
+    minima.finish();
     T* const dst = out + static_cast<int64_t>(out_offsets[r0 + i]) + chunk_base;
     if (solo) {
       // an empty row is zeros (minhash.cu:318); a row whose every run was skipped keeps the all-ones start value
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        int32_t const j = lane + kWave * k;
-        if (j < in_chunk) dst[j] = n > 0 ? m[k] : T{0};
-      }
+      minima.each([&](int32_t j, T v) {
+        if (j < in_chunk) dst[j] = n > 0 ? v : T{0};
+      });
     } else {
       __syncthreads();  // (the row before has been read out of red)
-#pragma unroll
-      for (int k = 0; k < K; ++k) red[wave][k * kWave + lane] = m[k];
+      minima.each([&](int32_t j, T v) { red[wave][j] = v; });
       __syncthreads();
       for (int j = threadIdx.x; j < in_chunk; j += kThreads) {
         T v = red[0][j];
@@ -948,18 +1050,17 @@ struct ListValidTimesP {
   __device__ uint64_t operator()(int64_t i) const { return in.valid(i) ? static_cast<uint64_t>(P) : 0; }
 };
 
-template <typename T, int K>
-void launch_ngrams(const ListView& v, int32_t ngrams, T seed, const T* a, const T* b, int32_t P, const int32_t* offsets, T* child,
+template <typename Minima, typename T = typename Minima::T>
+void launch_ngrams(const ListView& v, int32_t ngrams, T seed, Params<T> const& params, int32_t chunks, const int32_t* offsets, T* child,
                    hipStream_t stream)
 {
-  int32_t const chunks    = (P + K * kWave - 1) / (K * kWave);
   int const solo_per_wave = v.size >= kManyRows ? rows_per_wave(v.size) : 0;
   int32_t const group     = solo_per_wave > 0 ? solo_per_wave * kWaves : 1;
   int32_t const groups    = (v.size + group - 1) / group;
   dim3 grid(static_cast<unsigned>(std::min(groups, kMaxRowBlocks)), static_cast<unsigned>(chunks),
             static_cast<unsigned>((groups + kMaxRowBlocks - 1) / kMaxRowBlocks));
   ProfileScope ps("minhash_ngrams_kernel", stream);
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_ngrams_kernel<T, K>), grid, dim3(kThreads), 0, stream, v, ngrams, seed, a, b, P, offsets, child,
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_ngrams_kernel<Minima>), grid, dim3(kThreads), 0, stream, v, ngrams, seed, params, offsets, child,
                      solo_per_wave);
 }
 
@@ -1024,24 +1125,24 @@ nvtext_amd_status minhash_ngrams_impl(const nvtext_amd_list_strings_column* inpu
   v.offset   = input->offset;
   v.use_mask = (input->null_mask != nullptr && input->null_count > 0) ? 1 : 0;
   v.child    = make_view(input->child);
+  size_t const temp_bytes[2] = {v.use_mask ? scan_temp_bytes(rows) : 0, sizeof(T) == 8 ? static_cast<size_t>(groups_of(P)) * sizeof(filter64::Group) : 0};
+  TempParts<2> const temp(mr, temp_bytes, v.use_mask || sizeof(T) == 8);
+  if (!temp.ok()) {
+    nvtext_amd_list_column_free(out, stream_, mr_);
+    return fail(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");
+  }
   if (v.use_mask) {
-    Temp scan_tmp(mr, scan_temp_bytes(rows));
-    if (!scan_tmp.ok()) {
-      nvtext_amd_list_column_free(out, stream_, mr_);
-      return fail(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");
-    }
-    device_exclusive_scan(ListValidTimesP{v, P}, static_cast<int64_t>(rows), out->offsets, scan_tmp.as<uint64_t>(), stream);
+    device_exclusive_scan(ListValidTimesP{v, P}, static_cast<int64_t>(rows), out->offsets, temp.part<uint64_t>(0), stream);
   } else {
     hipLaunchKernelGGL(uniform_offsets_kernel, dim3((rows + 1 + 255) / 256), dim3(256), 0, stream, out->offsets, rows, P);
   }
-  T* child = static_cast<T*>(out->child);
+  auto* const laid_out = temp.part<filter64::Group>(1);
+  if constexpr (sizeof(T) == 8)
+    hipLaunchKernelGGL(minhash64_prepare_kernel, dim3(static_cast<unsigned>(groups_of(P))), dim3(kWave), 0, stream, a, b, P, laid_out);
   if (out->child_size > 0) {
-    if (P > 2 * kWave)
-      launch_ngrams<T, 4>(v, ngrams, seed, a, b, P, out->offsets, child, stream);
-    else if (P > kWave)
-      launch_ngrams<T, 2>(v, ngrams, seed, a, b, P, out->offsets, child, stream);
-    else
-      launch_ngrams<T, 1>(v, ngrams, seed, a, b, P, out->offsets, child, stream);
+    with_minima<T>(P, [&](auto which, int32_t chunks) {
+      launch_ngrams<typename decltype(which)::type>(v, ngrams, seed, Params<T>{a, b, P, laid_out}, chunks, out->offsets, static_cast<T*>(out->child), stream);
+    });
   }
   NVTEXT_HIP_TRY_OR(hipGetLastError(), nvtext_amd_list_column_free(out, stream_, mr_));
   return NVTEXT_AMD_SUCCESS;
@@ -1110,7 +1211,7 @@ nvtext_amd_status nvtext_amd_minhash_preallocated(const nvtext_amd_strings_colum
   if (input->null_mask) launch_copy_bitmask(out_null_mask, input->null_mask, input->offset, rows, stream);
   ColView const v = make_view(*input);
   // every value of the scratch that the kernels read is written earlier in this same call: nothing to clear
-  run_minhash<uint32_t>(v, seed, a, b, P, width, out_offsets, out_child, child_size, prefix, scan_tmp, stream);
+  run_minhash<uint32_t>(v, seed, a, b, P, width, out_offsets, out_child, child_size, prefix, scan_tmp, nullptr, stream);
   NVTEXT_HIP_TRY(hipGetLastError());
   return NVTEXT_AMD_SUCCESS;
 }
