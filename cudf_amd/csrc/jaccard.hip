@@ -152,7 +152,7 @@ struct Part {
 // A wavefront's own LDS for the tile it hashes.
 struct TileLds {
   alignas(16) uint32_t bytes[kTileWords];
-  uint16_t chars[kTile + kHalo];
+  uint16_t chars[kCharList];
   uint32_t later[kTile + kWave / 2];  // hashes that a first look at their bucket did not place
 };
 

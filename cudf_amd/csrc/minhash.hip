@@ -908,7 +908,7 @@ struct AlignedSrc {
   {
     uint32_t const o  = mis + i;
     uint32_t const j  = o >> 2;
-    uint32_t const lo = w[j];
+    uint32_t const lo = 4u * j < end ? w[j] : 0u;
     uint32_t const hi = 4u * (j + 1u) < end ? w[j + 1] : 0u;
     return __builtin_amdgcn_alignbit(hi, lo, (o & 3u) * 8u);
   }

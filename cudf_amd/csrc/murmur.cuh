@@ -30,7 +30,7 @@ __device__ __forceinline__ uint32_t keep_low_bytes(uint32_t v, int nbytes)
 }
 
 // Byte source over a dword array (an LDS tile): window byte i lives at byte offset base+i.
-// u32(i) may read up to 7 bytes past the window (callers mask what they do not need).
+// u32(i) may read up to 11 bytes past the window (callers mask what they do not need).
 struct WordSrc {
   const uint32_t* w;
   uint32_t base;
@@ -110,6 +110,13 @@ __device__ __forceinline__ uint64_t load_u64(Src const& src, uint32_t i)
   return (static_cast<uint64_t>(src.u32(i + 4)) << 32) | src.u32(i);
 }
 
+// The first n bytes (1 .. 8) of v.
+__device__ __forceinline__ uint64_t low_bytes64(uint64_t v, uint32_t n)
+{
+  uint32_t const s = 64u - 8u * n;
+  return (v << s) >> s;
+}
+
 // First 64-bit word of MurmurHash3_x64_128 with h1 = h2 = seed over window bytes [0, len).
 template <typename Src>
 __device__ __forceinline__ uint64_t murmur3_x64_128_lo(Src const& src, uint32_t len, uint64_t seed)
@@ -135,21 +142,17 @@ __device__ __forceinline__ uint64_t murmur3_x64_128_lo(Src const& src, uint32_t 
     h2 += h1;
     h2 = h2 * 5 + 0x38495ab5;
   }
-  int const rem = static_cast<int>(len & 15u);
+  uint32_t const rem = len & 15u;
   if (rem) {
     uint32_t const t = 16 * blocks;
     if (rem > 8) {
-      uint32_t const lo = keep_low_bytes(src.u32(t + 8), rem - 8);
-      uint32_t const hi = rem > 12 ? keep_low_bytes(src.u32(t + 12), rem - 12) : 0u;
-      uint64_t k2       = (static_cast<uint64_t>(hi) << 32) | lo;
+      uint64_t k2 = low_bytes64(load_u64(src, t + 8), rem - 8);
       k2 *= c2;
       k2 = rotl64(k2, 33);
       k2 *= c1;
       h2 ^= k2;
     }
-    uint32_t const lo = keep_low_bytes(src.u32(t), rem);
-    uint32_t const hi = rem > 4 ? keep_low_bytes(src.u32(t + 4), rem - 4) : 0u;
-    uint64_t k1       = (static_cast<uint64_t>(hi) << 32) | lo;
+    uint64_t k1 = low_bytes64(load_u64(src, t), rem < 8 ? rem : 8u);
     k1 *= c1;
     k1 = rotl64(k1, 31);
     k1 *= c2;

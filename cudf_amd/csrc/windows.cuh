@@ -13,6 +13,7 @@ constexpr int kWaves     = 4;                  // wavefronts per workgroup
 constexpr int kThreads   = kWaves * kWave;     // 256
 constexpr int kTile      = 256;                // window starts per wavefront tile
 constexpr int kHalo      = 128;                // bytes staged past the tile (windows up to 32 4-byte chars)
+constexpr int kCharList  = kTile + kHalo + 8;   // list of a tile's characters: one per staged byte, the end of the last one, padding
 constexpr int kTileWords = (kTile + kHalo + 16 + 32) / 4;  // +16 misalignment, +32 for whole blocks and the over-read of the hash tail
 
 // Windows repeat (text repeats its words: a tenth of the windows of a tile, a third within 4 KB of ordinary text), and a
@@ -27,7 +28,7 @@ struct WaveLds {
   alignas(16) uint32_t bytes[kTileWords];
   alignas(16) T hashes[kTile + 4];
   alignas(16) T recent[recent_entries<T>()];
-  uint16_t chars[kTile + kHalo];  // the characters that start in the staged bytes, in order: start | bytes << 9 (see CharMap)
+  uint16_t chars[kCharList];  // where the characters of the staged bytes start, in order (see CharMap)
 };
 
 // Stage row bytes [base, base+len) into dst (16-byte aligned); returns the byte offset of `base` inside it.
@@ -54,53 +55,50 @@ __device__ __forceinline__ uint32_t stage_bytes(const uint8_t* row, int64_t base
 // ASCII.  The reference walks from every window start byte by byte, adding up what each first byte of a character
 // says of its length until `width` characters are counted (cpp/include/cudf/strings/string_view.cuh:67-80).  Where
 // every character of the staged bytes ends exactly where the next one starts, that sum is the distance from the start
-// of character k to the end of character k + width - 1: the characters are listed in LDS (start | bytes << 9, in
-// order), a lane takes a character instead of a byte position, and a window costs two reads of the list.  Other tiles
-// (stray continuation bytes, first bytes that promise more than follows) keep the walk.
-static_assert(kTile + kHalo <= 512, "a character's start takes nine bits of its record");
+// of character k to the start of character k + width: the starts are listed in LDS, in order, and a lane takes a
+// character instead of a byte position, and a window costs two reads of the list.  Other tiles (stray continuation bytes,
+// first bytes that promise more than follows) keep the walk.  Which bytes continue a character and which ought to, by
+// the first bytes before them, are two 64-bit masks in scalar registers, equal where all is well.
 struct CharMap {
-  static __device__ __forceinline__ uint32_t start_of(uint32_t c) { return c & 0x1FFu; }
-  static __device__ __forceinline__ uint32_t end_of(uint32_t c) { return (c & 0x1FFu) + (c >> 9); }
   uint32_t count;    // characters that start in the staged bytes
   uint32_t windows;  // of them, in the tile's window starts (the first `cnt` staged bytes)
   bool exact;        // the list gives every window of the tile its length
-  bool at_row_end;   // the staged bytes reach the end of the row
 
   // staged: the tile's bytes in LDS, its first byte at byte offset `mis`; len of them are the row's, the first cnt are
-  // window starts; chars: the list (room for a character per staged byte).
+  // window starts; chars: the list (kCharList entries).
   __device__ __forceinline__ void build(const uint32_t* staged, uint32_t mis, uint32_t len, uint32_t cnt, bool reaches_row_end, uint16_t* chars,
                                         int lane)
   {
     const uint8_t* const sb = reinterpret_cast<const uint8_t*>(staged) + mis;
-    at_row_end              = reaches_row_end;
     count                   = 0;
     windows                 = 0;
+    uint64_t wrong = 0, carry = 0;         // carry: bytes that the characters of the 64 bytes before expect of these
+    uint32_t last_start = 0, last_end = 0; // of the last character
     for (uint32_t base = 0; base < len; base += kWave) {
       uint32_t const pos   = base + static_cast<uint32_t>(lane);
       uint32_t const b     = pos < len ? sb[pos] : 0x80u;
-      bool const start     = !is_utf8_continuation(b);
-      uint64_t const found = ballot64(start);
-      if (start) chars[count + lanes_below(found)] = static_cast<uint16_t>(pos | (static_cast<uint32_t>(bytes_in_utf8_byte(b)) << 9));
+      uint64_t const here  = len - base >= kWave ? ~0ull : (1ull << (len - base)) - 1ull;
+      uint64_t const found = ballot64(!is_utf8_continuation(b));
+      uint64_t const two = ballot64(b >= 0xC0u), three = ballot64(b >= 0xE0u), four = ballot64(b >= 0xF0u);
+      uint64_t const expected = (two << 1) | (three << 2) | (four << 3) | carry;
+      carry                   = (two >> 63) | (three >> 62) | (four >> 61);
+      // (bytes before the first character of the tile belong to one that began before it)
+      uint64_t const counted = count > 0 ? here : here & ~((found & (0ull - found)) - 1ull);
+      if (count > 0 || found != 0) wrong |= (expected ^ ~found) & counted;
+      if ((found >> lane) & 1u) chars[count + lanes_below(found)] = static_cast<uint16_t>(pos);
       count += static_cast<uint32_t>(__builtin_popcountll(found));
-      if (base < cnt) windows += static_cast<uint32_t>(__builtin_popcountll(ballot64(start && pos < cnt)));
+      if (base < cnt) windows += static_cast<uint32_t>(__builtin_popcountll(found & (cnt - base >= kWave ? ~0ull : (1ull << (cnt - base)) - 1ull)));
+      if (found != 0) {
+        uint32_t const top = 63u - static_cast<uint32_t>(__builtin_clzll(found));
+        last_start         = base + top;
+        last_end           = last_start + 1u + static_cast<uint32_t>((two >> top & 1u) + (three >> top & 1u) + (four >> top & 1u));
+      }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // every character but the first begins where the one before it ends
-    bool broken = false;
-    for (uint32_t k0 = 0; k0 < count; k0 += kWave) {
-      uint32_t const k = k0 + static_cast<uint32_t>(lane);
-      if (k >= 1 && k < count) broken = broken || end_of(chars[k - 1]) != start_of(chars[k]);
-    }
+    if (lane == 0) chars[count] = static_cast<uint16_t>(last_end);
+    wave_lds_fence();
     // the last one: ends with the row, or, when the row goes on, begins in the last four staged bytes (then every window
     // start of the tile, at least 4 * width bytes before the end of the staged bytes, has its `width` characters listed)
-    bool tail = false;
-    if (count > 0) {
-      uint32_t const last = chars[count - 1];
-      tail                = reaches_row_end ? end_of(last) == len : len - start_of(last) <= 4u;
-    }
-    exact = tail && ballot64(broken) == 0;
+    exact = wrong == 0 && count > 0 && (reaches_row_end ? last_end == len : len - last_start <= 4u);
   }
 
   // The window that begins with character k (k < windows): whether it counts, where it starts and its bytes.
@@ -108,15 +106,12 @@ struct CharMap {
   __device__ __forceinline__ bool window(uint32_t k, uint32_t len, bool row_start, int32_t width, const uint16_t* chars, uint32_t* pos,
                                          uint32_t* hlen) const
   {
-    uint32_t const first = start_of(chars[k]);
+    uint32_t const first = chars[k];
     *pos                 = first;
-    if (k + static_cast<uint32_t>(width) <= count) {
-      *hlen = end_of(chars[k + static_cast<uint32_t>(width) - 1u]) - first;
-      return true;
-    }
     // fewer than `width` characters are left (the staged bytes reach the end of the row): only the row's first position counts
-    *hlen = len - first;
-    return row_start && first == 0;
+    bool const whole = k + static_cast<uint32_t>(width) <= count;
+    *hlen            = (whole ? chars[k + static_cast<uint32_t>(width)] : len) - first;
+    return whole || (row_start && first == 0);
   }
 };
 
