@@ -386,58 +386,204 @@ __device__ __forceinline__ void forget_hashes(WaveLds<T>& lds, int lane)
   for (int i = lane; i < recent_entries<T>(); i += kWave) lds.recent[i] = T{0};
 }
 
-// Processes the window starts [s_begin, s_end) of one row with one wavefront and folds the
-// permuted hashes into the minima.
-template <typename Minima, typename T>
-__device__ __forceinline__ void process_section(const uint8_t* row, int64_t n, int64_t s_begin, int64_t s_end, T seed, int32_t width,
-                                                Minima& minima, WaveLds<T>& lds, int lane)
-{
-  using H = HashTraits<T>;
-  if (static_cast<int64_t>(width) * 4 <= kHalo) {
-    // usual case: a window (<= 4*width bytes) fits the halo staged behind every tile
-    forget_hashes(lds, lane);  // (the wave barrier after the first tile's staging comes before the first look)
-    for (int64_t base = s_begin; base < s_end; base += kTile) {
-      uint32_t const cnt = static_cast<uint32_t>(min(static_cast<int64_t>(kTile), s_end - base));
-      uint32_t count     = 0;  // compacted hashes so far (wave-uniform)
-      auto const hash    = [seed](WordSrc const& src, uint32_t len) {
-        T const hv = H::hash(src, len, seed);
-        return hv < 1 ? T{1} : hv;  // minhash.cu:141
-      };
-      hash_tile_windows<T>(row, n, base, cnt, width, lds.bytes, lds.chars, lane, hash, [&](auto const& valid, auto const& hv) {
-        for (auto const& h : hv) {
-          bool const fresh  = valid[&h - hv] && !seen_lately(lds, h);
-          uint64_t const vm = ballot64(fresh);
-          if (fresh) lds.hashes[count + lanes_below(vm)] = h;
-          count += static_cast<uint32_t>(__builtin_popcountll(vm));
-        }
-      });
-      minima.fold(lds.hashes, count);
-    }
-  } else {
-    // very wide windows: 64 starts at a time, bytes read straight from global memory
-    for (int64_t base = s_begin; base < s_end; base += kWave) {
-      int64_t const gpos = base + lane;
-      bool valid         = false;
-      T hv               = 0;
-      if (gpos < s_end) {
-        int64_t const remaining = n - gpos;
-        BoundedSrc const src{row + gpos, remaining};
-        uint32_t hlen;
-        uint32_t const readable = static_cast<uint32_t>(min(remaining, static_cast<int64_t>(width) * 4));
-        valid = window_at(src, row + gpos, remaining, readable, gpos == 0, false, width, &hlen);
-        if (valid) {
-          hv = H::hash(src, hlen, seed);
-          hv = hv < 1 ? T{1} : hv;
-        }
+// What is hashed: a column of strings, by windows of characters, or a column of lists of strings, by runs of elements.  A
+// row's length is what it is cut by (bytes; positions of runs), and process() folds the hashes of the part [begin, end) of
+// row i into the minima.
+template <typename T_>
+struct TextRows {
+  using T   = T_;
+  using Lds = WaveLds<T>;
+  static constexpr const char* kRowsName  = "minhash_rows_kernel";
+  static constexpr const char* kPartsName = "minhash_parts_kernel";
+  static constexpr int64_t kPart    = 4096;
+  static constexpr int64_t kMinPart = kTile;  // less would be staged for its halo
+  ColView col;
+  T seed;
+  int32_t width;
+
+  __device__ __forceinline__ int32_t rows() const { return col.size; }
+  __device__ __forceinline__ bool masked() const { return col.use_mask; }
+  __device__ __forceinline__ bool valid(int64_t i) const { return col.valid(i); }
+  __device__ __forceinline__ int64_t length(int64_t i) const { return col.off(i + 1) - col.off(i); }
+  __device__ __forceinline__ int64_t total() const { return col.off(col.size) - col.off(0); }
+  template <typename Minima>
+  __device__ __forceinline__ void process(int64_t i, int64_t begin, int64_t end, Minima& minima, Lds& lds, int lane) const
+  {
+    using H              = HashTraits<T>;
+    int64_t const o      = col.off(i);
+    int64_t const n      = col.off(i + 1) - o;
+    const uint8_t* const row = col.chars + o;
+    if (static_cast<int64_t>(width) * 4 <= kHalo) {
+      // usual case: a window (<= 4*width bytes) fits the halo staged behind every tile
+      forget_hashes(lds, lane);  // (the wave barrier after the first tile's staging comes before the first look)
+      for (int64_t base = begin; base < end; base += kTile) {
+        uint32_t const cnt = static_cast<uint32_t>(min(static_cast<int64_t>(kTile), end - base));
+        uint32_t count     = 0;  // compacted hashes so far (wave-uniform)
+        auto const hash    = [seed = seed](WordSrc const& src, uint32_t len) {
+          T const hv = H::hash(src, len, seed);
+          return hv < 1 ? T{1} : hv;  // minhash.cu:141
+        };
+        hash_tile_windows<T>(row, n, base, cnt, width, lds.bytes, lds.chars, lane, hash, [&](auto const& valid, auto const& hv) {
+          for (auto const& h : hv) {
+            bool const fresh  = valid[&h - hv] && !seen_lately(lds, h);
+            uint64_t const vm = ballot64(fresh);
+            if (fresh) lds.hashes[count + lanes_below(vm)] = h;
+            count += static_cast<uint32_t>(__builtin_popcountll(vm));
+          }
+        });
+        minima.fold(lds.hashes, count);
       }
-      uint64_t const vm = ballot64(valid);
-      if (valid) lds.hashes[lanes_below(vm)] = hv;
-      minima.fold(lds.hashes, static_cast<uint32_t>(__builtin_popcountll(vm)));
+    } else {
+      // very wide windows: 64 starts at a time, bytes read straight from global memory
+      for (int64_t base = begin; base < end; base += kWave) {
+        int64_t const gpos = base + lane;
+        bool valid         = false;
+        T hv               = 0;
+        if (gpos < end) {
+          int64_t const remaining = n - gpos;
+          BoundedSrc const src{row + gpos, remaining};
+          uint32_t hlen;
+          uint32_t const readable = static_cast<uint32_t>(min(remaining, static_cast<int64_t>(width) * 4));
+          valid = window_at(src, row + gpos, remaining, readable, gpos == 0, false, width, &hlen);
+          if (valid) {
+            hv = H::hash(src, hlen, seed);
+            hv = hv < 1 ? T{1} : hv;
+          }
+        }
+        uint64_t const vm = ballot64(valid);
+        if (valid) lds.hashes[lanes_below(vm)] = hv;
+        minima.fold(lds.hashes, static_cast<uint32_t>(__builtin_popcountll(vm)));
+      }
     }
   }
-}
+};
 
-// How the rows are shared out.  In a column of at least kManyRows rows a wavefront does the rows of up to kPartBytes
+struct ListView {
+  const int32_t* offsets;  // element index of the first element of row i + offset
+  const uint32_t* mask;
+  int32_t size;
+  int32_t offset;
+  int32_t use_mask;
+  ColView child;           // the elements
+
+  __device__ __forceinline__ int64_t off(int64_t i) const { return offsets[i + offset]; }
+  __device__ __forceinline__ bool valid(int64_t i) const
+  {
+    if (!use_mask) return true;
+    int64_t const b = i + offset;
+    return (mask[b >> 5] >> (b & 31)) & 1u;
+  }
+};
+
+// Byte source over global memory through aligned dword loads that overlap [p, p + len) only.
+struct AlignedSrc {
+  const uint32_t* w;  // aligned address at or below the first byte
+  uint32_t mis;       // first byte inside w[0]
+  uint32_t end;       // mis + len
+  __device__ __forceinline__ AlignedSrc(const uint8_t* p, uint32_t len)
+  {
+    mis = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p) & 3u);
+    w   = reinterpret_cast<const uint32_t*>(p - mis);
+    end = mis + len;
+  }
+  __device__ __forceinline__ uint32_t byte(uint32_t i) const { return reinterpret_cast<const uint8_t*>(w)[mis + i]; }
+  __device__ __forceinline__ uint32_t u32(uint32_t i) const
+  {
+    uint32_t const o  = mis + i;
+    uint32_t const j  = o >> 2;
+    uint32_t const lo = 4u * j < end ? w[j] : 0u;
+    uint32_t const hi = 4u * (j + 1u) < end ? w[j + 1] : 0u;
+    return __builtin_amdgcn_alignbit(hi, lo, (o & 3u) * 8u);
+  }
+};
+
+constexpr uint32_t kRunStageBytes = 4096;                           // longest stretch of chars hashed out of LDS
+constexpr uint32_t kRunStageWords = (kRunStageBytes + 16 + 32) / 4;  // + misalignment, + whole blocks and over-read of the hash tail
+constexpr uint32_t kRunHashes     = 256;                            // hashes folded together
+
+template <typename T>
+struct RunLds {
+  alignas(16) T hashes[kRunHashes + kWave];  // (padded to the stride of the fold, at most 63 more)
+  // the chars of the elements a wavefront is hashing (32-bit hash only: measured 13 % faster there, 9 % slower for the
+  // 64-bit hash, whose 16-byte steps cost more to assemble out of LDS than they save)
+  alignas(16) uint32_t bytes[sizeof(T) == 4 ? kRunStageWords : 4];
+};
+
+// The runs of elements of minhash_ngrams (cpp/src/text/minhash.cu:182-250).  Positions are list elements, 64 a trip; the hashes of up to four trips are folded together.
+template <typename T_>
+struct RunRows {
+  using T   = T_;
+  using Lds = RunLds<T>;
+  static constexpr const char* kRowsName  = "minhash_ngrams_rows_kernel";
+  static constexpr const char* kPartsName = "minhash_ngrams_parts_kernel";
+  static constexpr int64_t kPart    = 1024;
+  static constexpr int64_t kMinPart = kWave;
+  ListView col;
+  T seed;
+  int32_t ngrams;
+
+  __device__ __forceinline__ int32_t rows() const { return col.size; }
+  __device__ __forceinline__ bool masked() const { return col.use_mask; }
+  __device__ __forceinline__ bool valid(int64_t i) const { return col.valid(i); }
+  // minhash.cu:311-314 with width = ngrams: the positions that the permutation looks at
+  __device__ __forceinline__ int64_t length(int64_t i) const
+  {
+    int64_t const n = col.off(i + 1) - col.off(i);
+    return n == 0 ? 0 : max(static_cast<int64_t>(1), n - ngrams + 1);
+  }
+  __device__ __forceinline__ int64_t total() const { return col.off(col.size) - col.off(0); }
+  template <typename Minima>
+  __device__ __forceinline__ void process(int64_t i, int64_t begin, int64_t end, Minima& minima, Lds& lds, int lane) const
+  {
+    using H             = HashTraits<T>;
+    int64_t const first = col.off(i);
+    int64_t const n     = col.off(i + 1) - first;
+    // the bytes from the start of the lane's element to the end of the last element of its run (224-229), clamped to the
+    // row (218-222); asked for a trip ahead
+    int64_t bo, eo;
+    auto const ask = [&](int64_t base) {
+      int64_t const idx = min(base + lane, n - 1);
+      bo                = col.child.off(first + idx);
+      eo                = col.child.off(first + min(idx + ngrams, n - 1) + 1);
+    };
+    ask(begin);
+    uint32_t count = 0;
+    for (int64_t base = begin; base < end; base += kWave) {
+      int64_t const idx = base + lane;
+      // a clamped run counts only at element 0 (218-222); a null element starts no run (213-216)
+      bool const valid        = idx < end && (idx == 0 || idx + ngrams < n) && col.child.valid(first + idx);
+      int64_t const run_begin = bo;
+      uint32_t const run      = static_cast<uint32_t>(eo - bo);
+      T hv                    = 0;
+      // The runs of these 64 elements overlap and lie side by side in the chars: fetch that stretch once, with
+      // coalesced loads, and hash out of LDS (the hash walks a run dword by dword, each step a dependent read).
+      // A stretch too long for the buffer is hashed straight from memory.
+      int64_t const span_begin = static_cast<int64_t>(wave_bcast64(static_cast<uint64_t>(bo), 0));
+      int64_t const span_end   = static_cast<int64_t>(wave_bcast64(static_cast<uint64_t>(eo), kWave - 1));
+      if (base + kWave < end) ask(base + kWave);
+      if (sizeof(T) == 4 && span_end - span_begin <= static_cast<int64_t>(kRunStageBytes)) {
+        bool ascii;
+        uint32_t const mis = stage_bytes(col.child.chars, span_begin, static_cast<uint32_t>(span_end - span_begin), lds.bytes, lane, &ascii);
+        wave_lds_fence();
+        if (valid) hv = H::hash(WordSrc{lds.bytes, mis + static_cast<uint32_t>(run_begin - span_begin)}, run, seed);
+        wave_lds_fence();
+      } else if (valid) {
+        hv = H::hash(AlignedSrc(col.child.chars + run_begin, run), run, seed);
+      }
+      hv                = hv < 1 ? T{1} : hv;  // 237
+      uint64_t const vm = ballot64(valid);
+      if (valid) lds.hashes[count + lanes_below(vm)] = hv;
+      count += static_cast<uint32_t>(__builtin_popcountll(vm));
+      if (count > kRunHashes - kWave) {
+        minima.fold(lds.hashes, count);
+        count = 0;
+      }
+    }
+    minima.fold(lds.hashes, count);
+  }
+};
+
+// How the rows are shared out.  In a column of at least kManyRows rows a wavefront does the rows of up to kPart
 // bytes alone, several in turn (minhash_rows_kernel), and the longer ones are cut into parts; in a column of fewer rows
 // every row is cut into parts (minhash_parts_kernel), so that the device is full whatever the rows' lengths: 999
 // documents of 2 KB (256 parameters) with a workgroup each, and another launch for what lay beyond their first 16 KB,
@@ -449,8 +595,6 @@ __device__ __forceinline__ void process_section(const uint8_t* row, int64_t n, i
 // end: the host asks for as many rows per wavefront (a power of two, at most kMaxRowsPerWave) as leave at least
 // kMinRowGroups groups.
 constexpr int32_t kManyRows     = 131072;
-constexpr int64_t kPartBytes    = 4096;
-constexpr int64_t kMinPartBytes = 256;     // a tile: less would be staged for its halo
 constexpr int kMaxRowsPerWave   = 16;
 constexpr int32_t kMinRowGroups = 16384;  // sixteen times the workgroups that 256 CUs hold at four apiece
 inline int rows_per_wave(int32_t rows)
@@ -462,45 +606,46 @@ inline int rows_per_wave(int32_t rows)
 
 // The parts of every row: none for a null row and for the rows that minhash_rows_kernel does, one for an empty row (its
 // zeros have to be written).
+template <typename Source>
 struct RowParts {
-  ColView col;
-  int32_t waves;      // wavefronts that the device holds
-  int64_t row_bytes;  // rows of at most this many bytes are done by minhash_rows_kernel; -1: none is
-  // Bytes of a part: kPartBytes where that leaves every wavefront four parts and more, else a quarter of what each has to
-  // do, in columns of less than a kilobyte per wavefront all of it (a second round of parts would be longer than the
-  // imbalance it removes).
-  __device__ __forceinline__ int64_t part_bytes() const
+  Source source;
+  int32_t waves;  // wavefronts that the device holds
+  int64_t alone;  // rows of at most this length are done by minhash_rows_kernel; -1: none is
+  // Length of a part: kPart where that leaves every wavefront four parts and more, else a quarter of what each has to
+  // do, in columns of less than four of the smallest parts per wavefront all of it (a second round of parts would be
+  // longer than the imbalance it removes).
+  __device__ __forceinline__ int64_t part() const
   {
-    if (row_bytes >= 0) return kPartBytes;
-    int64_t const share = (col.off(col.size) - col.off(0)) / waves;
-    int64_t const bytes = ((share < 1024 ? share : share / 4) + kWave) / kWave * kWave;
-    return min(max(bytes, kMinPartBytes), kPartBytes);
+    if (alone >= 0) return Source::kPart;
+    int64_t const share  = source.total() / waves;
+    int64_t const length = ((share < 4 * Source::kMinPart ? share : share / 4) + kWave) / kWave * kWave;
+    return min(max(length, Source::kMinPart), Source::kPart);
   }
   __device__ __forceinline__ uint64_t operator()(int64_t i) const
   {
-    if (!col.valid(i)) return 0;
-    int64_t const n = col.off(i + 1) - col.off(i);
-    if (n <= row_bytes) return 0;
-    int64_t const bytes = part_bytes();
-    return n == 0 ? 1 : static_cast<uint64_t>((n + bytes - 1) / bytes);
+    if (!source.valid(i)) return 0;
+    int64_t const n = source.length(i);
+    if (n <= alone) return 0;
+    int64_t const length = part();
+    return n == 0 ? 1 : static_cast<uint64_t>((n + length - 1) / length);
   }
 };
 
-// One workgroup per (group of consecutive rows, parameter chunk): its wavefronts take the group's rows of up to kPartBytes
+// One workgroup per (group of consecutive rows, parameter chunk): its wavefronts take the group's rows of up to kPart
 // bytes one at a time from a counter in LDS, so that the four are done together whatever the rows' lengths; the minima
 // go from the registers to the result.  The groups lie along x and, beyond kMaxRowBlocks of them, along z.
-template <typename Minima, typename T = typename Minima::T>
-__global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_rows_kernel(ColView col, T seed, Params<T> params, int32_t width,
+template <typename Source, typename Minima, typename T = typename Minima::T>
+__global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_rows_kernel(Source source, Params<T> params,
                                                                                    const int32_t* __restrict__ out_offsets, T* __restrict__ out,
                                                                                    int per_wave)
 {
-  __shared__ WaveLds<T> lds[kWaves];
+  __shared__ typename Source::Lds lds[kWaves];
   __shared__ typename Minima::Lds minima_lds[kWaves];
   __shared__ uint32_t next_row;
 
   int const group_rows = per_wave * kWaves;
   int64_t const r0     = (static_cast<int64_t>(blockIdx.z) * gridDim.x + blockIdx.x) * group_rows;
-  if (r0 >= col.size) return;
+  if (r0 >= source.rows()) return;
   int const lane           = lane_id();
   int const wave           = threadIdx.x / kWave;
   int32_t const chunk_base = blockIdx.y * Minima::kParams;
@@ -508,7 +653,7 @@ __global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_rows_ker
   Minima minima(&minima_lds[wave], lane);
   minima.load(params, blockIdx.y);
 
-  int const rows_here = static_cast<int>(min(static_cast<int64_t>(group_rows), col.size - r0));
+  int const rows_here = static_cast<int>(min(static_cast<int64_t>(group_rows), source.rows() - r0));
   if (threadIdx.x == 0) next_row = 0;
   __syncthreads();
   for (;;) {
@@ -516,12 +661,11 @@ __global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_rows_ker
     if (lane == 0) t = static_cast<int>(atomicAdd(&next_row, 1u));
     int const i = __builtin_amdgcn_readfirstlane(t);  // (the same in every lane: what depends on it stays scalar)
     if (i >= rows_here) break;
-    if (!col.valid(r0 + i)) continue;
-    int64_t const o = col.off(r0 + i);
-    int64_t const n = col.off(r0 + i + 1) - o;
-    if (n > kPartBytes) continue;
+    if (!source.valid(r0 + i)) continue;
+    int64_t const n = source.length(r0 + i);
+    if (n > Source::kPart) continue;
     minima.reset();
-    if (n > 0) process_section(col.chars + o, n, 0, n, seed, width, minima, lds[wave], lane);
+    if (n > 0) source.process(r0 + i, 0, n, minima, lds[wave], lane);
     minima.finish();
     T* const dst = out + static_cast<int64_t>(out_offsets[r0 + i]) + chunk_base;
     minima.each([&](int32_t j, T v) {
@@ -535,18 +679,18 @@ __global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_rows_ker
 // than eight parts for every wavefront they are handed out by a counter, else by place (a counter answers about 150 M
 // requests a second: seven thousand wavefronts asking at once would wait 50 us).  The chunks of parameters come one
 // after the other in the same count.
-template <typename Minima, typename T = typename Minima::T>
-__global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_parts_kernel(RowParts parts, T seed, Params<T> params, int32_t width,
-                                                                                    int32_t chunks, const int32_t* __restrict__ out_offsets,
+template <typename Source, typename Minima, typename T = typename Minima::T>
+__global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_parts_kernel(RowParts<Source> parts, Params<T> params, int32_t chunks,
+                                                                                    const int32_t* __restrict__ out_offsets,
                                                                                     const uint32_t* __restrict__ prefix,
                                                                                     unsigned long long* __restrict__ counter, T* __restrict__ out)
 {
-  __shared__ WaveLds<T> lds[kWaves];
+  __shared__ typename Source::Lds lds[kWaves];
   __shared__ typename Minima::Lds minima_lds[kWaves];
-  ColView const& col    = parts.col;
-  uint32_t const total  = prefix[col.size];
+  Source const& source  = parts.source;
+  uint32_t const total  = prefix[source.rows()];
   uint64_t const tasks  = static_cast<uint64_t>(total) * static_cast<uint32_t>(chunks);
-  int64_t const bytes   = parts.part_bytes();
+  int64_t const length  = parts.part();
   int const lane        = lane_id();
   int const wave        = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
   uint64_t const nwaves = static_cast<uint64_t>(gridDim.x) * kWaves;
@@ -563,7 +707,7 @@ __global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_parts_ke
     int32_t const chunk_base = static_cast<int32_t>(chunk) * Minima::kParams;
     int32_t const in_chunk   = min(Minima::kSlots, params.count - chunk_base);
     // the last row r with prefix[r] <= t, 64 of them looked at in one step
-    int64_t r = 0, end = col.size;
+    int64_t r = 0, end = source.rows();
     while (end - r > 1) {
       int64_t const step = (end - r + kWave - 1) / kWave;
       int64_t const at   = r + lane * step;
@@ -571,13 +715,12 @@ __global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_parts_ke
       r += (below - 1) * step;
       end = min(end, r + step);
     }
-    int64_t const o   = col.off(r);
-    int64_t const n   = col.off(r + 1) - o;
-    int64_t const sb  = static_cast<int64_t>(t - prefix[r]) * bytes;
-    int64_t const se  = min(n, sb + bytes);
-    bool const shared = n > bytes;
+    int64_t const n     = source.length(r);
+    int64_t const begin = static_cast<int64_t>(t - prefix[r]) * length;
+    int64_t const till  = min(n, begin + length);
+    bool const shared   = n > length;
     minima.reset();
-    if (sb < se) process_section(col.chars + o, n, sb, se, seed, width, minima, lds[wave], lane);
+    if (begin < till) source.process(r, begin, till, minima, lds[wave], lane);
     minima.finish();
     T* const dst = out + static_cast<int64_t>(out_offsets[r]) + chunk_base;
     minima.each([&](int32_t j, T v) {
@@ -597,10 +740,11 @@ __global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_parts_ke
   }
 }
 
+template <typename Source>
 struct ValidTimesP {
-  ColView col;
+  Source source;
   int32_t P;
-  __device__ uint64_t operator()(int64_t i) const { return col.valid(i) ? static_cast<uint64_t>(P) : 0; }
+  __device__ uint64_t operator()(int64_t i) const { return source.valid(i) ? static_cast<uint64_t>(P) : 0; }
 };
 
 __global__ void uniform_offsets_kernel(int32_t* out, int32_t rows, int32_t P)
@@ -613,14 +757,14 @@ constexpr int32_t kMaxRowBlocks = 1 << 15;  // groups along x (a launch of 4 M r
 
 // The largest value into the slots of the rows that are done in several parts, and 0 into the counter of the parts: a
 // wavefront looks at 64 rows and fills those of them one after the other.
-template <typename T>
-__global__ void __launch_bounds__(kThreads) minhash_clear_kernel(RowParts parts, int32_t P, const int32_t* __restrict__ out_offsets,
+template <typename Source, typename T = typename Source::T>
+__global__ void __launch_bounds__(kThreads) minhash_clear_kernel(RowParts<Source> parts, int32_t P, const int32_t* __restrict__ out_offsets,
                                                                  unsigned long long* __restrict__ counter, T* __restrict__ out)
 {
   if (blockIdx.x == 0 && threadIdx.x == 0) *counter = 0;
   int const lane  = lane_id();
   int64_t const r = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  bool const many = r < parts.col.size && parts(r) > 1;
+  bool const many = r < parts.source.rows() && parts(r) > 1;
   int64_t const o = many ? out_offsets[r] : 0;
   for (uint64_t todo = ballot64(many); todo != 0; todo &= todo - 1) {
     T* const dst = out + static_cast<int64_t>(wave_bcast64(static_cast<uint64_t>(o), __builtin_ctzll(todo)));
@@ -639,12 +783,12 @@ __global__ void __launch_bounds__(kWave) minhash64_prepare_kernel(const uint64_t
 // rows (and finds the rows' places in the result where some are null), the others write the places where none is and
 // fill the result; the wavefronts of the workgroups from `fillers` + 1 on lay out the parameters of 64-bit hashes.
 constexpr int32_t kPlanRows = kScanSmallTiles * kScanTile;
-template <typename T>
-__global__ void __launch_bounds__(kScanThreads) minhash_plan_kernel(RowParts parts, Params<T> params, filter64::Group* groups, unsigned fillers,
+template <typename Source, typename T = typename Source::T>
+__global__ void __launch_bounds__(kScanThreads) minhash_plan_kernel(RowParts<Source> parts, Params<T> params, filter64::Group* groups, unsigned fillers,
                                                                     int32_t* __restrict__ out_offsets, uint32_t* __restrict__ prefix,
                                                                     unsigned long long* __restrict__ counter, T* __restrict__ out, int64_t out_size)
 {
-  int32_t const rows = parts.col.size;
+  int32_t const rows = parts.source.rows();
   int32_t const P    = params.count;
   if constexpr (sizeof(T) == 8) {
     if (blockIdx.x > fillers) {
@@ -656,7 +800,7 @@ __global__ void __launch_bounds__(kScanThreads) minhash_plan_kernel(RowParts par
   if (blockIdx.x > 0) {
     int64_t const first  = static_cast<int64_t>(blockIdx.x - 1) * kScanThreads + threadIdx.x;
     int64_t const stride = static_cast<int64_t>(fillers) * kScanThreads;
-    if (!parts.col.use_mask)
+    if (!parts.source.masked())
       for (int64_t i = first; i <= rows; i += stride) out_offsets[i] = static_cast<int32_t>(i * P);
     for (int64_t i = first; i < out_size; i += stride) out[i] = std::numeric_limits<T>::max();
     return;
@@ -669,7 +813,7 @@ __global__ void __launch_bounds__(kScanThreads) minhash_plan_kernel(RowParts par
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
       bool const in = base + k < rows;
-      vals[k]       = in ? parts(base + k) | (static_cast<uint64_t>(parts.col.valid(base + k)) << 32) : 0;
+      vals[k]       = in ? parts(base + k) | (static_cast<uint64_t>(parts.source.valid(base + k)) << 32) : 0;
       sum += vals[k];
     }
     uint64_t total;
@@ -678,7 +822,7 @@ __global__ void __launch_bounds__(kScanThreads) minhash_plan_kernel(RowParts par
     for (int k = 0; k < kScanItems; ++k) {
       if (base + k < rows) {
         prefix[base + k] = static_cast<uint32_t>(run);
-        if (parts.col.use_mask) out_offsets[base + k] = static_cast<int32_t>(run >> 32) * P;
+        if (parts.source.masked()) out_offsets[base + k] = static_cast<int32_t>(run >> 32) * P;
       }
       run += vals[k];
     }
@@ -687,26 +831,26 @@ __global__ void __launch_bounds__(kScanThreads) minhash_plan_kernel(RowParts par
   if (threadIdx.x == 0) {
     *counter     = 0;
     prefix[rows] = static_cast<uint32_t>(carry);
-    if (parts.col.use_mask) out_offsets[rows] = static_cast<int32_t>(carry >> 32) * P;
+    if (parts.source.masked()) out_offsets[rows] = static_cast<int32_t>(carry >> 32) * P;
   }
 }
 
-template <typename Minima, typename T = typename Minima::T>
-void launch_kernels(RowParts const& parts, T seed, Params<T> const& params, int32_t chunks, int32_t width, const int32_t* offsets,
+template <typename Minima, typename Source, typename T = typename Source::T>
+void launch_kernels(RowParts<Source> const& parts, int32_t rows, Params<T> const& params, int32_t chunks, const int32_t* offsets,
                     const uint32_t* prefix, unsigned long long* counter, T* child, hipStream_t stream)
 {
-  ColView const& v = parts.col;
-  if (v.size >= kManyRows) {
-    int const per_wave   = rows_per_wave(v.size);
-    int32_t const groups = (v.size + per_wave * kWaves - 1) / (per_wave * kWaves);
+  if (rows >= kManyRows) {
+    int const per_wave   = rows_per_wave(rows);
+    int32_t const groups = (rows + per_wave * kWaves - 1) / (per_wave * kWaves);
     dim3 grid(static_cast<unsigned>(std::min(groups, kMaxRowBlocks)), static_cast<unsigned>(chunks),
               static_cast<unsigned>((groups + kMaxRowBlocks - 1) / kMaxRowBlocks));
-    ProfileScope ps("minhash_rows_kernel", stream);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_rows_kernel<Minima>), grid, dim3(kThreads), 0, stream, v, seed, params, width, offsets, child, per_wave);
+    ProfileScope ps(Source::kRowsName, stream);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_rows_kernel<Source, Minima>), grid, dim3(kThreads), 0, stream, parts.source, params, offsets, child,
+                       per_wave);
   }
-  ProfileScope ps("minhash_parts_kernel", stream);
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_parts_kernel<Minima>), dim3(static_cast<unsigned>(parts.waves / kWaves)), dim3(kThreads), 0, stream, parts,
-                     seed, params, width, chunks, offsets, prefix, counter, child);
+  ProfileScope ps(Source::kPartsName, stream);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_parts_kernel<Source, Minima>), dim3(static_cast<unsigned>(parts.waves / kWaves)), dim3(kThreads), 0, stream,
+                     parts, params, chunks, offsets, prefix, counter, child);
 }
 
 // How the parameters of 32-bit hashes are shared out: chunks of K sets of 64 (every chunk hashes the windows again, and a lane without
@@ -770,38 +914,37 @@ void with_minima(int32_t P, Launch const& launch)
 // The launches of one minhash call: the row offsets of the result and the parts of every row, then the hashing kernels.
 // prefix holds rows + 1 values, scan_tmp scan_temp_bytes(rows) bytes and one 64-bit counter behind them; laid_out (64-bit
 // hashes) groups_of(P).
-template <typename T>
-void run_minhash(const ColView& v, T seed, const T* a, const T* b, int32_t P, int32_t width, int32_t* offsets, T* child, int64_t child_size,
+template <typename Source, typename T = typename Source::T>
+void run_minhash(Source const& source, int32_t rows, bool masked, const T* a, const T* b, int32_t P, int32_t* offsets, T* child, int64_t child_size,
                  uint32_t* prefix, uint64_t* scan_tmp, filter64::Group* laid_out, hipStream_t stream)
 {
-  int32_t const rows = v.size;
   int simd_waves = 0;
   with_minima<T>(P, [&](auto which, int32_t) { simd_waves = decltype(which)::type::kSimdWaves; });
-  RowParts const parts{v, device_cus() * 4 * simd_waves, rows >= kManyRows ? kPartBytes : -1};
+  RowParts<Source> const parts{source, device_cus() * 4 * simd_waves, rows >= kManyRows ? Source::kPart : -1};
   Params<T> const params{a, b, P, laid_out};
   auto* const counter = reinterpret_cast<unsigned long long*>(scan_tmp) + scan_temp_bytes(rows) / sizeof(uint64_t);
   if (rows <= kPlanRows) {
     int64_t const most    = std::max<int64_t>(child_size, rows + 1);
     unsigned const fillers = static_cast<unsigned>(std::min<int64_t>((most + 4 * kScanThreads - 1) / (4 * kScanThreads), 1024));
     unsigned const layers  = sizeof(T) == 8 ? static_cast<unsigned>((groups_of(P) + kScanThreads / kWave - 1) / (kScanThreads / kWave)) : 0u;
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_plan_kernel<T>), dim3(1 + fillers + layers), dim3(kScanThreads), 0, stream, parts, params, laid_out,
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_plan_kernel<Source>), dim3(1 + fillers + layers), dim3(kScanThreads), 0, stream, parts, params, laid_out,
                        fillers, offsets, prefix, counter, child, child_size);
   } else {
-    if (v.use_mask) {
-      device_exclusive_scan(ValidTimesP{v, P}, static_cast<int64_t>(rows), offsets, scan_tmp, stream);
+    if (masked) {
+      device_exclusive_scan(ValidTimesP<Source>{source, P}, static_cast<int64_t>(rows), offsets, scan_tmp, stream);
     } else {
       hipLaunchKernelGGL(uniform_offsets_kernel, dim3((rows + 1 + 255) / 256), dim3(256), 0, stream, offsets, rows, P);
     }
     if constexpr (sizeof(T) == 8)
       hipLaunchKernelGGL(minhash64_prepare_kernel, dim3(static_cast<unsigned>(groups_of(P))), dim3(kWave), 0, stream, a, b, P, laid_out);
     device_exclusive_scan(parts, static_cast<int64_t>(rows), prefix, scan_tmp, stream);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_clear_kernel<T>), dim3((rows + kThreads - 1) / kThreads), dim3(kThreads), 0, stream, parts, P, offsets, counter,
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_clear_kernel<Source>), dim3((rows + kThreads - 1) / kThreads), dim3(kThreads), 0, stream, parts, P, offsets, counter,
                        child);
   }
 
   if (child_size > 0) {
     with_minima<T>(P, [&](auto which, int32_t chunks) {
-      launch_kernels<typename decltype(which)::type>(parts, seed, params, chunks, width, offsets, prefix, counter, child, stream);
+      launch_kernels<typename decltype(which)::type>(parts, rows, params, chunks, offsets, prefix, counter, child, stream);
     });
   }
 }
@@ -865,7 +1008,7 @@ nvtext_amd_status minhash_impl(const nvtext_amd_strings_column* input, T seed, c
     nvtext_amd_list_column_free(out, stream_, mr_);
     return fail(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");
   }
-  run_minhash<T>(v, seed, a, b, P, width, out->offsets, static_cast<T*>(out->child), out->child_size, temp.part<uint32_t>(1),
+  run_minhash(TextRows<T>{v, seed, width}, rows, v.use_mask != 0, a, b, P, out->offsets, static_cast<T*>(out->child), out->child_size, temp.part<uint32_t>(1),
                  temp.part<uint64_t>(0), temp.part<filter64::Group>(2), stream);
   NVTEXT_HIP_TRY_OR(hipGetLastError(), nvtext_amd_list_column_free(out, stream_, mr_));
   return NVTEXT_AMD_SUCCESS;
@@ -873,197 +1016,6 @@ nvtext_amd_status minhash_impl(const nvtext_amd_strings_column* input, T seed, c
 
 
 // ------------------------------------------------------------------ minhash_ngrams / minhash64_ngrams
-// LIST<STRING> rows: the hashed items are runs of consecutive list elements instead of character windows
-// (cpp/src/text/minhash.cu:182-250); the permutation and the minimum are the ones above.
-struct ListView {
-  const int32_t* offsets;  // element index of the first element of row i + offset
-  const uint32_t* mask;
-  int32_t size;
-  int32_t offset;
-  int32_t use_mask;
-  ColView child;           // the elements
-
-  __device__ __forceinline__ int64_t off(int64_t i) const { return offsets[i + offset]; }
-  __device__ __forceinline__ bool valid(int64_t i) const
-  {
-    if (!use_mask) return true;
-    int64_t const b = i + offset;
-    return (mask[b >> 5] >> (b & 31)) & 1u;
-  }
-};
-
-// Byte source over global memory through aligned dword loads that overlap [p, p + len) only.
-struct AlignedSrc {
-  const uint32_t* w;  // aligned address at or below the first byte
-  uint32_t mis;       // first byte inside w[0]
-  uint32_t end;       // mis + len
-  __device__ __forceinline__ AlignedSrc(const uint8_t* p, uint32_t len)
-  {
-    mis = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(p) & 3u);
-    w   = reinterpret_cast<const uint32_t*>(p - mis);
-    end = mis + len;
-  }
-  __device__ __forceinline__ uint32_t byte(uint32_t i) const { return reinterpret_cast<const uint8_t*>(w)[mis + i]; }
-  __device__ __forceinline__ uint32_t u32(uint32_t i) const
-  {
-    uint32_t const o  = mis + i;
-    uint32_t const j  = o >> 2;
-    uint32_t const lo = 4u * j < end ? w[j] : 0u;
-    uint32_t const hi = 4u * (j + 1u) < end ? w[j + 1] : 0u;
-    return __builtin_amdgcn_alignbit(hi, lo, (o & 3u) * 8u);
-  }
-};
-
-constexpr uint32_t kNgramStageBytes = 4096;                             // longest stretch of chars hashed out of LDS
-constexpr uint32_t kNgramStageWords = (kNgramStageBytes + 16 + 32) / 4;  // + misalignment, + whole blocks and over-read of the hash tail
-
-// One workgroup per (group of consecutive rows, parameter chunk), as in minhash_rows_kernel: a row of up to
-// kNgramSoloPositions positions is done by one wavefront alone, 64 positions a trip (wavefront w takes the rows w, w + 4, .. of the group,
-// `solo_per_wave` of them), and its minima go from the registers to the result; a row of more positions is shared by the
-// four wavefronts, which take its positions 64 at a time in turn and combine through LDS, one such row after the other.
-// A column of fewer than 131,072 rows keeps one row to a workgroup, every row shared by the four wavefronts
-// (solo_per_wave 0): it needs its workgroups to fill the device and to even out its end (20,000 rows of 3,000 elements:
-// four rows to a workgroup were 8 % slower).
-constexpr int64_t kNgramSoloPositions = 2048;
-template <typename Minima, typename T = typename Minima::T>
-__global__ void __launch_bounds__(kThreads, sizeof(T) == 4 ? 6 : Minima::kSimdWaves) minhash_ngrams_kernel(ListView in, int32_t ngrams, T seed, Params<T> params,
-                                                                                     const int32_t* __restrict__ out_offsets, T* __restrict__ out,
-                                                                                     int solo_per_wave)
-{
-  using H = HashTraits<T>;
-  __shared__ alignas(16) T hashes[kWaves][2 * kWave];  // 64 hashes a trip, padded to the stride of the fold (at most 64 more)
-  __shared__ typename Minima::Lds minima_lds[kWaves];
-  __shared__ T red[kWaves][Minima::kSlots];
-  // the chars of the elements a wavefront is hashing (32-bit hash only: measured 13 % faster there, 9 % slower for the
-  // 64-bit hash, whose 16-byte steps cost more to assemble out of LDS than they save)
-  constexpr bool kStageRuns = sizeof(T) == 4;
-  __shared__ alignas(16) uint32_t run_bytes[kWaves][kStageRuns ? kNgramStageWords : 1];
-  __shared__ uint32_t next_row;
-
-  int const group_rows = solo_per_wave > 0 ? solo_per_wave * kWaves : 1;
-  int64_t const r0     = (static_cast<int64_t>(blockIdx.z) * gridDim.x + blockIdx.x) * group_rows;  // groups along x, then z
-  if (r0 >= in.size) return;
-  int64_t const solo_positions = solo_per_wave > 0 ? kNgramSoloPositions : -1;
-  int32_t const chunk_base     = blockIdx.y * Minima::kParams;
-  int32_t const in_chunk       = min(Minima::kSlots, params.count - chunk_base);
-  int const lane               = lane_id();
-  int const wave               = threadIdx.x / kWave;
-  Minima minima(&minima_lds[wave], lane);
-  minima.load(params, blockIdx.y);
-
-  int const rows_here = static_cast<int>(min(static_cast<int64_t>(group_rows), in.size - r0));
-  if (threadIdx.x == 0) next_row = 0;
-  __syncthreads();
-  // the short rows of the group first, each wavefront taking the next one whenever it is done with one; then, from
-  // `together` = 0 on, the rows that all four do together, one after the other (see minhash_rows_kernel)
-  int together = -1;
-  for (;;) {
-    int i;
-    if (together < 0) {
-      int t = 0;
-      if (lane == 0) t = static_cast<int>(atomicAdd(&next_row, 1u));
-      i = __builtin_amdgcn_readfirstlane(t);
-      if (i >= rows_here) {
-        together = 0;
-        continue;
-      }
-    } else {
-      if (together >= rows_here) break;
-      i = together++;
-    }
-    bool const solo = together < 0;
-    if (!in.valid(r0 + i)) continue;
-    int64_t const first = in.off(r0 + i);
-    int64_t const n     = in.off(r0 + i + 1) - first;
-    // minhash.cu:311-314 with width = ngrams: the positions that the permutation looks at
-    int64_t const positions = max(static_cast<int64_t>(1), n - ngrams + 1);
-    if (solo != (positions <= solo_positions)) continue;
-    minima.reset();
-    if (n > 0) {
-      int64_t const trip = solo ? kWave : kWaves * kWave;
-      for (int64_t base = solo ? 0 : static_cast<int64_t>(wave) * kWave; base < positions; base += trip) {
-        int64_t const idx = base + lane;
-        bool valid        = false;
-        T hv              = 0;
-        int64_t bo = 0, eo = 0;
-        if (idx < positions && in.child.valid(first + idx)) {  // 213-216: a null element starts no run
-          // 218-222: the run ends at element idx + ngrams, clamped to the row; a clamped run counts only at idx 0
-          int64_t const next = min(idx + ngrams, n - 1);
-          if (idx == 0 || next - idx >= ngrams) {
-            // 224-229: the bytes from the start of element idx to the end of element next
-            bo    = in.child.off(first + idx);
-            eo    = in.child.off(first + next + 1);
-            valid = true;
-          }
-        }
-        // The runs of these 64 elements overlap and lie side by side in the chars: fetch that stretch once, with
-        // coalesced loads, and hash out of LDS (the hash walks a run dword by dword, each step a dependent read).
-        // A stretch too long for the buffer is hashed straight from memory.
-        int64_t const span_begin = kStageRuns ? in.child.off(first + base) : 0;
-        int64_t const span_end   = kStageRuns ? in.child.off(first + min(base + kWave + ngrams, n)) : 0;
-        if (kStageRuns && span_end - span_begin <= static_cast<int64_t>(kNgramStageBytes)) {
-          bool ascii;
-          uint32_t const mis = stage_bytes(in.child.chars, span_begin, static_cast<uint32_t>(span_end - span_begin), run_bytes[wave], lane, &ascii);
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-          if (valid) {
-            WordSrc const src{run_bytes[wave], mis + static_cast<uint32_t>(bo - span_begin)};
-            hv = H::hash(src, static_cast<uint32_t>(eo - bo), seed);
-          }
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-        } else if (valid) {
-          AlignedSrc const src(in.child.chars + bo, static_cast<uint32_t>(eo - bo));
-          hv = H::hash(src, static_cast<uint32_t>(eo - bo), seed);
-        }
-        if (valid) hv = hv < 1 ? T{1} : hv;  // 237
-        uint64_t const vm = ballot64(valid);
-        if (valid) hashes[wave][lanes_below(vm)] = hv;
-        minima.fold(hashes[wave], static_cast<uint32_t>(__builtin_popcountll(vm)));
-      }
-    }
-    minima.finish();
-    T* const dst = out + static_cast<int64_t>(out_offsets[r0 + i]) + chunk_base;
-    if (solo) {
-      // an empty row is zeros (minhash.cu:318); a row whose every run was skipped keeps the all-ones start value
-      minima.each([&](int32_t j, T v) {
-        if (j < in_chunk) dst[j] = n > 0 ? v : T{0};
-      });
-    } else {
-      __syncthreads();  // (the row before has been read out of red)
-      minima.each([&](int32_t j, T v) { red[wave][j] = v; });
-      __syncthreads();
-      for (int j = threadIdx.x; j < in_chunk; j += kThreads) {
-        T v = red[0][j];
-#pragma unroll
-        for (int w = 1; w < kWaves; ++w) v = min(v, red[w][j]);
-        dst[j] = n > 0 ? v : T{0};
-      }
-    }
-  }
-}
-
-struct ListValidTimesP {
-  ListView in;
-  int32_t P;
-  __device__ uint64_t operator()(int64_t i) const { return in.valid(i) ? static_cast<uint64_t>(P) : 0; }
-};
-
-template <typename Minima, typename T = typename Minima::T>
-void launch_ngrams(const ListView& v, int32_t ngrams, T seed, Params<T> const& params, int32_t chunks, const int32_t* offsets, T* child,
-                   hipStream_t stream)
-{
-  int const solo_per_wave = v.size >= kManyRows ? rows_per_wave(v.size) : 0;
-  int32_t const group     = solo_per_wave > 0 ? solo_per_wave * kWaves : 1;
-  int32_t const groups    = (v.size + group - 1) / group;
-  dim3 grid(static_cast<unsigned>(std::min(groups, kMaxRowBlocks)), static_cast<unsigned>(chunks),
-            static_cast<unsigned>((groups + kMaxRowBlocks - 1) / kMaxRowBlocks));
-  ProfileScope ps("minhash_ngrams_kernel", stream);
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_ngrams_kernel<Minima>), grid, dim3(kThreads), 0, stream, v, ngrams, seed, params, offsets, child,
-                     solo_per_wave);
-}
-
 template <typename T>
 nvtext_amd_status minhash_ngrams_impl(const nvtext_amd_list_strings_column* input, int32_t ngrams, T seed, const T* a, const T* b,
                                       int64_t a_count, int64_t b_count, void* stream_, const nvtext_amd_allocator* mr_,
@@ -1125,25 +1077,15 @@ nvtext_amd_status minhash_ngrams_impl(const nvtext_amd_list_strings_column* inpu
   v.offset   = input->offset;
   v.use_mask = (input->null_mask != nullptr && input->null_count > 0) ? 1 : 0;
   v.child    = make_view(input->child);
-  size_t const temp_bytes[2] = {v.use_mask ? scan_temp_bytes(rows) : 0, sizeof(T) == 8 ? static_cast<size_t>(groups_of(P)) * sizeof(filter64::Group) : 0};
-  TempParts<2> const temp(mr, temp_bytes, v.use_mask || sizeof(T) == 8);
+  size_t const temp_bytes[3] = {scan_temp_bytes(rows) + sizeof(uint64_t), static_cast<size_t>(rows + 1) * sizeof(uint32_t),
+                                sizeof(T) == 8 ? static_cast<size_t>(groups_of(P)) * sizeof(filter64::Group) : 0};
+  TempParts<3> const temp(mr, temp_bytes);
   if (!temp.ok()) {
     nvtext_amd_list_column_free(out, stream_, mr_);
     return fail(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");
   }
-  if (v.use_mask) {
-    device_exclusive_scan(ListValidTimesP{v, P}, static_cast<int64_t>(rows), out->offsets, temp.part<uint64_t>(0), stream);
-  } else {
-    hipLaunchKernelGGL(uniform_offsets_kernel, dim3((rows + 1 + 255) / 256), dim3(256), 0, stream, out->offsets, rows, P);
-  }
-  auto* const laid_out = temp.part<filter64::Group>(1);
-  if constexpr (sizeof(T) == 8)
-    hipLaunchKernelGGL(minhash64_prepare_kernel, dim3(static_cast<unsigned>(groups_of(P))), dim3(kWave), 0, stream, a, b, P, laid_out);
-  if (out->child_size > 0) {
-    with_minima<T>(P, [&](auto which, int32_t chunks) {
-      launch_ngrams<typename decltype(which)::type>(v, ngrams, seed, Params<T>{a, b, P, laid_out}, chunks, out->offsets, static_cast<T*>(out->child), stream);
-    });
-  }
+  run_minhash(RunRows<T>{v, seed, ngrams}, rows, v.use_mask != 0, a, b, P, out->offsets, static_cast<T*>(out->child), out->child_size,
+              temp.part<uint32_t>(1), temp.part<uint64_t>(0), temp.part<filter64::Group>(2), stream);
   NVTEXT_HIP_TRY_OR(hipGetLastError(), nvtext_amd_list_column_free(out, stream_, mr_));
   return NVTEXT_AMD_SUCCESS;
 }
@@ -1211,7 +1153,7 @@ nvtext_amd_status nvtext_amd_minhash_preallocated(const nvtext_amd_strings_colum
   if (input->null_mask) launch_copy_bitmask(out_null_mask, input->null_mask, input->offset, rows, stream);
   ColView const v = make_view(*input);
   // every value of the scratch that the kernels read is written earlier in this same call: nothing to clear
-  run_minhash<uint32_t>(v, seed, a, b, P, width, out_offsets, out_child, child_size, prefix, scan_tmp, nullptr, stream);
+  run_minhash(TextRows<uint32_t>{v, seed, width}, rows, v.use_mask != 0, a, b, P, out_offsets, out_child, child_size, prefix, scan_tmp, nullptr, stream);
   NVTEXT_HIP_TRY(hipGetLastError());
   return NVTEXT_AMD_SUCCESS;
 }
