@@ -510,17 +510,39 @@ void device_exclusive_scan(F f, int64_t n, OutT* out, uint64_t* temp, hipStream_
 int device_cus();
 
 // ------------------------------------------------------------------ scalars for the host
-// A few KB of pinned host memory that kernels write and the host reads once the stream is synchronised (a copy of a
-// few bytes into ordinary host memory goes through a staging buffer and costs ten microseconds and more): eight 64-bit
-// words, and behind them room for kHostSampleWords 32-bit words.  One buffer per host thread, allocated at the thread's
-// first call and kept until the process ends; nullptr when the allocation failed (the callers then copy).
+// A few KB of pinned host memory that kernels write and the host reads (a copy of a few bytes into ordinary host memory
+// goes through a staging buffer and costs ten microseconds and more): eight 64-bit words, behind them room for
+// kHostSampleWords 32-bit words, and a word in a cache line of its own that says what has been written.  One buffer per
+// host thread, allocated at the thread's first call and kept until the process ends; nullptr when the allocation failed
+// (the callers then copy).
 constexpr size_t kHostSampleWords = 3 * 512;
-constexpr size_t kHostScalarBytes = 8 * sizeof(uint64_t) + kHostSampleWords * sizeof(uint32_t);
+constexpr size_t kHostPostedWord  = 8 + (kHostSampleWords / 2 + 7) / 8 * 8;  // (in 64-bit words)
+constexpr size_t kHostScalarBytes = (kHostPostedWord + 8) * sizeof(uint64_t);
 uint64_t* host_scalars();
+
+// Word from a kernel that what it (and the kernels before it on its stream) wrote to the pinned words is there.  The host
+// looks for it itself: it has the numbers some seven microseconds earlier than by waiting for the stream, and need not wait
+// for kernels behind this one.
+struct HostPost {
+  uint64_t* posted;
+  uint64_t ticket;
+  // by one thread, after what it is about has been written: by this thread, or before a barrier with a fence of its own
+  // (__threadfence_system) by the thread that wrote
+  __device__ __forceinline__ void send() const
+  {
+    __threadfence_system();
+    __hip_atomic_store(posted, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+};
+HostPost new_post();  // (only where host_scalars() gives memory)
+// Returns when it has been sent, or with the error that keeps it from being sent.
+hipError_t wait_for_post(HostPost const& post, hipStream_t stream);
+
 // *dst = *src
-void launch_publish(const uint64_t* src, uint64_t* dst, hipStream_t stream);
+void launch_publish(const uint64_t* src, uint64_t* dst, HostPost post, hipStream_t stream);
 // dst[0] = offsets[first_index], dst[1] = offsets[last_index] (offsets of 32 or 64 bits)
-void launch_read_two_offsets(const void* offsets, int is64, int64_t first_index, int64_t last_index, uint64_t* dst, hipStream_t stream);
+void launch_read_two_offsets(const void* offsets, int is64, int64_t first_index, int64_t last_index, uint64_t* dst, HostPost post,
+                             hipStream_t stream);
 
 // ------------------------------------------------------------------ bitmask copy
 // dst bit i = src bit (i + begin_bit); bits past `bits` are cleared

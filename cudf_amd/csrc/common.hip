@@ -4,6 +4,7 @@
 #include "common.cuh"
 
 #include <atomic>
+#include <chrono>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -149,10 +150,13 @@ __global__ void fill_u32_kernel(uint32_t* dst, uint32_t value, int64_t count)
 }  // namespace
 
 namespace {
-__global__ void read_two_offsets_kernel(const void* offsets, int is64, int64_t first_index, int64_t last_index, uint64_t* dst)
+__global__ void read_two_offsets_kernel(const void* offsets, int is64, int64_t first_index, int64_t last_index, uint64_t* dst, HostPost post)
 {
-  int64_t const i = threadIdx.x == 0 ? first_index : last_index;
-  dst[threadIdx.x] = static_cast<uint64_t>(is64 ? static_cast<const int64_t*>(offsets)[i] : static_cast<int64_t>(static_cast<const int32_t*>(offsets)[i]));
+  for (int k = 0; k < 2; ++k) {
+    int64_t const i = k == 0 ? first_index : last_index;
+    dst[k] = static_cast<uint64_t>(is64 ? static_cast<const int64_t*>(offsets)[i] : static_cast<int64_t>(static_cast<const int32_t*>(offsets)[i]));
+  }
+  post.send();
 }
 }  // namespace
 
@@ -181,24 +185,63 @@ uint64_t* host_scalars()
     slot.tried = true;
     void* p    = nullptr;
     // portable: usable whichever device the thread has current at a later call
-    if (hipHostMalloc(&p, kHostScalarBytes, hipHostMallocPortable) == hipSuccess) slot.p = static_cast<uint64_t*>(p);
-    else (void)hipGetLastError();
+    // coherent: what a running kernel writes can be seen
+    if (hipHostMalloc(&p, kHostScalarBytes, hipHostMallocPortable | hipHostMallocCoherent) == hipSuccess) {
+      slot.p                  = static_cast<uint64_t*>(p);
+      slot.p[kHostPostedWord] = 0;
+    } else {
+      (void)hipGetLastError();
+    }
   }
   return slot.p;
 }
 
-namespace {
-__global__ void publish_kernel(const uint64_t* __restrict__ src, uint64_t* __restrict__ dst) { *dst = *src; }
-}  // namespace
-
-void launch_publish(const uint64_t* src, uint64_t* dst, hipStream_t stream)
+HostPost new_post()
 {
-  hipLaunchKernelGGL(publish_kernel, dim3(1), dim3(1), 0, stream, src, dst);
+  thread_local uint64_t tickets = 0;
+  return HostPost{host_scalars() + kHostPostedWord, ++tickets};
 }
 
-void launch_read_two_offsets(const void* offsets, int is64, int64_t first_index, int64_t last_index, uint64_t* dst, hipStream_t stream)
+hipError_t wait_for_post(HostPost const& post, hipStream_t stream)
 {
-  hipLaunchKernelGGL(read_two_offsets_kernel, dim3(1), dim3(2), 0, stream, offsets, is64, first_index, last_index, dst);
+  auto const sent = [&] { return __atomic_load_n(post.posted, __ATOMIC_ACQUIRE) == post.ticket; };
+  auto asked = std::chrono::steady_clock::now();
+  for (;;) {
+    for (int look = 0; look < 64; ++look) {
+      if (sent()) return hipSuccess;
+      __builtin_ia32_pause();
+    }
+    // now and then the stream is asked: a kernel that failed sends nothing (seldom, because asking puts a marker on the
+    // stream: asked every 30 us, calls of 55 us took 67)
+    auto const now = std::chrono::steady_clock::now();
+    if (now - asked < std::chrono::milliseconds(2)) continue;
+    asked = now;
+    hipError_t const e = hipStreamQuery(stream);
+    if (e == hipErrorNotReady) {
+      (void)hipGetLastError();
+      continue;
+    }
+    if (e != hipSuccess) return e;
+    return sent() ? hipSuccess : hipErrorUnknown;
+  }
+}
+
+namespace {
+__global__ void publish_kernel(const uint64_t* __restrict__ src, uint64_t* __restrict__ dst, HostPost post)
+{
+  *dst = *src;
+  post.send();
+}
+}  // namespace
+
+void launch_publish(const uint64_t* src, uint64_t* dst, HostPost post, hipStream_t stream)
+{
+  hipLaunchKernelGGL(publish_kernel, dim3(1), dim3(1), 0, stream, src, dst, post);
+}
+
+void launch_read_two_offsets(const void* offsets, int is64, int64_t first_index, int64_t last_index, uint64_t* dst, HostPost post, hipStream_t stream)
+{
+  hipLaunchKernelGGL(read_two_offsets_kernel, dim3(1), dim3(1), 0, stream, offsets, is64, first_index, last_index, dst, post);
 }
 
 void launch_copy_bitmask(uint32_t* dst, const uint32_t* src, int32_t begin_bit, int32_t bits, hipStream_t stream)

@@ -355,6 +355,7 @@ __device__ __forceinline__ bool count_pair(ColView const& c1, ColView const& c2,
 // [8..9] = the most bytes a pair of the global list has (64 bits) -- then four counters (|A|, |B|, |A n B|, parts done) for
 // every entry of the list of pairs in parts, and `rows` entries for each list.
 constexpr int kListHeader = 16;
+constexpr int32_t kLookRows = 32768;  // see nvtext_amd_jaccard_index
 __host__ __device__ __forceinline__ size_t work_words(int64_t rows) { return kListHeader + static_cast<size_t>(kLists + 4) * static_cast<size_t>(rows); }
 __device__ __forceinline__ uint32_t* list_entries(uint32_t* work, int list, int64_t rows) { return work + kListHeader + (4 + list) * rows; }
 __device__ __forceinline__ uint32_t* part_counters(uint32_t* work) { return work + kListHeader; }
@@ -546,7 +547,13 @@ __global__ void and_bitmask_kernel(uint32_t* __restrict__ out, const uint32_t* _
   if (zeros) atomicAdd(nulls, zeros);
 }
 
-__global__ void publish_header_kernel(const uint32_t* __restrict__ work, uint32_t* __restrict__ host) { host[threadIdx.x] = work[threadIdx.x]; }
+__global__ void publish_header_kernel(const uint32_t* __restrict__ work, uint32_t* __restrict__ host, HostPost post)
+{
+  host[threadIdx.x] = work[threadIdx.x];
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) post.send();
+}
 
 }  // namespace
 }  // namespace nvtext_amd
@@ -606,28 +613,6 @@ nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* inpu
     unsigned const grid  = static_cast<unsigned>(std::min<int64_t>(groups, static_cast<int64_t>(cus) * 64));
     hipLaunchKernelGGL(jaccard_wave_kernel, dim3(grid), dim3(kThreads), 0, stream, v1, v2, width, values, lists, per_group);
   }
-  auto const grid_of = [&](int per_cu) { return dim3(static_cast<unsigned>(std::min<int64_t>(rows, static_cast<int64_t>(cus) * per_cu))); };
-  {
-    ProfileScope ps("jaccard_listed_kernel<1>", stream);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(jaccard_listed_kernel<1>), grid_of(28), dim3(kTierWaves[1] * kWave), 0, stream, v1, v2, width, values, lists);
-  }
-  {
-    ProfileScope ps("jaccard_listed_kernel<2>", stream);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(jaccard_listed_kernel<2>), grid_of(12), dim3(kTierWaves[2] * kWave), 0, stream, v1, v2, width, values, lists);
-  }
-  {
-    ProfileScope ps("jaccard_listed_kernel<3>", stream);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(jaccard_listed_kernel<3>), grid_of(8), dim3(kTierWaves[3] * kWave), 0, stream, v1, v2, width, values, lists);
-  }
-  {
-    ProfileScope ps("jaccard_listed_kernel<4>", stream);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(jaccard_listed_kernel<4>), grid_of(4), dim3(kTierWaves[4] * kWave), 0, stream, v1, v2, width, values, lists);
-  }
-  {
-    ProfileScope ps("jaccard_parts_kernel", stream);
-    hipLaunchKernelGGL(jaccard_parts_kernel, dim3(grid_of(1).x, static_cast<unsigned>(kMaxParts)), dim3(kTierWaves[kPartsTier] * kWave), 0, stream, v1,
-                       v2, width, values, lists);
-  }
   if (with_mask) {
     int32_t const words = (rows + 31) / 32;
     hipLaunchKernelGGL(and_bitmask_kernel, dim3((words + 255) / 256), dim3(256), 0, stream, out->null_mask,
@@ -636,15 +621,48 @@ nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* inpu
   }
   // what the host has to know: the header of the lists
   uint32_t copied[kListHeader] = {};
-  const uint32_t* head         = copied;
-  hipError_t e                 = hipSuccess;
-  if (uint64_t* const pinned = host_scalars()) {
-    hipLaunchKernelGGL(publish_header_kernel, dim3(1), dim3(kListHeader), 0, stream, lists, reinterpret_cast<uint32_t*>(pinned));
-    head = reinterpret_cast<const uint32_t*>(pinned);
-  } else {
-    e = hipMemcpyAsync(copied, lists, sizeof(copied), hipMemcpyDeviceToHost, stream);
+  uint64_t* const pinned       = host_scalars();
+  const uint32_t* const head   = pinned ? reinterpret_cast<const uint32_t*>(pinned) : copied;
+  auto const read_header       = [&]() -> hipError_t {
+    if (!pinned) {
+      hipError_t const e = hipMemcpyAsync(copied, lists, sizeof(copied), hipMemcpyDeviceToHost, stream);
+      return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+    }
+    HostPost const post = new_post();
+    hipLaunchKernelGGL(publish_header_kernel, dim3(1), dim3(kListHeader), 0, stream, lists, reinterpret_cast<uint32_t*>(pinned), post);
+    hipError_t const e = hipGetLastError();
+    return e == hipSuccess ? wait_for_post(post, stream) : e;
+  };
+  // In a column of few pairs the launches of the other kernels, most of which would find their lists empty, are more than
+  // the work: the host looks at the lists first and launches what has something to do (7 pairs of 300 bytes 48 -> 20 us).
+  // In a larger one the wait costs more than a few empty launches.
+  bool const look   = rows <= kLookRows;
+  hipError_t e      = look ? read_header() : hipSuccess;
+  auto const listed = [&](int list) { return look ? static_cast<int32_t>(head[list]) : rows; };
+  auto const grid_of = [&](int list, int per_cu) { return dim3(static_cast<unsigned>(std::min<int64_t>(listed(list), static_cast<int64_t>(cus) * per_cu))); };
+  if (e == hipSuccess && listed(0) > 0) {
+    ProfileScope ps("jaccard_listed_kernel<1>", stream);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(jaccard_listed_kernel<1>), grid_of(0, 28), dim3(kTierWaves[1] * kWave), 0, stream, v1, v2, width, values, lists);
   }
-  if (e == hipSuccess) e = hipStreamSynchronize(stream);
+  if (e == hipSuccess && listed(1) > 0) {
+    ProfileScope ps("jaccard_listed_kernel<2>", stream);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(jaccard_listed_kernel<2>), grid_of(1, 12), dim3(kTierWaves[2] * kWave), 0, stream, v1, v2, width, values, lists);
+  }
+  if (e == hipSuccess && listed(2) > 0) {
+    ProfileScope ps("jaccard_listed_kernel<3>", stream);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(jaccard_listed_kernel<3>), grid_of(2, 8), dim3(kTierWaves[3] * kWave), 0, stream, v1, v2, width, values, lists);
+  }
+  if (e == hipSuccess && listed(3) > 0) {
+    ProfileScope ps("jaccard_listed_kernel<4>", stream);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(jaccard_listed_kernel<4>), grid_of(3, 4), dim3(kTierWaves[4] * kWave), 0, stream, v1, v2, width, values, lists);
+  }
+  bool const in_parts = listed(kPartsList) > 0;
+  if (e == hipSuccess && in_parts) {
+    ProfileScope ps("jaccard_parts_kernel", stream);
+    hipLaunchKernelGGL(jaccard_parts_kernel, dim3(grid_of(kPartsList, 1).x, static_cast<unsigned>(kMaxParts)), dim3(kTierWaves[kPartsTier] * kWave), 0, stream,
+                       v1, v2, width, values, lists);
+  }
+  if (e == hipSuccess && in_parts) e = read_header();  // (a part can turn out too full: its pair is then on the list of the last kernel)
   if (e != hipSuccess) {
     nvtext_amd_fixed_column_free(out, stream_, mr_);
     return fail(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));

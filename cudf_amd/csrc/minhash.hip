@@ -617,17 +617,20 @@ struct RowParts {
   __device__ __forceinline__ int64_t part() const
   {
     if (alone >= 0) return Source::kPart;
-    int64_t const share  = source.total() / waves;
+    int64_t const share  = static_cast<int64_t>(static_cast<double>(source.total()) / waves);  // (whole division of 64 bits: a hundred instructions)
     int64_t const length = ((share < 4 * Source::kMinPart ? share : share / 4) + kWave) / kWave * kWave;
     return min(max(length, Source::kMinPart), Source::kPart);
   }
+  // ... of a row of length n that is not null
+  __device__ __forceinline__ uint32_t parts_of(int64_t n, uint32_t length) const
+  {
+    if (n <= alone) return 0;
+    if (n > 0xFFFFFFFFll) return static_cast<uint32_t>((n - 1) / length + 1);
+    return n == 0 ? 1u : (static_cast<uint32_t>(n) - 1u) / length + 1u;
+  }
   __device__ __forceinline__ uint64_t operator()(int64_t i) const
   {
-    if (!source.valid(i)) return 0;
-    int64_t const n = source.length(i);
-    if (n <= alone) return 0;
-    int64_t const length = part();
-    return n == 0 ? 1 : static_cast<uint64_t>((n + length - 1) / length);
+    return source.valid(i) ? parts_of(source.length(i), static_cast<uint32_t>(part())) : 0u;
   }
 };
 
@@ -782,9 +785,11 @@ __global__ void __launch_bounds__(kWave) minhash64_prepare_kernel(const uint64_t
 // Everything that comes before the hashing of a column of few rows, in one launch: workgroup 0 counts the parts of the
 // rows (and finds the rows' places in the result where some are null), the others write the places where none is and
 // fill the result; the wavefronts of the workgroups from `fillers` + 1 on lay out the parameters of 64-bit hashes.
-constexpr int32_t kPlanRows = kScanSmallTiles * kScanTile;
+constexpr int kPlanThreads  = 1024;
+constexpr int kPlanItems    = 4;
+constexpr int32_t kPlanRows = 2 * kPlanThreads * kPlanItems;
 template <typename Source, typename T = typename Source::T>
-__global__ void __launch_bounds__(kScanThreads) minhash_plan_kernel(RowParts<Source> parts, Params<T> params, filter64::Group* groups, unsigned fillers,
+__global__ void __launch_bounds__(kPlanThreads) minhash_plan_kernel(RowParts<Source> parts, Params<T> params, filter64::Group* groups, unsigned fillers,
                                                                     int32_t* __restrict__ out_offsets, uint32_t* __restrict__ prefix,
                                                                     unsigned long long* __restrict__ counter, T* __restrict__ out, int64_t out_size)
 {
@@ -792,34 +797,42 @@ __global__ void __launch_bounds__(kScanThreads) minhash_plan_kernel(RowParts<Sou
   int32_t const P    = params.count;
   if constexpr (sizeof(T) == 8) {
     if (blockIdx.x > fillers) {
-      int32_t const group = static_cast<int32_t>((blockIdx.x - fillers - 1) * (kScanThreads / kWave) + threadIdx.x / kWave);
+      int32_t const group = static_cast<int32_t>((blockIdx.x - fillers - 1) * (kPlanThreads / kWave) + threadIdx.x / kWave);
       if (group < groups_of(P)) filter64::prepare_group(params.a, params.b, P, group, &groups[group], lane_id());
       return;
     }
   }
   if (blockIdx.x > 0) {
-    int64_t const first  = static_cast<int64_t>(blockIdx.x - 1) * kScanThreads + threadIdx.x;
-    int64_t const stride = static_cast<int64_t>(fillers) * kScanThreads;
+    int64_t const first  = static_cast<int64_t>(blockIdx.x - 1) * kPlanThreads + threadIdx.x;
+    int64_t const stride = static_cast<int64_t>(fillers) * kPlanThreads;
     if (!parts.source.masked())
       for (int64_t i = first; i <= rows; i += stride) out_offsets[i] = static_cast<int32_t>(i * P);
     for (int64_t i = first; i < out_size; i += stride) out[i] = std::numeric_limits<T>::max();
     return;
   }
-  __shared__ uint64_t lds[kScanThreads / kWave + 1];
-  uint64_t carry = 0;  // parts in the low half, valid rows in the high half
-  for (int32_t tile = 0; tile < rows; tile += kScanTile) {
-    int32_t const base = tile + static_cast<int32_t>(threadIdx.x) * kScanItems;
-    uint64_t vals[kScanItems], sum = 0;
+  __shared__ uint64_t lds[kPlanThreads / kWave + 1];
+  uint32_t const length = static_cast<uint32_t>(parts.part());
+  uint64_t carry        = 0;  // parts in the low half, valid rows in the high half
+  for (int32_t tile = 0; tile < rows; tile += kPlanThreads * kPlanItems) {
+    int32_t const base = tile + static_cast<int32_t>(threadIdx.x) * kPlanItems;
+    int64_t n[kPlanItems];
+    bool valid[kPlanItems];
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
-      bool const in = base + k < rows;
-      vals[k]       = in ? parts(base + k) | (static_cast<uint64_t>(parts.source.valid(base + k)) << 32) : 0;
+    for (int k = 0; k < kPlanItems; ++k) {  // (without a branch: all loads in flight together)
+      int32_t const i = min(base + k, rows - 1);
+      n[k]            = parts.source.length(i);
+      valid[k]        = parts.source.valid(i) && base + k < rows;
+    }
+    uint64_t vals[kPlanItems], sum = 0;
+#pragma unroll
+    for (int k = 0; k < kPlanItems; ++k) {
+      vals[k] = valid[k] ? parts.parts_of(n[k], length) | (1ull << 32) : 0ull;
       sum += vals[k];
     }
     uint64_t total;
-    uint64_t run = block_exclusive_scan64<kScanThreads>(sum, lds, &total) + carry;
+    uint64_t run = block_exclusive_scan64<kPlanThreads>(sum, lds, &total) + carry;
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
+    for (int k = 0; k < kPlanItems; ++k) {
       if (base + k < rows) {
         prefix[base + k] = static_cast<uint32_t>(run);
         if (parts.source.masked()) out_offsets[base + k] = static_cast<int32_t>(run >> 32) * P;
@@ -925,9 +938,9 @@ void run_minhash(Source const& source, int32_t rows, bool masked, const T* a, co
   auto* const counter = reinterpret_cast<unsigned long long*>(scan_tmp) + scan_temp_bytes(rows) / sizeof(uint64_t);
   if (rows <= kPlanRows) {
     int64_t const most    = std::max<int64_t>(child_size, rows + 1);
-    unsigned const fillers = static_cast<unsigned>(std::min<int64_t>((most + 4 * kScanThreads - 1) / (4 * kScanThreads), 1024));
-    unsigned const layers  = sizeof(T) == 8 ? static_cast<unsigned>((groups_of(P) + kScanThreads / kWave - 1) / (kScanThreads / kWave)) : 0u;
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_plan_kernel<Source>), dim3(1 + fillers + layers), dim3(kScanThreads), 0, stream, parts, params, laid_out,
+    unsigned const fillers = static_cast<unsigned>(std::min<int64_t>((most + 4 * kPlanThreads - 1) / (4 * kPlanThreads), 256));
+    unsigned const layers  = sizeof(T) == 8 ? static_cast<unsigned>((groups_of(P) + kPlanThreads / kWave - 1) / (kPlanThreads / kWave)) : 0u;
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_plan_kernel<Source>), dim3(1 + fillers + layers), dim3(kPlanThreads), 0, stream, parts, params, laid_out,
                        fillers, offsets, prefix, counter, child, child_size);
   } else {
     if (masked) {

@@ -628,7 +628,7 @@ __global__ void __launch_bounds__(kNormThreads, 4) normalize_count_small_kernel(
 // byte, byte past the last, bytes of the result}.
 constexpr int kFinishThreads = 1024;
 __global__ void __launch_bounds__(kFinishThreads) normalize_finish_kernel(ColView col, int64_t most_bytes, const uint32_t* __restrict__ tile_bytes,
-                                                                          uint64_t* __restrict__ tile_offset, uint64_t* __restrict__ dst)
+                                                                          uint64_t* __restrict__ tile_offset, uint64_t* __restrict__ dst, HostPost post)
 {
   __shared__ uint64_t lds[kFinishThreads / kWave + 1];
   int64_t const first = col.off(0), last = col.off(col.size), n = last - first;
@@ -656,6 +656,7 @@ __global__ void __launch_bounds__(kFinishThreads) normalize_finish_kernel(ColVie
     dst[0] = static_cast<uint64_t>(first);
     dst[1] = static_cast<uint64_t>(last);
     dst[2] = carry;
+    post.send();
   }
 }
 
@@ -1038,17 +1039,18 @@ nvtext_amd_status nvtext_amd_normalize_characters(const nvtext_amd_strings_colum
   int64_t first = 0, last = 0;
   uint64_t total = 0;
   if (scalars) {
+    HostPost const post = new_post();
     if (small) {
       unsigned const grid = static_cast<unsigned>(std::min<size_t>(small_tiles, static_cast<size_t>(device_cus()) * 16));
       hipLaunchKernelGGL(normalize_count_small_kernel, dim3(grid), dim3(kNormThreads), 0, stream, view, small_bytes, tables, small_temps.part<uint32_t>(0),
                          small_temps.part<int32_t>(2));
       hipLaunchKernelGGL(normalize_finish_kernel, dim3(1), dim3(kFinishThreads), 0, stream, view, small_bytes, small_temps.part<uint32_t>(0),
-                         small_temps.part<uint64_t>(1), scalars);
+                         small_temps.part<uint64_t>(1), scalars, post);
     } else {
-      launch_read_two_offsets(input->offsets, input->offsets_is_int64 != 0, input->offset, static_cast<int64_t>(input->offset) + rows, scalars, stream);
+      launch_read_two_offsets(input->offsets, input->offsets_is_int64 != 0, input->offset, static_cast<int64_t>(input->offset) + rows, scalars, post, stream);
     }
     NVTEXT_HIP_TRY(hipGetLastError());
-    NVTEXT_HIP_TRY(hipStreamSynchronize(stream));
+    NVTEXT_HIP_TRY(wait_for_post(post, stream));
     first = static_cast<int64_t>(scalars[0]);
     last  = static_cast<int64_t>(scalars[1]);
     total = scalars[2];
@@ -1116,12 +1118,14 @@ nvtext_amd_status nvtext_amd_normalize_characters(const nvtext_amd_strings_colum
                        tile_row);
     device_exclusive_scan(TileBytes{tile_bytes}, tiles, tile_offset, temps.part<uint64_t>(2), stream);
     if (scalars) {
-      launch_publish(tile_offset + tiles, scalars, stream);
+      HostPost const post = new_post();
+      launch_publish(tile_offset + tiles, scalars, post, stream);
       e = hipGetLastError();
+      if (e == hipSuccess) e = wait_for_post(post, stream);
     } else {
       e = hipMemcpyAsync(&total, tile_offset + tiles, sizeof(total), hipMemcpyDeviceToHost, stream);
+      if (e == hipSuccess) e = hipStreamSynchronize(stream);
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(stream);
     if (e != hipSuccess) return release(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
     if (scalars) total = scalars[0];
   }

@@ -1889,8 +1889,7 @@ constexpr int kSampleBytes   = 512;
 constexpr int kSampleTail    = 208;  // bytes staged past a window: a word that starts in it ends there, or is kMaxWord bytes or more
 static_assert(3 * kSampleWindows <= kHostSampleWords, "a window's three counts fit the pinned words");
 
-// (skip_bytes: a column of at most so many bytes is not sampled)
-__global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, VocabTable table, int64_t skip_bytes, uint64_t* __restrict__ first_last,
+__global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, VocabTable table, uint64_t* __restrict__ first_last,
                                                                uint32_t* __restrict__ counts)
 {
   __shared__ uint32_t staged[(kSampleBytes + kSampleTail + 8) / 4 + 4];  // byte 4 + x of it: byte x of the window; byte 3: the one before
@@ -1901,7 +1900,6 @@ __global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, Vo
     first_last[1] = static_cast<uint64_t>(last);
   }
   int64_t const span    = last - first;
-  if (span <= skip_bytes) return;
   int64_t const windows = min(static_cast<int64_t>(kSampleWindows), (span + kSampleBytes - 1) / kSampleBytes);
   uint32_t words = 0, queued = 0, bytes = 0;
   if (static_cast<int64_t>(blockIdx.x) < windows) {
@@ -1950,25 +1948,28 @@ __global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, Vo
 
 // What the host needs to know before the emit pass: the number of tokens, whether a range ran out of word slots, the
 // queue entries reserved.
-__global__ void publish_state_kernel(const uint64_t* __restrict__ total, const uint32_t* __restrict__ flags, uint64_t* __restrict__ dst)
+__global__ void publish_state_kernel(const uint64_t* __restrict__ total, const uint32_t* __restrict__ flags, uint64_t* __restrict__ dst,
+                                     HostPost post)
 {
-  if (threadIdx.x == 0) dst[0] = *total;
-  if (threadIdx.x == 1) dst[1] = flags[kFlagOverflow];
-  if (threadIdx.x == 2) dst[2] = flags[kFlagQueueSize];
+  dst[0] = *total;
+  dst[1] = flags[kFlagOverflow];
+  dst[2] = flags[kFlagQueueSize];
+  post.send();
 }
 
-// The same, and the places of the ranges' tokens, after the one launch for a small column: one workgroup.  dst[0] = the
-// number of tokens, dst[1] = the ranges' notes together.
+// The same, and the places of the ranges' tokens, after the one launch for a small column: one workgroup.  dst = the view's
+// first and last offset, the number of tokens, the ranges' notes together (the last two mean nothing where the column is
+// not small).
 constexpr int kFinishThreads = 1024;
 __global__ void __launch_bounds__(kFinishThreads) wordpiece_finish_kernel(TileArgs a, int tile, int64_t* __restrict__ bases, uint32_t* __restrict__ again_count,
-                                                                          uint64_t* __restrict__ dst)
+                                                                          uint64_t* __restrict__ dst, HostPost post)
 {
   __shared__ uint64_t lds[kFinishThreads / kWave + 1];
   __shared__ uint32_t all_notes;
   int64_t const first_offset = a.col.off(0), bytes = a.col.off(a.col.size) - first_offset;
-  if (bytes <= 0 || bytes > a.most_bytes) return;
+  bool const small     = bytes > 0 && bytes <= a.most_bytes;
   int64_t const cbeg   = static_cast<int64_t>(reinterpret_cast<uintptr_t>(a.col.chars + first_offset) & 15u);
-  uint32_t const n     = static_cast<uint32_t>((cbeg + bytes + tile - 1) / tile);
+  uint32_t const n     = small ? static_cast<uint32_t>((cbeg + bytes + tile - 1) / tile) : 0u;
   uint32_t notes = 0;
   uint64_t carry = 0;
   if (threadIdx.x == 0) all_notes = 0;
@@ -1996,8 +1997,11 @@ __global__ void __launch_bounds__(kFinishThreads) wordpiece_finish_kernel(TileAr
   __syncthreads();
   if (threadIdx.x == 0) {
     *again_count = 0;
-    dst[0]       = carry;
-    dst[1]       = all_notes;
+    dst[0]       = static_cast<uint64_t>(first_offset);
+    dst[1]       = static_cast<uint64_t>(first_offset + bytes);
+    dst[2]       = carry;
+    dst[3]       = all_notes;
+    post.send();
   }
 }
 
@@ -2440,8 +2444,8 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   bool const limit = max_words_per_row > 0;
   // A column of few rows is probably small, and then the call is launches and waits more than work: everything up to the
   // number of tokens is put on the stream at once, for a column of up to kSmallRowBytes bytes a row and kSmallBytes in all,
-  // before the host knows how many bytes there are.  Where there are more, these kernels leave at once, the sample that
-  // follows them does what it does for a large column, and the call goes on from there.
+  // before the host knows how many bytes there are.  Where there are more, these kernels leave at once and the call goes on
+  // as for a large column.
   // (29 rows of 180 bytes: 87 us in eleven launches with two waits, 43 us in four with one; 32,768 rows of 120 bytes
   // 145 -> 60 us)
   bool const small = scalars && sampling && rows <= kSmallRows && g_forced_range_tiles.load(std::memory_order_relaxed) == 0;
@@ -2455,11 +2459,9 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
                                       (static_cast<size_t>(small_ranges) + 1) * sizeof(int64_t),
                                       (static_cast<size_t>(small_ranges) * kSmallQueue + 1) * sizeof(uint32_t),
                                       static_cast<size_t>(small_ranges) * kSmallQueue * sizeof(OovEntry)};
-  bool tried = false;
   if (small) {
     TempParts<8> const temps(mr, small_temp_bytes);
     if (temps.ok()) {
-      tried = true;
       TileArgs args{};
       args.col           = v;
       args.table         = vocabulary->table;
@@ -2482,11 +2484,10 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
         ProfileScope ps("wordpiece_word_kernel (small column)", stream);
         hipLaunchKernelGGL(kernel, dim3(std::min((small_ranges + kTokWaves - 1) / kTokWaves, kSmallGrid)), dim3(kTokThreads), 0, stream, args);
       }
-      hipLaunchKernelGGL(wordpiece_finish_kernel, dim3(1), dim3(kFinishThreads), 0, stream, args, kSmallTile, bases, again_count, scalars + 2);
-      hipLaunchKernelGGL(wordpiece_sample_kernel, dim3(kSampleWindows), dim3(kWave), 0, stream, v, vocabulary->table, small_bytes, scalars,
-                         reinterpret_cast<uint32_t*>(scalars + 8));
+      HostPost const post = new_post();
+      hipLaunchKernelGGL(wordpiece_finish_kernel, dim3(1), dim3(kFinishThreads), 0, stream, args, kSmallTile, bases, again_count, scalars, post);
       hipError_t e = hipGetLastError();
-      if (e == hipSuccess) e = hipStreamSynchronize(stream);
+      if (e == hipSuccess) e = wait_for_post(post, stream);
       if (e != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
       first_offset = static_cast<int64_t>(scalars[0]);
       last_offset  = static_cast<int64_t>(scalars[1]);
@@ -2513,17 +2514,15 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
       }
     }  // (no room for the temporaries of the largest column that it might be: as for a large column)
   }
-  bool const have_sample = tried && last_offset - first_offset > small_bytes;
   if (scalars) {
     uint32_t* const counts = reinterpret_cast<uint32_t*>(scalars + 8);
-    if (have_sample) {
-      // (the two offsets as well)
-    } else if (sampling)
-      hipLaunchKernelGGL(wordpiece_sample_kernel, dim3(kSampleWindows), dim3(kWave), 0, stream, v, vocabulary->table, int64_t{-1}, scalars, counts);
+    HostPost const post    = new_post();
+    if (sampling)
+      hipLaunchKernelGGL(wordpiece_sample_kernel, dim3(kSampleWindows), dim3(kWave), 0, stream, v, vocabulary->table, scalars, counts);
     else
-      launch_read_two_offsets(input->offsets, input->offsets_is_int64 != 0, input->offset, static_cast<int64_t>(input->offset) + rows, scalars, stream);
+      launch_read_two_offsets(input->offsets, input->offsets_is_int64 != 0, input->offset, static_cast<int64_t>(input->offset) + rows, scalars, post, stream);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess && !have_sample) e = hipStreamSynchronize(stream);
+    if (e == hipSuccess) e = sampling ? hipStreamSynchronize(stream) : wait_for_post(post, stream);
     if (e != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
     first_offset = static_cast<int64_t>(scalars[0]);
     last_offset  = static_cast<int64_t>(scalars[1]);
@@ -2682,12 +2681,13 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     // (cpp/include/cudf/detail/sizes_to_offsets_iterator.cuh:302-339)
     device_exclusive_scan(RangeTokensOf{tokens}, static_cast<int64_t>(nranges), bases, scan_tmp, stream);
     // the total (the last word of the scan's temporaries) and the first flag words: written to the pinned words by a
-    // kernel of one wavefront, or, without those, fetched in one copy (the flags lie right behind the scan's temporaries)
+    // kernel of one thread, or, without those, fetched in one copy (the flags lie right behind the scan's temporaries)
     uint32_t state[3] = {0, 0, 0};
     if (scalars) {
-      hipLaunchKernelGGL(publish_state_kernel, dim3(1), dim3(kWave), 0, stream, scan_tmp + scan_tiles(nranges), flags, scalars + 2);
+      HostPost const post = new_post();
+      hipLaunchKernelGGL(publish_state_kernel, dim3(1), dim3(1), 0, stream, scan_tmp + scan_tiles(nranges), flags, scalars + 2, post);
       hipError_t e = hipGetLastError();
-      if (e == hipSuccess) e = hipStreamSynchronize(stream);
+      if (e == hipSuccess) e = wait_for_post(post, stream);
       if (e != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
       total    = scalars[2];
       state[1] = static_cast<uint32_t>(scalars[3]);
