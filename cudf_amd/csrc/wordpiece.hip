@@ -167,6 +167,8 @@ namespace {
 
 constexpr int kTokWaves     = 4;
 constexpr int kTokThreads   = kTokWaves * kWave;
+// (word pass: two workgroups to a CU, six wavefronts per SIMD, that share the words in LDS; the launch for a small column is too short for those)
+constexpr int word_waves(bool small) { return small ? kTokWaves : 12; }
 constexpr int32_t kNone     = std::numeric_limits<int32_t>::min();
 constexpr int kOovKeep      = 7;     // tokens of an out-of-vocabulary word that are kept while it is tokenized
 // ------------------------------------------------------------------ where candidate keys live
@@ -860,10 +862,16 @@ struct TileArgs {
   uint32_t* counter;       // next range to hand out
   uint32_t* overflow;      // set when a range has more words than range_cap
   // one launch for all (INLINE): the most bytes it is for, and what it leaves in place of the counters and flags
+  const uint32_t* hot;     // slots of words that the sample found, kHotWords of them (nullptr: none)
   int64_t most_bytes;
   uint32_t* first_row_out; // as range_first_row
   uint32_t* range_notes;   // per range: kNoteSpill, kNoteAgain
 };
+// Words that the sample of the column met and found in the vocabulary, a wavefront's neighbours' and its own: text repeats
+// its frequent words, the first-level cache keeps the lines of few of them (a line of the table has four buckets, most of
+// them of rare words), and the word pass is bound by that cache and by the address unit before it (93 % busy).  Kept in
+// LDS, by the home bucket: whoever was met last, which is the more frequent word more often than not.
+constexpr uint32_t kHotWords = 512;
 constexpr uint32_t kNoteSpill = 1u;  // more words than range_cap, or more of them not in the vocabulary than queue_cap
 constexpr uint32_t kNoteAgain = 2u;  // a word of more tokens than a queue record keeps
 
@@ -982,8 +990,9 @@ __global__ void range_first_row_kernel(ColView col, int64_t first_offset, uint32
 // tokenizes the words that are not in the vocabulary itself, lanes <-> words, into the range's own part of the queue
 // (queue_cap records), where the other way leaves the out-of-vocabulary pass to put its results.
 template <int TILE, bool IS64, bool LIMIT, bool INLINE>
-__global__ void __launch_bounds__(kTokThreads, INLINE ? 4 : 6) wordpiece_word_kernel(TileArgs a)
+__global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wordpiece_word_kernel(TileArgs a)
 {
+  constexpr int kWaves = word_waves(INLINE);
   if constexpr (INLINE) {
     int64_t const first_offset = a.col.off(0), bytes = a.col.off(a.col.size) - first_offset;
     if (bytes <= 0 || bytes > a.most_bytes) return;
@@ -1000,9 +1009,22 @@ __global__ void __launch_bounds__(kTokThreads, INLINE ? 4 : 6) wordpiece_word_ke
   constexpr int kSubs         = kBlocks / kWave;
   constexpr uint32_t kWordCap = TileLds<TILE>::kWordCap;
   static_assert(kBlocks % kWave == 0, "whole wavefronts of blocks");
-  __shared__ TileLds<TILE> lds_all[kTokWaves];
+  __shared__ TileLds<TILE> lds_all[kWaves];
   __shared__ uint4 trim[17];
+  __shared__ uint4 hot[INLINE ? 1 : kHotWords];  // the key (at most 8 bytes), its id, its length
   fill_trim_table(trim);
+  if constexpr (!INLINE) {
+    for (uint32_t i = threadIdx.x; i < kHotWords; i += kWaves * kWave) {
+      uint4 v = make_uint4(0u, 0u, 0u, 0u);
+      if (a.hot) {
+        // (an entry that the sample left unwritten names any slot: a slot is a key and its id wherever it lies)
+        uint4 const slot = a.table.slots[a.hot[i] & (2u * a.table.bucket_mask + 1u)];
+        uint32_t const len = slot.x & 0xFFu;
+        if (slot.x != 0 && (slot.x & 0x100u) == 0 && len <= 8) v = make_uint4(slot.z, slot.w, slot.y & ~kSearchOn, len);
+      }
+      hot[i] = v;
+    }
+  }
   __syncthreads();
   TileLds<TILE>& lds  = lds_all[threadIdx.x / kWave];
   int const lane      = lane_id();
@@ -1024,11 +1046,11 @@ __global__ void __launch_bounds__(kTokThreads, INLINE ? 4 : 6) wordpiece_word_ke
   uint32_t q_pos = 0, q_lim = 0;  // this wavefront's reserved queue entries [q_pos, q_lim)
   uint32_t inline_range = 0;
 
-  uint32_t const my_number = blockIdx.x * kTokWaves + threadIdx.x / kWave;
+  uint32_t const my_number = blockIdx.x * kWaves + threadIdx.x / kWave;
   for (bool first = true;; first = false) {
     uint32_t range;
     if constexpr (INLINE) {
-      range = first ? static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(my_number))) : inline_range + gridDim.x * kTokWaves;
+      range = first ? static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(my_number))) : inline_range + gridDim.x * kWaves;
       inline_range = range;
     } else {
       range = next_unit(a.counter, first, my_number, lane);
@@ -1321,8 +1343,8 @@ __global__ void __launch_bounds__(kTokThreads, INLINE ? 4 : 6) wordpiece_word_ke
           uint32_t const rec = lds.word[active ? k : 0u];
           uint32_t const s   = rec & 0xFFFFu;
           uint32_t const wl  = (rec >> 16) - s + 1u;
-          // straight-line code: every lane reads a bucket (of whatever its first bytes are), and what it makes of it
-          // depends on the word's length afterwards; only a key of 9 to 16 bytes with the right tag needs a second
+          // straight-line code: every lane whose word is not at hand reads a bucket (of whatever its first bytes are), and
+          // what it makes of it depends on the word's length afterwards; only a key of 9 to 16 bytes with the right tag needs a second
           // read, of the key's bytes
           TileWord const tw{lds.bytes, 16u + s};
           uint32_t head[4];
@@ -1342,10 +1364,25 @@ __global__ void __launch_bounds__(kTokThreads, INLINE ? 4 : 6) wordpiece_word_ke
           pr.want            = slot_word0(hp.tag, 0u, wl16);
           pr.fp              = hp.fp;
           pr.bucket          = hp.bucket;
-          uint4 const s0 = table.slots[2 * pr.bucket];
-          uint4 const s1 = table.slots[2 * pr.bucket + 1];
+          uint4 s0 = make_uint4(0u, 0u, 0u, 0u), s1 = s0, known_word = s0;
+          bool is_hot = false;
+          if constexpr (INLINE) {
+            s0 = table.slots[2 * pr.bucket];
+            s1 = table.slots[2 * pr.bucket + 1];
+          } else {
+            known_word = hot[pr.bucket & (kHotWords - 1u)];
+            is_hot     = known_word.x == pr.k0 && known_word.y == pr.k1 && known_word.w == wl;
+            if (active && !is_hot) {
+              s0 = table.slots[2 * pr.bucket];
+              s1 = table.slots[2 * pr.bucket + 1];
+            }
+          }
           int32_t id  = kNone;
           uint32_t vd = verdict(pr, s0, s1, wl16, &id);
+          if (is_hot) {
+            id = static_cast<int32_t>(known_word.z);
+            vd = 1u;
+          }
           if (vd == 2u && wl > 8 && wl <= 16) vd = verdict_16(table, pr, s0, s1, head, &id);
           bool const too_long = wl >= kMaxWord;  // wordpiece_tokenize.cu:442-445, 738-741: one unknown token
           bool const found    = wl <= 16 && vd == 1u;
@@ -1890,7 +1927,7 @@ constexpr int kSampleTail    = 208;  // bytes staged past a window: a word that 
 static_assert(3 * kSampleWindows <= kHostSampleWords, "a window's three counts fit the pinned words");
 
 __global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, VocabTable table, uint64_t* __restrict__ first_last,
-                                                               uint32_t* __restrict__ counts)
+                                                               uint32_t* __restrict__ counts, uint32_t* __restrict__ hot)
 {
   __shared__ uint32_t staged[(kSampleBytes + kSampleTail + 8) / 4 + 4];  // byte 4 + x of it: byte x of the window; byte 3: the one before
   int const lane      = lane_id();
@@ -1934,6 +1971,7 @@ __global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, Vo
       uint4 const s0 = table.slots[2 * pr.bucket], s1 = table.slots[2 * pr.bucket + 1];
       int32_t id;
       uint32_t vd = verdict(pr, s0, s1, len, &id);
+      if (vd == 1u) hot[pr.bucket & (kHotWords - 1u)] = 2u * pr.bucket + (s0.z == pr.k0 && s0.w == pr.k1 ? 0u : 1u);
       if (vd == 2u && len > 8) vd = verdict_16(table, pr, s0, s1, k, &id);
       if (vd != 1u) ++queued;
     }
@@ -2514,11 +2552,14 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
       }
     }  // (no room for the temporaries of the largest column that it might be: as for a large column)
   }
+  Temp const hot(mr, scalars && sampling ? kHotWords * sizeof(uint32_t) : 0);
+  if (!hot.ok()) return give_up(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");
   if (scalars) {
     uint32_t* const counts = reinterpret_cast<uint32_t*>(scalars + 8);
     HostPost const post    = new_post();
     if (sampling)
-      hipLaunchKernelGGL(wordpiece_sample_kernel, dim3(kSampleWindows), dim3(kWave), 0, stream, v, vocabulary->table, scalars, counts);
+      hipLaunchKernelGGL(wordpiece_sample_kernel, dim3(kSampleWindows), dim3(kWave), 0, stream, v, vocabulary->table, scalars, counts,
+                         hot.as<uint32_t>());
     else
       launch_read_two_offsets(input->offsets, input->offsets_is_int64 != 0, input->offset, static_cast<int64_t>(input->offset) + rows, scalars, post, stream);
     hipError_t e = hipGetLastError();
@@ -2579,12 +2620,13 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   };
   void (*const word_kernel)(TileArgs) = is64 ? (limit ? wordpiece_word_kernel<kTile, true, true, false> : wordpiece_word_kernel<kTile, true, false, false>)
                                              : (limit ? wordpiece_word_kernel<kTile, false, true, false> : wordpiece_word_kernel<kTile, false, false, false>);
-  int64_t const word_resident = resident(reinterpret_cast<const void*>(word_kernel), kTokThreads, (is64 ? 2 : 0) + (limit ? 1 : 0));
+  int64_t const word_resident = resident(reinterpret_cast<const void*>(word_kernel), word_waves(false) * kWave, (is64 ? 2 : 0) + (limit ? 1 : 0));
   // A range is what a wavefront works through by itself, one tile after the other: kRangeTiles tiles when that still
   // leaves every wavefront of the word pass eight ranges or more (the last ones then end close together), fewer in a
   // smaller column (2M rows of 120 bytes: 0.34 -> 0.30 ms for the word pass).
+  constexpr int kWordWaves = word_waves(false);
   int range_tiles = kRangeTiles;
-  while (range_tiles > 1 && ntiles / range_tiles < 8 * word_resident * kTokWaves) range_tiles >>= 1;
+  while (range_tiles > 1 && ntiles / range_tiles < 8 * word_resident * kWordWaves) range_tiles >>= 1;
   // (tests, which have no column of a gigabyte to give, set the size through nvtext_amd_profile_set_range_tiles)
   if (int const want = g_forced_range_tiles.load(std::memory_order_relaxed)) range_tiles = want;
   int64_t const kRange    = static_cast<int64_t>(kTile) * range_tiles;
@@ -2592,7 +2634,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   if (nranges64 > 0x7FFFFFF0) return give_up(NVTEXT_AMD_LOGIC_ERROR, "words exceed internal limit");
   uint32_t const nranges = static_cast<uint32_t>(nranges64);
   unsigned const word_grid = static_cast<unsigned>(
-    std::min<int64_t>((static_cast<int64_t>(nranges) + kTokWaves - 1) / kTokWaves, word_resident));
+    std::min<int64_t>((static_cast<int64_t>(nranges) + kWordWaves - 1) / kWordWaves, word_resident));
   unsigned const oov_grid  = static_cast<unsigned>(resident(reinterpret_cast<const void*>(wordpiece_oov_kernel), kOovThreads, 4));
   unsigned const emit_grid = static_cast<unsigned>(
     std::min<int64_t>((static_cast<int64_t>(nranges) + kTokWaves - 1) / kTokWaves, resident(reinterpret_cast<const void*>(wordpiece_emit_kernel), kTokThreads, 5)));
@@ -2608,6 +2650,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   args.nranges      = nranges;
   args.range_tiles  = range_tiles;
   args.max_words    = max_words_per_row;
+  args.hot          = hot.as<uint32_t>();
 
   // Word slots per range and queue entries.  A range of ordinary text has a word per five or six bytes, and about a
   // word in forty of a large column is not in the vocabulary; the first attempt has room for five words per sixteen
@@ -2615,7 +2658,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   // language than the vocabulary's) makes the attempt fail, and the second has what the first found to be needed:
   // room for a word per byte, the exact number of queue entries.
   uint32_t range_cap      = static_cast<uint32_t>(kRange * 5 / 16);
-  uint64_t queue_capacity = static_cast<uint64_t>((last_offset - first_offset) >> 5) + static_cast<uint64_t>(word_grid) * kTokWaves * kQueueChunk + 4096;
+  uint64_t queue_capacity = static_cast<uint64_t>((last_offset - first_offset) >> 5) + static_cast<uint64_t>(word_grid) * kWordWaves * kQueueChunk + 4096;
   if (sample_bytes > 0) {
     // what the sample calls for, with half as much again for the ranges that are denser than the column as a whole
     // (never less than the sizes above: a sample can miss; the second attempt remains)
@@ -2624,7 +2667,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     range_cap = static_cast<uint32_t>(std::min<double>(static_cast<double>(kRange + 8), std::max<double>(range_cap, per_byte_words * 1.5 * static_cast<double>(kRange) + 256)));
     range_cap = (range_cap + 1u) & ~1u;  // (a range's slots begin at an even index)
     queue_capacity = std::max<uint64_t>(queue_capacity, static_cast<uint64_t>(per_byte_queued * 1.25 * static_cast<double>(last_offset - first_offset)) +
-                                                          static_cast<uint64_t>(word_grid) * kTokWaves * kQueueChunk + 4096);
+                                                          static_cast<uint64_t>(word_grid) * kWordWaves * kQueueChunk + 4096);
   }
   uint64_t total = 0;
   for (int attempt = 0;; ++attempt) {
@@ -2662,10 +2705,10 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     args.counter         = flags + kFlagWordUnits;
     args.overflow        = flags + kFlagOverflow;
     hipLaunchKernelGGL(range_first_row_kernel, dim3((nranges + 1 + 255) / 256), dim3(256), 0, stream, v, first_offset, cbeg, kRange, nranges, first_row,
-                       flags, word_grid * kTokWaves, oov_grid * kOovWaves);
+                       flags, word_grid * kWordWaves, oov_grid * kOovWaves);
     {
       ProfileScope ps("wordpiece_word_kernel", stream);
-      hipLaunchKernelGGL(word_kernel, dim3(word_grid), dim3(kTokThreads), 0, stream, args);
+      hipLaunchKernelGGL(word_kernel, dim3(word_grid), dim3(kWordWaves * kWave), 0, stream, args);
     }
     {
       ProfileScope ps("wordpiece_oov_kernel", stream);
@@ -2710,7 +2753,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
       // state[2] counts the chunks of kQueueChunk entries that the wavefronts reserved, the unused rest of each
       // wavefront's last chunk included; which ranges a wavefront gets differs from one attempt to the next, and with it
       // that rest: a chunk per wavefront on top of what this attempt reserved covers every assignment.
-      queue_capacity = std::max<uint64_t>(queue_capacity, static_cast<uint64_t>(state[2]) + static_cast<uint64_t>(word_grid) * kTokWaves * kQueueChunk);
+      queue_capacity = std::max<uint64_t>(queue_capacity, static_cast<uint64_t>(state[2]) + static_cast<uint64_t>(word_grid) * kWordWaves * kQueueChunk);
       continue;
     }
     if (total > static_cast<uint64_t>(std::numeric_limits<int32_t>::max())) return give_up(NVTEXT_AMD_OVERFLOW, "Size of output exceeds the column size limit");
