@@ -227,27 +227,6 @@ struct TileWord {
   }
 };
 
-// A word in global memory (emit pass, rare path).  key8 reads only aligned dwords that overlap the key.
-struct GlobalWord {
-  const uint8_t* p;
-  __device__ __forceinline__ uint32_t byte(uint32_t k) const { return p[k]; }
-  __device__ __forceinline__ void key8(uint32_t off, uint32_t len, uint32_t* k0, uint32_t* k1) const
-  {
-    const uint8_t* q    = p + off;
-    uint32_t const mis  = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(q) & 3u);
-    const uint32_t* a   = reinterpret_cast<const uint32_t*>(q - mis);
-    uint32_t const need = mis + (len < 8 ? len : 8);  // bytes from the aligned base
-    uint32_t const d0   = a[0];
-    uint32_t const d1   = need > 4 ? a[1] : 0u;
-    uint32_t const d2   = need > 8 ? a[2] : 0u;
-    uint32_t lo         = __builtin_amdgcn_alignbit(d1, d0, mis * 8u);
-    uint32_t hi         = __builtin_amdgcn_alignbit(d2, d1, mis * 8u);
-    trim_key8(len, lo, hi);
-    *k0 = lo;
-    *k1 = hi;
-  }
-};
-
 // A candidate key, ready to be probed: its first block (trimmed), tag word and home bucket.
 struct Probe {
   uint32_t k0, k1;  // key bytes [0, 8), zero padded
@@ -564,20 +543,6 @@ __device__ __forceinline__ uint32_t tokenize_oov_word(VocabTable const& t, W con
   return st.count;
 }
 
-// The same, out of line, for the callers' rare cases: the number of tokens of a word staged in LDS, and the tokens
-// of a word in memory written to dst[0 .. cnt) (cnt = the number counted before).
-__device__ __forceinline__ uint32_t count_oov_tokens(VocabTable const& t, const uint32_t* bytes, uint32_t start, uint32_t len)
-{
-  return tokenize_oov_word(t, TileWord{bytes, start}, len, [](uint32_t, int32_t) {});
-}
-__device__ __forceinline__ void write_oov_tokens(VocabTable const& t, const uint8_t* p, uint32_t len, uint32_t* dst, uint32_t cnt)
-{
-  tokenize_oov_word(t, GlobalWord{p}, len, [&](uint32_t j, int32_t id) {
-    if (j < cnt) dst[j] = static_cast<uint32_t>(id);
-  });
-}
-
-
 // Bit 7 of every byte of x that is a UTF-8 continuation byte (10xxxxxx); exact, no carries cross bytes.
 __device__ __forceinline__ uint32_t continuation_bytes(uint32_t x)
 {
@@ -827,6 +792,35 @@ struct OovResult {
 static_assert(sizeof(OovEntry) == 32 && sizeof(OovResult) == 32, "a queue record is two 16-byte stores");
 constexpr uint32_t kUnprobed = 0x100u;  // the word has not been looked up whole (more than 16 bytes; a key that may have been carried past its bucket)
 
+// The memo of a large column: text repeats its unknown words too.  The first ranges of the column (kMemoBytes) go through
+// the word pass and the out-of-vocabulary pass by themselves; their words that are not in the vocabulary, with the tokens
+// those passes found, are then a table that the word pass of the other ranges looks into, so that a word met before costs
+// one read of sixteen bytes and neither a queue record nor its pieces again.  An entry is the word's first twelve bytes
+// (longer ones are left out) and its length (0: none), the number of its tokens and where its result lies, behind the
+// queue's records, so that a word's slot names it as it names a queue record.  Of several words with one place the last
+// to ask has it, the more frequent one more often than not; a second place for each would cost every word a second
+// scattered read and save as much of the out-of-vocabulary pass.
+// (2 M rows of 256 bytes, 15 % of their words unknown, 40,000 different ones of those: 1463 -> 1244 us.)
+constexpr uint32_t kMemoBits    = 17;
+constexpr uint32_t kMemoEntries = 1u << kMemoBits;
+constexpr uint32_t kMemoWord    = 12;
+constexpr int64_t kMemoBytes    = 16 << 20;
+constexpr int64_t kMemoLeast    = 128 << 20;  // smaller columns: the second launches cost what the memo saves
+__device__ __forceinline__ uint32_t memo_place(uint64_t key_hash)
+{
+  uint32_t const x = (static_cast<uint32_t>(key_hash) * 0xC2B2AE35u + static_cast<uint32_t>(key_hash >> 32)) * 0x9E3779B1u;
+  return x >> (32u - kMemoBits);
+}
+// Whether the words of the first ranges repeat enough: words asked for places, and got so many between them.  (With most
+// of the places taken there may be any number of different words.)
+__device__ __forceinline__ bool memo_pays(uint32_t words, uint32_t places) { return words > 3u * places && places < kMemoEntries / 4u * 3u; }
+// the last dword of an entry
+__device__ __forceinline__ uint32_t memo_word(uint32_t len, uint32_t count, uint32_t at) { return len | (count << 4) | (at << 7); }
+__device__ __forceinline__ uint32_t memo_len(uint32_t w) { return w & 15u; }
+__device__ __forceinline__ uint32_t memo_tokens(uint32_t w) { return (w >> 4) & 7u; }
+__device__ __forceinline__ uint32_t memo_at(uint32_t w) { return w >> 7; }
+__device__ __forceinline__ uint64_t word_hash16(const uint32_t (&k)[4]) { return key_hash_next(key_hash_first(0u, k[0], k[1]), k[2], k[3], 1u); }
+
 template <int TILE>
 struct TileLds {
   static constexpr int kBlocks = TILE / 16;
@@ -862,6 +856,10 @@ struct TileArgs {
   uint32_t* counter;       // next range to hand out
   uint32_t* overflow;      // set when a range has more words than range_cap
   // one launch for all (INLINE): the most bytes it is for, and what it leaves in place of the counters and flags
+  uint32_t unit_begin;     // the ranges that this launch does: [unit_begin, unit_end)
+  uint32_t unit_end;
+  const uint4* memo;       // words met before and their tokens (nullptr: none), and what has been counted of them
+  const uint32_t* memo_count;
   const uint32_t* hot;     // slots of words that the sample found, kHotWords of them (nullptr: none)
   int64_t most_bytes;
   uint32_t* first_row_out; // as range_first_row
@@ -884,7 +882,10 @@ constexpr uint32_t kFlagLonger    = 1 * kFlagLine;                              
 constexpr uint32_t kFlagAgain     = 2 * kFlagLine;                              // words of more tokens than a queue record keeps
 constexpr uint32_t kFlagWordUnits = 3 * kFlagLine;                              // kCounterGroups work counters of the word pass, a line each
 constexpr uint32_t kFlagOovUnits  = kFlagWordUnits + kCounterGroups * kFlagLine;  // and of the out-of-vocabulary pass
-constexpr uint32_t kFlagWords     = kFlagOovUnits + kCounterGroups * kFlagLine;
+constexpr uint32_t kFlagWordUnits2 = kFlagOovUnits + kCounterGroups * kFlagLine;  // the same of the second launches, of a column that is done in two
+constexpr uint32_t kFlagOovUnits2  = kFlagWordUnits2 + kCounterGroups * kFlagLine;
+constexpr uint32_t kFlagMemo       = kFlagOovUnits2 + kCounterGroups * kFlagLine;  // words of the first ranges that the memo could take; keys that it took; queue entries of those ranges
+constexpr uint32_t kFlagWords      = kFlagMemo + kFlagLine;
 
 // The next unit of work for a wavefront of a persistent kernel: its first one is its own number in the grid, the
 // following ones come from a counter.  Atomics on one address run at about 150 M/s: eight thousand wavefronts that all
@@ -955,14 +956,18 @@ __device__ __forceinline__ uint32_t count_word_starts(const uint4* abase, int64_
 // and hands out the units g, g + kCounterGroups, ..).
 __global__ void range_first_row_kernel(ColView col, int64_t first_offset, uint32_t cbeg, int64_t range_bytes, uint32_t nranges,
                                        uint32_t* __restrict__ range_first_row, uint32_t* __restrict__ flags, uint32_t word_waves,
-                                       uint32_t oov_waves)
+                                       uint32_t oov_waves, uint32_t word_waves2, uint32_t* __restrict__ memo_owners)
 {
+  if (memo_owners)
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < kMemoEntries; i += gridDim.x * blockDim.x) memo_owners[i] = 0;
   if (blockIdx.x == 0) {
     for (uint32_t i = threadIdx.x; i < kFlagWords; i += blockDim.x) {
       uint32_t v = 0;
-      if (i >= kFlagWordUnits && i % kFlagLine == 0) {
-        uint32_t const c = (i - kFlagWordUnits) / kFlagLine;
-        v = ((c < kCounterGroups ? word_waves : oov_waves) + kCounterGroups - 1u - c % kCounterGroups) / kCounterGroups;
+      if (i >= kFlagWordUnits && i < kFlagMemo && i % kFlagLine == 0) {
+        uint32_t const c     = (i - kFlagWordUnits) / kFlagLine;
+        uint32_t const group = c / kCounterGroups;
+        uint32_t const waves = group == 0 ? word_waves : group == 2 ? word_waves2 : oov_waves;
+        v = (waves + kCounterGroups - 1u - c % kCounterGroups) / kCounterGroups;
       }
       flags[i] = v;
     }
@@ -1004,6 +1009,8 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
     a.ntiles       = (a.cend + TILE - 1) / TILE;
     a.nranges      = static_cast<uint32_t>(a.ntiles);
     a.range_tiles  = 1;
+    a.unit_begin   = 0;
+    a.unit_end     = a.nranges;
   }
   constexpr int kBlocks       = TILE / 16;
   constexpr int kSubs         = kBlocks / kWave;
@@ -1045,6 +1052,7 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
   uint16_t* const word16        = reinterpret_cast<uint16_t*>(lds.word);
   uint32_t q_pos = 0, q_lim = 0;  // this wavefront's reserved queue entries [q_pos, q_lim)
   uint32_t inline_range = 0;
+  bool const use_memo   = !INLINE && a.memo && memo_pays(a.memo_count[0], a.memo_count[1]);
 
   uint32_t const my_number = blockIdx.x * kWaves + threadIdx.x / kWave;
   for (bool first = true;; first = false) {
@@ -1053,9 +1061,9 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
       range = first ? static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(my_number))) : inline_range + gridDim.x * kWaves;
       inline_range = range;
     } else {
-      range = next_unit(a.counter, first, my_number, lane);
+      range = a.unit_begin + next_unit(a.counter, first, my_number, lane);
     }
-    if (range >= a.nranges) break;
+    if (range >= a.unit_end) break;
     int64_t t           = static_cast<int64_t>(range) * a.range_tiles;
     int64_t const t_end = min(t + a.range_tiles, a.ntiles);
     uint32_t r_cur;
@@ -1081,7 +1089,7 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
     }
     uint32_t cursor     = 0;  // words of this range so far
     uint32_t known      = 0;  // of them, in the vocabulary (or too long: one unknown token each)
-    uint32_t oov_tokens = 0;  // INLINE: tokens of the others, my lane's
+    uint32_t oov_tokens = 0;  // tokens of the others that are known here (INLINE: of all of them), my lane's
     uint32_t open_left  = 0;  // words the row that runs into the tile may still have (with a word limit)
     uint32_t* const region = a.arena + static_cast<int64_t>(range) * a.range_cap;
     bool spill             = false;
@@ -1328,9 +1336,9 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
 
         // ---- look the words up; the ones that are not in the vocabulary, or not decided here, go to the queue.
         // A round of 64 words has ten such words on average, too few for the work of building and storing their
-        // records: a round only gives each its place in the queue (which its slot names) and lists it, at the front
-        // of the list of words itself (entry c of the listed words never lies behind the word it came from); the
-        // records of all of them are built and stored afterwards, lanes <-> listed words.
+        // records: a round only lists them, at the front of the list of words itself (entry c of the listed words never
+        // lies behind the word it came from); what becomes of them, their slots and the records of those that go to the
+        // queue follow afterwards, lanes <-> listed words.
         if (cursor + nwc > a.range_cap) spill = true;
         uint32_t const room = q_lim - q_pos;  // left of the reserved entries: used up before the next ones are begun
         uint32_t fresh      = 0;              // where the next ones begin, once they are needed
@@ -1390,38 +1398,57 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
           uint32_t const defer = !active || too_long || found ? 0u : (wl > 16 || (vd == 2u && wl <= table.max_len[0])) ? 2u : 1u;
           uint32_t value       = too_long ? static_cast<uint32_t>(table.unk_id) : static_cast<uint32_t>(id);
           uint64_t const mm    = ballot64(defer != 0);
-          uint32_t const nm    = static_cast<uint32_t>(__builtin_popcountll(mm));
+          // (in one dword: where it starts, below 2048; what it is, 1 or 2; its length, below 200; its number, below 512)
+          if (defer != 0) lds.word[listed + lanes_below(mm)] = s | (defer << 11) | (wl << 13) | (k << 21);
+          listed += static_cast<uint32_t>(__builtin_popcountll(mm));
+          known += static_cast<uint32_t>(__builtin_popcountll(ballot64(active && defer == 0)));
+          if (active && defer == 0 && !spill) region[cursor + k] = value;
+        }
+        wave_lds_sync();
+        // the listed words: from the memo, or a queue record with the word's first 16 bytes, its length, its range and where it begins
+        uint32_t placed = 0;  // of them, in the queue
+        for (uint32_t c0 = 0; c0 < listed; c0 += kWave) {
+          uint32_t const c     = c0 + lane;
+          uint32_t const entry = lds.word[c < listed ? c : 0u];
+          uint32_t const s     = entry & 0x7FFu;
+          uint32_t const defer = (entry >> 11) & 3u;
+          uint32_t const wl    = (entry >> 13) & 0xFFu;
+          TileWord const tw{lds.bytes, 16u + s};
+          uint32_t head[4];
+          tw.head16(head);
+          uint4 const keep = trim[min(wl, 16u)];
+          bool queued      = c < listed;
+          uint32_t value   = 0;
+          if constexpr (!INLINE) {
+            head[0] &= keep.x;
+            head[1] &= keep.y;
+            head[2] &= keep.z;
+            head[3] &= keep.w;
+            if (use_memo && queued && wl <= kMemoWord) {
+              uint4 const e = a.memo[memo_place(word_hash16(head))];
+              if ((e.x == head[0]) & (e.y == head[1]) & (e.z == head[2]) & (memo_len(e.w) == wl)) {
+                queued = false;
+                value  = kOovMark | (a.queue_cap + memo_at(e.w));
+                oov_tokens += memo_tokens(e.w);
+              }
+            }
+          }
+          uint64_t const qm = ballot64(queued);
+          uint32_t const nq = static_cast<uint32_t>(__builtin_popcountll(qm));
           if constexpr (INLINE) {
-            if (listed + nm > room) spill = true;
-          } else if (listed + nm > room && !have_fresh) {
+            if (placed + nq > room) spill = true;
+          } else if (placed + nq > room && !have_fresh) {
             if (lane == 0) fresh = atomicAdd(a.queue_size, kQueueChunk);
             fresh      = wave_bcast(fresh, 0);
             have_fresh = true;
           }
-          if (defer != 0) {
-            uint32_t const c = listed + lanes_below(mm);
-            lds.word[c]      = rec | (defer << 12);  // (a word starts below 2048: bits 12 and 13 of its entry are free)
-            value            = kOovMark | queue_place(c);
-          }
-          listed += nm;
-          known += static_cast<uint32_t>(__builtin_popcountll(ballot64(active && defer == 0)));
-          if (active && !spill) region[cursor + k] = value;
-        }
-        wave_lds_sync();
-        // the records of the listed words: the word's first 16 bytes, its length, its range and where it begins
-        for (uint32_t c0 = 0; c0 < listed; c0 += kWave) {
-          uint32_t const c = c0 + lane;
-          if (c < listed) {
-            uint32_t const entry = lds.word[c];
-            uint32_t const s     = entry & 0xFFFu;
-            uint32_t const wl    = (entry >> 16) - s + 1u;
-            uint32_t const defer = (entry >> 12) & 3u;
-            TileWord const tw{lds.bytes, 16u + s};
-            uint32_t head[4];
-            tw.head16(head);
-            uint4 const keep = trim[min(wl, 16u)];
+          uint32_t const place = placed + lanes_below(qm);
+          uint32_t const q     = queue_place(place);
+          placed += nq;
+          if (queued) value = kOovMark | q;
+          if (c < listed && !spill) region[cursor + (entry >> 21)] = value;
+          if (queued) {
             int64_t const at = tb + s;
-            uint32_t const q = queue_place(c);
             if constexpr (INLINE) {
               int32_t tok[kOovKeep];
               auto const keep_token = [&](uint32_t j, int32_t id) {
@@ -1445,7 +1472,7 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
               }
               oov_tokens += count;
               if (count > kOovKeep) again = true;
-              if (c < room) {
+              if (place < room) {
                 uint4* const dst = reinterpret_cast<uint4*>(a.queue + q);
                 if (count <= kOovKeep) {
                   dst[0] = make_uint4(static_cast<uint32_t>(tok[0]), static_cast<uint32_t>(tok[1]), static_cast<uint32_t>(tok[2]), static_cast<uint32_t>(tok[3]));
@@ -1457,29 +1484,27 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
               }
             } else if (q < a.queue_cap) {
               uint4* const dst = reinterpret_cast<uint4*>(a.queue + q);
-              store_stream(dst, make_uint4(head[0] & keep.x, head[1] & keep.y, head[2] & keep.z, head[3] & keep.w));
+              store_stream(dst, make_uint4(head[0], head[1], head[2], head[3]));
               store_stream(dst + 1, make_uint4(wl | (defer == 2u ? kUnprobed : 0u), range, static_cast<uint32_t>(at),
                                                static_cast<uint32_t>(static_cast<uint64_t>(at) >> 32)));
             }
           }
         }
         if (INLINE) {
-          q_pos += min(listed, room);
-        } else if (listed > room) {
-          q_pos = fresh + (listed - room);
+          q_pos += min(placed, room);
+        } else if (placed > room) {
+          q_pos = fresh + (placed - room);
           q_lim = fresh + kQueueChunk;
         } else {
-          q_pos += listed;
+          q_pos += placed;
         }
         cursor += nwc;
         wave_lds_sync();
         if (w_hi == nw) break;
       }
     }
-    if constexpr (INLINE) {
-      known += wave_bcast(wave_inclusive_scan(oov_tokens), kWave - 1);
-      again = ballot64(again) != 0;
-    }
+    if (INLINE || use_memo) known += wave_bcast(wave_inclusive_scan(oov_tokens), kWave - 1);
+    if (INLINE) again = ballot64(again) != 0;
     if (lane == 0) {
       a.range_words[range]  = cursor;
       a.range_tokens[range] = known;
@@ -1505,7 +1530,8 @@ constexpr uint32_t kOovBlock = 512;
 constexpr int kRefillAt      = 32;
 constexpr int kOovWaves      = 16;  // (two workgroups to a CU, 73 KB of LDS each, 8 wavefronts per SIMD)
 constexpr int kOovThreads    = kOovWaves * kWave;
-constexpr int kRareThreads   = 256;  // the kernels for the few words that this one leaves
+constexpr int kRareThreads     = 256;  // the kernels for the few words that this one leaves
+constexpr unsigned kRareGroups = 2;    // per CU
 struct OovLds {
   alignas(16) uint4 staged[kWave][2];  // 64 queue entries
 };
@@ -1513,7 +1539,8 @@ struct OovLds {
 __global__ void __launch_bounds__(kOovThreads, 8) wordpiece_oov_kernel(VocabTable table, const uint4* abase, OovEntry* __restrict__ queue,
                                                                     const uint32_t* __restrict__ queue_size, uint32_t queue_cap,
                                                                     uint32_t* __restrict__ range_tokens, uint32_t* __restrict__ counter,
-                                                                    uint32_t* __restrict__ longer, uint32_t* __restrict__ longer_count)
+                                                                    uint32_t* __restrict__ longer, uint32_t* __restrict__ longer_count,
+                                                                    const uint32_t* __restrict__ queue_begin)
 {
   __shared__ OovLds lds_all[kOovWaves];
   __shared__ int32_t first_ids[512];  // the ids of the one-byte keys of both key spaces: looked at whenever a piece of a word begins
@@ -1530,6 +1557,8 @@ __global__ void __launch_bounds__(kOovThreads, 8) wordpiece_oov_kernel(VocabTabl
     reinterpret_cast<uint32_t*>(letters3)[i] = reinterpret_cast<const uint32_t*>(table.letters3)[i];
   __syncthreads();
   uint32_t const total = *queue_size;
+  uint32_t const begin = queue_begin ? *queue_begin / kOovBlock : 0u;  // (whole blocks: what the word pass reserves at a time)
+  static_assert(kOovBlock == kQueueChunk, "the entries of a launch of the word pass are whole blocks");
   OovLds& lds          = lds_all[threadIdx.x / kWave];
   int const lane       = lane_id();
 
@@ -1579,7 +1608,7 @@ __global__ void __launch_bounds__(kOovThreads, 8) wordpiece_oov_kernel(VocabTabl
   auto start_fetch = [&] {
     f_n = 0;
     if (next_fetch >= q_end && !no_more) {
-      uint32_t const block   = next_unit(counter, first_block, my_number, lane);
+      uint32_t const block   = begin + next_unit(counter, first_block, my_number, lane);
       first_block            = false;
       uint64_t const b_begin = static_cast<uint64_t>(block) * kOovBlock;
       if (b_begin >= total) {
@@ -1685,13 +1714,34 @@ __global__ void __launch_bounds__(kOovThreads, 8) wordpiece_oov_kernel(VocabTabl
   add_together(acc_count != 0);
 }
 
-// The queued words of more than 16 bytes, which the kernel above has listed: one lane per word, the general state
-// machine over the chars in memory.
+// A word of up to kMaxWord bytes, copied into the lane's row of LDS: the general state machine asks for bytes and keys one
+// after the other, and out of memory each of them was a wait (words of 17 bytes and more of 1.2 M rows of mixed scripts:
+// 82 us in the first of the two kernels below, 70 us from LDS).
+struct RareWords {
+  static constexpr uint32_t kRow = kMaxWord / 4 + 5;  // + misalignment, + what a key read touches past the word; odd
+  uint32_t row[kRareThreads][kRow];
+  __device__ __forceinline__ TileWord copy(const uint4* abase, int64_t at, uint32_t len)
+  {
+    uint32_t* const mine       = row[threadIdx.x];
+    uint32_t const mis         = static_cast<uint32_t>(at & 3);
+    const uint32_t* const from = reinterpret_cast<const uint32_t*>(abase) + (at >> 2);
+    uint32_t const n           = (mis + len + 3u) >> 2;
+    for (uint32_t i = 0; i < n; i += 4) {  // (dwords that hold bytes of the word, four in flight)
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) mine[i + k] = from[min(i + k, n - 1u)];
+    }
+    return TileWord{mine, mis};
+  }
+};
+static_assert(RareWords::kRow % 2 == 1, "the rows begin in different banks");
+
+// The queued words of more than 16 bytes, which the kernel above has listed: one lane per word, the general state machine.
 __global__ void __launch_bounds__(kRareThreads) wordpiece_oov_long_kernel(VocabTable table, const uint4* abase, OovEntry* __restrict__ queue,
                                                                          const uint32_t* __restrict__ queue_size, uint32_t queue_cap,
                                                                          const uint32_t* __restrict__ longer, const uint32_t* __restrict__ longer_count,
                                                                          uint32_t* __restrict__ range_tokens)
 {
+  __shared__ RareWords words;
   if (*queue_size > queue_cap) return;  // (see wordpiece_oov_kernel)
   uint32_t const n = *longer_count;
   for (uint32_t i = blockIdx.x * kRareThreads + threadIdx.x; i < n; i += gridDim.x * kRareThreads) {
@@ -1700,7 +1750,7 @@ __global__ void __launch_bounds__(kRareThreads) wordpiece_oov_long_kernel(VocabT
     uint32_t const wl  = e.len_flags & 0xFFu;
     int64_t const at   = static_cast<int64_t>((static_cast<uint64_t>(e.coord[1]) << 32) | e.coord[0]);
     int32_t tok[kOovKeep];
-    uint32_t const cnt = tokenize_oov_word(table, GlobalWord{reinterpret_cast<const uint8_t*>(abase) + at}, wl, [&](uint32_t j, int32_t id) {
+    uint32_t const cnt = tokenize_oov_word(table, words.copy(abase, at, wl), wl, [&](uint32_t j, int32_t id) {
 #pragma unroll
       for (int k = 0; k < kOovKeep; ++k)
         if (j == static_cast<uint32_t>(k)) tok[k] = id;
@@ -1715,6 +1765,73 @@ __global__ void __launch_bounds__(kRareThreads) wordpiece_oov_long_kernel(VocabT
     }
     atomicAdd(&range_tokens[e.range], cnt);
   }
+}
+
+// ------------------------------------------------------------------ the memo (see kMemoEntries)
+// Between the word pass and the out-of-vocabulary pass of the first ranges: every queued word of up to kMemoWord bytes
+// puts itself in its place (owners[e] = 1 + its queue entry).
+constexpr int kMemoThreads = 1024;  // (few workgroups: one atomic each)
+__global__ void __launch_bounds__(kMemoThreads) wordpiece_memo_claim_kernel(const OovEntry* __restrict__ queue, const uint32_t* __restrict__ queue_size,
+                                                                            uint32_t queue_cap, uint32_t* __restrict__ owners, uint32_t* __restrict__ counts)
+{
+  __shared__ uint32_t all;
+  if (threadIdx.x == 0) all = 0;
+  __syncthreads();
+  uint32_t const total = min(*queue_size, queue_cap);
+  uint32_t words       = 0;
+  for (uint32_t q = blockIdx.x * kMemoThreads + threadIdx.x; q < total; q += gridDim.x * kMemoThreads) {
+    const uint4* const e = reinterpret_cast<const uint4*>(queue + q);
+    uint4 const h = e[0], n = e[1];
+    uint32_t const wl = n.x & 0xFFu;
+    if (wl == 0 || wl > kMemoWord) continue;
+    uint32_t const head[4] = {h.x, h.y, h.z, h.w};
+    owners[memo_place(word_hash16(head))] = q + 1u;
+    ++words;
+  }
+  words = wave_bcast(wave_inclusive_scan(words), kWave - 1);
+  if (lane_id() == 0 && words != 0) atomicAdd(&all, words);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    if (all != 0) atomicAdd(&counts[0], all);
+    if (blockIdx.x == 0) counts[2] = *queue_size;
+  }
+}
+
+// Then the words of those that have a place, and where their results will lie.
+__global__ void __launch_bounds__(kMemoThreads) wordpiece_memo_keys_kernel(const OovEntry* __restrict__ queue, const uint32_t* __restrict__ owners,
+                                                                           uint4* __restrict__ memo, uint32_t* __restrict__ counts)
+{
+  __shared__ uint32_t scan[kMemoThreads / kWave + 1], first;
+  uint32_t const e     = blockIdx.x * kMemoThreads + threadIdx.x;
+  uint32_t const owner = owners[e];
+  uint32_t total;
+  uint32_t const rank = block_exclusive_scan<kMemoThreads>(owner != 0 ? 1u : 0u, scan, &total);
+  if (threadIdx.x == 0) first = atomicAdd(&counts[1], total);
+  __syncthreads();
+  uint4 v = make_uint4(0u, 0u, 0u, 0u);
+  if (owner != 0) {
+    const uint4* const q = reinterpret_cast<const uint4*>(queue + (owner - 1u));
+    v                    = q[0];
+    v.w                  = memo_word(q[1].x & 0xFFu, 0u, first + rank);
+  }
+  memo[e] = v;
+}
+
+// After the out-of-vocabulary pass of the first ranges: the results.
+__global__ void __launch_bounds__(kMemoThreads) wordpiece_memo_fill_kernel(const OovEntry* __restrict__ queue, const uint32_t* __restrict__ owners,
+                                                                           uint4* __restrict__ memo, OovEntry* __restrict__ results)
+{
+  uint32_t const e     = blockIdx.x * kMemoThreads + threadIdx.x;
+  uint32_t const owner = owners[e];
+  if (owner == 0) return;
+  const uint4* const r = reinterpret_cast<const uint4*>(queue + (owner - 1u));
+  uint4 const lo = r[0], hi = r[1];
+  uint32_t const w = memo[e].w;
+  // (a word of more tokens than a record keeps: its record says where it is, and it is no word of the memo)
+  memo[e].w = hi.w <= kOovKeep ? memo_word(memo_len(w), hi.w, memo_at(w)) : 0u;
+  uint4* const to = reinterpret_cast<uint4*>(results + memo_at(w));
+  to[0]           = lo;
+  to[1]           = hi;
 }
 
 // ------------------------------------------------------------------ emit pass
@@ -1889,13 +2006,14 @@ __global__ void __launch_bounds__(kRareThreads) wordpiece_retokenize_kernel(Voca
                                                                            const uint32_t* __restrict__ again, const uint32_t* __restrict__ again_count,
                                                                            int32_t* __restrict__ child)
 {
+  __shared__ RareWords words;
   uint32_t const n = *again_count;
   for (uint32_t i = blockIdx.x * kRareThreads + threadIdx.x; i < n; i += gridDim.x * kRareThreads) {
     OovEntry const e   = queue[again[i]];  // head[0] = place in the child, head[3] = coord[1], len_flags, range, coord[0] as they were; coord[1] = the count
     uint32_t const cnt = e.coord[1];
     int64_t const at   = static_cast<int64_t>((static_cast<uint64_t>(e.head[3]) << 32) | e.coord[0]);
     int32_t* const d   = child + e.head[0];
-    tokenize_oov_word(table, GlobalWord{reinterpret_cast<const uint8_t*>(abase) + at}, e.len_flags & 0xFFu, [&](uint32_t j, int32_t id) {
+    tokenize_oov_word(table, words.copy(abase, at, e.len_flags & 0xFFu), e.len_flags & 0xFFu, [&](uint32_t j, int32_t id) {
       if (j < cnt) d[j] = id;
     });
   }
@@ -2627,14 +2745,20 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   constexpr int kWordWaves = word_waves(false);
   int range_tiles = kRangeTiles;
   while (range_tiles > 1 && ntiles / range_tiles < 8 * word_resident * kWordWaves) range_tiles >>= 1;
+  // A large column with unknown words is done in two parts, the first for the memo: shorter ranges, so that the first part has
+  // enough of them to share out (tiles of 2 KB to a range: 1: 1388 us, 2: 1255, 4: 1243, 8: 1324).
+  bool const with_memo = cend >= kMemoLeast && sample_queued * 50 > sample_words;
+  if (with_memo) range_tiles = std::min(range_tiles, 4);
   // (tests, which have no column of a gigabyte to give, set the size through nvtext_amd_profile_set_range_tiles)
   if (int const want = g_forced_range_tiles.load(std::memory_order_relaxed)) range_tiles = want;
   int64_t const kRange    = static_cast<int64_t>(kTile) * range_tiles;
   int64_t const nranges64 = (ntiles + range_tiles - 1) / range_tiles;
   if (nranges64 > 0x7FFFFFF0) return give_up(NVTEXT_AMD_LOGIC_ERROR, "words exceed internal limit");
   uint32_t const nranges = static_cast<uint32_t>(nranges64);
-  unsigned const word_grid = static_cast<unsigned>(
-    std::min<int64_t>((static_cast<int64_t>(nranges) + kWordWaves - 1) / kWordWaves, word_resident));
+  uint32_t const first_part = with_memo ? std::min(nranges, static_cast<uint32_t>(kMemoBytes / kRange)) : nranges;  // ranges
+  auto const grid_for       = [&](uint32_t ranges) { return static_cast<unsigned>(std::min<int64_t>((static_cast<int64_t>(ranges) + kWordWaves - 1) / kWordWaves, word_resident)); };
+  unsigned const word_grid  = grid_for(first_part);
+  unsigned const word_grid2 = grid_for(nranges - first_part);  // (0: the column is done in one part)
   unsigned const oov_grid  = static_cast<unsigned>(resident(reinterpret_cast<const void*>(wordpiece_oov_kernel), kOovThreads, 4));
   unsigned const emit_grid = static_cast<unsigned>(
     std::min<int64_t>((static_cast<int64_t>(nranges) + kTokWaves - 1) / kTokWaves, resident(reinterpret_cast<const void*>(wordpiece_emit_kernel), kTokThreads, 5)));
@@ -2658,7 +2782,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   // language than the vocabulary's) makes the attempt fail, and the second has what the first found to be needed:
   // room for a word per byte, the exact number of queue entries.
   uint32_t range_cap      = static_cast<uint32_t>(kRange * 5 / 16);
-  uint64_t queue_capacity = static_cast<uint64_t>((last_offset - first_offset) >> 5) + static_cast<uint64_t>(word_grid) * kWordWaves * kQueueChunk + 4096;
+  uint64_t queue_capacity = static_cast<uint64_t>((last_offset - first_offset) >> 5) + static_cast<uint64_t>(word_grid + word_grid2) * kWordWaves * kQueueChunk + 4096;
   if (sample_bytes > 0) {
     // what the sample calls for, with half as much again for the ranges that are denser than the column as a whole
     // (never less than the sizes above: a sample can miss; the second attempt remains)
@@ -2667,22 +2791,24 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     range_cap = static_cast<uint32_t>(std::min<double>(static_cast<double>(kRange + 8), std::max<double>(range_cap, per_byte_words * 1.5 * static_cast<double>(kRange) + 256)));
     range_cap = (range_cap + 1u) & ~1u;  // (a range's slots begin at an even index)
     queue_capacity = std::max<uint64_t>(queue_capacity, static_cast<uint64_t>(per_byte_queued * 1.25 * static_cast<double>(last_offset - first_offset)) +
-                                                          static_cast<uint64_t>(word_grid) * kWordWaves * kQueueChunk + 4096);
+                                                          static_cast<uint64_t>(word_grid + word_grid2) * kWordWaves * kQueueChunk + 4096);
   }
   uint64_t total = 0;
   for (int attempt = 0;; ++attempt) {
-    if (queue_capacity > 0x7FFFFFF0ull) queue_capacity = 0x7FFFFFF0ull;
+    if (queue_capacity > 0x7FFFFFF0ull - kMemoEntries) queue_capacity = 0x7FFFFFF0ull - kMemoEntries;
     uint32_t const qcap        = static_cast<uint32_t>(queue_capacity);
-    size_t const temp_bytes[9] = {static_cast<size_t>(nranges) * range_cap * sizeof(uint32_t),
+    uint32_t const memo_entries = word_grid2 > 0 ? kMemoEntries : 0u;
+    size_t const temp_bytes[10] = {static_cast<size_t>(nranges) * range_cap * sizeof(uint32_t),
                                   (static_cast<size_t>(nranges) + 1) * sizeof(uint32_t),
                                   static_cast<size_t>(nranges) * sizeof(uint32_t),
                                   static_cast<size_t>(nranges) * sizeof(uint32_t),
                                   (static_cast<size_t>(nranges) + 1) * sizeof(int64_t),
                                   scan_temp_bytes(nranges),
                                   kFlagWords * sizeof(uint32_t),
-                                  static_cast<size_t>(qcap) * sizeof(OovEntry),
-                                  static_cast<size_t>(qcap) * sizeof(uint32_t)};
-    TempParts<9> const temps(mr, temp_bytes);
+                                  (static_cast<size_t>(qcap) + memo_entries) * sizeof(OovEntry),
+                                  static_cast<size_t>(qcap) * sizeof(uint32_t),
+                                  static_cast<size_t>(memo_entries) * (sizeof(uint4) + sizeof(uint32_t))};
+    TempParts<10> const temps(mr, temp_bytes);
     if (!temps.ok()) return give_up(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");
     uint32_t* const arena     = temps.part<uint32_t>(0);
     uint32_t* const first_row = temps.part<uint32_t>(1);
@@ -2702,22 +2828,38 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     args.queue           = queue;
     args.queue_cap       = qcap;
     args.queue_size      = flags + kFlagQueueSize;
-    args.counter         = flags + kFlagWordUnits;
     args.overflow        = flags + kFlagOverflow;
+    uint4* const memo      = temps.part<uint4>(9);
+    uint32_t* const owners = memo_entries ? reinterpret_cast<uint32_t*>(memo + kMemoEntries) : nullptr;
+    args.memo_count        = flags + kFlagMemo;
     hipLaunchKernelGGL(range_first_row_kernel, dim3((nranges + 1 + 255) / 256), dim3(256), 0, stream, v, first_offset, cbeg, kRange, nranges, first_row,
-                       flags, word_grid * kWordWaves, oov_grid * kOovWaves);
-    {
-      ProfileScope ps("wordpiece_word_kernel", stream);
-      hipLaunchKernelGGL(word_kernel, dim3(word_grid), dim3(kWordWaves * kWave), 0, stream, args);
-    }
-    {
-      ProfileScope ps("wordpiece_oov_kernel", stream);
-      hipLaunchKernelGGL(wordpiece_oov_kernel, dim3(oov_grid), dim3(kOovThreads), 0, stream, vocabulary->table, args.abase, queue, flags + kFlagQueueSize, qcap, tokens,
-                         flags + kFlagOovUnits, longer, flags + kFlagLonger);
+                       flags, word_grid * kWordWaves, oov_grid * kOovWaves, word_grid2 * kWordWaves, owners);
+    for (int part = 0; part < (word_grid2 > 0 ? 2 : 1); ++part) {
+      args.unit_begin = part == 0 ? 0u : first_part;
+      args.unit_end   = part == 0 ? first_part : nranges;
+      args.counter    = flags + (part == 0 ? kFlagWordUnits : kFlagWordUnits2);
+      args.memo       = part == 0 ? nullptr : memo;
+      {
+        ProfileScope ps("wordpiece_word_kernel", stream);
+        hipLaunchKernelGGL(word_kernel, dim3(part == 0 ? word_grid : word_grid2), dim3(kWordWaves * kWave), 0, stream, args);
+      }
+      if (part == 0 && owners) {
+        hipLaunchKernelGGL(wordpiece_memo_claim_kernel, dim3(static_cast<unsigned>(cus)), dim3(kMemoThreads), 0, stream, queue, flags + kFlagQueueSize, qcap,
+                           owners, flags + kFlagMemo);
+        hipLaunchKernelGGL(wordpiece_memo_keys_kernel, dim3(kMemoEntries / kMemoThreads), dim3(kMemoThreads), 0, stream, queue, owners, memo,
+                           flags + kFlagMemo);
+      }
+      {
+        ProfileScope ps("wordpiece_oov_kernel", stream);
+        hipLaunchKernelGGL(wordpiece_oov_kernel, dim3(oov_grid), dim3(kOovThreads), 0, stream, vocabulary->table, args.abase, queue, flags + kFlagQueueSize, qcap,
+                           tokens, flags + (part == 0 ? kFlagOovUnits : kFlagOovUnits2), longer, flags + kFlagLonger, part == 0 ? nullptr : flags + kFlagMemo + 2);
+      }
+      if (part == 0 && owners)
+        hipLaunchKernelGGL(wordpiece_memo_fill_kernel, dim3(kMemoEntries / kMemoThreads), dim3(kMemoThreads), 0, stream, queue, owners, memo, queue + qcap);
     }
     {
       ProfileScope ps("wordpiece_oov_long_kernel", stream);
-      hipLaunchKernelGGL(wordpiece_oov_long_kernel, dim3(static_cast<unsigned>(cus)), dim3(kRareThreads), 0, stream, vocabulary->table, args.abase, queue,
+      hipLaunchKernelGGL(wordpiece_oov_long_kernel, dim3(static_cast<unsigned>(cus) * kRareGroups), dim3(kRareThreads), 0, stream, vocabulary->table, args.abase, queue,
                          flags + kFlagQueueSize, qcap, longer, flags + kFlagLonger, tokens);
     }
     // where the tokens of each range go; the total decides the child size
@@ -2753,7 +2895,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
       // state[2] counts the chunks of kQueueChunk entries that the wavefronts reserved, the unused rest of each
       // wavefront's last chunk included; which ranges a wavefront gets differs from one attempt to the next, and with it
       // that rest: a chunk per wavefront on top of what this attempt reserved covers every assignment.
-      queue_capacity = std::max<uint64_t>(queue_capacity, static_cast<uint64_t>(state[2]) + static_cast<uint64_t>(word_grid) * kWordWaves * kQueueChunk);
+      queue_capacity = std::max<uint64_t>(queue_capacity, static_cast<uint64_t>(state[2]) + static_cast<uint64_t>(word_grid + word_grid2) * kWordWaves * kQueueChunk);
       continue;
     }
     if (total > static_cast<uint64_t>(std::numeric_limits<int32_t>::max())) return give_up(NVTEXT_AMD_OVERFLOW, "Size of output exceeds the column size limit");
@@ -2769,7 +2911,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
                          out->offsets, static_cast<int32_t*>(out->child), longer, flags + kFlagAgain);
       // (the list of longer words has served its purpose by now: its memory takes the list of words to do again, at most
       // one entry per queued word)
-      hipLaunchKernelGGL(wordpiece_retokenize_kernel, dim3(static_cast<unsigned>(cus)), dim3(kRareThreads), 0, stream, vocabulary->table, args.abase, queue,
+      hipLaunchKernelGGL(wordpiece_retokenize_kernel, dim3(static_cast<unsigned>(cus) * kRareGroups), dim3(kRareThreads), 0, stream, vocabulary->table, args.abase, queue,
                          longer, flags + kFlagAgain, static_cast<int32_t*>(out->child));
     }
     break;

@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from cudf_amd.arrow_host import HostStringsColumn
+from cudf_amd.arrow_host import HostListStringsColumn, HostStringsColumn
 
 pytestmark = pytest.mark.gpu
 
@@ -96,6 +96,44 @@ def test_minhash_row_counts(nv, orc, rows, nulls):
     assert nv.minhash64(dev(nv, host), 5, a, b, 4).to_host().equals(orc.minhash64(host, 5, a, b, 4, nthreads=8))
 
 
+@pytest.mark.parametrize("kind", ["zero", "small", "power", "digits of 2", "digits of 1", "wraps", "top"])
+def test_minhash64_parameters(nv, orc, kind):
+    """Parameters for which the fractions that decide what is computed exactly tie, lie at zero or at the wrap, or take their
+    sums to the ends of their range; rows of one window, of fewer than a block of 32 and of many, with windows that repeat."""
+    rng = np.random.default_rng(7)
+    p = (1 << 61) - 1
+    a = {"zero": [0, p, 2 * p], "small": [1, 2, 3, 5], "power": [1 << 60, 1 << 61, 1 << 63, 1 << 44, 1 << 43], "digits of 2": [0xAAAAAAAAAAAAAAAA],
+         "digits of 1": [0x5555555555555555], "wraps": [(1 << 64) - 1, p - 1, p + 1], "top": [(1 << 44) - 1, (1 << 64) - (1 << 44)]}[kind]
+    b = [0, 1, p - 1, p, p + 7, (1 << 61) - 8, (1 << 64) - 1, 1 << 44, (1 << 44) - 1]
+    pairs = np.array([(x, y) for x in a for y in b], np.uint64)
+    a, b = pairs[:, 0].copy(), pairs[:, 1].copy()
+    host = mixed_rows(rng, [5, 6, 30, 36, 37, 300, 3000, 40_000])
+    text = HostStringsColumn.from_pylist(["abcdefgh" * 500, "a" * 3000, "the same words " * 400, "naïve 漢字 " * 60])
+    for column in (host, text):
+        assert nv.minhash64(dev(nv, column), 5, a, b, 5).to_host().equals(orc.minhash64(column, 5, a, b, 5, nthreads=8))
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("ngrams", [2, 5])
+@pytest.mark.parametrize("count", [1, 130])
+def test_minhash_ngrams_parts_of_rows(nv, orc, bits, ngrams, count):
+    """Lists one element around a trip of 64 positions, around the four that are folded together and around parts of 1024,
+    shorter than a run, empty, and among 131,072 others; elements that are null or empty; a view."""
+    rng = np.random.default_rng(count)
+    call, ref = (nv.minhash_ngrams, orc.minhash_ngrams) if bits == 32 else (nv.minhash64_ngrams, orc.minhash64_ngrams)
+    a, b = params(rng, count, bits)
+    edges = [0, 1, 2, 5, 6, 7, 63, 64, 65, 68, 69, 255, 256, 260, 261, 1024, 1028, 1029, 2053, 5000]
+    for lens in (edges + edges[::-1], edges + [1, 0, 3] * 43_691 if count == 1 else edges):
+        offsets = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+        n = int(offsets[-1])
+        child = mixed_rows(rng, rng.integers(0, 12, n), nulls=range(10, n, 97))
+        lists = HostListStringsColumn(offsets, child, None, len(lens), 0, 0)
+        d = nv.DeviceListStringsColumn.from_host(lists)
+        assert call(d, ngrams, 5, a, b).to_host().equals(ref(lists, ngrams, 5, a, b, nthreads=8))
+        assert call(d.slice(2, len(lens) - 1, 0), ngrams, 5, a, b).to_host().equals(
+            ref(HostListStringsColumn(offsets, child, None, len(lens) - 3, 2, 0), ngrams, 5, a, b, nthreads=8))
+
+
 def words_column(rng, lens, vocabulary, oov):
     """Rows of about these many bytes: words of the vocabulary, and `oov` of them random letters."""
     stems = [w for w in vocabulary if not w.startswith("##") and not w.startswith("[")]
@@ -145,6 +183,29 @@ def test_tokenize_where_small_columns_end(nv, orc, rows, each):
     offsets = np.linspace(0, rows * each, rows + 1).astype(np.int32)
     host = HostStringsColumn(text.chars, offsets, None, rows, 0, 0)
     assert nv.wordpiece_tokenize(dev(nv, host), vocabulary, 50).to_host().equals(orc.wordpiece_tokenize(host, reference, 50, nthreads=8))
+
+
+@pytest.mark.parametrize("different", [1, 3000, 60_000, 500_000])
+@pytest.mark.parametrize("limit, wide", [(0, False), (60, True)])
+def test_tokenize_words_met_before(nv, orc, different, limit, wide):
+    """Columns around the 128 MiB from which the unknown words of the first ranges are kept: few different ones, many, and
+    too many to keep; of 1 to 20 bytes (kept: up to 12), of one token and of more than seven; offsets of 32 and 64 bits."""
+    rng = np.random.default_rng(different)
+    hv = HostStringsColumn.from_pylist(VOCABULARY)
+    vocabulary, reference = nv.WordPieceVocabulary(dev(nv, hv)), orc.Vocabulary(hv)
+    cells = np.full((different + 40, 24), 0x20, np.uint8)
+    for i in range(40):
+        word = VOCABULARY[2 + i % 20] if i % 2 else "hello"
+        cells[i, : len(word)] = np.frombuffer(word.encode(), np.uint8)
+    size = rng.integers(1, 21, different)
+    letters = rng.choice(np.frombuffer(b"abcdefgxyz", np.uint8), (different, 20))
+    cells[40:, :20] = np.where(np.arange(20) < size[:, None], letters, 0x20)
+    for total in ((128 << 20) - 24 * 64, (128 << 20) + 24 * 64):
+        n = total // 24
+        chars = cells[np.where(rng.random(n) < 0.5, rng.integers(0, 40, n), rng.integers(40, different + 40, n))].reshape(-1)
+        offsets = np.arange(0, n * 24 + 1, 24 * 64, dtype=np.int64 if wide else np.int32)
+        host = HostStringsColumn(chars[: offsets[-1]], offsets, None, offsets.size - 1, 0, 0)
+        assert nv.wordpiece_tokenize(dev(nv, host), vocabulary, limit).to_host().equals(orc.wordpiece_tokenize(host, reference, limit, nthreads=8))
 
 
 @pytest.mark.parametrize("rows, each", [(1, 1), (3, 2047), (3, 2048), (61, 300), (4, 65_535), (4, 65_537), (131_072, 9), (131_073, 9), (30_000, 2300)])
