@@ -800,9 +800,10 @@ constexpr uint32_t kUnprobed = 0x100u;  // the word has not been looked up whole
 // queue's records, so that a word's slot names it as it names a queue record.  Of several words with one place the last
 // to ask has it, the more frequent one more often than not; a second place for each would cost every word a second
 // scattered read and save as much of the out-of-vocabulary pass.
-// (2 M rows of 256 bytes, 15 % of their words unknown, 40,000 different ones of those: 1463 -> 1244 us.)
-constexpr uint32_t kMemoBits    = 17;
+// (2 M rows of 256 bytes, 15 % of their words unknown, 40,000 different ones of those: 1463 -> 1172 us.)
+constexpr uint32_t kMemoBits    = 20;  // (17: 1242 us, 18: 1205, 19: 1185, 20: 1172: few words share a place, and only those touched take cache)
 constexpr uint32_t kMemoEntries = 1u << kMemoBits;
+constexpr uint32_t kMemoResults = 1u << 18;  // words that it keeps at most
 constexpr uint32_t kMemoWord    = 12;
 constexpr int64_t kMemoBytes    = 16 << 20;
 constexpr int64_t kMemoLeast    = 128 << 20;  // smaller columns: the second launches cost what the memo saves
@@ -813,7 +814,7 @@ __device__ __forceinline__ uint32_t memo_place(uint64_t key_hash)
 }
 // Whether the words of the first ranges repeat enough: words asked for places, and got so many between them.  (With most
 // of the places taken there may be any number of different words.)
-__device__ __forceinline__ bool memo_pays(uint32_t words, uint32_t places) { return words > 3u * places && places < kMemoEntries / 4u * 3u; }
+__device__ __forceinline__ bool memo_pays(uint32_t words, uint32_t places) { return words > 3u * places && places < kMemoEntries / 2u; }
 // the last dword of an entry
 __device__ __forceinline__ uint32_t memo_word(uint32_t len, uint32_t count, uint32_t at) { return len | (count << 4) | (at << 7); }
 __device__ __forceinline__ uint32_t memo_len(uint32_t w) { return w & 15u; }
@@ -1809,7 +1810,7 @@ __global__ void __launch_bounds__(kMemoThreads) wordpiece_memo_keys_kernel(const
   if (threadIdx.x == 0) first = atomicAdd(&counts[1], total);
   __syncthreads();
   uint4 v = make_uint4(0u, 0u, 0u, 0u);
-  if (owner != 0) {
+  if (owner != 0 && first + rank < kMemoResults) {
     const uint4* const q = reinterpret_cast<const uint4*>(queue + (owner - 1u));
     v                    = q[0];
     v.w                  = memo_word(q[1].x & 0xFFu, 0u, first + rank);
@@ -1823,10 +1824,10 @@ __global__ void __launch_bounds__(kMemoThreads) wordpiece_memo_fill_kernel(const
 {
   uint32_t const e     = blockIdx.x * kMemoThreads + threadIdx.x;
   uint32_t const owner = owners[e];
-  if (owner == 0) return;
+  uint32_t const w     = memo[e].w;
+  if (owner == 0 || w == 0) return;
   const uint4* const r = reinterpret_cast<const uint4*>(queue + (owner - 1u));
   uint4 const lo = r[0], hi = r[1];
-  uint32_t const w = memo[e].w;
   // (a word of more tokens than a record keeps: its record says where it is, and it is no word of the memo)
   memo[e].w = hi.w <= kOovKeep ? memo_word(memo_len(w), hi.w, memo_at(w)) : 0u;
   uint4* const to = reinterpret_cast<uint4*>(results + memo_at(w));
@@ -2795,7 +2796,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   }
   uint64_t total = 0;
   for (int attempt = 0;; ++attempt) {
-    if (queue_capacity > 0x7FFFFFF0ull - kMemoEntries) queue_capacity = 0x7FFFFFF0ull - kMemoEntries;
+    if (queue_capacity > 0x7FFFFFF0ull - kMemoResults) queue_capacity = 0x7FFFFFF0ull - kMemoResults;
     uint32_t const qcap        = static_cast<uint32_t>(queue_capacity);
     uint32_t const memo_entries = word_grid2 > 0 ? kMemoEntries : 0u;
     size_t const temp_bytes[10] = {static_cast<size_t>(nranges) * range_cap * sizeof(uint32_t),
@@ -2805,7 +2806,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
                                   (static_cast<size_t>(nranges) + 1) * sizeof(int64_t),
                                   scan_temp_bytes(nranges),
                                   kFlagWords * sizeof(uint32_t),
-                                  (static_cast<size_t>(qcap) + memo_entries) * sizeof(OovEntry),
+                                  (static_cast<size_t>(qcap) + (memo_entries ? kMemoResults : 0u)) * sizeof(OovEntry),
                                   static_cast<size_t>(qcap) * sizeof(uint32_t),
                                   static_cast<size_t>(memo_entries) * (sizeof(uint4) + sizeof(uint32_t))};
     TempParts<10> const temps(mr, temp_bytes);
