@@ -383,7 +383,9 @@ __device__ __forceinline__ bool seen_lately(WaveLds<T>& lds, T hv)
 template <typename T>
 __device__ __forceinline__ void forget_hashes(WaveLds<T>& lds, int lane)
 {
-  for (int i = lane; i < recent_entries<T>(); i += kWave) lds.recent[i] = T{0};
+  constexpr int kEach = 16 / sizeof(T);
+#pragma unroll
+  for (int i = 0; i < recent_entries<T>() / kEach; i += kWave) reinterpret_cast<uint4*>(lds.recent)[i + lane] = make_uint4(0u, 0u, 0u, 0u);
 }
 
 // What is hashed: a column of strings, by windows of characters, or a column of lists of strings, by runs of elements.  A
@@ -395,6 +397,7 @@ struct TextRows {
   using Lds = WaveLds<T>;
   static constexpr const char* kRowsName  = "minhash_rows_kernel";
   static constexpr const char* kPartsName = "minhash_parts_kernel";
+  static constexpr int kSimdWaves   = sizeof(T) == 4 ? 6 : 4;  // wavefronts per SIMD that its LDS leaves room for
   static constexpr int64_t kPart    = 4096;
   static constexpr int64_t kMinPart = kTile;  // less would be staged for its halo
   ColView col;
@@ -516,6 +519,7 @@ struct RunRows {
   using Lds = RunLds<T>;
   static constexpr const char* kRowsName  = "minhash_ngrams_rows_kernel";
   static constexpr const char* kPartsName = "minhash_ngrams_parts_kernel";
+  static constexpr int kSimdWaves   = sizeof(T) == 4 ? 7 : 4;
   static constexpr int64_t kPart    = 1024;
   static constexpr int64_t kMinPart = kWave;
   ListView col;
@@ -634,11 +638,15 @@ struct RowParts {
   }
 };
 
+// Wavefronts per SIMD that the kernels are compiled for.
+template <typename Source, typename Minima>
+constexpr int simd_waves() { return Source::kSimdWaves < Minima::kSimdWaves ? Source::kSimdWaves : Minima::kSimdWaves; }
+
 // One workgroup per (group of consecutive rows, parameter chunk): its wavefronts take the group's rows of up to kPart
 // bytes one at a time from a counter in LDS, so that the four are done together whatever the rows' lengths; the minima
 // go from the registers to the result.  The groups lie along x and, beyond kMaxRowBlocks of them, along z.
 template <typename Source, typename Minima, typename T = typename Minima::T>
-__global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_rows_kernel(Source source, Params<T> params,
+__global__ void __launch_bounds__(kThreads, (simd_waves<Source, Minima>())) minhash_rows_kernel(Source source, Params<T> params,
                                                                                    const int32_t* __restrict__ out_offsets, T* __restrict__ out,
                                                                                    int per_wave)
 {
@@ -683,7 +691,7 @@ __global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_rows_ker
 // requests a second: seven thousand wavefronts asking at once would wait 50 us).  The chunks of parameters come one
 // after the other in the same count.
 template <typename Source, typename Minima, typename T = typename Minima::T>
-__global__ void __launch_bounds__(kThreads, Minima::kSimdWaves) minhash_parts_kernel(RowParts<Source> parts, Params<T> params, int32_t chunks,
+__global__ void __launch_bounds__(kThreads, (simd_waves<Source, Minima>())) minhash_parts_kernel(RowParts<Source> parts, Params<T> params, int32_t chunks,
                                                                                     const int32_t* __restrict__ out_offsets,
                                                                                     const uint32_t* __restrict__ prefix,
                                                                                     unsigned long long* __restrict__ counter, T* __restrict__ out)
@@ -931,9 +939,9 @@ template <typename Source, typename T = typename Source::T>
 void run_minhash(Source const& source, int32_t rows, bool masked, const T* a, const T* b, int32_t P, int32_t* offsets, T* child, int64_t child_size,
                  uint32_t* prefix, uint64_t* scan_tmp, filter64::Group* laid_out, hipStream_t stream)
 {
-  int simd_waves = 0;
-  with_minima<T>(P, [&](auto which, int32_t) { simd_waves = decltype(which)::type::kSimdWaves; });
-  RowParts<Source> const parts{source, device_cus() * 4 * simd_waves, rows >= kManyRows ? Source::kPart : -1};
+  int waves = 0;
+  with_minima<T>(P, [&](auto which, int32_t) { waves = simd_waves<Source, typename decltype(which)::type>(); });
+  RowParts<Source> const parts{source, device_cus() * 4 * waves, rows >= kManyRows ? Source::kPart : -1};
   Params<T> const params{a, b, P, laid_out};
   auto* const counter = reinterpret_cast<unsigned long long*>(scan_tmp) + scan_temp_bytes(rows) / sizeof(uint64_t);
   if (rows <= kPlanRows) {

@@ -16,12 +16,14 @@ constexpr int kHalo      = 128;                // bytes staged past the tile (wi
 constexpr int kCharList  = kTile + kHalo + 8;   // list of a tile's characters: one per staged byte, the end of the last one, padding
 constexpr int kTileWords = (kTile + kHalo + 16 + 32) / 4;  // +16 misalignment, +32 for whole blocks and the over-read of the hash tail
 
-// Windows repeat (text repeats its words: a tenth of the windows of a tile, a third within 4 KB of ordinary text), and a
-// hash that has been folded once changes no minimum when it is folded again.  Every wavefront keeps the hashes it
-// saw last in a small direct-mapped table and drops a hash that it finds there; what the table has forgotten is folded
-// again, which costs time and nothing else.  Cleared (hashes are never 0) whenever the wavefront begins a row.
+// Windows repeat (of 2 KB of ordinary text three in four are different, of 16 KB little more than half), and a hash that
+// has been folded once changes no minimum when it is folded again.  Every wavefront keeps the hashes it saw last in a
+// small direct-mapped table and drops a hash that it finds there; what the table has forgotten is folded again, which
+// costs time and nothing else.  Cleared (hashes are never 0) whenever the wavefront begins a row.  As many entries as leave
+// six (64-bit hashes: four) workgroups to a CU: 400,000 documents of 2 KB, 256 parameters: 256 entries 8.80 ms, 512: 8.45,
+// 1024: 8.17; 64-bit hashes of 20,011 long rows: 256: 4.13 ms, 512: 4.05, 1024: 4.85 (three workgroups).
 template <typename T>
-constexpr int recent_entries() { return 256; }  // (512 costs the kernels a workgroup per CU: slower but for the longest rows)
+constexpr int recent_entries() { return sizeof(T) == 4 ? 1024 : 512; }
 
 template <typename T>
 struct WaveLds {
