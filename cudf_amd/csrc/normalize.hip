@@ -17,8 +17,8 @@
 struct nvtext_amd_character_normalizer {
   int device            = 0;
   int32_t do_lower      = 0;
-  uint32_t* ascii       = nullptr;  // device, 128: slot 0 | slot 1 << 8 | slot 2 << 16 | bytes << 24 of the code points below 0x80
-  uint4* bmp            = nullptr;  // device, 65536: {slot 0, slot 1, slot 2, bytes} of the code points below 0x10000
+  uint32_t* ascii       = nullptr;  // device, 256: slot 0 | slot 1 << 8 | slot 2 << 16 | bytes << 24 of the code points below 0x80, zeros
+  uint4* bmp            = nullptr;  // device, 65536: {slot 0, slot 1, slot 2, bytes} of the code points below 0x10000, and 65536 of their strings
   uint32_t* entries     = nullptr;  // device, kCodepoints: category << 24 | multi << 23 | replacement
   uint64_t* second      = nullptr;  // device, kCodepoints: second << 32 | third replacement code point
   uint8_t* token_chars  = nullptr;  // device: the special tokens, sorted then lower-cased
@@ -55,8 +55,9 @@ constexpr int64_t kSmallBytes    = 64 << 20;
 constexpr int kStageBytes  = 4 * kNormTile;  // output bytes of a tile that are assembled in LDS; a tile with more writes them one by one
 
 struct NormTables {
-  const uint32_t* ascii;  // 128 entries: the slots of the code points below 0x80
-  const uint4* bmp;       // 65536 entries: the three slots and their bytes together, of the code points below 0x10000
+  const uint32_t* ascii;  // 256 entries: the slots of the code points below 0x80, then zeros (a byte that is no such character gives nothing)
+  const uint4* bmp;       // 65536 entries: the three slots and their bytes together, of the code points below 0x10000; and 65536
+                          // more: those slots side by side, as a string of up to 12 bytes, and its bytes
   const uint32_t* entries;
   const uint64_t* second;
   const uint8_t* token_chars;
@@ -133,7 +134,8 @@ constexpr int kWaveLeads = 256;  // first bytes of longer characters per wavefro
 template <bool SLOTS>
 struct NormLds {
   alignas(16) uint32_t raw[kRawWords];  // the input bytes of the tile and its surroundings, zero outside the column
-  uint32_t ascii[128];                 // code points below 0x80: slot 0 | slot 1 << 8 | slot 2 << 16 | bytes << 24
+  uint32_t ascii[256];                 // code points below 0x80: slot 0 | slot 1 << 8 | slot 2 << 16 | bytes << 24; then zeros
+  uint8_t sizes[SLOTS ? 4 : 256];      // their bytes (the pass that counts)
   union {
     // first byte of slot k of tile position i - kSlotBase; only filled where special tokens can be.  A first byte
     // tells '[', ']', a space and a-z from everything else, which is all the special tokens look at or change.
@@ -151,6 +153,7 @@ struct NormLds {
 // The slots of the tile positions a lane owns (kNormItems * lane ..): consecutive bytes in, consecutive bytes out.
 struct Owned {
   uint32_t s[kNormItems][3];
+  uint32_t widest;  // the most bytes of a position, or somewhat more (the pass that writes)
 };
 
 // Slot `at` of the flat slot sequence (three per position).
@@ -270,6 +273,40 @@ __device__ __forceinline__ uint32_t wide_slots(uint32_t w, NormTables const& t, 
   return e.w;
 }
 
+// The bytes of up to three slots side by side, first slot first: (lo, hi) = bytes 0..7 and 8..11.
+__host__ __device__ __forceinline__ void slots_to_string(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t& d0, uint32_t& d1, uint32_t& d2)
+{
+  uint32_t const b0  = bytes_of(s0);
+  uint32_t const b01 = b0 + bytes_of(s1);  // <= 8
+  uint64_t lo        = s0 | (static_cast<uint64_t>(s1) << (8u * b0));
+  uint64_t const t   = s2;
+  uint32_t const sh  = 8u * b01;
+  lo |= b01 < 8u ? t << (sh & 63u) : 0ull;
+  d2 = b01 >= 8u ? s2 : b01 > 4u ? static_cast<uint32_t>(t >> ((64u - sh) & 63u)) : 0u;
+  d0 = static_cast<uint32_t>(lo);
+  d1 = static_cast<uint32_t>(lo >> 32);
+}
+
+// The string that the character whose bytes start `w` turns into (12 bytes, zero padded), and its bytes.
+__device__ __forceinline__ uint32_t wide_string(uint32_t w, NormTables const& t, uint32_t& d0, uint32_t& d1, uint32_t& d2)
+{
+  uint32_t cp = decode_short(w);
+  if ((w & 0xFFu) >= 0xF0u) {
+    cp = decode(w & 0xFFu, (w >> 8) & 0xFFu, (w >> 16) & 0xFFu, w >> 24);
+    if (cp >= 0x10000u) {
+      uint32_t s0, s1, s2;
+      slots_of(cp, t, s0, s1, s2);
+      slots_to_string(s0, s1, s2, d0, d1, d2);
+      return bytes_of(s0) + bytes_of(s1) + bytes_of(s2);
+    }
+  }
+  uint4 const e = t.bmp[0x10000u + cp];
+  d0            = e.x;
+  d1            = e.y;
+  d2            = e.z;
+  return e.w;
+}
+
 // Bytes that the character whose bytes start `w` produces, without its slots.
 __device__ __forceinline__ uint32_t wide_size(uint32_t w, NormTables const& t)
 {
@@ -295,8 +332,7 @@ __device__ __forceinline__ uint32_t owned_slots(NormLds<S> const& lds, uint64_t 
 #pragma unroll
   for (int j = 0; j < kNormItems; ++j) {
     uint32_t const b = static_cast<uint32_t>(lo64 >> (8 * j)) & 0xFFu;
-    uint32_t const e = lds.ascii[b & 0x7Fu];  // read in any case: no branch
-    uint32_t const d = b < 0x80u ? e : 0u;
+    uint32_t const d = lds.ascii[b];
     mine.s[j][0]     = d & 0xFFu;
     mine.s[j][1]     = (d >> 8) & 0xFFu;
     mine.s[j][2]     = (d >> 16) & 0xFFu;
@@ -326,20 +362,6 @@ __device__ __forceinline__ uint32_t owned_slots(NormLds<S> const& lds, uint64_t 
   return sum;
 }
 
-// The bytes of up to three slots side by side, first slot first: (lo, hi) = bytes 0..7 and 8..11.
-__device__ __forceinline__ void slots_to_string(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t& d0, uint32_t& d1, uint32_t& d2)
-{
-  uint32_t const b0  = bytes_of(s0);
-  uint32_t const b01 = b0 + bytes_of(s1);  // <= 8
-  uint64_t lo        = s0 | (static_cast<uint64_t>(s1) << (8u * b0));
-  uint64_t const t   = s2;
-  uint32_t const sh  = 8u * b01;
-  lo |= b01 < 8u ? t << (sh & 63u) : 0ull;
-  d2 = b01 >= 8u ? s2 : b01 > 4u ? static_cast<uint32_t>(t >> ((64u - sh) & 63u)) : 0u;
-  d0 = static_cast<uint32_t>(lo);
-  d1 = static_cast<uint32_t>(lo >> 32);
-}
-
 // owned_slots for the pass that writes: what each position turns into as a string of bytes (mine.s[j][0..2] = bytes
 // 0..11, zero padded) instead of slots, ready to be placed.
 template <bool S>
@@ -350,30 +372,33 @@ __device__ __forceinline__ uint32_t owned_strings(NormLds<S> const& lds, uint64_
 #pragma unroll
   for (int j = 0; j < kNormItems; ++j) {
     uint32_t const b = static_cast<uint32_t>(lo64 >> (8 * j)) & 0xFFu;
-    uint32_t const e = lds.ascii[b & 0x7Fu];  // read in any case: no branch
-    uint32_t const d = b < 0x80u ? e : 0u;
+    uint32_t const d = lds.ascii[b];
     mine.s[j][0]     = d & 0xFFFFFFu;  // one byte per slot, empty slots last: the slots side by side are the string
     mine.s[j][1]     = 0u;
     mine.s[j][2]     = 0u;
     size[j]          = d >> 24;
     sum += size[j];
   }
+  mine.widest    = 3u;
   uint64_t leads = lo64 & (lo64 << 1) & 0x8080808080808080ull;  // bit 7 of the bytes >= 0xC0
   while (leads) {
     int const at = (__ffsll(static_cast<long long>(leads)) - 1) >> 3;
     leads &= leads - 1ull;
     uint32_t const w = static_cast<uint32_t>((at < 4 ? lo64 : hi64) >> (8 * (at & 3)));
-    uint32_t s0, s1, s2, d0, d1, d2;
-    uint32_t const bytes = wide_slots(w, t, s0, s1, s2);
-    slots_to_string(s0, s1, s2, d0, d1, d2);
+    uint32_t d0, d1, d2;
+    uint32_t const bytes = wide_string(w, t, d0, d1, d2);
     sum += bytes;
+    mine.widest = max(mine.widest, bytes);
 #pragma unroll
     for (int j = 0; j < kNormItems; ++j) {
       uint32_t const here = static_cast<uint32_t>((static_cast<int32_t>(j ^ at) - 1) >> 31);  // all ones where j == at
       mine.s[j][0] = (mine.s[j][0] & ~here) | (d0 & here);
       mine.s[j][1] = (mine.s[j][1] & ~here) | (d1 & here);
-      mine.s[j][2] = (mine.s[j][2] & ~here) | (d2 & here);
       size[j]      = (size[j] & ~here) | (bytes & here);
+    }
+    if (ballot64(bytes > 8u) != 0) {  // (seldom: the third dwords are zeros otherwise)
+#pragma unroll
+      for (int j = 0; j < kNormItems; ++j) mine.s[j][2] = j == at ? d2 : mine.s[j][2];
     }
   }
   return sum;
@@ -399,8 +424,7 @@ __device__ __forceinline__ uint32_t owned_dense(NormLds<SLOTS>& lds, uint64_t lo
 #pragma unroll
   for (int j = 0; j < kNormItems; ++j) {
     uint32_t const b = static_cast<uint32_t>(lo64 >> (8 * j)) & 0xFFu;
-    uint32_t const e = lds.ascii[b & 0x7Fu];  // read in any case: no branch
-    sum += b < 0x80u ? e >> 24 : 0u;
+    sum += lds.sizes[b];
   }
   uint64_t const leads  = lo64 & (lo64 << 1) & 0x8080808080808080ull;  // bit 7 of the bytes >= 0xC0
   uint32_t const mine_n = static_cast<uint32_t>(__builtin_popcountll(leads));
@@ -447,7 +471,8 @@ __device__ __forceinline__ uint32_t tile_slots(NormLds<SLOTS>& lds, const uint8_
   int const tid = threadIdx.x;
   // stage [t0 - kRawBefore, t0 + kNormTile + kRawAfter) with one aligned 16-byte load per lane (the first 131 lanes);
   // bytes outside [0, n) read as 0.  Everything is requested before anything is waited for.
-  uint32_t const table_entry = tid < 128 ? t.ascii[tid] : 0u;
+  static_assert(kNormThreads == 256, "a table entry per lane");
+  uint32_t const table_entry = t.ascii[tid];
   const uint8_t* const wb    = chars + t0 - kRawBefore;
   uint32_t const mis         = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(wb) & 15u);
   if (tid < kRawWords / 4) {
@@ -469,7 +494,8 @@ __device__ __forceinline__ uint32_t tile_slots(NormLds<SLOTS>& lds, const uint8_
     }
     *reinterpret_cast<uint4*>(&lds.raw[4 * tid]) = v;
   }
-  if (tid < 128) lds.ascii[tid] = table_entry;
+  lds.ascii[tid] = table_entry;
+  if constexpr (!SLOTS) lds.sizes[tid] = static_cast<uint8_t>(table_entry >> 24);
   if (tid == 0) lds.bracket = 0u;
   lds_barrier();
 
@@ -545,7 +571,8 @@ __device__ __forceinline__ uint32_t tile_slots(NormLds<SLOTS>& lds, const uint8_
       lds_barrier();
       apply_special_tokens(lds, t);
       // the tokens only ever empty a slot or turn its letter into upper case: take over the first bytes that changed
-      sum = 0;
+      sum         = 0;
+      mine.widest = 0;
 #pragma unroll
       for (int j = 0; j < kNormItems; ++j) {
 #pragma unroll
@@ -568,6 +595,7 @@ __device__ __forceinline__ uint32_t tile_slots(NormLds<SLOTS>& lds, const uint8_
         }
         size[j] = bytes_of(mine.s[j][0]) + bytes_of(mine.s[j][1]) + bytes_of(mine.s[j][2]);
         sum += size[j];
+        mine.widest = max(mine.widest, size[j]);
         if (SLOTS) slots_to_string(mine.s[j][0], mine.s[j][1], mine.s[j][2], mine.s[j][0], mine.s[j][1], mine.s[j][2]);
       }
     }
@@ -735,10 +763,7 @@ __global__ void __launch_bounds__(kNormThreads) normalize_write_kernel(ColView c
     uint8_t* const sb   = reinterpret_cast<uint8_t*>(lds.staged);
     uint32_t o          = lead + before;
     uint32_t const mine_end = o + sum;
-    uint32_t big = 0;
-#pragma unroll
-    for (int j = 0; j < kNormItems; ++j) big |= (mine.s[j][0] >> 24) | mine.s[j][1] | mine.s[j][2];
-    if (ballot64(big != 0u) == 0) {
+    if (ballot64(mine.widest > 3u) == 0) {
       // no position of the wavefront turns into more than three bytes: a position's bytes travel together, as one
       // (unaligned) dword whose spare bytes the next positions overwrite.  A position that starts in the lane's last
       // three bytes is skipped; those bytes are kept in `last` (the four bytes written last, newest on top) and
@@ -757,8 +782,7 @@ __global__ void __launch_bounds__(kNormThreads) normalize_write_kernel(ColView c
     } else {
       // longer strings: every position's bytes (zero padded) are or-ed into the aligned dwords they fall into;
       // the buffer was cleared, and what the neighbours put into a shared dword is theirs
-      bool const past8 = ballot64(mine.s[0][2] | mine.s[1][2] | mine.s[2][2] | mine.s[3][2] | mine.s[4][2] | mine.s[5][2] | mine.s[6][2] |
-                                  mine.s[7][2]) != 0;
+      bool const past8 = ballot64(mine.widest > 8u) != 0;
 #pragma unroll
       for (int j = 0; j < kNormItems; ++j) {
         uint32_t const sh   = 8u * (o & 3u);
@@ -937,7 +961,7 @@ nvtext_amd_status nvtext_amd_character_normalizer_create(int32_t do_lower_case, 
   }
 
   // the slots of the one-byte code points, decided here once (the rules of slots_of)
-  uint32_t ascii[128];
+  uint32_t ascii[256] = {};
   for (uint32_t cp = 0; cp < 128u; ++cp) {
     uint32_t const e = entries[cp], cat = (e >> 24) & 7u;
     uint32_t d       = 0;
@@ -950,13 +974,16 @@ nvtext_amd_status nvtext_amd_character_normalizer_create(int32_t do_lower_case, 
   }
 
   // the finished slots of the Basic Multilingual Plane (the rules of slots_of, run here once per code point)
-  std::vector<uint4> bmp(0x10000);
+  std::vector<uint4> bmp(2 * 0x10000);
   {
     NormTables const host_tables{nullptr, nullptr, entries.data(), second.data(), nullptr, nullptr, 0, do_lower_case ? 1 : 0};
     for (uint32_t cp = 0; cp < 0x10000u; ++cp) {
       uint32_t s0, s1, s2;
       slots_of(cp, host_tables, s0, s1, s2);
       bmp[cp] = make_uint4(s0, s1, s2, bytes_of(s0) + bytes_of(s1) + bytes_of(s2));
+      uint32_t d0, d1, d2;
+      slots_to_string(s0, s1, s2, d0, d1, d2);
+      bmp[0x10000 + cp] = make_uint4(d0, d1, d2, bmp[cp].w);
     }
   }
 
@@ -980,7 +1007,7 @@ nvtext_amd_status nvtext_amd_character_normalizer_create(int32_t do_lower_case, 
   }
   hipError_t e = hipGetDevice(&obj->device);
   if (e != hipSuccess) return fail_with(e);
-  bool ok = obj->store.allocate(&obj->ascii, 128) && obj->store.allocate(&obj->bmp, bmp.size()) &&
+  bool ok = obj->store.allocate(&obj->ascii, 256) && obj->store.allocate(&obj->bmp, bmp.size()) &&
             obj->store.allocate(&obj->entries, entries.size()) && obj->store.allocate(&obj->second, second.size());
   if (ok && !tokens.empty())
     ok = obj->store.allocate(&obj->token_offset, token_offsets.size()) && obj->store.allocate(&obj->token_chars, std::max<size_t>(token_chars.size(), 1));
