@@ -462,11 +462,14 @@ __device__ __forceinline__ uint32_t owned_dense(NormLds<SLOTS>& lds, uint64_t lo
   return sum;
 }
 
-// One tile: the slots of the lane's positions, special tokens applied.  Returns the bytes they produce.  Without
-// SLOTS only that number is wanted: the slots are then built only in tiles that may hold a special token.
+// The lane's eight bytes of a tile and the four after them, the tile staged in LDS with its surroundings, the ASCII table
+// beside it; `mis`: what the tile's alignment puts in front of them.
+struct OwnBytes {
+  uint32_t own0, own1, next;
+  uint32_t mis, shift;
+};
 template <bool SLOTS>
-__device__ __forceinline__ uint32_t tile_slots(NormLds<SLOTS>& lds, const uint8_t* chars, int64_t t0, int64_t n, NormTables const& t, Owned& mine,
-                                               uint32_t (&size)[kNormItems])
+__device__ __forceinline__ OwnBytes stage_tile(NormLds<SLOTS>& lds, const uint8_t* chars, int64_t t0, int64_t n, NormTables const& t)
 {
   int const tid = threadIdx.x;
   // stage [t0 - kRawBefore, t0 + kNormTile + kRawAfter) with one aligned 16-byte load per lane (the first 131 lanes);
@@ -506,6 +509,18 @@ __device__ __forceinline__ uint32_t tile_slots(NormLds<SLOTS>& lds, const uint8_
   uint32_t const own0 = __builtin_amdgcn_alignbit(r1, r0, shift);
   uint32_t const own1 = __builtin_amdgcn_alignbit(r2, r1, shift);
   uint32_t const next = __builtin_amdgcn_alignbit(r3, r2, shift);
+  return OwnBytes{own0, own1, next, mis, shift};
+}
+
+// One tile: the slots of the lane's positions, special tokens applied.  Returns the bytes they produce.  Without
+// SLOTS only that number is wanted: the slots are then built only in tiles that may hold a special token.
+template <bool SLOTS>
+__device__ __forceinline__ uint32_t tile_slots(NormLds<SLOTS>& lds, const uint8_t* chars, int64_t t0, int64_t n, NormTables const& t, Owned& mine,
+                                               uint32_t (&size)[kNormItems])
+{
+  int const tid      = threadIdx.x;
+  OwnBytes const own = stage_tile(lds, chars, t0, n, t);
+  uint32_t const own0 = own.own0, own1 = own.own1, next = own.next, mis = own.mis, shift = own.shift;
   uint64_t const lo64 = (static_cast<uint64_t>(own1) << 32) | own0;
   uint64_t const hi64 = (static_cast<uint64_t>(next) << 32) | own1;
   // (the pass that wants the slots keeps them in registers all the way: listing the longer characters for it as well
@@ -704,32 +719,104 @@ __global__ void __launch_bounds__(256) normalize_tile_rows_kernel(ColView col, i
   tile_row[tile] = static_cast<int32_t>(lo);
 }
 
-// Writes the tile's bytes at tile_offset[tile] and the output offset of every row that starts in the tile.
-__global__ void __launch_bounds__(kNormThreads) normalize_write_kernel(ColView col, int64_t first, int64_t n, NormTables t,
-                                                                       const uint64_t* __restrict__ tile_offset,
-                                                                       const int32_t* __restrict__ tile_row, uint8_t* __restrict__ out_chars,
-                                                                       void* __restrict__ out_offsets, int offsets_are_int64)
-{
-  __shared__ NormLds<true> lds;
-  int const tid        = threadIdx.x;
-  int64_t const t0     = static_cast<int64_t>(blockIdx.x) * kNormTile;
-  uint64_t const base  = tile_offset[blockIdx.x];
-  // the rows that start in this tile are looked up now; the barriers below do not wait for global loads, so this
-  // one is back when the tile is done
-  int64_t const rows     = col.size;
-  int64_t const my_row   = static_cast<int64_t>(tile_row[blockIdx.x]) + tid;
-  // the rows that start in this tile end where the next tile's begin (the last tile also takes the end of the last row)
-  int64_t const row_end  = blockIdx.x + 1 == gridDim.x ? rows + 1 : static_cast<int64_t>(tile_row[blockIdx.x + 1]);
-  uint32_t start_lo = 0, start_hi = 0;  // the raw offset entry; not touched before the end
-  if (my_row <= rows) {
-    if (col.is64) {
-      uint2 const v = static_cast<const uint2*>(col.offsets)[my_row + col.offset];
-      start_lo      = v.x;
-      start_hi      = v.y;
-    } else {
-      start_lo = static_cast<const uint32_t*>(col.offsets)[my_row + col.offset];
+// The rows that start in a tile: looked up when the tile begins (the barriers do not wait for global loads, so that the
+// lane's own is back when the tile is done), given their places at its end.
+struct TileRows {
+  int64_t my_row, row_end;
+  uint32_t start_lo, start_hi;  // the raw offset entry of my_row; not touched before the end
+  __device__ __forceinline__ void request(ColView const& col, const int32_t* tile_row, uint32_t tile, uint32_t tiles)
+  {
+    int64_t const rows = col.size;
+    my_row             = static_cast<int64_t>(tile_row[tile]) + threadIdx.x;
+    // the rows that start in this tile end where the next tile's begin (the last tile also takes the end of the last row)
+    row_end  = tile + 1 == tiles ? rows + 1 : static_cast<int64_t>(tile_row[tile + 1]);
+    start_lo = start_hi = 0;
+    if (my_row <= rows) {
+      if (col.is64) {
+        uint2 const v = static_cast<const uint2*>(col.offsets)[my_row + col.offset];
+        start_lo      = v.x;
+        start_hi      = v.y;
+      } else {
+        start_lo = static_cast<const uint32_t*>(col.offsets)[my_row + col.offset];
+      }
     }
   }
+  // rows whose first byte lies in [t0, t1) -- in [t0, n] for the last tile -- start at base + prefix
+  __device__ __forceinline__ void place(ColView const& col, int64_t first, int64_t t0, uint64_t base, const uint16_t* prefix, void* out_offsets,
+                                        int offsets_are_int64) const
+  {
+    int64_t const my_start = (col.is64 ? static_cast<int64_t>((static_cast<uint64_t>(start_hi) << 32) | start_lo)
+                                       : static_cast<int64_t>(static_cast<int32_t>(start_lo))) - first;
+    for (int64_t r = my_row; r < row_end; r += kNormThreads) {  // (more than one trip only in a tile of very short rows)
+      int64_t const p   = r == my_row ? my_start : col.off(r) - first;
+      uint64_t const at = base + prefix[p - t0];
+      if (offsets_are_int64) static_cast<int64_t*>(out_offsets)[r] = static_cast<int64_t>(at);
+      else static_cast<int32_t*>(out_offsets)[r] = static_cast<int32_t>(at);
+    }
+  }
+};
+
+// The tile's bytes from LDS, where they lie as they will lie in memory from the dword at or below dst on, to memory.
+__device__ __forceinline__ void store_staged(const uint32_t* staged, uint8_t* dst, uint32_t lead, uint32_t total)
+{
+  int const tid           = threadIdx.x;
+  const uint8_t* const sb = reinterpret_cast<const uint8_t*>(staged);
+  uint32_t const end      = lead + total;
+  uint32_t const w_lo     = (lead + 3u) >> 2;
+  uint32_t const w_hi     = end >> 2;
+  uint32_t* const dw      = reinterpret_cast<uint32_t*>(dst - lead);
+  for (uint32_t w = w_lo + tid; w < w_hi; w += kNormThreads) store_stream(dw + w, staged[w]);
+  uint32_t const head_end   = min(4u * w_lo, end);
+  uint32_t const tail_begin = max(4u * w_hi, head_end);
+  if (tid < 4) {
+    uint32_t const at = lead + tid;
+    if (at < head_end) (dst - lead)[at] = sb[at];
+  } else if (tid < 8) {
+    uint32_t const at = tail_begin + (tid - 4);
+    if (at < end) (dst - lead)[at] = sb[at];
+  }
+}
+
+// The buffer that the output bytes are assembled in starts out as zeros.
+__device__ __forceinline__ void clear_staged(NormLds<true>& lds)
+{
+  int const tid = threadIdx.x;
+  for (int i = tid; i < static_cast<int>(sizeof(lds.staged) / 16); i += kNormThreads) reinterpret_cast<uint4*>(lds.staged)[i] = make_uint4(0u, 0u, 0u, 0u);
+  if (tid < static_cast<int>(sizeof(lds.staged) % 16) / 4) lds.staged[sizeof(lds.staged) / 16 * 4 + tid] = 0u;
+}
+
+// A lane's eight one-byte characters (three bytes at most each, `text` in the low bytes, their number in the top one) in a
+// wavefront that has no others: a position's bytes travel together, as one (unaligned) dword whose spare bytes the next
+// positions overwrite.  A position that starts in the lane's last three bytes is skipped; those bytes are kept in `last`
+// (the four bytes written last, newest on top) and stored one by one at the end.  o: where the lane's bytes go, sum: their
+// number.
+template <typename Text, typename Size>
+__device__ __forceinline__ void place_short(uint8_t* sb, uint32_t o, uint32_t sum, Text const& text, Size const& size)
+{
+  uint32_t const mine_end = o + sum;
+  uint32_t last           = 0;
+#pragma unroll
+  for (int j = 0; j < kNormItems; ++j) {
+    uint32_t const three = text(j), n = size(j);
+    if (n != 0u && o + 4u <= mine_end) __builtin_memcpy(sb + o, &three, 4);
+    last = __builtin_amdgcn_alignbit(three, last, 8u * n);
+    o += n;
+  }
+  if (sum >= 1u) sb[mine_end - 1u] = static_cast<uint8_t>(last >> 24);
+  if (sum >= 2u) sb[mine_end - 2u] = static_cast<uint8_t>(last >> 16);
+  if (sum >= 3u) sb[mine_end - 3u] = static_cast<uint8_t>(last >> 8);
+}
+
+// Writes the tile's bytes at tile_offset[tile] and the output offset of every row that starts in the tile.
+__device__ __forceinline__ void write_tile(NormLds<true>& lds, uint32_t tile, uint32_t tiles, ColView const& col, int64_t first, int64_t n,
+                                           NormTables const& t, const uint64_t* tile_offset, const int32_t* tile_row, uint8_t* out_chars,
+                                           void* out_offsets, int offsets_are_int64)
+{
+  int const tid        = threadIdx.x;
+  int64_t const t0     = static_cast<int64_t>(tile) * kNormTile;
+  uint64_t const base  = tile_offset[tile];
+  TileRows tile_rows;
+  tile_rows.request(col, tile_row, tile, tiles);
   Owned mine;
   uint32_t size[kNormItems];
   uint32_t const sum = tile_slots<true>(lds, col.chars + first, t0, n, t, mine, size);
@@ -737,8 +824,7 @@ __global__ void __launch_bounds__(kNormThreads) normalize_write_kernel(ColView c
   // and the first byte placed); in a tile that went through the special tokens it lies where the slots' first bytes
   // were, which the other wavefronts may still be reading
   if (t.tokens > 0 && lds.bracket != 0u) lds_barrier();
-  for (int i = tid; i < static_cast<int>(sizeof(lds.staged) / 16); i += kNormThreads) reinterpret_cast<uint4*>(lds.staged)[i] = make_uint4(0u, 0u, 0u, 0u);
-  if (tid < static_cast<int>(sizeof(lds.staged) % 16) / 4) lds.staged[sizeof(lds.staged) / 16 * 4 + tid] = 0u;
+  clear_staged(lds);
   uint32_t total;
   uint32_t const before = block_exclusive_scan_lds<kNormThreads>(sum, lds.scan, &total);
   {
@@ -762,23 +848,9 @@ __global__ void __launch_bounds__(kNormThreads) normalize_write_kernel(ColView c
     uint32_t const lead = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(dst) & 3u);
     uint8_t* const sb   = reinterpret_cast<uint8_t*>(lds.staged);
     uint32_t o          = lead + before;
-    uint32_t const mine_end = o + sum;
     if (ballot64(mine.widest > 3u) == 0) {
-      // no position of the wavefront turns into more than three bytes: a position's bytes travel together, as one
-      // (unaligned) dword whose spare bytes the next positions overwrite.  A position that starts in the lane's last
-      // three bytes is skipped; those bytes are kept in `last` (the four bytes written last, newest on top) and
-      // stored one by one at the end.
-      uint32_t last = 0;
-#pragma unroll
-      for (int j = 0; j < kNormItems; ++j) {
-        uint32_t const three = mine.s[j][0];
-        if (size[j] != 0u && o + 4u <= mine_end) __builtin_memcpy(sb + o, &three, 4);
-        last = __builtin_amdgcn_alignbit(three, last, 8u * size[j]);
-        o += size[j];
-      }
-      if (sum >= 1u) sb[mine_end - 1u] = static_cast<uint8_t>(last >> 24);
-      if (sum >= 2u) sb[mine_end - 2u] = static_cast<uint8_t>(last >> 16);
-      if (sum >= 3u) sb[mine_end - 3u] = static_cast<uint8_t>(last >> 8);
+      // no position of the wavefront turns into more than three bytes
+      place_short(sb, o, sum, [&](int j) { return mine.s[j][0]; }, [&](int j) { return size[j]; });
     } else {
       // longer strings: every position's bytes (zero padded) are or-ed into the aligned dwords they fall into;
       // the buffer was cleared, and what the neighbours put into a shared dword is theirs
@@ -801,20 +873,7 @@ __global__ void __launch_bounds__(kNormThreads) normalize_write_kernel(ColView c
       }
     }
     lds_barrier();
-    uint32_t const end  = lead + total;
-    uint32_t const w_lo = (lead + 3u) >> 2;
-    uint32_t const w_hi = end >> 2;
-    uint32_t* const dw  = reinterpret_cast<uint32_t*>(dst - lead);
-    for (uint32_t w = w_lo + tid; w < w_hi; w += kNormThreads) store_stream(dw + w, lds.staged[w]);
-    uint32_t const head_end   = min(4u * w_lo, end);
-    uint32_t const tail_begin = max(4u * w_hi, head_end);
-    if (tid < 4) {
-      uint32_t const at = lead + tid;
-      if (at < head_end) (dst - lead)[at] = sb[at];
-    } else if (tid < 8) {
-      uint32_t const at = tail_begin + (tid - 4);
-      if (at < end) (dst - lead)[at] = sb[at];
-    }
+    store_staged(lds.staged, dst, lead, total);
   } else {
     // more than four output bytes per input byte (only input that is not UTF-8 gets there): byte by byte
     uint8_t* o = dst + before;
@@ -824,15 +883,129 @@ __global__ void __launch_bounds__(kNormThreads) normalize_write_kernel(ColView c
     lds_barrier();  // lds.prefix is complete for the rows below
   }
 
-  // rows whose first byte lies in [t0, t1) -- in [t0, n] for the last tile -- start at base + prefix
-  int64_t const my_start = (col.is64 ? static_cast<int64_t>((static_cast<uint64_t>(start_hi) << 32) | start_lo)
-                                     : static_cast<int64_t>(static_cast<int32_t>(start_lo))) - first;
-  for (int64_t r = my_row; r < row_end; r += kNormThreads) {  // (more than one trip only in a tile of very short rows)
-    int64_t const p = r == my_row ? my_start : col.off(r) - first;
-    uint64_t const at = base + lds.prefix[p - t0];
-    if (offsets_are_int64) static_cast<int64_t*>(out_offsets)[r] = static_cast<int64_t>(at);
-    else static_cast<int32_t*>(out_offsets)[r] = static_cast<int32_t>(at);
+  tile_rows.place(col, first, t0, base, lds.prefix, out_offsets, offsets_are_int64);
+}
+
+// The same, done here for ordinary text; tiles that may hold a special token, characters that turn into more than eight
+// bytes and more first bytes of longer characters side by side than text has go through write_tile().
+// What bounds it is the number of vector instructions (400 a wavefront, issued in 83 % of the cycles).  A lane keeps its one-byte characters as the table gives them and
+// up to four longer ones beside them, each in registers of its own (instead of a string for every position, into which
+// a longer character was selected eight times); where each goes in the lane's output comes from the eight sizes, a byte
+// each, multiplied by 0x01..01.
+constexpr int kLongChars = 4;  // of two bytes and more in eight bytes
+__global__ void __launch_bounds__(kNormThreads, 6) normalize_write_kernel(ColView col, int64_t first, int64_t n, NormTables t,
+                                                                       const uint64_t* __restrict__ tile_offset,
+                                                                       const int32_t* __restrict__ tile_row, uint8_t* __restrict__ out_chars,
+                                                                       void* __restrict__ out_offsets, int offsets_are_int64)
+{
+  __shared__ NormLds<true> lds;
+  int const tid       = threadIdx.x;
+  uint32_t const tile = blockIdx.x;
+  int64_t const t0    = static_cast<int64_t>(tile) * kNormTile;
+  uint64_t const base = tile_offset[tile];
+  TileRows tile_rows;
+  tile_rows.request(col, tile_row, tile, gridDim.x);
+  OwnBytes const own  = stage_tile(lds, col.chars + first, t0, n, t);
+  uint64_t const lo64 = (static_cast<uint64_t>(own.own1) << 32) | own.own0;
+  uint64_t const hi64 = (static_cast<uint64_t>(own.next) << 32) | own.own1;
+  uint32_t text[kNormItems];
+#pragma unroll
+  for (int j = 0; j < kNormItems; ++j) text[j] = lds.ascii[static_cast<uint32_t>(lo64 >> (8 * j)) & 0xFFu];
+  // the sizes of the positions, a byte each
+  auto const top_bytes = [](uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+    return __builtin_amdgcn_perm(b, a, 0x0c0c0703u) | __builtin_amdgcn_perm(d, c, 0x07030c0cu);
+  };
+  uint64_t sizes = (static_cast<uint64_t>(top_bytes(text[4], text[5], text[6], text[7])) << 32) | top_bytes(text[0], text[1], text[2], text[3]);
+  uint64_t leads = lo64 & (lo64 << 1) & 0x8080808080808080ull;  // bit 7 of the bytes >= 0xC0
+  bool const any_long = ballot64(leads != 0) != 0;
+  bool other          = false;  // the tile is not for this kernel
+  uint32_t d0[kLongChars] = {}, d1[kLongChars] = {}, at8[kLongChars] = {};
+  if (any_long) {
+    // all reads of the table in flight together
+    uint4 e[kLongChars];
+#pragma unroll
+    for (int k = 0; k < kLongChars; ++k) {
+      bool const have    = leads != 0;
+      uint32_t const bit = static_cast<uint32_t>(__builtin_ctzll(leads | 0x8000000000000000ull));  // 8 * position + 7
+      leads &= leads - 1ull;
+      at8[k]           = bit - 7u;
+      uint32_t const w = static_cast<uint32_t>((bit < 32u ? lo64 : hi64) >> (at8[k] & 31u));
+      e[k]             = make_uint4(0u, 0u, 0u, 0u);
+      if (have) e[k] = t.bmp[0x10000u + decode_short(w)];
+      if (ballot64(have && (w & 0xFFu) >= 0xF0u) != 0) {  // four bytes (seldom)
+        if (have && (w & 0xFFu) >= 0xF0u) e[k].w = wide_string(w, t, e[k].x, e[k].y, e[k].z);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kLongChars; ++k) {
+      d0[k] = e[k].x;
+      d1[k] = e[k].y;
+      sizes += static_cast<uint64_t>(e[k].w) << at8[k];
+      other = other || e[k].w > 8u || d0[k] == 0x205B20u;  // (" [ ": an over-long '[')
+    }
   }
+  other = other || leads != 0;
+  if (t.tokens > 0) {
+    other = other || has_byte(own.own0, '[') || has_byte(own.own1, '[');
+    if (tid < kNormItems) {  // the positions before the tile (five needed): a '[' or an over-long one
+      const uint8_t* const b = reinterpret_cast<const uint8_t*>(lds.raw) + own.mis + tid;
+      static_assert(kRawBefore == kNormItems, "the bytes staged before the tile");
+      other = other || b[0] == '[' || b[0] == 0xC1u || (b[0] == 0xE0u && b[1] < 0xA0u) || (b[0] == 0xF0u && b[1] < 0x90u);
+    }
+  }
+  if (ballot64(other) != 0 && lane_id() == 0) lds.bracket = 1u;
+  clear_staged(lds);
+  // where each position's bytes begin in the lane's: the sums of the sizes before it (96 at most)
+  uint32_t const in0 = static_cast<uint32_t>(sizes) * 0x01010101u;
+  uint32_t const in1 = static_cast<uint32_t>(sizes >> 32) * 0x01010101u + (in0 >> 24) * 0x01010101u;
+  uint32_t const ex0 = in0 << 8, ex1 = __builtin_amdgcn_alignbit(in1, in0, 24);
+  uint32_t const sum = in1 >> 24;
+  uint32_t total;
+  uint32_t const before = block_exclusive_scan_lds<kNormThreads>(sum, lds.scan, &total);
+  if (lds.bracket != 0u || total > static_cast<uint32_t>(kStageBytes)) {
+    lds_barrier();  // (everybody has read that)
+    write_tile(lds, tile, gridDim.x, col, first, n, t, tile_offset, tile_row, out_chars, out_offsets, offsets_are_int64);
+    return;
+  }
+  {
+    uint32_t const both = before * 0x00010001u;
+    auto const two      = [&](uint32_t v, uint32_t which) { return __builtin_amdgcn_perm(0u, v, which) + both; };
+    *reinterpret_cast<uint4*>(&lds.prefix[kNormItems * tid]) =
+      make_uint4(two(ex0, 0x0c010c00u), two(ex0, 0x0c030c02u), two(ex1, 0x0c010c00u), two(ex1, 0x0c030c02u));
+    if (tid == kNormThreads - 1) lds.prefix[kNormTile] = static_cast<uint16_t>(before + sum);
+  }
+  uint8_t* const dst  = out_chars + base;
+  uint32_t const lead = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(dst) & 3u);
+  uint32_t const o    = lead + before;
+  if (!any_long) {
+    place_short(reinterpret_cast<uint8_t*>(lds.staged), o, sum, [&](int j) { return text[j] & 0xFFFFFFu; }, [&](int j) { return text[j] >> 24; });
+  } else {
+    // every string (zero padded) is or-ed into the aligned dwords it falls into; the buffer was cleared, and what the
+    // neighbours put into a shared dword is theirs
+#pragma unroll
+    for (int j = 0; j < kNormItems; ++j) {
+      uint32_t const at  = o + (((j < 4 ? ex0 : ex1) >> (8 * (j & 3))) & 0xFFu);
+      uint32_t* const to = lds.staged + (at >> 2);
+      uint64_t const v   = static_cast<uint64_t>(text[j] & 0xFFFFFFu) << (8u * (at & 3u));
+      atomicOr(to, static_cast<uint32_t>(v));
+      atomicOr(to + 1, static_cast<uint32_t>(v >> 32));
+    }
+    uint64_t const ex = (static_cast<uint64_t>(ex1) << 32) | ex0;
+#pragma unroll
+    for (int k = 0; k < kLongChars; ++k) {
+      if (ballot64(d0[k] != 0u) == 0) break;  // (a lane's are its first ones; one that turns into nothing has no dword either)
+      uint32_t const at  = o + (static_cast<uint32_t>(ex >> at8[k]) & 0xFFu);
+      uint32_t const sh  = 8u * (at & 3u);
+      uint32_t* const to = lds.staged + (at >> 2);
+      uint64_t const a = static_cast<uint64_t>(d0[k]) << sh, b = static_cast<uint64_t>(d1[k]) << sh;
+      atomicOr(to, static_cast<uint32_t>(a));
+      atomicOr(to + 1, static_cast<uint32_t>(a >> 32) | static_cast<uint32_t>(b));
+      if (ballot64((b >> 32) != 0) != 0) atomicOr(to + 2, static_cast<uint32_t>(b >> 32));
+    }
+  }
+  lds_barrier();
+  store_staged(lds.staged, dst, lead, total);
+  tile_rows.place(col, first, t0, base, lds.prefix, out_offsets, offsets_are_int64);
 }
 
 struct TileBytes {
@@ -1167,8 +1340,7 @@ nvtext_amd_status nvtext_amd_normalize_characters(const nvtext_amd_strings_colum
   {
     ProfileScope ps("normalize_write_kernel", stream);
     hipLaunchKernelGGL(normalize_write_kernel, dim3(static_cast<unsigned>(tiles)), dim3(kNormThreads), 0, stream, view, first, n, tables,
-                       tile_offset, tile_row, reinterpret_cast<uint8_t*>(out->chars), out->offsets,
-                       out->offsets_is_int64);
+                       tile_offset, tile_row, reinterpret_cast<uint8_t*>(out->chars), out->offsets, out->offsets_is_int64);
   }
   e = hipGetLastError();
   if (e != hipSuccess) return release(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
