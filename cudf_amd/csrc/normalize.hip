@@ -920,12 +920,14 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_kernel(ColVie
   bool const any_long = ballot64(leads != 0) != 0;
   bool other          = false;  // the tile is not for this kernel
   uint32_t d0[kLongChars] = {}, d1[kLongChars] = {}, at8[kLongChars] = {};
+  uint64_t holders[kLongChars] = {};  // the lanes that have a k-th longer character, whatever it turns into
   if (any_long) {
     // all reads of the table in flight together
     uint4 e[kLongChars];
 #pragma unroll
     for (int k = 0; k < kLongChars; ++k) {
       bool const have    = leads != 0;
+      holders[k]         = ballot64(have);
       uint32_t const bit = static_cast<uint32_t>(__builtin_ctzll(leads | 0x8000000000000000ull));  // 8 * position + 7
       leads &= leads - 1ull;
       at8[k]           = bit - 7u;
@@ -993,7 +995,7 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_kernel(ColVie
     uint64_t const ex = (static_cast<uint64_t>(ex1) << 32) | ex0;
 #pragma unroll
     for (int k = 0; k < kLongChars; ++k) {
-      if (ballot64(d0[k] != 0u) == 0) break;  // (a lane's are its first ones; one that turns into nothing has no dword either)
+      if (holders[k] == 0) break;
       uint32_t const at  = o + (static_cast<uint32_t>(ex >> at8[k]) & 0xFFu);
       uint32_t const sh  = 8u * (at & 3u);
       uint32_t* const to = lds.staged + (at >> 2);

@@ -143,6 +143,25 @@ def test_normalize_malformed_utf8(nv, onorm, do_lower):
             check(nv, onorm, strings(rows), do_lower, ["[PAD]"], f"over-long bracket {opener!r} shift {shift}")
 
 
+@pytest.mark.parametrize("tokens", [(), ("[x]",)])
+@pytest.mark.parametrize("do_lower", [True, False])
+def test_normalize_characters_that_turn_into_nothing(nv, onorm, do_lower, tokens):
+    # a character that is removed and one to three that are kept behind it, at every byte of a lane and of a wavefront,
+    # with nothing but ASCII around them; then the same in every lane
+    host_rows = []
+    for removed in "\ufeff\u200b\u00ad\ufffd\u0301":
+        for kept in ("\u00e9", "\u00e9\u00f1", "\u00fc\u6f22", "\u00e9\u0301\u00f1\u00fc", "\U0001f600\u00e9"):
+            for at in range(512):
+                host_rows.append(("a" * at + removed + kept).encode().ljust(1024, b"b"))
+    host = strings(host_rows)
+    exp = onorm.normalize_characters_native(host, do_lower, [t.encode() for t in tokens], nthreads=8)
+    assert_same(run(nv, host, do_lower, tokens), exp, "one in a wavefront")
+    host = strings([("x" * k + (removed + "\u00e9 abc") * 400) for removed in "\ufeff\u200b\u00ad\ufffd\u0301" for k in range(16)])
+    exp = onorm.normalize_characters_native(host, do_lower, [t.encode() for t in tokens], nthreads=8)
+    assert_same(run(nv, host, do_lower, tokens), exp, "in every lane")
+    assert run(nv, strings(["\ufeff\u00e9 abc", "\u200b\u00f1 x"]), True, tokens).to_pylist() == [b"e abc", b"n x"]
+
+
 def test_normalize_nulls_keep_their_bytes_and_empty_shapes(nv, onorm):
     # a null row whose offsets still span bytes: the flat pass normalizes them like any others
     base = strings(["Ab.", "Cd!", "", "Ef"])
