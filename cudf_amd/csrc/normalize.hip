@@ -466,7 +466,7 @@ __device__ __forceinline__ uint32_t owned_dense(NormLds<SLOTS>& lds, uint64_t lo
 // beside it; `mis`: what the tile's alignment puts in front of them.
 struct OwnBytes {
   uint32_t own0, own1, next;
-  uint32_t mis, shift;
+  uint32_t mis;
 };
 template <bool SLOTS>
 __device__ __forceinline__ OwnBytes stage_tile(NormLds<SLOTS>& lds, const uint8_t* chars, int64_t t0, int64_t n, NormTables const& t)
@@ -509,7 +509,20 @@ __device__ __forceinline__ OwnBytes stage_tile(NormLds<SLOTS>& lds, const uint8_
   uint32_t const own0 = __builtin_amdgcn_alignbit(r1, r0, shift);
   uint32_t const own1 = __builtin_amdgcn_alignbit(r2, r1, shift);
   uint32_t const next = __builtin_amdgcn_alignbit(r3, r2, shift);
-  return OwnBytes{own0, own1, next, mis, shift};
+  return OwnBytes{own0, own1, next, mis};
+}
+
+// Whether a special token may open in one of the eight positions before the tile (five needed): the first eight lanes
+// decode the character that begins at theirs, so that an over-long '[' is one here exactly if it is one to the slots.
+// Both passes ask this: one that took a tile for free of tokens while the other applied them would give it another size.
+template <bool SLOTS>
+__device__ __forceinline__ bool opener_before(NormLds<SLOTS> const& lds, uint32_t mis)
+{
+  if (threadIdx.x >= kRawBefore) return false;
+  uint32_t const off = mis + threadIdx.x;
+  uint32_t const w   = __builtin_amdgcn_alignbit(lds.raw[(off >> 2) + 1], lds.raw[off >> 2], 8u * (off & 3u));
+  uint32_t const b0  = w & 0xFFu;
+  return b0 < 0xC0u ? b0 == '[' : decode(b0, (w >> 8) & 0xFFu, (w >> 16) & 0xFFu, w >> 24) == '[';
 }
 
 // One tile: the slots of the lane's positions, special tokens applied.  Returns the bytes they produce.  Without
@@ -520,7 +533,7 @@ __device__ __forceinline__ uint32_t tile_slots(NormLds<SLOTS>& lds, const uint8_
 {
   int const tid      = threadIdx.x;
   OwnBytes const own = stage_tile(lds, chars, t0, n, t);
-  uint32_t const own0 = own.own0, own1 = own.own1, next = own.next, mis = own.mis, shift = own.shift;
+  uint32_t const own0 = own.own0, own1 = own.own1, next = own.next, mis = own.mis;
   uint64_t const lo64 = (static_cast<uint64_t>(own1) << 32) | own0;
   uint64_t const hi64 = (static_cast<uint64_t>(next) << 32) | own1;
   // (the pass that wants the slots keeps them in registers all the way: listing the longer characters for it as well
@@ -533,8 +546,8 @@ __device__ __forceinline__ uint32_t tile_slots(NormLds<SLOTS>& lds, const uint8_
   if (t.tokens > 0) {
     // A special token starts at a position whose slot 1 is '['.  Tiles without one skip the exchange through LDS.
     // No code point's replacement is a '[', so it takes a '[' byte or an over-long encoding of it, which starts
-    // with 0xC1, 0xE0 or 0xF0: that is what decides for the positions before the tile (eight looked at, five
-    // needed) and, when the slots have not been built, for the lane's own bytes (a superset, which is harmless).
+    // with 0xC1, 0xE0 or 0xF0: that is what decides for the lane's own bytes when the slots have not been built (a
+    // superset, which is harmless).
     bool bracket = false;
     if (SLOTS) {
       // (strings: a '[' is padded like all punctuation, so it is the middle byte of " [ ")
@@ -546,11 +559,7 @@ __device__ __forceinline__ uint32_t tile_slots(NormLds<SLOTS>& lds, const uint8_
         bracket = bracket || has_byte(own0, 0xC1u) || has_byte(own0, 0xE0u) || has_byte(own0, 0xF0u) || has_byte(own1, 0xC1u) ||
                   has_byte(own1, 0xE0u) || has_byte(own1, 0xF0u);
     }
-    if (tid < 2) {
-      int const at     = static_cast<int>(mis >> 2) + tid;
-      uint32_t const v = __builtin_amdgcn_alignbit(lds.raw[at + 1], lds.raw[at], shift);
-      bracket          = bracket || has_byte(v, '[') || has_byte(v, 0xC1u) || has_byte(v, 0xE0u) || has_byte(v, 0xF0u);
-    }
+    bracket = bracket || opener_before(lds, mis);
     if (ballot64(bracket) != 0 && lane_id() == 0) lds.bracket = 1u;
     lds_barrier();
     if (lds.bracket != 0u) {
@@ -947,14 +956,7 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_kernel(ColVie
     }
   }
   other = other || leads != 0;
-  if (t.tokens > 0) {
-    other = other || has_byte(own.own0, '[') || has_byte(own.own1, '[');
-    if (tid < kNormItems) {  // the positions before the tile (five needed): a '[' or an over-long one
-      const uint8_t* const b = reinterpret_cast<const uint8_t*>(lds.raw) + own.mis + tid;
-      static_assert(kRawBefore == kNormItems, "the bytes staged before the tile");
-      other = other || b[0] == '[' || b[0] == 0xC1u || (b[0] == 0xE0u && b[1] < 0xA0u) || (b[0] == 0xF0u && b[1] < 0x90u);
-    }
-  }
+  if (t.tokens > 0) other = other || has_byte(own.own0, '[') || has_byte(own.own1, '[') || opener_before(lds, own.mis);
   if (ballot64(other) != 0 && lane_id() == 0) lds.bracket = 1u;
   clear_staged(lds);
   // where each position's bytes begin in the lane's: the sums of the sizes before it (96 at most)

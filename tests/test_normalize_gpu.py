@@ -162,6 +162,29 @@ def test_normalize_characters_that_turn_into_nothing(nv, onorm, do_lower, tokens
     assert run(nv, strings(["\ufeff\u00e9 abc", "\u200b\u00f1 x"]), True, tokens).to_pylist() == [b"e abc", b"n x"]
 
 
+# every encoding of '[' that decodes to it: the top two bits of the bytes behind the first do not matter
+OPENERS = [b"["] + [bytes([0xC1, c | 0x1B]) for c in (0, 0x40, 0x80, 0xC0)]
+OPENERS += [bytes([0xE0, b | 1, c | 0x1B]) for b in (0, 0x40, 0x80, 0xC0) for c in (0, 0x40, 0x80, 0xC0)]
+OPENERS += [bytes([0xF0, a, b | 1, c | 0x1B]) for a in (0, 0x40, 0x80, 0xC0) for b in (0, 0x40, 0x80, 0xC0) for c in (0, 0x40, 0x80, 0xC0)]
+
+
+@pytest.mark.parametrize("do_lower", [True, False])
+def test_normalize_openers_before_a_tile(nv, onorm, do_lower):
+    # a special token that opens in the last bytes of a tile of 2048 bytes and closes in the next, whatever the '[' is
+    # written as; then the same with the column's end behind it, and what only looks like one (0xE0 0xA1.., 0xF0 0x90..)
+    near = [b"\xc2\x9b", b"\xe0\x82\x9b", b"\xe0\xa1\x9b", b"\xf0\x90\x81\x9b", b"\xf1\x80\x81\x9b", b"\xf8\x80\x81\x9b", b"\xe1\x81\x9b"]
+    rows = [(b"a" * (2048 - 8 + shift) + opener + b"x] y").ljust(4096, b"b") for opener in OPENERS + near for shift in range(11)]
+    host = strings(rows)
+    exp = onorm.normalize_characters_native(host, do_lower, [b"[x]"], nthreads=8)
+    token = b"[X]" if do_lower else b"[x]"
+    assert sum(r.count(token) for r in exp.to_pylist()) >= 11 * 20  # (a second byte that begins a character of its own is no token)
+    assert_same(run(nv, host, do_lower, ["[x]"]), exp, "between tiles")
+    for opener in OPENERS:
+        for shift in (3, 5, 7):
+            host = strings([b"a" * (2048 - 8 + shift) + opener + b"x]"])
+            check(nv, onorm, host, do_lower, ["[x]"], f"{opener!r} shift {shift}, the last tile")
+
+
 def test_normalize_nulls_keep_their_bytes_and_empty_shapes(nv, onorm):
     # a null row whose offsets still span bytes: the flat pass normalizes them like any others
     base = strings(["Ab.", "Cd!", "", "Ef"])
