@@ -30,6 +30,7 @@ constexpr int kUnitShift   = 61 - kUnits;    // a unit is 2^44 of a product
 constexpr int kKeyShift    = 32 - kUnits;    // fractions are compared at the top of a dword; what is below says whose it is
 constexpr uint64_t kPrime  = (1ull << 61) - 1;
 constexpr uint32_t kNoKey  = 0xFFFFFFFFu;
+constexpr uint32_t kLargest = 0x4081FFFFu;   // a sum (between 4 and 8) with the largest fraction
 
 // What the host side of a call lays out for a group of 32 parameters: the registers of the two matrix instructions, lane
 // by lane, and the slack of every parameter.

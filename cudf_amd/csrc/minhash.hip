@@ -321,9 +321,13 @@ struct Minima64 {
   {
     wave_lds_fence();
     if (count == 0) return;
-    // the last block is filled up with different ones: with equal ones a least fraction would be the second least too
+    // The last block is filled up with hashes of the row, and their sums are set to the largest fraction: their digits are
+    // zeros, so that the sum is what it starts from.  (Left as they come out, a least fraction that the filling repeats is
+    // the second least of its lane as well, and all of the lane's hashes are computed exactly: one parameter in seven of a
+    // row of 56 windows.  200,000 lists of 30 elements, 128 parameters: 2282 -> 557 us; 1,000,003 rows of 512 bytes, 64
+    // parameters: 7251 -> 6818 us.)
     uint32_t const rest = (0u - count) & 31u;
-    if (static_cast<uint32_t>(lane) < rest) hashes[count + lane] = hashes[count > 32u ? static_cast<uint32_t>(lane) : static_cast<uint32_t>(lane) % count];
+    if (static_cast<uint32_t>(lane) < rest) hashes[count + lane] = hashes[0];
     wave_lds_fence();
     filter64::Sums start;
 #pragma unroll
@@ -333,7 +337,16 @@ struct Minima64 {
 #pragma unroll
     for (int g = 0; g < G; ++g) least[g] = second[g] = filter64::kNoKey;
     for (uint32_t block = 0; block < count; block += 32u) {
-      filter64::V8 const digits = filter64::digits_of(hashes[block + static_cast<uint32_t>(lane % 32)]);
+      filter64::V8 digits = filter64::digits_of(hashes[block + static_cast<uint32_t>(lane % 32)]);
+      if (count - block < 32u) {
+        int const left      = static_cast<int>(count - block);
+        int const mine      = lane % 32 < left ? -1 : 0;
+        int const left_here = left - static_cast<int>(filter64::hash_of_sum(0, lane));  // (compared with numbers that are the same in every lane)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) digits[d] &= mine;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) start[r] = static_cast<int>(filter64::hash_of_sum(r, 0)) < left_here ? start[r] : __uint_as_float(filter64::kLargest);
+      }
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         filter64::Sums const sums = filter64::sums_of(digits, pieces[g][0], pieces[g][1], scale[0], scale[1], start);

@@ -113,6 +113,18 @@ def test_minhash64_parameters(nv, orc, kind):
         assert nv.minhash64(dev(nv, column), 5, a, b, 5).to_host().equals(orc.minhash64(column, 5, a, b, 5, nthreads=8))
 
 
+@pytest.mark.parametrize("count", [1, 32, 33, 70, 128, 260])
+def test_minhash64_last_blocks(nv, orc, count):
+    """Rows of 1 to 130 windows and of some above 256: every fill of a block of 32 hashes, all of them different and with
+    one that repeats; the parameters in one group of 32 and in several."""
+    rng = np.random.default_rng(count)
+    a, b = params(rng, count, 64)
+    lens = list(range(5, 135)) + list(range(256, 300))
+    rows = [random_text(rng, n).decode() for n in lens] + ["ab" * (n // 2) + "xyz"[: n % 3] for n in lens]
+    host = HostStringsColumn.from_pylist(rows)
+    assert nv.minhash64(dev(nv, host), 5, a, b, 5).to_host().equals(orc.minhash64(host, 5, a, b, 5, nthreads=8))
+
+
 @pytest.mark.parametrize("bits", [32, 64])
 @pytest.mark.parametrize("ngrams", [2, 5])
 @pytest.mark.parametrize("count", [1, 130])
