@@ -11,8 +11,9 @@
 //     K running minima in registers and streams the tile's hashes through LDS
 //     broadcast reads, so the inner loop is v_mad_u64_u32 + v_min only;
 //   * a wavefront does a row alone, or a part of it: rows are cut into parts of at most 4 KiB (of
-//     fewer bytes in a column too small to give every wavefront of the device one of that size),
-//     and the parts of a row meet in the result with an atomic minimum;
+//     fewer bytes in a column too small to give every wavefront of the device several of that size),
+//     the parts of a row meet in the result with an atomic minimum, and the wavefronts take short rows
+//     several at a time;
 //   * in a tile with characters of more than one byte the wavefront lists the characters first,
 //     so that a lane takes a character and reads its window's length instead of walking to it;
 //     hashes that the wavefront has folded lately are dropped (a minimum does not mind).
@@ -29,11 +30,14 @@
 #include <type_traits>
 
 // Scratch of nvtext_amd_minhash_preallocated, the entry point that allocates nothing: the part counts of the
-// rows (rows + 1 values) and behind them the tile sums of the scans and the counter of the parts.  Every device holds its own copy of the array
-// for as long as the library is loaded (4.2 MB).
+// rows (rows + 1 values) and behind them the tile sums of the scans and the counters of the units of work.  Every device holds
+// its own copy of the array for as long as the library is loaded (4.2 MB).
 constexpr int32_t kPreallocatedMaxRows = NVTEXT_AMD_MINHASH_PREALLOCATED_MAX_ROWS;
 constexpr size_t kScratchPrefixBytes   = (static_cast<size_t>(kPreallocatedMaxRows) + 1 + 63) / 64 * 64 * sizeof(uint32_t);
-constexpr size_t kScratchScanBytes     = (static_cast<size_t>(kPreallocatedMaxRows) / nvtext_amd::kScanTile + 3) * sizeof(uint64_t);
+constexpr int kCounterGroups           = 32;    // counters of units of work
+constexpr int kCounterLine             = 16;    // 64-bit words from one to the next: a 128-byte line each
+constexpr size_t kCounterBytes         = (kCounterGroups + 1) * kCounterLine * sizeof(uint64_t);
+constexpr size_t kScratchScanBytes     = (static_cast<size_t>(kPreallocatedMaxRows) / nvtext_amd::kScanTile + 2 + 15) / 16 * 128 + kCounterBytes;
 static __device__ __align__(256) unsigned char scratch[kScratchPrefixBytes + kScratchScanBytes];
 
 namespace nvtext_amd {
@@ -408,11 +412,11 @@ template <typename T_>
 struct TextRows {
   using T   = T_;
   using Lds = WaveLds<T>;
-  static constexpr const char* kRowsName  = "minhash_rows_kernel";
-  static constexpr const char* kPartsName = "minhash_parts_kernel";
+  static constexpr const char* kName = "minhash_parts_kernel";
   static constexpr int kSimdWaves   = sizeof(T) == 4 ? 6 : 4;  // wavefronts per SIMD that its LDS leaves room for
   static constexpr int64_t kPart    = 4096;
   static constexpr int64_t kMinPart = kTile;  // less would be staged for its halo
+  static constexpr int kPartCost    = 64;
   ColView col;
   T seed;
   int32_t width;
@@ -530,11 +534,11 @@ template <typename T_>
 struct RunRows {
   using T   = T_;
   using Lds = RunLds<T>;
-  static constexpr const char* kRowsName  = "minhash_ngrams_rows_kernel";
-  static constexpr const char* kPartsName = "minhash_ngrams_parts_kernel";
+  static constexpr const char* kName = "minhash_ngrams_parts_kernel";
   static constexpr int kSimdWaves   = sizeof(T) == 4 ? 7 : 4;
   static constexpr int64_t kPart    = 1024;
   static constexpr int64_t kMinPart = kWave;
+  static constexpr int kPartCost    = 32;
   ListView col;
   T seed;
   int32_t ngrams;
@@ -600,48 +604,29 @@ struct RunRows {
   }
 };
 
-// How the rows are shared out.  In a column of at least kManyRows rows a wavefront does the rows of up to kPart
-// bytes alone, several in turn (minhash_rows_kernel), and the longer ones are cut into parts; in a column of fewer rows
-// every row is cut into parts (minhash_parts_kernel), so that the device is full whatever the rows' lengths: 999
-// documents of 2 KB (256 parameters) with a workgroup each, and another launch for what lay beyond their first 16 KB,
-// took 282 us for 23 us of arithmetic, most of it spent on the longest document; 42 us in parts.  20,011 rows of 16 KB
-// (uint64, 128 parameters) 9.0 -> 7.4 ms, the long rows of 400,000 documents of 2 KB 9.7 -> 9.2 ms.
-// A workgroup lasts as long as its slowest wavefront, and rows differ in length: with one row per wavefront the others
-// waited for the longest of four (8 M rows of about 500 bytes: 88 ms; four rows per wavefront 80 ms, sixteen 77 ms).
-// More rows per workgroup mean fewer workgroups, and the column needs them all to fill the device and to even out its
-// end: the host asks for as many rows per wavefront (a power of two, at most kMaxRowsPerWave) as leave at least
-// kMinRowGroups groups.
-constexpr int32_t kManyRows     = 131072;
-constexpr int kMaxRowsPerWave   = 16;
-constexpr int32_t kMinRowGroups = 16384;  // sixteen times the workgroups that 256 CUs hold at four apiece
-inline int rows_per_wave(int32_t rows)
-{
-  int rpw = 1;
-  while (rpw < kMaxRowsPerWave && rows / (2 * rpw * kWaves) >= kMinRowGroups) rpw *= 2;
-  return rpw;
-}
-
-// The parts of every row: none for a null row and for the rows that minhash_rows_kernel does, one for an empty row (its
-// zeros have to be written).
+// How the rows are shared out: every row is cut into parts of one length, the parts are numbered row after row
+// (prefix), and a wavefront takes a unit of work, a few consecutive parts, at a time.
 template <typename Source>
 struct RowParts {
   Source source;
   int32_t waves;  // wavefronts that the device holds
-  int64_t alone;  // rows of at most this length are done by minhash_rows_kernel; -1: none is
+  // What every wavefront has to do.
+  __device__ __forceinline__ int64_t share() const
+  {
+    return static_cast<int64_t>(static_cast<double>(source.total()) / waves);  // (whole division of 64 bits: a hundred instructions)
+  }
   // Length of a part: kPart where that leaves every wavefront four parts and more, else a quarter of what each has to
   // do, in columns of less than four of the smallest parts per wavefront all of it (a second round of parts would be
   // longer than the imbalance it removes).
   __device__ __forceinline__ int64_t part() const
   {
-    if (alone >= 0) return Source::kPart;
-    int64_t const share  = static_cast<int64_t>(static_cast<double>(source.total()) / waves);  // (whole division of 64 bits: a hundred instructions)
-    int64_t const length = ((share < 4 * Source::kMinPart ? share : share / 4) + kWave) / kWave * kWave;
+    int64_t const all    = share();
+    int64_t const length = ((all < 4 * Source::kMinPart ? all : all / 4) + kWave) / kWave * kWave;
     return min(max(length, Source::kMinPart), Source::kPart);
   }
-  // ... of a row of length n that is not null
+  // The parts of a row of length n that is not null, one of an empty row (its zeros have to be written).
   __device__ __forceinline__ uint32_t parts_of(int64_t n, uint32_t length) const
   {
-    if (n <= alone) return 0;
     if (n > 0xFFFFFFFFll) return static_cast<uint32_t>((n - 1) / length + 1);
     return n == 0 ? 1u : (static_cast<uint32_t>(n) - 1u) / length + 1u;
   }
@@ -649,119 +634,138 @@ struct RowParts {
   {
     return source.valid(i) ? parts_of(source.length(i), static_cast<uint32_t>(part())) : 0u;
   }
+  // Parts to a unit: an eighth of the parts there are for a wavefront, and no more than make up kPart (with what a part
+  // costs beside its length); and whether one counter keeps up with handing the units out.  It answers 150 M requests a
+  // second, and a unit costs about one instruction a position for its hash and 1.5 for every 64 parameters: one counter
+  // where that takes the device twice as long.  (Of 131,071 rows of 3000 bytes, 260 parameters, 32 groups with a counter
+  // each took 4.57 ms, one counter 4.42: the groups are not done at one time.  With 26 parameters one counter took 2.10
+  // ms, 32 took 1.25.)
+  __device__ __forceinline__ uint32_t per_unit(uint32_t total, int32_t params, bool* one_counter) const
+  {
+    float const mean    = static_cast<float>(source.total()) / static_cast<float>(max(total, 1u));
+    uint32_t const most = static_cast<uint32_t>(static_cast<float>(Source::kPart) / (mean + static_cast<float>(Source::kPartCost)));
+    uint32_t const each = max(1u, min(total / (8u * static_cast<uint32_t>(waves)), most));
+    *one_counter        = mean * static_cast<float>(each) * (1.0f + static_cast<float>(params) / 43.0f) >= 8192.0f;
+    return each;
+  }
 };
 
 // Wavefronts per SIMD that the kernels are compiled for.
 template <typename Source, typename Minima>
 constexpr int simd_waves() { return Source::kSimdWaves < Minima::kSimdWaves ? Source::kSimdWaves : Minima::kSimdWaves; }
 
-// One workgroup per (group of consecutive rows, parameter chunk): its wavefronts take the group's rows of up to kPart
-// bytes one at a time from a counter in LDS, so that the four are done together whatever the rows' lengths; the minima
-// go from the registers to the result.  The groups lie along x and, beyond kMaxRowBlocks of them, along z.
-template <typename Source, typename Minima, typename T = typename Minima::T>
-__global__ void __launch_bounds__(kThreads, (simd_waves<Source, Minima>())) minhash_rows_kernel(Source source, Params<T> params,
-                                                                                   const int32_t* __restrict__ out_offsets, T* __restrict__ out,
-                                                                                   int per_wave)
+// The row r that part t is one of, prefix[r] <= t < prefix[r + 1], is one of 64 rows from the returned one on, of which
+// *near is prefix (rows + 1 of them), a lane a row; not the last.  Looked for first where rows of equal numbers of parts
+// would have it, then where the parts missing from there would lie, then with 64 rows to a step.
+__device__ __forceinline__ int64_t row_of(const uint32_t* __restrict__ prefix, int64_t rows, uint32_t total, uint32_t t, int lane, uint32_t* near)
 {
-  __shared__ typename Source::Lds lds[kWaves];
-  __shared__ typename Minima::Lds minima_lds[kWaves];
-  __shared__ uint32_t next_row;
-
-  int const group_rows = per_wave * kWaves;
-  int64_t const r0     = (static_cast<int64_t>(blockIdx.z) * gridDim.x + blockIdx.x) * group_rows;
-  if (r0 >= source.rows()) return;
-  int const lane           = lane_id();
-  int const wave           = threadIdx.x / kWave;
-  int32_t const chunk_base = blockIdx.y * Minima::kParams;
-  int32_t const in_chunk   = min(Minima::kSlots, params.count - chunk_base);
-  Minima minima(&minima_lds[wave], lane);
-  minima.load(params, blockIdx.y);
-
-  int const rows_here = static_cast<int>(min(static_cast<int64_t>(group_rows), source.rows() - r0));
-  if (threadIdx.x == 0) next_row = 0;
-  __syncthreads();
-  for (;;) {
-    int t = 0;
-    if (lane == 0) t = static_cast<int>(atomicAdd(&next_row, 1u));
-    int const i = __builtin_amdgcn_readfirstlane(t);  // (the same in every lane: what depends on it stays scalar)
-    if (i >= rows_here) break;
-    if (!source.valid(r0 + i)) continue;
-    int64_t const n = source.length(r0 + i);
-    if (n > Source::kPart) continue;
-    minima.reset();
-    if (n > 0) source.process(r0 + i, 0, n, minima, lds[wave], lane);
-    minima.finish();
-    T* const dst = out + static_cast<int64_t>(out_offsets[r0 + i]) + chunk_base;
-    minima.each([&](int32_t j, T v) {
-      if (j < in_chunk) dst[j] = n > 0 ? v : T{0};  // an empty row is zeros (minhash.cu:318)
-    });
+  float const slope = static_cast<float>(rows) / static_cast<float>(total);
+  int64_t guess     = static_cast<int64_t>(static_cast<float>(t) * slope);
+#pragma unroll
+  for (int probe = 0; probe < 2; ++probe) {
+    int64_t const from  = __builtin_amdgcn_readfirstlane(static_cast<int>(min(max(guess - kWave / 2, static_cast<int64_t>(0)), rows)));
+    *near               = from + lane <= rows ? prefix[from + lane] : 0xFFFFFFFFu;
+    uint64_t const upto = ballot64(*near <= t);
+    if (upto != 0 && upto != ~0ull) return from;
+    int32_t const ahead = static_cast<int32_t>(t - wave_bcast(*near, kWave / 2));
+    guess += static_cast<int64_t>(static_cast<float>(ahead) * slope);
   }
+  int64_t r = 0, end = rows;
+  while (end - r > 1) {
+    int64_t const step = (end - r + kWave - 1) / kWave;
+    int64_t const at   = r + lane * step;
+    int const below    = __builtin_popcountll(ballot64(at < end && prefix[min(at, end - 1)] <= t));
+    r += (below - 1) * step;
+    end = min(end, r + step);
+  }
+  *near = r + lane <= rows ? prefix[r + lane] : 0xFFFFFFFFu;
+  return r;
 }
 
-// Parts of rows, a wavefront each: part t is one of the row r with prefix[r] <= t < prefix[r + 1].  A row of one part is
-// stored, the parts of the others meet with an atomic minimum (their slots hold the largest value before).  With more
-// than eight parts for every wavefront they are handed out by a counter, else by place (a counter answers about 150 M
-// requests a second: seven thousand wavefronts asking at once would wait 50 us).  The chunks of parameters come one
-// after the other in the same count.
+// Part t is one of the row r with prefix[r] <= t < prefix[r + 1].  A row of one part is stored, the parts of the others
+// meet with an atomic minimum (their slots hold the largest value before).  A wavefront's first unit is its own number in
+// the grid, the following ones come from counters: an address answers about 150 M requests a second, which a column of
+// short rows exceeds, so there are thirty-two of them, and rows much shorter than a wavefront's share are asked for several at
+// a time (131,071 rows of 300 bytes, 64 parameters: one counter and a request a row 1621 us).  Where the parts
+// of a unit lie is read once for 64 rows, a lane each.  The chunks of parameters come one after the other in the same count.
 template <typename Source, typename Minima, typename T = typename Minima::T>
 __global__ void __launch_bounds__(kThreads, (simd_waves<Source, Minima>())) minhash_parts_kernel(RowParts<Source> parts, Params<T> params, int32_t chunks,
                                                                                     const int32_t* __restrict__ out_offsets,
                                                                                     const uint32_t* __restrict__ prefix,
-                                                                                    unsigned long long* __restrict__ counter, T* __restrict__ out)
+                                                                                    unsigned long long* __restrict__ counters, T* __restrict__ out)
 {
   __shared__ typename Source::Lds lds[kWaves];
   __shared__ typename Minima::Lds minima_lds[kWaves];
   Source const& source  = parts.source;
-  uint32_t const total  = prefix[source.rows()];
-  uint64_t const tasks  = static_cast<uint64_t>(total) * static_cast<uint32_t>(chunks);
+  int64_t const rows    = source.rows();
   int64_t const length  = parts.part();
+  uint32_t const total  = prefix[rows];
+  bool one_counter;
+  uint32_t const each   = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(parts.per_unit(total, params.count, &one_counter))));
+  uint32_t const units  = total / each + (total % each != 0 ? 1u : 0u);
+  uint64_t const all    = static_cast<uint64_t>(units) * static_cast<uint32_t>(chunks);
   int const lane        = lane_id();
   int const wave        = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
-  uint64_t const nwaves = static_cast<uint64_t>(gridDim.x) * kWaves;
+  uint32_t const me     = blockIdx.x * kWaves + static_cast<uint32_t>(wave);
   uint32_t chunk        = 0;
   Minima minima(&minima_lds[wave], lane);
   minima.load(params, 0);
-  for (uint64_t task = static_cast<uint64_t>(blockIdx.x) * kWaves + wave; task < tasks;) {
-    uint32_t const t = static_cast<uint32_t>(task - static_cast<uint64_t>(chunk) * total);
-    if (t >= total) {  // the next chunk of parameters
-      ++chunk;
-      minima.load(params, static_cast<int32_t>(chunk));
-      continue;
-    }
+  for (uint64_t unit = me; unit < all;) {
+    while (unit >= static_cast<uint64_t>(chunk + 1u) * units) minima.load(params, static_cast<int32_t>(++chunk));  // (the next chunk of parameters)
     int32_t const chunk_base = static_cast<int32_t>(chunk) * Minima::kParams;
     int32_t const in_chunk   = min(Minima::kSlots, params.count - chunk_base);
-    // the last row r with prefix[r] <= t, 64 of them looked at in one step
-    int64_t r = 0, end = source.rows();
-    while (end - r > 1) {
-      int64_t const step = (end - r + kWave - 1) / kWave;
-      int64_t const at   = r + lane * step;
-      int const below    = __builtin_popcountll(ballot64(at < end && prefix[min(at, end - 1)] <= t));
-      r += (below - 1) * step;
-      end = min(end, r + step);
+    uint32_t t               = static_cast<uint32_t>(unit - static_cast<uint64_t>(chunk) * units) * each;
+    uint32_t const t_end     = total - t < each ? total : t + each;
+    int64_t base  = 0;  // near: prefix of the rows from there on, a lane a row
+    uint32_t near = 0xFFFFFFFFu;
+    for (; t < t_end; ++t) {
+      uint64_t upto = ballot64(near <= t);
+      if (upto == 0 || upto == ~0ull) {
+        base = row_of(prefix, rows, total, t, lane, &near);
+        upto = ballot64(near <= t);
+      }
+      int const at         = __builtin_popcountll(upto) - 1;  // (less than 63: the row after that of t begins behind t)
+      int64_t const r      = base + at;
+      uint32_t const first = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(near), at));
+      uint32_t const k     = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(near), at + 1)) - first;
+      int64_t const n      = source.length(r);
+      int64_t const begin  = static_cast<int64_t>(t - first) * length;
+      int64_t const end    = min(n, begin + length);
+      minima.reset();
+      if (begin < end) source.process(r, begin, end, minima, lds[wave], lane);
+      minima.finish();
+      T* const dst = out + static_cast<int64_t>(out_offsets[r]) + chunk_base;
+      minima.each([&](int32_t j, T v) {
+        if (j >= in_chunk) return;
+        if (k == 1)
+          dst[j] = n > 0 ? v : T{0};  // an empty row is zeros (minhash.cu:318)
+        else if (v != std::numeric_limits<T>::max())
+          atomicMin(&dst[j], v);
+      });
     }
-    int64_t const n     = source.length(r);
-    int64_t const begin = static_cast<int64_t>(t - prefix[r]) * length;
-    int64_t const till  = min(n, begin + length);
-    bool const shared   = n > length;
-    minima.reset();
-    if (begin < till) source.process(r, begin, till, minima, lds[wave], lane);
-    minima.finish();
-    T* const dst = out + static_cast<int64_t>(out_offsets[r]) + chunk_base;
-    minima.each([&](int32_t j, T v) {
-      if (j >= in_chunk) return;
-      if (!shared)
-        dst[j] = n > 0 ? v : T{0};  // an empty row is zeros (minhash.cu:318)
-      else if (v != std::numeric_limits<T>::max())
-        atomicMin(&dst[j], v);
-    });
-    if (tasks <= 8 * nwaves) {
-      task += nwaves;
-    } else {
-      unsigned long long next = 0;
-      if (lane == 0) next = atomicAdd(counter, 1ull);
-      task = nwaves + wave_bcast64(next, 0);
-    }
+    if (all <= static_cast<uint64_t>(parts.waves)) break;
+    uint32_t const group    = one_counter ? kCounterGroups : me % kCounterGroups;
+    unsigned long long next = 0;
+    if (lane == 0) next = atomicAdd(&counters[group * kCounterLine], 1ull);
+    next = wave_bcast64(next, 0);
+    unit = one_counter ? next : next * kCounterGroups + group;
   }
+}
+
+// The parameters of 64-bit hashes, laid out for the matrix cores.
+constexpr int groups_of(int32_t P) { return (P + filter64::kGroup - 1) / filter64::kGroup; }
+
+// The counters start past the units that the wavefronts take by their place: counter g serves the wavefronts g,
+// g + kCounterGroups, .. and hands out the units g, g + kCounterGroups, ..; the one behind them serves all.
+__device__ __forceinline__ void start_counters(unsigned long long* counters, int32_t waves)
+{
+  int const g = static_cast<int>(threadIdx.x);
+  if (g <= kCounterGroups) counters[g * kCounterLine] = static_cast<unsigned long long>(g < kCounterGroups ? (waves + kCounterGroups - 1 - g) / kCounterGroups : waves);
+}
+
+__global__ void __launch_bounds__(kWave) minhash64_prepare_kernel(const uint64_t* a, const uint64_t* b, int32_t P, filter64::Group* groups)
+{
+  filter64::prepare_group(a, b, P, static_cast<int32_t>(blockIdx.x), &groups[blockIdx.x], lane_id());
 }
 
 template <typename Source>
@@ -777,15 +781,13 @@ __global__ void uniform_offsets_kernel(int32_t* out, int32_t rows, int32_t P)
   if (i <= rows) out[i] = static_cast<int32_t>(i * P);
 }
 
-constexpr int32_t kMaxRowBlocks = 1 << 15;  // groups along x (a launch of 4 M rows, 64 to a group, has two layers along z: the tests reach them)
-
-// The largest value into the slots of the rows that are done in several parts, and 0 into the counter of the parts: a
+// The largest value into the slots of the rows that are done in several parts, and the counters of the units: a
 // wavefront looks at 64 rows and fills those of them one after the other.
 template <typename Source, typename T = typename Source::T>
 __global__ void __launch_bounds__(kThreads) minhash_clear_kernel(RowParts<Source> parts, int32_t P, const int32_t* __restrict__ out_offsets,
-                                                                 unsigned long long* __restrict__ counter, T* __restrict__ out)
+                                                                 unsigned long long* __restrict__ counters, T* __restrict__ out)
 {
-  if (blockIdx.x == 0 && threadIdx.x == 0) *counter = 0;
+  if (blockIdx.x == 0) start_counters(counters, parts.waves);
   int const lane  = lane_id();
   int64_t const r = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
   bool const many = r < parts.source.rows() && parts(r) > 1;
@@ -794,13 +796,6 @@ __global__ void __launch_bounds__(kThreads) minhash_clear_kernel(RowParts<Source
     T* const dst = out + static_cast<int64_t>(wave_bcast64(static_cast<uint64_t>(o), __builtin_ctzll(todo)));
     for (int32_t j = lane; j < P; j += kWave) dst[j] = std::numeric_limits<T>::max();
   }
-}
-
-// The parameters of 64-bit hashes, laid out for the matrix cores.
-constexpr int groups_of(int32_t P) { return (P + filter64::kGroup - 1) / filter64::kGroup; }
-__global__ void __launch_bounds__(kWave) minhash64_prepare_kernel(const uint64_t* a, const uint64_t* b, int32_t P, filter64::Group* groups)
-{
-  filter64::prepare_group(a, b, P, static_cast<int32_t>(blockIdx.x), &groups[blockIdx.x], lane_id());
 }
 
 // Everything that comes before the hashing of a column of few rows, in one launch: workgroup 0 counts the parts of the
@@ -812,7 +807,7 @@ constexpr int32_t kPlanRows = 2 * kPlanThreads * kPlanItems;
 template <typename Source, typename T = typename Source::T>
 __global__ void __launch_bounds__(kPlanThreads) minhash_plan_kernel(RowParts<Source> parts, Params<T> params, filter64::Group* groups, unsigned fillers,
                                                                     int32_t* __restrict__ out_offsets, uint32_t* __restrict__ prefix,
-                                                                    unsigned long long* __restrict__ counter, T* __restrict__ out, int64_t out_size)
+                                                                    unsigned long long* __restrict__ counters, T* __restrict__ out, int64_t out_size)
 {
   int32_t const rows = parts.source.rows();
   int32_t const P    = params.count;
@@ -832,6 +827,7 @@ __global__ void __launch_bounds__(kPlanThreads) minhash_plan_kernel(RowParts<Sou
     return;
   }
   __shared__ uint64_t lds[kPlanThreads / kWave + 1];
+  start_counters(counters, parts.waves);
   uint32_t const length = static_cast<uint32_t>(parts.part());
   uint64_t carry        = 0;  // parts in the low half, valid rows in the high half
   for (int32_t tile = 0; tile < rows; tile += kPlanThreads * kPlanItems) {
@@ -863,28 +859,9 @@ __global__ void __launch_bounds__(kPlanThreads) minhash_plan_kernel(RowParts<Sou
     carry += total;
   }
   if (threadIdx.x == 0) {
-    *counter     = 0;
     prefix[rows] = static_cast<uint32_t>(carry);
     if (parts.source.masked()) out_offsets[rows] = static_cast<int32_t>(carry >> 32) * P;
   }
-}
-
-template <typename Minima, typename Source, typename T = typename Source::T>
-void launch_kernels(RowParts<Source> const& parts, int32_t rows, Params<T> const& params, int32_t chunks, const int32_t* offsets,
-                    const uint32_t* prefix, unsigned long long* counter, T* child, hipStream_t stream)
-{
-  if (rows >= kManyRows) {
-    int const per_wave   = rows_per_wave(rows);
-    int32_t const groups = (rows + per_wave * kWaves - 1) / (per_wave * kWaves);
-    dim3 grid(static_cast<unsigned>(std::min(groups, kMaxRowBlocks)), static_cast<unsigned>(chunks),
-              static_cast<unsigned>((groups + kMaxRowBlocks - 1) / kMaxRowBlocks));
-    ProfileScope ps(Source::kRowsName, stream);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_rows_kernel<Source, Minima>), grid, dim3(kThreads), 0, stream, parts.source, params, offsets, child,
-                       per_wave);
-  }
-  ProfileScope ps(Source::kPartsName, stream);
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_parts_kernel<Source, Minima>), dim3(static_cast<unsigned>(parts.waves / kWaves)), dim3(kThreads), 0, stream,
-                     parts, params, chunks, offsets, prefix, counter, child);
 }
 
 // How the parameters of 32-bit hashes are shared out: chunks of K sets of 64 (every chunk hashes the windows again, and a lane without
@@ -945,24 +922,23 @@ void with_minima(int32_t P, Launch const& launch)
   }
 }
 
-// The launches of one minhash call: the row offsets of the result and the parts of every row, then the hashing kernels.
-// prefix holds rows + 1 values, scan_tmp scan_temp_bytes(rows) bytes and one 64-bit counter behind them; laid_out (64-bit
-// hashes) groups_of(P).
+// The launches of one minhash call: the places of the rows in the result and their parts, then the hashing kernel.
+// prefix holds rows + 1 values, scan_tmp scan_temp_bytes(rows) bytes up to the next line of 128 and the counters behind them; laid_out (64-bit hashes) groups_of(P).
 template <typename Source, typename T = typename Source::T>
 void run_minhash(Source const& source, int32_t rows, bool masked, const T* a, const T* b, int32_t P, int32_t* offsets, T* child, int64_t child_size,
                  uint32_t* prefix, uint64_t* scan_tmp, filter64::Group* laid_out, hipStream_t stream)
 {
   int waves = 0;
   with_minima<T>(P, [&](auto which, int32_t) { waves = simd_waves<Source, typename decltype(which)::type>(); });
-  RowParts<Source> const parts{source, device_cus() * 4 * waves, rows >= kManyRows ? Source::kPart : -1};
+  RowParts<Source> const parts{source, device_cus() * 4 * waves};
   Params<T> const params{a, b, P, laid_out};
-  auto* const counter = reinterpret_cast<unsigned long long*>(scan_tmp) + scan_temp_bytes(rows) / sizeof(uint64_t);
+  auto* const counters = reinterpret_cast<unsigned long long*>(scan_tmp) + (scan_temp_bytes(rows) + 127) / 128 * 16;
   if (rows <= kPlanRows) {
     int64_t const most    = std::max<int64_t>(child_size, rows + 1);
     unsigned const fillers = static_cast<unsigned>(std::min<int64_t>((most + 4 * kPlanThreads - 1) / (4 * kPlanThreads), 256));
     unsigned const layers  = sizeof(T) == 8 ? static_cast<unsigned>((groups_of(P) + kPlanThreads / kWave - 1) / (kPlanThreads / kWave)) : 0u;
     hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_plan_kernel<Source>), dim3(1 + fillers + layers), dim3(kPlanThreads), 0, stream, parts, params, laid_out,
-                       fillers, offsets, prefix, counter, child, child_size);
+                       fillers, offsets, prefix, counters, child, child_size);
   } else {
     if (masked) {
       device_exclusive_scan(ValidTimesP<Source>{source, P}, static_cast<int64_t>(rows), offsets, scan_tmp, stream);
@@ -972,13 +948,16 @@ void run_minhash(Source const& source, int32_t rows, bool masked, const T* a, co
     if constexpr (sizeof(T) == 8)
       hipLaunchKernelGGL(minhash64_prepare_kernel, dim3(static_cast<unsigned>(groups_of(P))), dim3(kWave), 0, stream, a, b, P, laid_out);
     device_exclusive_scan(parts, static_cast<int64_t>(rows), prefix, scan_tmp, stream);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_clear_kernel<Source>), dim3((rows + kThreads - 1) / kThreads), dim3(kThreads), 0, stream, parts, P, offsets, counter,
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_clear_kernel<Source>), dim3((rows + kThreads - 1) / kThreads), dim3(kThreads), 0, stream, parts, P, offsets, counters,
                        child);
   }
 
   if (child_size > 0) {
     with_minima<T>(P, [&](auto which, int32_t chunks) {
-      launch_kernels<typename decltype(which)::type>(parts, rows, params, chunks, offsets, prefix, counter, child, stream);
+      using Minima = typename decltype(which)::type;
+      ProfileScope ps(Source::kName, stream);
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_parts_kernel<Source, Minima>), dim3(static_cast<unsigned>(parts.waves / kWaves)), dim3(kThreads), 0, stream,
+                         parts, params, chunks, offsets, prefix, counters, child);
     });
   }
 }
@@ -1035,7 +1014,7 @@ nvtext_amd_status minhash_impl(const nvtext_amd_strings_column* input, T seed, c
   }
 
   ColView const v = make_view(*input);
-  size_t const temp_bytes[3] = {scan_temp_bytes(rows) + sizeof(uint64_t), static_cast<size_t>(rows + 1) * sizeof(uint32_t),
+  size_t const temp_bytes[3] = {(scan_temp_bytes(rows) + 127) / 128 * 128 + kCounterBytes, static_cast<size_t>(rows + 1) * sizeof(uint32_t),
                                 sizeof(T) == 8 ? static_cast<size_t>(groups_of(P)) * sizeof(filter64::Group) : 0};
   TempParts<3> const temp(mr, temp_bytes);
   if (!temp.ok()) {
@@ -1111,7 +1090,7 @@ nvtext_amd_status minhash_ngrams_impl(const nvtext_amd_list_strings_column* inpu
   v.offset   = input->offset;
   v.use_mask = (input->null_mask != nullptr && input->null_count > 0) ? 1 : 0;
   v.child    = make_view(input->child);
-  size_t const temp_bytes[3] = {scan_temp_bytes(rows) + sizeof(uint64_t), static_cast<size_t>(rows + 1) * sizeof(uint32_t),
+  size_t const temp_bytes[3] = {(scan_temp_bytes(rows) + 127) / 128 * 128 + kCounterBytes, static_cast<size_t>(rows + 1) * sizeof(uint32_t),
                                 sizeof(T) == 8 ? static_cast<size_t>(groups_of(P)) * sizeof(filter64::Group) : 0};
   TempParts<3> const temp(mr, temp_bytes);
   if (!temp.ok()) {

@@ -85,7 +85,7 @@ def test_minhash_parts_of_rows(nv, orc, bits, count):
 @pytest.mark.parametrize("rows", [8192, 8193, 131_071, 131_072])
 @pytest.mark.parametrize("nulls", [False, True])
 def test_minhash_row_counts(nv, orc, rows, nulls):
-    """Around the row counts at which the plan takes several launches and at which short rows are done in groups."""
+    """Around the row counts at which the plan takes several launches, and around 128 tiles of 1024 rows."""
     rng = np.random.default_rng(rows)
     lens = rng.integers(0, 12, rows)
     lens[[0, 7, rows // 2, rows - 1]] = [4097, 4096, 30_000, 9000]
@@ -94,6 +94,24 @@ def test_minhash_row_counts(nv, orc, rows, nulls):
     assert nv.minhash(dev(nv, host), 5, a, b, 4).to_host().equals(orc.minhash(host, 5, a, b, 4, nthreads=8))
     a, b = params(rng, 3, 64)
     assert nv.minhash64(dev(nv, host), 5, a, b, 4).to_host().equals(orc.minhash64(host, 5, a, b, 4, nthreads=8))
+
+
+@pytest.mark.parametrize("rows", [70_000, 120_000, 300_000])
+@pytest.mark.parametrize("bits, count", [(32, 5), (32, 330), (64, 5), (64, 130)])
+def test_minhash_units_of_rows(nv, orc, rows, bits, count):
+    """Columns whose rows are handed out one and several at a time: rows of a few windows and empty ones, runs of thousands
+    of null rows between them (where the rows are not where an even column would have them), long rows first, in the middle
+    and last; the parameters in one chunk and in several."""
+    if rows * count > 20_000_000:
+        rows //= 5
+    rng = np.random.default_rng(rows)
+    lens = rng.integers(0, 10, rows)
+    lens[[0, rows // 2, rows - 1]] = 20_000, 40_001, 9_999
+    nulls = np.unique(np.concatenate([np.arange(rows // 8, rows // 8 + rows // 4), np.arange(rows // 2 + 1, rows // 2 + 66), [5, rows - 2]]))
+    host = mixed_rows(rng, lens, nulls=tuple(nulls.tolist()))
+    call, ref = (nv.minhash, orc.minhash) if bits == 32 else (nv.minhash64, orc.minhash64)
+    a, b = params(rng, count, bits)
+    assert call(dev(nv, host), 5, a, b, 4).to_host().equals(ref(host, 5, a, b, 4, nthreads=8))
 
 
 @pytest.mark.parametrize("kind", ["zero", "small", "power", "digits of 2", "digits of 1", "wraps", "top"])
