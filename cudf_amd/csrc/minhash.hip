@@ -10,7 +10,7 @@
 //   * it then switches to lanes <-> parameters: every lane keeps K (a, b) pairs and
 //     K running minima in registers and streams the tile's hashes through LDS
 //     broadcast reads, so the inner loop is v_mad_u64_u32 + v_min only;
-//   * a wavefront does a row alone, or a part of it: rows are cut into parts of at most 4 KiB (of
+//   * a wavefront does a row alone, or a part of it: rows are cut into parts of at most 6 KiB (of
 //     fewer bytes in a column too small to give every wavefront of the device several of that size),
 //     the parts of a row meet in the result with an atomic minimum, and the wavefronts take short rows
 //     several at a time;
@@ -30,15 +30,15 @@
 #include <type_traits>
 
 // Scratch of nvtext_amd_minhash_preallocated, the entry point that allocates nothing: the part counts of the
-// rows (rows + 1 values) and behind them the tile sums of the scans and the counters of the units of work.  Every device holds
+// rows (rows + 1 values) and behind them the sums of the plan and the counters of the units of work.  Every device holds
 // its own copy of the array for as long as the library is loaded (4.2 MB).
 constexpr int32_t kPreallocatedMaxRows = NVTEXT_AMD_MINHASH_PREALLOCATED_MAX_ROWS;
 constexpr size_t kScratchPrefixBytes   = (static_cast<size_t>(kPreallocatedMaxRows) + 1 + 63) / 64 * 64 * sizeof(uint32_t);
+constexpr int kSumTiles                = 1024;  // tiles of rows at most, whose sums the plan of a larger column adds up
 constexpr int kCounterGroups           = 32;    // counters of units of work
 constexpr int kCounterLine             = 16;    // 64-bit words from one to the next: a 128-byte line each
-constexpr size_t kCounterBytes         = (kCounterGroups + 1) * kCounterLine * sizeof(uint64_t);
-constexpr size_t kScratchScanBytes     = (static_cast<size_t>(kPreallocatedMaxRows) / nvtext_amd::kScanTile + 2 + 15) / 16 * 128 + kCounterBytes;
-static __device__ __align__(256) unsigned char scratch[kScratchPrefixBytes + kScratchScanBytes];
+constexpr size_t kPlanBytes            = ((kCounterGroups + 1) * kCounterLine + kSumTiles) * sizeof(uint64_t);
+static __device__ __align__(256) unsigned char scratch[kScratchPrefixBytes + kPlanBytes];
 
 namespace nvtext_amd {
 namespace {
@@ -414,7 +414,7 @@ struct TextRows {
   using Lds = WaveLds<T>;
   static constexpr const char* kName = "minhash_parts_kernel";
   static constexpr int kSimdWaves   = sizeof(T) == 4 ? 6 : 4;  // wavefronts per SIMD that its LDS leaves room for
-  static constexpr int64_t kPart    = 4096;
+  static constexpr int64_t kPart    = 2816;  // (parts of up to one and a half: 4096 is no faster, and the end of the kernel is uneven by one of them)
   static constexpr int64_t kMinPart = kTile;  // less would be staged for its halo
   static constexpr int kPartCost    = 64;
   ColView col;
@@ -536,7 +536,7 @@ struct RunRows {
   using Lds = RunLds<T>;
   static constexpr const char* kName = "minhash_ngrams_parts_kernel";
   static constexpr int kSimdWaves   = sizeof(T) == 4 ? 7 : 4;
-  static constexpr int64_t kPart    = 1024;
+  static constexpr int64_t kPart    = 704;
   static constexpr int64_t kMinPart = kWave;
   static constexpr int kPartCost    = 32;
   ListView col;
@@ -604,7 +604,7 @@ struct RunRows {
   }
 };
 
-// How the rows are shared out: every row is cut into parts of one length, the parts are numbered row after row
+// How the rows are shared out: every row is cut into parts of about one length, the parts are numbered row after row
 // (prefix), and a wavefront takes a unit of work, a few consecutive parts, at a time.
 template <typename Source>
 struct RowParts {
@@ -616,23 +616,40 @@ struct RowParts {
     return static_cast<int64_t>(static_cast<double>(source.total()) / waves);  // (whole division of 64 bits: a hundred instructions)
   }
   // Length of a part: kPart where that leaves every wavefront four parts and more, else a quarter of what each has to
-  // do, in columns of less than four of the smallest parts per wavefront all of it (a second round of parts would be
-  // longer than the imbalance it removes).
-  __device__ __forceinline__ int64_t part() const
+  // do, in columns of less than four of the smallest parts per wavefront half of it (20,000 rows of 300 bytes, 64
+  // parameters: the whole share 60 us, half of it 52, a quarter 54; 8,193 lists of 200 elements, 128 parameters: 42, 39,
+  // 45).  Parts of a row of length n that is not null: as many as come nearest to the length, so that none is a remainder
+  // (a row of up to one and a half stays whole), but in a column of fewer rows than wavefronts, where some would be left
+  // without work, as many as keep each within the length (5,000 lists of 130 elements: 23.6 us, the nearest 25.4).  An
+  // empty row has one (its zeros have to be written).  Any number from one to the row's trips will do: what a division
+  // would give is not needed.
+  struct Cut {
+    float per_length, more;
+  };
+  __device__ __forceinline__ Cut cut() const
   {
     int64_t const all    = share();
-    int64_t const length = ((all < 4 * Source::kMinPart ? all : all / 4) + kWave) / kWave * kWave;
-    return min(max(length, Source::kMinPart), Source::kPart);
+    int64_t const length = (all / (all < 4 * Source::kMinPart ? 2 : 4) + kWave) / kWave * kWave;
+    float const within   = static_cast<float>(min(max(length, Source::kMinPart), Source::kPart));
+    return Cut{__builtin_amdgcn_rcpf(within), source.rows() <= waves ? within - 1.0f : within / 2.0f};
   }
-  // The parts of a row of length n that is not null, one of an empty row (its zeros have to be written).
-  __device__ __forceinline__ uint32_t parts_of(int64_t n, uint32_t length) const
+  __device__ __forceinline__ uint32_t parts_of(int64_t n, Cut const& c) const
   {
-    if (n > 0xFFFFFFFFll) return static_cast<uint32_t>((n - 1) / length + 1);
-    return n == 0 ? 1u : (static_cast<uint32_t>(n) - 1u) / length + 1u;
+    return max(1u, static_cast<uint32_t>((static_cast<float>(n) + c.more) * c.per_length));
   }
-  __device__ __forceinline__ uint64_t operator()(int64_t i) const
+  // Part i of k of a row of length n: whole trips of 64 (of 256, four of which are staged or folded together, where a part
+  // has several of those), as even as they come.  A row has at least as many trips as parts.
+  __device__ __forceinline__ void bounds(int64_t n, uint32_t i, uint32_t k, int64_t* begin, int64_t* end) const
   {
-    return source.valid(i) ? parts_of(source.length(i), static_cast<uint32_t>(part())) : 0u;
+    *begin = 0;
+    *end   = n;
+    if (k == 1) return;
+    uint32_t const trip  = n >= static_cast<int64_t>(k) * 1024 ? 256u : 64u;
+    uint64_t const trips = static_cast<uint64_t>(n + trip - 1) / trip;
+    uint64_t const each  = trips >> 32 ? trips / k : static_cast<uint32_t>(trips) / k;
+    uint32_t const more  = static_cast<uint32_t>(trips - each * k);
+    *begin = static_cast<int64_t>(trip * (each * i + min(i, more)));
+    *end   = min(n, *begin + static_cast<int64_t>(trip * (each + (i < more ? 1u : 0u))));
   }
   // Parts to a unit: an eighth of the parts there are for a wavefront, and no more than make up kPart (with what a part
   // costs beside its length); and whether one counter keeps up with handing the units out.  It answers 150 M requests a
@@ -642,10 +659,10 @@ struct RowParts {
   // ms, 32 took 1.25.)
   __device__ __forceinline__ uint32_t per_unit(uint32_t total, int32_t params, bool* one_counter) const
   {
-    float const mean    = static_cast<float>(source.total()) / static_cast<float>(max(total, 1u));
-    uint32_t const most = static_cast<uint32_t>(static_cast<float>(Source::kPart) / (mean + static_cast<float>(Source::kPartCost)));
+    float const mean    = static_cast<float>(source.total()) * __builtin_amdgcn_rcpf(static_cast<float>(max(total, 1u)));
+    uint32_t const most = static_cast<uint32_t>(static_cast<float>(Source::kPart) * __builtin_amdgcn_rcpf(mean + static_cast<float>(Source::kPartCost)));
     uint32_t const each = max(1u, min(total / (8u * static_cast<uint32_t>(waves)), most));
-    *one_counter        = mean * static_cast<float>(each) * (1.0f + static_cast<float>(params) / 43.0f) >= 8192.0f;
+    *one_counter        = mean * static_cast<float>(each) * static_cast<float>(43 + params) >= 43.0f * 8192.0f;
     return each;
   }
 };
@@ -659,9 +676,9 @@ constexpr int simd_waves() { return Source::kSimdWaves < Minima::kSimdWaves ? So
 // would have it, then where the parts missing from there would lie, then with 64 rows to a step.
 __device__ __forceinline__ int64_t row_of(const uint32_t* __restrict__ prefix, int64_t rows, uint32_t total, uint32_t t, int lane, uint32_t* near)
 {
-  float const slope = static_cast<float>(rows) / static_cast<float>(total);
+  float const slope = static_cast<float>(rows) * __builtin_amdgcn_rcpf(static_cast<float>(total));
   int64_t guess     = static_cast<int64_t>(static_cast<float>(t) * slope);
-#pragma unroll
+#pragma unroll 1
   for (int probe = 0; probe < 2; ++probe) {
     int64_t const from  = __builtin_amdgcn_readfirstlane(static_cast<int>(min(max(guess - kWave / 2, static_cast<int64_t>(0)), rows)));
     *near               = from + lane <= rows ? prefix[from + lane] : 0xFFFFFFFFu;
@@ -698,7 +715,6 @@ __global__ void __launch_bounds__(kThreads, (simd_waves<Source, Minima>())) minh
   __shared__ typename Minima::Lds minima_lds[kWaves];
   Source const& source  = parts.source;
   int64_t const rows    = source.rows();
-  int64_t const length  = parts.part();
   uint32_t const total  = prefix[rows];
   bool one_counter;
   uint32_t const each   = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(parts.per_unit(total, params.count, &one_counter))));
@@ -729,8 +745,8 @@ __global__ void __launch_bounds__(kThreads, (simd_waves<Source, Minima>())) minh
       uint32_t const first = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(near), at));
       uint32_t const k     = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(near), at + 1)) - first;
       int64_t const n      = source.length(r);
-      int64_t const begin  = static_cast<int64_t>(t - first) * length;
-      int64_t const end    = min(n, begin + length);
+      int64_t begin, end;
+      parts.bounds(n, t - first, k, &begin, &end);
       minima.reset();
       if (begin < end) source.process(r, begin, end, minima, lds[wave], lane);
       minima.finish();
@@ -763,63 +779,38 @@ __device__ __forceinline__ void start_counters(unsigned long long* counters, int
   if (g <= kCounterGroups) counters[g * kCounterLine] = static_cast<unsigned long long>(g < kCounterGroups ? (waves + kCounterGroups - 1 - g) / kCounterGroups : waves);
 }
 
-__global__ void __launch_bounds__(kWave) minhash64_prepare_kernel(const uint64_t* a, const uint64_t* b, int32_t P, filter64::Group* groups)
-{
-  filter64::prepare_group(a, b, P, static_cast<int32_t>(blockIdx.x), &groups[blockIdx.x], lane_id());
-}
-
+// The parts of a row in the low half, a valid row in the high half.
 template <typename Source>
-struct ValidTimesP {
-  Source source;
-  int32_t P;
-  __device__ uint64_t operator()(int64_t i) const { return source.valid(i) ? static_cast<uint64_t>(P) : 0; }
-};
-
-__global__ void uniform_offsets_kernel(int32_t* out, int32_t rows, int32_t P)
+__device__ __forceinline__ uint64_t parts_and_rows(RowParts<Source> const& parts, typename RowParts<Source>::Cut const& cut, int64_t n, bool valid)
 {
-  int64_t const i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i <= rows) out[i] = static_cast<int32_t>(i * P);
+  return valid ? parts.parts_of(n, cut) | (1ull << 32) : 0ull;
 }
 
-// The largest value into the slots of the rows that are done in several parts, and the counters of the units: a
-// wavefront looks at 64 rows and fills those of them one after the other.
-template <typename Source, typename T = typename Source::T>
-__global__ void __launch_bounds__(kThreads) minhash_clear_kernel(RowParts<Source> parts, int32_t P, const int32_t* __restrict__ out_offsets,
-                                                                 unsigned long long* __restrict__ counters, T* __restrict__ out)
-{
-  if (blockIdx.x == 0) start_counters(counters, parts.waves);
-  int const lane  = lane_id();
-  int64_t const r = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  bool const many = r < parts.source.rows() && parts(r) > 1;
-  int64_t const o = many ? out_offsets[r] : 0;
-  for (uint64_t todo = ballot64(many); todo != 0; todo &= todo - 1) {
-    T* const dst = out + static_cast<int64_t>(wave_bcast64(static_cast<uint64_t>(o), __builtin_ctzll(todo)));
-    for (int32_t j = lane; j < P; j += kWave) dst[j] = std::numeric_limits<T>::max();
-  }
-}
-
-// Everything that comes before the hashing of a column of few rows, in one launch: workgroup 0 counts the parts of the
-// rows (and finds the rows' places in the result where some are null), the others write the places where none is and
-// fill the result; the wavefronts of the workgroups from `fillers` + 1 on lay out the parameters of 64-bit hashes.
+// Everything that comes before the hashing of a column of few rows, in one launch: the first workgroups take 1024 rows each
+// and find their parts (and, where some are null, the rows' places in the result), what lies before their rows every one
+// counts by itself (one workgroup for all rows was bound by its arithmetic: 8,000 rows of 300 bytes, 64 parameters, 36.2 us
+// the call, with this 32.6; up to 1023 rows have a kernel of their own: one that could take eight times as many takes 0.8
+// of 15 us longer); `fillers` more write the places where no row is null and fill the result; the wavefronts of
+// the workgroups behind them lay out the parameters of 64-bit hashes.
 constexpr int kPlanThreads  = 1024;
-constexpr int kPlanItems    = 4;
-constexpr int32_t kPlanRows = 2 * kPlanThreads * kPlanItems;
-template <typename Source, typename T = typename Source::T>
-__global__ void __launch_bounds__(kPlanThreads) minhash_plan_kernel(RowParts<Source> parts, Params<T> params, filter64::Group* groups, unsigned fillers,
-                                                                    int32_t* __restrict__ out_offsets, uint32_t* __restrict__ prefix,
+constexpr int kPlanTiles    = 8;
+constexpr int32_t kPlanRows = kPlanThreads * kPlanTiles;
+template <int TILES, typename Source, typename T = typename Source::T>
+__global__ void __launch_bounds__(kPlanThreads) minhash_plan_kernel(RowParts<Source> parts, Params<T> params, filter64::Group* groups, unsigned tiles,
+                                                                    unsigned fillers, int32_t* __restrict__ out_offsets, uint32_t* __restrict__ prefix,
                                                                     unsigned long long* __restrict__ counters, T* __restrict__ out, int64_t out_size)
 {
   int32_t const rows = parts.source.rows();
   int32_t const P    = params.count;
   if constexpr (sizeof(T) == 8) {
-    if (blockIdx.x > fillers) {
-      int32_t const group = static_cast<int32_t>((blockIdx.x - fillers - 1) * (kPlanThreads / kWave) + threadIdx.x / kWave);
+    if (blockIdx.x >= tiles + fillers) {
+      int32_t const group = static_cast<int32_t>((blockIdx.x - tiles - fillers) * (kPlanThreads / kWave) + threadIdx.x / kWave);
       if (group < groups_of(P)) filter64::prepare_group(params.a, params.b, P, group, &groups[group], lane_id());
       return;
     }
   }
-  if (blockIdx.x > 0) {
-    int64_t const first  = static_cast<int64_t>(blockIdx.x - 1) * kPlanThreads + threadIdx.x;
+  if (blockIdx.x >= tiles) {
+    int64_t const first  = static_cast<int64_t>(blockIdx.x - tiles) * kPlanThreads + threadIdx.x;
     int64_t const stride = static_cast<int64_t>(fillers) * kPlanThreads;
     if (!parts.source.masked())
       for (int64_t i = first; i <= rows; i += stride) out_offsets[i] = static_cast<int32_t>(i * P);
@@ -827,40 +818,96 @@ __global__ void __launch_bounds__(kPlanThreads) minhash_plan_kernel(RowParts<Sou
     return;
   }
   __shared__ uint64_t lds[kPlanThreads / kWave + 1];
-  start_counters(counters, parts.waves);
-  uint32_t const length = static_cast<uint32_t>(parts.part());
-  uint64_t carry        = 0;  // parts in the low half, valid rows in the high half
-  for (int32_t tile = 0; tile < rows; tile += kPlanThreads * kPlanItems) {
-    int32_t const base = tile + static_cast<int32_t>(threadIdx.x) * kPlanItems;
-    int64_t n[kPlanItems];
-    bool valid[kPlanItems];
+  // all loads in flight together, those of the rows before what depends on the whole column's length
+  int64_t n[TILES];
+  bool valid[TILES];
 #pragma unroll
-    for (int k = 0; k < kPlanItems; ++k) {  // (without a branch: all loads in flight together)
-      int32_t const i = min(base + k, rows - 1);
-      n[k]            = parts.source.length(i);
-      valid[k]        = parts.source.valid(i) && base + k < rows;
+  for (unsigned k = 0; k < TILES; ++k) {
+    n[k]     = 0;
+    valid[k] = false;
+    if (k <= blockIdx.x) {
+      int32_t const i = static_cast<int32_t>(k * kPlanThreads + threadIdx.x);
+      n[k]            = parts.source.length(min(i, rows - 1));
+      valid[k]        = i < rows && parts.source.valid(min(i, rows - 1));
     }
-    uint64_t vals[kPlanItems], sum = 0;
-#pragma unroll
-    for (int k = 0; k < kPlanItems; ++k) {
-      vals[k] = valid[k] ? parts.parts_of(n[k], length) | (1ull << 32) : 0ull;
-      sum += vals[k];
-    }
-    uint64_t total;
-    uint64_t run = block_exclusive_scan64<kPlanThreads>(sum, lds, &total) + carry;
-#pragma unroll
-    for (int k = 0; k < kPlanItems; ++k) {
-      if (base + k < rows) {
-        prefix[base + k] = static_cast<uint32_t>(run);
-        if (parts.source.masked()) out_offsets[base + k] = static_cast<int32_t>(run >> 32) * P;
-      }
-      run += vals[k];
-    }
-    carry += total;
   }
-  if (threadIdx.x == 0) {
-    prefix[rows] = static_cast<uint32_t>(carry);
-    if (parts.source.masked()) out_offsets[rows] = static_cast<int32_t>(carry >> 32) * P;
+  if (blockIdx.x == 0) start_counters(counters, parts.waves);
+  auto const cut  = parts.cut();
+  uint64_t before = 0, mine = 0;
+#pragma unroll
+  for (unsigned k = 0; k < TILES; ++k) {
+    uint64_t const v = parts_and_rows(parts, cut, n[k], valid[k]);
+    before += k < blockIdx.x ? v : 0ull;
+    mine = k == blockIdx.x ? v : mine;
+  }
+  uint64_t carry = 0, total;
+  if (blockIdx.x > 0) block_exclusive_scan64<kPlanThreads>(before, lds, &carry);
+  uint64_t const run = carry + block_exclusive_scan64<kPlanThreads>(mine, lds, &total);
+  int32_t const i    = static_cast<int32_t>(blockIdx.x * kPlanThreads + threadIdx.x);
+  if (i <= rows) {  // (rows + 1 of them)
+    prefix[i] = static_cast<uint32_t>(run);
+    if (parts.source.masked()) out_offsets[i] = static_cast<int32_t>(run >> 32) * P;
+  }
+}
+
+// The same for a column of more rows, in two launches: the sums of tiles of rows (parts in the low half, valid rows in the
+// high half; the workgroups behind them lay out the parameters of 64-bit hashes), then, from the sums of the tiles before,
+// the places of every row, and the largest value into the slots of the rows that are done in several parts: a wavefront
+// looks at 64 rows and fills those of them one after the other.  A tile is `passes` times 256 rows, so that there are at
+// most kSumTiles.
+inline int32_t sum_passes(int32_t rows) { return (rows - 1) / (kThreads * kSumTiles) + 1; }
+
+template <typename Source, typename T = typename Source::T>
+__global__ void __launch_bounds__(kThreads) minhash_sums_kernel(RowParts<Source> parts, Params<T> params, filter64::Group* groups, int32_t tiles, int32_t passes,
+                                                                uint64_t* __restrict__ sums)
+{
+  if constexpr (sizeof(T) == 8) {
+    if (static_cast<int32_t>(blockIdx.x) >= tiles) {
+      int32_t const group = (static_cast<int32_t>(blockIdx.x) - tiles) * kWaves + static_cast<int32_t>(threadIdx.x / kWave);
+      if (group < groups_of(params.count)) filter64::prepare_group(params.a, params.b, params.count, group, &groups[group], lane_id());
+      return;
+    }
+  }
+  __shared__ uint64_t lds[kWaves + 1];
+  auto const cut = parts.cut();
+  uint64_t sum   = 0;
+  for (int32_t pass = 0; pass < passes; ++pass) {
+    int64_t const i = (static_cast<int64_t>(blockIdx.x) * passes + pass) * kThreads + threadIdx.x;
+    if (i < parts.source.rows()) sum += parts_and_rows(parts, cut, parts.source.length(i), parts.source.valid(i));
+  }
+  uint64_t total;
+  block_exclusive_scan64<kThreads>(sum, lds, &total);
+  if (threadIdx.x == 0) sums[blockIdx.x] = total;
+}
+
+template <typename Source, typename T = typename Source::T>
+__global__ void __launch_bounds__(kThreads) minhash_places_kernel(RowParts<Source> parts, int32_t P, int32_t passes, const uint64_t* __restrict__ sums,
+                                                                  int32_t* __restrict__ out_offsets, uint32_t* __restrict__ prefix,
+                                                                  unsigned long long* __restrict__ counters, T* __restrict__ out)
+{
+  __shared__ uint64_t lds[kWaves + 1];
+  if (blockIdx.x == 0) start_counters(counters, parts.waves);
+  int32_t const rows = parts.source.rows();
+  auto const cut     = parts.cut();
+  uint64_t mine = 0, carry;
+  for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kThreads) mine += sums[i];
+  block_exclusive_scan64<kThreads>(mine, lds, &carry);
+  int const lane = lane_id();
+  for (int32_t pass = 0; pass < passes; ++pass) {
+    int64_t const i  = (static_cast<int64_t>(blockIdx.x) * passes + pass) * kThreads + threadIdx.x;
+    uint64_t const v = i < rows ? parts_and_rows(parts, cut, parts.source.length(i), parts.source.valid(i)) : 0ull;
+    uint64_t total;
+    uint64_t const before = block_exclusive_scan64<kThreads>(v, lds, &total) + carry;
+    carry += total;
+    int32_t const place = parts.source.masked() ? static_cast<int32_t>(before >> 32) * P : static_cast<int32_t>(i * P);
+    if (i <= rows) {
+      prefix[i]      = static_cast<uint32_t>(before);
+      out_offsets[i] = place;
+    }
+    for (uint64_t todo = ballot64(static_cast<uint32_t>(v) > 1u); todo != 0; todo &= todo - 1) {
+      T* const dst = out + __builtin_amdgcn_readlane(place, __builtin_ctzll(todo));
+      for (int32_t j = lane; j < P; j += kWave) dst[j] = std::numeric_limits<T>::max();
+    }
   }
 }
 
@@ -923,33 +970,31 @@ void with_minima(int32_t P, Launch const& launch)
 }
 
 // The launches of one minhash call: the places of the rows in the result and their parts, then the hashing kernel.
-// prefix holds rows + 1 values, scan_tmp scan_temp_bytes(rows) bytes up to the next line of 128 and the counters behind them; laid_out (64-bit hashes) groups_of(P).
+// prefix holds rows + 1 values, plan kPlanBytes; laid_out (64-bit hashes) groups_of(P).
 template <typename Source, typename T = typename Source::T>
-void run_minhash(Source const& source, int32_t rows, bool masked, const T* a, const T* b, int32_t P, int32_t* offsets, T* child, int64_t child_size,
-                 uint32_t* prefix, uint64_t* scan_tmp, filter64::Group* laid_out, hipStream_t stream)
+void run_minhash(Source const& source, int32_t rows, const T* a, const T* b, int32_t P, int32_t* offsets, T* child, int64_t child_size,
+                 uint32_t* prefix, uint64_t* plan, filter64::Group* laid_out, hipStream_t stream)
 {
   int waves = 0;
   with_minima<T>(P, [&](auto which, int32_t) { waves = simd_waves<Source, typename decltype(which)::type>(); });
   RowParts<Source> const parts{source, device_cus() * 4 * waves};
   Params<T> const params{a, b, P, laid_out};
-  auto* const counters = reinterpret_cast<unsigned long long*>(scan_tmp) + (scan_temp_bytes(rows) + 127) / 128 * 16;
-  if (rows <= kPlanRows) {
-    int64_t const most    = std::max<int64_t>(child_size, rows + 1);
+  auto* const counters = reinterpret_cast<unsigned long long*>(plan);
+  auto const layers    = [&](int threads) { return sizeof(T) == 8 ? (groups_of(P) + threads / kWave - 1) / (threads / kWave) : 0; };
+  if (rows < kPlanRows) {
+    int64_t const most     = std::max<int64_t>(child_size, rows + 1);
     unsigned const fillers = static_cast<unsigned>(std::min<int64_t>((most + 4 * kPlanThreads - 1) / (4 * kPlanThreads), 256));
-    unsigned const layers  = sizeof(T) == 8 ? static_cast<unsigned>((groups_of(P) + kPlanThreads / kWave - 1) / (kPlanThreads / kWave)) : 0u;
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_plan_kernel<Source>), dim3(1 + fillers + layers), dim3(kPlanThreads), 0, stream, parts, params, laid_out,
-                       fillers, offsets, prefix, counters, child, child_size);
+    unsigned const tiles   = static_cast<unsigned>(rows / kPlanThreads + 1);
+    auto const plan_rows   = tiles == 1 ? minhash_plan_kernel<1, Source> : minhash_plan_kernel<kPlanTiles, Source>;
+    hipLaunchKernelGGL(plan_rows, dim3(tiles + fillers + static_cast<unsigned>(layers(kPlanThreads))), dim3(kPlanThreads), 0, stream, parts, params, laid_out,
+                       tiles, fillers, offsets, prefix, counters, child, child_size);
   } else {
-    if (masked) {
-      device_exclusive_scan(ValidTimesP<Source>{source, P}, static_cast<int64_t>(rows), offsets, scan_tmp, stream);
-    } else {
-      hipLaunchKernelGGL(uniform_offsets_kernel, dim3((rows + 1 + 255) / 256), dim3(256), 0, stream, offsets, rows, P);
-    }
-    if constexpr (sizeof(T) == 8)
-      hipLaunchKernelGGL(minhash64_prepare_kernel, dim3(static_cast<unsigned>(groups_of(P))), dim3(kWave), 0, stream, a, b, P, laid_out);
-    device_exclusive_scan(parts, static_cast<int64_t>(rows), prefix, scan_tmp, stream);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_clear_kernel<Source>), dim3((rows + kThreads - 1) / kThreads), dim3(kThreads), 0, stream, parts, P, offsets, counters,
-                       child);
+    uint64_t* const sums = plan + (kCounterGroups + 1) * kCounterLine;
+    int32_t const passes = sum_passes(rows), tiles = (rows - 1) / (kThreads * passes) + 1;
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_sums_kernel<Source>), dim3(static_cast<unsigned>(tiles + layers(kThreads))), dim3(kThreads), 0, stream, parts,
+                       params, laid_out, tiles, passes, sums);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_places_kernel<Source>), dim3(static_cast<unsigned>(rows / (kThreads * passes) + 1)), dim3(kThreads), 0, stream,
+                       parts, P, passes, sums, offsets, prefix, counters, child);
   }
 
   if (child_size > 0) {
@@ -1014,14 +1059,14 @@ nvtext_amd_status minhash_impl(const nvtext_amd_strings_column* input, T seed, c
   }
 
   ColView const v = make_view(*input);
-  size_t const temp_bytes[3] = {(scan_temp_bytes(rows) + 127) / 128 * 128 + kCounterBytes, static_cast<size_t>(rows + 1) * sizeof(uint32_t),
+  size_t const temp_bytes[3] = {kPlanBytes, static_cast<size_t>(rows + 1) * sizeof(uint32_t),
                                 sizeof(T) == 8 ? static_cast<size_t>(groups_of(P)) * sizeof(filter64::Group) : 0};
   TempParts<3> const temp(mr, temp_bytes);
   if (!temp.ok()) {
     nvtext_amd_list_column_free(out, stream_, mr_);
     return fail(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");
   }
-  run_minhash(TextRows<T>{v, seed, width}, rows, v.use_mask != 0, a, b, P, out->offsets, static_cast<T*>(out->child), out->child_size, temp.part<uint32_t>(1),
+  run_minhash(TextRows<T>{v, seed, width}, rows, a, b, P, out->offsets, static_cast<T*>(out->child), out->child_size, temp.part<uint32_t>(1),
                  temp.part<uint64_t>(0), temp.part<filter64::Group>(2), stream);
   NVTEXT_HIP_TRY_OR(hipGetLastError(), nvtext_amd_list_column_free(out, stream_, mr_));
   return NVTEXT_AMD_SUCCESS;
@@ -1090,14 +1135,14 @@ nvtext_amd_status minhash_ngrams_impl(const nvtext_amd_list_strings_column* inpu
   v.offset   = input->offset;
   v.use_mask = (input->null_mask != nullptr && input->null_count > 0) ? 1 : 0;
   v.child    = make_view(input->child);
-  size_t const temp_bytes[3] = {(scan_temp_bytes(rows) + 127) / 128 * 128 + kCounterBytes, static_cast<size_t>(rows + 1) * sizeof(uint32_t),
+  size_t const temp_bytes[3] = {kPlanBytes, static_cast<size_t>(rows + 1) * sizeof(uint32_t),
                                 sizeof(T) == 8 ? static_cast<size_t>(groups_of(P)) * sizeof(filter64::Group) : 0};
   TempParts<3> const temp(mr, temp_bytes);
   if (!temp.ok()) {
     nvtext_amd_list_column_free(out, stream_, mr_);
     return fail(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");
   }
-  run_minhash(RunRows<T>{v, seed, ngrams}, rows, v.use_mask != 0, a, b, P, out->offsets, static_cast<T*>(out->child), out->child_size,
+  run_minhash(RunRows<T>{v, seed, ngrams}, rows, a, b, P, out->offsets, static_cast<T*>(out->child), out->child_size,
               temp.part<uint32_t>(1), temp.part<uint64_t>(0), temp.part<filter64::Group>(2), stream);
   NVTEXT_HIP_TRY_OR(hipGetLastError(), nvtext_amd_list_column_free(out, stream_, mr_));
   return NVTEXT_AMD_SUCCESS;
@@ -1161,12 +1206,12 @@ nvtext_amd_status nvtext_amd_minhash_preallocated(const nvtext_amd_strings_colum
   nvtext_amd_status const st = scratch_of_current_device(&base);
   if (st != NVTEXT_AMD_SUCCESS) return st;
   uint32_t* const prefix   = reinterpret_cast<uint32_t*>(base);
-  uint64_t* const scan_tmp = reinterpret_cast<uint64_t*>(base + kScratchPrefixBytes);
+  uint64_t* const plan     = reinterpret_cast<uint64_t*>(base + kScratchPrefixBytes);
 
   if (input->null_mask) launch_copy_bitmask(out_null_mask, input->null_mask, input->offset, rows, stream);
   ColView const v = make_view(*input);
   // every value of the scratch that the kernels read is written earlier in this same call: nothing to clear
-  run_minhash(TextRows<uint32_t>{v, seed, width}, rows, v.use_mask != 0, a, b, P, out_offsets, out_child, child_size, prefix, scan_tmp, nullptr, stream);
+  run_minhash(TextRows<uint32_t>{v, seed, width}, rows, a, b, P, out_offsets, out_child, child_size, prefix, plan, nullptr, stream);
   NVTEXT_HIP_TRY(hipGetLastError());
   return NVTEXT_AMD_SUCCESS;
 }

@@ -71,8 +71,8 @@ def params(rng, count, bits):
 @pytest.mark.parametrize("bits", [32, 64])
 @pytest.mark.parametrize("count", [1, 33, 64, 128, 260, 700])
 def test_minhash_parts_of_rows(nv, orc, bits, count):
-    """Rows one byte around one part and several, parts of 256 bytes (little text) and of 4096 (8 MB and more), the
-    parameters in one chunk and in several, null and empty rows between them."""
+    """Rows one byte around one part and several, parts of 256 bytes (little text) and more (33 MB), the parameters in one
+    chunk and in several, null and empty rows between them."""
     rng = np.random.default_rng(count)
     edges = [0, 1, 4, 5, 63, 64, 65, 255, 256, 257, 511, 513, 4095, 4096, 4097, 8192, 8193, 20_000]
     call, ref = (nv.minhash, orc.minhash) if bits == 32 else (nv.minhash64, orc.minhash64)
@@ -82,10 +82,10 @@ def test_minhash_parts_of_rows(nv, orc, bits, count):
         assert call(dev(nv, host), 5, a, b, 5).to_host().equals(ref(host, 5, a, b, 5, nthreads=8))
 
 
-@pytest.mark.parametrize("rows", [8192, 8193, 131_071, 131_072])
+@pytest.mark.parametrize("rows", [1023, 1024, 1025, 8191, 8192, 8193, 131_071, 131_072, 262_144, 262_145])
 @pytest.mark.parametrize("nulls", [False, True])
 def test_minhash_row_counts(nv, orc, rows, nulls):
-    """Around the row counts at which the plan takes several launches, and around 128 tiles of 1024 rows."""
+    """Around the tiles of 1024 rows of the plan, the rows from which it takes two launches and those from which its tiles grow."""
     rng = np.random.default_rng(rows)
     lens = rng.integers(0, 12, rows)
     lens[[0, 7, rows // 2, rows - 1]] = [4097, 4096, 30_000, 9000]
@@ -94,6 +94,19 @@ def test_minhash_row_counts(nv, orc, rows, nulls):
     assert nv.minhash(dev(nv, host), 5, a, b, 4).to_host().equals(orc.minhash(host, 5, a, b, 4, nthreads=8))
     a, b = params(rng, 3, 64)
     assert nv.minhash64(dev(nv, host), 5, a, b, 4).to_host().equals(orc.minhash64(host, 5, a, b, 4, nthreads=8))
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("filler, short", [(0, 0), (0, 9000), (20, 0), (20, 9000), (75, 0)])
+def test_minhash_even_parts(nv, orc, bits, filler, short):
+    """Rows of all lengths up to five parts of 2816 bytes, in columns whose parts are the smallest, larger and the largest
+    (20 and 75 MB of other rows), with fewer rows than wavefronts (each part within the length) and with more (the nearest)."""
+    rng = np.random.default_rng(filler + short)
+    lens = np.concatenate([np.arange(0, 14_500, 97), [1_000_000] * filler, np.full(short, 90)])
+    host = mixed_rows(rng, rng.permutation(lens))
+    call, ref = (nv.minhash, orc.minhash) if bits == 32 else (nv.minhash64, orc.minhash64)
+    a, b = params(rng, 3, bits)
+    assert call(dev(nv, host), 5, a, b, 5).to_host().equals(ref(host, 5, a, b, 5, nthreads=8))
 
 
 @pytest.mark.parametrize("rows", [70_000, 120_000, 300_000])
@@ -147,7 +160,7 @@ def test_minhash64_last_blocks(nv, orc, count):
 @pytest.mark.parametrize("ngrams", [2, 5])
 @pytest.mark.parametrize("count", [1, 130])
 def test_minhash_ngrams_parts_of_rows(nv, orc, bits, ngrams, count):
-    """Lists one element around a trip of 64 positions, around the four that are folded together and around parts of 1024,
+    """Lists one element around a trip of 64 positions, around the four that are folded together and around several parts,
     shorter than a run, empty, and among 131,072 others; elements that are null or empty; a view."""
     rng = np.random.default_rng(count)
     call, ref = (nv.minhash_ngrams, orc.minhash_ngrams) if bits == 32 else (nv.minhash64_ngrams, orc.minhash64_ngrams)
