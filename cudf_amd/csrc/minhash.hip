@@ -99,7 +99,7 @@ __host__ __device__ inline Packing packing_for(int32_t P)
 // parameters and fold every other trip each (see Packing).
 constexpr uint32_t kFoldTrip = 4;
 template <int K>
-__device__ __forceinline__ void fold32(const uint32_t* hashes, uint32_t padded, uint32_t first, uint32_t stride, const uint32_t (&a)[K],
+__device__ __forceinline__ void fold_all(const uint32_t* hashes, uint32_t padded, uint32_t first, uint32_t stride, const uint32_t (&a)[K],
                                        const uint32_t (&b)[K], uint32_t (&m)[K])
 {
   for (uint32_t i = first; i < padded; i += stride) {
@@ -117,6 +117,82 @@ __device__ __forceinline__ void fold32(const uint32_t* hashes, uint32_t padded, 
   }
 }
 
+// The same for 64-bit hashes, every product computed whole (see filter64.cuh for the permutation).
+//
+// ((h * a + b) mod 2^64) folded once mod 2^61 - 1, that is (x & p) + (x >> 61) for the 64-bit x, at most p + 7, for two
+// hashes and one (a, b): x = h.lo * a.lo + b is a 64-bit multiply-add; the two cross products, of which only the low
+// dwords count, are two more, chained, and their sum goes to the high dword of x with a 32-bit add; the fold is a shift
+// and a mask of that dword and one more multiply-add (q * 1 + x) for the carry.  The chained pairs of the two hashes stand
+// interleaved, so that neither waits for its own first half.
+__device__ __forceinline__ void fold_pair(uint64_t h0, uint64_t h1, uint64_t a, uint64_t b, uint32_t one, uint64_t* y0, uint64_t* y1)
+{
+  uint32_t const al = static_cast<uint32_t>(a), ah = static_cast<uint32_t>(a >> 32);
+  uint32_t const l0 = static_cast<uint32_t>(h0), u0 = static_cast<uint32_t>(h0 >> 32);
+  uint32_t const l1 = static_cast<uint32_t>(h1), u1 = static_cast<uint32_t>(h1 >> 32);
+  uint64_t c0, c1;
+  asm("v_mad_u64_u32 %0, vcc, %2, %6, 0\n\t"
+      "v_mad_u64_u32 %1, vcc, %4, %6, 0\n\t"
+      "v_mad_u64_u32 %0, vcc, %3, %7, %0\n\t"
+      "v_mad_u64_u32 %1, vcc, %5, %7, %1"
+      : "=&v"(c0), "=&v"(c1)
+      : "v"(l0), "v"(u0), "v"(l1), "v"(u1), "v"(ah), "v"(al)
+      : "vcc");
+  uint64_t const x0 = static_cast<uint64_t>(l0) * al + b;
+  uint64_t const x1 = static_cast<uint64_t>(l1) * al + b;
+  uint32_t xh0      = static_cast<uint32_t>(x0 >> 32) + static_cast<uint32_t>(c0);
+  uint32_t xh1      = static_cast<uint32_t>(x1 >> 32) + static_cast<uint32_t>(c1);
+  uint32_t const q0 = xh0 >> 29, q1 = xh1 >> 29;
+  xh0 &= 0x1FFFFFFFu;
+  xh1 &= 0x1FFFFFFFu;
+  *y0 = static_cast<uint64_t>(q0) * one + ((static_cast<uint64_t>(xh0) << 32) | static_cast<uint32_t>(x0));
+  *y1 = static_cast<uint64_t>(q1) * one + ((static_cast<uint64_t>(xh1) << 32) | static_cast<uint32_t>(x1));
+}
+
+// min of two values below 2^62 in one instruction: such bit patterns are non-negative finite doubles (or denormals, which
+// this code object keeps: float_denorm_mode_16_64 = 3), and those order like the integers.  An operand that is all ones
+// (the start value, a NaN pattern) loses to the other.
+__device__ __forceinline__ uint64_t min_below_2_62(uint64_t m, uint64_t y)
+{
+  uint64_t r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(m), "v"(y));
+  return r;
+}
+
+template <int K>
+__device__ __forceinline__ void fold_all(const uint64_t* hashes, uint32_t padded, uint32_t first, uint32_t stride, const uint64_t (&a)[K],
+                                         const uint64_t (&b)[K], uint64_t (&m)[K])
+{
+  // The last "subtract p if y >= p" is left out: it takes a y whose top dword is at least 0x1FFFFFFF (one product in
+  // 2^29), which a running maximum tells; if there is one all hashes are folded again exactly.  (Values that ought to
+  // have been reduced are above all that are, so that they have displaced none.)
+  uint32_t top = 0;
+  uint32_t one;  // the number 1 where the compiler does not see it: q * one + x stays one multiply-add
+  asm("s_mov_b32 %0, 1" : "=s"(one));
+  for (uint32_t i = first; i < padded; i += stride) {
+    uint64_t h[kFoldTrip];
+#pragma unroll
+    for (uint32_t j = 0; j < kFoldTrip; ++j) h[j] = hashes[i + j];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+#pragma unroll
+      for (uint32_t j = 0; j < kFoldTrip; j += 2) {
+        uint64_t y0, y1;
+        fold_pair(h[j], h[j + 1], a[k], b[k], one, &y0, &y1);
+        top  = max(max(top, static_cast<uint32_t>(y0 >> 32)), static_cast<uint32_t>(y1 >> 32));
+        m[k] = min_below_2_62(min_below_2_62(m[k], y0), y1);
+      }
+    }
+  }
+  if (ballot64(top >= 0x1FFFFFFFu) != 0) {
+    // (every lane folds every hash here: a minimum does not mind the hashes of the other sets)
+    for (uint32_t i = 0; i < padded; ++i) {
+      uint64_t const h = hashes[i];
+#pragma unroll
+      for (int k = 0; k < K; ++k) m[k] = min(m[k], filter64::exact(h, a[k], b[k]));
+    }
+  }
+}
+
 // What the kernels are given of the parameters.
 template <typename T>
 struct Params {
@@ -129,22 +205,24 @@ struct Params {
 // The minima of a row (or of a part of one) over the parameters of a chunk, by one wavefront: load() the chunk, reset(),
 // fold() hashes out of LDS as often as needed, finish(), each(put) calls put(j, minimum) for the parameters.
 
-// uint32: K sets of 64 parameters, a lane has one of each set; with TAIL the parameters beyond the last full set, when
+// Every product computed: K sets of 64 parameters, a lane has one of each set; with TAIL the parameters beyond the last full set, when
 // there are at most 32 of them, are one more (a, b) pair per lane, shared out over sets of lanes as Packing describes, so
 // that they cost the fold a share of a full set (4 parameters beyond 256: a sixteenth) instead of a whole one.
-template <int K, bool TAIL>
-struct Minima32 {
-  using T = uint32_t;
+template <typename T_, int K, bool TAIL>
+struct MinimaAll {
+  using T = T_;
   struct Lds {};
   static constexpr int kParams = K * kWave;                       // of a chunk
   static constexpr int kSlots  = (K + (TAIL ? 1 : 0)) * kWave;    // (with TAIL there is one chunk)
-  static constexpr int kSimdWaves = 7;                             // wavefronts per SIMD that the registers are held to
+  // wavefronts per SIMD that the registers are held to (64-bit hashes, 256 parameters: five spill nine registers, and
+  // 20,000 lists of 200 elements take 306 us, with four 318)
+  static constexpr int kSimdWaves = sizeof(T) == 4 ? 7 : 5;
   T a[K], b[K], m[K];
   T tail_a[1], tail_b[1], tail_m[1];
   Packing pk, tail_pk;
   int lane;
 
-  __device__ __forceinline__ Minima32(Lds*, int lane_) : lane(lane_) {}
+  __device__ __forceinline__ MinimaAll(Lds*, int lane_) : lane(lane_) {}
   __device__ __forceinline__ void load(Params<T> const& p, int32_t chunk)
   {
     pk = K == 1 ? packing_for(p.count) : Packing{kWave, 1};
@@ -180,10 +258,10 @@ struct Minima32 {
     wave_lds_fence();
     // the usual case keeps the loop counter out of the vector registers
     if (K > 1 || pk.groups == 1)
-      fold32<K>(hashes, padded, 0u, kFoldTrip, a, b, m);
+      fold_all<K>(hashes, padded, 0u, kFoldTrip, a, b, m);
     else
-      fold32<K>(hashes, padded, pk.first(lane, kFoldTrip), pk.stride(kFoldTrip), a, b, m);
-    if (TAIL) fold32<1>(hashes, padded, tail_pk.first(lane, kFoldTrip), tail_pk.stride(kFoldTrip), tail_a, tail_b, tail_m);
+      fold_all<K>(hashes, padded, pk.first(lane, kFoldTrip), pk.stride(kFoldTrip), a, b, m);
+    if (TAIL) fold_all<1>(hashes, padded, tail_pk.first(lane, kFoldTrip), tail_pk.stride(kFoldTrip), tail_a, tail_b, tail_m);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
@@ -202,7 +280,7 @@ struct Minima32 {
   }
 };
 
-// uint64: G groups of 32 parameters, each product to 17 bits by the matrix cores (see filter64.cuh), 32 hashes at a time.
+// 64-bit hashes: G groups of 32 parameters, each product to 17 bits by the matrix cores (see filter64.cuh), 32 hashes at a time.
 // A lane has a parameter of every group and half of the hashes.  Of the hashes that lie in LDS (`fold`) it finds the
 // least fraction, whose hash it is, and the second least: two matrix instructions, 16 shifts that put the fractions in
 // order with a number below them and 23 minima, medians and maxima for 1,024 products, without a branch.  Per row and
@@ -413,6 +491,7 @@ struct TextRows {
   using T   = T_;
   using Lds = WaveLds<T>;
   static constexpr const char* kName = "minhash_parts_kernel";
+  static constexpr bool kShortRows   = false;  // no more is known of their lengths than the kernels read
   static constexpr int kSimdWaves   = sizeof(T) == 4 ? 6 : 4;  // wavefronts per SIMD that its LDS leaves room for
   static constexpr int64_t kPart    = 2816;  // (parts of up to one and a half: 4096 is no faster, and the end of the kernel is uneven by one of them)
   static constexpr int64_t kMinPart = kTile;  // less would be staged for its halo
@@ -535,7 +614,8 @@ struct RunRows {
   using T   = T_;
   using Lds = RunLds<T>;
   static constexpr const char* kName = "minhash_ngrams_parts_kernel";
-  static constexpr int kSimdWaves   = sizeof(T) == 4 ? 7 : 4;
+  static constexpr bool kShortRows   = true;
+  static constexpr int kSimdWaves   = sizeof(T) == 4 ? 7 : 5;
   static constexpr int64_t kPart    = 704;
   static constexpr int64_t kMinPart = kWave;
   static constexpr int kPartCost    = 32;
@@ -940,9 +1020,32 @@ struct Which {
   using type = M;
 };
 template <typename T, typename Launch>
-void with_minima(int32_t P, Launch const& launch)
+void with_all_products(int32_t P, Launch const& launch)
 {
-  if constexpr (sizeof(T) == 8) {
+  Sharing const sh     = sharing_for(P);
+  int32_t const chunks = sh.tail ? 1 : (P + sh.k * kWave - 1) / (sh.k * kWave);
+  switch (sh.k * 2 + (sh.tail ? 1 : 0)) {
+    case 10: launch(Which<MinimaAll<T, 5, false>>{}, chunks); break;
+    case 9: launch(Which<MinimaAll<T, 4, true>>{}, chunks); break;
+    case 8: launch(Which<MinimaAll<T, 4, false>>{}, chunks); break;
+    case 7: launch(Which<MinimaAll<T, 3, true>>{}, chunks); break;
+    case 6: launch(Which<MinimaAll<T, 3, false>>{}, chunks); break;
+    case 5: launch(Which<MinimaAll<T, 2, true>>{}, chunks); break;
+    case 4: launch(Which<MinimaAll<T, 2, false>>{}, chunks); break;
+    case 3: launch(Which<MinimaAll<T, 1, true>>{}, chunks); break;
+    default: launch(Which<MinimaAll<T, 1, false>>{}, chunks); break;
+  }
+}
+template <typename Source, typename Launch>
+void with_minima(int32_t P, bool short_rows, Launch const& launch)
+{
+  using T = typename Source::T;
+  if constexpr (sizeof(T) == 4) {
+    with_all_products<T>(P, launch);
+  } else {
+    if constexpr (Source::kShortRows) {
+      if (short_rows) return with_all_products<T>(P, launch);
+    }
     // as few chunks as four groups each allow (every chunk hashes the windows again), of equal size
     int const groups     = groups_of(P);
     int32_t const chunks = (groups + 3) / 4;
@@ -952,35 +1055,36 @@ void with_minima(int32_t P, Launch const& launch)
       case 3: launch(Which<Minima64<3>>{}, chunks); break;
       default: launch(Which<Minima64<4>>{}, chunks); break;
     }
-  } else {
-    Sharing const sh     = sharing_for(P);
-    int32_t const chunks = sh.tail ? 1 : (P + sh.k * kWave - 1) / (sh.k * kWave);
-    switch (sh.k * 2 + (sh.tail ? 1 : 0)) {
-      case 10: launch(Which<Minima32<5, false>>{}, chunks); break;
-      case 9: launch(Which<Minima32<4, true>>{}, chunks); break;
-      case 8: launch(Which<Minima32<4, false>>{}, chunks); break;
-      case 7: launch(Which<Minima32<3, true>>{}, chunks); break;
-      case 6: launch(Which<Minima32<3, false>>{}, chunks); break;
-      case 5: launch(Which<Minima32<2, true>>{}, chunks); break;
-      case 4: launch(Which<Minima32<2, false>>{}, chunks); break;
-      case 3: launch(Which<Minima32<1, true>>{}, chunks); break;
-      default: launch(Which<Minima32<1, false>>{}, chunks); break;
-    }
   }
+}
+
+// Rows of 64-bit hashes shorter than this on average have all their products computed whole.  The matrix cores spare 7
+// vector instructions a product and wavefront and cost some 800 for every 64 parameters of a row, for what has to be
+// computed exactly at its end; and as their registers take 128 parameters at most, not 320, more chunks, each of which
+// hashes the row again (20 instructions a position: runs of words come from memory).  Lists of 60 elements, 131,072 rows,
+// 128 parameters: whole 367 us, matrix cores 426; of 130: 799 and 824; of 200: 1150 and 1076; 20,000 of 200, 256
+// parameters: 306 and 319, of 800: 1152 and 986; 30,000 of 1200, 260 parameters: 2483 and 3187.
+inline double short_row_length(int32_t P)
+{
+  Sharing const sh     = sharing_for(P);
+  int32_t const chunks = sh.tail ? 1 : (P + sh.k * kWave - 1) / (sh.k * kWave);
+  double const sets    = sh.tail ? sh.k + packing_for(P - sh.k * kWave).ppad / 64.0 : static_cast<double>(chunks * sh.k);
+  double const spared  = 7.0 * sets - 20.0 * ((groups_of(P) + 3) / 4 - chunks);
+  return spared > 0.0 ? 800.0 * sets / spared : std::numeric_limits<double>::max();
 }
 
 // The launches of one minhash call: the places of the rows in the result and their parts, then the hashing kernel.
 // prefix holds rows + 1 values, plan kPlanBytes; laid_out (64-bit hashes) groups_of(P).
 template <typename Source, typename T = typename Source::T>
-void run_minhash(Source const& source, int32_t rows, const T* a, const T* b, int32_t P, int32_t* offsets, T* child, int64_t child_size,
+void run_minhash(Source const& source, int32_t rows, bool short_rows, const T* a, const T* b, int32_t P, int32_t* offsets, T* child, int64_t child_size,
                  uint32_t* prefix, uint64_t* plan, filter64::Group* laid_out, hipStream_t stream)
 {
   int waves = 0;
-  with_minima<T>(P, [&](auto which, int32_t) { waves = simd_waves<Source, typename decltype(which)::type>(); });
+  with_minima<Source>(P, short_rows, [&](auto which, int32_t) { waves = simd_waves<Source, typename decltype(which)::type>(); });
   RowParts<Source> const parts{source, device_cus() * 4 * waves};
   Params<T> const params{a, b, P, laid_out};
   auto* const counters = reinterpret_cast<unsigned long long*>(plan);
-  auto const layers    = [&](int threads) { return sizeof(T) == 8 ? (groups_of(P) + threads / kWave - 1) / (threads / kWave) : 0; };
+  auto const layers    = [&](int threads) { return laid_out ? (groups_of(P) + threads / kWave - 1) / (threads / kWave) : 0; };
   if (rows < kPlanRows) {
     int64_t const most     = std::max<int64_t>(child_size, rows + 1);
     unsigned const fillers = static_cast<unsigned>(std::min<int64_t>((most + 4 * kPlanThreads - 1) / (4 * kPlanThreads), 256));
@@ -998,7 +1102,7 @@ void run_minhash(Source const& source, int32_t rows, const T* a, const T* b, int
   }
 
   if (child_size > 0) {
-    with_minima<T>(P, [&](auto which, int32_t chunks) {
+    with_minima<Source>(P, short_rows, [&](auto which, int32_t chunks) {
       using Minima = typename decltype(which)::type;
       ProfileScope ps(Source::kName, stream);
       hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_parts_kernel<Source, Minima>), dim3(static_cast<unsigned>(parts.waves / kWaves)), dim3(kThreads), 0, stream,
@@ -1066,7 +1170,7 @@ nvtext_amd_status minhash_impl(const nvtext_amd_strings_column* input, T seed, c
     nvtext_amd_list_column_free(out, stream_, mr_);
     return fail(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");
   }
-  run_minhash(TextRows<T>{v, seed, width}, rows, a, b, P, out->offsets, static_cast<T*>(out->child), out->child_size, temp.part<uint32_t>(1),
+  run_minhash(TextRows<T>{v, seed, width}, rows, false, a, b, P, out->offsets, static_cast<T*>(out->child), out->child_size, temp.part<uint32_t>(1),
                  temp.part<uint64_t>(0), temp.part<filter64::Group>(2), stream);
   NVTEXT_HIP_TRY_OR(hipGetLastError(), nvtext_amd_list_column_free(out, stream_, mr_));
   return NVTEXT_AMD_SUCCESS;
@@ -1135,6 +1239,8 @@ nvtext_amd_status minhash_ngrams_impl(const nvtext_amd_list_strings_column* inpu
   v.offset   = input->offset;
   v.use_mask = (input->null_mask != nullptr && input->null_count > 0) ? 1 : 0;
   v.child    = make_view(input->child);
+  // (a view's child may hold more elements than the view: then the other way is taken, with the same result)
+  bool const short_rows = sizeof(T) == 8 && static_cast<double>(input->child.size) < short_row_length(P) * rows;
   size_t const temp_bytes[3] = {kPlanBytes, static_cast<size_t>(rows + 1) * sizeof(uint32_t),
                                 sizeof(T) == 8 ? static_cast<size_t>(groups_of(P)) * sizeof(filter64::Group) : 0};
   TempParts<3> const temp(mr, temp_bytes);
@@ -1142,8 +1248,8 @@ nvtext_amd_status minhash_ngrams_impl(const nvtext_amd_list_strings_column* inpu
     nvtext_amd_list_column_free(out, stream_, mr_);
     return fail(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");
   }
-  run_minhash(RunRows<T>{v, seed, ngrams}, rows, a, b, P, out->offsets, static_cast<T*>(out->child), out->child_size,
-              temp.part<uint32_t>(1), temp.part<uint64_t>(0), temp.part<filter64::Group>(2), stream);
+  run_minhash(RunRows<T>{v, seed, ngrams}, rows, short_rows, a, b, P, out->offsets, static_cast<T*>(out->child), out->child_size,
+              temp.part<uint32_t>(1), temp.part<uint64_t>(0), short_rows ? nullptr : temp.part<filter64::Group>(2), stream);
   NVTEXT_HIP_TRY_OR(hipGetLastError(), nvtext_amd_list_column_free(out, stream_, mr_));
   return NVTEXT_AMD_SUCCESS;
 }
@@ -1211,7 +1317,7 @@ nvtext_amd_status nvtext_amd_minhash_preallocated(const nvtext_amd_strings_colum
   if (input->null_mask) launch_copy_bitmask(out_null_mask, input->null_mask, input->offset, rows, stream);
   ColView const v = make_view(*input);
   // every value of the scratch that the kernels read is written earlier in this same call: nothing to clear
-  run_minhash(TextRows<uint32_t>{v, seed, width}, rows, a, b, P, out_offsets, out_child, child_size, prefix, plan, nullptr, stream);
+  run_minhash(TextRows<uint32_t>{v, seed, width}, rows, false, a, b, P, out_offsets, out_child, child_size, prefix, plan, nullptr, stream);
   NVTEXT_HIP_TRY(hipGetLastError());
   return NVTEXT_AMD_SUCCESS;
 }

@@ -127,17 +127,21 @@ def test_minhash_units_of_rows(nv, orc, rows, bits, count):
     assert call(dev(nv, host), 5, a, b, 4).to_host().equals(ref(host, 5, a, b, 4, nthreads=8))
 
 
-@pytest.mark.parametrize("kind", ["zero", "small", "power", "digits of 2", "digits of 1", "wraps", "top"])
-def test_minhash64_parameters(nv, orc, kind):
-    """Parameters for which the fractions that decide what is computed exactly tie, lie at zero or at the wrap, or take their
-    sums to the ends of their range; rows of one window, of fewer than a block of 32 and of many, with windows that repeat."""
-    rng = np.random.default_rng(7)
+def hard_parameters(kind):
     p = (1 << 61) - 1
     a = {"zero": [0, p, 2 * p], "small": [1, 2, 3, 5], "power": [1 << 60, 1 << 61, 1 << 63, 1 << 44, 1 << 43], "digits of 2": [0xAAAAAAAAAAAAAAAA],
          "digits of 1": [0x5555555555555555], "wraps": [(1 << 64) - 1, p - 1, p + 1], "top": [(1 << 44) - 1, (1 << 64) - (1 << 44)]}[kind]
     b = [0, 1, p - 1, p, p + 7, (1 << 61) - 8, (1 << 64) - 1, 1 << 44, (1 << 44) - 1]
     pairs = np.array([(x, y) for x in a for y in b], np.uint64)
-    a, b = pairs[:, 0].copy(), pairs[:, 1].copy()
+    return pairs[:, 0].copy(), pairs[:, 1].copy()
+
+
+@pytest.mark.parametrize("kind", ["zero", "small", "power", "digits of 2", "digits of 1", "wraps", "top"])
+def test_minhash64_parameters(nv, orc, kind):
+    """Parameters for which the fractions that decide what is computed exactly tie, lie at zero or at the wrap, or take their
+    sums to the ends of their range; rows of one window, of fewer than a block of 32 and of many, with windows that repeat."""
+    rng = np.random.default_rng(7)
+    a, b = hard_parameters(kind)
     host = mixed_rows(rng, [5, 6, 30, 36, 37, 300, 3000, 40_000])
     text = HostStringsColumn.from_pylist(["abcdefgh" * 500, "a" * 3000, "the same words " * 400, "naïve 漢字 " * 60])
     for column in (host, text):
@@ -175,6 +179,34 @@ def test_minhash_ngrams_parts_of_rows(nv, orc, bits, ngrams, count):
         assert call(d, ngrams, 5, a, b).to_host().equals(ref(lists, ngrams, 5, a, b, nthreads=8))
         assert call(d.slice(2, len(lens) - 1, 0), ngrams, 5, a, b).to_host().equals(
             ref(HostListStringsColumn(offsets, child, None, len(lens) - 3, 2, 0), ngrams, 5, a, b, nthreads=8))
+
+
+@pytest.mark.parametrize("mean", [3, 113, 115, 420])
+@pytest.mark.parametrize("count", [1, 26, 64, 128, 130, 256, 320, 330])
+def test_minhash64_ngrams_short_and_long_lists(nv, orc, mean, count):
+    """Lists shorter and longer than the average from which products go to the matrix cores (114 elements with 128 parameters
+    and fewer, 400 with 256, none with 130 and 320); the parameters in one set, several, with a rest and in two chunks."""
+    rng = np.random.default_rng(mean + count)
+    lens = np.full(150, mean)
+    lens[[3, 60]] += [1, -1]
+    lens[[5, 6, 7]] = 0, 1, 2 * mean
+    lens[8] -= int(lens.sum()) - 150 * mean if mean > 3 else 0
+    offsets = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    child = mixed_rows(rng, rng.integers(0, 9, int(offsets[-1])), nulls=(4,))
+    lists = HostListStringsColumn(offsets, child, None, 150, 0, 0)
+    a, b = params(rng, count, 64)
+    assert nv.minhash64_ngrams(nv.DeviceListStringsColumn.from_host(lists), 3, 5, a, b).to_host().equals(orc.minhash64_ngrams(lists, 3, 5, a, b, nthreads=8))
+
+
+@pytest.mark.parametrize("kind", ["zero", "small", "power", "digits of 2", "digits of 1", "wraps", "top"])
+def test_minhash64_ngrams_parameters(nv, orc, kind):
+    """The same of short lists, whose products are computed whole: sums at p and beyond, which are reduced only where one occurs."""
+    rng = np.random.default_rng(8)
+    a, b = hard_parameters(kind)
+    lens = np.array([1, 2, 3, 6, 7, 8, 64, 66, 70, 100])
+    offsets = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    lists = HostListStringsColumn(offsets, mixed_rows(rng, rng.integers(0, 9, int(offsets[-1]))), None, lens.size, 0, 0)
+    assert nv.minhash64_ngrams(nv.DeviceListStringsColumn.from_host(lists), 2, 5, a, b).to_host().equals(orc.minhash64_ngrams(lists, 2, 5, a, b, nthreads=8))
 
 
 def words_column(rng, lens, vocabulary, oov):
