@@ -986,6 +986,40 @@ __global__ void range_first_row_kernel(ColView col, int64_t first_offset, uint32
   range_first_row[g] = lo;
 }
 
+// A column that is put on the stream whole before its size is known (see nvtext_amd_wordpiece_tokenize).  One launch that
+// does everything per tile beats the three passes up to about 50 MB of text (16 MB of the benchmark's rows 125 against
+// 245 us, 32 MB 211 against 286, 48 MB 300 against 319, 60 MB 359 against 337), after which the passes' better use of the
+// lanes tells; it stops at 32 MB for its temporaries.
+// These are sized for the bytes that a column of so many rows is guessed to have at most, kSmallGuess a row (kSmallSure in
+// any case), and for kSmallLeastSlots and kSmallLeastQueue of every tile of that;
+// the tiles that there are share them out, up to kSmallSlots and kSmallQueue each.  A column of more bytes (up to
+// kSmallRowBytes a row and kSmallBytes in all), or with a tile that needs more, is done once more, in what its bytes take.  (32,768 rows of 120 bytes held 224 MB where room for 32 MB
+// of text with a word per two bytes was set aside, and 31 MB this way, 45 us both; 8,192 rows of 3000 bytes, done once more,
+// 182 MB instead of 241 and 162 us instead of 150; the passes of a large column take 197 MB and 258 us.)
+constexpr int32_t kSmallRows        = 131072;
+constexpr int64_t kSmallRowBytes    = 4096;
+constexpr int64_t kSmallGuess       = 256;
+constexpr int64_t kSmallLeast       = 256 << 10;
+constexpr int64_t kSmallSure        = 8 << 20;
+constexpr int64_t kSmallBytes       = 32 << 20;
+constexpr int kSmallTile            = 1024;
+constexpr uint32_t kSmallSlots      = kSmallTile / 2 + 8;  // words of a tile: one letter and a space each (rows of one letter go the other way)
+constexpr uint32_t kSmallLeastSlots = kSmallTile / 4 + 8;  // (six bytes to a word and its space are ordinary)
+constexpr uint32_t kSmallQueue      = kSmallTile / 8;      // words of a tile that are not in the vocabulary (one in 37 bytes on the benchmark's rows)
+constexpr uint32_t kSmallLeastQueue = kSmallTile / 16;
+constexpr unsigned kSmallGrid       = 2048;                // workgroups at most: a wavefront then takes several tiles
+// What every one of `tiles` tiles gets of the slots and of the queue's records (an even number of slots).
+__host__ __device__ inline uint32_t small_slots(uint32_t slots, uint32_t tiles)
+{
+  uint32_t const each = slots / tiles;
+  return (each < kSmallSlots ? each : kSmallSlots) & ~1u;
+}
+__host__ __device__ inline uint32_t small_queue(uint32_t records, uint32_t tiles)
+{
+  uint32_t const each = records / tiles;
+  return each < kSmallQueue ? each : kSmallQueue;
+}
+
 // One tile at a time per wavefront: stage its bytes (and the 256 after it) in LDS; mark the row starts in it; find
 // word starts and ends (lanes <-> 16-byte blocks: spaces by SWAR, row starts as extra separators); with a word limit,
 // drop the words past each row's limit; list the words (word k pairs start k with end k); look all of them up (lanes
@@ -1012,6 +1046,8 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
     a.range_tiles  = 1;
     a.unit_begin   = 0;
     a.unit_end     = a.nranges;
+    a.range_cap    = small_slots(a.range_cap, a.nranges);  // (of all: shared out)
+    a.queue_cap    = small_queue(a.queue_cap, a.nranges);
   }
   constexpr int kBlocks       = TILE / 16;
   constexpr int kSubs         = kBlocks / kWave;
@@ -2029,18 +2065,6 @@ __global__ void __launch_bounds__(kRareThreads) wordpiece_retokenize_kernel(Voca
 // looked up whole.  It runs on the offsets alone, before the host knows where the bytes begin, and leaves the view's
 // first and last offset for the host as well: the call synchronises once for both.
 constexpr int kSampleWindows = 512;
-// A column that is put on the stream whole before its size is known (see nvtext_amd_wordpiece_tokenize).  One launch that
-// does everything per tile beats the three passes up to about 50 MB of text (16 MB of the benchmark's rows 125 against
-// 245 us, 32 MB 211 against 286, 48 MB 300 against 319, 60 MB 359 against 337), after which the passes' better use of the
-// lanes tells; it stops at 32 MB for its temporaries, six bytes per byte that the column might have.
-constexpr int32_t kSmallRows     = 131072;
-constexpr int64_t kSmallRowBytes = 4096;
-constexpr int64_t kSmallLeast    = 256 << 10;
-constexpr int64_t kSmallBytes    = 32 << 20;
-constexpr int kSmallTile         = 1024;
-constexpr uint32_t kSmallSlots   = kSmallTile / 2 + 8;  // words of a tile: one letter and a space each (rows of one letter go the other way)
-constexpr unsigned kSmallGrid    = 2048;                // workgroups at most: a wavefront then takes several tiles
-constexpr uint32_t kSmallQueue   = kSmallTile / 8;  // words of a tile that are not in the vocabulary (one in 37 bytes on the benchmark's rows)
 constexpr int kSampleBytes   = 512;
 constexpr int kSampleTail    = 208;  // bytes staged past a window: a word that starts in it ends there, or is kMaxWord bytes or more
 static_assert(3 * kSampleWindows <= kHostSampleWords, "a window's three counts fit the pinned words");
@@ -2600,76 +2624,83 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   bool const is64  = input->offsets_is_int64 != 0;
   bool const limit = max_words_per_row > 0;
   // A column of few rows is probably small, and then the call is launches and waits more than work: everything up to the
-  // number of tokens is put on the stream at once, for a column of up to kSmallRowBytes bytes a row and kSmallBytes in all,
-  // before the host knows how many bytes there are.  Where there are more, these kernels leave at once and the call goes on
-  // as for a large column.
+  // number of tokens is put on the stream at once, before the host knows how many bytes there are.  Where there are more
+  // than were guessed, these kernels leave at once; up to small_most the same follows with the temporaries that the bytes
+  // take (which is also done where a tile had not enough of them), beyond the call goes on as for a large column.
   // (29 rows of 180 bytes: 87 us in eleven launches with two waits, 43 us in four with one; 32,768 rows of 120 bytes
   // 145 -> 60 us)
-  bool const small = scalars && sampling && rows <= kSmallRows && g_forced_range_tiles.load(std::memory_order_relaxed) == 0;
-  int64_t const small_bytes = small ? std::min(std::max(static_cast<int64_t>(rows) * kSmallRowBytes, kSmallLeast), kSmallBytes) : 0;
-  uint32_t const small_ranges = static_cast<uint32_t>(small_bytes / kSmallTile + 1);
-  size_t const small_temp_bytes[8] = {static_cast<size_t>(small_ranges) * kSmallSlots * sizeof(uint32_t),
-                                      (static_cast<size_t>(small_ranges) + 1) * sizeof(uint32_t),
-                                      static_cast<size_t>(small_ranges) * sizeof(uint32_t),
-                                      static_cast<size_t>(small_ranges) * sizeof(uint32_t),
-                                      static_cast<size_t>(small_ranges) * sizeof(uint32_t),
-                                      (static_cast<size_t>(small_ranges) + 1) * sizeof(int64_t),
-                                      (static_cast<size_t>(small_ranges) * kSmallQueue + 1) * sizeof(uint32_t),
-                                      static_cast<size_t>(small_ranges) * kSmallQueue * sizeof(OovEntry)};
-  if (small) {
-    TempParts<8> const temps(mr, small_temp_bytes);
-    if (temps.ok()) {
-      TileArgs args{};
-      args.col           = v;
-      args.table         = vocabulary->table;
-      args.max_words     = max_words_per_row;
-      args.range_cap     = kSmallSlots;
-      args.arena         = temps.part<uint32_t>(0);
-      args.first_row_out = temps.part<uint32_t>(1);
-      args.range_words   = temps.part<uint32_t>(2);
-      args.range_tokens  = temps.part<uint32_t>(3);
-      args.range_notes   = temps.part<uint32_t>(4);
-      args.offsets_out   = out->offsets;
-      args.queue         = temps.part<OovEntry>(7);
-      args.queue_cap     = kSmallQueue;
-      args.most_bytes    = small_bytes;
-      int64_t* const bases        = temps.part<int64_t>(5);
-      uint32_t* const again_count = temps.part<uint32_t>(6);
-      void (*const kernel)(TileArgs) = is64 ? (limit ? wordpiece_word_kernel<kSmallTile, true, true, true> : wordpiece_word_kernel<kSmallTile, true, false, true>)
-                                            : (limit ? wordpiece_word_kernel<kSmallTile, false, true, true> : wordpiece_word_kernel<kSmallTile, false, false, true>);
-      {
-        ProfileScope ps("wordpiece_word_kernel (small column)", stream);
-        hipLaunchKernelGGL(kernel, dim3(std::min((small_ranges + kTokWaves - 1) / kTokWaves, kSmallGrid)), dim3(kTokThreads), 0, stream, args);
+  bool const small    = scalars && sampling && rows <= kSmallRows && g_forced_range_tiles.load(std::memory_order_relaxed) == 0;
+  int64_t const small_most = std::min(std::max(rows * kSmallRowBytes, kSmallLeast), kSmallBytes);
+  int64_t small_bytes      = small ? std::min(std::max(rows * kSmallGuess, kSmallSure), small_most) : 0;
+  for (int attempt = 0; attempt < 2 && small_bytes > 0; ++attempt) {
+    uint32_t const most_ranges  = static_cast<uint32_t>(small_bytes / kSmallTile + 2);
+    uint32_t const slots        = most_ranges * (attempt == 0 ? kSmallLeastSlots : kSmallSlots);
+    uint32_t const records      = most_ranges * (attempt == 0 ? kSmallLeastQueue : kSmallQueue);
+    size_t const temp_bytes[8]  = {static_cast<size_t>(slots) * sizeof(uint32_t),
+                                   (static_cast<size_t>(most_ranges) + 1) * sizeof(uint32_t),
+                                   static_cast<size_t>(most_ranges) * sizeof(uint32_t),
+                                   static_cast<size_t>(most_ranges) * sizeof(uint32_t),
+                                   static_cast<size_t>(most_ranges) * sizeof(uint32_t),
+                                   (static_cast<size_t>(most_ranges) + 1) * sizeof(int64_t),
+                                   (static_cast<size_t>(records) + 1) * sizeof(uint32_t),
+                                   static_cast<size_t>(records) * sizeof(OovEntry)};
+    TempParts<8> const temps(mr, temp_bytes);
+    if (!temps.ok()) break;  // (no room: as for a large column)
+    TileArgs args{};
+    args.col           = v;
+    args.table         = vocabulary->table;
+    args.max_words     = max_words_per_row;
+    args.range_cap     = slots;
+    args.arena         = temps.part<uint32_t>(0);
+    args.first_row_out = temps.part<uint32_t>(1);
+    args.range_words   = temps.part<uint32_t>(2);
+    args.range_tokens  = temps.part<uint32_t>(3);
+    args.range_notes   = temps.part<uint32_t>(4);
+    args.offsets_out   = out->offsets;
+    args.queue         = temps.part<OovEntry>(7);
+    args.queue_cap     = records;
+    args.most_bytes    = small_bytes;
+    int64_t* const bases        = temps.part<int64_t>(5);
+    uint32_t* const again_count = temps.part<uint32_t>(6);
+    void (*const kernel)(TileArgs) = is64 ? (limit ? wordpiece_word_kernel<kSmallTile, true, true, true> : wordpiece_word_kernel<kSmallTile, true, false, true>)
+                                          : (limit ? wordpiece_word_kernel<kSmallTile, false, true, true> : wordpiece_word_kernel<kSmallTile, false, false, true>);
+    {
+      ProfileScope ps("wordpiece_word_kernel (small column)", stream);
+      hipLaunchKernelGGL(kernel, dim3(std::min((most_ranges + kTokWaves - 1) / kTokWaves, kSmallGrid)), dim3(kTokThreads), 0, stream, args);
+    }
+    HostPost const post = new_post();
+    hipLaunchKernelGGL(wordpiece_finish_kernel, dim3(1), dim3(kFinishThreads), 0, stream, args, kSmallTile, bases, again_count, scalars, post);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = wait_for_post(post, stream);
+    if (e != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
+    first_offset = static_cast<int64_t>(scalars[0]);
+    last_offset  = static_cast<int64_t>(scalars[1]);
+    int64_t const bytes = last_offset - first_offset;
+    if (bytes <= 0 || bytes > small_most) break;
+    const uint8_t* const first_byte = v.chars + first_offset;
+    uint32_t const cbeg             = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(first_byte) & 15u);
+    uint32_t const nranges          = static_cast<uint32_t>((cbeg + bytes + kSmallTile - 1) / kSmallTile);
+    if (bytes <= small_bytes && (scalars[3] & kNoteSpill) == 0) {
+      uint64_t const total = scalars[2];
+      out->child_size      = static_cast<int64_t>(total);
+      out->child_bytes     = static_cast<size_t>(total) * sizeof(int32_t);
+      if (total) {
+        out->child = mr.allocate(out->child_bytes);
+        if (!out->child) return give_up(NVTEXT_AMD_ALLOC_FAILED, "child allocation failed");
       }
-      HostPost const post = new_post();
-      hipLaunchKernelGGL(wordpiece_finish_kernel, dim3(1), dim3(kFinishThreads), 0, stream, args, kSmallTile, bases, again_count, scalars, post);
-      hipError_t e = hipGetLastError();
-      if (e == hipSuccess) e = wait_for_post(post, stream);
-      if (e != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
-      first_offset = static_cast<int64_t>(scalars[0]);
-      last_offset  = static_cast<int64_t>(scalars[1]);
-      if (last_offset > first_offset && last_offset - first_offset <= small_bytes && (scalars[3] & kNoteSpill) == 0) {
-        uint64_t const total = scalars[2];
-        out->child_size      = static_cast<int64_t>(total);
-        out->child_bytes     = static_cast<size_t>(total) * sizeof(int32_t);
-        if (total) {
-          out->child = mr.allocate(out->child_bytes);
-          if (!out->child) return give_up(NVTEXT_AMD_ALLOC_FAILED, "child allocation failed");
-        }
-        const uint8_t* const first_byte = v.chars + first_offset;
-        uint32_t const cbeg             = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(first_byte) & 15u);
-        uint32_t const nranges          = static_cast<uint32_t>((cbeg + (last_offset - first_offset) + kSmallTile - 1) / kSmallTile);
-        ProfileScope ps("wordpiece_emit_kernel", stream);
-        hipLaunchKernelGGL(wordpiece_emit_kernel, dim3((nranges + kTokWaves - 1) / kTokWaves), dim3(kTokThreads), 0, stream, nranges, args.arena, kSmallSlots,
-                           args.range_words, bases, args.first_row_out, args.queue, out->offsets, static_cast<int32_t*>(out->child), again_count + 1,
-                           again_count);
-        if (scalars[3] & kNoteAgain)
-          hipLaunchKernelGGL(wordpiece_retokenize_kernel, dim3(64), dim3(kRareThreads), 0, stream, vocabulary->table,
-                             reinterpret_cast<const uint4*>(first_byte - cbeg), args.queue, again_count + 1, again_count, static_cast<int32_t*>(out->child));
-        if (hipGetLastError() != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, "kernel launch failed");
-        return NVTEXT_AMD_SUCCESS;
-      }
-    }  // (no room for the temporaries of the largest column that it might be: as for a large column)
+      ProfileScope ps("wordpiece_emit_kernel", stream);
+      hipLaunchKernelGGL(wordpiece_emit_kernel, dim3((nranges + kTokWaves - 1) / kTokWaves), dim3(kTokThreads), 0, stream, nranges, args.arena,
+                         small_slots(slots, nranges), args.range_words, bases, args.first_row_out, args.queue, out->offsets,
+                         static_cast<int32_t*>(out->child), again_count + 1, again_count);
+      if (scalars[3] & kNoteAgain)
+        hipLaunchKernelGGL(wordpiece_retokenize_kernel, dim3(64), dim3(kRareThreads), 0, stream, vocabulary->table,
+                           reinterpret_cast<const uint4*>(first_byte - cbeg), args.queue, again_count + 1, again_count, static_cast<int32_t*>(out->child));
+      if (hipGetLastError() != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, "kernel launch failed");
+      return NVTEXT_AMD_SUCCESS;
+    }
+    // more bytes than were guessed, or a tile that needs more than its share; with the most a tile is given: a large column's way
+    bool const full = bytes <= small_bytes && small_slots(slots, nranges) == kSmallSlots && small_queue(records, nranges) == kSmallQueue;
+    small_bytes     = full ? 0 : bytes;
   }
   Temp const hot(mr, scalars && sampling ? kHotWords * sizeof(uint32_t) : 0);
   if (!hot.ok()) return give_up(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");

@@ -248,6 +248,44 @@ def test_tokenize_small_columns(nv, orc, limit, oov):
             assert nv.wordpiece_tokenize(d.slice(3, host.size - 2, 0), vocabulary, limit).to_host().equals(orc.wordpiece_tokenize(view, reference, limit))
 
 
+def test_tokenize_small_columns_hold_little_memory(nv):
+    """32,768 rows of about 120 bytes: the temporaries of a call do not grow to what the largest column of so many rows takes."""
+    import torch
+    rng = np.random.default_rng(5)
+    words = words_column(rng, [120] * 64, VOCABULARY, 0.1)
+    n = int(words.offsets[-1])
+    offsets = (np.arange(512)[:, None] * n + np.asarray(words.offsets[:-1])).reshape(-1)
+    host = HostStringsColumn(np.tile(words.chars[:n], 512), np.append(offsets, 512 * n).astype(np.int32), None, 512 * 64, 0, 0)
+    column, vocabulary = dev(nv, host), nv.WordPieceVocabulary(dev(nv, HostStringsColumn.from_pylist(VOCABULARY)))
+    nv.wordpiece_tokenize(column, vocabulary, 0)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    held = torch.cuda.memory_allocated()
+    nv.wordpiece_tokenize(column, vocabulary, 0)
+    assert torch.cuda.max_memory_allocated() - held < 16 * host.chars.size
+
+
+@pytest.mark.parametrize("limit", [0, 40])
+@pytest.mark.parametrize("megabytes", [3, 6, 7.99, 8.01, 20])
+@pytest.mark.parametrize("dense", ["", "a b ", "abcq hello world "])
+def test_tokenize_small_columns_again(nv, orc, megabytes, dense, limit):
+    """Columns of fewer and of more bytes than their rows let one guess (8 MiB), with room for all that a tile is given and
+    for half of it; in some a few tiles have more words, or more unknown ones, than that half."""
+    rng = np.random.default_rng(int(megabytes))
+    hv = HostStringsColumn.from_pylist(VOCABULARY)
+    vocabulary, reference = nv.WordPieceVocabulary(dev(nv, hv)), orc.Vocabulary(hv)
+    piece = words_column(rng, [200_000], VOCABULARY, 0.1).chars
+    total = int(megabytes * (1 << 20))
+    chars = np.tile(piece, total // piece.size + 1)[:total].copy()
+    if dense:
+        patch = np.frombuffer((dense * (5000 // len(dense))).encode(), np.uint8)
+        for at in (100_000, total // 2, total - 9000):
+            chars[at: at + patch.size] = patch
+    offsets = np.linspace(0, total, 4001).astype(np.int32)
+    host = HostStringsColumn(chars, offsets, None, 4000, 0, 0)
+    assert nv.wordpiece_tokenize(dev(nv, host), vocabulary, limit).to_host().equals(orc.wordpiece_tokenize(host, reference, limit, nthreads=8))
+
+
 @pytest.mark.parametrize("rows, each", [(4, 65_537), (4, 65_535), (131_072, 10), (131_073, 10), (9000, 3800)])
 def test_tokenize_where_small_columns_end(nv, orc, rows, each):
     """Around the bytes (256 KiB; 32 MiB) and the rows up to which a column is put on the stream before its size is known."""
