@@ -322,12 +322,16 @@ def test_tokenize_words_met_before(nv, orc, different, limit, wide):
 
 
 @pytest.mark.parametrize("rows, each", [(1, 1), (3, 2047), (3, 2048), (61, 300), (4, 65_535), (4, 65_537), (131_072, 9), (131_073, 9), (30_000, 2300)])
-def test_normalize_where_small_columns_end(nv, rows, each):
+@pytest.mark.parametrize("brackets", [True, False])
+def test_normalize_where_small_columns_end(nv, rows, each, brackets):
     """Tiles of 2048 bytes and their remainders, and the bytes (256 KiB; 64 MiB) and rows up to which a column is worked on
-    before its size is known; a view of it too."""
+    before its size is known; a view of it too.  With a special token in every tile, which is then written the long way, and
+    without."""
     from oracle import normalize_py
     rng = np.random.default_rng(rows)
     text = "Héllo Wörld, [CLS] naïve 漢字! ΑΒΓ don't [sep] plain words and more plain words of text "
+    if not brackets:
+        text = text.replace("[", "\u200b").replace("]", "\u0301")
     chars = np.frombuffer((text * (rows * each // len(text) + 1)).encode(), np.uint8).copy()
     cuts = np.sort(rng.integers(0, chars.size, rows - 1)) if rows > 1 else np.zeros(0, np.int64)
     while True:  # whole characters

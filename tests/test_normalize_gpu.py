@@ -9,7 +9,7 @@ from tests.golden_cases import strings
 
 pytestmark = pytest.mark.gpu
 
-TILE = 1024  # input bytes per workgroup in the library: cases below put interesting bytes around its multiples
+TILE = 2048  # input bytes per workgroup in the library: cases below put interesting bytes around its multiples
 
 
 @pytest.fixture(scope="module")
