@@ -933,7 +933,8 @@ __global__ void __launch_bounds__(kPlanThreads) minhash_plan_kernel(RowParts<Sou
 // The same for a column of more rows, in two launches: the sums of tiles of rows (parts in the low half, valid rows in the
 // high half; the workgroups behind them lay out the parameters of 64-bit hashes), then, from the sums of the tiles before,
 // the places of every row, and the largest value into the slots of the rows that are done in several parts: a wavefront
-// looks at 64 rows and fills those of them one after the other.  A tile is `passes` times 256 rows, so that there are at
+// fills those of sixteen rows, one after the other (of 64: 8,193 lists of 400 elements, 256 parameters, 83.3 us the call, with this 77.4; 0.6 us more
+// where no row is cut).  A tile is `passes` times 256 rows, so that there are at
 // most kSumTiles.
 inline int32_t sum_passes(int32_t rows) { return (rows - 1) / (kThreads * kSumTiles) + 1; }
 
@@ -960,32 +961,44 @@ __global__ void __launch_bounds__(kThreads) minhash_sums_kernel(RowParts<Source>
   if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
+constexpr int kPlaceThreads = 1024;  // four wavefronts take the rows, all sixteen fill
 template <typename Source, typename T = typename Source::T>
-__global__ void __launch_bounds__(kThreads) minhash_places_kernel(RowParts<Source> parts, int32_t P, int32_t passes, const uint64_t* __restrict__ sums,
-                                                                  int32_t* __restrict__ out_offsets, uint32_t* __restrict__ prefix,
-                                                                  unsigned long long* __restrict__ counters, T* __restrict__ out)
+__global__ void __launch_bounds__(kPlaceThreads) minhash_places_kernel(RowParts<Source> parts, int32_t P, int32_t passes, const uint64_t* __restrict__ sums,
+                                                                       int32_t* __restrict__ out_offsets, uint32_t* __restrict__ prefix,
+                                                                       unsigned long long* __restrict__ counters, T* __restrict__ out)
 {
-  __shared__ uint64_t lds[kWaves + 1];
+  constexpr int kFill = kThreads / (kPlaceThreads / kWave);  // rows of the tile whose slots a wavefront fills
+  __shared__ uint64_t lds[kPlaceThreads / kWave + 1];
+  __shared__ uint64_t several[kWaves];
+  __shared__ int32_t places[kThreads];
   if (blockIdx.x == 0) start_counters(counters, parts.waves);
   int32_t const rows = parts.source.rows();
   auto const cut     = parts.cut();
+  int const tid = static_cast<int>(threadIdx.x), lane = lane_id(), wave = tid / kWave;
   uint64_t mine = 0, carry;
-  for (uint32_t i = threadIdx.x; i < blockIdx.x; i += kThreads) mine += sums[i];
-  block_exclusive_scan64<kThreads>(mine, lds, &carry);
-  int const lane = lane_id();
+  if (threadIdx.x < blockIdx.x) mine = sums[threadIdx.x];
+  static_assert(kSumTiles == kPlaceThreads, "a sum per thread");
+  block_exclusive_scan64<kPlaceThreads>(mine, lds, &carry);
   for (int32_t pass = 0; pass < passes; ++pass) {
-    int64_t const i  = (static_cast<int64_t>(blockIdx.x) * passes + pass) * kThreads + threadIdx.x;
-    uint64_t const v = i < rows ? parts_and_rows(parts, cut, parts.source.length(i), parts.source.valid(i)) : 0ull;
+    int64_t const i  = (static_cast<int64_t>(blockIdx.x) * passes + pass) * kThreads + tid;
+    uint64_t const v = tid < kThreads && i < rows ? parts_and_rows(parts, cut, parts.source.length(i), parts.source.valid(i)) : 0ull;
     uint64_t total;
-    uint64_t const before = block_exclusive_scan64<kThreads>(v, lds, &total) + carry;
+    uint64_t const before = block_exclusive_scan64<kPlaceThreads>(v, lds, &total) + carry;  // (its barriers: the tile before is filled)
     carry += total;
     int32_t const place = parts.source.masked() ? static_cast<int32_t>(before >> 32) * P : static_cast<int32_t>(i * P);
-    if (i <= rows) {
-      prefix[i]      = static_cast<uint32_t>(before);
-      out_offsets[i] = place;
+    if (tid < kThreads) {
+      if (i <= rows) {
+        prefix[i]      = static_cast<uint32_t>(before);
+        out_offsets[i] = place;
+      }
+      places[tid]       = place;
+      uint64_t const is = ballot64(static_cast<uint32_t>(v) > 1u);
+      if (lane == 0) several[wave] = is;
     }
-    for (uint64_t todo = ballot64(static_cast<uint32_t>(v) > 1u); todo != 0; todo &= todo - 1) {
-      T* const dst = out + __builtin_amdgcn_readlane(place, __builtin_ctzll(todo));
+    __syncthreads();
+    uint32_t const word = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(several[wave * kFill / kWave] >> (wave * kFill % kWave))));
+    for (uint32_t todo = word & ((1u << kFill) - 1u); todo != 0; todo &= todo - 1) {
+      T* const dst = out + places[wave * kFill + __builtin_ctz(todo)];
       for (int32_t j = lane; j < P; j += kWave) dst[j] = std::numeric_limits<T>::max();
     }
   }
@@ -1097,7 +1110,7 @@ void run_minhash(Source const& source, int32_t rows, bool short_rows, const T* a
     int32_t const passes = sum_passes(rows), tiles = (rows - 1) / (kThreads * passes) + 1;
     hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_sums_kernel<Source>), dim3(static_cast<unsigned>(tiles + layers(kThreads))), dim3(kThreads), 0, stream, parts,
                        params, laid_out, tiles, passes, sums);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_places_kernel<Source>), dim3(static_cast<unsigned>(rows / (kThreads * passes) + 1)), dim3(kThreads), 0, stream,
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(minhash_places_kernel<Source>), dim3(static_cast<unsigned>(rows / (kThreads * passes) + 1)), dim3(kPlaceThreads), 0, stream,
                        parts, P, passes, sums, offsets, prefix, counters, child);
   }
 
