@@ -27,38 +27,40 @@ HBM_PEAK_GBS = 8000.0
 #
 # HBM bytes per launch (fetched, written) of the tokenizer kernels on the full C2 workload: FETCH_SIZE / WRITE_SIZE
 # scaled by a copy kernel of known size.
-TRAFFIC_SOURCE = "profiles/hbm_traffic_pmc_all_workloads.md (library sources at commit 692bfef)"
+TRAFFIC_SOURCE = "profiles/hbm_traffic_pmc_all_workloads.md (library sources at commit ed349d2)"
 MEASURED_TRAFFIC_C2 = {
-    "range_first_row_kernel": (15968662, 248800),
-    "wordpiece_word_kernel": (1742880831, 1556229099),
-    "wordpiece_oov_kernel": (861252878, 857545519),
-    "wordpiece_emit_kernel": (1393668802, 905164798),
+    "range_first_row_kernel": (16690033, 4691648),
+    "wordpiece_word_kernel": (1877599521, 1980403784),
+    "wordpiece_oov_kernel": (909629066, 876921109),
+    "wordpiece_emit_kernel": (1406373429, 901158342),
 }
 # (the fetch counter prices a read that misses L2 at a whole 128-byte line whatever was asked for, and counts the misses
-# that the Infinity Cache serves: most of what the tokenizer fetches on C5 is lines of its 8 MB table)
+# that the Infinity Cache serves: most of what the tokenizer fetches on C5 is lines of its 8 MB table and of its memo)
 MEASURED_TRAFFIC_C5_TOKENIZE = {
-    "range_first_row_kernel": (119625264, 995168),
-    "wordpiece_word_kernel": (24310186114, 5163209271),
-    "wordpiece_oov_kernel": (21481440462, 2092868777),
-    "wordpiece_emit_kernel": (4729690208, 3361303065),
+    "range_first_row_kernel": (228889997, 6184320),
+    "wordpiece_word_kernel": (24716537736, 6764651040),
+    "wordpiece_oov_kernel": (21534003902, 2154592293),
+    "wordpiece_emit_kernel": (4801165018, 3328190789),
 }
 MEASURED_TRAFFIC_C5_NORMALIZE = {
-    "normalize_count_kernel": (4575175068, 63532928),
-    "normalize_tile_rows_kernel": (73449328, 7941632),
-    "normalize_write_kernel": (5469615636, 4672395239),
+    "normalize_count_kernel": (4574918838, 63532928),
+    "normalize_tile_rows_kernel": (73443184, 7941632),
+    "normalize_write_kernel": (5468197637, 4674942398),
 }
 # minhash: VALU wave-instructions executed per (window, parameter) of a wavefront (SQ_INSTS_VALU / (windows x P / 64)) and
 # the share of SIMD cycles that issued one (SQ_INSTS_VALU x 4 / (1024 SIMDs x kernel cycles), capped at 1: adds and
-# moves issue in fewer than 4 cycles).  The floor is the instruction sequence of the inner loop: uint32, one
-# v_mad_u64_u32 per product and one v_min3_u32 per two (1.5); uint64, three v_mad_u64_u32 and a 32-bit add for (h * a + b)
-# mod 2^64, a shift, a mask and one more v_mad_u64_u32 for the fold mod 2^61-1, one v_min_f64, one v_max3_u32 per two
-# products (8.5).  Every window of the input counts as one, also those whose hash the wavefront met lately and does not
-# fold again (windows of a row repeat, most in long rows: that is how C4 comes so near the floor).
-VALU_SOURCE = "profiles/valu_issue_pmc_all_workloads.md (library sources at commit 692bfef)"
+# moves issue in fewer than 4 cycles).  A product that is folded takes, in the inner loop: uint32, one v_mad_u64_u32 and
+# half a v_min3_u32 (1.5); uint64, where the matrix cores find products to 17 bits, 40.5 instructions for the 16 products
+# that a lane has of 1,024 (2.53), beside two matrix instructions of 32 cycles, which keep the matrix cores busy for 40 %
+# of the time that takes.  Windows of a row repeat, and a window met before need not be folded again: the floor counts the
+# different windows of a row only (their share is found on the first rows of the workload), the measured figure is over
+# all of them.
+VALU_SOURCE = "profiles/valu_issue_pmc_all_workloads.md (library sources at commit ed349d2)"
+PRODUCT_INST = {32: 1.5, 64: 2.53}
 MINHASH_VALU = {
-    "C3": {"floor": 1.5, "measured": 1.72, "issue": 0.97},
-    "C4": {"floor": 8.5, "measured": 8.73, "issue": 0.88},
-    "C5": {"floor": 8.5, "measured": 13.08, "issue": 1.05},
+    "C3": {"bits": 32, "measured": 1.48, "issue": 1.04},
+    "C4": {"bits": 64, "measured": 3.89, "issue": 0.87},
+    "C5": {"bits": 64, "measured": 7.19, "issue": 0.84},
 }
 
 
@@ -157,8 +159,8 @@ def measure(fn, steps, warmup, capi, torch):
 
 
 def kernel_times(fn, reps, capi, torch):
-    """Average duration of each library kernel, from HIP events recorded by the library on the
-    stream it launches on."""
+    """Duration of each library kernel per call, all its launches of the call together, from HIP events recorded by the
+    library on the stream it launches on."""
     capi.profile_enable(True)
     capi.profile_read()
     acc = {}
@@ -168,7 +170,7 @@ def kernel_times(fn, reps, capi, torch):
         for name, ms in capi.profile_read():
             acc.setdefault(name, []).append(ms)
     capi.profile_enable(False)
-    return {k: sum(v) / len(v) for k, v in acc.items()}
+    return {k: sum(v) / reps for k, v in acc.items()}
 
 
 def hbm_roofline(alg_bytes, sec, kt, traffic=None):
@@ -186,12 +188,30 @@ def hbm_roofline(alg_bytes, sec, kt, traffic=None):
             "kernel_frac": round(alg_bytes / (kt[dom] * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)}
 
 
-def valu_object(name):
-    """minhash is bound by VALU issue: the share of the SIMDs' issue slots that the floor sequence of the inner loop
-    would need, floor / measured instructions per permutation x measured issue rate.  It cannot exceed 1."""
+def distinct_windows(col, width, most_bytes=1 << 20):
+    """The share of the windows of a row that differ from all others of the row, over the first rows of a column that
+    hold most_bytes (long rows are cut to 64 KiB)."""
+    windows = different = used = 0
+    for i in range(col.size):
+        begin, end = int(col.offsets[col.offset + i]), int(col.offsets[col.offset + i + 1])
+        text = col.chars[begin: min(end, begin + (1 << 16))].tobytes().decode("utf-8", "ignore")
+        n = max(len(text) - width + 1, 0)
+        windows += n
+        different += len({text[k: k + width] for k in range(n)})
+        used += end - begin
+        if used >= most_bytes:
+            break
+    return different / windows if windows else 1.0
+
+
+def valu_object(name, share):
+    """minhash is bound by VALU issue: the share of the SIMDs' issue slots that the inner loop's instructions for the
+    different windows need, floor / measured instructions per permutation x measured issue rate."""
     v = MINHASH_VALU[name]
-    return {"bound": "valu issue", "floor_inst_per_perm": v["floor"], "measured_inst_per_perm": v["measured"],
-            "valu_issue": v["issue"], "frac": round(v["floor"] / v["measured"] * min(1.0, v["issue"]), 3), "source": VALU_SOURCE}
+    floor = PRODUCT_INST[v["bits"]] * share
+    return {"bound": "valu issue", "floor_inst_per_perm": round(floor, 3), "distinct_windows": round(share, 3),
+            "measured_inst_per_perm": v["measured"], "valu_issue": v["issue"],
+            "frac": round(floor / v["measured"] * min(1.0, v["issue"]), 3), "source": VALU_SOURCE}
 
 
 # Peak of the VALUs: 1024 SIMDs x 2.4 GHz / 4 cycles per wave64 instruction = 614.4 G wave-instructions/s
@@ -199,11 +219,12 @@ def valu_object(name):
 VALU_WAVE_INST_PER_S = 1024 * 2.4e9 / 4
 
 
-def valu_from_rate(perm_per_s, bits):
-    """For a leg without a counter run of its own: the share of the VALUs' peak issue rate that the floor sequence of the
-    inner loop alone accounts for at the measured permutation rate (64 permutations per wave-instruction)."""
-    floor = 1.5 if bits == 32 else 8.5
-    return {"bound": "valu issue", "floor_inst_per_perm": floor,
+def valu_from_rate(perm_per_s, bits, share):
+    """For a leg without a counter run of its own: the share of the VALUs' peak issue rate that the inner loop's
+    instructions for the different windows account for at the measured permutation rate (64 permutations per
+    wave-instruction)."""
+    floor = PRODUCT_INST[bits] * share
+    return {"bound": "valu issue", "floor_inst_per_perm": round(floor, 3), "distinct_windows": round(share, 3),
             "frac": round(perm_per_s / 64 * floor / VALU_WAVE_INST_PER_S, 3), "source": "measured rate x floor / peak issue rate"}
 
 
@@ -335,7 +356,7 @@ def main():
                         "input_GBps": round(ib / msec / 1e9, 2), "mrows_per_s": round(w.rows.size / msec / 1e6, 3),
                         "gperm_per_s": round(windows * p["P"] / msec / 1e9, 1)})
             if args.minhash_scale == 1.0:
-                leg["valu"] = valu_object(name)
+                leg["valu"] = valu_object(name, distinct_windows(w.rows, p["width"]))
             if orc:
                 n = min(w.rows.size, 20000 if name == "C3" else 2000)
                 smp = w.rows.slice(0, n)
@@ -518,7 +539,7 @@ def main():
         mleg.update({"input_GBps": round(ib / msec / 1e9, 2), "mrows_per_s": round(w.rows.size / msec / 1e6, 3),
                      "windows": windows, "parameters": p["P"], "gperm_per_s": round(windows * p["P"] / msec / 1e9, 1)})
         if args.minhash_scale == 1.0:
-            mleg["valu"] = valu_object("C5")
+            mleg["valu"] = valu_object("C5", distinct_windows(w.rows, p["width"]))
         leg["minhash64"] = mleg
         if orc:
             n = min(w.rows.size, 400_000)
@@ -583,7 +604,7 @@ def reference_shapes(args, orc, _capi, datagen, nvtext, HostStringsColumn, np, t
                     windows = int(np.maximum(lengths - (width - 1), (lengths > 0).astype(np.int64)).sum())
                     leg.update({"num_rows": rows, "row_width": row_width, "hash_width": width, "parameters": nparams, "hash_type": bits,
                                 "input_GBps": round(ib / msec / 1e9, 2), "gperm_per_s": round(windows * nparams / msec / 1e9, 1),
-                                "valu": valu_from_rate(windows * nparams / msec, bits)})
+                                "valu": valu_from_rate(windows * nparams / msec, bits, distinct_windows(col, width, 1 << 18))})
                     if orc:
                         n = (400 if bits == 32 else 100) * 28_000 // row_width
                         smp = col.slice(0, n)
