@@ -203,7 +203,8 @@ struct Params {
 };
 
 // The minima of a row (or of a part of one) over the parameters of a chunk, by one wavefront: load() the chunk, reset(),
-// fold() hashes out of LDS as often as needed, finish(), each(put) calls put(j, minimum) for the parameters.
+// fold() hashes out of LDS as often as needed (the number returned are left for the next time, in front, unless it is the
+// last), finish(), each(put) calls put(j, minimum) for the parameters.
 
 // Every product computed: K sets of 64 parameters, a lane has one of each set; with TAIL the parameters beyond the last full set, when
 // there are at most 32 of them, are one more (a, b) pair per lane, shared out over sets of lanes as Packing describes, so
@@ -246,10 +247,10 @@ struct MinimaAll {
     tail_m[0] = std::numeric_limits<T>::max();
   }
   // hashes: `count` of them, and room for 63 more
-  __device__ __forceinline__ void fold(T* hashes, uint32_t count)
+  __device__ __forceinline__ uint32_t fold(T* hashes, uint32_t count, bool)
   {
     wave_lds_fence();
-    if (count == 0) return;
+    if (count == 0) return 0;
     // a duplicate never changes a minimum
     uint32_t stride = K > 1 ? kFoldTrip : pk.stride(kFoldTrip);  // a power of two, at most 64
     if (TAIL) stride = max(stride, tail_pk.stride(kFoldTrip));
@@ -264,6 +265,7 @@ struct MinimaAll {
     if (TAIL) fold_all<1>(hashes, padded, tail_pk.first(lane, kFoldTrip), tail_pk.stride(kFoldTrip), tail_a, tail_b, tail_m);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
+    return 0;
   }
   __device__ __forceinline__ void finish()
   {
@@ -398,11 +400,15 @@ struct Minima64 {
     }
   }
 
-  // hashes: `count` of them (at most 2^11 blocks of 32), and room up to the next multiple of 32
-  __device__ __forceinline__ void fold(T* hashes, uint32_t count)
+  // hashes: `count` of them (at most 2^11 blocks of 32), and room up to the next multiple of 32.  Whole blocks are done,
+  // the last time the rest as well: a block that is filled up costs what a whole one does and 50 instructions more (131,071
+  // rows of 3000 bytes, 128 parameters: a rest after every 256 windows 5633 us, one a part 5403).
+  __device__ __forceinline__ uint32_t fold(T* hashes, uint32_t count, bool last)
   {
     wave_lds_fence();
-    if (count == 0) return;
+    uint32_t const later = last ? 0u : count & 31u;
+    count -= later;
+    if (count == 0) return later;
     // The last block is filled up with hashes of the row, and their sums are set to the largest fraction: their digits are
     // zeros, so that the sum is what it starts from.  (Left as they come out, a least fraction that the filling repeats is
     // the second least of its lane as well, and all of the lane's hashes are computed exactly: one parameter in seven of a
@@ -448,8 +454,14 @@ struct Minima64 {
     }
 #pragma unroll
     for (int g = 0; g < G; ++g) settle(g, least[g], second[g], hashes, count);
+    if (later > 0) {
+      T const h = hashes[count + static_cast<uint32_t>(lane % 32)];
+      wave_lds_fence();
+      if (static_cast<uint32_t>(lane) < later) hashes[lane] = h;
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
+    return later;
   }
   __device__ __forceinline__ void finish()
   {
@@ -493,7 +505,10 @@ struct TextRows {
   static constexpr const char* kName = "minhash_parts_kernel";
   static constexpr bool kShortRows   = false;  // no more is known of their lengths than the kernels read
   static constexpr int kSimdWaves   = sizeof(T) == 4 ? 6 : 4;  // wavefronts per SIMD that its LDS leaves room for
-  static constexpr int64_t kPart    = 2816;  // (parts of up to one and a half: 4096 is no faster, and the end of the kernel is uneven by one of them)
+  // (parts of up to one and a half of it.  The end of the kernel is uneven by one of them; what a part costs beside its
+  // length is little with 32-bit hashes, for which 4096 is no faster, and a twentieth with 64-bit ones: 60,000 rows of
+  // 14,000 bytes, 128 parameters: 2816: 13.07 ms, 4096: 12.87, 6144: 12.99, which loses 3 % where rows are shorter)
+  static constexpr int64_t kPart    = sizeof(T) == 4 ? 2816 : 4096;
   static constexpr int64_t kMinPart = kTile;  // less would be staged for its halo
   static constexpr int kPartCost    = 64;
   ColView col;
@@ -515,9 +530,9 @@ struct TextRows {
     if (static_cast<int64_t>(width) * 4 <= kHalo) {
       // usual case: a window (<= 4*width bytes) fits the halo staged behind every tile
       forget_hashes(lds, lane);  // (the wave barrier after the first tile's staging comes before the first look)
+      uint32_t count = 0;  // hashes that wait to be folded (wave-uniform)
       for (int64_t base = begin; base < end; base += kTile) {
         uint32_t const cnt = static_cast<uint32_t>(min(static_cast<int64_t>(kTile), end - base));
-        uint32_t count     = 0;  // compacted hashes so far (wave-uniform)
         auto const hash    = [seed = seed](WordSrc const& src, uint32_t len) {
           T const hv = H::hash(src, len, seed);
           return hv < 1 ? T{1} : hv;  // minhash.cu:141
@@ -530,10 +545,11 @@ struct TextRows {
             count += static_cast<uint32_t>(__builtin_popcountll(vm));
           }
         });
-        minima.fold(lds.hashes, count);
+        count = minima.fold(lds.hashes, count, base + kTile >= end);
       }
     } else {
       // very wide windows: 64 starts at a time, bytes read straight from global memory
+      uint32_t count = 0;
       for (int64_t base = begin; base < end; base += kWave) {
         int64_t const gpos = base + lane;
         bool valid         = false;
@@ -550,8 +566,8 @@ struct TextRows {
           }
         }
         uint64_t const vm = ballot64(valid);
-        if (valid) lds.hashes[lanes_below(vm)] = hv;
-        minima.fold(lds.hashes, static_cast<uint32_t>(__builtin_popcountll(vm)));
+        if (valid) lds.hashes[count + lanes_below(vm)] = hv;
+        count = minima.fold(lds.hashes, count + static_cast<uint32_t>(__builtin_popcountll(vm)), base + kWave >= end);
       }
     }
   }
@@ -675,12 +691,12 @@ struct RunRows {
       uint64_t const vm = ballot64(valid);
       if (valid) lds.hashes[count + lanes_below(vm)] = hv;
       count += static_cast<uint32_t>(__builtin_popcountll(vm));
-      if (count > kRunHashes - kWave) {
-        minima.fold(lds.hashes, count);
+      if (count > kRunHashes - kWave) {  // (whole blocks but where elements are null)
+        minima.fold(lds.hashes, count, true);
         count = 0;
       }
     }
-    minima.fold(lds.hashes, count);
+    minima.fold(lds.hashes, count, true);
   }
 };
 
@@ -733,16 +749,17 @@ struct RowParts {
   }
   // Parts to a unit: an eighth of the parts there are for a wavefront, and no more than make up kPart (with what a part
   // costs beside its length); and whether one counter keeps up with handing the units out.  It answers 150 M requests a
-  // second, and a unit costs about one instruction a position for its hash and 1.5 for every 64 parameters: one counter
-  // where that takes the device twice as long.  (Of 131,071 rows of 3000 bytes, 260 parameters, 32 groups with a counter
-  // each took 4.57 ms, one counter 4.42: the groups are not done at one time.  With 26 parameters one counter took 2.10
-  // ms, 32 took 1.25.)
+  // second, and a position costs about one instruction for its hash and 1.5 for every 64 parameters (64-bit hashes: four
+  // and 2.5): one counter where a unit takes some 8192, which is twice what the device gets through meanwhile.  (Of
+  // 131,071 rows of 3000 bytes, 260 parameters, 32 groups with a counter each took 4.57 ms, one counter 4.42: the groups
+  // are not done at one time.  With 26 parameters one counter took 2.10 ms, 32 took 1.25.)
   __device__ __forceinline__ uint32_t per_unit(uint32_t total, int32_t params, bool* one_counter) const
   {
     float const mean    = static_cast<float>(source.total()) * __builtin_amdgcn_rcpf(static_cast<float>(max(total, 1u)));
     uint32_t const most = static_cast<uint32_t>(static_cast<float>(Source::kPart) * __builtin_amdgcn_rcpf(mean + static_cast<float>(Source::kPartCost)));
     uint32_t const each = max(1u, min(total / (8u * static_cast<uint32_t>(waves)), most));
-    *one_counter        = mean * static_cast<float>(each) * static_cast<float>(43 + params) >= 43.0f * 8192.0f;
+    float const work    = sizeof(typename Source::T) == 4 ? static_cast<float>(43 + params) / 43.0f : static_cast<float>(100 + params) / 25.0f;
+    *one_counter        = mean * static_cast<float>(each) * work >= 8192.0f;
     return each;
   }
 };
@@ -797,7 +814,7 @@ __global__ void __launch_bounds__(kThreads, (simd_waves<Source, Minima>())) minh
   int64_t const rows    = source.rows();
   uint32_t const total  = prefix[rows];
   bool one_counter;
-  uint32_t const each   = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(parts.per_unit(total, params.count, &one_counter))));
+  uint32_t const each   = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(parts.per_unit(total, min(params.count, Minima::kSlots), &one_counter))));
   uint32_t const units  = total / each + (total % each != 0 ? 1u : 0u);
   uint64_t const all    = static_cast<uint64_t>(units) * static_cast<uint32_t>(chunks);
   int const lane        = lane_id();

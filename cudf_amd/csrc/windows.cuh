@@ -28,7 +28,7 @@ constexpr int recent_entries() { return sizeof(T) == 4 ? 1024 : 512; }
 template <typename T>
 struct WaveLds {
   alignas(16) uint32_t bytes[kTileWords];
-  alignas(16) T hashes[kTile + 4];
+  alignas(16) T hashes[kTile + (sizeof(T) == 4 ? 4 : 36)];  // (64-bit ones: up to 31 of the tile before in front)
   alignas(16) T recent[recent_entries<T>()];
   uint16_t chars[kCharList];  // where the characters of the staged bytes start, in order (see CharMap)
 };
