@@ -27,25 +27,25 @@ HBM_PEAK_GBS = 8000.0
 #
 # HBM bytes per launch (fetched, written) of the tokenizer kernels on the full C2 workload: FETCH_SIZE / WRITE_SIZE
 # scaled by a copy kernel of known size.
-TRAFFIC_SOURCE = "profiles/hbm_traffic_pmc_all_workloads.md (library sources at commit ed349d2)"
+TRAFFIC_SOURCE = "profiles/hbm_traffic_pmc_all_workloads.md (library sources at commit 75677a8)"
 MEASURED_TRAFFIC_C2 = {
-    "range_first_row_kernel": (16690033, 4691648),
-    "wordpiece_word_kernel": (1877599521, 1980403784),
-    "wordpiece_oov_kernel": (909629066, 876921109),
-    "wordpiece_emit_kernel": (1406373429, 901158342),
+    "range_first_row_kernel": (16690018, 4691648),
+    "wordpiece_word_kernel": (1876821281, 1979659097),
+    "wordpiece_oov_kernel": (909811327, 878370418),
+    "wordpiece_emit_kernel": (1406376802, 901145955),
 }
 # (the fetch counter prices a read that misses L2 at a whole 128-byte line whatever was asked for, and counts the misses
 # that the Infinity Cache serves: most of what the tokenizer fetches on C5 is lines of its 8 MB table and of its memo)
 MEASURED_TRAFFIC_C5_TOKENIZE = {
-    "range_first_row_kernel": (228889997, 6184320),
-    "wordpiece_word_kernel": (24716537736, 6764651040),
-    "wordpiece_oov_kernel": (21534003902, 2154592293),
-    "wordpiece_emit_kernel": (4801165018, 3328190789),
+    "range_first_row_kernel": (231340168, 6184320),
+    "wordpiece_word_kernel": (24724356379, 6767157192),
+    "wordpiece_oov_kernel": (21537812574, 2154480839),
+    "wordpiece_emit_kernel": (4801143244, 3328126492),
 }
 MEASURED_TRAFFIC_C5_NORMALIZE = {
-    "normalize_count_kernel": (4574918838, 63532928),
-    "normalize_tile_rows_kernel": (73443184, 7941632),
-    "normalize_write_kernel": (5468197637, 4674942398),
+    "normalize_count_kernel": (4574919108, 63532927),
+    "normalize_tile_rows_kernel": (73443774, 7941632),
+    "normalize_write_kernel": (5468198057, 4674851582),
 }
 # minhash: VALU wave-instructions executed per (window, parameter) of a wavefront (SQ_INSTS_VALU / (windows x P / 64)) and
 # the share of SIMD cycles that issued one (SQ_INSTS_VALU x 4 / (1024 SIMDs x kernel cycles), capped at 1: adds and
@@ -55,12 +55,12 @@ MEASURED_TRAFFIC_C5_NORMALIZE = {
 # of the time that takes.  Windows of a row repeat, and a window met before need not be folded again: the floor counts the
 # different windows of a row only (their share is found on the first rows of the workload), the measured figure is over
 # all of them.
-VALU_SOURCE = "profiles/valu_issue_pmc_all_workloads.md (library sources at commit ed349d2)"
+VALU_SOURCE = "profiles/valu_issue_pmc_all_workloads.md (library sources at commit 75677a8)"
 PRODUCT_INST = {32: 1.5, 64: 2.53}
 MINHASH_VALU = {
     "C3": {"bits": 32, "measured": 1.48, "issue": 1.04},
-    "C4": {"bits": 64, "measured": 3.89, "issue": 0.87},
-    "C5": {"bits": 64, "measured": 7.19, "issue": 0.84},
+    "C4": {"bits": 64, "measured": 3.59, "issue": 0.86},
+    "C5": {"bits": 64, "measured": 6.91, "issue": 0.84},
 }
 
 
