@@ -12,8 +12,8 @@
 // fraction is the low 17 bits of the pattern.  Element 31 adds b and what the rounding may have taken away, so that the
 // fraction found is always 1 to `slack` units above X: a hash can only be the minimum if its fraction is at most the
 // least one found plus the slack.  (A sum that passes 1 comes out small: fractions below the slack are not trusted.)
-// Exact products in the vector ALUs take 8.5 instructions each; this takes 1.7, and an exact product for one in some
-// hundred.
+// Exact products in the vector ALUs take 8.5 instructions each; this takes 2.5 (39.5 for the 16 products a lane of 1,024,
+// and the two matrix instructions), and an exact product for one in some hundred.
 #pragma once
 
 #include "common.cuh"

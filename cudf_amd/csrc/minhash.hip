@@ -5,15 +5,17 @@
 // 390-424 size partitioning) with one fused pass and no chars-sized temporary:
 //
 //   * a wavefront owns a section of a row.  Per 256-position tile it stages the bytes
-//     in LDS (coalesced aligned dword loads), hashes the windows with lanes <-> window
+//     in LDS (coalesced aligned 16-byte loads), hashes the windows with lanes <-> window
 //     starts, and compacts the hashes into LDS;
-//   * it then switches to lanes <-> parameters: every lane keeps K (a, b) pairs and
+//   * it then switches to lanes <-> parameters.  32-bit hashes: every lane keeps K (a, b) pairs and
 //     K running minima in registers and streams the tile's hashes through LDS
-//     broadcast reads, so the inner loop is v_mad_u64_u32 + v_min only;
-//   * a wavefront does a row alone, or a part of it: rows are cut into parts of at most 6 KiB (of
-//     fewer bytes in a column too small to give every wavefront of the device several of that size),
-//     the parts of a row meet in the result with an atomic minimum, and the wavefronts take short rows
-//     several at a time;
+//     broadcast reads, so the inner loop is v_mad_u64_u32 + v_min only (MinimaAll).  64-bit hashes:
+//     the matrix cores find which products can be the minimum, and only those are computed
+//     (Minima64, filter64.cuh);
+//   * a wavefront does a row alone, or a part of it: rows are cut into even parts of at most 4.2 KB
+//     (64-bit hashes: 6 KiB; of fewer bytes in a column too small to give every wavefront of the device
+//     several of that size), the parts of a row meet in the result with an atomic minimum, and the
+//     wavefronts take short parts several at a time;
 //   * in a tile with characters of more than one byte the wavefront lists the characters first,
 //     so that a lane takes a character and reads its window's length instead of walking to it;
 //     hashes that the wavefront has folded lately are dropped (a minimum does not mind).
@@ -1088,8 +1090,9 @@ void with_minima(int32_t P, bool short_rows, Launch const& launch)
   }
 }
 
-// Rows of 64-bit hashes shorter than this on average have all their products computed whole.  The matrix cores spare 7
-// vector instructions a product and wavefront and cost some 800 for every 64 parameters of a row, for what has to be
+// Rows of 64-bit hashes shorter than this on average have all their products computed whole.  The matrix cores spare the
+// time of 7 vector instructions a product and wavefront (2.5 of them instead of 8.5, most of which are multiplications and
+// take longer) and cost some 800 for every 64 parameters of a row, for what has to be
 // computed exactly at its end; and as their registers take 128 parameters at most, not 320, more chunks, each of which
 // hashes the row again (20 instructions a position: runs of words come from memory).  Lists of 60 elements, 131,072 rows,
 // 128 parameters: whole 367 us, matrix cores 426; of 130: 799 and 824; of 200: 1150 and 1076; 20,000 of 200, 256
