@@ -95,7 +95,7 @@ def test_minhash_random_vs_oracle(nv, orc, utf8, P, width):
 
 
 def test_minhash_long_rows_cross_workgroups(nv, orc):
-    """Rows longer than one workgroup span (16 KiB) take the multi-workgroup + atomic-min route."""
+    """Rows of many parts, which meet in the result with an atomic minimum, among rows of one."""
     rng = np.random.default_rng(5)
     words = ["".join(rng.choice(list("abcdefghij"), int(rng.integers(1, 9)))) for _ in range(500)]
 
@@ -121,8 +121,8 @@ def test_minhash_long_rows_cross_workgroups(nv, orc):
 @pytest.mark.parametrize("P", [65, 68, 72, 80, 96, 129, 150, 200, 224, 260, 273, 288])
 def test_minhash_parameters_beyond_the_last_full_set_of_64(nv, orc, P):
     """65 to 288 parameters of which at most 32 lie beyond the last full set of 64: those share the lanes of a wavefront in
-    sets (4, 8, 16 or 32 lanes to a set) beside the full sets.  Short rows (a wavefront each), rows shared by a workgroup
-    and rows of several spans (the extra workgroups, merged with atomic minima), empty and null rows."""
+    sets (4, 8, 16 or 32 lanes to a set) beside the full sets.  Rows of one part, rows of several (which meet with an
+    atomic minimum), empty and null rows."""
     rng = np.random.default_rng(3000 + P)
     rows = random_rows(rng, 40, 900, utf8=True) + ["a", "", None, "abcdefg " * 700, "".join(rng.choice(list("abcdefghijk "), 50000)),
                                                    "é漢x " * 9000, "q" * 16384, "r" * 16385, "ab"]
@@ -138,16 +138,14 @@ def test_minhash_parameters_beyond_the_last_full_set_of_64(nv, orc, P):
 
 @pytest.mark.parametrize("rows", [140_000, 300_000, 600_000, 1_100_000])
 def test_minhash_many_rows_several_short_rows_to_a_wavefront(nv, orc, rows):
-    """From 131,072 rows on a wavefront takes 2, 4, 8 and, from 1,048,576 rows on, 16 short rows of its workgroup's group
-    instead of one.  Mostly rows of a few bytes, nulls and empty rows among them, rows of the group's last places, rows
-    just below and above the lengths that a wavefront does alone (1024 bytes, 4096 with several rows to a wavefront), and
-    rows of several workgroup spans."""
+    """Columns whose units of work are many short rows: mostly rows of a few bytes, nulls and empty rows among them, rows
+    around 1024 and 4096 bytes, and rows of several parts among them."""
     from cudf_amd.arrow_host import HostStringsColumn, pack_validity
     rng = np.random.default_rng(rows)
     lengths = rng.integers(0, 24, rows)
-    lengths[rng.integers(0, rows, rows // 200)] = rng.integers(1000, 1050, rows // 200)   # either side of 1024 bytes
-    lengths[rng.integers(0, rows, 60)] = rng.integers(4080, 4112, 60)                      # and of 4096 (the limit with several rows to a wavefront)
-    lengths[rng.integers(0, rows, 40)] = rng.integers(5000, 70000, 40)                     # shared by a workgroup; extra workgroups
+    lengths[rng.integers(0, rows, rows // 200)] = rng.integers(1000, 1050, rows // 200)   # around 1024 bytes
+    lengths[rng.integers(0, rows, 60)] = rng.integers(4080, 4112, 60)                      # and 4096
+    lengths[rng.integers(0, rows, 40)] = rng.integers(5000, 70000, 40)                     # in several parts
     lengths[-1] = 1500
     lengths[-2] = 3
     offsets = np.zeros(rows + 1, np.int64)
@@ -164,15 +162,15 @@ def test_minhash_many_rows_several_short_rows_to_a_wavefront(nv, orc, rows):
     a64 = rng.integers(1, 2**64, 5, dtype=np.uint64)
     b64 = rng.integers(0, 2**64, 5, dtype=np.uint64)
     assert_same(nv.minhash64(col, 6, a64, b64, 7).to_host(), orc.minhash64(host, 6, a64, b64, 7, nthreads=8), f"minhash64 rows={rows}")
-    # a slice whose first row is not the first of a group
+    # a slice
     lo, hi = 3, rows - 5
     hs = host.slice(lo, hi)
     assert_same(nv.minhash(col.slice(lo, hi, hs.null_count), 5, a32, b32, 4).to_host(), orc.minhash(hs, 5, a32, b32, 4, nthreads=8), f"sliced rows={rows}")
 
 
 def test_minhash_few_parameters_share_the_lanes_of_a_wavefront(nv, orc):
-    """With at most 32 parameters the lanes work in sets that each fold a part of the hashes; long rows (every wavefront
-    of a workgroup, the extra workgroups) and rows of fewer windows than sets must still give the minimum over all."""
+    """With at most 32 parameters the lanes work in sets that each fold a part of the hashes; long rows (in several
+    parts) and rows of fewer windows than sets must still give the minimum over all."""
     rng = np.random.default_rng(26)
     rows = random_rows(rng, 60, 3000) + ["k" * 40000, "".join(rng.choice(list("abcdefg "), 70000)), "ab", "abc", "abcd", "abcdefgh", "", None]
     host = strings(rows)
@@ -187,7 +185,7 @@ def test_minhash_few_parameters_share_the_lanes_of_a_wavefront(nv, orc):
 
 
 def test_minhash_more_rows_than_a_grid_has_workgroups(nv, orc):
-    """More rows than a launch has workgroups along x (2^15 groups of them, 64 rows each at this size): the rest lie along z."""
+    """More rows than the plan has tiles of 256 (1024 of them): a tile takes several passes."""
     rows = (1 << 22) + 12345
     rng = np.random.default_rng(17)
     lengths = rng.integers(0, 6, rows)
@@ -342,9 +340,8 @@ def test_minhash_ngrams_random_vs_oracle(nv, orc, P, ngrams):
 
 @pytest.mark.parametrize("rows", [150_000, 1_100_000])
 def test_minhash_ngrams_many_rows_several_short_rows_to_a_wavefront(nv, orc, rows):
-    """From 131,072 rows on a wavefront takes several short rows of its workgroup's group (16 from 1,048,576 rows on) and
-    does a row of up to 2048 positions alone.  Mostly rows of a few elements, empty and null rows and null elements among
-    them, rows either side of 2048 positions, a row of many more."""
+    """Columns whose units of work are many short rows: mostly rows of a few elements, empty and null rows and null
+    elements among them, rows around 2048 positions (in several parts), a row of many more."""
     from cudf_amd.arrow_host import HostListStringsColumn, HostStringsColumn, pack_validity
     rng = np.random.default_rng(rows + 1)
     sizes = rng.integers(0, 7, rows)

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 def _column(rng, rows, long_rows, with_nulls):
     lengths = rng.integers(0, 400, rows)
-    lengths[rng.integers(0, rows, long_rows)] = rng.integers(16385, 60000, long_rows)  # rows that take extra workgroups
+    lengths[rng.integers(0, rows, long_rows)] = rng.integers(16385, 60000, long_rows)  # rows in several parts
     offsets = np.zeros(rows + 1, np.int32)
     np.cumsum(lengths, out=offsets[1:])
     chars = rng.integers(97, 123, int(offsets[-1]), dtype=np.uint8)
