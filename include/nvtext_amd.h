@@ -222,7 +222,8 @@ nvtext_amd_status nvtext_amd_minhash64_ngrams(const nvtext_amd_list_strings_colu
  * For every row r: A, B = the sets of non-zero MurmurHash3_x86_32(seed 0) values of the `width`-character
  * windows of input1[r], input2[r] (the window rule of nvtext_amd_minhash); result[r] = |A n B| / |A u B| as
  * float32 (0 when both sets are empty).  A row that is null in either input is null in the result (its value
- * is unspecified); the result has a null mask only if an input has nulls.  Synchronises the stream once.
+ * is unspecified); the result has a null mask only if an input has nulls.  Waits for a number from the stream once
+ * (twice in a column of up to 32,768 pairs with some of more than 23 KB).
  * Limit: two rows of one pair may have 2^32 / 3 bytes together (1.43 GB); beyond that NVTEXT_AMD_OVERFLOW. */
 nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* input1,
                                            const nvtext_amd_strings_column* input2,
@@ -269,7 +270,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
  * removed (control and format characters; accents when lower-casing), replaced by a space (whitespace) or
  * replaced by its lower-cased, accent-stripped form of one to three code points.  special_tokens (NULL or
  * empty for none) are bracketed tokens such as "[PAD]" that keep their case and their brackets unpadded;
- * nulls among them give INVALID_ARGUMENT.  The tables (14.4 MB) come from `mr` on `stream` (NULL: hipMalloc)
+ * nulls among them give INVALID_ARGUMENT.  The tables (15.5 MB) come from `mr` on `stream` (NULL: hipMalloc)
  * and go back the same way in _destroy: the allocator's ctx and the stream must outlive the object.  Belongs to
  * the device that is current at creation; immutable and shareable between concurrent calls. */
 nvtext_amd_status nvtext_amd_character_normalizer_create(int32_t do_lower_case,
@@ -285,8 +286,9 @@ void nvtext_amd_character_normalizer_destroy(nvtext_amd_character_normalizer* no
  * cpp/src/text/normalize.cu:491-573): the BERT basic-tokenizer clean-up that precedes wordpiece_tokenize.
  * Works on the bytes between the first and the last offset of the view as one flat sequence, so a null row
  * keeps whatever its offsets span and the result has the input's validity.  Result: STRING column (int64
- * offsets when it holds INT32_MAX bytes or more).  Synchronises the stream twice (the byte range of the view,
- * the size of the result). */
+ * offsets when it holds INT32_MAX bytes or more).  Waits for numbers from the stream twice (the byte range of the
+ * view, the size of the result), in a small column once; the kernel that writes the result may still be at work when
+ * the call returns. */
 nvtext_amd_status nvtext_amd_normalize_characters(const nvtext_amd_strings_column* input,
                                                   const nvtext_amd_character_normalizer* normalizer,
                                                   void* stream,
