@@ -1,19 +1,17 @@
-// The minimum of the 64-bit permutations ((h * a + b) mod 2^64) mod p, p = 2^61 - 1, over many hashes h, with most of the
-// products computed to 17 bits by the matrix cores and only the few that can be the minimum computed exactly.
+// The minimum of the 64-bit permutations ((h * a + b) mod 2^64) mod p, p = 2^61 - 1, over many hashes h, with the products
+// computed to 16 bits by the matrix cores and only those of the few blocks of hashes that can hold the minimum computed exactly.
 //
 // What is minimised is, up to an addend of at most 7 (and the wrap from p to 0), the low 61 bits of h * a + b, that is the
 // fraction X = frac((h * a + b) / 2^61).  With the hash cut into 2-bit digits u_i (i = 0 .. 30) X is the fraction of
 //     b / 2^61 + sum over i of u_i * f_i,   f_i = frac(a * 4^i / 2^61),
 // a matrix product of the digits of 32 hashes with the fractions of 32 parameters.  The f_i are rounded to the nearest
-// multiple of 2^-17 (a unit) and cut into four pieces of 5, 5, 5 and 2 bits, which fp6 (e2m3) holds exactly, the digits are
+// multiple of 2^-16 (a unit) and cut into four pieces of 4, 5, 5 and 2 bits, which fp6 (e2m3) holds exactly, the digits are
 // 2-bit patterns that fp4 (e2m1) reads as u / 2; a K-block of 32 elements of v_mfma_scale_f32_32x32x64_f8f6f4 takes the 31
-// digits with one piece, whose weight is the block's scale.  Two instructions (64 cycles) give 1,024 sums of all four
+// digits with one piece, whose weight is the block's scale.  Two instructions give 1,024 sums of all four
 // pieces, exact in units: they start from 6.0, so that every sum lies in [4, 8), where an fp32 step is one unit, and the
-// fraction is the low 17 bits of the pattern.  Element 31 adds b and what the rounding may have taken away, so that the
-// fraction found is always 1 to `slack` units above X: a hash can only be the minimum if its fraction is at most the
-// least one found plus the slack.  (A sum that passes 1 comes out small: fractions below the slack are not trusted.)
-// Exact products in the vector ALUs take 8.5 instructions each; this takes 2.5 (39.5 for the 16 products a lane of 1,024,
-// and the two matrix instructions), and an exact product for one in some hundred.
+// fraction is the low 16 bits of the pattern: 16-bit minima take the sums as they are.  Element 31 adds b and what the
+// rounding may have taken away, so that the fraction found is always 1 to `slack` units above X, modulo 1: a product can
+// only be less than v if its fraction is at most that of v plus the slack.
 #pragma once
 
 #include "common.cuh"
@@ -25,12 +23,10 @@ using Sums = float __attribute__((ext_vector_type(16)));
 using V8   = int __attribute__((ext_vector_type(8)));
 
 constexpr int kGroup       = 32;             // parameters of one matrix instruction
-constexpr int kUnits       = 17;             // bits of a fraction
-constexpr int kUnitShift   = 61 - kUnits;    // a unit is 2^44 of a product
-constexpr int kKeyShift    = 32 - kUnits;    // fractions are compared at the top of a dword; what is below says whose it is
+constexpr int kUnits       = 16;             // bits of a fraction
+constexpr int kUnitShift   = 61 - kUnits;    // a unit is 2^45 of a product
 constexpr uint64_t kPrime  = (1ull << 61) - 1;
-constexpr uint32_t kNoKey  = 0xFFFFFFFFu;
-constexpr uint32_t kLargest = 0x4081FFFFu;   // a sum (between 4 and 8) with the largest fraction
+constexpr float kStart     = 6.0f;           // what the sums start from: its low 16 bits are zeros
 
 // What the host side of a call lays out for a group of 32 parameters: the registers of the two matrix instructions, lane
 // by lane, and the slack of every parameter.
@@ -51,7 +47,7 @@ constexpr int kScaleOne = 127;
 // A number of at most 16 in size as fp6 (e2m3), in eighths.
 __host__ __device__ inline uint32_t fp6_eighths(int v) { return v < 0 ? 32u | static_cast<uint32_t>(-v) : static_cast<uint32_t>(v); }
 
-// Piece j of n, |n| <= 2^16 units.
+// Piece j of n, |n| <= 2^15 units.
 __host__ __device__ inline int piece_of(int32_t n, int j)
 {
   int const d3 = ((n + 2) & 3) - 2;
@@ -104,9 +100,6 @@ __host__ __device__ inline uint64_t exact(uint64_t h, uint64_t a, uint64_t b)
   return y >= kPrime ? y - kPrime : y;
 }
 
-// The largest key of a fraction.
-__device__ __forceinline__ uint32_t key_ceiling(uint32_t key) { return key | ((1u << kKeyShift) - 1u); }
-
 // The digits of a hash as the matrix instruction reads them, element 31 set to 1.0 (which counts as a digit of 2).
 __device__ __forceinline__ V8 digits_of(uint64_t h)
 {
@@ -132,8 +125,20 @@ __device__ __forceinline__ Sums sums_of(V8 const& digits, const uint32_t (&p0)[6
   return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(digits, b1, s, kFp4, kFp6, 0, kScaleOne, 0, scale1);
 }
 
-// The hash (of 32) that sum r of a lane belongs to.
-__device__ __forceinline__ uint32_t hash_of_sum(uint32_t r, int lane) { return 8u * (r >> 2) + 4u * (static_cast<uint32_t>(lane) >> 5) + (r & 3u); }
+// The least fraction of a lane's sixteen sums, by two-way minima of 16 bits: they issue every two cycles (2.2 measured), a
+// three-way one takes 8.9, and packed in pairs they need what packs them.  (The compiler forms the three-way ones, so only the
+// first eight are its own: it also waits for the matrix cores there.)
+__device__ __forceinline__ uint32_t least_of(Sums const& s)
+{
+  uint32_t k[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) k[r] = __builtin_elementwise_min(static_cast<uint16_t>(__float_as_uint(s[2 * r])), static_cast<uint16_t>(__float_as_uint(s[2 * r + 1])));
+#pragma unroll
+  for (int d = 4; d >= 1; d >>= 1)
+#pragma unroll
+    for (int r = 0; r < d; ++r) asm("v_min_u16 %0, %1, %2" : "=v"(k[r]) : "v"(k[r]), "v"(k[r + d]));
+  return k[0];
+}
 
 // One wavefront lays a group out: lane l parameter l % 32.
 __device__ __forceinline__ void prepare_group(const uint64_t* a, const uint64_t* b, int32_t P, int32_t group, Group* to, int lane)

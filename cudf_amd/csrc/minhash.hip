@@ -10,8 +10,8 @@
 //   * it then switches to lanes <-> parameters.  32-bit hashes: every lane keeps K (a, b) pairs and
 //     K running minima in registers and streams the tile's hashes through LDS
 //     broadcast reads, so the inner loop is v_mad_u64_u32 + v_min only (MinimaAll).  64-bit hashes:
-//     the matrix cores find which products can be the minimum, and only those are computed
-//     (Minima64, filter64.cuh);
+//     the matrix cores find which few of them can give the minimum, and only their products are
+//     computed (Minima64, filter64.cuh);
 //   * a wavefront does a row alone, or a part of it: rows are cut into even parts of at most 4.2 KB
 //     (64-bit hashes: 6 KiB; of fewer bytes in a column too small to give every wavefront of the device
 //     several of that size), the parts of a row meet in the result with an atomic minimum, and the
@@ -27,6 +27,7 @@
 #include "murmur.cuh"
 #include "windows.cuh"
 
+#include <algorithm>
 #include <limits>
 #include <mutex>
 #include <type_traits>
@@ -284,217 +285,239 @@ struct MinimaAll {
   }
 };
 
-// 64-bit hashes: G groups of 32 parameters, each product to 17 bits by the matrix cores (see filter64.cuh), 32 hashes at a time.
-// A lane has a parameter of every group and half of the hashes.  Of the hashes that lie in LDS (`fold`) it finds the
-// least fraction, whose hash it is, and the second least: two matrix instructions, 16 shifts that put the fractions in
-// order with a number below them and 23 minima, medians and maxima for 1,024 products, without a branch.  Per row and
-// group it keeps the least fraction so far and its hash (`best`, `best_hash`: not computed exactly until it has to be)
-// and the largest fraction that can still belong to the minimum (`limit`).  A fraction that is less than the best by
-// more than the slack takes its place; of two within the slack of each other one is computed exactly, and so is one
-// below the slack, which may have come round from the top; where the second least is not above the limit either, all of
-// the lane's hashes are (one parameter in fifty of 256 hashes).
-template <int G>
+// 64-bit hashes: GROUPS groups of 32 parameters, AT_ONCE at a time, each product to 16 bits by the matrix cores (see filter64.cuh),
+// 32 hashes at a time.  A lane has a parameter of every group and half of the hashes.  The hashes gather in LDS until kFoldFrom
+// are there or the part ends; then, for every block of 32, the least of the lane's sixteen fractions is ranked, with the
+// number of its half block below it, among the least three so far.  When all blocks are through, a lane takes one of the
+// parameters of two groups, and the sixteen products of the half block that comes first are computed exactly; their minimum
+// says which fractions can belong to a smaller one: the half block that comes second is computed as well if it is one of those
+// (one parameter in nine of 1000 hashes), all hashes are if the third is.
+// What bounds it: 1,024 products take 150 to 165 cycles of a SIMD, 86 of them the two matrix instructions, beside which the
+// vector ALUs stand still but for some 20, 33 the sixteen-bit minima, 20 the ranking (with the shifts and three-way minima of
+// whole dwords that put every single product in order before: 160 beside the matrix instructions; 20,011 long rows, 128
+// parameters 3.73 -> 2.80 ms, 30,000 rows of 3000 bytes, 260 parameters 3.00 -> 2.06, 20,000 lists of 480 words, 256 parameters 627 -> 346 us).
+template <int GROUPS, int AT_ONCE>
 struct Minima64 {
   using T = uint64_t;
-  static constexpr int kParams    = G * filter64::kGroup;
+  static constexpr int kParams    = GROUPS * filter64::kGroup;
   static constexpr int kSlots     = kParams;
-  static constexpr int kSimdWaves = G <= 2 ? 4 : 3;  // (four with three groups and more: registers are spilled)
+  static constexpr int kSimdWaves = AT_ONCE <= 2 ? 4 : 3;  // (the registers of 127 to 157 numbers)
   struct Lds {
-    unsigned long long exact[kParams];  // the least value computed exactly, of every parameter
-    T hash[2 * kWave];                  // what is waiting to be computed exactly: the hash
-    uint8_t param[2 * kWave];           // and the parameter
+    alignas(16) T minima[kParams];
   };
-  uint32_t pieces[G][2][6];
-  uint32_t slack[G], limit[G], best[G];
-  T best_hash[G];
-  int scale[2];
-  uint32_t waiting;
   Params<T> params;
   int32_t base;  // first parameter of the chunk
   Lds* lds;
   int lane;
 
-  __device__ __forceinline__ Minima64(Lds* lds_, int lane_) : lds(lds_), lane(lane_)
-  {
-    scale[0] = filter64::scale_of(0, lane);
-    scale[1] = filter64::scale_of(1, lane);
-  }
+  __device__ __forceinline__ Minima64(Lds* lds_, int lane_) : lds(lds_), lane(lane_) {}
   __device__ __forceinline__ void load(Params<T> const& p, int32_t chunk)
   {
-    params             = p;
-    base               = chunk * kParams;
-    int32_t const last = (p.count - 1) / filter64::kGroup;
+    params = p;
+    base   = chunk * kParams;
+  }
+  __device__ __forceinline__ void reset()
+  {
+    for (int j = lane; j < kParams; j += kWave) lds->minima[j] = std::numeric_limits<T>::max();
+  }
+
+  // The least product of the sixteen hashes of a half block.
+  static __device__ __forceinline__ T exact(const T* hashes, uint32_t half_block, T a, T b)
+  {
+    // (hashes 4 .. 7, 12 .. 15, .. of a block for the upper half)
+    const ulonglong2* const from = reinterpret_cast<const ulonglong2*>(hashes + (half_block >> 1) * 32u + (half_block & 1u) * 4u);
+    T m          = std::numeric_limits<T>::max();
+    uint32_t top = 0, one;
+    asm("s_mov_b32 %0, 1" : "=s"(one));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      ulonglong2 const h = from[(i >> 1) * 4 + (i & 1)];
+      T y0, y1;
+      fold_pair(h.x, h.y, a, b, one, &y0, &y1);
+      top = max(max(top, static_cast<uint32_t>(y0 >> 32)), static_cast<uint32_t>(y1 >> 32));
+      m   = min_below_2_62(min_below_2_62(m, y0), y1);
+    }
+    // (see fold_all: p and what is above it ought to have been reduced)
+    if (ballot64(top >= 0x1FFFFFFFu) != 0) {
+#pragma unroll 1
+      for (int i = 0; i < 8; ++i) {
+        ulonglong2 const h = from[(i >> 1) * 4 + (i & 1)];
+        m = min(min(m, filter64::exact(h.x, a, b)), filter64::exact(h.y, a, b));
+      }
+    }
+    return m;
+  }
+
+  // What no fraction of a product less than v exceeds.
+  static __device__ __forceinline__ uint32_t limit_of(T v, uint32_t slack)
+  {
+    return static_cast<uint32_t>(min((v >> filter64::kUnitShift) + slack, static_cast<T>(0xFFFFu)));
+  }
+
+  struct Ranked {
+    uint32_t first, second, third;
+    // (what comes before stays in order: the old ones are read before they are written)
+    __device__ __forceinline__ void add(uint32_t key)
+    {
+      third  = median(second, third, key);
+      second = median(first, second, key);
+      first  = min(first, key);
+    }
+    // The first three of both halves of the wavefront.
+    __device__ __forceinline__ void merge_halves()
+    {
+      auto const f = __builtin_amdgcn_permlane32_swap(first, first, false, false);
+      auto const s = __builtin_amdgcn_permlane32_swap(second, second, false, false);
+      auto const t = __builtin_amdgcn_permlane32_swap(third, third, false, false);
+      first  = min(f[0], f[1]);
+      second = min(min(max(f[0], f[1]), s[0]), s[1]);
+      third  = min(min(t[0], t[1]), min(max(f[0], s[1]), max(f[1], s[0])));
+    }
+  };
+
+  // The parameters of two groups, a lane each (index j of the chunk; a single group: both halves have the same).
+  __device__ __forceinline__ void settle(Ranked const& of_lower, Ranked const& of_upper, int j, const T* hashes, uint32_t count)
+  {
+    bool const upper = lane >= filter64::kGroup;
+    Ranked const r{upper ? of_upper.first : of_lower.first, upper ? of_upper.second : of_lower.second, upper ? of_upper.third : of_lower.third};
+    int32_t const at     = min(base + j, params.count - 1);
+    T const a = params.a[at], b = params.b[at];
+    uint32_t const slack = params.groups[at / filter64::kGroup].slack[at % filter64::kGroup];
+    T m                  = min(lds->minima[j], exact(hashes, r.first & 0xFFFFu, a, b));
+    uint64_t todo        = ballot64(r.second >> 16 <= limit_of(m, slack));
+    if (todo != 0) {
+      // few parameters (one in six of 1000 hashes): the products of four of them at a time, sixteen lanes each
+      lds->minima[j] = m;
+      wave_lds_fence();
+      do {
+        int who[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          who[i] = todo != 0 ? static_cast<int>(__builtin_ctzll(todo)) : who[i == 0 ? 0 : i - 1];
+          todo &= todo - 1;
+        }
+        int const of          = lane < 32 ? (lane < 16 ? who[0] : who[1]) : (lane < 48 ? who[2] : who[3]);
+        T const wa            = __shfl(static_cast<unsigned long long>(a), of), wb = __shfl(static_cast<unsigned long long>(b), of);
+        uint32_t const half   = __shfl(r.second, of) & 0xFFFFu;
+        uint32_t const within = static_cast<uint32_t>(lane) & 15u;
+        T const v             = filter64::exact(hashes[(half >> 1) * 32u + (half & 1u) * 4u + (within >> 2) * 8u + (within & 3u)], wa, wb);
+        unsigned long long* const to = reinterpret_cast<unsigned long long*>(&lds->minima[__shfl(j, of)]);
+        if (v < *to) atomicMin(to, static_cast<unsigned long long>(v));
+      } while (todo != 0);
+      wave_lds_fence();
+      m = lds->minima[j];
+      for (todo = ballot64(r.third >> 16 <= limit_of(m, slack)); todo != 0; todo &= todo - 1) {
+        int const who = static_cast<int>(__builtin_ctzll(todo));
+        T const wa = wave_bcast64(a, who), wb = wave_bcast64(b, who);
+        T v = std::numeric_limits<T>::max();
+        for (uint32_t i = lane; i < count; i += kWave) v = min(v, filter64::exact(hashes[i], wa, wb));
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) v = min(v, static_cast<T>(__shfl_xor(static_cast<unsigned long long>(v), d)));
+        if (lane == who) m = min(m, v);
+      }
+    }
+    lds->minima[j] = m;
+  }
+
+  template <int G>
+  __device__ __forceinline__ void fold_groups(int32_t first, const T* hashes, uint32_t count)
+  {
+    asm("" : "+s"(first));  // (the pieces are read anew for every fold: not kept in registers while windows are hashed)
+    int32_t const last = (params.count - 1) / filter64::kGroup;
+    uint32_t pieces[G][2][6];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      filter64::Group const& from = p.groups[min(chunk * G + g, last)];
+      filter64::Group const& from = params.groups[min(base / filter64::kGroup + first + g, last)];
 #pragma unroll
       for (int k = 0; k < 2; ++k)
 #pragma unroll
         for (int d = 0; d < 6; ++d) pieces[g][k][d] = from.pieces[k][d][lane];
-      slack[g] = from.slack[lane % filter64::kGroup] << filter64::kKeyShift;
     }
-  }
-  __device__ __forceinline__ void reset()
-  {
-    waiting = 0;
+    filter64::Sums start;
 #pragma unroll
-    for (int g = 0; g < G; ++g) limit[g] = best[g] = filter64::kNoKey;
-    for (int j = lane; j < kParams; j += kWave) lds->exact[j] = ~0ull;
-  }
-
-  __device__ __forceinline__ void compute(int at, T h)
-  {
-    int32_t const j            = min(base + at, params.count - 1);
-    unsigned long long const v = filter64::exact(h, params.a[j], params.b[j]);
-    if (v < lds->exact[at]) atomicMin(&lds->exact[at], v);
-  }
-  // Computes the first 64 of those waiting, or all of them.
-  __device__ __forceinline__ void compute_waiting()
-  {
-    wave_lds_fence();
-    if (static_cast<uint32_t>(lane) < waiting) compute(lds->param[lane], lds->hash[lane]);
-    if (waiting > kWave) {
-      T const h       = lds->hash[kWave + lane];
-      uint8_t const j = lds->param[kWave + lane];
-      wave_lds_fence();
-      lds->hash[lane]  = h;
-      lds->param[lane] = j;
-      waiting -= kWave;
-    } else {
-      waiting = 0;
+    for (int r = 0; r < 16; ++r) start[r] = filter64::kStart;
+    asm("" : "+v"(start));  // (one set of registers, not one filled anew for every block)
+    int const scale[2] = {filter64::scale_of(0, lane), filter64::scale_of(1, lane)};
+    Ranked ranked[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) ranked[g] = Ranked{kNoKey, kNoKey, kNoKey};
+    uint32_t half_block = static_cast<uint32_t>(lane) >> 5;
+    for (uint32_t i = 0; i < count; i += 32u, half_block += 2u) {
+      filter64::V8 const digits = filter64::digits_of(hashes[i + static_cast<uint32_t>(lane % 32)]);
+#pragma unroll
+      for (int g = 0; g < G; ++g) ranked[g].add(filter64::least_of(filter64::sums_of(digits, pieces[g][0], pieces[g][1], scale[0], scale[1], start)) << 16 | half_block);
     }
-  }
-  __device__ __forceinline__ void wait(bool yes, int g, T h)
-  {
-    uint64_t const who = ballot64(yes);
-    if (who == 0) return;
-    if (yes) {
-      uint32_t const at = waiting + lanes_below(who);
-      lds->hash[at]     = h;
-      lds->param[at]    = static_cast<uint8_t>(g * filter64::kGroup + lane % filter64::kGroup);
-    }
-    waiting += static_cast<uint32_t>(__builtin_popcountll(who));
-    if (waiting >= kWave) compute_waiting();
-  }
-
-  // The least and the second least key of a group's products with the hashes: what becomes of them.
-  __device__ __forceinline__ void settle(int g, uint32_t least, uint32_t second, const T* hashes, uint32_t count)
-  {
-    bool const certain = least >= slack[g];
-    if (certain) limit[g] = min(limit[g], add_saturating(filter64::key_ceiling(least), slack[g]));
-    limit[g]      = min_of_halves(limit[g]);
-    bool const in = least <= limit[g];
-    if (ballot64(in) == 0) return;
-    T const h         = hashes[(least >> 4 & 0x7FFu) * 32u + filter64::hash_of_sum(least & 15u, lane)];
-    bool const better = certain && least < best[g];
-    bool const near   = best[g] != filter64::kNoKey && add_saturating(least, slack[g]) >= best[g] && h != best_hash[g];
-    wait(in && (!certain || near), g, certain && better ? best_hash[g] : h);
-    if (in && better) {
-      best[g]      = least;
-      best_hash[g] = h;
-    }
-    for (uint64_t todo = ballot64(second <= limit[g]); todo != 0; todo &= todo - 1) {
-      int const who    = static_cast<int>(__builtin_ctzll(todo));
-      uint32_t const n = (count + 31u) / 32u * 16u;  // hashes that the lane has
-      int at           = g * filter64::kGroup + who % filter64::kGroup;
-      asm("" : "+v"(at));  // (an address that the compiler knows to be the same in every lane: it builds a loop over the lanes)
-      for (uint32_t i = lane; i < n; i += kWave) compute(at, hashes[(i >> 4) * 32u + filter64::hash_of_sum(i & 15u, who)]);
+#pragma unroll
+    for (int g = 0; g < G; ++g) ranked[g].merge_halves();
+#pragma unroll
+    for (int g = 0; g < G; g += 2) {
+      bool const two = g + 1 < G;
+      settle(ranked[g], ranked[two ? g + 1 : g], (first + g) * filter64::kGroup + (two ? lane : lane % filter64::kGroup), hashes, count);
     }
   }
 
-  // hashes: `count` of them (at most 2^11 blocks of 32), and room up to the next multiple of 32.  Whole blocks are done,
-  // the last time the rest as well: a block that is filled up costs what a whole one does and 50 instructions more (131,071
-  // rows of 3000 bytes, 128 parameters: a rest after every 256 windows 5633 us, one a part 5403).
+  // hashes: `count` of them, and room up to the next multiple of 32.  They are left to gather until kFoldFrom are there.
   __device__ __forceinline__ uint32_t fold(T* hashes, uint32_t count, bool last)
   {
+    if (count < kFoldFrom && !last) return count;
+    if (count == 0) return 0;
     wave_lds_fence();
-    uint32_t const later = last ? 0u : count & 31u;
-    count -= later;
-    if (count == 0) return later;
-    // The last block is filled up with hashes of the row, and their sums are set to the largest fraction: their digits are
-    // zeros, so that the sum is what it starts from.  (Left as they come out, a least fraction that the filling repeats is
-    // the second least of its lane as well, and all of the lane's hashes are computed exactly: one parameter in seven of a
-    // row of 56 windows.  200,000 lists of 30 elements, 128 parameters: 2282 -> 557 us; 1,000,003 rows of 512 bytes, 64
-    // parameters: 7251 -> 6818 us.)
+    // (a hash that is there twice does not change a minimum)
     uint32_t const rest = (0u - count) & 31u;
     if (static_cast<uint32_t>(lane) < rest) hashes[count + lane] = hashes[0];
     wave_lds_fence();
-    filter64::Sums start;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) start[r] = 6.0f;
-    asm("" : "+v"(start));  // (one set of registers, not one filled anew for every block)
-    uint32_t least[G], second[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) least[g] = second[g] = filter64::kNoKey;
-    for (uint32_t block = 0; block < count; block += 32u) {
-      filter64::V8 digits = filter64::digits_of(hashes[block + static_cast<uint32_t>(lane % 32)]);
-      if (count - block < 32u) {
-        int const left      = static_cast<int>(count - block);
-        int const mine      = lane % 32 < left ? -1 : 0;
-        int const left_here = left - static_cast<int>(filter64::hash_of_sum(0, lane));  // (compared with numbers that are the same in every lane)
-#pragma unroll
-        for (int d = 0; d < 4; ++d) digits[d] &= mine;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) start[r] = static_cast<int>(filter64::hash_of_sum(r, 0)) < left_here ? start[r] : __uint_as_float(filter64::kLargest);
-      }
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        filter64::Sums const sums = filter64::sums_of(digits, pieces[g][0], pieces[g][1], scale[0], scale[1], start);
-        uint32_t key[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) key[r] = (__float_as_uint(sums[r]) << filter64::kKeyShift) | static_cast<uint32_t>(r);
-        uint32_t one = min(key[0], key[1]), two = max(key[0], key[1]);
-#pragma unroll
-        for (int r = 2; r < 16; r += 2) {
-          two = min(two, median(one, key[r], key[r + 1]));
-          one = min(min(one, key[r]), key[r + 1]);
-        }
-        one |= block >> 1;  // (16 times the number of the block)
-        second[g] = min(min(second[g], two), max(least[g], one));
-        least[g]  = min(least[g], one);
-      }
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g) settle(g, least[g], second[g], hashes, count);
-    if (later > 0) {
-      T const h = hashes[count + static_cast<uint32_t>(lane % 32)];
-      wave_lds_fence();
-      if (static_cast<uint32_t>(lane) < later) hashes[lane] = h;
-    }
+#pragma unroll 1
+    for (int g = 0; g + AT_ONCE <= GROUPS; g += AT_ONCE) fold_groups<AT_ONCE>(g, hashes, count + rest);
+    if constexpr (GROUPS % AT_ONCE != 0) fold_groups<GROUPS % AT_ONCE>(GROUPS / AT_ONCE * AT_ONCE, hashes, count + rest);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    return later;
+    return 0;
   }
-  __device__ __forceinline__ void finish()
-  {
-#pragma unroll
-    for (int g = 0; g < G; ++g) wait(best[g] <= limit[g] && best[g] != filter64::kNoKey, g, best_hash[g]);
-    if (waiting > 0) compute_waiting();
-    wave_lds_fence();
-  }
+  __device__ __forceinline__ void finish() { wave_lds_fence(); }
   template <typename Put>
   __device__ __forceinline__ void each(Put const& put) const
   {
-    for (int j = lane; j < kParams; j += kWave) put(j, static_cast<T>(lds->exact[j]));
+    for (int j = lane; j < kParams; j += kWave) put(j, lds->minima[j]);
     __builtin_amdgcn_wave_barrier();
   }
+  static constexpr uint32_t kNoKey = 0xFFFFFFFFu;
 };
 
-// Whether the wavefront has met this hash lately (it is noted either way).  Called by the lanes that have a hash.
-template <typename T>
-__device__ __forceinline__ bool seen_lately(WaveLds<T>& lds, T hv)
+// Puts the fresh ones of a trip's hashes (a lane with `valid` has one) behind the `count` that wait in lds.hashes: those that
+// the wavefront has not met lately.
+__device__ __forceinline__ void gather(WaveLds<uint32_t>& lds, bool valid, uint32_t hv, uint32_t* count)
 {
-  T* const at  = &lds.recent[static_cast<uint32_t>(hv) & (recent_entries<T>() - 1)];
-  T const was  = *at;
-  *at          = hv;
-  return was == hv;
+  bool fresh = false;
+  if (valid) {
+    uint32_t* const at = &lds.recent[hv & (kRecentEntries - 1)];
+    fresh              = *at != hv;
+    *at                = hv;
+  }
+  uint64_t const vm = ballot64(fresh);
+  if (fresh) lds.hashes[*count + lanes_below(vm)] = hv;
+  *count += static_cast<uint32_t>(__builtin_popcountll(vm));
+}
+// 64-bit hashes: the table says where among the hashes that were gathered (and perhaps folded since, in the same part) it may be
+__device__ __forceinline__ void gather(WaveLds<uint64_t>& lds, bool valid, uint64_t hv, uint32_t* count)
+{
+  uint16_t* const at = &lds.recent[static_cast<uint32_t>(hv) & (kRecentEntries - 1)];
+  bool const fresh   = valid && lds.hashes[*at] != hv;
+  uint64_t const vm  = ballot64(fresh);
+  if (fresh) {
+    uint32_t const place = *count + lanes_below(vm);
+    lds.hashes[place]    = hv;
+    *at                  = static_cast<uint16_t>(place);
+  }
+  *count += static_cast<uint32_t>(__builtin_popcountll(vm));
 }
 template <typename T>
 __device__ __forceinline__ void forget_hashes(WaveLds<T>& lds, int lane)
 {
-  constexpr int kEach = 16 / sizeof(T);
+  // (0 is no hash; a place of 64-bit hashes is the one behind all others, which holds 0)
+  uint32_t const none = sizeof(T) == 4 ? 0u : kNoPlace * 0x10001u;
+  if (sizeof(T) == 8 && lane == 0) lds.hashes[kNoPlace] = 0;
 #pragma unroll
-  for (int i = 0; i < recent_entries<T>() / kEach; i += kWave) reinterpret_cast<uint4*>(lds.recent)[i + lane] = make_uint4(0u, 0u, 0u, 0u);
+  for (int i = 0; i < static_cast<int>(sizeof(lds.recent) / 16); i += kWave) reinterpret_cast<uint4*>(lds.recent)[i + lane] = make_uint4(none, none, none, none);
 }
 
 // What is hashed: a column of strings, by windows of characters, or a column of lists of strings, by runs of elements.  A
@@ -506,6 +529,9 @@ struct TextRows {
   using Lds = WaveLds<T>;
   static constexpr const char* kName = "minhash_parts_kernel";
   static constexpr bool kShortRows   = false;  // no more is known of their lengths than the kernels read
+  // groups of 64-bit parameters at a time where there are six and more, whose minima leave LDS for three workgroups only: four
+  // (30,000 rows of 3000 bytes, 200 parameters: two 1709 us, three 1780, four 1631)
+  static constexpr int kManyGroups   = 4;
   static constexpr int kSimdWaves   = sizeof(T) == 4 ? 6 : 4;  // wavefronts per SIMD that its LDS leaves room for
   // (parts of up to one and a half of it.  The end of the kernel is uneven by one of them; what a part costs beside its
   // length is little with 32-bit hashes, for which 4096 is no faster, and a twentieth with 64-bit ones: 60,000 rows of
@@ -529,30 +555,23 @@ struct TextRows {
     int64_t const o      = col.off(i);
     int64_t const n      = col.off(i + 1) - o;
     const uint8_t* const row = col.chars + o;
-    if (static_cast<int64_t>(width) * 4 <= kHalo) {
-      // usual case: a window (<= 4*width bytes) fits the halo staged behind every tile
-      forget_hashes(lds, lane);  // (the wave barrier after the first tile's staging comes before the first look)
-      uint32_t count = 0;  // hashes that wait to be folded (wave-uniform)
-      for (int64_t base = begin; base < end; base += kTile) {
+    // usual case: a window (<= 4*width bytes) fits the halo staged behind every tile
+    bool const narrow  = static_cast<int64_t>(width) * 4 <= kHalo;
+    int64_t const step = narrow ? kTile : kWave;
+    forget_hashes(lds, lane);  // (the wave barrier after the first tile's staging comes before the first look)
+    uint32_t count = 0;  // hashes that wait to be folded (wave-uniform)
+    for (int64_t base = begin; base < end; base += step) {
+      if (narrow) {
         uint32_t const cnt = static_cast<uint32_t>(min(static_cast<int64_t>(kTile), end - base));
         auto const hash    = [seed = seed](WordSrc const& src, uint32_t len) {
           T const hv = H::hash(src, len, seed);
           return hv < 1 ? T{1} : hv;  // minhash.cu:141
         };
         hash_tile_windows<T>(row, n, base, cnt, width, lds.bytes, lds.chars, lane, hash, [&](auto const& valid, auto const& hv) {
-          for (auto const& h : hv) {
-            bool const fresh  = valid[&h - hv] && !seen_lately(lds, h);
-            uint64_t const vm = ballot64(fresh);
-            if (fresh) lds.hashes[count + lanes_below(vm)] = h;
-            count += static_cast<uint32_t>(__builtin_popcountll(vm));
-          }
+          for (auto const& h : hv) gather(lds, valid[&h - hv], h, &count);
         });
-        count = minima.fold(lds.hashes, count, base + kTile >= end);
-      }
-    } else {
-      // very wide windows: 64 starts at a time, bytes read straight from global memory
-      uint32_t count = 0;
-      for (int64_t base = begin; base < end; base += kWave) {
+      } else {
+        // very wide windows: 64 starts at a time, bytes read straight from global memory
         int64_t const gpos = base + lane;
         bool valid         = false;
         T hv               = 0;
@@ -569,8 +588,9 @@ struct TextRows {
         }
         uint64_t const vm = ballot64(valid);
         if (valid) lds.hashes[count + lanes_below(vm)] = hv;
-        count = minima.fold(lds.hashes, count + static_cast<uint32_t>(__builtin_popcountll(vm)), base + kWave >= end);
+        count += static_cast<uint32_t>(__builtin_popcountll(vm));
       }
+      count = minima.fold(lds.hashes, count, base + step >= end);
     }
   }
 };
@@ -616,11 +636,12 @@ struct AlignedSrc {
 
 constexpr uint32_t kRunStageBytes = 4096;                           // longest stretch of chars hashed out of LDS
 constexpr uint32_t kRunStageWords = (kRunStageBytes + 16 + 32) / 4;  // + misalignment, + whole blocks and over-read of the hash tail
-constexpr uint32_t kRunHashes     = 256;                            // hashes folded together
+template <typename T>
+constexpr uint32_t run_hashes() { return sizeof(T) == 4 ? 256 : 512; }  // hashes folded together
 
 template <typename T>
 struct RunLds {
-  alignas(16) T hashes[kRunHashes + kWave];  // (padded to the stride of the fold, at most 63 more)
+  alignas(16) T hashes[run_hashes<T>() + kWave];  // (padded to the stride of the fold, at most 63 more)
   // the chars of the elements a wavefront is hashing (32-bit hash only: measured 13 % faster there, 9 % slower for the
   // 64-bit hash, whose 16-byte steps cost more to assemble out of LDS than they save)
   alignas(16) uint32_t bytes[sizeof(T) == 4 ? kRunStageWords : 4];
@@ -633,6 +654,7 @@ struct RunRows {
   using Lds = RunLds<T>;
   static constexpr const char* kName = "minhash_ngrams_parts_kernel";
   static constexpr bool kShortRows   = true;
+  static constexpr int kManyGroups   = 2;  // (four wavefronts: 20,000 lists of 480, 256 parameters 363 us, with three and four groups 405)
   static constexpr int kSimdWaves   = sizeof(T) == 4 ? 7 : 5;
   static constexpr int64_t kPart    = 704;
   static constexpr int64_t kMinPart = kWave;
@@ -693,7 +715,7 @@ struct RunRows {
       uint64_t const vm = ballot64(valid);
       if (valid) lds.hashes[count + lanes_below(vm)] = hv;
       count += static_cast<uint32_t>(__builtin_popcountll(vm));
-      if (count > kRunHashes - kWave) {  // (whole blocks but where elements are null)
+      if (count > run_hashes<T>() - kWave) {  // (whole blocks but where elements are null)
         minima.fold(lds.hashes, count, true);
         count = 0;
       }
@@ -768,7 +790,12 @@ struct RowParts {
 
 // Wavefronts per SIMD that the kernels are compiled for.
 template <typename Source, typename Minima>
-constexpr int simd_waves() { return Source::kSimdWaves < Minima::kSimdWaves ? Source::kSimdWaves : Minima::kSimdWaves; }
+constexpr int simd_waves()
+{
+  // (as many workgroups to a CU; LDS is given out in pieces of 1280 bytes)
+  constexpr int kPiece = 1280, kPieces = (kWaves * static_cast<int>(sizeof(typename Source::Lds) + sizeof(typename Minima::Lds)) + kPiece - 1) / kPiece;
+  return std::min({Source::kSimdWaves, Minima::kSimdWaves, 160 * 1024 / kPiece / kPieces});
+}
 
 // The row r that part t is one of, prefix[r] <= t < prefix[r + 1], is one of 64 rows from the returned one on, of which
 // *near is prefix (rows + 1 of them), a lane a row; not the last.  Looked for first where rows of equal numbers of parts
@@ -1068,6 +1095,9 @@ void with_all_products(int32_t P, Launch const& launch)
     default: launch(Which<MinimaAll<T, 1, false>>{}, chunks); break;
   }
 }
+// Up to nine groups of 32 parameters in one chunk (every chunk hashes the windows again), beyond that chunks of equal size of
+// at most eight.
+constexpr int32_t chunks_of(int groups) { return groups <= 9 ? 1 : (groups + 7) / 8; }
 template <typename Source, typename Launch>
 void with_minima(int32_t P, bool short_rows, Launch const& launch)
 {
@@ -1078,32 +1108,38 @@ void with_minima(int32_t P, bool short_rows, Launch const& launch)
     if constexpr (Source::kShortRows) {
       if (short_rows) return with_all_products<T>(P, launch);
     }
-    // as few chunks as four groups each allow (every chunk hashes the windows again), of equal size
     int const groups     = groups_of(P);
-    int32_t const chunks = (groups + 3) / 4;
+    int32_t const chunks = chunks_of(groups);
     switch ((groups + chunks - 1) / chunks) {
-      case 1: launch(Which<Minima64<1>>{}, chunks); break;
-      case 2: launch(Which<Minima64<2>>{}, chunks); break;
-      case 3: launch(Which<Minima64<3>>{}, chunks); break;
-      default: launch(Which<Minima64<4>>{}, chunks); break;
+      case 1: launch(Which<Minima64<1, 1>>{}, chunks); break;
+      case 2: launch(Which<Minima64<2, 2>>{}, chunks); break;
+      case 3: launch(Which<Minima64<3, 2>>{}, chunks); break;
+      case 4: launch(Which<Minima64<4, 2>>{}, chunks); break;
+      case 5: launch(Which<Minima64<5, 2>>{}, chunks); break;
+      case 6: launch(Which<Minima64<6, Source::kManyGroups>>{}, chunks); break;
+      case 7: launch(Which<Minima64<7, Source::kManyGroups>>{}, chunks); break;
+      case 8: launch(Which<Minima64<8, Source::kManyGroups>>{}, chunks); break;
+      default: launch(Which<Minima64<9, Source::kManyGroups>>{}, chunks); break;
     }
   }
 }
 
-// Rows of 64-bit hashes shorter than this on average have all their products computed whole.  The matrix cores spare the
-// time of 7 vector instructions a product and wavefront (2.5 of them instead of 8.5, most of which are multiplications and
-// take longer) and cost some 800 for every 64 parameters of a row, for what has to be
-// computed exactly at its end; and as their registers take 128 parameters at most, not 320, more chunks, each of which
-// hashes the row again (20 instructions a position: runs of words come from memory).  Lists of 60 elements, 131,072 rows,
-// 128 parameters: whole 367 us, matrix cores 426; of 130: 799 and 824; of 200: 1150 and 1076; 20,000 of 200, 256
-// parameters: 306 and 319, of 800: 1152 and 986; 30,000 of 1200, 260 parameters: 2483 and 3187.
+// Rows of 64-bit hashes shorter than this on average have all their products computed whole.  In units of what a hash and 64
+// parameters cost whole: hash and 32 parameters on the matrix cores 0.225, a chunk of parameters that hashes the row again
+// 0.5 an element, a pair of groups 36 a row for what is computed exactly at its end; and where the lanes share out few
+// parameters, the hashes of a row are filled up to a whole stride.  131,072 lists of 60 elements (fewer of longer ones, 3 to 6 M
+// elements in all), us whole and on the matrix cores: 26 parameters, 60: 181 and 213, 130: 157 and 168, 250: 147 and 150; 64
+// parameters, 60: 213 and 228, 130: 194 and 177; 128 parameters, 30: 227 and 328, 60: 286 and 298, 130: 278 and 218, 250: 272 and
+// 183; 256 parameters, 60: 239 and 236, 130: 240 and 165; 260 parameters, 15: 607 and 691, 30: 499 and 471, 60: 339 and 286.
 inline double short_row_length(int32_t P)
 {
   Sharing const sh     = sharing_for(P);
   int32_t const chunks = sh.tail ? 1 : (P + sh.k * kWave - 1) / (sh.k * kWave);
-  double const sets    = sh.tail ? sh.k + packing_for(P - sh.k * kWave).ppad / 64.0 : static_cast<double>(chunks * sh.k);
-  double const spared  = 7.0 * sets - 20.0 * ((groups_of(P) + 3) / 4 - chunks);
-  return spared > 0.0 ? 800.0 * sets / spared : std::numeric_limits<double>::max();
+  Packing const few    = packing_for(sh.tail ? P - sh.k * kWave : P);
+  double const sets    = sh.tail || P <= 32 ? (sh.tail ? sh.k : 0) + few.ppad / 64.0 : static_cast<double>(chunks * sh.k);
+  int const groups     = groups_of(P);
+  double const spared  = sets - 0.225 * groups - 0.5 * (chunks_of(groups) - chunks);
+  return spared > 0.0 ? 36.0 * ((groups + 1) / 2) / spared - few.groups * static_cast<double>(kFoldTrip) : std::numeric_limits<double>::max();
 }
 
 // The launches of one minhash call: the places of the rows in the result and their parts, then the hashing kernel.

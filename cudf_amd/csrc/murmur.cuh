@@ -110,53 +110,42 @@ __device__ __forceinline__ uint64_t load_u64(Src const& src, uint32_t i)
   return (static_cast<uint64_t>(src.u32(i + 4)) << 32) | src.u32(i);
 }
 
-// The first n bytes (1 .. 8) of v.
-__device__ __forceinline__ uint64_t low_bytes64(uint64_t v, uint32_t n)
-{
-  uint32_t const s = 64u - 8u * n;
-  return (v << s) >> s;
-}
+// The first n bytes (0 .. 8) of v.
+__device__ __forceinline__ uint64_t low_bytes64(uint64_t v, uint32_t n) { return n == 0 ? 0 : v & (~0ull >> (64u - 8u * n)); }
 
-// First 64-bit word of MurmurHash3_x64_128 with h1 = h2 = seed over window bytes [0, len).
+// First 64-bit word of MurmurHash3_x64_128 with h1 = h2 = seed over window bytes [0, len).  What is left of the key after
+// its blocks of 16 is treated as a block is up to where the halves are mixed: zeros in place of missing bytes change nothing,
+// and lanes with keys either side of 16 bytes go one way (before, the ones waited while the others did their blocks).
 template <typename Src>
 __device__ __forceinline__ uint64_t murmur3_x64_128_lo(Src const& src, uint32_t len, uint64_t seed)
 {
   uint64_t const c1 = 0x87c37b91114253d5ull, c2 = 0x4cf5ad432745937full;
   uint64_t h1 = seed, h2 = seed;
-  uint32_t const blocks = len >> 4;
-  for (uint32_t i = 0; i < blocks; ++i) {
-    uint64_t k1 = load_u64(src, 16 * i);
-    uint64_t k2 = load_u64(src, 16 * i + 8);
+  for (uint32_t t = 0; t < len; t += 16) {
+    uint32_t const left = len - t;
+    uint64_t k1 = low_bytes64(load_u64(src, t), min(left, 8u));
     k1 *= c1;
     k1 = rotl64(k1, 31);
     k1 *= c2;
     h1 ^= k1;
-    h1 = rotl64(h1, 27);
-    h1 += h2;
-    h1 = h1 * 5 + 0x52dce729;
-    k2 *= c2;
-    k2 = rotl64(k2, 33);
-    k2 *= c1;
-    h2 ^= k2;
-    h2 = rotl64(h2, 31);
-    h2 += h1;
-    h2 = h2 * 5 + 0x38495ab5;
-  }
-  uint32_t const rem = len & 15u;
-  if (rem) {
-    uint32_t const t = 16 * blocks;
-    if (rem > 8) {
-      uint64_t k2 = low_bytes64(load_u64(src, t + 8), rem - 8);
+    uint64_t k2 = 0;
+    if (left > 8) {
+      k2 = low_bytes64(load_u64(src, t + 8), min(left, 16u) - 8u);
       k2 *= c2;
       k2 = rotl64(k2, 33);
       k2 *= c1;
+    }
+    if (left >= 16) {
+      h1 = rotl64(h1, 27);
+      h1 += h2;
+      h1 = h1 * 5 + 0x52dce729;
+      h2 ^= k2;
+      h2 = rotl64(h2, 31);
+      h2 += h1;
+      h2 = h2 * 5 + 0x38495ab5;
+    } else {
       h2 ^= k2;
     }
-    uint64_t k1 = low_bytes64(load_u64(src, t), rem < 8 ? rem : 8u);
-    k1 *= c1;
-    k1 = rotl64(k1, 31);
-    k1 *= c2;
-    h1 ^= k1;
   }
   h1 ^= len;
   h2 ^= len;

@@ -7,6 +7,8 @@
 #include "common.cuh"
 #include "murmur.cuh"
 
+#include <type_traits>
+
 namespace nvtext_amd {
 
 constexpr int kWaves     = 4;                  // wavefronts per workgroup
@@ -16,20 +18,25 @@ constexpr int kHalo      = 128;                // bytes staged past the tile (wi
 constexpr int kCharList  = kTile + kHalo + 8;   // list of a tile's characters: one per staged byte, the end of the last one, padding
 constexpr int kTileWords = (kTile + kHalo + 16 + 32) / 4;  // +16 misalignment, +32 for whole blocks and the over-read of the hash tail
 
+// 64-bit hashes: so many are gathered before they meet the parameters, which costs as much for few as for many where it ends
+// (the exact products).  What leaves four workgroups to a CU with up to 160 parameters: 20,011 long rows, 128 parameters:
+// 352: 2860 us, 416: 2802; with more, three: 448 of them and a wavefront less are 5 to 12 % slower where 416 would do.
+constexpr uint32_t kFoldFrom = 416;
+
 // Windows repeat (of 2 KB of ordinary text three in four are different, of 16 KB little more than half), and a hash that
 // has been folded once changes no minimum when it is folded again.  Every wavefront keeps the hashes it saw last in a
-// small direct-mapped table and drops a hash that it finds there; what the table has forgotten is folded again, which
+// small direct-mapped table (of 64-bit hashes, the places that they have among those gathered: 2 KB for 1024 where 512
+// hashes took 4) and drops a hash that it finds there; what the table has forgotten is folded again, which
 // costs time and nothing else.  Cleared (hashes are never 0) whenever the wavefront begins a row.  As many entries as leave
-// six (64-bit hashes: four) workgroups to a CU: 400,000 documents of 2 KB, 256 parameters: 256 entries 8.80 ms, 512: 8.45,
-// 1024: 8.17; 64-bit hashes of 20,011 long rows: 256: 4.13 ms, 512: 4.05, 1024: 4.85 (three workgroups).
-template <typename T>
-constexpr int recent_entries() { return sizeof(T) == 4 ? 1024 : 512; }
-
+// six (64-bit hashes: four) workgroups to a CU: 400,000 documents of 2 KB, 256 parameters of 32 bits: 256 entries 8.80 ms,
+// 512: 8.45, 1024: 8.17.
+constexpr uint32_t kRecentEntries = 1024;
+constexpr uint32_t kNoPlace       = kFoldFrom + kTile + 31;
 template <typename T>
 struct WaveLds {
   alignas(16) uint32_t bytes[kTileWords];
-  alignas(16) T hashes[kTile + (sizeof(T) == 4 ? 4 : 36)];  // (64-bit ones: up to 31 of the tile before in front)
-  alignas(16) T recent[recent_entries<T>()];
+  alignas(16) T hashes[sizeof(T) == 4 ? kTile + 4 : kNoPlace + 1];
+  alignas(16) std::conditional_t<sizeof(T) == 4, T, uint16_t> recent[kRecentEntries];
   uint16_t chars[kCharList];  // where the characters of the staged bytes start, in order (see CharMap)
 };
 

@@ -160,6 +160,21 @@ def test_minhash64_last_blocks(nv, orc, count):
     assert nv.minhash64(dev(nv, host), 5, a, b, 5).to_host().equals(orc.minhash64(host, 5, a, b, 5, nthreads=8))
 
 
+@pytest.mark.parametrize("count", [33, 97, 160, 161, 193, 225, 288, 289])
+def test_minhash64_gathered_hashes(nv, orc, count):
+    """Rows of as many windows as are gathered before they meet the parameters (416) and as a tile of 256 more gives, one
+    less and more, whole blocks of 32 or not, in a column long enough that they are not cut; every number of groups of
+    parameters that are done two, four or one at a time, and two chunks; windows that repeat within what is remembered."""
+    rng = np.random.default_rng(count)
+    a, b = params(rng, count, 64)
+    windows = [1, 255, 256, 257, 400, 415, 416, 417, 447, 448, 449, 511, 512, 513, 671, 672, 673, 700]
+    rows = [random_text(rng, n + 4).decode() for n in windows * 800]
+    words = ["ox", "a", "tree", "mill", "saturn", "of"]
+    rows += [" ".join(words[i] for i in rng.integers(0, 6, 160)) for _ in range(800)]
+    host = HostStringsColumn.from_pylist(rows)
+    assert nv.minhash64(dev(nv, host), 5, a, b, 5).to_host().equals(orc.minhash64(host, 5, a, b, 5, nthreads=8))
+
+
 @pytest.mark.parametrize("bits", [32, 64])
 @pytest.mark.parametrize("ngrams", [2, 5])
 @pytest.mark.parametrize("count", [1, 130])
