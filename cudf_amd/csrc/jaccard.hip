@@ -234,7 +234,7 @@ template <bool IN_LDS>
 __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2, Pair const& pair, int32_t width, PairSet<IN_LDS> const& set,
                                             uint32_t* in1, uint32_t* in2, Part part, TileLds& lds, int wave, int nwaves, int lane)
 {
-  auto const hash = [](auto const& src, uint32_t len) { return murmur3_x86_32_unmixed(src, len, 0u); };  // jaccard.cu:258: seed 0
+  auto const hash = [](auto const& src, uint32_t len, auto& h) { murmur3_x86_32_unmixed(src, len, 0u, h); };  // jaccard.cu:258: seed 0
   bool ok         = true;
   if (static_cast<int64_t>(width) * 4 <= kHalo) {
     int64_t const even   = pair.bytes() / (nwaves * kWave) * kWave;
@@ -281,12 +281,13 @@ __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2
     int64_t const n        = row == 0 ? pair.n1 : pair.n2;
     for (int64_t gpos = static_cast<int64_t>(wave) * kWave + lane; gpos < n; gpos += nwaves * kWave) {
       int64_t const remaining = n - gpos;
-      BoundedSrc const src{r + gpos, remaining};
+      BoundedSrc const src[1] = {{r + gpos, remaining}};
       uint32_t hlen;
       uint32_t const readable = static_cast<uint32_t>(min(remaining, static_cast<int64_t>(width) * 4));
-      if (window_at(src, r + gpos, remaining, readable, gpos == 0, false, width, &hlen)) {
-        uint32_t const hv = hash(src, hlen);
-        if (hv != 0u && part.holds(hv)) ok = set.insert(hv, row == 0 ? in1 : in2) && ok;
+      if (window_at(src[0], r + gpos, remaining, readable, gpos == 0, false, width, &hlen)) {
+        uint32_t hv[1];
+        hash(src, hlen, hv);
+        if (hv[0] != 0u && part.holds(hv[0])) ok = set.insert(hv[0], row == 0 ? in1 : in2) && ok;
       }
     }
   }

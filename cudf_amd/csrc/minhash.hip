@@ -50,20 +50,25 @@ template <typename T>
 struct HashTraits;
 template <>
 struct HashTraits<uint32_t> {
-  template <typename Src>
-  static __device__ __forceinline__ uint32_t hash(Src const& src, uint32_t len, uint32_t seed)
+  // (0 is no hash: minhash.cu:141, 237)
+  template <int N, typename Src>
+  static __device__ __forceinline__ void hash(Src const (&src)[N], uint32_t len, uint32_t seed, uint32_t (&h)[N])
   {
-    return murmur3_x86_32(src, len, seed);
+    murmur3_x86_32<N>(src, len, seed, h);
+#pragma unroll
+    for (int n = 0; n < N; ++n) h[n] = max(h[n], 1u);
   }
   // Permutation (minhash.cu:350-351) in uint32 arithmetic: the product and sum wrap mod 2^32, after
   // which "% (2^61-1)" and "& max" change nothing: (hv * a + b), see Fold.
 };
 template <>
 struct HashTraits<uint64_t> {
-  template <typename Src>
-  static __device__ __forceinline__ uint64_t hash(Src const& src, uint32_t len, uint64_t seed)
+  template <int N, typename Src>
+  static __device__ __forceinline__ void hash(Src const (&src)[N], uint32_t len, uint64_t seed, uint64_t (&h)[N])
   {
-    return murmur3_x64_128_lo(src, len, seed);  // minhash.cu:138: first word of the 128-bit hash
+    murmur3_x64_128_lo<N>(src, len, seed, h);  // minhash.cu:138: first word of the 128-bit hash
+#pragma unroll
+    for (int n = 0; n < N; ++n) h[n] += h[n] == 0 ? 1u : 0u;
   }
   // Permutation (minhash.cu:350-351): ((hv*a + b) mod 2^64) % (2^61-1), see filter64.cuh.
 };
@@ -485,30 +490,46 @@ struct Minima64 {
 
 // Puts the fresh ones of a trip's hashes (a lane with `valid` has one) behind the `count` that wait in lds.hashes: those that
 // the wavefront has not met lately.
-__device__ __forceinline__ void gather(WaveLds<uint32_t>& lds, bool valid, uint32_t hv, uint32_t* count)
+template <int N>
+__device__ __forceinline__ void gather(WaveLds<uint32_t>& lds, bool const (&valid)[N], uint32_t const (&hv)[N], uint32_t* count)
 {
-  bool fresh = false;
-  if (valid) {
-    uint32_t* const at = &lds.recent[hv & (kRecentEntries - 1)];
-    fresh              = *at != hv;
-    *at                = hv;
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    bool fresh = false;
+    if (valid[n]) {
+      uint32_t* const at = &lds.recent[hv[n] & (kRecentEntries - 1)];
+      fresh              = *at != hv[n];
+      *at                = hv[n];
+    }
+    uint64_t const vm = ballot64(fresh);
+    if (fresh) lds.hashes[*count + lanes_below(vm)] = hv[n];
+    *count += static_cast<uint32_t>(__builtin_popcountll(vm));
   }
-  uint64_t const vm = ballot64(fresh);
-  if (fresh) lds.hashes[*count + lanes_below(vm)] = hv;
-  *count += static_cast<uint32_t>(__builtin_popcountll(vm));
 }
 // 64-bit hashes: the table says where among the hashes that were gathered (and perhaps folded since, in the same part) it may be
-__device__ __forceinline__ void gather(WaveLds<uint64_t>& lds, bool valid, uint64_t hv, uint32_t* count)
+template <int N>
+__device__ __forceinline__ void gather(WaveLds<uint64_t>& lds, bool const (&valid)[N], uint64_t const (&hv)[N], uint32_t* count)
 {
-  uint16_t* const at = &lds.recent[static_cast<uint32_t>(hv) & (kRecentEntries - 1)];
-  bool const fresh   = valid && lds.hashes[*at] != hv;
-  uint64_t const vm  = ballot64(fresh);
-  if (fresh) {
-    uint32_t const place = *count + lanes_below(vm);
-    lds.hashes[place]    = hv;
-    *at                  = static_cast<uint16_t>(place);
+  uint16_t* at[N];
+  uint32_t place[N];
+  bool fresh[N];
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    at[n]    = &lds.recent[static_cast<uint32_t>(hv[n]) & (kRecentEntries - 1)];
+    place[n] = *at[n];
   }
-  *count += static_cast<uint32_t>(__builtin_popcountll(vm));
+#pragma unroll
+  for (int n = 0; n < N; ++n) fresh[n] = valid[n] && lds.hashes[place[n]] != hv[n];
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    uint64_t const vm = ballot64(fresh[n]);
+    if (fresh[n]) {
+      place[n]             = *count + lanes_below(vm);
+      lds.hashes[place[n]] = hv[n];
+      *at[n]               = static_cast<uint16_t>(place[n]);
+    }
+    *count += static_cast<uint32_t>(__builtin_popcountll(vm));
+  }
 }
 template <typename T>
 __device__ __forceinline__ void forget_hashes(WaveLds<T>& lds, int lane)
@@ -563,31 +584,25 @@ struct TextRows {
     for (int64_t base = begin; base < end; base += step) {
       if (narrow) {
         uint32_t const cnt = static_cast<uint32_t>(min(static_cast<int64_t>(kTile), end - base));
-        auto const hash    = [seed = seed](WordSrc const& src, uint32_t len) {
-          T const hv = H::hash(src, len, seed);
-          return hv < 1 ? T{1} : hv;  // minhash.cu:141
-        };
+        auto const hash    = [seed = seed](auto const& src, uint32_t len, auto& h) { H::hash(src, len, seed, h); };
         hash_tile_windows<T>(row, n, base, cnt, width, lds.bytes, lds.chars, lane, hash, [&](auto const& valid, auto const& hv) {
-          for (auto const& h : hv) gather(lds, valid[&h - hv], h, &count);
+          gather(lds, valid, hv, &count);
         });
       } else {
         // very wide windows: 64 starts at a time, bytes read straight from global memory
         int64_t const gpos = base + lane;
         bool valid         = false;
-        T hv               = 0;
+        T hv[1]            = {0};
         if (gpos < end) {
           int64_t const remaining = n - gpos;
-          BoundedSrc const src{row + gpos, remaining};
+          BoundedSrc const src[1] = {{row + gpos, remaining}};
           uint32_t hlen;
           uint32_t const readable = static_cast<uint32_t>(min(remaining, static_cast<int64_t>(width) * 4));
-          valid = window_at(src, row + gpos, remaining, readable, gpos == 0, false, width, &hlen);
-          if (valid) {
-            hv = H::hash(src, hlen, seed);
-            hv = hv < 1 ? T{1} : hv;
-          }
+          valid = window_at(src[0], row + gpos, remaining, readable, gpos == 0, false, width, &hlen);
+          if (valid) H::hash(src, hlen, seed, hv);
         }
         uint64_t const vm = ballot64(valid);
-        if (valid) lds.hashes[count + lanes_below(vm)] = hv;
+        if (valid) lds.hashes[count + lanes_below(vm)] = hv[0];
         count += static_cast<uint32_t>(__builtin_popcountll(vm));
       }
       count = minima.fold(lds.hashes, count, base + step >= end);
@@ -624,13 +639,11 @@ struct AlignedSrc {
     end = mis + len;
   }
   __device__ __forceinline__ uint32_t byte(uint32_t i) const { return reinterpret_cast<const uint8_t*>(w)[mis + i]; }
-  __device__ __forceinline__ uint32_t u32(uint32_t i) const
+  __device__ __forceinline__ uint32_t dword(uint32_t k) const
   {
-    uint32_t const o  = mis + i;
-    uint32_t const j  = o >> 2;
-    uint32_t const lo = 4u * j < end ? w[j] : 0u;
-    uint32_t const hi = 4u * (j + 1u) < end ? w[j + 1] : 0u;
-    return __builtin_amdgcn_alignbit(hi, lo, (o & 3u) * 8u);
+    uint32_t const lo = 4u * k < end ? w[k] : 0u;
+    uint32_t const hi = 4u * (k + 1u) < end ? w[k + 1] : 0u;
+    return __builtin_amdgcn_alignbit(hi, lo, mis * 8u);
   }
 };
 
@@ -695,7 +708,7 @@ struct RunRows {
       bool const valid        = idx < end && (idx == 0 || idx + ngrams < n) && col.child.valid(first + idx);
       int64_t const run_begin = bo;
       uint32_t const run      = static_cast<uint32_t>(eo - bo);
-      T hv                    = 0;
+      T hv[1]                 = {0};
       // The runs of these 64 elements overlap and lie side by side in the chars: fetch that stretch once, with
       // coalesced loads, and hash out of LDS (the hash walks a run dword by dword, each step a dependent read).
       // A stretch too long for the buffer is hashed straight from memory.
@@ -706,14 +719,15 @@ struct RunRows {
         bool ascii;
         uint32_t const mis = stage_bytes(col.child.chars, span_begin, static_cast<uint32_t>(span_end - span_begin), lds.bytes, lane, &ascii);
         wave_lds_fence();
-        if (valid) hv = H::hash(WordSrc{lds.bytes, mis + static_cast<uint32_t>(run_begin - span_begin)}, run, seed);
+        WordSrc const src[1] = {WordSrc(lds.bytes, mis + static_cast<uint32_t>(run_begin - span_begin))};
+        if (valid) H::hash(src, run, seed, hv);
         wave_lds_fence();
       } else if (valid) {
-        hv = H::hash(AlignedSrc(col.child.chars + run_begin, run), run, seed);
+        AlignedSrc const src[1] = {AlignedSrc(col.child.chars + run_begin, run)};
+        H::hash(src, run, seed, hv);
       }
-      hv                = hv < 1 ? T{1} : hv;  // 237
       uint64_t const vm = ballot64(valid);
-      if (valid) lds.hashes[count + lanes_below(vm)] = hv;
+      if (valid) lds.hashes[count + lanes_below(vm)] = hv[0];
       count += static_cast<uint32_t>(__builtin_popcountll(vm));
       if (count > run_hashes<T>() - kWave) {  // (whole blocks but where elements are null)
         minima.fold(lds.hashes, count, true);

@@ -14,15 +14,6 @@ namespace nvtext_amd {
 __device__ __forceinline__ uint32_t rotl32(uint32_t x, int r) { return __builtin_amdgcn_alignbit(x, x, 32 - r); }
 __device__ __forceinline__ uint64_t rotl64(uint64_t x, int r) { return (x << r) | (x >> (64 - r)); }
 
-// Dword starting at byte offset `o` of the dword array `w` (reads w[o/4] and w[o/4+1]).
-__device__ __forceinline__ uint32_t load_u32_at(const uint32_t* w, uint32_t o)
-{
-  uint32_t const i  = o >> 2;
-  uint32_t const lo = w[i];
-  uint32_t const hi = w[i + 1];
-  return __builtin_amdgcn_alignbit(hi, lo, (o & 3u) * 8u);
-}
-
 __device__ __forceinline__ uint32_t keep_low_bytes(uint32_t v, int nbytes)
 {
   // nbytes in [0, 4]
@@ -30,12 +21,14 @@ __device__ __forceinline__ uint32_t keep_low_bytes(uint32_t v, int nbytes)
 }
 
 // Byte source over a dword array (an LDS tile): window byte i lives at byte offset base+i.
-// u32(i) may read up to 11 bytes past the window (callers mask what they do not need).
+// dword(k), bytes 4k to 4k + 3 of the window, may read up to 11 bytes past the window (callers mask what they do not need).
+// (A shift of two aligned dwords: an unaligned read of LDS takes a cycle a lane.)
 struct WordSrc {
-  const uint32_t* w;
-  uint32_t base;
-  __device__ __forceinline__ uint32_t byte(uint32_t i) const { return reinterpret_cast<const uint8_t*>(w)[base + i]; }
-  __device__ __forceinline__ uint32_t u32(uint32_t i) const { return load_u32_at(w, base + i); }
+  const uint32_t* at;  // the dword with the window's first byte
+  uint32_t mis;        // where in it
+  __device__ __forceinline__ WordSrc(const uint32_t* w, uint32_t base) : at(w + (base >> 2)), mis(base & 3u) {}
+  __device__ __forceinline__ uint32_t byte(uint32_t i) const { return reinterpret_cast<const uint8_t*>(at)[mis + i]; }
+  __device__ __forceinline__ uint32_t dword(uint32_t k) const { return __builtin_amdgcn_alignbit(at[k + 1], at[k], 8u * mis); }
 };
 
 // Byte source over global memory that never touches a byte at or past `avail`
@@ -44,54 +37,56 @@ struct BoundedSrc {
   const uint8_t* p;
   int64_t avail;
   __device__ __forceinline__ uint32_t byte(uint32_t i) const { return p[i]; }
-  __device__ __forceinline__ uint32_t u32(uint32_t i) const
+  __device__ __forceinline__ uint32_t dword(uint32_t k) const
   {
     uint32_t v = 0;
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if (static_cast<int64_t>(i) + k < avail) v |= static_cast<uint32_t>(p[i + k]) << (8 * k);
+    for (int j = 0; j < 4; ++j)
+      if (4 * static_cast<int64_t>(k) + j < avail) v |= static_cast<uint32_t>(p[4 * k + j]) << (8 * j);
     return v;
   }
 };
 
-// Hash of window bytes [0, len) of `src` before its final mix.  The mix is a bijection that keeps 0, so where hashes are
-// only compared with one another and with 0 this does as well.
-template <typename Src>
-__device__ __forceinline__ uint32_t murmur3_x86_32_unmixed(Src const& src, uint32_t len, uint32_t seed)
+// The hashes take N windows of one length at a time, step by step: their chains of reads and multiplications run side by side.
+
+// Hashes of window bytes [0, len) of every `src` before their final mix.  The mix is a bijection that keeps 0, so where hashes
+// are only compared with one another and with 0 these do as well.
+template <int N, typename Src>
+__device__ __forceinline__ void murmur3_x86_32_unmixed(Src const (&src)[N], uint32_t len, uint32_t seed, uint32_t (&h)[N])
 {
   uint32_t const c1 = 0xcc9e2d51u, c2 = 0x1b873593u;
-  uint32_t h1           = seed;
   uint32_t const blocks = len >> 2;
+#pragma unroll
+  for (int n = 0; n < N; ++n) h[n] = seed;
   for (uint32_t i = 0; i < blocks; ++i) {
-    uint32_t k1 = src.u32(4 * i);
-    k1 *= c1;
-    k1 = rotl32(k1, 15);
-    k1 *= c2;
-    h1 ^= k1;
-    h1 = rotl32(h1, 13);
-    h1 = h1 * 5u + 0xe6546b64u;
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      uint32_t const k1 = rotl32(src[n].dword(i) * c1, 15) * c2;
+      h[n]              = rotl32(h[n] ^ k1, 13) * 5u + 0xe6546b64u;
+    }
   }
   uint32_t const rem = len & 3u;
   if (rem) {
-    uint32_t k1 = keep_low_bytes(src.u32(4 * blocks), static_cast<int>(rem));
-    k1 *= c1;
-    k1 = rotl32(k1, 15);
-    k1 *= c2;
-    h1 ^= k1;
+#pragma unroll
+    for (int n = 0; n < N; ++n) h[n] ^= rotl32(keep_low_bytes(src[n].dword(blocks), static_cast<int>(rem)) * c1, 15) * c2;
   }
-  return h1 ^ len;
+#pragma unroll
+  for (int n = 0; n < N; ++n) h[n] ^= len;
 }
 
-template <typename Src>
-__device__ __forceinline__ uint32_t murmur3_x86_32(Src const& src, uint32_t len, uint32_t seed)
+template <int N, typename Src>
+__device__ __forceinline__ void murmur3_x86_32(Src const (&src)[N], uint32_t len, uint32_t seed, uint32_t (&h)[N])
 {
-  uint32_t h1 = murmur3_x86_32_unmixed(src, len, seed);
-  h1 ^= h1 >> 16;
-  h1 *= 0x85ebca6bu;
-  h1 ^= h1 >> 13;
-  h1 *= 0xc2b2ae35u;
-  h1 ^= h1 >> 16;
-  return h1;
+  murmur3_x86_32_unmixed<N>(src, len, seed, h);
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    uint32_t h1 = h[n];
+    h1 ^= h1 >> 16;
+    h1 *= 0x85ebca6bu;
+    h1 ^= h1 >> 13;
+    h1 *= 0xc2b2ae35u;
+    h[n] = h1 ^ (h1 >> 16);
+  }
 }
 
 __device__ __forceinline__ uint64_t fmix64(uint64_t k)
@@ -104,57 +99,55 @@ __device__ __forceinline__ uint64_t fmix64(uint64_t k)
   return k;
 }
 
-template <typename Src>
-__device__ __forceinline__ uint64_t load_u64(Src const& src, uint32_t i)
-{
-  return (static_cast<uint64_t>(src.u32(i + 4)) << 32) | src.u32(i);
-}
-
 // The first n bytes (0 .. 8) of v.
 __device__ __forceinline__ uint64_t low_bytes64(uint64_t v, uint32_t n) { return n == 0 ? 0 : v & (~0ull >> (64u - 8u * n)); }
 
-// First 64-bit word of MurmurHash3_x64_128 with h1 = h2 = seed over window bytes [0, len).  What is left of the key after
+// First 64-bit words of MurmurHash3_x64_128 with h1 = h2 = seed over window bytes [0, len).  What is left of the key after
 // its blocks of 16 is treated as a block is up to where the halves are mixed: zeros in place of missing bytes change nothing,
 // and lanes with keys either side of 16 bytes go one way (before, the ones waited while the others did their blocks).
-template <typename Src>
-__device__ __forceinline__ uint64_t murmur3_x64_128_lo(Src const& src, uint32_t len, uint64_t seed)
+template <int N, typename Src>
+__device__ __forceinline__ void murmur3_x64_128_lo(Src const (&src)[N], uint32_t len, uint64_t seed, uint64_t (&h)[N])
 {
   uint64_t const c1 = 0x87c37b91114253d5ull, c2 = 0x4cf5ad432745937full;
-  uint64_t h1 = seed, h2 = seed;
+  uint64_t h1[N], h2[N];
+#pragma unroll
+  for (int n = 0; n < N; ++n) h1[n] = h2[n] = seed;
   for (uint32_t t = 0; t < len; t += 16) {
-    uint32_t const left = len - t;
-    uint64_t k1 = low_bytes64(load_u64(src, t), min(left, 8u));
-    k1 *= c1;
-    k1 = rotl64(k1, 31);
-    k1 *= c2;
-    h1 ^= k1;
-    uint64_t k2 = 0;
+    uint32_t const left = len - t, at = t / 4u;
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      uint64_t const k1 = static_cast<uint64_t>(src[n].dword(at + 1)) << 32 | src[n].dword(at);
+      h1[n] ^= rotl64(low_bytes64(k1, min(left, 8u)) * c1, 31) * c2;
+    }
+    uint64_t k2[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) k2[n] = 0;
     if (left > 8) {
-      k2 = low_bytes64(load_u64(src, t + 8), min(left, 16u) - 8u);
-      k2 *= c2;
-      k2 = rotl64(k2, 33);
-      k2 *= c1;
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        uint64_t const k = static_cast<uint64_t>(src[n].dword(at + 3)) << 32 | src[n].dword(at + 2);
+        k2[n]            = rotl64(low_bytes64(k, min(left, 16u) - 8u) * c2, 33) * c1;
+      }
     }
     if (left >= 16) {
-      h1 = rotl64(h1, 27);
-      h1 += h2;
-      h1 = h1 * 5 + 0x52dce729;
-      h2 ^= k2;
-      h2 = rotl64(h2, 31);
-      h2 += h1;
-      h2 = h2 * 5 + 0x38495ab5;
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        h1[n] = (rotl64(h1[n], 27) + h2[n]) * 5 + 0x52dce729;
+        h2[n] = (rotl64(h2[n] ^ k2[n], 31) + h1[n]) * 5 + 0x38495ab5;
+      }
     } else {
-      h2 ^= k2;
+#pragma unroll
+      for (int n = 0; n < N; ++n) h2[n] ^= k2[n];
     }
   }
-  h1 ^= len;
-  h2 ^= len;
-  h1 += h2;
-  h2 += h1;
-  h1 = fmix64(h1);
-  h2 = fmix64(h2);
-  h1 += h2;
-  return h1;
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    h1[n] ^= len;
+    h2[n] ^= len;
+    h1[n] += h2[n];
+    h2[n] += h1[n];
+    h[n] = fmix64(h1[n]) + fmix64(h2[n]);
+  }
 }
 
 }  // namespace nvtext_amd

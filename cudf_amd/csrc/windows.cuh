@@ -165,10 +165,10 @@ __device__ __forceinline__ bool window_at(Src const& src, const uint8_t* g, int6
   return first || left <= 0;
 }
 
-// The windows that start in [base, base + cnt) of a row of n bytes (cnt <= kTile, 4 * width <= kHalo): `hash(src, bytes)`
-// of each goes to `sink(valid, hash)`, which every lane of the wavefront calls together, with arrays of one window per
-// lane or of two (two chains of LDS reads and multiplies in flight instead of one).  `bytes` and `chars` are the
-// wavefront's own LDS.
+// The windows that start in [base, base + cnt) of a row of n bytes (cnt <= kTile, 4 * width <= kHalo): `hash(src, bytes, h)`
+// of each (arrays of one source and hash or of two, of one length) goes to `sink(valid, h)`, which every lane of the wavefront
+// calls together, with arrays of one window per lane or of two (two chains of LDS reads and multiplies in flight instead of
+// one).  `bytes` and `chars` are the wavefront's own LDS.
 template <typename T, typename Hash, typename Sink>
 __device__ __forceinline__ void hash_tile_windows(const uint8_t* row, int64_t n, int64_t base, uint32_t cnt, int32_t width, uint32_t* bytes,
                                                   uint16_t* chars, int lane, Hash const& hash, Sink&& sink)
@@ -191,15 +191,19 @@ __device__ __forceinline__ void hash_tile_windows(const uint8_t* row, int64_t n,
     uint32_t q = 0;
     for (; q + kWave < starts; q += 2 * kWave) {
       // (a lane beyond the last window hashes the bytes of that one: no branch)
-      uint32_t const p      = q + lane;
-      bool const valid[2]   = {true, p + kWave < starts};
-      T const hv[2]         = {hash(WordSrc{bytes, mis + p}, width_all), hash(WordSrc{bytes, mis + min(p + kWave, starts - 1u)}, width_all)};
+      uint32_t const p     = q + lane;
+      bool const valid[2]  = {true, p + kWave < starts};
+      WordSrc const src[2] = {WordSrc(bytes, mis + p), WordSrc(bytes, mis + min(p + kWave, starts - 1u))};
+      T hv[2];
+      hash(src, width_all, hv);
       sink(valid, hv);
     }
     if (q < starts) {
-      uint32_t const p    = q + lane;
-      bool const valid[1] = {p < starts};
-      T const hv[1]       = {hash(WordSrc{bytes, mis + min(p, starts - 1u)}, width_all)};
+      uint32_t const p     = q + lane;
+      bool const valid[1]  = {p < starts};
+      WordSrc const src[1] = {WordSrc(bytes, mis + min(p, starts - 1u))};
+      T hv[1];
+      hash(src, width_all, hv);
       sink(valid, hv);
     }
   } else {
@@ -220,10 +224,11 @@ __device__ __forceinline__ void hash_tile_windows(const uint8_t* row, int64_t n,
           valid[0] = map.window(item, len, base == 0, width, chars, &p, &hlen);
         } else {
           int64_t const gpos = base + p;
-          WordSrc const at{bytes, mis + p};
+          WordSrc const at(bytes, mis + p);
           valid[0] = window_at(at, row + gpos, n - gpos, len - p, gpos == 0, all_ascii, width, &hlen);
         }
-        if (valid[0]) hv[0] = hash(WordSrc{bytes, mis + p}, hlen);
+        WordSrc const src[1] = {WordSrc(bytes, mis + p)};
+        if (valid[0]) hash(src, hlen, hv);
       }
       sink(valid, hv);
     }
