@@ -5,24 +5,24 @@
 // and common values with a warp per row (66-170, 196-400).
 //
 // Here a row pair needs no sort and no temporary: the window hashes of both rows go into ONE open-addressing set in
-// LDS with two membership bits per slot, "seen in row 1" and "seen in row 2".  |A|, |B| and |A n B| are then population
-// counts of the two bit arrays and of their AND.
+// LDS whose slots also say "seen in row 1" and "seen in row 2".  |A|, |B| and |A n B| are then counts of these marks.
 //
-// What bounds it: LDS traffic and the vector instructions of hash and probe, about as much of each; HBM sees the chars
-// once.  Hence
-//   * buckets of four slots, read with one 16-byte LDS read: a hash that is there already (text repeats its words, and
-//     the two rows are near-duplicates more often than not) costs that read and no compare-and-swap, and a probe seldom
-//     goes on to a second bucket, for which the whole wavefront would wait;
-//   * the membership bit is or-ed without asking for the old value: nothing waits for it;
+// What bounds it: vector instructions, some 100 per 64 windows, a third of them the hash, issued in three quarters of the
+// cycles, and LDS, busy for half of the time; HBM sees the chars once.  Hence
+//   * buckets of four slots, read with one 16-byte LDS read: a probe seldom goes on to a second bucket, for which the whole
+//     wavefront would wait; what one look does not place is put aside and placed 64 at a time;
+//   * value and marks in one word (PackedSet): no address and no mask to be made for a mark;
+//   * every wavefront of a pair hashes as many windows as the others, to 64, and the sets are left empty by the pass that
+//     counts: two barriers a pair;
 //   * sets of five sizes, the smallest that holds a pair: what a CU can hide of the LDS latency is the number of
-//     wavefronts that its 160 KB of sets allow.  A wavefront sizes the pairs, does the shortest itself, each with a set
-//     of its own, and lists the others, each for the kernel with the set that fits it;
+//     wavefronts that its 160 KB of sets allow (as does the number of scalar registers: eight per SIMD have 96 each).  A
+//     wavefront sizes the pairs, does the shortest itself, each with a set of its own, and lists the others, each for the
+//     kernel with the set that fits it;
 //   * a pair too long for one set in LDS is cut by hash value into up to kMaxParts parts of equal size, a workgroup each,
 //     which hash the whole pair and keep their part (hashing is the cheap half); the counts of the parts add up.  Only
 //     pairs beyond that use a set in global memory, whose atomics run at a fiftieth of the rate (1,600 such pairs among
 //     250,000 of 2 KB rows: 3.7 of the call's 9.6 ms before the parts).
-// 250,001 pairs of 2 KB rows (1.02 GB): 9.6 ms with a compare-and-swap on every window and four sizes of sets, 4.4 ms
-// now (230 GB/s); about 100 vector instructions per 64 windows, a quarter of them the hash, issued in 70 % of the cycles.
+// 250,001 pairs of 2 KB rows (1.02 GB): 4.08 ms with whole values, bits in arrays and tiles in turn, 3.5 ms now (290 GB/s).
 #include "common.cuh"
 #include "murmur.cuh"
 #include "windows.cuh"
@@ -36,8 +36,10 @@ namespace {
 // The tiers: slots of the set, wavefronts that share it, and the most bytes of a pair, which keep the load at or below
 // 0.8 when no window repeats.
 constexpr int kTiers              = 5;
-constexpr uint32_t kSlots[kTiers] = {1024, 4096, 8064, 14336, 29440};
-constexpr int kTierWaves[kTiers]  = {1, 4, 8, 8, 16};  // 7, 27, 53, 80 and 163 KB of LDS a workgroup
+constexpr uint32_t kSlots[kTiers] = {1024, 4096, 7008, 15488, 29440};
+constexpr int kTierWaves[kTiers]  = {1, 4, 8, 12, 16};  // 6, 23, 41, 81 and 144 KB of LDS a workgroup
+constexpr int kSimdWaves[kTiers]  = {6, 7, 8, 6, 4};    // wavefronts per SIMD that these leave room for
+static_assert(kSlots[kTiers - 1] / 4 <= 255 * kTierWaves[kTiers - 1] * kWave, "the counters of a lane");
 constexpr int64_t most_bytes(uint32_t slots) { return static_cast<int64_t>(slots) * 4 / 5; }
 // the lists of pairs: tiers 1 to 4 (list = tier - 1), pairs in parts, pairs for the set in global memory
 constexpr int kPartsList  = kTiers - 1;
@@ -57,10 +59,97 @@ __device__ __forceinline__ int list_of(int64_t bytes)
   return list < kPartsList ? list : parts_of(bytes) <= kMaxParts ? kPartsList : kGlobalList;
 }
 
-// An insert-only set of non-zero uint32 values, in buckets of four slots that fill from the first to the last.  Beside it
-// a bit array for each row: bit s says that the value in slot s occurs there.
-// Where the set lies in global memory (IN_LDS false), reads of it go past the CU's own cache, which does not see what
-// the atomics changed.
+// Insert-only sets of non-zero uint32 values, in buckets of four slots that fill from the first to the last.  A value's home
+// bucket is what the top of its product with an odd number says.  place_at() has one look at bucket home + distance for each of
+// N values: `left` stays where the value is not in the set now, marked as its row's; `taken` tells whether the bucket is full
+// of others, so that the next one is to be looked at.
+//
+// The set of a pair whose windows LDS has room for.  A slot holds 24 bits of the value's product, which tell the values of one
+// home bucket apart where there are 256 buckets and more, how many buckets from home it lies (6 bits), and two bits that say
+// which rows it occurs in: one compare-and-swap places a value and marks it, a value that is there already is marked with
+// an or of a constant to the same address, and counting is a pass over the slots.  (With whole values and the bits in arrays
+// of their own a look took 65 vector instructions for 128 windows, beside 65 for their hashes; now 55.)
+struct PackedSet {
+  static constexpr uint32_t kValue    = 0x00FFFFFFu;
+  static constexpr uint32_t kFar      = 64;  // buckets from home that can be told
+  static constexpr int kDistanceAt    = 25;
+  static constexpr uint32_t kSame     = 0x7EFFFFFFu;  // value and distance
+  static constexpr uint32_t kLeast    = 1024;         // slots
+  using Mark                          = uint32_t;
+  using Place                         = int32_t;      // in a row, where the pairs are short
+  uint32_t* slots;  // 0 = empty; 16-byte aligned
+  uint32_t buckets;
+
+  static __device__ __forceinline__ Mark mark(bool second) { return second ? 0x80000000u : 0x01000000u; }
+  // Counts marks: the top bytes of four slots side by side, a counter a byte for each row and for both (at most 255 times four
+  // slots: a third of the instructions that shifts and additions slot by slot take, 15 of 109 per 64 windows of a pair of 2 KB).
+  struct Count {
+    uint32_t in1 = 0, in2 = 0, both = 0;
+    __device__ __forceinline__ void add(uint4 v)
+    {
+      constexpr uint32_t kOnes = 0x01010101u;
+      uint32_t const a = __builtin_amdgcn_perm(v.y, v.x, 0x0C0C0703u) | __builtin_amdgcn_perm(v.w, v.z, 0x07030C0Cu), b = a >> 7;
+      in1 += a & kOnes;
+      in2 += b & kOnes;
+      both += a & b & kOnes;
+    }
+    __device__ __forceinline__ void get(uint32_t (&u)[3]) const
+    {
+      u[0] = __builtin_amdgcn_sad_u8(in1, 0u, 0u);
+      u[1] = __builtin_amdgcn_sad_u8(in2, 0u, 0u);
+      u[2] = __builtin_amdgcn_sad_u8(both, 0u, 0u);
+    }
+  };
+
+  template <int N>
+  __device__ __forceinline__ void place_at(bool (&left)[N], const uint32_t (&h)[N], const uint32_t (&bucket)[N], const uint32_t (&distance)[N], Mark mark,
+                                           bool (&taken)[N]) const
+  {
+    uint4 v[N];
+    uint32_t id[N], s[N], full[N], old[N];
+    bool tried[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = reinterpret_cast<const uint4*>(slots)[bucket[k]];
+    __builtin_amdgcn_sched_barrier(0);  // (all reads on their way before the first is waited for)
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      id[k] = (product(h[k]) & kValue) | distance[k] << kDistanceAt;
+      // 1 as long as the slots so far hold other values (0 where one is empty or holds this one)
+      uint32_t const a0 = least(1u, v[k].x, (v[k].x ^ id[k]) & kSame);
+      uint32_t const a1 = least(a0, v[k].y, (v[k].y ^ id[k]) & kSame);
+      uint32_t const a2 = least(a1, v[k].z, (v[k].z ^ id[k]) & kSame);
+      full[k]           = least(a2, v[k].w, (v[k].w ^ id[k]) & kSame);
+      s[k]              = 4u * bucket[k] + (a0 + a1 + a2);
+      taken[k]          = full[k] != 0u;
+      tried[k]          = left[k] & !taken[k];
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      old[k] = id[k] ^ 1u;  // (another one)
+      // (also where the slot holds the value already: cheaper than telling the two apart first)
+      if (tried[k]) old[k] = atomicCAS(&slots[s[k]], 0u, id[k] | mark);
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      bool const there = tried[k] & (((old[k] ^ id[k]) & kSame) == 0u);
+      if (there) atomicOr(&slots[s[k]], mark);
+      left[k] = left[k] & !(there | (tried[k] & (old[k] == 0u)));  // (else another value came first)
+    }
+  }
+  static __device__ __forceinline__ uint32_t product(uint32_t h) { return h * 0x9E3779B1u; }
+  __device__ __forceinline__ uint32_t home(uint32_t h) const { return __umulhi(product(h), buckets); }
+  // (written out: the compiler makes a comparison and a selection of the minimum with 1)
+  static __device__ __forceinline__ uint32_t least(uint32_t a, uint32_t b, uint32_t c)
+  {
+    uint32_t m;
+    asm("v_min3_u32 %0, %1, %2, %3" : "=v"(m) : "v"(a), "v"(b), "v"(c));
+    return m;
+  }
+};
+
+// Whole values, and beside them a bit array for each row: bit s says that the value in slot s occurs there.  Of any size, and
+// never full before its last slot is: where a packed set finds no place within kFar buckets (values made for it), and in
+// global memory (IN_LDS false), where reads go past the CU's own cache, which does not see what the atomics changed.
 template <bool IN_LDS>
 __device__ __forceinline__ uint32_t set_word(const uint32_t* p)
 {
@@ -68,77 +157,57 @@ __device__ __forceinline__ uint32_t set_word(const uint32_t* p)
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 template <bool IN_LDS>
-struct PairSet {
-  uint32_t* slots;   // 0 = empty; 16-byte aligned
+struct PlainSet {
+  static constexpr uint32_t kFar = 0xFFFFFFFFu;
+  using Mark                     = uint32_t*;
+  using Place                    = int64_t;
+  uint32_t* slots;
   uint32_t buckets;
+  uint32_t *in1, *in2;
 
+  __device__ __forceinline__ Mark mark(bool second) const { return second ? in2 : in1; }
   __device__ __forceinline__ uint32_t home(uint32_t h) const { return __umulhi(h * 0x9E3779B1u, buckets); }
-
-  // One look at one bucket for each of N values: `done` where the value is in the set now, and
-  // its row's bit set; `taken` is 1 where the bucket is full of others, else 0.
   template <int N>
-  __device__ __forceinline__ void insert_at(const bool (&want)[N], const uint32_t (&h)[N], const uint32_t (&bucket)[N], uint32_t* in, bool (&done)[N], uint32_t (&taken)[N]) const
+  __device__ __forceinline__ void place_at(bool (&left)[N], const uint32_t (&h)[N], const uint32_t (&bucket)[N], const uint32_t (&)[N], Mark in,
+                                           bool (&taken)[N]) const
   {
-    uint32_t s[N], old[N];
-    uint4 v[N];
-#pragma unroll
-    for (int k = 0; k < N; ++k) v[k] = read(bucket[k]);
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-      // a_j: 1 as long as slots 0 .. j hold other values (min(v, v ^ h) is 0 where the slot is empty or holds h)
-      uint32_t const a0 = min(min(1u, v[k].x), v[k].x ^ h[k]);
-      uint32_t const a1 = min(min(a0, v[k].y), v[k].y ^ h[k]);
-      uint32_t const a2 = min(min(a1, v[k].z), v[k].z ^ h[k]);
-      uint32_t const a3 = min(min(a2, v[k].w), v[k].w ^ h[k]);
-      s[k]     = 4u * bucket[k] + (a0 + a1 + a2);
-      taken[k] = a3;
-      done[k]  = want[k] && a3 == 0u;
+      taken[k] = false;
+      if (!left[k]) continue;
+      uint32_t s = 4u * bucket[k], v = 0;
+      for (int j = 0; j < 4; ++j, ++s) {
+        v = set_word<IN_LDS>(&slots[s]);
+        if (v == 0u) v = atomicCAS(&slots[s], 0u, h[k]);
+        if (v == 0u || v == h[k]) break;
+      }
+      taken[k] = s == 4u * bucket[k] + 4u;
+      if (!taken[k]) {
+        atomicOr(&in[s >> 5], 1u << (s & 31u));
+        left[k] = false;
+      }
     }
-    // (also where the slot holds h already: cheaper than telling the two apart first)
-#pragma unroll
-    for (int k = 0; k < N; ++k)
-      if (done[k]) old[k] = atomicCAS(&slots[s[k]], 0u, h[k]);
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-      done[k] = done[k] && (old[k] == 0u || old[k] == h[k]);  // else another value came first
-      if (done[k]) atomicOr(&in[s[k] >> 5], 1u << (s[k] & 31u));
-    }
-  }
-
-  __device__ __forceinline__ uint4 read(uint32_t bucket) const
-  {
-    uint4 v;
-    if (IN_LDS) {
-      v = reinterpret_cast<const uint4*>(slots)[bucket];
-    } else {
-      v.x = set_word<false>(&slots[4u * bucket]);
-      v.y = set_word<false>(&slots[4u * bucket + 1u]);
-      v.z = set_word<false>(&slots[4u * bucket + 2u]);
-      v.w = set_word<false>(&slots[4u * bucket + 3u]);
-    }
-    return v;
-  }
-
-  // From a bucket on, until the value is in the set.  false: every bucket is full (a set sized by the bytes of its pair
-  // has room for every window; a part of one, whose share of the hashes is only near the average, may not).
-  __device__ __forceinline__ bool insert(uint32_t h, uint32_t* in) const
-  {
-    uint32_t const v[1] = {h};
-    bool const want[1]  = {true};
-    uint32_t bucket[1]  = {home(h)};
-    for (uint32_t probes = 0; probes < buckets;) {
-      uint32_t taken[1];
-      bool done[1];
-      insert_at<1>(want, v, bucket, in, done, taken);
-      if (done[0]) return true;
-      if (taken[0] != 0u) {
-        ++probes;
-        if (++bucket[0] == buckets) bucket[0] = 0u;
-      }  // (else another value came first: once more, at most until the bucket is full)
-    }
-    return false;
   }
 };
+
+// From its home bucket on, until the value is in the set.  false: no place.
+template <typename Set>
+__device__ __forceinline__ bool place(Set const& set, uint32_t value, typename Set::Mark mark)
+{
+  uint32_t const h[1]  = {value};
+  uint32_t bucket[1]   = {set.home(value)}, distance[1] = {0u};
+  uint32_t const most  = min(set.buckets, Set::kFar);
+  while (distance[0] < most) {
+    bool left[1] = {true}, taken[1];
+    set.template place_at<1>(left, h, bucket, distance, mark, taken);
+    if (!left[0]) return true;
+    if (taken[0]) {
+      ++distance[0];
+      if (++bucket[0] == set.buckets) bucket[0] = 0u;
+    }  // (else another value came first: once more, at most until the bucket is full)
+  }
+  return false;
+}
 
 // A share of the hashes by value, for pairs that are cut into parts (other bits than the set's own multiplication uses).
 struct Part {
@@ -150,10 +219,11 @@ struct Part {
 };
 
 // A wavefront's own LDS for the tile it hashes.
+constexpr uint32_t kLater = 3 * kWave / 2;
 struct TileLds {
   alignas(16) uint32_t bytes[kTileWords];
   uint16_t chars[kCharList];
-  uint32_t later[kTile + kWave / 2];  // hashes that a first look at their bucket did not place
+  uint32_t later[kLater];  // hashes that a first look at their bucket did not place
 };
 
 __device__ __forceinline__ float index_of(uint32_t count1, uint32_t count2, uint32_t intersects)
@@ -211,10 +281,10 @@ __device__ __forceinline__ Pair uniform_pair_at(ColView const& c1, ColView const
   return p;
 }
 
-// Slots for a pair: room for twice its windows, which are at most its bytes, or what the tier has (whole words of bits).
+// Slots for a pair: room for twice its windows, which are at most its bytes, or what the tier has.
 __device__ __forceinline__ uint32_t slots_for(int64_t bytes, uint32_t most)
 {
-  return static_cast<uint32_t>(min(static_cast<int64_t>(most), (2 * bytes + 63) / 32 * 32));
+  return static_cast<uint32_t>(min(static_cast<int64_t>(most), max((2 * bytes + 63) / 32 * 32, static_cast<int64_t>(PackedSet::kLeast))));
 }
 
 // ... and in global memory: room for one and a half times its windows.
@@ -225,53 +295,65 @@ __device__ __host__ __forceinline__ uint64_t slots_for_global(int64_t bytes)
   return s;
 }
 
-// Hashes the windows of both rows (jaccard.cu:249-292) and inserts the non-zero hashes into the set.  The tiles of the
-// two rows, one list, go to `nwaves` wavefronts in turn; those of a short pair are cut finer than kTile so that each has
-// one.  false: the set was full.
+// Hashes the windows of both rows (jaccard.cu:249-292) and inserts the non-zero hashes into the set.  The two rows, one list
+// of units of 64 window starts, are shared out evenly among `nwaves` wavefronts, which take up to kTile starts of a row at a
+// time.  (Whole tiles in turn left some of four wavefronts a tile more than the others: pairs of 0.8 to 3.3 KB 5 % slower.)
+// false: a value found no place.
 // Nearly every hash finds its place with one look at one bucket, but in most rounds of 64 some lane does not: those are
 // put aside and placed 64 at a time, so that a round does not wait for its slowest lane.
-template <bool IN_LDS>
-__device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2, Pair const& pair, int32_t width, PairSet<IN_LDS> const& set,
-                                            uint32_t* in1, uint32_t* in2, Part part, TileLds& lds, int wave, int nwaves, int lane)
+template <typename Set>
+__device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2, Pair const& pair, int32_t width, Set const& set, Part part, TileLds& lds,
+                                            int wave, int nwaves, int lane)
 {
   auto const hash = [](auto const& src, uint32_t len, auto& h) { murmur3_x86_32_unmixed(src, len, 0u, h); };  // jaccard.cu:258: seed 0
   bool ok         = true;
   if (static_cast<int64_t>(width) * 4 <= kHalo) {
-    int64_t const even   = pair.bytes() / (nwaves * kWave) * kWave;
-    int32_t const tile   = static_cast<int32_t>(min(max(even, static_cast<int64_t>(kWave)), static_cast<int64_t>(kTile)));
-    int64_t const tiles1 = (pair.n1 + tile - 1) / tile, tiles = tiles1 + (pair.n2 + tile - 1) / tile;
+    using Place        = typename Set::Place;
+    Place const n1 = static_cast<Place>(pair.n1), n2 = static_cast<Place>(pair.n2);
+    const uint8_t *const row1 = c1.chars + pair.o1, *const row2 = c2.chars + pair.o2;
+    Place const units1 = (n1 + kWave - 1) / kWave, units = units1 + (n2 + kWave - 1) / kWave;
+    Place const last   = units * (wave + 1) / nwaves;
     uint32_t later = 0, later1 = 0;  // hashes put aside, and how many of them (the first ones) are row 1's: the same in every lane
-    for (int64_t t = wave; t < tiles; t += nwaves) {
-      bool const second      = t >= tiles1;
-      const uint8_t* const r = second ? c2.chars + pair.o2 : c1.chars + pair.o1;
-      int64_t const n        = second ? pair.n2 : pair.n1;
-      uint32_t* const in     = second ? in2 : in1;
-      int64_t const base     = (second ? t - tiles1 : t) * tile;
-      uint32_t const cnt     = static_cast<uint32_t>(min(static_cast<int64_t>(tile), n - base));
+    bool second    = false;
+    auto const place_later = [&] {
+      if (!second) later1 = later;
+      for (uint32_t i = lane; i < later; i += kWave) ok = place(set, lds.later[i], set.mark(i >= later1)) && ok;
+      later = later1 = 0;
+    };
+    for (Place unit = units * wave / nwaves; unit < last;) {
+      second                 = unit >= units1;
+      const uint8_t* const r = second ? row2 : row1;
+      Place const n          = second ? n2 : n1;
+      auto const mark        = set.mark(second);
+      Place const base       = (second ? unit - units1 : unit) * kWave;
+      Place const end        = min(unit + kTile / kWave, second ? last : min(last, units1));
+      uint32_t const cnt     = static_cast<uint32_t>(min((end - unit) * kWave, n - base));
+      unit                   = end;
       hash_tile_windows<uint32_t>(r, n, base, cnt, width, lds.bytes, lds.chars, lane, hash, [&](auto const& valid, auto const& hv) {
         constexpr int N = sizeof(hv) / sizeof(hv[0]);
-        bool want[N], done[N];
-        uint32_t bucket[N], taken[N];
+        bool left[N], taken[N];
+        uint32_t bucket[N], home[N];
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-          want[k]   = valid[k] && hv[k] != 0u && part.holds(hv[k]);  // 282-286: zero hashes are dropped
+          left[k]   = valid[k] & (hv[k] != 0u) & part.holds(hv[k]);  // 282-286: zero hashes are dropped
           bucket[k] = set.home(hv[k]);
+          home[k]   = 0u;
         }
-        set.template insert_at<N>(want, hv, bucket, in, done, taken);
+        set.template place_at<N>(left, hv, bucket, home, mark, taken);
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-          bool const left      = want[k] && !done[k];
-          uint64_t const which = ballot64(left);
-          if (left) lds.later[later + lanes_below(which)] = hv[k];
-          later += static_cast<uint32_t>(__builtin_popcountll(which));
+          uint64_t const which = ballot64(left[k]);
+          if (which != 0) {
+            if (later + static_cast<uint32_t>(__builtin_popcountll(which)) > kLater) place_later();
+            if (left[k]) lds.later[later + lanes_below(which)] = hv[k];
+            later += static_cast<uint32_t>(__builtin_popcountll(which));
+          }
         }
       });
       if (!second) later1 = later;
-      if (later >= kWave / 2 || t + nwaves >= tiles) {
-        for (uint32_t i = lane; i < later; i += kWave) ok = set.insert(lds.later[i], i < later1 ? in1 : in2) && ok;
-        later = later1 = 0;
-      }
+      if (later >= kWave) place_later();
     }
+    place_later();
     return ok;
   }
   // very wide windows: bytes straight from global memory
@@ -287,7 +369,7 @@ __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2
       if (window_at(src[0], r + gpos, remaining, readable, gpos == 0, false, width, &hlen)) {
         uint32_t hv[1];
         hash(src, hlen, hv);
-        if (hv[0] != 0u && part.holds(hv[0])) ok = set.insert(hv[0], row == 0 ? in1 : in2) && ok;
+        if (hv[0] != 0u && part.holds(hv[0])) ok = place(set, hv[0], set.mark(row != 0)) && ok;
       }
     }
   }
@@ -298,59 +380,97 @@ template <int WAVES>
 struct PairScratch {
   TileLds tile[WAVES];
   uint32_t sums[3][WAVES];
-  uint32_t full;
+  uint32_t full;        // the last pair (counted from 1) whose packed set was full
+  uint32_t plain_full;  // whether the plain one was
 };
 
-// One row pair (or a part of it) by WAVES wavefronts with a set of `nslots` slots (a multiple of 32): clears
-// the set, inserts both rows, counts.  The counts are thread 0's; false (everywhere) when the set was full.
-template <int WAVES, bool IN_LDS>
-__device__ __forceinline__ bool count_pair(ColView const& c1, ColView const& c2, Pair const& pair, int32_t width, Part part, uint32_t* slots,
-                                           uint32_t* in1, uint32_t* in2, uint32_t nslots, PairScratch<WAVES>& scratch, uint32_t (&counts)[3])
+// The sums over a workgroup; what it writes to `scratch` the next pair overwrites behind a barrier of its own.
+template <int WAVES>
+__device__ __forceinline__ void add_up(uint32_t (&u)[3], PairScratch<WAVES>& scratch, int wave, int lane, uint32_t (&counts)[3])
 {
-  constexpr uint32_t kPairThreads = WAVES * kWave;
-  int const lane = lane_id();
-  int const wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
-  // (the arrays are 16-byte aligned: whole uint4 stores)
-  for (uint32_t i = threadIdx.x; i < nslots / 4; i += kPairThreads) reinterpret_cast<uint4*>(slots)[i] = make_uint4(0u, 0u, 0u, 0u);
-  for (uint32_t i = threadIdx.x; i < nslots / 32; i += kPairThreads) {
-    in1[i] = 0u;
-    in2[i] = 0u;
-  }
-  if (threadIdx.x == 0) scratch.full = 0u;
-  __syncthreads();
-  PairSet<IN_LDS> const set{slots, nslots / 4};
-  bool const ok = insert_pair(c1, c2, pair, width, set, in1, in2, part, scratch.tile[wave], wave, WAVES, lane);
-  if (!ok) scratch.full = 1u;
-  __syncthreads();
-  uint32_t u[3] = {0, 0, 0};
-  for (uint32_t i = threadIdx.x; i < nslots / 32; i += kPairThreads) {
-    uint32_t const a = set_word<IN_LDS>(&in1[i]), b = set_word<IN_LDS>(&in2[i]);
-    u[0] += __builtin_popcount(a);
-    u[1] += __builtin_popcount(b);
-    u[2] += __builtin_popcount(a & b);
-  }
-  if (IN_LDS) {  // (a wavefront's counts fit 16 bits: two sums in one)
-    u[0] = wave_inclusive_scan(u[0] | (u[1] << 16));
-    u[1] = u[0] >> 16;
-    u[0] &= 0xFFFFu;
-    u[2] = wave_inclusive_scan(u[2]);
-  } else {
-    for (int k = 0; k < 3; ++k) u[k] = wave_inclusive_scan(u[k]);
-  }
+  for (int k = 0; k < 3; ++k) u[k] = wave_inclusive_scan(u[k]);
   if (lane == kWave - 1) {
 #pragma unroll
     for (int k = 0; k < 3; ++k) scratch.sums[k][wave] = u[k];
   }
-  bool const full = scratch.full != 0u;
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     counts[k] = 0;
     for (int w = 0; w < WAVES; ++w) counts[k] += scratch.sums[k][w];
   }
-  // (the next pair's set is cleared by now at most: what it overwrites of `scratch` it overwrites after its own barrier)
+}
+template <int WAVES, bool IN_LDS>
+__device__ __forceinline__ bool count_pair_plain(ColView const& c1, ColView const& c2, Pair const& pair, int32_t width, Part part, PlainSet<IN_LDS> const& set,
+                                                 PairScratch<WAVES>& scratch, uint32_t (&counts)[3])
+{
+  constexpr uint32_t kPairThreads = WAVES * kWave;
+  int const lane = lane_id();
+  int const wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
+  uint32_t const words = set.buckets / 8;  // of bits
+  for (uint32_t i = threadIdx.x; i < 4 * set.buckets; i += kPairThreads) set.slots[i] = 0u;
+  for (uint32_t i = threadIdx.x; i < words; i += kPairThreads) {
+    set.in1[i] = 0u;
+    set.in2[i] = 0u;
+  }
+  if (threadIdx.x == 0) scratch.plain_full = 0u;
+  __syncthreads();
+  bool const ok = insert_pair(c1, c2, pair, width, set, part, scratch.tile[wave], wave, WAVES, lane);
+  if (!ok) scratch.plain_full = 1u;
+  __syncthreads();
+  uint32_t u[3] = {0, 0, 0};
+  for (uint32_t i = threadIdx.x; i < words; i += kPairThreads) {
+    uint32_t const a = set_word<IN_LDS>(&set.in1[i]), b = set_word<IN_LDS>(&set.in2[i]);
+    u[0] += __builtin_popcount(a);
+    u[1] += __builtin_popcount(b);
+    u[2] += __builtin_popcount(a & b);
+  }
+  bool const full = scratch.plain_full != 0u;
+  add_up(u, scratch, wave, lane, counts);
   return !full;
 }
+// The plain set where a packed one of `nslots` slots lies in LDS: sixteen of seventeen of its words are slots, the others the
+// bits.  (Room for the windows of the longest pair of a tier all the same: 0.8 * 17 / 16.)
+__device__ __forceinline__ PlainSet<true> plain_in(uint32_t* slots, uint32_t nslots)
+{
+  uint32_t const words = nslots / 34;  // of bits, of a row
+  return PlainSet<true>{slots, 8 * words, slots + 32 * words, slots + 33 * words};
+}
+// One row pair (or a part of it) by WAVES wavefronts with a set of `nslots` slots (a multiple of 32): inserts both rows, counts,
+// and leaves the set empty, as it was before (start_pairs).  `number`: of the pair among the workgroup's, from 1.  The counts are
+// thread 0's; false (everywhere) when the set was full.
+template <int WAVES>
+__device__ __forceinline__ void start_pairs(uint32_t* slots, uint32_t nslots, PairScratch<WAVES>& scratch)
+{
+  // (the slots are 16-byte aligned: whole uint4 stores)
+  for (uint32_t i = threadIdx.x; i < nslots / 4; i += WAVES * kWave) reinterpret_cast<uint4*>(slots)[i] = make_uint4(0u, 0u, 0u, 0u);
+  if (threadIdx.x == 0) scratch.full = 0u;
+  __syncthreads();
+}
+template <int WAVES>
+__device__ __forceinline__ bool count_pair(ColView const& c1, ColView const& c2, Pair const& pair, int32_t width, Part part, uint32_t* slots, uint32_t nslots,
+                                           PairScratch<WAVES>& scratch, uint32_t number, uint32_t (&counts)[3])
+{
+  int const lane = lane_id();
+  int const wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
+  bool const ok  = insert_pair(c1, c2, pair, width, PackedSet{slots, nslots / 4}, part, scratch.tile[wave], wave, WAVES, lane);
+  if (!ok) scratch.full = number;
+  __syncthreads();
+  bool const full = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(scratch.full))) == number;
+  PackedSet::Count in;
+  for (uint32_t i = threadIdx.x; i < nslots / 4; i += WAVES * kWave) {
+    uint4* const four = reinterpret_cast<uint4*>(slots) + i;
+    in.add(*four);
+    *four = make_uint4(0u, 0u, 0u, 0u);
+  }
+  uint32_t u[3];
+  in.get(u);
+  add_up(u, scratch, wave, lane, counts);
+  return !full;
+}
+// A pair that found its packed set full is marked in its list, and done once more with a plain set when the workgroup is through
+// with the others (not right away: the registers that takes are then not taken from the usual case).
+constexpr uint32_t kOnceMore = 0x80000000u;  // (rows are fewer)
 
 // Work lists in `work`: a header of 16 words -- [i] = pairs on list i, [kLists] = null rows of the result,
 // [8..9] = the most bytes a pair of the global list has (64 bits) -- then four counters (|A|, |B|, |A n B|, parts done) for
@@ -368,9 +488,9 @@ __device__ __forceinline__ void list_for_global(uint32_t* work, int64_t rows, in
 
 struct WaveSetLds {
   alignas(16) uint32_t slots[kSlots[0]];
-  uint32_t in1[kSlots[0] / 32], in2[kSlots[0] / 32];
   TileLds tile;
 };
+static_assert(kSlots[0] == PackedSet::kLeast, "every pair of a wavefront takes all slots");
 
 // A workgroup sizes `per_group` consecutive pairs at once (at most kThreads: threads <-> pairs, coalesced offset loads),
 // lists those that need more than a wavefront's own set for the later kernels with one atomic per list (atomics on one
@@ -412,56 +532,94 @@ __global__ void __launch_bounds__(kThreads) jaccard_wave_kernel(ColView c1, ColV
       if (list == kPartsList) reinterpret_cast<uint4*>(part_counters(work))[at] = make_uint4(0u, 0u, 0u, 0u);
       if (list == kGlobalList) atomicMax(reinterpret_cast<unsigned long long*>(&work[8]), static_cast<unsigned long long>(all));
     }
+    bool again = false;
     for (;;) {
       uint32_t t = 0;
       if (lane == 0) t = atomicAdd(&next, 1u);
       t = wave_bcast(t, 0);
       if (t >= solos) break;
-      uint32_t const pr     = solo[t];
-      Pair const q          = uniform_pair_at(c1, c2, pr);
-      uint32_t const nslots = slots_for(q.bytes(), kSlots[0]);
-      for (uint32_t i = lane; i < nslots / 4; i += kWave) reinterpret_cast<uint4*>(lds.slots)[i] = make_uint4(0u, 0u, 0u, 0u);
-      if (static_cast<uint32_t>(lane) < nslots / 32) {
-        lds.in1[lane] = 0u;
-        lds.in2[lane] = 0u;
+      uint32_t const pr = solo[t];
+      Pair const q      = uniform_pair_at(c1, c2, pr);
+      for (uint32_t i = lane; i < kSlots[0] / 4; i += kWave) reinterpret_cast<uint4*>(lds.slots)[i] = make_uint4(0u, 0u, 0u, 0u);
+      wave_sync();
+      bool const ok = insert_pair(c1, c2, q, width, PackedSet{lds.slots, kSlots[0] / 4}, Part{0, 1}, lds.tile, 0, 1, lane);
+      wave_sync();
+      if (ballot64(!ok) != 0) {
+        if (lane == 0) solo[t] = pr | kOnceMore;
+        again = true;
+        continue;
       }
+      PackedSet::Count in;
+      uint32_t u[3];
+      for (uint32_t i = lane; i < kSlots[0] / 4; i += kWave) in.add(reinterpret_cast<const uint4*>(lds.slots)[i]);
+      in.get(u);
+      uint32_t const u1 = wave_inclusive_scan(u[0] | u[1] << 16);  // (at most 1024 in either half)
+      u[2]              = wave_inclusive_scan(u[2]);
+      if (lane == kWave - 1) out[pr] = index_of(u1 & 0xFFFFu, u1 >> 16, u[2]);
       wave_sync();
-      PairSet<true> const set{lds.slots, nslots / 4};
-      insert_pair(c1, c2, q, width, set, lds.in1, lds.in2, Part{0, 1}, lds.tile, 0, 1, lane);  // (the set has room for every window)
+    }
+    if (!again) continue;
+    // what was marked so far: this wavefront's own at least
+    for (uint32_t t = 0; t < solos; ++t) {
       wave_sync();
-      uint32_t u1 = 0, both = 0;
-      if (static_cast<uint32_t>(lane) < nslots / 32) {  // at most 32 words of bits
-        uint32_t const a = lds.in1[lane], b = lds.in2[lane];
-        u1   = __builtin_popcount(a) | (static_cast<uint32_t>(__builtin_popcount(b)) << 16);
-        both = __builtin_popcount(a & b);
+      uint32_t const pr = solo[t] & ~kOnceMore;
+      uint32_t first    = 0;
+      if (lane == 0) first = atomicAnd(&solo[t], ~kOnceMore);  // (one of the wavefronts takes it)
+      if ((wave_bcast(first, 0) & kOnceMore) == 0u) continue;
+      for (uint32_t i = lane; i < kSlots[0]; i += kWave) lds.slots[i] = 0u;
+      wave_sync();
+      PlainSet<true> const plain = plain_in(lds.slots, kSlots[0]);
+      insert_pair(c1, c2, uniform_pair_at(c1, c2, pr), width, plain, Part{0, 1}, lds.tile, 0, 1, lane);
+      wave_sync();
+      uint32_t u[3] = {0, 0, 0};
+      for (uint32_t i = lane; i < plain.buckets / 8; i += kWave) {
+        u[0] += __builtin_popcount(plain.in1[i]);
+        u[1] += __builtin_popcount(plain.in2[i]);
+        u[2] += __builtin_popcount(plain.in1[i] & plain.in2[i]);
       }
-      u1   = wave_inclusive_scan(u1);  // (at most 1024 in either half)
-      both = wave_inclusive_scan(both);
-      if (lane == kWave - 1) out[pr] = index_of(u1 & 0xFFFFu, u1 >> 16, both);
-      wave_sync();
+      for (uint32_t& x : u) x = wave_inclusive_scan(x);
+      if (lane == kWave - 1) out[pr] = index_of(u[0], u[1], u[2]);
     }
   }
 }
 
 // The pairs of a tier's list, one workgroup of WAVES wavefronts and one set of SLOTS slots per pair.
 template <int TIER>
-__global__ void __launch_bounds__(kTierWaves[TIER] * kWave) jaccard_listed_kernel(ColView c1, ColView c2, int32_t width, float* __restrict__ out,
+__global__ void __launch_bounds__(kTierWaves[TIER] * kWave, kSimdWaves[TIER]) jaccard_listed_kernel(ColView c1, ColView c2, int32_t width, float* __restrict__ out,
                                                                                   uint32_t* __restrict__ work)
 {
   constexpr uint32_t SLOTS = kSlots[TIER];
   constexpr int WAVES      = kTierWaves[TIER];
   __shared__ alignas(16) uint32_t slots[SLOTS];
-  __shared__ uint32_t in1[SLOTS / 32], in2[SLOTS / 32];
   __shared__ PairScratch<WAVES> scratch;
   int64_t const rows   = c1.size;
   uint32_t const count = work[TIER - 1];
+  if (blockIdx.x >= count) return;
+  uint32_t* const entries = list_entries(work, TIER - 1, rows);
+  start_pairs(slots, SLOTS, scratch);
+  uint32_t number = 0;
+  bool again      = false;
   for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
-    uint32_t const r      = list_entries(work, TIER - 1, rows)[i];
-    Pair const pair       = uniform_pair_at(c1, c2, r);
-    uint32_t const nslots = slots_for(pair.bytes(), SLOTS);
+    uint32_t const r = entries[i];
+    Pair const pair  = uniform_pair_at(c1, c2, r);
     uint32_t counts[3];
-    count_pair<WAVES, true>(c1, c2, pair, width, Part{0, 1}, slots, in1, in2, nslots, scratch, counts);
-    if (threadIdx.x == 0) out[r] = index_of(counts[0], counts[1], counts[2]);
+    bool const ok = count_pair<WAVES>(c1, c2, pair, width, Part{0, 1}, slots, slots_for(pair.bytes(), SLOTS), scratch, ++number, counts);
+    if (!ok) {
+      again = true;
+      if (threadIdx.x == 0) entries[i] = r | kOnceMore;
+    } else if (threadIdx.x == 0) {
+      out[r] = index_of(counts[0], counts[1], counts[2]);
+    }
+  }
+  if (!again) return;
+  __syncthreads();  // (what thread 0 wrote is there)
+  for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
+    uint32_t const r = *const_cast<volatile uint32_t*>(&entries[i]);
+    if ((r & kOnceMore) == 0u) continue;
+    uint32_t counts[3];
+    count_pair_plain<WAVES>(c1, c2, uniform_pair_at(c1, c2, r & ~kOnceMore), width, Part{0, 1}, plain_in(slots, SLOTS), scratch, counts);
+    if (threadIdx.x == 0) out[r & ~kOnceMore] = index_of(counts[0], counts[1], counts[2]);
+    __syncthreads();
   }
 }
 
@@ -475,17 +633,19 @@ __global__ void __launch_bounds__(kTierWaves[kPartsTier] * kWave) jaccard_parts_
   constexpr uint32_t SLOTS = kSlots[kPartsTier];
   constexpr int WAVES      = kTierWaves[kPartsTier];
   __shared__ alignas(16) uint32_t slots[SLOTS];
-  __shared__ uint32_t in1[SLOTS / 32], in2[SLOTS / 32];
   __shared__ PairScratch<WAVES> scratch;
   int64_t const rows   = c1.size;
   uint32_t const count = work[kPartsList];
+  if (blockIdx.x >= count) return;
+  start_pairs(slots, SLOTS, scratch);
+  uint32_t number = 0;
   for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
     uint32_t const r  = list_entries(work, kPartsList, rows)[i];
     Pair const pair   = uniform_pair_at(c1, c2, r);
     Part const part{blockIdx.y, static_cast<uint32_t>(parts_of(pair.bytes()))};
     if (part.part >= part.parts) continue;
     uint32_t counts[3];
-    bool const ok = count_pair<WAVES, true>(c1, c2, pair, width, part, slots, in1, in2, SLOTS, scratch, counts);
+    bool const ok = count_pair<WAVES>(c1, c2, pair, width, part, slots, SLOTS, scratch, ++number, counts);
     if (threadIdx.x == 0) {
       uint32_t* const at = part_counters(work) + 4 * static_cast<int64_t>(i);
       for (int k = 0; k < 3; ++k) atomicAdd(&at[k], counts[k]);
@@ -517,7 +677,8 @@ __global__ void __launch_bounds__(kThreads) jaccard_global_kernel(ColView c1, Co
     Pair const pair     = uniform_pair_at(c1, c2, r);
     uint32_t const need = static_cast<uint32_t>(slots_for_global(pair.bytes()));
     uint32_t counts[3];
-    count_pair<kWaves, false>(c1, c2, pair, width, Part{0, 1}, mine, mine + table_slots, mine + table_slots + table_slots / 32, need, scratch, counts);
+    count_pair_plain<kWaves, false>(c1, c2, pair, width, Part{0, 1}, PlainSet<false>{mine, need / 4, mine + table_slots, mine + table_slots + table_slots / 32},
+                                    scratch, counts);
     if (threadIdx.x == 0) out[r] = index_of(counts[0], counts[1], counts[2]);
     __syncthreads();
   }

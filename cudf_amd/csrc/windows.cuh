@@ -168,13 +168,14 @@ __device__ __forceinline__ bool window_at(Src const& src, const uint8_t* g, int6
 // The windows that start in [base, base + cnt) of a row of n bytes (cnt <= kTile, 4 * width <= kHalo): `hash(src, bytes, h)`
 // of each (arrays of one source and hash or of two, of one length) goes to `sink(valid, h)`, which every lane of the wavefront
 // calls together, with arrays of one window per lane or of two (two chains of LDS reads and multiplies in flight instead of
-// one).  `bytes` and `chars` are the wavefront's own LDS.
-template <typename T, typename Hash, typename Sink>
-__device__ __forceinline__ void hash_tile_windows(const uint8_t* row, int64_t n, int64_t base, uint32_t cnt, int32_t width, uint32_t* bytes,
+// one).  `bytes` and `chars` are the wavefront's own LDS.  Place: a type for places in the row (32 bits take half the scalar
+// registers and instructions).
+template <typename T, typename Place, typename Hash, typename Sink>
+__device__ __forceinline__ void hash_tile_windows(const uint8_t* row, Place n, Place base, uint32_t cnt, int32_t width, uint32_t* bytes,
                                                   uint16_t* chars, int lane, Hash const& hash, Sink&& sink)
 {
   uint32_t const halo = static_cast<uint32_t>(width) * 4u;
-  uint32_t const len  = static_cast<uint32_t>(min(n - base, static_cast<int64_t>(cnt + halo)));
+  uint32_t const len  = static_cast<uint32_t>(min(n - base, static_cast<Place>(cnt + halo)));
   bool all_ascii;
   uint32_t const mis = stage_bytes(row, base, len, bytes, lane, &all_ascii);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -183,7 +184,7 @@ __device__ __forceinline__ void hash_tile_windows(const uint8_t* row, int64_t n,
   // In a tile of one-byte characters of a row of at least `width` bytes every window is `width` bytes long: the
   // hash then runs with a length that the compiler knows to be the same in every lane (its loops over the
   // blocks and the tail become scalar branches instead of masked ones).
-  bool const plain         = all_ascii && n >= static_cast<int64_t>(width);
+  bool const plain         = all_ascii && n >= static_cast<Place>(width);
   uint32_t const width_all = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(width));
   if (plain) {
     // (len and width fit 32 bits, and the last window of the row ends with it)
@@ -223,7 +224,7 @@ __device__ __forceinline__ void hash_tile_windows(const uint8_t* row, int64_t n,
         if (map.exact) {
           valid[0] = map.window(item, len, base == 0, width, chars, &p, &hlen);
         } else {
-          int64_t const gpos = base + p;
+          Place const gpos = base + static_cast<Place>(p);
           WordSrc const at(bytes, mis + p);
           valid[0] = window_at(at, row + gpos, n - gpos, len - p, gpos == 0, all_ascii, width, &hlen);
         }

@@ -30,6 +30,53 @@ def random_text(rng, n, alphabet=b"abcdefghijklmnopqrstuvwxyz"):
 
 
 @pytest.mark.parametrize("width", [2, 7, 40])
+def test_jaccard_sets_and_shares(nv, orc, width):
+    """Pairs one byte around the most that each set takes (4/5 of 1024, 4096, 7008, 15488 and 29440 slots), rows one window
+    around whole units of 64, and of very different lengths, so that a wavefront's share ends in the one or the other."""
+    rng = np.random.default_rng(width)
+    sizes = [(n * 4 // 5 + d) // 2 * 2 for n in (1024, 4096, 7008, 15488, 29440) for d in (0, 2)]
+    lens = [(n // 2 + d, n // 2 - d) for n in sizes for d in (0, 1, n // 3)]
+    lens += [(64 * k + width - 1 + d, 64 * m + width - 1 + e) for k, m in ((1, 0), (4, 5), (9, 23), (31, 16)) for d in (-1, 0, 1) for e in (-1, 0, 1)]
+    left = [random_text(rng, max(n, 0)).decode() for n, _ in lens]
+    right = [(a[: m // 2] + random_text(rng, max(m, 0) - len(a[: m // 2])).decode()) for a, (_, m) in zip(left, lens)]
+    h1, h2 = HostStringsColumn.from_pylist(left), HostStringsColumn.from_pylist(right)
+    got, exp = nv.jaccard_index(dev(nv, h1), dev(nv, h2), width).to_host(), orc.jaccard_index(h1, h2, width, nthreads=8)
+    assert np.array_equal(got.values.view(np.uint32), exp.values.view(np.uint32))
+
+
+def home_buckets(words, buckets):
+    """Where windows of four bytes belong in a set: the top of the product of their hash (MurmurHash3_x86_32, seed 0, without
+    the final mix)."""
+    with np.errstate(over="ignore"):
+        k = words * np.uint32(0xCC9E2D51)
+        k = (k << np.uint32(15) | k >> np.uint32(17)) * np.uint32(0x1B873593)
+        h = ((k << np.uint32(13) | k >> np.uint32(19)) * np.uint32(5) + np.uint32(0xE6546B64)) ^ np.uint32(4)
+        return (h * np.uint32(0x9E3779B1)).astype(np.uint64) * np.uint64(buckets) >> np.uint64(32)
+
+
+@pytest.mark.parametrize("count", [90, 190, 450, 1000])
+def test_jaccard_values_of_one_bucket(nv, orc, count):
+    """Words that all belong in one bucket: 90 that find a place within the 64 buckets that a packed set looks at from there,
+    and more than these hold (the last is 111, 179 and 393 buckets from home), so that the pair is done with a plain set,
+    among pairs that are not."""
+    rng = np.random.default_rng(count)
+    letters = np.arange(97, 123, dtype=np.uint32)
+    words = (letters[:, None, None, None] | letters[:, None, None] << 8 | letters[:, None] << 16 | letters << 24).astype(np.uint32).ravel()
+    slots = min({90: 1024, 190: 1024, 450: 4096, 1000: 15488}[count], max(1024, (2 * 4 * count + 63) // 32 * 32))
+    home = home_buckets(words, slots // 4)
+    near = words[home // max(1, slots // 4 // 256) == 77 % (slots // 4)][:count]
+    assert len(near) > 80
+    text = near.view(np.uint8).reshape(-1, 4)
+    row = lambda pick: bytes(text[pick].ravel()).decode()
+    n = len(text)
+    left = [row(np.arange(n * 3 // 4)), "some other text", row(np.arange(n // 2))] * 3
+    right = [row(np.arange(n * 3 // 4, n)), "another text", row(np.arange(n // 2, n))] * 3
+    h1, h2 = HostStringsColumn.from_pylist(left), HostStringsColumn.from_pylist(right)
+    got, exp = nv.jaccard_index(dev(nv, h1), dev(nv, h2), 4).to_host(), orc.jaccard_index(h1, h2, 4, nthreads=8)
+    assert np.array_equal(got.values.view(np.uint32), exp.values.view(np.uint32))
+
+
+@pytest.mark.parametrize("width", [2, 7, 40])
 def test_jaccard_pair_sizes(nv, orc, width):
     """Pairs one byte around the most that each set takes (4/5 of 1024, 4096, 8064, 14336 and 29440 slots), around one
     and several parts of 20,000 bytes, and around the most parts (16); no window repeats, so the sets are as full as they get."""
