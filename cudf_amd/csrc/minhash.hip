@@ -510,23 +510,16 @@ __device__ __forceinline__ void gather(WaveLds<uint32_t>& lds, bool const (&vali
 template <int N>
 __device__ __forceinline__ void gather(WaveLds<uint64_t>& lds, bool const (&valid)[N], uint64_t const (&hv)[N], uint32_t* count)
 {
-  uint16_t* at[N];
-  uint32_t place[N];
-  bool fresh[N];
+  // (one after the other: the second of a lane's windows finds those of the first, 20,011 long rows 2759 -> 2711 us)
 #pragma unroll
   for (int n = 0; n < N; ++n) {
-    at[n]    = &lds.recent[static_cast<uint32_t>(hv[n]) & (kRecentEntries - 1)];
-    place[n] = *at[n];
-  }
-#pragma unroll
-  for (int n = 0; n < N; ++n) fresh[n] = valid[n] && lds.hashes[place[n]] != hv[n];
-#pragma unroll
-  for (int n = 0; n < N; ++n) {
-    uint64_t const vm = ballot64(fresh[n]);
-    if (fresh[n]) {
-      place[n]             = *count + lanes_below(vm);
-      lds.hashes[place[n]] = hv[n];
-      *at[n]               = static_cast<uint16_t>(place[n]);
+    uint16_t* const at = &lds.recent[static_cast<uint32_t>(hv[n]) & (kRecentEntries - 1)];
+    bool const fresh   = valid[n] && lds.hashes[*at] != hv[n];
+    uint64_t const vm  = ballot64(fresh);
+    if (fresh) {
+      uint32_t const place = *count + lanes_below(vm);
+      lds.hashes[place]    = hv[n];
+      *at                  = static_cast<uint16_t>(place);
     }
     *count += static_cast<uint32_t>(__builtin_popcountll(vm));
   }
