@@ -76,7 +76,6 @@ struct PackedSet {
   static constexpr uint32_t kSame     = 0x7EFFFFFFu;  // value and distance
   static constexpr uint32_t kLeast    = 1024;         // slots
   using Mark                          = uint32_t;
-  using Place                         = int32_t;      // in a row, where the pairs are short
   uint32_t* slots;  // 0 = empty; 16-byte aligned
   uint32_t buckets;
 
@@ -160,7 +159,6 @@ template <bool IN_LDS>
 struct PlainSet {
   static constexpr uint32_t kFar = 0xFFFFFFFFu;
   using Mark                     = uint32_t*;
-  using Place                    = int64_t;
   uint32_t* slots;
   uint32_t buckets;
   uint32_t *in1, *in2;
@@ -308,11 +306,10 @@ __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2
   auto const hash = [](auto const& src, uint32_t len, auto& h) { murmur3_x86_32_unmixed(src, len, 0u, h); };  // jaccard.cu:258: seed 0
   bool ok         = true;
   if (static_cast<int64_t>(width) * 4 <= kHalo) {
-    using Place        = typename Set::Place;
-    Place const n1 = static_cast<Place>(pair.n1), n2 = static_cast<Place>(pair.n2);
+    int32_t const n1 = static_cast<int32_t>(pair.n1), n2 = static_cast<int32_t>(pair.n2);  // (1.43 GB together at most)
     const uint8_t *const row1 = c1.chars + pair.o1, *const row2 = c2.chars + pair.o2;
-    Place const units1 = (n1 + kWave - 1) / kWave, units = units1 + (n2 + kWave - 1) / kWave;
-    Place const last   = units * (wave + 1) / nwaves;
+    int32_t const units1 = (n1 + kWave - 1) / kWave, units = units1 + (n2 + kWave - 1) / kWave;
+    int32_t const last   = static_cast<int32_t>(static_cast<int64_t>(units) * (wave + 1) / nwaves);
     uint32_t later = 0, later1 = 0;  // hashes put aside, and how many of them (the first ones) are row 1's: the same in every lane
     bool second    = false;
     auto const place_later = [&] {
@@ -320,16 +317,16 @@ __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2
       for (uint32_t i = lane; i < later; i += kWave) ok = place(set, lds.later[i], set.mark(i >= later1)) && ok;
       later = later1 = 0;
     };
-    for (Place unit = units * wave / nwaves; unit < last;) {
+    for (int32_t unit = static_cast<int32_t>(static_cast<int64_t>(units) * wave / nwaves); unit < last;) {
       second                 = unit >= units1;
       const uint8_t* const r = second ? row2 : row1;
-      Place const n          = second ? n2 : n1;
+      int32_t const n        = second ? n2 : n1;
       auto const mark        = set.mark(second);
-      Place const base       = (second ? unit - units1 : unit) * kWave;
-      Place const end        = min(unit + kTile / kWave, second ? last : min(last, units1));
+      int32_t const base     = (second ? unit - units1 : unit) * kWave;
+      int32_t const end      = min(unit + kTile / kWave, second ? last : min(last, units1));
       uint32_t const cnt     = static_cast<uint32_t>(min((end - unit) * kWave, n - base));
       unit                   = end;
-      hash_tile_windows<uint32_t>(r, n, base, cnt, width, lds.bytes, lds.chars, lane, hash, [&](auto const& valid, auto const& hv) {
+      hash_tile_windows<uint32_t>(r, n, 0, true, base, cnt, width, lds.bytes, lds.chars, lane, hash, [&](auto const& valid, auto const& hv) {
         constexpr int N = sizeof(hv) / sizeof(hv[0]);
         bool left[N], taken[N];
         uint32_t bucket[N], home[N];

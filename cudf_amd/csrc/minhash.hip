@@ -566,39 +566,41 @@ struct TextRows {
   __device__ __forceinline__ void process(int64_t i, int64_t begin, int64_t end, Minima& minima, Lds& lds, int lane) const
   {
     using H              = HashTraits<T>;
-    int64_t const o      = col.off(i);
-    int64_t const n      = col.off(i + 1) - o;
-    const uint8_t* const row = col.chars + o;
-    // usual case: a window (<= 4*width bytes) fits the halo staged behind every tile
-    bool const narrow  = static_cast<int64_t>(width) * 4 <= kHalo;
-    int64_t const step = narrow ? kTile : kWave;
+    int64_t const o          = col.off(i);
+    int64_t const left       = col.off(i + 1) - o - begin;  // bytes from the part's first to the row's last
+    const uint8_t* const row = col.chars + o + begin;
+    int32_t const span       = static_cast<int32_t>(end - begin);
     forget_hashes(lds, lane);  // (the wave barrier after the first tile's staging comes before the first look)
-    uint32_t count = 0;  // hashes that wait to be folded (wave-uniform)
-    for (int64_t base = begin; base < end; base += step) {
+    uint32_t count = 0;        // hashes that wait to be folded (wave-uniform)
+    // usual case: a window (<= 4*width bytes) fits the halo staged behind every tile
+    bool const narrow = static_cast<int64_t>(width) * 4 <= kHalo;
+    int32_t const n   = static_cast<int32_t>(min(left, static_cast<int64_t>(1) << 30));
+    for (int32_t base = 0; base < span;) {
       if (narrow) {
-        uint32_t const cnt = static_cast<uint32_t>(min(static_cast<int64_t>(kTile), end - base));
+        uint32_t const cnt = static_cast<uint32_t>(min(kTile, span - base));
         auto const hash    = [seed = seed](auto const& src, uint32_t len, auto& h) { H::hash(src, len, seed, h); };
-        hash_tile_windows<T>(row, n, base, cnt, width, lds.bytes, lds.chars, lane, hash, [&](auto const& valid, auto const& hv) {
-          gather(lds, valid, hv, &count);
-        });
+        hash_tile_windows<T>(row, n, left - n, begin == 0, base, cnt, width, lds.bytes, lds.chars, lane, hash,
+                             [&](auto const& valid, auto const& hv) { gather(lds, valid, hv, &count); });
+        base += kTile;
       } else {
         // very wide windows: 64 starts at a time, bytes read straight from global memory
-        int64_t const gpos = base + lane;
-        bool valid         = false;
-        T hv[1]            = {0};
-        if (gpos < end) {
-          int64_t const remaining = n - gpos;
-          BoundedSrc const src[1] = {{row + gpos, remaining}};
+        int32_t const pos = base + lane;
+        bool valid        = false;
+        T hv[1]           = {0};
+        if (pos < span) {
+          int64_t const remaining = left - pos;
+          BoundedSrc const src[1] = {{row + pos, remaining}};
           uint32_t hlen;
           uint32_t const readable = static_cast<uint32_t>(min(remaining, static_cast<int64_t>(width) * 4));
-          valid = window_at(src[0], row + gpos, remaining, readable, gpos == 0, false, width, &hlen);
+          valid = window_at(src[0], row + pos, remaining, readable, begin == 0 && pos == 0, false, width, &hlen);
           if (valid) H::hash(src, hlen, seed, hv);
         }
         uint64_t const vm = ballot64(valid);
         if (valid) lds.hashes[count + lanes_below(vm)] = hv[0];
         count += static_cast<uint32_t>(__builtin_popcountll(vm));
+        base += kWave;
       }
-      count = minima.fold(lds.hashes, count, base + step >= end);
+      count = minima.fold(lds.hashes, count, base >= span);
     }
   }
 };

@@ -165,44 +165,45 @@ __device__ __forceinline__ bool window_at(Src const& src, const uint8_t* g, int6
   return first || left <= 0;
 }
 
-// The windows that start in [base, base + cnt) of a row of n bytes (cnt <= kTile, 4 * width <= kHalo): `hash(src, bytes, h)`
-// of each (arrays of one source and hash or of two, of one length) goes to `sink(valid, h)`, which every lane of the wavefront
-// calls together, with arrays of one window per lane or of two (two chains of LDS reads and multiplies in flight instead of
-// one).  `bytes` and `chars` are the wavefront's own LDS.  Place: a type for places in the row (32 bits take half the scalar
-// registers and instructions).
-template <typename T, typename Place, typename Hash, typename Sink>
-__device__ __forceinline__ void hash_tile_windows(const uint8_t* row, Place n, Place base, uint32_t cnt, int32_t width, uint32_t* bytes,
-                                                  uint16_t* chars, int lane, Hash const& hash, Sink&& sink)
+// The windows that start in [base, base + cnt) of (the rest of) a row, n bytes from `row` on (cnt <= kTile, 4 * width <= kHalo):
+// `hash(src, bytes, h)` of each (arrays of one source and hash or of two, of one length) goes to `sink(valid, h)`, which every
+// lane of the wavefront calls together, with arrays of one window per lane or of two (two chains of LDS reads and multiplies
+// in flight instead of one).  `bytes` and `chars` are the wavefront's own LDS.  starts: `row` is the row's first byte.  Places
+// have 32 bits, which take half the scalar registers and instructions; `beyond` more bytes than n belong to a row that is
+// longer.
+template <typename T, typename Hash, typename Sink>
+__device__ __forceinline__ void hash_tile_windows(const uint8_t* row, int32_t n, int64_t beyond, bool starts, int32_t base, uint32_t cnt, int32_t width,
+                                                  uint32_t* bytes, uint16_t* chars, int lane, Hash const& hash, Sink&& sink)
 {
   uint32_t const halo = static_cast<uint32_t>(width) * 4u;
-  uint32_t const len  = static_cast<uint32_t>(min(n - base, static_cast<Place>(cnt + halo)));
+  uint32_t const len  = min(static_cast<uint32_t>(n - base), cnt + halo);
   bool all_ascii;
   uint32_t const mis = stage_bytes(row, base, len, bytes, lane, &all_ascii);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  // In a tile of one-byte characters of a row of at least `width` bytes every window is `width` bytes long: the
+  // In a tile of one-byte characters of a row that has `width` bytes and more every window is `width` bytes long: the
   // hash then runs with a length that the compiler knows to be the same in every lane (its loops over the
   // blocks and the tail become scalar branches instead of masked ones).
-  bool const plain         = all_ascii && n >= static_cast<Place>(width);
+  bool const plain         = all_ascii && (!starts || n >= width);
   uint32_t const width_all = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(width));
   if (plain) {
-    // (len and width fit 32 bits, and the last window of the row ends with it)
-    uint32_t const starts = min(cnt, len - min(len, width_all - 1u));
+    // (the last window of the row ends with it)
+    uint32_t const starts_here = min(cnt, len - min(len, width_all - 1u));
     uint32_t q = 0;
-    for (; q + kWave < starts; q += 2 * kWave) {
+    for (; q + kWave < starts_here; q += 2 * kWave) {
       // (a lane beyond the last window hashes the bytes of that one: no branch)
       uint32_t const p     = q + lane;
-      bool const valid[2]  = {true, p + kWave < starts};
-      WordSrc const src[2] = {WordSrc(bytes, mis + p), WordSrc(bytes, mis + min(p + kWave, starts - 1u))};
+      bool const valid[2]  = {true, p + kWave < starts_here};
+      WordSrc const src[2] = {WordSrc(bytes, mis + p), WordSrc(bytes, mis + min(p + kWave, starts_here - 1u))};
       T hv[2];
       hash(src, width_all, hv);
       sink(valid, hv);
     }
-    if (q < starts) {
+    if (q < starts_here) {
       uint32_t const p     = q + lane;
-      bool const valid[1]  = {p < starts};
-      WordSrc const src[1] = {WordSrc(bytes, mis + min(p, starts - 1u))};
+      bool const valid[1]  = {p < starts_here};
+      WordSrc const src[1] = {WordSrc(bytes, mis + min(p, starts_here - 1u))};
       T hv[1];
       hash(src, width_all, hv);
       sink(valid, hv);
@@ -213,7 +214,7 @@ __device__ __forceinline__ void hash_tile_windows(const uint8_t* row, Place n, P
     // walking.  (A row shorter than `width` comes here too, whatever its bytes.)
     CharMap map;
     map.exact = false;
-    if (!all_ascii) map.build(bytes, mis, len, cnt, base + len == n, chars, lane);
+    if (!all_ascii) map.build(bytes, mis, len, cnt, base + static_cast<int32_t>(len) == n, chars, lane);
     uint32_t const items = map.exact ? map.windows : cnt;  // characters, or byte positions
     for (uint32_t q = 0; q < items; q += kWave) {
       uint32_t const item = q + lane;
@@ -221,12 +222,13 @@ __device__ __forceinline__ void hash_tile_windows(const uint8_t* row, Place n, P
       T hv[1]             = {0};
       if (item < items) {
         uint32_t p = item, hlen;
+        bool const first = starts && base == 0;
         if (map.exact) {
-          valid[0] = map.window(item, len, base == 0, width, chars, &p, &hlen);
+          valid[0] = map.window(item, len, first, width, chars, &p, &hlen);
         } else {
-          Place const gpos = base + static_cast<Place>(p);
           WordSrc const at(bytes, mis + p);
-          valid[0] = window_at(at, row + gpos, n - gpos, len - p, gpos == 0, all_ascii, width, &hlen);
+          int32_t const here = base + static_cast<int32_t>(p);
+          valid[0] = window_at(at, row + here, n - here + beyond, len - p, first && p == 0, all_ascii, width, &hlen);
         }
         WordSrc const src[1] = {WordSrc(bytes, mis + p)};
         if (valid[0]) hash(src, hlen, hv);
