@@ -317,16 +317,42 @@ __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2
       for (uint32_t i = lane; i < later; i += kWave) ok = place(set, lds.later[i], set.mark(i >= later1)) && ok;
       later = later1 = 0;
     };
-    for (int32_t unit = static_cast<int32_t>(static_cast<int64_t>(units) * wave / nwaves); unit < last;) {
-      second                 = unit >= units1;
-      const uint8_t* const r = second ? row2 : row1;
-      int32_t const n        = second ? n2 : n1;
-      auto const mark        = set.mark(second);
-      int32_t const base     = (second ? unit - units1 : unit) * kWave;
-      int32_t const end      = min(unit + kTile / kWave, second ? last : min(last, units1));
-      uint32_t const cnt     = static_cast<uint32_t>(min((end - unit) * kWave, n - base));
-      unit                   = end;
-      hash_tile_windows<uint32_t>(r, n, 0, true, base, cnt, width, lds.bytes, lds.chars, lane, hash, [&](auto const& valid, auto const& hv) {
+    struct At {
+      bool second;
+      const uint8_t* row;
+      int32_t n, base, end;
+      uint32_t cnt;
+    };
+    auto const tile_at = [&](int32_t unit) {
+      At a;
+      a.second = unit >= units1;
+      a.row    = a.second ? row2 : row1;
+      a.n      = a.second ? n2 : n1;
+      a.base   = (a.second ? unit - units1 : unit) * kWave;
+      a.end    = min(unit + kTile / kWave, a.second ? last : min(last, units1));
+      a.cnt    = static_cast<uint32_t>(min((a.end - unit) * kWave, a.n - a.base));
+      return a;
+    };
+    TileBytes tile;  // asked for a tile ahead
+    auto const fetch = [&](At const& a) { tile.fetch(a.row + a.base, tile_length(a.n, a.base, a.cnt, width), lane); };
+    int32_t const first = static_cast<int32_t>(static_cast<int64_t>(units) * wave / nwaves);
+    At ahead{};
+    if (first < last) {
+      ahead = tile_at(first);
+      fetch(ahead);
+    }
+    for (int32_t unit = first; unit < last;) {
+      At const a      = ahead;
+      second          = a.second;
+      auto const mark = set.mark(second);
+      unit            = a.end;
+      auto const next = [&] {
+        if (unit < last) {
+          ahead = tile_at(unit);
+          fetch(ahead);
+        }
+      };
+      hash_tile_windows<uint32_t>(tile, next, a.row, a.n, 0, true, a.base, a.cnt, width, lds.bytes, lds.chars, lane, hash, [&](auto const& valid, auto const& hv) {
         constexpr int N = sizeof(hv) / sizeof(hv[0]);
         bool left[N], taken[N];
         uint32_t bucket[N], home[N];

@@ -575,11 +575,18 @@ struct TextRows {
     // usual case: a window (<= 4*width bytes) fits the halo staged behind every tile
     bool const narrow = static_cast<int64_t>(width) * 4 <= kHalo;
     int32_t const n   = static_cast<int32_t>(min(left, static_cast<int64_t>(1) << 30));
+    auto const starts_at = [&](int32_t base) { return static_cast<uint32_t>(min(kTile, span - base)); };
+    TileBytes tile;  // asked for a tile ahead
+    auto const fetch = [&](int32_t base) { tile.fetch(row + base, tile_length(n, base, starts_at(base), width), lane); };
+    if (narrow) fetch(0);
     for (int32_t base = 0; base < span;) {
       if (narrow) {
-        uint32_t const cnt = static_cast<uint32_t>(min(kTile, span - base));
+        uint32_t const cnt = starts_at(base);
         auto const hash    = [seed = seed](auto const& src, uint32_t len, auto& h) { H::hash(src, len, seed, h); };
-        hash_tile_windows<T>(row, n, left - n, begin == 0, base, cnt, width, lds.bytes, lds.chars, lane, hash,
+        auto const next    = [&] {
+          if (base + kTile < span) fetch(base + kTile);
+        };
+        hash_tile_windows<T>(tile, next, row, n, left - n, begin == 0, base, cnt, width, lds.bytes, lds.chars, lane, hash,
                              [&](auto const& valid, auto const& hv) { gather(lds, valid, hv, &count); });
         base += kTile;
       } else {
@@ -711,8 +718,7 @@ struct RunRows {
       int64_t const span_end   = static_cast<int64_t>(wave_bcast64(static_cast<uint64_t>(eo), kWave - 1));
       if (base + kWave < end) ask(base + kWave);
       if (sizeof(T) == 4 && span_end - span_begin <= static_cast<int64_t>(kRunStageBytes)) {
-        bool ascii;
-        uint32_t const mis = stage_bytes(col.child.chars, span_begin, static_cast<uint32_t>(span_end - span_begin), lds.bytes, lane, &ascii);
+        uint32_t const mis = stage_bytes(col.child.chars, span_begin, static_cast<uint32_t>(span_end - span_begin), lds.bytes, lane);
         wave_lds_fence();
         WordSrc const src[1] = {WordSrc(lds.bytes, mis + static_cast<uint32_t>(run_begin - span_begin))};
         if (valid) H::hash(src, run, seed, hv);

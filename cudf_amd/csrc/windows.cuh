@@ -40,23 +40,36 @@ struct WaveLds {
   uint16_t chars[kCharList];  // where the characters of the staged bytes start, in order (see CharMap)
 };
 
-// Stage row bytes [base, base+len) into dst (16-byte aligned); returns the byte offset of `base` inside it.
-// Only aligned 16-byte blocks that overlap the range are read (a lane a block: one load and one LDS write for a tile).
-// *all_ascii: no byte of these blocks has its top bit set (wave-uniform); a byte beyond ASCII next to the range costs
-// the caller its shorter way and nothing else.
-__device__ __forceinline__ uint32_t stage_bytes(const uint8_t* row, int64_t base, uint32_t len, uint32_t* dst, int lane, bool* all_ascii)
+// The aligned 16-byte blocks that bytes [at, at + len) lie in, a lane a block (at most 64 of them): fetch() asks for them and does
+// not wait, stage() puts them into LDS.  Only blocks that overlap the range are read.
+struct TileBytes {
+  uint4 block;
+  uint32_t mis;  // byte offset of `at` in the first block
+  uint32_t blocks;
+  __device__ __forceinline__ void fetch(const uint8_t* at, uint32_t len, int lane)
+  {
+    mis    = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(at) & 15u);
+    blocks = (mis + len + 15u) >> 4;
+    block  = make_uint4(0u, 0u, 0u, 0u);
+    if (static_cast<uint32_t>(lane) < blocks) block = reinterpret_cast<const uint4*>(at - mis)[lane];
+  }
+  // dst: 16-byte aligned.  *all_ascii: no byte of these blocks has its top bit set (wave-uniform); a byte beyond ASCII next to
+  // the range costs the caller its shorter way and nothing else.
+  __device__ __forceinline__ void stage(uint32_t* dst, int lane, bool* all_ascii) const
+  {
+    if (static_cast<uint32_t>(lane) < blocks) reinterpret_cast<uint4*>(dst)[lane] = block;
+    *all_ascii = ballot64(((block.x | block.y | block.z | block.w) & 0x80808080u) != 0) == 0;
+  }
+};
+
+// Stage row bytes [base, base+len), any number of them, into dst (16-byte aligned); returns the byte offset of `base` inside it.
+__device__ __forceinline__ uint32_t stage_bytes(const uint8_t* row, int64_t base, uint32_t len, uint32_t* dst, int lane)
 {
   const uint8_t* g   = row + base;
   uint32_t const mis = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(g) & 15u);
   const uint4* ap    = reinterpret_cast<const uint4*>(g - mis);
   uint32_t const nb  = (mis + len + 15u) >> 4;
-  uint32_t hibits    = 0;
-  for (uint32_t i = lane; i < nb; i += kWave) {
-    uint4 const v                     = ap[i];
-    reinterpret_cast<uint4*>(dst)[i]  = v;
-    hibits |= v.x | v.y | v.z | v.w;
-  }
-  *all_ascii = ballot64((hibits & 0x80808080u) != 0) == 0;
+  for (uint32_t i = lane; i < nb; i += kWave) reinterpret_cast<uint4*>(dst)[i] = ap[i];
   return mis;
 }
 
@@ -170,15 +183,20 @@ __device__ __forceinline__ bool window_at(Src const& src, const uint8_t* g, int6
 // lane of the wavefront calls together, with arrays of one window per lane or of two (two chains of LDS reads and multiplies
 // in flight instead of one).  `bytes` and `chars` are the wavefront's own LDS.  starts: `row` is the row's first byte.  Places
 // have 32 bits, which take half the scalar registers and instructions; `beyond` more bytes than n belong to a row that is
-// longer.
-template <typename T, typename Hash, typename Sink>
-__device__ __forceinline__ void hash_tile_windows(const uint8_t* row, int32_t n, int64_t beyond, bool starts, int32_t base, uint32_t cnt, int32_t width,
-                                                  uint32_t* bytes, uint16_t* chars, int lane, Hash const& hash, Sink&& sink)
+// longer.  tile: the row's bytes from base on, tile_length() of them; when they are in LDS, next() may ask for others.
+__device__ __forceinline__ uint32_t tile_length(int32_t n, int32_t base, uint32_t cnt, int32_t width)
 {
-  uint32_t const halo = static_cast<uint32_t>(width) * 4u;
-  uint32_t const len  = min(static_cast<uint32_t>(n - base), cnt + halo);
+  return min(static_cast<uint32_t>(n - base), cnt + static_cast<uint32_t>(width) * 4u);
+}
+template <typename T, typename Next, typename Hash, typename Sink>
+__device__ __forceinline__ void hash_tile_windows(TileBytes& tile, Next&& next, const uint8_t* row, int32_t n, int64_t beyond, bool starts, int32_t base, uint32_t cnt,
+                                                  int32_t width, uint32_t* bytes, uint16_t* chars, int lane, Hash const& hash, Sink&& sink)
+{
+  uint32_t const len = tile_length(n, base, cnt, width);
+  uint32_t const mis = tile.mis;
   bool all_ascii;
-  uint32_t const mis = stage_bytes(row, base, len, bytes, lane, &all_ascii);
+  tile.stage(bytes, lane, &all_ascii);
+  next();
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
