@@ -160,57 +160,107 @@ struct Owned {
 template <bool S>
 __device__ __forceinline__ uint8_t& flat_slot(NormLds<S>& lds, int at) { return lds.slot[at % 3][at / 3]; }
 
-// Compares the candidate in flat slots [from, to] (spaces and empty slots skipped, one byte per character) with
-// special token `i`: < 0, 0, > 0 as the candidate sorts before, equal to or after it.
-template <bool S>
-__device__ int compare_candidate(NormLds<S>& lds, int from, int to, NormTables const& t, int32_t i)
-{
-  const uint8_t* tok = t.token_chars + t.token_offset[i];
-  int32_t const tl   = t.token_offset[i + 1] - t.token_offset[i];
-  int32_t j          = 0;
-  for (int at = from; at <= to; ++at) {
-    uint32_t const c = flat_slot(lds, at);
-    if (c == 0u || c == 0x20u) continue;
-    if (j >= tl) return 1;
-    uint32_t const b = tok[j++];
-    if (c != b) return c < b ? -1 : 1;
-  }
-  return j < tl ? -1 : 0;
-}
-
 __device__ __forceinline__ bool has_byte(uint32_t v, uint32_t byte)
 {
   uint32_t const x = v ^ (byte * 0x01010101u);
   return ((x - 0x01010101u) & ~x & 0x80808080u) != 0u;
 }
 
+// Bit 7 of every byte of v that is `byte`.
+__device__ __forceinline__ uint64_t bytes_equal(uint64_t v, uint32_t byte)
+{
+  uint64_t const low = 0x7F7F7F7F7F7F7F7Full, x = v ^ (byte * 0x0101010101010101ull);
+  return ~(((x & low) + low) | x | low);
+}
+
+// What may be a special token: its characters, spaces and empty slots left out, eight to a word and the first on top.
+constexpr int kCandidateWords = 3;
+struct Candidate {
+  uint64_t word[kCandidateWords];
+  int32_t size;  // 18 at most
+};
+
+// < 0, 0, > 0 as the candidate sorts before, equal to or after special token `i`.  (Behind their ends both are zeros: where
+// those decide, the shorter one is the smaller.)
+__device__ __forceinline__ int compare_candidate(Candidate const& c, NormTables const& t, int32_t i)
+{
+  int32_t const at = t.token_offset[i], size = t.token_offset[i + 1] - at;
+#pragma unroll
+  for (int w = 0; w < kCandidateWords; ++w) {
+    uint64_t token = 0;
+    if (8 * w < size) {
+      __builtin_memcpy(&token, t.token_chars + at + 8 * w, 8);  // (there are eight bytes more than the tokens')
+      token = __builtin_bswap64(token);
+      if (size - 8 * w < 8) token &= ~0ull << (8 * (8 * w + 8 - size));
+    }
+    if (c.word[w] != token) return c.word[w] < token ? -1 : 1;
+  }
+  return c.size < size ? -1 : c.size > size ? 1 : 0;
+}
+
 // Whether a special token opens at slot index i (its slot 1 holds '['): the flat slot of its ']' if so, else -1.
-// special_tokens_kernel, cpp/src/text/normalize.cu:283-301.
+// special_tokens_kernel, cpp/src/text/normalize.cu:283-301.  The 21 slots of seven positions are read at once and searched
+// in registers: one by one from LDS, with a token's bytes one by one from memory, most of the time of text with tokens was
+// that of the reads (200 MB with a token every 280 bytes 3778 -> 2747 us, every 2800 bytes 2039 -> 1706).
 template <bool S>
 __device__ int token_opens_at(NormLds<S>& lds, NormTables const& t, int i)
 {
   if (lds.slot[1][i] != '[') return -1;
-  int const from = 3 * i + 1;
-  int to         = -1;
-  for (int at = from + 1; at < from + 18; ++at) {
-    if (flat_slot(lds, at) == ']') {
-      to = at;
-      break;
+  uint64_t slot[3], closing[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    __builtin_memcpy(&slot[k], &lds.slot[k][i], 8);
+    closing[k] = bytes_equal(slot[k], ']');
+  }
+  // the first ']' of the 17 slots after the '[' and the one behind it: slot k of position p is number 3 * p + k, numbers 2..18
+  closing[0] &= 0x00FFFFFFFFFFFF00ull;
+  closing[1] &= 0x0000FFFFFFFFFF00ull;
+  closing[2] &= 0x0000FFFFFFFFFFFFull;
+  int last = 99;
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    if (closing[k] != 0) last = min(last, 3 * (__builtin_ctzll(closing[k]) >> 3) + k);
+  if (last == 99) return -1;
+  Candidate c{};
+  uint64_t word = 0;
+  for (int at = 1, k = 1; at <= last; ++at) {
+    uint32_t const b = static_cast<uint32_t>(k == 0 ? slot[0] : k == 1 ? slot[1] : slot[2]) & 0xFFu;
+    if (b != 0u && b != 0x20u) {
+      word = (word << 8) | b;
+      ++c.size;
+      if (c.size == 8) {
+        c.word[0] = word;
+        word      = 0;
+      } else if (c.size == 16) {
+        c.word[1] = word;
+        word      = 0;
+      }
+    }
+    if (++k == 3) {
+      k = 0;
+      slot[0] >>= 8;
+      slot[1] >>= 8;
+      slot[2] >>= 8;
     }
   }
-  if (to < 0) return -1;
+  if ((c.size & 7) != 0) {
+    word <<= 8 * (8 - (c.size & 7));
+    if (c.size < 8) c.word[0] = word;
+    else if (c.size < 16) c.word[1] = word;
+    else c.word[2] = word;
+  }
   int32_t first = 0, count = t.tokens;  // thrust::binary_search: lower_bound by halving, then !(value < *it)
   while (count > 0) {
     int32_t const half = count >> 1;
-    if (compare_candidate(lds, from, to, t, first + half) > 0) {
+    if (compare_candidate(c, t, first + half) > 0) {
       first += half + 1;
       count -= half + 1;
     } else {
       count = half;
     }
   }
-  if (first >= t.tokens || compare_candidate(lds, from, to, t, first) < 0) return -1;
-  return to;
+  if (first >= t.tokens || compare_candidate(c, t, first) < 0) return -1;
+  return 3 * i + last;
 }
 
 // special_tokens_kernel (normalize.cu:270-316) over lds.slot, in two steps so that every decision reads unchanged
@@ -1187,7 +1237,7 @@ nvtext_amd_status nvtext_amd_character_normalizer_create(int32_t do_lower_case, 
   bool ok = obj->store.allocate(&obj->ascii, 256) && obj->store.allocate(&obj->bmp, bmp.size()) &&
             obj->store.allocate(&obj->entries, entries.size()) && obj->store.allocate(&obj->second, second.size());
   if (ok && !tokens.empty())
-    ok = obj->store.allocate(&obj->token_offset, token_offsets.size()) && obj->store.allocate(&obj->token_chars, std::max<size_t>(token_chars.size(), 1));
+    ok = obj->store.allocate(&obj->token_offset, token_offsets.size()) && obj->store.allocate(&obj->token_chars, token_chars.size() + 8);
   if (!ok) return fail_with(hipErrorOutOfMemory);
   e = hipMemcpyAsync(obj->ascii, ascii, sizeof(ascii), hipMemcpyHostToDevice, stream);
   if (e == hipSuccess) e = hipMemcpyAsync(obj->bmp, bmp.data(), bmp.size() * sizeof(uint4), hipMemcpyHostToDevice, stream);
@@ -1195,7 +1245,8 @@ nvtext_amd_status nvtext_amd_character_normalizer_create(int32_t do_lower_case, 
   if (e == hipSuccess) e = hipMemcpyAsync(obj->second, second.data(), second.size() * sizeof(uint64_t), hipMemcpyHostToDevice, stream);
   if (e == hipSuccess && !tokens.empty())
     e = hipMemcpyAsync(obj->token_offset, token_offsets.data(), token_offsets.size() * sizeof(int32_t), hipMemcpyHostToDevice, stream);
-  if (e == hipSuccess && !token_chars.empty()) e = hipMemcpyAsync(obj->token_chars, token_chars.data(), token_chars.size(), hipMemcpyHostToDevice, stream);
+  token_chars.append(8, '\0');
+  if (e == hipSuccess && !tokens.empty()) e = hipMemcpyAsync(obj->token_chars, token_chars.data(), token_chars.size(), hipMemcpyHostToDevice, stream);
   hipError_t const synced = hipStreamSynchronize(stream);  // the host copies die at return
   if (e == hipSuccess) e = synced;
   if (e != hipSuccess) return fail_with(e);
