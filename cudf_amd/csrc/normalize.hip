@@ -19,6 +19,7 @@ struct nvtext_amd_character_normalizer {
   int32_t do_lower      = 0;
   uint32_t* ascii       = nullptr;  // device, 256: slot 0 | slot 1 << 8 | slot 2 << 16 | bytes << 24 of the code points below 0x80, zeros
   uint4* bmp            = nullptr;  // device, 65536: {slot 0, slot 1, slot 2, bytes} of the code points below 0x10000, and 65536 of their strings
+  uint8_t* sizes        = nullptr;  // device, 65536: the bytes alone
   uint32_t* entries     = nullptr;  // device, kCodepoints: category << 24 | multi << 23 | replacement
   uint64_t* second      = nullptr;  // device, kCodepoints: second << 32 | third replacement code point
   uint8_t* token_chars  = nullptr;  // device: the special tokens, sorted then lower-cased
@@ -58,6 +59,7 @@ struct NormTables {
   const uint32_t* ascii;  // 256 entries: the slots of the code points below 0x80, then zeros (a byte that is no such character gives nothing)
   const uint4* bmp;       // 65536 entries: the three slots and their bytes together, of the code points below 0x10000; and 65536
                           // more: those slots side by side, as a string of up to 12 bytes, and its bytes
+  const uint8_t* sizes;   // 65536: the bytes alone (in a sixteenth of the memory, for the pass that counts)
   const uint32_t* entries;
   const uint64_t* second;
   const uint8_t* token_chars;
@@ -129,7 +131,7 @@ __host__ __device__ __forceinline__ void slots_of(uint32_t cp, NormTables const&
   }
 }
 
-constexpr int kWaveLeads = 256;  // first bytes of longer characters per wavefront (512 input bytes) that the counting pass lists
+constexpr int kWaveLeads = 256;  // first bytes of longer characters per wavefront (512 input bytes) that the counting pass lists: two in four bytes
 
 template <bool SLOTS>
 struct NormLds {
@@ -144,7 +146,7 @@ struct NormLds {
   };
   union {
     alignas(16) uint16_t prefix[kNormTile + 8];  // bytes the tile writes before each position; [tile] = all of them
-    uint16_t lead_pos[kNormThreads / kWave][kWaveLeads];  // (before that: the tile positions of the first bytes of a wavefront's longer characters)
+    uint16_t lead_pos[kNormThreads / kWave][kWaveLeads];  // (before that: where in raw the longer characters of a wavefront begin)
   };
   uint32_t scan[kNormThreads / kWave + 1];
   uint32_t bracket;  // some lane of the tile saw what can open a special token
@@ -267,9 +269,8 @@ __device__ int token_opens_at(NormLds<S>& lds, NormTables const& t, int i)
 // slots.  A lane looks at its own positions; the first kBefore lanes also at the positions before the tile (a '['
 // in the positions after the tile belongs to the next tile).
 template <bool S>
-__device__ void apply_special_tokens(NormLds<S>& lds, NormTables const& t)
+__device__ void apply_special_tokens(NormLds<S>& lds, NormTables const& t, int tid)
 {
-  int const tid = threadIdx.x;
   int found_to[kNormItems + 1];
 #pragma unroll
   for (int k = 0; k <= kNormItems; ++k) {
@@ -294,14 +295,14 @@ __device__ void apply_special_tokens(NormLds<S>& lds, NormTables const& t)
   lds_barrier();
 }
 
-// Code point of a character of two or three bytes whose bytes start `w` (first byte below 0xF0): decode() without
-// its branches.
+// Code point of a character of two or three bytes whose bytes start `w` (first byte between 0xC0 and 0xEF): decode()
+// without its branches.  The three bytes are turned round, a character of two bytes is moved to the end (0xC0..0xDF, which
+// have bit 5 clear, look like a continuation byte there), and shifts to the right and masks, which take half the time of
+// shifts to the left, put the pieces together: 21 cycles a wavefront instead of 40.
 __device__ __forceinline__ uint32_t decode_short(uint32_t w)
 {
-  uint32_t const b1    = (w >> 8) & 0x3Fu;
-  uint32_t const two   = ((w & 0x1Fu) << 6) | b1;
-  uint32_t const three = ((w & 0x0Fu) << 12) | (b1 << 6) | ((w >> 16) & 0x3Fu);
-  return (w & 0xFFu) < 0xE0u ? two : three;
+  uint32_t const p = __builtin_amdgcn_perm(0u, w, 0x0c000102u) >> ((~w & 0x20u) >> 2);
+  return ((p >> 4) & 0xF000u) | ((p >> 2) & 0x0FC0u) | (p & 0x3Fu);
 }
 
 // Slots of the character whose bytes start `w` (first byte in the low bits) and the bytes they hold together.  The
@@ -357,8 +358,8 @@ __device__ __forceinline__ uint32_t wide_string(uint32_t w, NormTables const& t,
   return e.w;
 }
 
-// Bytes that the character whose bytes start `w` produces, without its slots.
-__device__ __forceinline__ uint32_t wide_size(uint32_t w, NormTables const& t)
+// Bytes that the character whose bytes start `w` produces, without its slots; opener: whether it is a '['.
+__device__ __forceinline__ uint32_t wide_size(uint32_t w, NormTables const& t, bool& opener)
 {
   uint32_t cp = decode_short(w);
   if ((w & 0xFFu) >= 0xF0u) {
@@ -369,7 +370,8 @@ __device__ __forceinline__ uint32_t wide_size(uint32_t w, NormTables const& t)
       return bytes_of(s0) + bytes_of(s1) + bytes_of(s2);
     }
   }
-  return t.bmp[cp].w;
+  opener = opener || cp == '[';
+  return t.sizes[cp];
 }
 
 // The slots (and sizes) of the eight positions whose bytes are lo64; hi64 = bytes 4..11.  Returns the bytes they produce.
@@ -462,55 +464,91 @@ __device__ __forceinline__ void wave_lds_sync()
 }
 
 // The bytes that the wavefront's 512 positions produce, for the pass that only sizes the output (a lane's return value
-// holds the sizes of characters that are not its own: only the sum over the wavefront means something).
+// holds the sizes of characters that are not its own: only the sum over the wavefront means something; so does `opener`,
+// whether one of the longer characters is an over-long '[').
 // One-byte characters go through the table in LDS, lanes <-> bytes.  The first bytes of longer characters are few
-// and unevenly spread (none in English text, every other byte in Cyrillic or Greek), and each needs a read of the
-// code point tables: the wavefront lists them and goes through the list lanes <-> characters, every lane at work.
+// and unevenly spread (none in English text, every other byte in Cyrillic or Greek), and each needs a read of a table
+// by code point: the wavefront lists them and goes through the list lanes <-> characters, every lane at work.  Text
+// has no more than two of them in four bytes, which is what the list is built for.
 // `byte0` = the byte offset in lds.raw of the tile's first byte.
 template <bool SLOTS>
-__device__ __forceinline__ uint32_t owned_dense(NormLds<SLOTS>& lds, uint64_t lo64, uint64_t hi64, uint32_t byte0, NormTables const& t)
+__device__ __forceinline__ uint32_t owned_dense(NormLds<SLOTS>& lds, uint32_t own0, uint32_t own1, uint32_t next, uint32_t byte0, NormTables const& t,
+                                                int tid, bool& opener)
 {
   uint32_t sum = 0;
 #pragma unroll
-  for (int j = 0; j < kNormItems; ++j) {
-    uint32_t const b = static_cast<uint32_t>(lo64 >> (8 * j)) & 0xFFu;
-    sum += lds.sizes[b];
-  }
-  uint64_t const leads  = lo64 & (lo64 << 1) & 0x8080808080808080ull;  // bit 7 of the bytes >= 0xC0
-  uint32_t const mine_n = static_cast<uint32_t>(__builtin_popcountll(leads));
-  uint32_t const incl   = wave_inclusive_scan(mine_n);
-  uint32_t const first  = incl - mine_n;
-  uint32_t const all    = wave_bcast(incl, kWave - 1);
-  if (all == 0) return sum;
-  if (all > static_cast<uint32_t>(kWaveLeads)) {
-    // more than every other byte begins a character: not text; every lane walks its own
-    uint64_t l = leads;
+  for (int j = 0; j < 4; ++j) sum += lds.sizes[(own0 >> (8 * j)) & 0xFFu];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) sum += lds.sizes[(own1 >> (8 * j)) & 0xFFu];
+  uint32_t const leads0 = own0 & (own0 << 1) & 0x80808080u, leads1 = own1 & (own1 << 1) & 0x80808080u;  // bit 7 of the bytes >= 0xC0
+  if (ballot64((leads0 | leads1) != 0u) == 0) return sum;
+  uint32_t const more0 = leads0 & (leads0 - 1u), more1 = leads1 & (leads1 - 1u);
+  if (ballot64(((more0 & (more0 - 1u)) | (more1 & (more1 - 1u))) != 0u) != 0) {
+    // three of four bytes begin a character: not text; every lane walks its own
+    uint64_t const lo64 = (static_cast<uint64_t>(own1) << 32) | own0, hi64 = (static_cast<uint64_t>(next) << 32) | own1;
+    uint64_t l          = (static_cast<uint64_t>(leads1) << 32) | leads0;
     while (l) {
       int const at = (__ffsll(static_cast<long long>(l)) - 1) >> 3;
       l &= l - 1ull;
-      sum += wide_size(static_cast<uint32_t>((at < 4 ? lo64 : hi64) >> (8 * (at & 3))), t);
+      sum += wide_size(static_cast<uint32_t>((at < 4 ? lo64 : hi64) >> (8 * (at & 3))), t, opener);
     }
     return sum;
   }
-  int const lane       = lane_id();
-  uint16_t* const list = lds.lead_pos[threadIdx.x / kWave];
+  uint32_t const n0   = static_cast<uint32_t>(__builtin_popcount(leads0));
+  uint32_t const n    = n0 + static_cast<uint32_t>(__builtin_popcount(leads1));
+  uint32_t const incl = wave_inclusive_scan(n);
+  uint32_t const all  = wave_bcast(incl, kWave - 1);
+  uint16_t* const list = lds.lead_pos[tid / kWave];
   {
-    uint32_t i = first;
-#pragma unroll
-    for (int j = 0; j < kNormItems; ++j) {
-      bool const is = ((leads >> (8 * j + 7)) & 1ull) != 0;
-      if (is) list[i] = static_cast<uint16_t>(kNormItems * threadIdx.x + j);
-      i += is ? 1u : 0u;
-    }
+    uint32_t const at = byte0 + kNormItems * tid;
+    uint16_t* to      = list + (incl - n);
+    if (leads0 != 0u) to[0] = static_cast<uint16_t>(at + (static_cast<uint32_t>(__builtin_ctz(leads0)) >> 3));
+    if (more0 != 0u) to[1] = static_cast<uint16_t>(at + (static_cast<uint32_t>(__builtin_ctz(more0)) >> 3));
+    to += n0;
+    if (leads1 != 0u) to[0] = static_cast<uint16_t>(at + 4u + (static_cast<uint32_t>(__builtin_ctz(leads1)) >> 3));
+    if (more1 != 0u) to[1] = static_cast<uint16_t>(at + 4u + (static_cast<uint32_t>(__builtin_ctz(more1)) >> 3));
   }
   wave_lds_sync();
-  for (uint32_t r = lane; r < all; r += kWave) {
-    uint32_t const off = byte0 + list[r];
+  for (uint32_t r = lane_id(); r < all; r += kWave) {
+    uint32_t const off = list[r];
     uint32_t const w   = __builtin_amdgcn_alignbit(lds.raw[(off >> 2) + 1], lds.raw[off >> 2], 8u * (off & 3u));
-    sum += wide_size(w, t);
+    sum += wide_size(w, t, opener);
   }
   return sum;
 }
+
+// v, of which the compiler does not know that it is the same in every trip of a loop: it keeps no sums of it over the trips
+// then, for which it would spill registers (normalize_count_small_kernel: 128 and 74 spilled -> 91 and none; 20000 rows of
+// 300 bytes 70 -> 35 us a call).
+__device__ __forceinline__ int same_again(int v)
+{
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// The 16 bytes at `block`, which are the column's bytes from position p on; bytes outside [0, n) read as 0.
+__device__ __forceinline__ uint4 load_within(const uint4* block, int64_t p, int64_t n)
+{
+  uint4 v = make_uint4(0u, 0u, 0u, 0u);
+  if (p + 15 >= 0 && p < n) {
+    v = load_stream(block);
+    if (p < 0 || p + 16 > n) {  // the first or the last block of the column: clear what lies outside
+      uint32_t* const part = &v.x;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        int64_t const q = p + 4 * k;
+        uint32_t keep   = 0xFFFFFFFFu;
+        if (q < 0) keep = q <= -4 ? 0u : keep << (8 * static_cast<uint32_t>(-q));
+        if (q + 4 > n) keep = q >= n ? 0u : keep & (0xFFFFFFFFu >> (8 * static_cast<uint32_t>(q + 4 - n)));
+        part[k] &= keep;
+      }
+    }
+  }
+  return v;
+}
+
+// Whether everything that is staged of the tile at t0 lies within the column.
+__device__ __forceinline__ bool tile_is_inside(int64_t t0, int64_t n) { return t0 >= kRawBefore + 15 && t0 + 4 * kRawWords - kRawBefore <= n; }
 
 // The lane's eight bytes of a tile and the four after them, the tile staged in LDS with its surroundings, the ASCII table
 // beside it; `mis`: what the tile's alignment puts in front of them.
@@ -519,9 +557,8 @@ struct OwnBytes {
   uint32_t mis;
 };
 template <bool SLOTS>
-__device__ __forceinline__ OwnBytes stage_tile(NormLds<SLOTS>& lds, const uint8_t* chars, int64_t t0, int64_t n, NormTables const& t)
+__device__ __forceinline__ OwnBytes stage_tile(NormLds<SLOTS>& lds, const uint8_t* chars, int64_t t0, int64_t n, NormTables const& t, int tid)
 {
-  int const tid = threadIdx.x;
   // stage [t0 - kRawBefore, t0 + kNormTile + kRawAfter) with one aligned 16-byte load per lane (the first 131 lanes);
   // bytes outside [0, n) read as 0.  Everything is requested before anything is waited for.
   static_assert(kNormThreads == 256, "a table entry per lane");
@@ -530,21 +567,8 @@ __device__ __forceinline__ OwnBytes stage_tile(NormLds<SLOTS>& lds, const uint8_
   uint32_t const mis         = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(wb) & 15u);
   if (tid < kRawWords / 4) {
     int64_t const p = t0 - kRawBefore - mis + 16 * static_cast<int64_t>(tid);  // column position of the block's first byte
-    uint4 v         = make_uint4(0u, 0u, 0u, 0u);
-    if (p + 15 >= 0 && p < n) {
-      v = load_stream(reinterpret_cast<const uint4*>(wb - mis) + tid);
-      if (p < 0 || p + 16 > n) {  // the first or the last block of the column: clear what lies outside
-        uint32_t* const part = &v.x;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          int64_t const q = p + 4 * k;
-          uint32_t keep   = 0xFFFFFFFFu;
-          if (q < 0) keep = q <= -4 ? 0u : keep << (8 * static_cast<uint32_t>(-q));
-          if (q + 4 > n) keep = q >= n ? 0u : keep & (0xFFFFFFFFu >> (8 * static_cast<uint32_t>(q + 4 - n)));
-          part[k] &= keep;
-        }
-      }
-    }
+    const uint4* const block = reinterpret_cast<const uint4*>(wb - mis) + tid;
+    uint4 const v            = tile_is_inside(t0, n) ? load_stream(block) : load_within(block, p, n);
     *reinterpret_cast<uint4*>(&lds.raw[4 * tid]) = v;
   }
   lds.ascii[tid] = table_entry;
@@ -565,54 +589,51 @@ __device__ __forceinline__ OwnBytes stage_tile(NormLds<SLOTS>& lds, const uint8_
 // Whether a special token may open in one of the eight positions before the tile (five needed): the first eight lanes
 // decode the character that begins at theirs, so that an over-long '[' is one here exactly if it is one to the slots.
 // Both passes ask this: one that took a tile for free of tokens while the other applied them would give it another size.
-template <bool SLOTS>
-__device__ __forceinline__ bool opener_before(NormLds<SLOTS> const& lds, uint32_t mis)
+__device__ __forceinline__ bool opener_before(const uint32_t* raw, uint32_t lane, uint32_t mis)
 {
-  if (threadIdx.x >= kRawBefore) return false;
-  uint32_t const off = mis + threadIdx.x;
-  uint32_t const w   = __builtin_amdgcn_alignbit(lds.raw[(off >> 2) + 1], lds.raw[off >> 2], 8u * (off & 3u));
+  if (lane >= kRawBefore) return false;
+  uint32_t const off = mis + lane;
+  uint32_t const w   = __builtin_amdgcn_alignbit(raw[(off >> 2) + 1], raw[off >> 2], 8u * (off & 3u));
   uint32_t const b0  = w & 0xFFu;
   return b0 < 0xC0u ? b0 == '[' : decode(b0, (w >> 8) & 0xFFu, (w >> 16) & 0xFFu, w >> 24) == '[';
 }
 
 // One tile: the slots of the lane's positions, special tokens applied.  Returns the bytes they produce.  Without
-// SLOTS only that number is wanted: the slots are then built only in tiles that may hold a special token.
-template <bool SLOTS>
-__device__ __forceinline__ uint32_t tile_slots(NormLds<SLOTS>& lds, const uint8_t* chars, int64_t t0, int64_t n, NormTables const& t, Owned& mine,
-                                               uint32_t (&size)[kNormItems])
+// SLOTS only that number is wanted: the slots are then built only in tiles that may hold a special token.  MARKED: the tile
+// is known to be one.
+template <bool SLOTS, bool MARKED = false>
+__device__ __forceinline__ uint32_t tile_slots(NormLds<SLOTS>& lds, const uint8_t* chars, int64_t t0, int64_t n, NormTables const& t, int tid,
+                                               Owned& mine, uint32_t (&size)[kNormItems])
 {
-  int const tid      = threadIdx.x;
-  OwnBytes const own = stage_tile(lds, chars, t0, n, t);
+  OwnBytes const own = stage_tile(lds, chars, t0, n, t, tid);
   uint32_t const own0 = own.own0, own1 = own.own1, next = own.next, mis = own.mis;
   uint64_t const lo64 = (static_cast<uint64_t>(own1) << 32) | own0;
   uint64_t const hi64 = (static_cast<uint64_t>(next) << 32) | own1;
   // (the pass that wants the slots keeps them in registers all the way: listing the longer characters for it as well
   // saves it 4 % of its instructions and costs it two of its seven wavefronts per SIMD, 8.6 -> 10.7 ms on the
   // multilingual workload; the pass that only counts gains 13 % from the list)
-  uint32_t sum;
+  uint32_t sum  = 0;
+  bool overlong = false;
   if constexpr (SLOTS) sum = owned_strings(lds, lo64, hi64, t, mine, size);
-  else sum = owned_dense(lds, lo64, hi64, mis + kRawBefore, t);
+  else if constexpr (!MARKED) sum = owned_dense(lds, own0, own1, next, mis + kRawBefore, t, tid, overlong);
 
   if (t.tokens > 0) {
     // A special token starts at a position whose slot 1 is '['.  Tiles without one skip the exchange through LDS.
-    // No code point's replacement is a '[', so it takes a '[' byte or an over-long encoding of it, which starts
-    // with 0xC1, 0xE0 or 0xF0: that is what decides for the lane's own bytes when the slots have not been built (a
-    // superset, which is harmless).
-    bool bracket = false;
-    if (SLOTS) {
-      // (strings: a '[' is padded like all punctuation, so it is the middle byte of " [ ")
+    // No code point's replacement is a '[', so it takes a '[' byte or an over-long encoding of it: that is what
+    // decides when the slots have not been built.
+    if constexpr (!MARKED) {
+      bool bracket = opener_before(lds.raw, tid, mis);
+      if constexpr (SLOTS) {
+        // (strings: a '[' is padded like all punctuation, so it is the middle byte of " [ ")
 #pragma unroll
-      for (int j = 0; j < kNormItems; ++j) bracket |= ((mine.s[j][0] >> 8) & 0xFFu) == '[';
-    } else {
-      bracket = has_byte(own0, '[') || has_byte(own1, '[');
-      if ((lo64 & (lo64 << 1) & 0x8080808080808080ull) != 0)
-        bracket = bracket || has_byte(own0, 0xC1u) || has_byte(own0, 0xE0u) || has_byte(own0, 0xF0u) || has_byte(own1, 0xC1u) ||
-                  has_byte(own1, 0xE0u) || has_byte(own1, 0xF0u);
+        for (int j = 0; j < kNormItems; ++j) bracket |= ((mine.s[j][0] >> 8) & 0xFFu) == '[';
+      } else {
+        bracket = bracket || overlong || has_byte(own0, '[') || has_byte(own1, '[');
+      }
+      if (ballot64(bracket) != 0 && lane_id() == 0) lds.bracket = 1u;
+      lds_barrier();
     }
-    bracket = bracket || opener_before(lds, mis);
-    if (ballot64(bracket) != 0 && lane_id() == 0) lds.bracket = 1u;
-    lds_barrier();
-    if (lds.bracket != 0u) {
+    if (MARKED || lds.bracket != 0u) {
       owned_slots(lds, lo64, hi64, t, mine, size);  // (the slots themselves, whatever mine held)
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
@@ -643,7 +664,7 @@ __device__ __forceinline__ uint32_t tile_slots(NormLds<SLOTS>& lds, const uint8_
         lds.slot[2][kSlotBase + pos] = static_cast<uint8_t>(s2);
       }
       lds_barrier();
-      apply_special_tokens(lds, t);
+      apply_special_tokens(lds, t, tid);
       // the tokens only ever empty a slot or turn its letter into upper case: take over the first bytes that changed
       sum         = 0;
       mine.widest = 0;
@@ -682,13 +703,144 @@ __global__ void __launch_bounds__(kNormThreads, 8) normalize_count_kernel(const 
                                                                        uint32_t* __restrict__ tile_bytes)
 {
   __shared__ NormLds<false> lds;
+  int const tid    = threadIdx.x;
   int64_t const t0 = static_cast<int64_t>(blockIdx.x) * kNormTile;
   Owned mine;
   uint32_t size[kNormItems];
-  uint32_t const sum = tile_slots<false>(lds, chars, t0, n, t, mine, size);
+  uint32_t const sum = tile_slots<false>(lds, chars, t0, n, t, tid, mine, size);
   uint32_t total;
   block_exclusive_scan_lds<kNormThreads>(sum, lds.scan, &total);
   if (threadIdx.x == 0) tile_bytes[blockIdx.x] = total;
+}
+
+// The same for a column of many tiles: every wavefront takes a whole one, with a list of its longer characters, and waits
+// for no other.  Tiles that may hold a special token are left for the workgroup to do together at the end, as
+// normalize_count_kernel does them.
+// What bounds it is instructions again: with a workgroup a tile half the time went on barriers, on starting, on staging
+// the table and on a list for every 512 bytes.  766 MB of mixed text 461 -> 290 us; several tiles for a wavefront, with the bytes
+// of the next one on their way, no faster.  A small column has too few wavefronts this way: of 17 MB 73.5 us a call with a
+// workgroup a tile and 75.5 with this, of 34 MB 110 and 108, of 67 MB 180 and 172.
+constexpr int kTileWaves          = kNormThreads / kWave;
+constexpr int kLaneWords          = kNormTile / kWave / 4;  // dwords of a tile per lane, two of every 512 bytes
+constexpr int64_t kManyTiles      = 12288;                  // a column of so many tiles
+union CountLds {
+  struct {
+    alignas(16) uint32_t raw[kTileWaves][kRawWords];
+    uint16_t leads[kTileWaves][kNormTile / 2];  // where in raw the longer characters of a tile begin
+  };
+  NormLds<false> tile;
+};
+__global__ void __launch_bounds__(kNormThreads, 8) normalize_count_tiles_kernel(const uint8_t* __restrict__ chars, int64_t n, uint32_t tiles,
+                                                                             NormTables t, uint32_t* __restrict__ tile_bytes)
+{
+  __shared__ CountLds lds;
+  __shared__ uint8_t sizes[256];
+  __shared__ uint32_t left[kTileWaves];  // the tiles left for the end
+  uint32_t const wave  = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = lane_id();
+  uint32_t const tile0 = blockIdx.x * kTileWaves, tile = tile0 + wave;
+  int64_t const t0     = static_cast<int64_t>(tile) * kNormTile;
+  uint32_t const mis   = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(chars - kRawBefore) & 15u);  // (of every tile: they are 2048 bytes apart)
+  uint32_t* const raw  = lds.raw[wave];
+  bool opener          = false;
+  uint32_t const table_entry = t.ascii[threadIdx.x];
+  bool const third = lane < kRawWords / 4 - 2 * kWave;
+  uint4 v[3];
+  if (tile < tiles) {
+    const uint4* const block = reinterpret_cast<const uint4*>(chars + t0 - kRawBefore - mis) + lane;
+    if (tile_is_inside(t0, n)) {
+      v[0] = load_stream(block);
+      v[1] = load_stream(block + kWave);
+      if (third) v[2] = load_stream(block + 2 * kWave);
+    } else {
+      int64_t const p = t0 - kRawBefore - mis + 16 * static_cast<int64_t>(lane);
+      v[0]            = load_within(block, p, n);
+      v[1]            = load_within(block + kWave, p + 16 * kWave, n);
+      if (third) v[2] = load_within(block + 2 * kWave, p + 32 * kWave, n);
+    }
+  }
+  sizes[threadIdx.x] = static_cast<uint8_t>(table_entry >> 24);
+  lds_barrier();
+  bool marked = false;
+  if (tile < tiles) {
+    reinterpret_cast<uint4*>(raw)[lane]         = v[0];
+    reinterpret_cast<uint4*>(raw)[lane + kWave] = v[1];
+    if (third) reinterpret_cast<uint4*>(raw)[lane + 2 * kWave] = v[2];
+    wave_lds_sync();
+    const uint32_t* const own_raw = raw + ((mis + kRawBefore) >> 2) + 2 * lane;
+    uint32_t const shift          = 8u * (mis & 3u);
+    uint32_t sum = 0, many = 0, n_leads = 0;
+    uint32_t leads[kLaneWords];  // bit 7 of the bytes >= 0xC0
+#pragma unroll
+    for (int q = 0; q < kLaneWords / 2; ++q) {
+      const uint32_t* const r = own_raw + q * (2 * kWave);
+      uint32_t const r0 = r[0], r1 = r[1], r2 = r[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        uint32_t const own = h ? __builtin_amdgcn_alignbit(r2, r1, shift) : __builtin_amdgcn_alignbit(r1, r0, shift);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum += sizes[(own >> (8 * j)) & 0xFFu];
+        uint32_t const l    = own & (own << 1) & 0x80808080u;
+        uint32_t const more = l & (l - 1u);
+        leads[2 * q + h]    = l;
+        many |= more & (more - 1u);
+        n_leads += static_cast<uint32_t>(__builtin_popcount(l));
+        opener = opener || has_byte(own, '[');
+      }
+    }
+    opener = opener || opener_before(raw, lane, mis);
+    marked = t.tokens > 0 && ballot64(opener) != 0;
+    if (!marked && ballot64(n_leads != 0u) != 0) {
+      uint32_t const at = mis + kRawBefore + kNormItems * lane;
+      if (ballot64(many != 0u) != 0) {
+        // three of four bytes begin a character: not text; every lane walks its own
+#pragma unroll
+        for (int k = 0; k < kLaneWords; ++k) {
+          uint32_t l = leads[k];
+          while (l != 0u) {
+            uint32_t const off = at + (k / 2) * (kWave * kNormItems) + 4 * (k & 1) + (static_cast<uint32_t>(__builtin_ctz(l)) >> 3);
+            l &= l - 1u;
+            sum += wide_size(__builtin_amdgcn_alignbit(raw[(off >> 2) + 1], raw[off >> 2], 8u * (off & 3u)), t, opener);
+          }
+        }
+      } else {
+        uint32_t const incl  = wave_inclusive_scan(n_leads);
+        uint32_t const all   = wave_bcast(incl, kWave - 1);
+        uint16_t* const list = lds.leads[wave];
+        uint16_t* to         = list + (incl - n_leads);
+#pragma unroll
+        for (int k = 0; k < kLaneWords; ++k) {
+          uint32_t const l = leads[k], more = l & (l - 1u);
+          uint32_t const off = at + (k / 2) * (kWave * kNormItems) + 4 * (k & 1);
+          if (l != 0u) to[0] = static_cast<uint16_t>(off + (static_cast<uint32_t>(__builtin_ctz(l)) >> 3));
+          if (more != 0u) to[1] = static_cast<uint16_t>(off + (static_cast<uint32_t>(__builtin_ctz(more)) >> 3));
+          to += __builtin_popcount(l);
+        }
+        wave_lds_sync();
+        for (uint32_t r = lane; r < all; r += kWave) {
+          uint32_t const off = list[r];
+          sum += wide_size(__builtin_amdgcn_alignbit(raw[(off >> 2) + 1], raw[off >> 2], 8u * (off & 3u)), t, opener);
+        }
+      }
+    }
+    marked = t.tokens > 0 && ballot64(opener) != 0;
+    sum    = wave_inclusive_scan(sum);
+    if (!marked && lane == kWave - 1) tile_bytes[tile] = sum;
+  }
+  if (t.tokens == 0) return;
+  if (lane == 0) left[wave] = marked ? 1u : 0u;
+  lds_barrier();
+#pragma unroll 1
+  for (int k = 0; k < kTileWaves; ++k) {
+    if (__builtin_amdgcn_readfirstlane(static_cast<int>(left[k])) == 0) continue;
+    int const tid       = same_again(threadIdx.x);
+    Owned mine;
+    uint32_t size[kNormItems];
+    uint32_t const bytes = tile_slots<false, true>(lds.tile, chars, static_cast<int64_t>(tile0 + k) * kNormTile, n, t, tid, mine, size);
+    uint32_t total;
+    block_exclusive_scan_lds<kNormThreads>(bytes, lds.tile.scan, &total);
+    if (threadIdx.x == 0) tile_bytes[tile0 + k] = total;
+    lds_barrier();
+  }
 }
 
 // The same for a column whose size the host does not know yet: where its bytes lie the kernel reads from the offsets (a
@@ -716,9 +868,10 @@ __global__ void __launch_bounds__(kNormThreads, 4) normalize_count_small_kernel(
       }
       if (lane_id() == 0) tile_row[tile] = static_cast<int32_t>(lo);
     }
+    int const tid = same_again(threadIdx.x);
     Owned mine;
     uint32_t size[kNormItems];
-    uint32_t const sum = tile_slots<false>(lds, col.chars + first, t0, n, t, mine, size);
+    uint32_t const sum = tile_slots<false>(lds, col.chars + first, t0, n, t, tid, mine, size);
     uint32_t total;
     block_exclusive_scan_lds<kNormThreads>(sum, lds.scan, &total);
     if (threadIdx.x == 0) tile_bytes[tile] = total;
@@ -878,7 +1031,7 @@ __device__ __forceinline__ void write_tile(NormLds<true>& lds, uint32_t tile, ui
   tile_rows.request(col, tile_row, tile, tiles);
   Owned mine;
   uint32_t size[kNormItems];
-  uint32_t const sum = tile_slots<true>(lds, col.chars + first, t0, n, t, mine, size);
+  uint32_t const sum = tile_slots<true>(lds, col.chars + first, t0, n, t, tid, mine, size);
   // the buffer that the output bytes are assembled in starts out as zeros (the scan's barriers stand between this
   // and the first byte placed); in a tile that went through the special tokens it lies where the slots' first bytes
   // were, which the other wavefronts may still be reading
@@ -964,7 +1117,7 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_kernel(ColVie
   uint64_t const base = tile_offset[tile];
   TileRows tile_rows;
   tile_rows.request(col, tile_row, tile, gridDim.x);
-  OwnBytes const own  = stage_tile(lds, col.chars + first, t0, n, t);
+  OwnBytes const own  = stage_tile(lds, col.chars + first, t0, n, t, tid);
   uint64_t const lo64 = (static_cast<uint64_t>(own.own1) << 32) | own.own0;
   uint64_t const hi64 = (static_cast<uint64_t>(own.next) << 32) | own.own1;
   uint32_t text[kNormItems];
@@ -1006,7 +1159,7 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_kernel(ColVie
     }
   }
   other = other || leads != 0;
-  if (t.tokens > 0) other = other || has_byte(own.own0, '[') || has_byte(own.own1, '[') || opener_before(lds, own.mis);
+  if (t.tokens > 0) other = other || has_byte(own.own0, '[') || has_byte(own.own1, '[') || opener_before(lds.raw, tid, own.mis);
   if (ballot64(other) != 0 && lane_id() == 0) lds.bracket = 1u;
   clear_staged(lds);
   // where each position's bytes begin in the lane's: the sums of the sizes before it (96 at most)
@@ -1202,12 +1355,14 @@ nvtext_amd_status nvtext_amd_character_normalizer_create(int32_t do_lower_case, 
 
   // the finished slots of the Basic Multilingual Plane (the rules of slots_of, run here once per code point)
   std::vector<uint4> bmp(2 * 0x10000);
+  std::vector<uint8_t> sizes(0x10000);
   {
-    NormTables const host_tables{nullptr, nullptr, entries.data(), second.data(), nullptr, nullptr, 0, do_lower_case ? 1 : 0};
+    NormTables const host_tables{nullptr, nullptr, nullptr, entries.data(), second.data(), nullptr, nullptr, 0, do_lower_case ? 1 : 0};
     for (uint32_t cp = 0; cp < 0x10000u; ++cp) {
       uint32_t s0, s1, s2;
       slots_of(cp, host_tables, s0, s1, s2);
-      bmp[cp] = make_uint4(s0, s1, s2, bytes_of(s0) + bytes_of(s1) + bytes_of(s2));
+      bmp[cp]   = make_uint4(s0, s1, s2, bytes_of(s0) + bytes_of(s1) + bytes_of(s2));
+      sizes[cp] = static_cast<uint8_t>(bmp[cp].w);
       uint32_t d0, d1, d2;
       slots_to_string(s0, s1, s2, d0, d1, d2);
       bmp[0x10000 + cp] = make_uint4(d0, d1, d2, bmp[cp].w);
@@ -1235,12 +1390,13 @@ nvtext_amd_status nvtext_amd_character_normalizer_create(int32_t do_lower_case, 
   hipError_t e = hipGetDevice(&obj->device);
   if (e != hipSuccess) return fail_with(e);
   bool ok = obj->store.allocate(&obj->ascii, 256) && obj->store.allocate(&obj->bmp, bmp.size()) &&
-            obj->store.allocate(&obj->entries, entries.size()) && obj->store.allocate(&obj->second, second.size());
+            obj->store.allocate(&obj->sizes, sizes.size()) && obj->store.allocate(&obj->entries, entries.size()) && obj->store.allocate(&obj->second, second.size());
   if (ok && !tokens.empty())
     ok = obj->store.allocate(&obj->token_offset, token_offsets.size()) && obj->store.allocate(&obj->token_chars, token_chars.size() + 8);
   if (!ok) return fail_with(hipErrorOutOfMemory);
   e = hipMemcpyAsync(obj->ascii, ascii, sizeof(ascii), hipMemcpyHostToDevice, stream);
   if (e == hipSuccess) e = hipMemcpyAsync(obj->bmp, bmp.data(), bmp.size() * sizeof(uint4), hipMemcpyHostToDevice, stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(obj->sizes, sizes.data(), sizes.size(), hipMemcpyHostToDevice, stream);
   if (e == hipSuccess) e = hipMemcpyAsync(obj->entries, entries.data(), entries.size() * sizeof(uint32_t), hipMemcpyHostToDevice, stream);
   if (e == hipSuccess) e = hipMemcpyAsync(obj->second, second.data(), second.size() * sizeof(uint64_t), hipMemcpyHostToDevice, stream);
   if (e == hipSuccess && !tokens.empty())
@@ -1282,7 +1438,7 @@ nvtext_amd_status nvtext_amd_normalize_characters(const nvtext_amd_strings_colum
   // kSmallRowBytes bytes a row and kSmallBytes in all, before the host knows how many bytes there are; one wait instead of
   // two.  Where there are more these kernels leave at once.  (61 rows of 300 bytes: 74 -> 32 us)
   ColView const view = make_view(*input);
-  NormTables const tables{normalizer->ascii, normalizer->bmp, normalizer->entries, normalizer->second, normalizer->token_chars, normalizer->token_offset, normalizer->tokens,
+  NormTables const tables{normalizer->ascii, normalizer->bmp, normalizer->sizes, normalizer->entries, normalizer->second, normalizer->token_chars, normalizer->token_offset, normalizer->tokens,
                           normalizer->do_lower};
   uint64_t* const scalars = host_scalars();  // pinned words that kernels write for the host (nullptr: copy instead)
   bool small              = scalars && input->chars && rows <= kSmallRows;
@@ -1366,8 +1522,14 @@ nvtext_amd_status nvtext_amd_normalize_characters(const nvtext_amd_strings_colum
     uint32_t* const tile_bytes = temps.part<uint32_t>(0);
     {
       ProfileScope ps("normalize_count_kernel", stream);
-      hipLaunchKernelGGL(normalize_count_kernel, dim3(static_cast<unsigned>(tiles)), dim3(kNormThreads), 0, stream, view.chars + first, n, tables,
-                         tile_bytes);
+      if (tiles >= kManyTiles) {
+        int64_t const grid = (tiles + kTileWaves - 1) / kTileWaves;
+        hipLaunchKernelGGL(normalize_count_tiles_kernel, dim3(static_cast<unsigned>(grid)), dim3(kNormThreads), 0, stream, view.chars + first, n,
+                           static_cast<uint32_t>(tiles), tables, tile_bytes);
+      } else {
+        hipLaunchKernelGGL(normalize_count_kernel, dim3(static_cast<unsigned>(tiles)), dim3(kNormThreads), 0, stream, view.chars + first, n, tables,
+                           tile_bytes);
+      }
     }
     hipLaunchKernelGGL(normalize_tile_rows_kernel, dim3(static_cast<unsigned>((tiles + 255) / 256)), dim3(256), 0, stream, view, first, tiles,
                        tile_row);

@@ -276,3 +276,31 @@ def test_normalize_feeds_the_tokenizer(nv, onorm):
     exp = orc.wordpiece_tokenize(onorm.normalize_characters(host, True, [b"[CLS]"]), orc.Vocabulary(vocab), 0)
     assert got.equals(exp)
     assert got.child.size > 3 * 3000
+
+
+@pytest.mark.parametrize("kind", ["plain", "tokens", "bytes"])
+@pytest.mark.parametrize("skip,extra", [(0, 0), (1, 1), (2, 2047), (3, 12345)])
+def test_normalize_wavefront_a_tile(nv, onorm, kind, skip, extra):
+    """Columns so large that a wavefront counts whole tiles, and just below that: the tiles' number is no multiple of the
+    workgroups', characters and special tokens lie across every border, the first byte has any alignment."""
+    rng = np.random.default_rng(7 + skip)
+    pieces = [b"word", b" ", b" a", b"Th", b"\xc3\xa9t\xc3\xa9", "漢字".encode(), "Жи".encode(), b".", b"),", b"\t", "\U0001F600".encode()]
+    if kind != "plain":
+        pieces += [b"[", b"]", b"[SEP]", b" [sep] ", b"[ Pad ]", b"\xc1\x9bSEP]", b"\xe0\x81\x9bPAD]"]
+    if kind == "bytes":
+        pieces += [b"\xff", b"\x80\x80", b"\xc3\xc3\xe4", b"\xf0\xf0\xf0\xf0\xf0\xf0\xf0\xf0", b"\xc3", b"\0"]
+    which = rng.integers(0, len(pieces), 60001)
+    if kind == "tokens":
+        which = np.where(rng.random(which.size) < 0.97, rng.integers(0, 11, which.size), which)
+    part = np.frombuffer(b"".join(pieces[i] for i in which), np.uint8)
+    for tiles in (12288, 12287) if skip == 0 else (12288 + 64 * skip + 3,):
+        n = tiles * TILE - (TILE - 1) + extra
+        rows = 2500
+        chars = np.resize(part, n + 40)
+        ends = np.sort(rng.integers(40, n + 40, rows - 1))
+        offsets = np.concatenate([[0], np.arange(1, skip + 1) * 11, ends, [n + 40]]).astype(np.int32)
+        host = HostStringsColumn(chars, offsets, None, rows + skip, 0, 0).slice(skip, rows + skip)
+        tokens = () if kind == "plain" else ("[SEP]", "[PAD]")
+        got = run(nv, host, True, tokens)
+        exp = onorm.normalize_characters_native(host, True, [t.encode() for t in tokens], 8)
+        assert_same(got, exp, f"{kind} {tiles}")
