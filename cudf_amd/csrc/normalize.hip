@@ -55,10 +55,12 @@ constexpr int64_t kSmallLeast    = 256 << 10;
 constexpr int64_t kSmallBytes    = 64 << 20;
 constexpr int kStageBytes  = 4 * kNormTile;  // output bytes of a tile that are assembled in LDS; a tile with more writes them one by one
 
+constexpr uint32_t kNotShort = 0x80000000u;  // beside the bytes of a string: there are more than eight, or it is the " [ " that may open a special token
+
 struct NormTables {
   const uint32_t* ascii;  // 256 entries: the slots of the code points below 0x80, then zeros (a byte that is no such character gives nothing)
   const uint4* bmp;       // 65536 entries: the three slots and their bytes together, of the code points below 0x10000; and 65536
-                          // more: those slots side by side, as a string of up to 12 bytes, and its bytes
+                          // more: those slots side by side, as a string of up to 12 bytes, and its bytes (with kNotShort)
   const uint8_t* sizes;   // 65536: the bytes alone (in a sixteenth of the memory, for the pass that counts)
   const uint32_t* entries;
   const uint64_t* second;
@@ -355,7 +357,7 @@ __device__ __forceinline__ uint32_t wide_string(uint32_t w, NormTables const& t,
   d0            = e.x;
   d1            = e.y;
   d2            = e.z;
-  return e.w;
+  return e.w & 0xFFu;
 }
 
 // Bytes that the character whose bytes start `w` produces, without its slots; opener: whether it is a '['.
@@ -1022,9 +1024,8 @@ __device__ __forceinline__ void place_short(uint8_t* sb, uint32_t o, uint32_t su
 // Writes the tile's bytes at tile_offset[tile] and the output offset of every row that starts in the tile.
 __device__ __forceinline__ void write_tile(NormLds<true>& lds, uint32_t tile, uint32_t tiles, ColView const& col, int64_t first, int64_t n,
                                            NormTables const& t, const uint64_t* tile_offset, const int32_t* tile_row, uint8_t* out_chars,
-                                           void* out_offsets, int offsets_are_int64)
+                                           void* out_offsets, int offsets_are_int64, int tid)
 {
-  int const tid        = threadIdx.x;
   int64_t const t0     = static_cast<int64_t>(tile) * kNormTile;
   uint64_t const base  = tile_offset[tile];
   TileRows tile_rows;
@@ -1171,7 +1172,7 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_kernel(ColVie
   uint32_t const before = block_exclusive_scan_lds<kNormThreads>(sum, lds.scan, &total);
   if (lds.bracket != 0u || total > static_cast<uint32_t>(kStageBytes)) {
     lds_barrier();  // (everybody has read that)
-    write_tile(lds, tile, gridDim.x, col, first, n, t, tile_offset, tile_row, out_chars, out_offsets, offsets_are_int64);
+    write_tile(lds, tile, gridDim.x, col, first, n, t, tile_offset, tile_row, out_chars, out_offsets, offsets_are_int64, tid);
     return;
   }
   {
@@ -1213,6 +1214,238 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_kernel(ColVie
   lds_barrier();
   store_staged(lds.staged, dst, lead, total);
   tile_rows.place(col, first, t0, base, lds.prefix, out_offsets, offsets_are_int64);
+}
+
+// The same for a column of many tiles, a wavefront a tile as in normalize_count_tiles_kernel: in steps of 512 bytes, whose
+// output is laid out in the wavefront's own part of LDS; the dword that a step leaves unfinished is the next one's first.
+// Tiles that are not for this kernel are left for the workgroup to do together at the end.
+// What bounds it is vector instructions, the reads and or-writes of LDS beside them.  Longer characters are taken by fours
+// of bytes, two at most in each, with 32-bit arithmetic only; one-byte characters are placed in pairs; a row's place comes
+// from the lane that its first byte is with, not from a list of all places.  766 MB of mixed text 1250 -> 1010 us; a call with a
+// workgroup a tile and with this: 17 MB mixed 73.9 and 76.1 us, ASCII 68.0 and 63.3, 34 MB 105 and 102, 92.3 and 79.2, 134 MB
+// mixed 296 and 256.
+constexpr int kStep       = kWave * kNormItems;  // input bytes of a step
+constexpr int kStepBytes  = 4 * kStep;           // of output; a tile with more in a step is left
+union WriteLds {
+  struct {
+    alignas(16) uint32_t raw[kTileWaves][kRawWords];
+    alignas(16) uint32_t staged[kTileWaves][kStepBytes / 4 + 4];
+  };
+  NormLds<true> tile;
+};
+__global__ void __launch_bounds__(kNormThreads, 6) normalize_write_tiles_kernel(ColView col, int64_t first, int64_t n, uint32_t tiles, NormTables t,
+                                                                             const uint64_t* __restrict__ tile_offset,
+                                                                             const int32_t* __restrict__ tile_row, uint8_t* __restrict__ out_chars,
+                                                                             void* __restrict__ out_offsets, int offsets_are_int64)
+{
+  __shared__ WriteLds lds;
+  __shared__ uint32_t ascii[256];
+  __shared__ uint32_t left[kTileWaves];  // the tiles left for the end
+  uint32_t const wave  = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = lane_id();
+  uint32_t const tile0 = blockIdx.x * kTileWaves, tile = tile0 + wave;
+  int64_t const t0     = static_cast<int64_t>(tile) * kNormTile;
+  const uint8_t* const chars = col.chars + first;
+  uint32_t const mis         = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(chars - kRawBefore) & 15u);
+  uint32_t* const raw        = lds.raw[wave];
+  uint32_t* const staged     = lds.staged[wave];
+  uint32_t const table_entry = t.ascii[threadIdx.x];
+  bool const third           = lane < kRawWords / 4 - 2 * kWave;
+  uint4 v[3];
+  int64_t row = 0, row_end = 0;  // the lane's row, of those that begin in the tile
+  uint32_t row_at = ~0u;         // where in the tile
+  auto const look_up = [&]() {
+    row_at = row < row_end ? static_cast<uint32_t>(col.off(row) - first - t0) : ~0u;
+  };
+  if (tile < tiles) {
+    const uint4* const block = reinterpret_cast<const uint4*>(chars + t0 - kRawBefore - mis) + lane;
+    if (tile_is_inside(t0, n)) {
+      v[0] = load_stream(block);
+      v[1] = load_stream(block + kWave);
+      if (third) v[2] = load_stream(block + 2 * kWave);
+    } else {
+      int64_t const p = t0 - kRawBefore - mis + 16 * static_cast<int64_t>(lane);
+      v[0]            = load_within(block, p, n);
+      v[1]            = load_within(block + kWave, p + 16 * kWave, n);
+      if (third) v[2] = load_within(block + 2 * kWave, p + 32 * kWave, n);
+    }
+    // the rows that start in this tile end where the next tile's begin (the last tile also takes the end of the last row)
+    row     = static_cast<int64_t>(tile_row[tile]) + lane;
+    row_end = tile + 1 == tiles ? static_cast<int64_t>(col.size) + 1 : static_cast<int64_t>(tile_row[tile + 1]);
+    look_up();
+  }
+  ascii[threadIdx.x] = table_entry;
+  for (int i = lane; i < (kStepBytes / 4 + 4) / 4; i += kWave) reinterpret_cast<uint4*>(staged)[i] = make_uint4(0u, 0u, 0u, 0u);
+  lds_barrier();
+  bool marked = false;
+  if (tile < tiles) {
+    reinterpret_cast<uint4*>(raw)[lane]         = v[0];
+    reinterpret_cast<uint4*>(raw)[lane + kWave] = v[1];
+    if (third) reinterpret_cast<uint4*>(raw)[lane + 2 * kWave] = v[2];
+    wave_lds_sync();
+    uint64_t const base  = tile_offset[tile];
+    uint8_t* const dst   = out_chars + base;
+    uint32_t const lead  = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(dst) & 3u);
+    uint32_t* const dw   = reinterpret_cast<uint32_t*>(dst - lead);
+    uint32_t const shift = 8u * (mis & 3u);
+    uint32_t words       = 0;     // full dwords of the tile that are in memory
+    uint32_t in_first    = lead;  // bytes in the first dword of the buffer already
+    uint32_t done        = 0;     // bytes that the steps before produced
+    bool const opened    = t.tokens > 0 && ballot64(opener_before(raw, lane, mis)) != 0;
+    const uint32_t* own_raw = raw + ((mis + kRawBefore) >> 2) + 2 * lane;
+    marked                  = opened;
+#pragma unroll 1
+    for (uint32_t from = 0; from < kNormTile && !marked; from += kStep, own_raw += kStep / 4) {
+      uint32_t const r0 = own_raw[0], r1 = own_raw[1], r2 = own_raw[2], r3 = own_raw[3];
+      uint32_t const own[3] = {__builtin_amdgcn_alignbit(r1, r0, shift), __builtin_amdgcn_alignbit(r2, r1, shift), __builtin_amdgcn_alignbit(r3, r2, shift)};
+      uint32_t text[kNormItems];
+#pragma unroll
+      for (int j = 0; j < kNormItems; ++j) text[j] = ascii[(own[j / 4] >> (8 * (j & 3))) & 0xFFu];
+      // the sizes of the positions, a byte each
+      auto const top_bytes = [](uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+        return __builtin_amdgcn_perm(b, a, 0x0c0c0703u) | __builtin_amdgcn_perm(d, c, 0x07030c0cu);
+      };
+      uint32_t sizes[2] = {top_bytes(text[0], text[1], text[2], text[3]), top_bytes(text[4], text[5], text[6], text[7])};
+      uint32_t const leads[2] = {own[0] & (own[0] << 1) & 0x80808080u, own[1] & (own[1] << 1) & 0x80808080u};  // bit 7 of the bytes >= 0xC0
+      bool const any_long = ballot64((leads[0] | leads[1]) != 0u) != 0;
+      bool other          = t.tokens > 0 && (has_byte(own[0], '[') || has_byte(own[1], '['));
+      // up to two longer characters in each four bytes: text has no more
+      uint32_t d0[4] = {}, d1[4] = {}, at8[4] = {};
+      uint64_t holders[4] = {};
+      if (any_long) {
+        uint4 e[4];
+        uint32_t flags = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          uint32_t const all = leads[k / 2], l = k & 1 ? all & (all - 1u) : all;
+          holders[k]         = ballot64(l != 0u);
+          e[k]               = make_uint4(0u, 0u, 0u, 0u);
+          if (holders[k] != 0) {
+            at8[k]           = static_cast<uint32_t>(__builtin_ctz(l | 0x80000000u)) & 24u;  // 8 * position
+            uint32_t const w = __builtin_amdgcn_alignbit(own[k / 2 + 1], own[k / 2], at8[k]);
+            if (l != 0u) e[k] = t.bmp[0x10000u + decode_short(w)];
+            bool const four = l != 0u && (w & 0xFFu) >= 0xF0u;
+            if (ballot64(four) != 0) {  // (seldom)
+              if (four) {
+                e[k].w = wide_string(w, t, e[k].x, e[k].y, e[k].z);
+                if (e[k].w > 8u || e[k].x == 0x205B20u) e[k].w |= kNotShort;
+              }
+            }
+          }
+          if (k & 1) flags |= l & (l - 1u);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          d0[k] = e[k].x;
+          d1[k] = e[k].y;
+          flags |= e[k].w;
+          sizes[k / 2] += e[k].w << at8[k];
+        }
+        other = other || (flags & (kNotShort | 0x808080u)) != 0u;
+      }
+      // where each position's bytes begin in the lane's: the sums of the sizes before it (88 at most)
+      uint32_t const in0 = sizes[0] * 0x01010101u;
+      uint32_t const in1 = sizes[1] * 0x01010101u + (in0 >> 24) * 0x01010101u;
+      uint32_t const ex0 = in0 << 8, ex1 = __builtin_amdgcn_alignbit(in1, in0, 24);
+      uint32_t const sum    = in1 >> 24;
+      uint32_t const incl   = wave_inclusive_scan(sum);
+      uint32_t const total  = wave_bcast(incl, kWave - 1);
+      uint32_t const before = incl - sum;
+      if (ballot64(other) != 0 || total > static_cast<uint32_t>(kStepBytes)) {
+        marked = true;
+        break;
+      }
+      // the rows that begin in the step (the end of the last row may lie behind the last tile's last byte)
+      uint32_t const row_limit = from + kStep == kNormTile ? kNormTile + 1u : from + kStep;
+      while (true) {
+        bool const here = row_at >= from && row_at < row_limit;
+        if (ballot64(here) != 0) {
+          uint32_t const local = row_at - from;
+          int const source     = static_cast<int>(local >> 1) & ~3;  // 4 * (local / 8)
+          uint32_t const of0   = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(source, static_cast<int>(ex0)));
+          uint32_t const of1   = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(source, static_cast<int>(ex1)));
+          uint32_t const lanes = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(source, static_cast<int>(before)));
+          uint32_t const in    = ((local & 4u ? of1 : of0) >> (8u * (local & 3u))) & 0xFFu;
+          if (here) {
+            uint64_t const at = base + done + (local >= static_cast<uint32_t>(kStep) ? total : lanes + in);
+            if (offsets_are_int64) static_cast<int64_t*>(out_offsets)[row] = static_cast<int64_t>(at);
+            else static_cast<int32_t*>(out_offsets)[row] = static_cast<int32_t>(at);
+          }
+        }
+        if (wave_bcast(row_at, kWave - 1) >= row_limit) break;
+        row += kWave;  // (more than 64 rows)
+        look_up();
+      }
+      // the one-byte characters in pairs: every string (zero padded) is or-ed into the aligned dwords it falls into; the
+      // buffer holds zeros, and what the neighbours put into a shared dword is theirs
+      uint32_t const o = in_first + before;
+      uint64_t pair[4];
+      uint32_t sixes = 0;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        uint32_t const a = text[2 * p], b = text[2 * p + 1];
+        pair[p] = (static_cast<uint64_t>(b & 0xFFFFFFu) << ((a >> 21) & 0x18u)) | (a & 0xFFFFFFu);
+        sixes |= static_cast<uint32_t>(pair[p] >> 32);
+      }
+      bool const any_six = ballot64(sixes > 0xFFu) != 0;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        // (a longer character may stand in front of the second: the place is counted from there)
+        uint32_t const second = ((p < 2 ? ex0 : ex1) >> (16 * (p & 1) + 8)) & 0xFFu;
+        uint32_t const at     = o + second - (text[2 * p] >> 24);
+        uint32_t const sh     = 8u * (at & 3u);
+        uint32_t* const to    = staged + (at >> 2);
+        uint64_t const both   = pair[p] << sh;
+        atomicOr(to, static_cast<uint32_t>(both));
+        atomicOr(to + 1, static_cast<uint32_t>(both >> 32));
+        if (any_six) atomicOr(to + 2, (static_cast<uint32_t>(pair[p] >> 32) >> 8) >> (24u - sh));
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (holders[k] == 0) continue;
+        uint32_t const at   = o + (((k < 2 ? ex0 : ex1) >> at8[k]) & 0xFFu);
+        uint32_t const sh   = 8u * (at & 3u);
+        uint32_t* const to  = staged + (at >> 2);
+        uint64_t const both = ((static_cast<uint64_t>(d1[k]) << 32) | d0[k]) << sh;
+        uint32_t const past = (d1[k] >> 8) >> (24u - sh);
+        atomicOr(to, static_cast<uint32_t>(both));
+        atomicOr(to + 1, static_cast<uint32_t>(both >> 32));
+        if (ballot64(past != 0u) != 0) atomicOr(to + 2, past);
+      }
+      wave_lds_sync();
+      // the full dwords to memory, zeros in their place; the unfinished one to the front
+      uint32_t const end = in_first + total, full = end >> 2;
+      uint32_t const rest = staged[full];
+      for (uint32_t w = lane; w < full; w += kWave) {
+        uint32_t const d = staged[w];
+        staged[w]        = 0u;
+        if (words + w != 0 || lead == 0) {
+          store_stream(dw + words + w, d);
+        } else {  // (the tile's first dword has bytes of the tile before)
+          for (uint32_t b = lead; b < 4u; ++b) reinterpret_cast<uint8_t*>(dw)[b] = static_cast<uint8_t>(d >> (8u * b));
+        }
+      }
+      wave_lds_sync();
+      if (lane == 0) {
+        staged[full] = 0u;
+        staged[0]    = rest;
+      }
+      wave_lds_sync();
+      words += full;
+      in_first = end & 3u;
+      done += total;
+    }
+    if (!marked && lane >= (words == 0 ? lead : 0u) && lane < in_first)
+      reinterpret_cast<uint8_t*>(dw + words)[lane] = static_cast<uint8_t>(staged[0] >> (8u * lane));
+    if (marked) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // what has been written is there before other wavefronts write it anew
+  }
+  if (lane == 0) left[wave] = marked ? 1u : 0u;
+  lds_barrier();
+#pragma unroll 1
+  for (int k = 0; k < kTileWaves; ++k) {
+    if (__builtin_amdgcn_readfirstlane(static_cast<int>(left[k])) == 0) continue;
+    write_tile(lds.tile, tile0 + k, tiles, col, first, n, t, tile_offset, tile_row, out_chars, out_offsets, offsets_are_int64, same_again(threadIdx.x));
+    lds_barrier();
+  }
 }
 
 struct TileBytes {
@@ -1365,7 +1598,7 @@ nvtext_amd_status nvtext_amd_character_normalizer_create(int32_t do_lower_case, 
       sizes[cp] = static_cast<uint8_t>(bmp[cp].w);
       uint32_t d0, d1, d2;
       slots_to_string(s0, s1, s2, d0, d1, d2);
-      bmp[0x10000 + cp] = make_uint4(d0, d1, d2, bmp[cp].w);
+      bmp[0x10000 + cp] = make_uint4(d0, d1, d2, bmp[cp].w | (bmp[cp].w > 8u || d0 == 0x205B20u ? kNotShort : 0u));
     }
   }
 
@@ -1556,8 +1789,15 @@ nvtext_amd_status nvtext_amd_normalize_characters(const nvtext_amd_strings_colum
   }
   {
     ProfileScope ps("normalize_write_kernel", stream);
-    hipLaunchKernelGGL(normalize_write_kernel, dim3(static_cast<unsigned>(tiles)), dim3(kNormThreads), 0, stream, view, first, n, tables,
-                       tile_offset, tile_row, reinterpret_cast<uint8_t*>(out->chars), out->offsets, out->offsets_is_int64);
+    if (tiles >= kManyTiles) {
+      int64_t const grid = (tiles + kTileWaves - 1) / kTileWaves;
+      hipLaunchKernelGGL(normalize_write_tiles_kernel, dim3(static_cast<unsigned>(grid)), dim3(kNormThreads), 0, stream, view, first, n,
+                         static_cast<uint32_t>(tiles), tables, tile_offset, tile_row, reinterpret_cast<uint8_t*>(out->chars), out->offsets,
+                         out->offsets_is_int64);
+    } else {
+      hipLaunchKernelGGL(normalize_write_kernel, dim3(static_cast<unsigned>(tiles)), dim3(kNormThreads), 0, stream, view, first, n, tables,
+                         tile_offset, tile_row, reinterpret_cast<uint8_t*>(out->chars), out->offsets, out->offsets_is_int64);
+    }
   }
   e = hipGetLastError();
   if (e != hipSuccess) return release(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
