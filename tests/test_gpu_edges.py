@@ -409,3 +409,27 @@ def test_normalize_where_small_columns_end(nv, rows, each, brackets):
         got = nv.normalize_characters(d.slice(lo, hi, 0), normalizer).to_host()
         exp = normalize_py.normalize_characters_native(host.slice(lo, hi), True, [b"[CLS]", b"[SEP]"], nthreads=8)
         assert np.array_equal(got.chars, exp.chars) and np.array_equal(got.offsets, exp.offsets)
+
+
+@pytest.mark.parametrize("width", [2, 5, 17])
+@pytest.mark.parametrize("lead", [0, 1, 3])
+def test_characters_of_a_tile(nv, orc, width, lead):
+    """Rows of several scripts and of bytes that are no UTF-8 (continuation bytes in front, in the middle and alone, characters
+    cut off by the end of the row), of lengths around the tiles of 256 bytes, with any alignment of the first byte."""
+    rng = np.random.default_rng(10 * width + lead)
+    pieces = [b"a", b"xyz", "é".encode(), "漢字".encode(), "\U0001F600".encode(), b"\x80", b"\xbf\x80\x80\x80\x80", b"\xe6\xbc", b"\xff", b"\xf0\x9f"]
+    rows = []
+    for shares in ([8, 8, 8, 8, 8, 0, 0, 0, 0, 0], [4, 2, 8, 1, 1, 1, 0, 0, 0, 0], [1, 1, 1, 1, 1, 1, 1, 1, 1, 1], [0, 0, 1, 9, 0, 0, 0, 0, 0, 0], [0, 0, 0, 0, 0, 4, 1, 0, 0, 0]):
+        p = np.array(shares) / np.sum(shares)
+        for size in [1, 7, 63, 64, 65, 127, 128, 129, 250, 255, 256, 257, 258, 261, 383, 384, 385, 511, 512, 513, 767, 768, 769, 1500]:
+            rows.append(b"".join(pieces[i] for i in rng.choice(len(pieces), size, p=p))[:size])
+    chars = np.frombuffer(b"#" * lead + b"".join(rows), np.uint8).copy()
+    offsets = np.concatenate([[0], lead + np.concatenate([[0], np.cumsum([len(r) for r in rows])])]).astype(np.int32)
+    host = HostStringsColumn(chars, offsets, None, len(rows) + 1, 0, 0).slice(1, len(rows) + 1)
+    for bits in (32, 64):
+        a, b = params(rng, 40, bits)
+        call, ref = (nv.minhash, orc.minhash) if bits == 32 else (nv.minhash64, orc.minhash64)
+        assert call(dev(nv, host), 5, a, b, width).to_host().equals(ref(host, 5, a, b, width, nthreads=8))
+    h1, h2 = host.slice(0, len(rows) - 1), host.slice(1, len(rows))
+    got, exp = nv.jaccard_index(dev(nv, h1), dev(nv, h2), width).to_host(), orc.jaccard_index(h1, h2, width, nthreads=8)
+    assert np.array_equal(got.values.view(np.uint32), exp.values.view(np.uint32))
