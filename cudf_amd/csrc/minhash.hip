@@ -231,7 +231,10 @@ struct MinimaAll {
   Packing pk, tail_pk;
   int lane;
 
-  __device__ __forceinline__ MinimaAll(Lds*, int lane_) : lane(lane_) {}
+  static constexpr int kLeast = 0;
+  __device__ __forceinline__ MinimaAll(Lds*, int lane_, bool) : lane(lane_) {}
+  __device__ __forceinline__ int32_t stride() const { return kParams; }
+  __device__ __forceinline__ int32_t slots() const { return kSlots; }
   __device__ __forceinline__ void load(Params<T> const& p, int32_t chunk)
   {
     pk = K == 1 ? packing_for(p.count) : Packing{kWave, 1};
@@ -311,15 +314,27 @@ struct Minima64 {
     alignas(16) T minima[kParams];
   };
   Params<T> params;
-  int32_t base;  // first parameter of the chunk
+  int32_t base;    // first parameter of the chunk
+  int32_t groups;  // of the chunk: GROUPS or kLeast
+  uint32_t warm;   // (see load)
   Lds* lds;
   int lane;
+  static constexpr int kLeast = GROUPS < 2 ? GROUPS : 2;  // groups of a chunk in a column with too few units of work for all wavefronts
 
-  __device__ __forceinline__ Minima64(Lds* lds_, int lane_) : lds(lds_), lane(lane_) {}
+  __device__ __forceinline__ Minima64(Lds* lds_, int lane_, bool few) : groups(few ? kLeast : GROUPS), warm(0), lds(lds_), lane(lane_) {}
+  __device__ __forceinline__ int32_t stride() const { return slots(); }  // parameters from a chunk to the next
+  __device__ __forceinline__ int32_t slots() const { return groups * filter64::kGroup; }
+  static __device__ __forceinline__ int32_t chunks_of_least(int32_t count) { return (count + kLeast * filter64::kGroup - 1) / (kLeast * filter64::kGroup); }
+  // What the first groups have in memory is asked for here, a cache line a lane, and waited for where it is used: the plan has
+  // just written it, and a read then takes two microseconds.
   __device__ __forceinline__ void load(Params<T> const& p, int32_t chunk)
   {
     params = p;
-    base   = chunk * kParams;
+    base   = chunk * slots();
+    int32_t const first   = base / filter64::kGroup, last = (params.count - 1) / filter64::kGroup;
+    const uint8_t* const at = reinterpret_cast<const uint8_t*>(params.groups + min(first, last));
+    int32_t const size      = static_cast<int32_t>(sizeof(filter64::Group)) * min(kLeast, last - min(first, last) + 1);
+    warm = *reinterpret_cast<const uint32_t*>(at + min(128 * lane, size - 4));
   }
   __device__ __forceinline__ void reset()
   {
@@ -380,19 +395,22 @@ struct Minima64 {
     }
   };
 
-  // The parameters of two groups, a lane each (index j of the chunk; a single group: both halves have the same).
-  __device__ __forceinline__ void settle(Ranked const& of_lower, Ranked const& of_upper, int j, const T* hashes, uint32_t count)
+  // The parameters of two groups, a lane each (index j of the chunk; a single group: both halves have the same, the lower one
+  // acts).  Lanes beyond the last parameter have its products, but go through nothing more for them: a row for which the last
+  // of 260 parameters needs a second half block kept a wavefront busy with it 28 times over (100 rows of 2000 bytes 67 -> 33 us).
+  __device__ __forceinline__ void settle(Ranked const& of_lower, Ranked const& of_upper, int j, bool two, const T* hashes, uint32_t count)
   {
     bool const upper = lane >= filter64::kGroup;
+    bool const acts  = base + j < params.count && (two || !upper);
     Ranked const r{upper ? of_upper.first : of_lower.first, upper ? of_upper.second : of_lower.second, upper ? of_upper.third : of_lower.third};
     int32_t const at     = min(base + j, params.count - 1);
     T const a = params.a[at], b = params.b[at];
     uint32_t const slack = params.groups[at / filter64::kGroup].slack[at % filter64::kGroup];
     T m                  = min(lds->minima[j], exact(hashes, r.first & 0xFFFFu, a, b));
-    uint64_t todo        = ballot64(r.second >> 16 <= limit_of(m, slack));
+    uint64_t todo        = ballot64(acts && r.second >> 16 <= limit_of(m, slack));
     if (todo != 0) {
       // few parameters (one in six of 1000 hashes): the products of four of them at a time, sixteen lanes each
-      lds->minima[j] = m;
+      if (acts) lds->minima[j] = m;
       wave_lds_fence();
       do {
         int who[4];
@@ -411,7 +429,7 @@ struct Minima64 {
       } while (todo != 0);
       wave_lds_fence();
       m = lds->minima[j];
-      for (todo = ballot64(r.third >> 16 <= limit_of(m, slack)); todo != 0; todo &= todo - 1) {
+      for (todo = ballot64(acts && r.third >> 16 <= limit_of(m, slack)); todo != 0; todo &= todo - 1) {
         int const who = static_cast<int>(__builtin_ctzll(todo));
         T const wa = wave_bcast64(a, who), wb = wave_bcast64(b, who);
         T v = std::numeric_limits<T>::max();
@@ -421,13 +439,17 @@ struct Minima64 {
         if (lane == who) m = min(m, v);
       }
     }
-    lds->minima[j] = m;
+    if (acts) lds->minima[j] = m;
   }
 
   template <int G>
   __device__ __forceinline__ void fold_groups(int32_t first, const T* hashes, uint32_t count)
   {
     asm("" : "+s"(first));  // (the pieces are read anew for every fold: not kept in registers while windows are hashed)
+    asm volatile("" : : "v"(warm));
+    // (the parameters are asked for before the blocks, so that they are near when the products are computed)
+    int32_t const j0    = min(base + first * filter64::kGroup + G * (lane & 31), params.count - 1);
+    uint32_t const near = *reinterpret_cast<const uint32_t*>(lane < 32 ? params.a + j0 : params.b + j0);
     int32_t const last = (params.count - 1) / filter64::kGroup;
     uint32_t pieces[G][2][6];
 #pragma unroll
@@ -452,12 +474,13 @@ struct Minima64 {
 #pragma unroll
       for (int g = 0; g < G; ++g) ranked[g].add(filter64::least_of(filter64::sums_of(digits, pieces[g][0], pieces[g][1], scale[0], scale[1], start)) << 16 | half_block);
     }
+    asm volatile("" : : "v"(near));
 #pragma unroll
     for (int g = 0; g < G; ++g) ranked[g].merge_halves();
 #pragma unroll
     for (int g = 0; g < G; g += 2) {
       bool const two = g + 1 < G;
-      settle(ranked[g], ranked[two ? g + 1 : g], (first + g) * filter64::kGroup + (two ? lane : lane % filter64::kGroup), hashes, count);
+      settle(ranked[g], ranked[two ? g + 1 : g], (first + g) * filter64::kGroup + (two ? lane : lane % filter64::kGroup), two, hashes, count);
     }
   }
 
@@ -471,9 +494,15 @@ struct Minima64 {
     uint32_t const rest = (0u - count) & 31u;
     if (static_cast<uint32_t>(lane) < rest) hashes[count + lane] = hashes[0];
     wave_lds_fence();
+    if (GROUPS > kLeast && AT_ONCE != kLeast && groups == kLeast) {
+      fold_groups<kLeast>(0, hashes, count + rest);
+    } else {
 #pragma unroll 1
-    for (int g = 0; g + AT_ONCE <= GROUPS; g += AT_ONCE) fold_groups<AT_ONCE>(g, hashes, count + rest);
-    if constexpr (GROUPS % AT_ONCE != 0) fold_groups<GROUPS % AT_ONCE>(GROUPS / AT_ONCE * AT_ONCE, hashes, count + rest);
+      for (int g = 0; g + AT_ONCE <= groups; g += AT_ONCE) fold_groups<AT_ONCE>(g, hashes, count + rest);
+      if constexpr (GROUPS % AT_ONCE != 0) {
+        if (groups == GROUPS) fold_groups<GROUPS % AT_ONCE>(GROUPS / AT_ONCE * AT_ONCE, hashes, count + rest);
+      }
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     return 0;
@@ -482,7 +511,7 @@ struct Minima64 {
   template <typename Put>
   __device__ __forceinline__ void each(Put const& put) const
   {
-    for (int j = lane; j < kParams; j += kWave) put(j, lds->minima[j]);
+    for (int j = lane; j < slots(); j += kWave) put(j, lds->minima[j]);
     __builtin_amdgcn_wave_barrier();
   }
   static constexpr uint32_t kNoKey = 0xFFFFFFFFu;
@@ -745,6 +774,7 @@ template <typename Source>
 struct RowParts {
   Source source;
   int32_t waves;  // wavefronts that the device holds
+  int32_t least;  // the least part: Source::kMinPart, more where the products of a row are computed exactly at its end
   // What every wavefront has to do.
   __device__ __forceinline__ int64_t share() const
   {
@@ -765,7 +795,7 @@ struct RowParts {
   {
     int64_t const all    = share();
     int64_t const length = (all / (all < 4 * Source::kMinPart ? 2 : 4) + kWave) / kWave * kWave;
-    float const within   = static_cast<float>(min(max(length, Source::kMinPart), Source::kPart));
+    float const within   = static_cast<float>(min(max(length, static_cast<int64_t>(least)), Source::kPart));
     return Cut{__builtin_amdgcn_rcpf(within), source.rows() <= waves ? within - 1.0f : within / 2.0f};
   }
   __device__ __forceinline__ uint32_t parts_of(int64_t n, Cut const& c) const
@@ -860,17 +890,26 @@ __global__ void __launch_bounds__(kThreads, (simd_waves<Source, Minima>())) minh
   bool one_counter;
   uint32_t const each   = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(parts.per_unit(total, min(params.count, Minima::kSlots), &one_counter))));
   uint32_t const units  = total / each + (total % each != 0 ? 1u : 0u);
+  // 64-bit hashes: chunks of two groups of parameters where the wavefronts suffice for that (the windows are hashed for each
+  // of them, by wavefronts that had nothing to do): 100 rows of 2000 bytes, 128 parameters 21 -> 18 us;
+  // with twice or four times as many units as wavefronts it is no gain: 50 rows of 16 KB 33.2 us whole, 36.4 in chunks of two groups
+  bool few = false;
+  if constexpr (Minima::kLeast != 0) {
+    int32_t const least = Minima::chunks_of_least(params.count);
+    few                 = static_cast<uint64_t>(units) * static_cast<uint32_t>(least) <= static_cast<uint64_t>(parts.waves);
+    if (few) chunks = least;
+  }
   uint64_t const all    = static_cast<uint64_t>(units) * static_cast<uint32_t>(chunks);
   int const lane        = lane_id();
   int const wave        = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
   uint32_t const me     = blockIdx.x * kWaves + static_cast<uint32_t>(wave);
   uint32_t chunk        = 0;
-  Minima minima(&minima_lds[wave], lane);
+  Minima minima(&minima_lds[wave], lane, few);
   minima.load(params, 0);
   for (uint64_t unit = me; unit < all;) {
     while (unit >= static_cast<uint64_t>(chunk + 1u) * units) minima.load(params, static_cast<int32_t>(++chunk));  // (the next chunk of parameters)
-    int32_t const chunk_base = static_cast<int32_t>(chunk) * Minima::kParams;
-    int32_t const in_chunk   = min(Minima::kSlots, params.count - chunk_base);
+    int32_t const chunk_base = static_cast<int32_t>(chunk) * minima.stride();
+    int32_t const in_chunk   = min(minima.slots(), params.count - chunk_base);
     uint32_t t               = static_cast<uint32_t>(unit - static_cast<uint64_t>(chunk) * units) * each;
     uint32_t const t_end     = total - t < each ? total : t + each;
     int64_t base  = 0;  // near: prefix of the rows from there on, a lane a row
@@ -1165,7 +1204,10 @@ void run_minhash(Source const& source, int32_t rows, bool short_rows, const T* a
 {
   int waves = 0;
   with_minima<Source>(P, short_rows, [&](auto which, int32_t) { waves = simd_waves<Source, typename decltype(which)::type>(); });
-  RowParts<Source> const parts{source, device_cus() * 4 * waves};
+  // Runs of elements on the matrix cores: a part ends with exact products, which 64 runs are too few for (200 lists of 2500 elements,
+  // 256 parameters: parts of 64 and more 51 us, of 128 and more 41; 500 of them 65 and 61).
+  int32_t const least = static_cast<int32_t>(Source::kMinPart) * (sizeof(T) == 8 && !short_rows && Source::kMinPart == kWave ? 2 : 1);
+  RowParts<Source> const parts{source, device_cus() * 4 * waves, least};
   Params<T> const params{a, b, P, laid_out};
   auto* const counters = reinterpret_cast<unsigned long long*>(plan);
   auto const layers    = [&](int threads) { return laid_out ? (groups_of(P) + threads / kWave - 1) / (threads / kWave) : 0; };
@@ -1324,7 +1366,10 @@ nvtext_amd_status minhash_ngrams_impl(const nvtext_amd_list_strings_column* inpu
   v.use_mask = (input->null_mask != nullptr && input->null_count > 0) ? 1 : 0;
   v.child    = make_view(input->child);
   // (a view's child may hold more elements than the view: then the other way is taken, with the same result)
-  bool const short_rows = sizeof(T) == 8 && static_cast<double>(input->child.size) < short_row_length(P) * rows;
+  // Few elements have all their products computed as well: the plan need not lay the parameters out (256 parameters, whole and
+  // on the matrix cores: 31,000 elements 14.5 and 19.2 us, 126,000 23.1 and 26.7, 252,000 30.3 and 28.5).
+  constexpr int32_t kFewElements = 200000;
+  bool const short_rows = sizeof(T) == 8 && (input->child.size < kFewElements || static_cast<double>(input->child.size) < short_row_length(P) * rows);
   size_t const temp_bytes[3] = {kPlanBytes, static_cast<size_t>(rows + 1) * sizeof(uint32_t),
                                 sizeof(T) == 8 ? static_cast<size_t>(groups_of(P)) * sizeof(filter64::Group) : 0};
   TempParts<3> const temp(mr, temp_bytes);

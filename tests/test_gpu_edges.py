@@ -433,3 +433,30 @@ def test_characters_of_a_tile(nv, orc, width, lead):
     h1, h2 = host.slice(0, len(rows) - 1), host.slice(1, len(rows))
     got, exp = nv.jaccard_index(dev(nv, h1), dev(nv, h2), width).to_host(), orc.jaccard_index(h1, h2, width, nthreads=8)
     assert np.array_equal(got.values.view(np.uint32), exp.values.view(np.uint32))
+
+
+@pytest.mark.parametrize("count", [26, 64, 100, 260])
+@pytest.mark.parametrize("elements", [199_999, 200_000])
+def test_minhash64_ngrams_few_elements(nv, orc, count, elements):
+    """Lists of so many elements that their products are found on the matrix cores, and one less; the last group of parameters
+    full or not."""
+    rng = np.random.default_rng(count)
+    a, b = params(rng, count, 64)
+    lens = [700] * 280
+    lens += [elements - sum(lens)]
+    offsets = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    child = mixed_rows(rng, rng.integers(0, 12, elements))
+    lists = HostListStringsColumn(offsets, child, None, len(lens), 0, 0)
+    got = nv.minhash64_ngrams(nv.DeviceListStringsColumn.from_host(lists), 3, 5, a, b).to_host()
+    assert got.equals(orc.minhash64_ngrams(lists, 3, 5, a, b, nthreads=8))
+
+
+@pytest.mark.parametrize("rows", [3, 40, 700])
+@pytest.mark.parametrize("count", [1, 26, 33, 65, 100, 129, 260, 300])
+def test_minhash64_few_units(nv, orc, rows, count):
+    """Columns of fewer parts than wavefronts, done by chunks of two groups of parameters, and of some more; the last group
+    full or not."""
+    rng = np.random.default_rng(count)
+    a, b = params(rng, count, 64)
+    host = HostStringsColumn.from_pylist([random_text(rng, n).decode() for n in rng.integers(0, 200_000 // rows, rows)])
+    assert nv.minhash64(dev(nv, host), 5, a, b, 8).to_host().equals(orc.minhash64(host, 5, a, b, 8, nthreads=8))
