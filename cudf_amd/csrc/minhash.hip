@@ -303,7 +303,7 @@ struct MinimaAll {
 // What bounds it: 1,024 products take 150 to 165 cycles of a SIMD, 86 of them the two matrix instructions, beside which the
 // vector ALUs stand still but for some 20, 33 the sixteen-bit minima, 20 the ranking (with the shifts and three-way minima of
 // whole dwords that put every single product in order before: 160 beside the matrix instructions; 20,011 long rows, 128
-// parameters 3.73 -> 2.80 ms, 30,000 rows of 3000 bytes, 260 parameters 3.00 -> 2.06, 20,000 lists of 480 words, 256 parameters 627 -> 346 us).
+// parameters 3.73 -> 2.72 ms, 30,000 rows of 3000 bytes, 260 parameters 3.00 -> 2.06, 20,000 lists of 480 words, 256 parameters 627 -> 346 us).
 template <int GROUPS, int AT_ONCE>
 struct Minima64 {
   using T = uint64_t;

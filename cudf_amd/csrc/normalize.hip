@@ -2,8 +2,8 @@
 // (cpp/src/text/normalize.cu:219-573).
 //
 // The reference expands every input byte into three uint32 slots in global memory, fixes the special tokens up
-// in a second kernel, reduces the slots to row sizes and compacts them.  Here a workgroup takes a tile of
-// 2048 input bytes (plus a few either side), each lane keeps the slots of eight consecutive bytes in registers,
+// in a second kernel, reduces the slots to row sizes and compacts them.  Here a workgroup (in a large column a
+// wavefront) takes a tile of 2048 input bytes, plus a few either side, eight consecutive bytes to a lane,
 // and the column is walked twice: once to learn how many bytes each tile produces, once to write them,
 // coalesced, at the offsets a scan of those counts gives.  HBM sees the input twice and the output once; the
 // slots never leave the CU.
