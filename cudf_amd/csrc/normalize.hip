@@ -1217,19 +1217,21 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_kernel(ColVie
 }
 
 // The same for a column of many tiles, a wavefront a tile as in normalize_count_tiles_kernel: in steps of 512 bytes, whose
-// output is laid out in the wavefront's own part of LDS; the dword that a step leaves unfinished is the next one's first.
+// output is laid out in the wavefront's own part of LDS; the line that a step leaves unfinished is the next one's first.
 // Tiles that are not for this kernel are left for the workgroup to do together at the end.
 // What bounds it is vector instructions, the reads and or-writes of LDS beside them.  Longer characters are taken by fours
 // of bytes, two at most in each, with 32-bit arithmetic only; one-byte characters are placed in pairs; a row's place comes
-// from the lane that its first byte is with, not from a list of all places.  766 MB of mixed text 1250 -> 1010 us; a call with a
-// workgroup a tile and with this: 17 MB mixed 73.9 and 76.1 us, ASCII 68.0 and 63.3, 34 MB 105 and 102, 92.3 and 79.2, 134 MB
-// mixed 296 and 256.
+// from the lane that its first byte is with, not from a list of all places.  A step stores whole lines (of dwords: 10.2 GB of HBM
+// writes for 4.2 GB of output, and 2 to 4 % slower).  766 MB of mixed text 1250 -> 995 us; a call with a workgroup a tile and with
+// this: 17 MB mixed 73.9 and 76.1 us, ASCII 68.0 and 63.3, 34 MB 105 and 99, 92.3 and 75.6, 134 MB mixed 296 and 254.
 constexpr int kStep       = kWave * kNormItems;  // input bytes of a step
 constexpr int kStepBytes  = 4 * kStep;           // of output; a tile with more in a step is left
+constexpr int kLine       = 128;                 // bytes; a step stores whole lines only
+constexpr int kStepWords  = (kStepBytes + kLine) / 4 + 4;
 union WriteLds {
   struct {
     alignas(16) uint32_t raw[kTileWaves][kRawWords];
-    alignas(16) uint32_t staged[kTileWaves][kStepBytes / 4 + 4];
+    alignas(16) uint32_t staged[kTileWaves][kStepWords];
   };
   NormLds<true> tile;
 };
@@ -1274,7 +1276,7 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_tiles_kernel(
     look_up();
   }
   ascii[threadIdx.x] = table_entry;
-  for (int i = lane; i < (kStepBytes / 4 + 4) / 4; i += kWave) reinterpret_cast<uint4*>(staged)[i] = make_uint4(0u, 0u, 0u, 0u);
+  for (int i = lane; i < kStepWords / 4; i += kWave) reinterpret_cast<uint4*>(staged)[i] = make_uint4(0u, 0u, 0u, 0u);
   lds_barrier();
   bool marked = false;
   if (tile < tiles) {
@@ -1284,11 +1286,20 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_tiles_kernel(
     wave_lds_sync();
     uint64_t const base  = tile_offset[tile];
     uint8_t* const dst   = out_chars + base;
-    uint32_t const lead  = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(dst) & 3u);
+    uint32_t const lead  = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(dst) & (kLine - 1));
     uint32_t* const dw   = reinterpret_cast<uint32_t*>(dst - lead);
     uint32_t const shift = 8u * (mis & 3u);
-    uint32_t words       = 0;     // full dwords of the tile that are in memory
-    uint32_t in_first    = lead;  // bytes in the first dword of the buffer already
+    uint32_t words       = 0;     // dwords of the tile's lines that are in memory
+    uint32_t in_first    = lead;  // bytes of the buffer's first line that are there already
+    // dword w of the buffer, of the bytes [from, to) that are the tile's
+    auto const put = [&](uint32_t w, uint32_t d, uint32_t from, uint32_t to) {
+      if (4u * w >= from && 4u * w + 4u <= to) {
+        store_stream(dw + words + w, d);
+      } else {
+        for (uint32_t b = max(4u * w, from); b < min(4u * w + 4u, to); ++b)
+          reinterpret_cast<uint8_t*>(dw + words)[b] = static_cast<uint8_t>(d >> (8u * (b & 3u)));
+      }
+    };
     uint32_t done        = 0;     // bytes that the steps before produced
     bool const opened    = t.tokens > 0 && ballot64(opener_before(raw, lane, mis)) != 0;
     const uint32_t* own_raw = raw + ((mis + kRawBefore) >> 2) + 2 * lane;
@@ -1412,30 +1423,31 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_tiles_kernel(
         if (ballot64(past != 0u) != 0) atomicOr(to + 2, past);
       }
       wave_lds_sync();
-      // the full dwords to memory, zeros in their place; the unfinished one to the front
-      uint32_t const end = in_first + total, full = end >> 2;
-      uint32_t const rest = staged[full];
-      for (uint32_t w = lane; w < full; w += kWave) {
-        uint32_t const d = staged[w];
-        staged[w]        = 0u;
-        if (words + w != 0 || lead == 0) {
-          store_stream(dw + words + w, d);
-        } else {  // (the tile's first dword has bytes of the tile before)
-          for (uint32_t b = lead; b < 4u; ++b) reinterpret_cast<uint8_t*>(dw)[b] = static_cast<uint8_t>(d >> (8u * b));
+      // the whole lines to memory, zeros in their place; the unfinished one to the front
+      uint32_t const end = in_first + total, full = end / kLine * (kLine / 4);
+      uint32_t const rest = lane < kLine / 4 ? staged[full + lane] : 0u;
+      if (words != 0 || lead == 0) {
+        for (uint32_t w = lane; w < full; w += kWave) {
+          store_stream(dw + words + w, staged[w]);
+          staged[w] = 0u;
+        }
+      } else {  // (the tile's first line has bytes of the tile before)
+        for (uint32_t w = lane; w < full; w += kWave) {
+          put(w, staged[w], lead, 4u * full);
+          staged[w] = 0u;
         }
       }
       wave_lds_sync();
-      if (lane == 0) {
-        staged[full] = 0u;
-        staged[0]    = rest;
+      if (lane < kLine / 4) {
+        staged[full + lane] = 0u;
+        staged[lane]        = rest;
       }
       wave_lds_sync();
       words += full;
-      in_first = end & 3u;
+      in_first = end % kLine;
       done += total;
     }
-    if (!marked && lane >= (words == 0 ? lead : 0u) && lane < in_first)
-      reinterpret_cast<uint8_t*>(dw + words)[lane] = static_cast<uint8_t>(staged[0] >> (8u * lane));
+    if (!marked && lane < kLine / 4) put(lane, staged[lane], words == 0 ? lead : 0u, in_first);
     if (marked) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // what has been written is there before other wavefronts write it anew
   }
   if (lane == 0) left[wave] = marked ? 1u : 0u;
