@@ -719,12 +719,22 @@ __global__ void __launch_bounds__(kNormThreads, 8) normalize_count_kernel(const 
 // for no other.  Tiles that may hold a special token are left for the workgroup to do together at the end, as
 // normalize_count_kernel does them.
 // What bounds it is instructions again: with a workgroup a tile half the time went on barriers, on starting, on staging
-// the table and on a list for every 512 bytes.  766 MB of mixed text 461 -> 290 us; several tiles for a wavefront, with the bytes
+// the table and on a list for every 512 bytes.  766 MB of mixed text 461 -> 266 us; several tiles for a wavefront, with the bytes
 // of the next one on their way, no faster.  A small column has too few wavefronts this way: of 17 MB 73.5 us a call with a
 // workgroup a tile and 75.5 with this, of 34 MB 110 and 108, of 67 MB 180 and 172.
 constexpr int kTileWaves          = kNormThreads / kWave;
 constexpr int kLaneWords          = kNormTile / kWave / 4;  // dwords of a tile per lane, two of every 512 bytes
 constexpr int64_t kManyTiles      = 12288;                  // a column of so many tiles
+// Whether there is nothing for the end.  (Asked before the loop over the four: what the compiler gets ready for that loop it spills
+// to memory, 5 GB of HBM writes beside the 4.2 GB of a result.)
+__device__ __forceinline__ bool none_left(const uint32_t (&left)[kTileWaves])
+{
+  uint32_t any = 0;
+#pragma unroll
+  for (int k = 0; k < kTileWaves; ++k) any |= left[k];
+  return __builtin_amdgcn_readfirstlane(static_cast<int>(any)) == 0;
+}
+
 union CountLds {
   struct {
     alignas(16) uint32_t raw[kTileWaves][kRawWords];
@@ -831,6 +841,7 @@ __global__ void __launch_bounds__(kNormThreads, 8) normalize_count_tiles_kernel(
   if (t.tokens == 0) return;
   if (lane == 0) left[wave] = marked ? 1u : 0u;
   lds_barrier();
+  if (none_left(left)) return;
 #pragma unroll 1
   for (int k = 0; k < kTileWaves; ++k) {
     if (__builtin_amdgcn_readfirstlane(static_cast<int>(left[k])) == 0) continue;
@@ -1221,9 +1232,9 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_kernel(ColVie
 // Tiles that are not for this kernel are left for the workgroup to do together at the end.
 // What bounds it is vector instructions, the reads and or-writes of LDS beside them.  Longer characters are taken by fours
 // of bytes, two at most in each, with 32-bit arithmetic only; one-byte characters are placed in pairs; a row's place comes
-// from the lane that its first byte is with, not from a list of all places.  A step stores whole lines (of dwords: 10.2 GB of HBM
-// writes for 4.2 GB of output, and 2 to 4 % slower).  766 MB of mixed text 1250 -> 995 us; a call with a workgroup a tile and with
-// this: 17 MB mixed 73.9 and 76.1 us, ASCII 68.0 and 63.3, 34 MB 105 and 99, 92.3 and 75.6, 134 MB mixed 296 and 254.
+// from the lane that its first byte is with, not from a list of all places.  A step stores whole lines
+// (of dwords: 2 to 4 % slower).  766 MB of mixed text 1250 -> 927 us; a call with a workgroup a tile and with
+// this: 17 MB mixed 73.9 and 76.1 us, ASCII 68.0 and 63.3, 34 MB 105 and 94, 92.3 and 70.8, 134 MB mixed 296 and 235.
 constexpr int kStep       = kWave * kNormItems;  // input bytes of a step
 constexpr int kStepBytes  = 4 * kStep;           // of output; a tile with more in a step is left
 constexpr int kLine       = 128;                 // bytes; a step stores whole lines only
@@ -1452,6 +1463,7 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_tiles_kernel(
   }
   if (lane == 0) left[wave] = marked ? 1u : 0u;
   lds_barrier();
+  if (none_left(left)) return;
 #pragma unroll 1
   for (int k = 0; k < kTileWaves; ++k) {
     if (__builtin_amdgcn_readfirstlane(static_cast<int>(left[k])) == 0) continue;
