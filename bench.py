@@ -27,40 +27,40 @@ HBM_PEAK_GBS = 8000.0
 #
 # HBM bytes per launch (fetched, written) of the tokenizer kernels on the full C2 workload: FETCH_SIZE / WRITE_SIZE
 # scaled by a copy kernel of known size.
-TRAFFIC_SOURCE = "profiles/hbm_traffic_pmc_all_workloads.md (library sources at commit 75677a8)"
+TRAFFIC_SOURCE = "profiles/hbm_traffic_pmc_all_workloads.md (library sources at commit 0ec04b2)"
 MEASURED_TRAFFIC_C2 = {
-    "range_first_row_kernel": (16690018, 4691648),
-    "wordpiece_word_kernel": (1876821281, 1979659097),
-    "wordpiece_oov_kernel": (909811327, 878370418),
-    "wordpiece_emit_kernel": (1406376802, 901145955),
+    "range_first_row_kernel": (16690003, 4691648),
+    "wordpiece_word_kernel": (1876864981, 1978118882),
+    "wordpiece_oov_kernel": (909080378, 875698598),
+    "wordpiece_emit_kernel": (1406378820, 901102157),
 }
 # (the fetch counter prices a read that misses L2 at a whole 128-byte line whatever was asked for, and counts the misses
 # that the Infinity Cache serves: most of what the tokenizer fetches on C5 is lines of its 8 MB table and of its memo)
 MEASURED_TRAFFIC_C5_TOKENIZE = {
-    "range_first_row_kernel": (231340168, 6184320),
-    "wordpiece_word_kernel": (24724356379, 6767157192),
-    "wordpiece_oov_kernel": (21537812574, 2154480839),
-    "wordpiece_emit_kernel": (4801143244, 3328126492),
+    "range_first_row_kernel": (227044913, 6184320),
+    "wordpiece_word_kernel": (24710276233, 6765646192),
+    "wordpiece_oov_kernel": (21540135196, 2153960620),
+    "wordpiece_emit_kernel": (4801087252, 3328148076),
 }
 MEASURED_TRAFFIC_C5_NORMALIZE = {
-    "normalize_count_kernel": (4574919108, 63532927),
-    "normalize_tile_rows_kernel": (73443774, 7941632),
-    "normalize_write_kernel": (5468198057, 4674851582),
+    "normalize_count_kernel": (4196028351, 15883232),
+    "normalize_tile_rows_kernel": (73439045, 7941632),
+    "normalize_write_kernel": (4464463216, 4405365019),
 }
 # minhash: VALU wave-instructions executed per (window, parameter) of a wavefront (SQ_INSTS_VALU / (windows x P / 64)) and
 # the share of SIMD cycles that issued one (SQ_INSTS_VALU x 4 / (1024 SIMDs x kernel cycles), capped at 1: adds and
 # moves issue in fewer than 4 cycles).  A product that is folded takes, in the inner loop: uint32, one v_mad_u64_u32 and
-# half a v_min3_u32 (1.5); uint64, where the matrix cores find products to 17 bits, 40.5 instructions for the 16 products
-# that a lane has of 1,024 (2.53), beside two matrix instructions of 32 cycles, which keep the matrix cores busy for 40 %
+# half a v_min3_u32 (1.5); uint64, where the matrix cores find products to 16 bits, 15 two-way minima and 5 that rank the
+# least for the 16 products that a lane has of 1,024 (1.25), beside two matrix instructions that take more than half
 # of the time that takes.  Windows of a row repeat, and a window met before need not be folded again: the floor counts the
 # different windows of a row only (their share is found on the first rows of the workload), the measured figure is over
 # all of them.
-VALU_SOURCE = "profiles/valu_issue_pmc_all_workloads.md (library sources at commit 75677a8)"
-PRODUCT_INST = {32: 1.5, 64: 2.53}
+VALU_SOURCE = "profiles/valu_issue_pmc_all_workloads.md (library sources at commit 0ec04b2)"
+PRODUCT_INST = {32: 1.5, 64: 1.25}
 MINHASH_VALU = {
-    "C3": {"bits": 32, "measured": 1.48, "issue": 1.04},
-    "C4": {"bits": 64, "measured": 3.59, "issue": 0.86},
-    "C5": {"bits": 64, "measured": 6.91, "issue": 0.84},
+    "C3": {"bits": 32, "measured": 1.47, "issue": 1.05},
+    "C4": {"bits": 64, "measured": 2.80, "issue": 1.00},
+    "C5": {"bits": 64, "measured": 6.04, "issue": 0.96},
 }
 
 
