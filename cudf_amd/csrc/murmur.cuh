@@ -112,8 +112,8 @@ __device__ __forceinline__ void murmur3_x64_128_lo(Src const (&src)[N], uint32_t
   uint64_t h1[N], h2[N];
 #pragma unroll
   for (int n = 0; n < N; ++n) h1[n] = h2[n] = seed;
-  for (uint32_t t = 0; t < len; t += 16) {
-    uint32_t const left = len - t, at = t / 4u;
+  // (what is left is counted, not where the block begins: that wraps where the last one begins in the last 15 bytes below 2^32)
+  for (uint32_t left = len, at = 0; left != 0; left -= min(left, 16u), at += 4) {
 #pragma unroll
     for (int n = 0; n < N; ++n) {
       uint64_t const k1 = static_cast<uint64_t>(src[n].dword(at + 1)) << 32 | src[n].dword(at);
