@@ -1385,10 +1385,14 @@ nvtext_amd_status minhash_ngrams_impl(const nvtext_amd_list_strings_column* inpu
   v.use_mask = (input->null_mask != nullptr && input->null_count > 0) ? 1 : 0;
   v.child    = make_view(input->child);
   // (a view's child may hold more elements than the view: then the other way is taken, with the same result)
-  // Few elements have all their products computed as well: the plan need not lay the parameters out (256 parameters, whole and
-  // on the matrix cores: 31,000 elements 14.5 and 19.2 us, 126,000 23.1 and 26.7, 252,000 30.3 and 28.5).
+  // Few elements have all their products computed as well, while there are not many of these: the plan need not lay the parameters
+  // out.  The lines are where no length of list is slower on the matrix cores (us whole and there: lists of 2500 elements, 256
+  // parameters, 160,000 elements 23.4 and 26.9, 260,000 32.1 and 31.1; lists of 150, 512 parameters, 160,000: 39.6 and 44.6; 1024,
+  // 90,000: 43.4 and 46.4, 130,000: 55.8 and 56.0, of 2500 52.8 and 47.2; 2048, 60,000: 54.1 and 55.0, of 2500 54.0 and 43.2).
   constexpr int32_t kFewElements = 200000;
-  bool const short_rows = sizeof(T) == 8 && (input->child.size < kFewElements || static_cast<double>(input->child.size) < short_row_length(P) * rows);
+  constexpr int64_t kFewProducts = 125000000;
+  bool const few        = input->child.size < kFewElements && static_cast<int64_t>(input->child.size) * P < kFewProducts;
+  bool const short_rows = sizeof(T) == 8 && (few || static_cast<double>(input->child.size) < short_row_length(P) * rows);
   size_t const temp_bytes[3] = {kPlanBytes, static_cast<size_t>(rows + 1) * sizeof(uint32_t),
                                 sizeof(T) == 8 ? static_cast<size_t>(groups_of(P)) * sizeof(filter64::Group) : 0};
   TempParts<3> const temp(mr, temp_bytes);

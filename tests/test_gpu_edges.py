@@ -435,14 +435,13 @@ def test_characters_of_a_tile(nv, orc, width, lead):
     assert np.array_equal(got.values.view(np.uint32), exp.values.view(np.uint32))
 
 
-@pytest.mark.parametrize("count", [26, 64, 100, 260])
-@pytest.mark.parametrize("elements", [199_999, 200_000])
+@pytest.mark.parametrize("elements, count", [(n, c) for c in (26, 64, 100, 260) for n in (199_999, 200_000)] + [(122_070, 1024), (122_071, 1024)])
 def test_minhash64_ngrams_few_elements(nv, orc, count, elements):
-    """Lists of so many elements that their products are found on the matrix cores, and one less; the last group of parameters
-    full or not."""
+    """Lists of so many elements (200,000), or of so many products of them and the parameters (125,000,000), that these are found on the
+    matrix cores, and one element less; the last group of parameters full or not."""
     rng = np.random.default_rng(count)
     a, b = params(rng, count, 64)
-    lens = [700] * 280
+    lens = [700] * (elements // 714)
     lens += [elements - sum(lens)]
     offsets = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     child = mixed_rows(rng, rng.integers(0, 12, elements))
