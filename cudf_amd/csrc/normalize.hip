@@ -1243,6 +1243,7 @@ union WriteLds {
   struct {
     alignas(16) uint32_t raw[kTileWaves][kRawWords];
     alignas(16) uint32_t staged[kTileWaves][kStepWords];
+    uint32_t third[kTileWaves][4][kWave];  // the last four bytes of strings of more than eight
   };
   NormLds<true> tile;
 };
@@ -1333,6 +1334,10 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_tiles_kernel(
       // up to two longer characters in each four bytes: text has no more
       uint32_t d0[4] = {}, d1[4] = {}, at8[4] = {};
       uint64_t holders[4] = {};
+      // Strings of more than eight bytes, those of most Hangul syllables in lower case: their last four go through LDS to a pass of their
+      // own.  (Left for the workgroup as before, 80 MB of Korean text took 377 us, with a workgroup a tile 369, and takes 238; in
+      // registers, or with a branch for each of the four, other text took 1 to 10 % longer.)
+      bool any_wide       = false;
       if (any_long) {
         uint4 e[4];
         uint32_t flags = 0;
@@ -1355,14 +1360,26 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_tiles_kernel(
           }
           if (k & 1) flags |= l & (l - 1u);
         }
+        flags |= e[0].w | e[1].w | e[2].w | e[3].w;
+        if (ballot64((flags & (kNotShort | 0x808080u)) != 0u) != 0) {  // (seldom)
+          // (read from the table once more: whole entries above are 7 to 10 % of other text's time)
+          any_wide = true;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            uint32_t const more  = leads[k / 2] & (leads[k / 2] - 1u), w = __builtin_amdgcn_alignbit(own[k / 2 + 1], own[k / 2], at8[k]);
+            bool const not_short = (e[k].w & kNotShort) != 0u;
+            e[k].w &= 0xFFu;
+            // (" [ ": an over-long '[')
+            other = other || (more & (more - 1u)) != 0u || (not_short && (e[k].w <= 8u || (w & 0xFFu) >= 0xF0u));
+            lds.third[wave][k][lane] = not_short ? t.bmp[0x10000u + decode_short(w)].z : 0u;
+          }
+        }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           d0[k] = e[k].x;
           d1[k] = e[k].y;
-          flags |= e[k].w;
           sizes[k / 2] += e[k].w << at8[k];
         }
-        other = other || (flags & (kNotShort | 0x808080u)) != 0u;
       }
       // where each position's bytes begin in the lane's: the sums of the sizes before it (88 at most)
       uint32_t const in0 = sizes[0] * 0x01010101u;
@@ -1432,6 +1449,15 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_tiles_kernel(
         atomicOr(to, static_cast<uint32_t>(both));
         atomicOr(to + 1, static_cast<uint32_t>(both >> 32));
         if (ballot64(past != 0u) != 0) atomicOr(to + 2, past);
+      }
+      if (any_wide) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          uint32_t const at    = o + (((k < 2 ? ex0 : ex1) >> at8[k]) & 0xFFu) + 8u;
+          uint64_t const third = static_cast<uint64_t>(lds.third[wave][k][lane]) << (8u * (at & 3u));
+          atomicOr(staged + (at >> 2), static_cast<uint32_t>(third));
+          atomicOr(staged + (at >> 2) + 1, static_cast<uint32_t>(third >> 32));
+        }
       }
       wave_lds_sync();
       // the whole lines to memory, zeros in their place; the unfinished one to the front

@@ -278,18 +278,24 @@ def test_normalize_feeds_the_tokenizer(nv, onorm):
     assert got.child.size > 3 * 3000
 
 
-@pytest.mark.parametrize("kind", ["plain", "tokens", "bytes"])
+@pytest.mark.parametrize("kind", ["plain", "tokens", "bytes", "wide"])
 @pytest.mark.parametrize("skip,extra", [(0, 0), (1, 1), (2, 2047), (3, 12345)])
 def test_normalize_wavefront_a_tile(nv, onorm, kind, skip, extra):
     """Columns so large that a wavefront counts whole tiles, and just below that: the tiles' number is no multiple of the
-    workgroups', characters and special tokens lie across every border, the first byte has any alignment."""
+    workgroups', characters and special tokens lie across every border, the first byte has any alignment.  "wide":
+    characters that turn into nine and twelve bytes, alone, side by side and in every place, few over-long brackets among them."""
     rng = np.random.default_rng(7 + skip)
     pieces = [b"word", b" ", b" a", b"Th", b"\xc3\xa9t\xc3\xa9", "漢字".encode(), "Жи".encode(), b".", b"),", b"\t", "\U0001F600".encode()]
-    if kind != "plain":
+    if kind == "wide":
+        pieces = ["한글각".encode(), "힣".encode(), "가".encode(), "a각b".encode(), "\U0001D160".encode(), "\U0001D15Fé".encode()] * 2 + pieces
+        pieces.append(b"\xc1\x9bSEP]")
+    elif kind != "plain":
         pieces += [b"[", b"]", b"[SEP]", b" [sep] ", b"[ Pad ]", b"\xc1\x9bSEP]", b"\xe0\x81\x9bPAD]"]
     if kind == "bytes":
         pieces += [b"\xff", b"\x80\x80", b"\xc3\xc3\xe4", b"\xf0\xf0\xf0\xf0\xf0\xf0\xf0\xf0", b"\xc3", b"\0"]
     which = rng.integers(0, len(pieces), 60001)
+    if kind == "wide":
+        which = np.where(rng.random(which.size) < 0.9997, rng.integers(0, len(pieces) - 1, which.size), len(pieces) - 1)
     if kind == "tokens":
         which = np.where(rng.random(which.size) < 0.97, rng.integers(0, 11, which.size), which)
     part = np.frombuffer(b"".join(pieces[i] for i in which), np.uint8)
