@@ -29,13 +29,16 @@ def random_text(rng, n, alphabet=b"abcdefghijklmnopqrstuvwxyz"):
     return bytes(rng.choice(np.frombuffer(alphabet, np.uint8), n))
 
 
+JACCARD_SLOTS = (1024, 4096, 7008, 15488, 29440)  # of the sets in LDS
+
+
 @pytest.mark.parametrize("width", [2, 7, 40])
 def test_jaccard_sets_and_shares(nv, orc, width):
-    """Pairs one byte around the most that each set takes (4/5 of 1024, 4096, 7008, 15488 and 29440 slots), rows one window
+    """Pairs of the most bytes that each set takes (4/5 of 1024, 4096, 7008, 15488 and 29440 slots) and of one more, rows one window
     around whole units of 64, and of very different lengths, so that a wavefront's share ends in the one or the other."""
     rng = np.random.default_rng(width)
-    sizes = [(n * 4 // 5 + d) // 2 * 2 for n in (1024, 4096, 7008, 15488, 29440) for d in (0, 2)]
-    lens = [(n // 2 + d, n // 2 - d) for n in sizes for d in (0, 1, n // 3)]
+    sizes = [n * 4 // 5 + d for n in JACCARD_SLOTS for d in (0, 1)]
+    lens = [(n // 2 + d, n - n // 2 - d) for n in sizes for d in (0, 1, n // 3)]
     lens += [(64 * k + width - 1 + d, 64 * m + width - 1 + e) for k, m in ((1, 0), (4, 5), (9, 23), (31, 16)) for d in (-1, 0, 1) for e in (-1, 0, 1)]
     left = [random_text(rng, max(n, 0)).decode() for n, _ in lens]
     right = [(a[: m // 2] + random_text(rng, max(m, 0) - len(a[: m // 2])).decode()) for a, (_, m) in zip(left, lens)]
@@ -44,29 +47,54 @@ def test_jaccard_sets_and_shares(nv, orc, width):
     assert np.array_equal(got.values.view(np.uint32), exp.values.view(np.uint32))
 
 
-def home_buckets(words, buckets):
-    """Where windows of four bytes belong in a set: the top of the product of their hash (MurmurHash3_x86_32, seed 0, without
-    the final mix)."""
+def jaccard_set(size):
+    """The slots of the set that a pair of so many bytes gets, and the parts that it is cut into."""
+    if size <= 1024 * 4 // 5:
+        return 1024, 1
+    tier = next((n for n in JACCARD_SLOTS if size <= n * 4 // 5), None)
+    return (29440, -(-size // 20_000)) if tier is None else (min(tier, max(1024, (2 * size + 63) // 32 * 32)), 1)
+
+
+def jaccard_places(words, buckets, parts):
+    """Where windows of four bytes belong in a set, and in which part: the top of products of their hash (MurmurHash3_x86_32, seed
+    0, without the final mix)."""
+    def top(v, n):
+        return v.astype(np.uint64) * np.uint64(n) >> np.uint64(32)
     with np.errstate(over="ignore"):
         k = words * np.uint32(0xCC9E2D51)
         k = (k << np.uint32(15) | k >> np.uint32(17)) * np.uint32(0x1B873593)
         h = ((k << np.uint32(13) | k >> np.uint32(19)) * np.uint32(5) + np.uint32(0xE6546B64)) ^ np.uint32(4)
-        return (h * np.uint32(0x9E3779B1)).astype(np.uint64) * np.uint64(buckets) >> np.uint64(32)
+        return top(h * np.uint32(0x9E3779B1), buckets), top((h ^ h >> np.uint32(15)) * np.uint32(0x85EBCA6B), parts)
 
 
-@pytest.mark.parametrize("count", [90, 190, 450, 1000])
-def test_jaccard_values_of_one_bucket(nv, orc, count):
-    """Words that all belong in one bucket: 90 that find a place within the 64 buckets that a packed set looks at from there,
-    and more than these hold (the last is 111, 179 and 393 buckets from home), so that the pair is done with a plain set,
-    among pairs that are not."""
+def furthest_from_home(text, buckets, parts):
+    """Buckets from the home of a window of four bytes to where it finds a place, the most of part 0."""
+    windows = np.unique(text[:-3] | text[1:-2].astype(np.uint32) << 8 | text[2:-1].astype(np.uint32) << 16 | text[3:].astype(np.uint32) << 24)
+    home, part = jaccard_places(windows, buckets, parts)
+    filled, furthest = [0] * buckets, 0
+    for b in home[part == 0].tolist():
+        far = 0
+        while filled[b] == 4:
+            b, far = (b + 1) % buckets, far + 1
+        filled[b] += 1
+        furthest = max(furthest, far)
+    return furthest
+
+
+@pytest.mark.parametrize("count, slots, parts", [(90, 1024, 1), (190, 1024, 1), (600, 4096, 1), (1000, 7008, 1), (2000, 15488, 1), (5000, 29440, 1), (7000, 29440, 2)])
+def test_jaccard_values_of_neighbouring_buckets(nv, orc, count, slots, parts):
+    """Words that belong in one bucket of their set, or in a few side by side: 90 that find a place within the 64 buckets that a
+    packed set looks at from there, and so many in sets of every size that some do not, so that the pair is done once more with
+    a plain set, or, where one of its parts has them all, with the one in global memory; among pairs that are not."""
     rng = np.random.default_rng(count)
+    assert jaccard_set(4 * count) == (slots, parts)
     letters = np.arange(97, 123, dtype=np.uint32)
     words = (letters[:, None, None, None] | letters[:, None, None] << 8 | letters[:, None] << 16 | letters << 24).astype(np.uint32).ravel()
-    slots = min({90: 1024, 190: 1024, 450: 4096, 1000: 15488}[count], max(1024, (2 * 4 * count + 63) // 32 * 32))
-    home = home_buckets(words, slots // 4)
-    near = words[home // max(1, slots // 4 // 256) == 77 % (slots // 4)][:count]
-    assert len(near) > 80
-    text = near.view(np.uint8).reshape(-1, 4)
+    home, part = jaccard_places(words, slots // 4, parts)
+    from_there = np.flatnonzero((part == 0) & (home >= 77))
+    near = from_there[np.argsort(home[from_there], kind="stable")][:count]
+    text = rng.permutation(words[near]).view(np.uint8).reshape(-1, 4)
+    assert (furthest_from_home(text.ravel(), slots // 4, parts) >= 64) == (count != 90)
     row = lambda pick: bytes(text[pick].ravel()).decode()
     n = len(text)
     left = [row(np.arange(n * 3 // 4)), "some other text", row(np.arange(n // 2))] * 3
@@ -78,10 +106,10 @@ def test_jaccard_values_of_one_bucket(nv, orc, count):
 
 @pytest.mark.parametrize("width", [2, 7, 40])
 def test_jaccard_pair_sizes(nv, orc, width):
-    """Pairs one byte around the most that each set takes (4/5 of 1024, 4096, 8064, 14336 and 29440 slots), around one
+    """Pairs of the most bytes that each set takes (4/5 of its slots) and of one more, around one
     and several parts of 20,000 bytes, and around the most parts (16); no window repeats, so the sets are as full as they get."""
     rng = np.random.default_rng(width)
-    sizes = [n * 4 // 5 + d for n in (1024, 4096, 8064, 14336, 29440) for d in (0, 1)]
+    sizes = [n * 4 // 5 + d for n in JACCARD_SLOTS for d in (0, 1)]
     sizes += [40_000, 40_001, 60_001, 320_000, 320_001, 1, 2, 63, 64, 65]
     left, right = [], []
     for n in sizes:

@@ -310,3 +310,30 @@ def test_normalize_wavefront_a_tile(nv, onorm, kind, skip, extra):
         got = run(nv, host, True, tokens)
         exp = onorm.normalize_characters_native(host, True, [t.encode() for t in tokens], 8)
         assert_same(got, exp, f"{kind} {tiles}")
+
+
+@pytest.mark.parametrize("per_tile", [1, 63, 64, 65, 128, 129, 700])
+def test_normalize_rows_of_a_wavefronts_tile(nv, onorm, per_tile):
+    """Tiles that a wavefront writes alone, with as many rows in each as it has lanes, one less and more, twice as many, and
+    rows that are mostly empty; some begin in the last byte of a tile, the last row ends with the last tile."""
+    rng = np.random.default_rng(per_tile)
+    tiles = 12288
+    part = np.frombuffer(("word Été 漢字, (a) " * 30).encode(), np.uint8)
+    chars = np.resize(part, tiles * TILE)
+    ends = np.concatenate([np.sort(rng.integers(0, TILE, (64, per_tile)), axis=1)] * (tiles // 64)) + TILE * np.arange(tiles)[:, None]
+    ends[5, -1] = 6 * TILE - 1
+    offsets = np.concatenate([[0], ends.ravel(), [tiles * TILE] * 3]).astype(np.int64)
+    host = HostStringsColumn(chars, offsets, None, offsets.size - 1, 0, 0)
+    assert_same(run(nv, host, True, ("[SEP]",)), onorm.normalize_characters_native(host, True, [b"[SEP]"], 8), f"{per_tile} rows")
+
+
+@pytest.mark.parametrize("rows, tiles", [(131_072, 12288), (131_072, 12287), (40_000, 16384)])
+def test_normalize_wavefront_a_tile_after_one_wait(nv, onorm, rows, tiles):
+    """Columns of few enough rows and bytes (64 MiB) to be worked on before their size is known, and of so many tiles that a
+    wavefront writes each; one tile less."""
+    rng = np.random.default_rng(rows + tiles)
+    chars = np.resize(np.frombuffer("Some [SEP] words, Été 漢字 Жи 각 and more plain words of text. ".encode(), np.uint8), tiles * TILE)
+    offsets = np.concatenate([[0], np.sort(rng.integers(0, tiles * TILE, rows - 1)), [tiles * TILE]]).astype(np.int32)
+    host = HostStringsColumn(chars, offsets, None, rows, 0, 0)
+    for tokens in ((), ("[SEP]",)):
+        assert_same(run(nv, host, True, tokens), onorm.normalize_characters_native(host, True, [t.encode() for t in tokens], 8), f"{tokens}")
