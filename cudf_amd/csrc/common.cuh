@@ -312,21 +312,12 @@ __device__ __forceinline__ void wave_lds_fence()
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ uint32_t add_saturating(uint32_t a, uint32_t b) { return __builtin_elementwise_add_sat(a, b); }
-
 // (written out, the compiler shares its inner minimum with a three-way minimum next to it, which then takes two instructions)
 __device__ __forceinline__ uint32_t median(uint32_t a, uint32_t b, uint32_t c)
 {
   uint32_t m;
   asm("v_med3_u32 %0, %1, %2, %3" : "=v"(m) : "v"(a), "v"(b), "v"(c));
   return m;
-}
-
-// The smaller of what a lane and the one 32 places away hold.
-__device__ __forceinline__ uint32_t min_of_halves(uint32_t v)
-{
-  auto const both = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  return min(both[0], both[1]);
 }
 
 // Workgroup exclusive scan of one uint32 per thread.  `lds` needs (blockDim/64 + 1) words.
