@@ -4,10 +4,11 @@
 A step is one wordpiece_tokenize call over the whole synthetic batch of configuration C2
 (4M rows, lognormal mean 256 B, Zipf(1.1) words over a 30,522-entry vocabulary, 15 % OOV,
 int32 offsets, max_words_per_row=128), inputs resident in HBM, output allocation included.
-Prints one JSON line: input GB/s as `value`, plus Mrows/s, the roofline of the whole call,
-the host-oracle baseline on a bounded sample, the minhash / minhash64 figures (configurations
-C3 / C4 at a stated scale), the UTF-8 pipeline of C5 and the reference's own benchmark shapes.
-Every leg carries the mean and the median step time and the device memory a call holds at its peak.
+Prints one JSON line: input GB/s as `value`, plus Mrows/s, the roofline of the whole call, the
+host-oracle baseline on a bounded sample, and of every other leg (minhash / minhash64 on
+configurations C3 / C4, minhash_ngrams, jaccard_index, the UTF-8 pipeline of C5, the reference's own
+benchmark shapes) milliseconds, input GB/s and parity.  Everything measured (the mean and the median
+step time, kernels, the device memory a call holds at its peak, ...) goes to stderr as one line before it.
 """
 import argparse
 import json
@@ -561,8 +562,34 @@ def main():
     if line is None:
         line = {"metric": "input GB/s + Mrows/s, wordpiece_tokenize & minhash, 1 MI355X, % of roofline", "value": None, "unit": "GB/s",
                 "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "legs": sorted(legs)}
-    line.update(extra)
-    print(json.dumps(line), flush=True)
+    log("[bench] everything: " + json.dumps({**line, **extra}))
+    if line.get("roofline"):
+        line["roofline"] = {k: v for k, v in line["roofline"].items() if k not in ("traffic_per_kernel", "traffic_source", "all_kernels_ms")}
+    if line.get("cpu_baseline"):
+        line["cpu_baseline"] = {k: v for k, v in line["cpu_baseline"].items() if k not in ("cores_from", "hardware_concurrency")}
+    print(json.dumps({**line, "legs": legs_in_short(extra)}), flush=True)
+
+
+def legs_in_short(extra):
+    """[ms per call, input GB/s] of every leg, and the names of those that differ from the host oracle."""
+    short, failed = {}, []
+
+    def figures(name, leg):
+        if "FAIL" in str(leg.get("parity", "")):
+            failed.append(name)
+        return [leg["ms_per_step"], leg.get("input_GBps")]
+
+    def add(name, leg):
+        if isinstance(leg, list):
+            short[name] = [figures(f"{name}.{i}", part) for i, part in enumerate(leg)]
+        elif "ms_per_step" in leg:
+            short[name] = figures(name, leg)
+        else:
+            for key, part in leg.items():
+                if isinstance(part, (dict, list)):
+                    add(f"{name}.{key}" if name else key, part)
+    add("", extra)
+    return {**short, "differ_from_oracle": failed}
 
 
 def reference_shapes(args, orc, _capi, datagen, nvtext, HostStringsColumn, np, torch):
