@@ -86,7 +86,8 @@ __host__ __device__ inline uint32_t lay_out(uint64_t a, uint64_t b, Put&& put)
   // 31 counts twice
   uint64_t const need = (((b & kPrime) + 3 * low) >> kUnitShift) + 2;
   int32_t bias        = static_cast<int32_t>((need + 1) & ((1u << kUnits) - 2));
-  // the sums have 32 wholes of room on either side and take at most 31.1 (every digit of a / 2^61 to the base 4 is 1, or 2)
+  // the sums have 64 wholes of room on either side (2^22 units around 6.0) and take at most 31.2 (every digit of a / 2^61 to the base 4
+  // is 1, or 2)
   if (above > below) bias -= 1 << kUnits;
   put(31, bias / 2);
   return static_cast<uint32_t>((3 * (low + high)) >> kUnitShift) + 4;

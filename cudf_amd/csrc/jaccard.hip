@@ -66,7 +66,7 @@ __device__ __forceinline__ int list_of(int64_t bytes)
 //
 // The set of a pair whose windows LDS has room for.  A slot holds 24 bits of the value's product, which tell the values of one
 // home bucket apart where there are 256 buckets and more, how many buckets from home it lies (6 bits), and two bits that say
-// which rows it occurs in: one compare-and-swap places a value and marks it, a value that is there already is marked with
+// which rows it occurs in: one compare-and-swap places a value and marks it, where that finds the value there already it is marked with
 // an or of a constant to the same address, and counting is a pass over the slots.  (With whole values and the bits in arrays
 // of their own a look took 65 vector instructions for 128 windows, beside 65 for their hashes; now 55.)
 struct PackedSet {

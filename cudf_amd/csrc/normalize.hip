@@ -719,7 +719,7 @@ __global__ void __launch_bounds__(kNormThreads, 8) normalize_count_kernel(const 
 // for no other.  Tiles that may hold a special token are left for the workgroup to do together at the end, as
 // normalize_count_kernel does them.
 // What bounds it is instructions again: with a workgroup a tile half the time went on barriers, on starting, on staging
-// the table and on a list for every 512 bytes.  766 MB of mixed text 461 -> 266 us; several tiles for a wavefront, with the bytes
+// the table and on a list for every 512 bytes.  766 MB of mixed text 461 -> 255 to 266 us (traced); several tiles for a wavefront, with the bytes
 // of the next one on their way, no faster.  A small column has too few wavefronts this way: of 17 MB 73.5 us a call with a
 // workgroup a tile and 75.5 with this, of 34 MB 110 and 108, of 67 MB 180 and 172.
 constexpr int kTileWaves          = kNormThreads / kWave;
@@ -1233,8 +1233,8 @@ __global__ void __launch_bounds__(kNormThreads, 6) normalize_write_kernel(ColVie
 // What bounds it is vector instructions, the reads and or-writes of LDS beside them.  Longer characters are taken by fours
 // of bytes, two at most in each, with 32-bit arithmetic only; one-byte characters are placed in pairs; a row's place comes
 // from the lane that its first byte is with, not from a list of all places.  A step stores whole lines
-// (of dwords: 2 to 4 % slower).  766 MB of mixed text 1250 -> 927 us; a call with a workgroup a tile and with
-// this: 17 MB mixed 73.9 and 76.1 us, ASCII 68.0 and 63.3, 34 MB 105 and 94, 92.3 and 70.8, 134 MB mixed 296 and 235.
+// (of dwords: 2 to 4 % slower).  766 MB of mixed text 1250 -> 883 to 927 us (traced, as the call then takes 1209 us and more; without
+// a trace 1125); a call with a workgroup a tile and with this: 17 MB mixed 73.9 and 76.1 us, ASCII 68.0 and 63.3, 34 MB 105 and 94, 92.3 and 70.8, 134 MB mixed 296 and 235.
 constexpr int kStep       = kWave * kNormItems;  // input bytes of a step
 constexpr int kStepBytes  = 4 * kStep;           // of output; a tile with more in a step is left
 constexpr int kLine       = 128;                 // bytes; a step stores whole lines only

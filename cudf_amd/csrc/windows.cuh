@@ -27,7 +27,7 @@ constexpr uint32_t kFoldFrom = 416;
 // has been folded once changes no minimum when it is folded again.  Every wavefront keeps the hashes it saw last in a
 // small direct-mapped table (of 64-bit hashes, the places that they have among those gathered: 2 KB for 1024 where 512
 // hashes took 4) and drops a hash that it finds there; what the table has forgotten is folded again, which
-// costs time and nothing else.  Cleared (hashes are never 0) whenever the wavefront begins a row.  As many entries as leave
+// costs time and nothing else.  Cleared (hashes are never 0) whenever the wavefront begins a part of a row.  As many entries as leave
 // six (64-bit hashes: four) workgroups to a CU: 400,000 documents of 2 KB, 256 parameters of 32 bits: 256 entries 8.80 ms,
 // 512: 8.45, 1024: 8.17.
 constexpr uint32_t kRecentEntries = 1024;
