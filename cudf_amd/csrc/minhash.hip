@@ -680,6 +680,7 @@ struct ListView {
 
 // Byte source over global memory through aligned dword loads that overlap [p, p + len) only.
 struct AlignedSrc {
+  static constexpr bool kInTile = false;
   const uint32_t* w;  // aligned address at or below the first byte
   uint32_t mis;       // first byte inside w[0]
   uint32_t end;       // mis + len

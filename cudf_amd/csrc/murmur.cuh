@@ -24,6 +24,7 @@ __device__ __forceinline__ uint32_t keep_low_bytes(uint32_t v, int nbytes)
 // dword(k), bytes 4k to 4k + 3 of the window, may read up to 11 bytes past the window (callers mask what they do not need).
 // (A shift of two aligned dwords: an unaligned read of LDS takes a cycle a lane.)
 struct WordSrc {
+  static constexpr bool kInTile = true;  // its windows are no longer than a tile of a row
   const uint32_t* at;  // the dword with the window's first byte
   uint32_t mis;        // where in it
   __device__ __forceinline__ WordSrc(const uint32_t* w, uint32_t base) : at(w + (base >> 2)), mis(base & 3u) {}
@@ -34,6 +35,7 @@ struct WordSrc {
 // Byte source over global memory that never touches a byte at or past `avail`
 // (slow; used only for windows too wide for the LDS tile).
 struct BoundedSrc {
+  static constexpr bool kInTile = false;
   const uint8_t* p;
   int64_t avail;
   __device__ __forceinline__ uint32_t byte(uint32_t i) const { return p[i]; }
@@ -112,8 +114,10 @@ __device__ __forceinline__ void murmur3_x64_128_lo(Src const (&src)[N], uint32_t
   uint64_t h1[N], h2[N];
 #pragma unroll
   for (int n = 0; n < N; ++n) h1[n] = h2[n] = seed;
-  // (what is left is counted, not where the block begins: that wraps where the last one begins in the last 15 bytes below 2^32)
-  for (uint32_t left = len, at = 0; left != 0; left -= min(left, 16u), at += 4) {
+  // (behind the last block of a length just below 2^32 the place of the next one has wrapped: the byte before it tells)
+  bool more = len != 0;
+  for (uint32_t t = 0; more; t += 16, more = Src::kInTile ? t < len : t - 1u < len - 1u) {
+    uint32_t const left = len - t, at = t / 4u;
 #pragma unroll
     for (int n = 0; n < N; ++n) {
       uint64_t const k1 = static_cast<uint64_t>(src[n].dword(at + 1)) << 32 | src[n].dword(at);

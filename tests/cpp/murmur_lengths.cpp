@@ -17,7 +17,9 @@ using std::min;
 static inline uint32_t key_dword(uint64_t k) { return static_cast<uint32_t>(k) * 0x9E3779B1u ^ static_cast<uint32_t>(k >> 7); }
 static inline uint64_t key_byte(uint64_t i) { return key_dword(i / 4) >> (8 * (i % 4)) & 0xFFu; }
 
+template <bool IN_TILE>
 struct Bytes {
+  static constexpr bool kInTile = IN_TILE;
   mutable uint32_t furthest = 0;
   uint32_t byte(uint32_t i) const { return static_cast<uint32_t>(key_byte(i)); }
   uint32_t dword(uint32_t k) const
@@ -75,17 +77,17 @@ static void check(bool same, uint32_t len)
   std::printf("%u bytes: another hash\n", len);
   std::exit(1);
 }
-template <int N>
+template <int N, bool IN_TILE>
 static void check64(uint32_t len)
 {
-  Bytes const src[N] = {};
+  Bytes<IN_TILE> const src[N] = {};
   uint64_t h[N];
   nvtext_amd::murmur3_x64_128_lo<N>(src, len, 7, h);
   for (uint64_t const v : h) check(v == published64(len, 7), len);
 }
 static void check32(uint32_t len)
 {
-  Bytes const src[1] = {};
+  Bytes<false> const src[1] = {};
   uint32_t h[1];
   nvtext_amd::murmur3_x86_32<1>(src, len, 42, h);
   check(h[0] == published32(len, 42), len);
@@ -94,10 +96,11 @@ static void check32(uint32_t len)
 int main()
 {
   for (uint32_t len = 0; len <= 100; ++len) {
-    check64<2>(len);
+    check64<2, true>(len);
+    check64<1, false>(len);
     check32(len);
   }
-  check64<1>(0xFFFFFFF1u);
-  check64<1>(0xFFFFFFFFu);
+  check64<1, false>(0xFFFFFFF1u);
+  check64<1, false>(0xFFFFFFFFu);
   std::puts("ok");
 }
