@@ -28,7 +28,7 @@ HBM_PEAK_GBS = 8000.0
 #
 # HBM bytes per launch (fetched, written) of the tokenizer kernels on the full C2 workload: FETCH_SIZE / WRITE_SIZE
 # scaled by a copy kernel of known size.
-TRAFFIC_SOURCE = "profiles/hbm_traffic_pmc_all_workloads.md (library sources at commit 0ec04b2)"
+TRAFFIC_SOURCE = "profiles/hbm_traffic_pmc_all_workloads.md (library sources at commits 0ec04b2 and 7bda594)"
 MEASURED_TRAFFIC_C2 = {
     "range_first_row_kernel": (16690003, 4691648),
     "wordpiece_word_kernel": (1876864981, 1978118882),
@@ -46,7 +46,7 @@ MEASURED_TRAFFIC_C5_TOKENIZE = {
 MEASURED_TRAFFIC_C5_NORMALIZE = {
     "normalize_count_kernel": (4196028351, 15883232),
     "normalize_tile_rows_kernel": (73439045, 7941632),
-    "normalize_write_kernel": (4464463216, 4405365019),
+    "normalize_write_kernel": (4464519373, 4403901338),
 }
 # minhash: VALU wave-instructions executed per (window, parameter) of a wavefront (SQ_INSTS_VALU / (windows x P / 64)) and
 # the share of SIMD cycles that issued one (SQ_INSTS_VALU x 4 / (1024 SIMDs x kernel cycles), capped at 1: adds and
@@ -56,12 +56,12 @@ MEASURED_TRAFFIC_C5_NORMALIZE = {
 # of the time that takes.  Windows of a row repeat, and a window met before need not be folded again: the floor counts the
 # different windows of a row only (their share is found on the first rows of the workload), the measured figure is over
 # all of them.
-VALU_SOURCE = "profiles/valu_issue_pmc_all_workloads.md (library sources at commit 0ec04b2)"
+VALU_SOURCE = "profiles/valu_issue_pmc_all_workloads.md (library sources at commits 0ec04b2 and 7bda594)"
 PRODUCT_INST = {32: 1.5, 64: 1.25}
 MINHASH_VALU = {
     "C3": {"bits": 32, "measured": 1.47, "issue": 1.05},
-    "C4": {"bits": 64, "measured": 2.80, "issue": 1.00},
-    "C5": {"bits": 64, "measured": 6.04, "issue": 0.96},
+    "C4": {"bits": 64, "measured": 2.81, "issue": 1.01},
+    "C5": {"bits": 64, "measured": 6.06, "issue": 0.98},
 }
 
 
