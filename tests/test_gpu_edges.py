@@ -56,26 +56,27 @@ def jaccard_set(size):
 
 
 def jaccard_places(words, buckets, parts):
-    """Where windows of four bytes belong in a set, and in which part: the top of products of their hash (MurmurHash3_x86_32, seed
-    0, without the final mix)."""
+    """Where windows of four bytes belong in a set, which step they take from a bucket that is full to the next, and in which part
+    they are: by the top and the low bits of products of their hash (MurmurHash3_x86_32, seed 0, without the final mix)."""
     def top(v, n):
         return v.astype(np.uint64) * np.uint64(n) >> np.uint64(32)
     with np.errstate(over="ignore"):
         k = words * np.uint32(0xCC9E2D51)
         k = (k << np.uint32(15) | k >> np.uint32(17)) * np.uint32(0x1B873593)
         h = ((k << np.uint32(13) | k >> np.uint32(19)) * np.uint32(5) + np.uint32(0xE6546B64)) ^ np.uint32(4)
-        return top(h * np.uint32(0x9E3779B1), buckets), top((h ^ h >> np.uint32(15)) * np.uint32(0x85EBCA6B), parts)
+        p = h * np.uint32(0x9E3779B1)
+        return top(p, buckets), (p & np.uint32(15)) * 2 + 1, top((h ^ h >> np.uint32(15)) * np.uint32(0x85EBCA6B), parts)
 
 
 def furthest_from_home(text, buckets, parts):
-    """Buckets from the home of a window of four bytes to where it finds a place, the most of part 0."""
+    """Steps from the home of a window of four bytes to where it finds a place, the most of part 0."""
     windows = np.unique(text[:-3] | text[1:-2].astype(np.uint32) << 8 | text[2:-1].astype(np.uint32) << 16 | text[3:].astype(np.uint32) << 24)
-    home, part = jaccard_places(windows, buckets, parts)
+    home, step, part = jaccard_places(windows, buckets, parts)
     filled, furthest = [0] * buckets, 0
-    for b in home[part == 0].tolist():
+    for b, s in zip(home[part == 0].tolist(), step[part == 0].tolist()):
         far = 0
-        while filled[b] == 4:
-            b, far = (b + 1) % buckets, far + 1
+        while filled[b] == 4 and far < 500:
+            b, far = (b + s) % buckets, far + 1
         filled[b] += 1
         furthest = max(furthest, far)
     return furthest
@@ -83,15 +84,16 @@ def furthest_from_home(text, buckets, parts):
 
 @pytest.mark.parametrize("count, slots, parts", [(90, 1024, 1), (190, 1024, 1), (600, 4096, 1), (1000, 7008, 1), (2000, 15488, 1), (5000, 29440, 1), (7000, 29440, 2)])
 def test_jaccard_values_of_neighbouring_buckets(nv, orc, count, slots, parts):
-    """Words that belong in one bucket of their set, or in a few side by side: 90 that find a place within the 64 buckets that a
-    packed set looks at from there, and so many in sets of every size that some do not, so that the pair is done once more with
-    a plain set, or, where one of its parts has them all, with the one in global memory; among pairs that are not."""
+    """Words that belong in one bucket of their set, or in a few side by side, and take the same steps from there: 90 that find a
+    place within the 64 buckets that a packed set looks at, and so many in sets of every size that some do not, so that the pair
+    is done once more with a plain set, or, where one of its parts has them all, with the one in global memory; among pairs that
+    are not."""
     rng = np.random.default_rng(count)
     assert jaccard_set(4 * count) == (slots, parts)
-    letters = np.arange(97, 123, dtype=np.uint32)
+    letters = np.concatenate([np.arange(65, 91), np.arange(97, 123)]).astype(np.uint32)
     words = (letters[:, None, None, None] | letters[:, None, None] << 8 | letters[:, None] << 16 | letters << 24).astype(np.uint32).ravel()
-    home, part = jaccard_places(words, slots // 4, parts)
-    from_there = np.flatnonzero((part == 0) & (home >= 77))
+    home, step, part = jaccard_places(words, slots // 4, parts)
+    from_there = np.flatnonzero((part == 0) & (home >= 77) & (step == 1))
     near = from_there[np.argsort(home[from_there], kind="stable")][:count]
     text = rng.permutation(words[near]).view(np.uint8).reshape(-1, 4)
     assert (furthest_from_home(text.ravel(), slots // 4, parts) >= 64) == (count != 90)
