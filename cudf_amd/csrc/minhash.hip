@@ -891,6 +891,13 @@ __device__ __forceinline__ int64_t row_of(const uint32_t* __restrict__ prefix, i
   return r;
 }
 
+// The parts of a row of so many look at its slots before they ask for a minimum there: an address answers one request at a time,
+// which is what one long row took most of its time with, and of thousands of parts a dozen lower a slot.  (What is read may be
+// larger than what is there by then, never smaller.)  One row of 3 MB, 26 parameters of 32 bits 146 -> 51 us, 128 264 -> 107, of 64 bits
+// 171 -> 74; a list of 3 million elements, 64 parameters 452 -> 95.  In rows of fewer parts the read is waited for in vain: 40 rows of 300 KB
+// (600 parts), 128 parameters 88 -> 114, a row of 500 KB (1950) 53 either way, of 700 KB 71 -> 54.
+constexpr uint32_t kCrowd = 2048;
+
 // Part t is one of the row r with prefix[r] <= t < prefix[r + 1].  A row of one part is stored, the parts of the others
 // meet with an atomic minimum (their slots hold the largest value before).  A wavefront's first unit is its own number in
 // the grid, the following ones come from counters: an address answers about 150 M requests a second, which a column of
@@ -952,13 +959,19 @@ __global__ void __launch_bounds__(kThreads, (simd_waves<Source, Minima>())) minh
       if (begin < end) source.process(r, begin, end, minima, lds[wave], lane);
       minima.finish();
       T* const dst = out + static_cast<int64_t>(out_offsets[r]) + chunk_base;
-      minima.each([&](int32_t j, T v) {
-        if (j >= in_chunk) return;
-        if (k == 1)
-          dst[j] = n > 0 ? v : T{0};  // an empty row is zeros (minhash.cu:318)
-        else if (v != std::numeric_limits<T>::max())
-          atomicMin(&dst[j], v);
-      });
+      if (k < kCrowd) {
+        minima.each([&](int32_t j, T v) {
+          if (j >= in_chunk) return;
+          if (k == 1)
+            dst[j] = n > 0 ? v : T{0};  // an empty row is zeros (minhash.cu:318)
+          else if (v != std::numeric_limits<T>::max())
+            atomicMin(&dst[j], v);
+        });
+      } else {
+        minima.each([&](int32_t j, T v) {
+          if (j < in_chunk && v < __hip_atomic_load(&dst[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(&dst[j], v);
+        });
+      }
     }
     if (all <= static_cast<uint64_t>(parts.waves)) break;
     uint32_t const group    = one_counter ? kCounterGroups : me % kCounterGroups;

@@ -159,6 +159,24 @@ def test_minhash_parts_of_rows(nv, orc, bits, count):
         assert call(dev(nv, host), 5, a, b, 5).to_host().equals(ref(host, 5, a, b, 5, nthreads=8))
 
 
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("count", [1, 64, 130, 260])
+def test_minhash_rows_of_thousands_of_parts(nv, orc, bits, count):
+    """Rows and lists that are cut into as many parts as look at a slot before they lower it (2048), a few less and twice as many,
+    beside short ones."""
+    rng = np.random.default_rng(count)
+    a, b = params(rng, count, bits)
+    call, ref = (nv.minhash, orc.minhash) if bits == 32 else (nv.minhash64, orc.minhash64)
+    for lens in ([2048 * 256 - 300, 5], [2048 * 256 + 300], [0, 1_100_000, 40]):
+        host = mixed_rows(rng, lens)
+        assert call(dev(nv, host), 5, a, b, 5).to_host().equals(ref(host, 5, a, b, 5, nthreads=8))
+    call, ref = (nv.minhash_ngrams, orc.minhash_ngrams) if bits == 32 else (nv.minhash64_ngrams, orc.minhash64_ngrams)
+    for lens in ([2048 * 64 - 100, 3], [0, 2048 * 128 + 500, 7]):
+        offsets = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+        lists = HostListStringsColumn(offsets, mixed_rows(rng, rng.integers(0, 9, int(offsets[-1]))), None, len(lens), 0, 0)
+        assert call(nv.DeviceListStringsColumn.from_host(lists), 2, 5, a, b).to_host().equals(ref(lists, 2, 5, a, b, nthreads=8))
+
+
 @pytest.mark.parametrize("rows", [1023, 1024, 1025, 8191, 8192, 8193, 131_071, 131_072, 262_144, 262_145])
 @pytest.mark.parametrize("nulls", [False, True])
 def test_minhash_row_counts(nv, orc, rows, nulls):
