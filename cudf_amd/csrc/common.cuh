@@ -529,6 +529,20 @@ HostPost new_post();  // (only where host_scalars() gives memory)
 // Returns when it has been sent, or with the error that keeps it from being sent.
 hipError_t wait_for_post(HostPost const& post, hipStream_t stream);
 
+// What the workgroups of one launch add up between them, so that the last to arrive knows the sum and need not be another
+// kernel: `sum` counts them in its upper bits.  Zeros between launches, which the last workgroup sees to.  Every host thread has
+// one of its own on every device (device memory of the library, no allocation; nullptr for more than kMostArrivals threads at a
+// time), given back when the thread ends.  For entry points that wait until the last workgroup has spoken: the thread's next call,
+// on whatever stream, then finds zeros.
+struct alignas(128) Arrivals {
+  unsigned long long sum;
+  uint32_t notes;
+};
+constexpr int kMostArrivals = 1024;
+Arrivals* thread_arrivals();
+// After a failure it may hold anything: no thread gets it any more.
+void forsake_thread_arrivals();
+
 // *dst = *src
 void launch_publish(const uint64_t* src, uint64_t* dst, HostPost post, hipStream_t stream);
 // dst[0] = offsets[first_index], dst[1] = offsets[last_index] (offsets of 32 or 64 bits)

@@ -196,6 +196,70 @@ uint64_t* host_scalars()
   return slot.p;
 }
 
+namespace {
+__device__ Arrivals g_arrivals[kMostArrivals];  // zeros when the library is loaded
+
+// The numbers that no thread has.  (Never destroyed: threads end after the objects of the library do.)
+struct FreeArrivals {
+  std::mutex lock;
+  std::vector<int> numbers;
+  FreeArrivals()
+  {
+    for (int i = kMostArrivals; i-- > 0;) numbers.push_back(i);
+  }
+};
+FreeArrivals& free_arrivals()
+{
+  static FreeArrivals* const all = new FreeArrivals;
+  return *all;
+}
+struct ThreadArrivals {
+  static constexpr int kDevices = 64;
+  int number                    = -1;
+  bool forsaken                 = false;
+  Arrivals* first[kDevices]     = {};  // of the device's array
+  ThreadArrivals()
+  {
+    FreeArrivals& all = free_arrivals();
+    std::lock_guard<std::mutex> const guard(all.lock);
+    if (!all.numbers.empty()) {
+      number = all.numbers.back();
+      all.numbers.pop_back();
+    }
+  }
+  ~ThreadArrivals()
+  {
+    if (number < 0 || forsaken) return;
+    FreeArrivals& all = free_arrivals();
+    std::lock_guard<std::mutex> const guard(all.lock);
+    all.numbers.push_back(number);
+  }
+};
+ThreadArrivals& of_this_thread()
+{
+  thread_local ThreadArrivals mine;
+  return mine;
+}
+}  // namespace
+
+Arrivals* thread_arrivals()
+{
+  ThreadArrivals& mine = of_this_thread();
+  int device           = 0;
+  if (mine.number < 0 || mine.forsaken || hipGetDevice(&device) != hipSuccess || device < 0 || device >= ThreadArrivals::kDevices) return nullptr;
+  if (!mine.first[device]) {
+    void* p = nullptr;
+    if (hipGetSymbolAddress(&p, HIP_SYMBOL(g_arrivals)) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    mine.first[device] = static_cast<Arrivals*>(p);
+  }
+  return mine.first[device] + mine.number;
+}
+
+void forsake_thread_arrivals() { of_this_thread().forsaken = true; }
+
 HostPost new_post()
 {
   thread_local uint64_t tickets = 0;

@@ -171,8 +171,9 @@ namespace {
 
 constexpr int kTokWaves     = 4;
 constexpr int kTokThreads   = kTokWaves * kWave;
-// (word pass: two workgroups to a CU, six wavefronts per SIMD, that share the words in LDS; the launch for a small column is too short for those)
-constexpr int word_waves(bool small) { return small ? kTokWaves : 12; }
+// (word pass: two workgroups to a CU, six wavefronts per SIMD, that share the words in LDS; the launch for a small column, too
+// short for those, has two workgroups to a CU as well, of four wavefronts per SIMD)
+constexpr int word_waves(bool small) { return small ? 8 : 12; }
 constexpr int32_t kNone     = std::numeric_limits<int32_t>::min();
 constexpr int kOovKeep      = 7;     // tokens of an out-of-vocabulary word that are kept while it is tokenized
 // ------------------------------------------------------------------ where candidate keys live
@@ -868,7 +869,11 @@ struct TileArgs {
   const uint32_t* hot;     // slots of words that the sample found, kHotWords of them (nullptr: none)
   int64_t most_bytes;
   uint32_t* first_row_out; // as range_first_row
-  uint32_t* range_notes;   // per range: kNoteSpill, kNoteAgain
+  uint64_t* block_tokens;  // tokens of each workgroup's ranges
+  uint32_t* again_count;   // words of more tokens than a queue record keeps (the emit pass counts them)
+  Arrivals* arrivals;      // what the workgroups have added up between them, and where the last of them leaves it for the host
+  uint64_t* host;
+  HostPost post;
 };
 // Words that the sample of the column met and found in the vocabulary, a wavefront's neighbours' and its own: text repeats
 // its frequent words, the first-level cache keeps the lines of few of them (a line of the table has four buckets, most of
@@ -1012,7 +1017,7 @@ constexpr uint32_t kSmallSlots      = kSmallTile / 2 + 8;  // words of a tile: o
 constexpr uint32_t kSmallLeastSlots = kSmallTile / 4 + 8;  // (six bytes to a word and its space are ordinary)
 constexpr uint32_t kSmallQueue      = kSmallTile / 8;      // words of a tile that are not in the vocabulary (one in 37 bytes on the benchmark's rows)
 constexpr uint32_t kSmallLeastQueue = kSmallTile / 16;
-constexpr unsigned kSmallGrid       = 2048;                // workgroups at most: a wavefront then takes several tiles
+constexpr unsigned kSmallGrid       = 512;                 // workgroups at most (two to a CU): a wavefront then takes several tiles
 // What every one of `tiles` tiles gets of the slots and of the queue's records (an even number of slots).
 __host__ __device__ inline uint32_t small_slots(uint32_t slots, uint32_t tiles)
 {
@@ -1025,6 +1030,26 @@ __host__ __device__ inline uint32_t small_queue(uint32_t records, uint32_t tiles
   return each < kSmallQueue ? each : kSmallQueue;
 }
 
+// By one thread of the launch for a small column: the view's first and last offset, the number of tokens, the tiles' notes
+// together (the last two mean nothing where the column is not small).
+__device__ __forceinline__ void tell_host(TileArgs const& a, int64_t first_offset, int64_t bytes, uint64_t tokens, uint32_t notes)
+{
+  *a.again_count = 0;
+  a.host[0]      = static_cast<uint64_t>(first_offset);
+  a.host[1]      = static_cast<uint64_t>(first_offset + bytes);
+  a.host[2]      = tokens;
+  a.host[3]      = notes;
+  a.post.send();
+}
+
+// The tiles are shared out in blocks of neighbours, a workgroup's wavefronts taking theirs one after the other: how many
+// tiles a block has where `grid` workgroups were launched.
+__host__ __device__ inline uint32_t small_block(uint32_t tiles, uint32_t grid)
+{
+  uint32_t const each = (tiles + grid - 1) / grid;
+  return each > static_cast<uint32_t>(word_waves(true)) ? each : static_cast<uint32_t>(word_waves(true));
+}
+
 // One tile at a time per wavefront: stage its bytes (and the 256 after it) in LDS; mark the row starts in it; find
 // word starts and ends (lanes <-> 16-byte blocks: spaces by SWAR, row starts as extra separators); with a word limit,
 // drop the words past each row's limit; list the words (word k pairs start k with end k); look all of them up (lanes
@@ -1033,14 +1058,19 @@ __host__ __device__ inline uint32_t small_queue(uint32_t records, uint32_t tiles
 // INLINE (a small column, where the launches and the waits for one another would be most of the call): a range is one
 // tile; where the bytes lie and which rows the range has the wavefront finds out itself, from the offsets; and it
 // tokenizes the words that are not in the vocabulary itself, lanes <-> words, into the range's own part of the queue
-// (queue_cap records), where the other way leaves the out-of-vocabulary pass to put its results.
+// (queue_cap records), where the other way leaves the out-of-vocabulary pass to put its results.  The number of tokens is
+// added up on the way, one atomic a workgroup, whose answer tells the last workgroup the total: it tells the host, which
+// then needs no further kernel to wait for (one that added up the tiles and told the host took 4 to 11 us and a launch).
 template <int TILE, bool IS64, bool LIMIT, bool INLINE>
 __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wordpiece_word_kernel(TileArgs a)
 {
   constexpr int kWaves = word_waves(INLINE);
   if constexpr (INLINE) {
     int64_t const first_offset = a.col.off(0), bytes = a.col.off(a.col.size) - first_offset;
-    if (bytes <= 0 || bytes > a.most_bytes) return;
+    if (bytes <= 0 || bytes > a.most_bytes) {
+      if (blockIdx.x == 0 && threadIdx.x == 0) tell_host(a, first_offset, bytes, 0, 0);
+      return;
+    }
     const uint8_t* const first_byte = a.col.chars + first_offset;
     a.first_offset = first_offset;
     a.cbeg         = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(first_byte) & 15u);
@@ -1049,8 +1079,10 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
     a.ntiles       = (a.cend + TILE - 1) / TILE;
     a.nranges      = static_cast<uint32_t>(a.ntiles);
     a.range_tiles  = 1;
-    a.unit_begin   = 0;
-    a.unit_end     = a.nranges;
+    uint32_t const block = small_block(a.nranges, gridDim.x);
+    if (blockIdx.x * block >= a.nranges) return;
+    a.unit_begin   = blockIdx.x * block;
+    a.unit_end     = min(a.nranges, a.unit_begin + block);
     a.range_cap    = small_slots(a.range_cap, a.nranges);  // (of all: shared out)
     a.queue_cap    = small_queue(a.queue_cap, a.nranges);
   }
@@ -1061,7 +1093,14 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
   __shared__ TileLds<TILE> lds_all[kWaves];
   __shared__ uint4 trim[17];
   __shared__ uint4 hot[INLINE ? 1 : kHotWords];  // the key (at most 8 bytes), its id, its length
+  __shared__ uint32_t small_next, small_tokens, small_notes;  // INLINE: the next tile of the block; what its tiles have
   fill_trim_table(trim);
+  if constexpr (INLINE) {
+    if (threadIdx.x == 0) {
+      small_next   = a.unit_begin + kWaves;
+      small_tokens = small_notes = 0;
+    }
+  }
   if constexpr (!INLINE) {
     for (uint32_t i = threadIdx.x; i < kHotWords; i += kWaves * kWave) {
       uint4 v = make_uint4(0u, 0u, 0u, 0u);
@@ -1093,15 +1132,20 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
   const uint8_t* const lds_byte = reinterpret_cast<const uint8_t*>(lds.bytes);
   uint16_t* const word16        = reinterpret_cast<uint16_t*>(lds.word);
   uint32_t q_pos = 0, q_lim = 0;  // this wavefront's reserved queue entries [q_pos, q_lim)
-  uint32_t inline_range = 0;
+  uint32_t block_known = 0, block_notes = 0;  // INLINE: of the tiles of this wavefront
   bool const use_memo   = !INLINE && a.memo && memo_pays(a.memo_count[0], a.memo_count[1]);
 
   uint32_t const my_number = blockIdx.x * kWaves + threadIdx.x / kWave;
   for (bool first = true;; first = false) {
     uint32_t range;
     if constexpr (INLINE) {
-      range = first ? static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(my_number))) : inline_range + gridDim.x * kWaves;
-      inline_range = range;
+      if (first) {
+        range = a.unit_begin + static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave)));
+      } else {
+        uint32_t n = 0;
+        if (lane == 0) n = atomicAdd(&small_next, 1u);
+        range = wave_bcast(n, 0);
+      }
     } else {
       range = a.unit_begin + next_unit(a.counter, first, my_number, lane);
     }
@@ -1550,13 +1594,39 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
     if (lane == 0) {
       a.range_words[range]  = cursor;
       a.range_tokens[range] = known;
-      if (INLINE)
-        a.range_notes[range] = (spill ? kNoteSpill : 0u) | (again ? kNoteAgain : 0u);
-      else if (spill)
-        *a.overflow = 1u;
+      if (!INLINE && spill) *a.overflow = 1u;
+    }
+    if (INLINE) {
+      block_known += known;
+      block_notes |= (spill ? kNoteSpill : 0u) | (again ? kNoteAgain : 0u);
     }
   }
-  if (INLINE) return;
+  if constexpr (INLINE) {
+    if (lane == 0) {
+      atomicAdd(&small_tokens, block_known);
+      if (block_notes != 0) atomicOr(&small_notes, block_notes);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      uint32_t const blocks     = (a.nranges + small_block(a.nranges, gridDim.x) - 1) / small_block(a.nranges, gridDim.x);
+      a.block_tokens[blockIdx.x] = small_tokens;
+      if (small_notes != 0) {  // (seldom; it has to be there when the last workgroup arrives)
+        atomicOr(&a.arrivals->notes, small_notes);
+        __threadfence();
+      }
+      // how many have arrived, and above 40 bits of their tokens: no other memory has to be seen for the total
+      unsigned long long const mine = (1ull << 40) | small_tokens;
+      unsigned long long const all  = atomicAdd(&a.arrivals->sum, mine) + mine;
+      if ((all >> 40) == blocks) {
+        uint32_t notes = 0;
+        // (left as it was found: zeros for the next call)
+        atomicExch(&a.arrivals->sum, 0ull);
+        notes = atomicExch(&a.arrivals->notes, 0u);
+        tell_host(a, a.first_offset, a.cend - a.cbeg, all & ((1ull << 40) - 1ull), notes);
+      }
+    }
+    return;
+  }
   // the reserved entries that no word took
   for (uint32_t q = q_pos + lane; q < q_lim; q += kWave)
     if (q < a.queue_cap) a.queue[q].len_flags = 0;
@@ -1890,8 +1960,13 @@ __global__ void __launch_bounds__(kMemoThreads) wordpiece_memo_fill_kernel(const
 // side in LDS first and written 64 at a time, the same tokens take a third of the instructions (0.69 -> 0.55 ms on
 // 3.2 GB of text with one word in seven from the queue).
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+// SMALL (after the launch for a small column): where a range's tokens go is added up here, by its wavefront, from the
+// tokens of the blocks of `block` ranges before its own and of the ranges before it in that.
+template <bool SMALL>
 __global__ void __launch_bounds__(kTokThreads, 8) wordpiece_emit_kernel(uint32_t nranges, const uint32_t* __restrict__ arena, uint32_t range_cap,
                                                                      const uint32_t* __restrict__ range_words, const int64_t* __restrict__ range_base,
+                                                                     const uint64_t* __restrict__ block_tokens,
+                                                                     const uint32_t* __restrict__ range_tokens, uint32_t block,
                                                                      const uint32_t* __restrict__ range_first_row, OovEntry* __restrict__ queue,
                                                                      int32_t* __restrict__ offsets, int32_t* __restrict__ child,
                                                                      uint32_t* __restrict__ again, uint32_t* __restrict__ again_count)
@@ -1911,7 +1986,16 @@ __global__ void __launch_bounds__(kTokThreads, 8) wordpiece_emit_kernel(uint32_t
     // (a range's slots begin at an even index, and so does a lane's pair)
     const uint32_t* const slots = arena + static_cast<int64_t>(range) * range_cap;
     uint32_t const nwords       = range_words[range];
-    int64_t const base          = range_base[range];
+    int64_t base;
+    if constexpr (SMALL) {
+      uint32_t const mine = range / block;
+      uint64_t before     = 0;
+      for (uint32_t i = lane; i < mine; i += kWave) before += block_tokens[i];
+      for (uint32_t i = mine * block + lane; i < range; i += kWave) before += range_tokens[i];
+      base = static_cast<int64_t>(wave_bcast64(wave_inclusive_scan64(before), kWave - 1));
+    } else {
+      base = range_base[range];
+    }
     int32_t* const dst0         = child + base;
     uint32_t r_win              = range_first_row[range];  // the 64 rows being placed: r_win + lane, the first row_used of them done
     uint32_t const r_end        = range_first_row[range + 1];
@@ -2141,54 +2225,6 @@ __global__ void publish_state_kernel(const uint64_t* __restrict__ total, const u
   dst[1] = flags[kFlagOverflow];
   dst[2] = flags[kFlagQueueSize];
   post.send();
-}
-
-// The same, and the places of the ranges' tokens, after the one launch for a small column: one workgroup.  dst = the view's
-// first and last offset, the number of tokens, the ranges' notes together (the last two mean nothing where the column is
-// not small).
-constexpr int kFinishThreads = 1024;
-__global__ void __launch_bounds__(kFinishThreads) wordpiece_finish_kernel(TileArgs a, int tile, int64_t* __restrict__ bases, uint32_t* __restrict__ again_count,
-                                                                          uint64_t* __restrict__ dst, HostPost post)
-{
-  __shared__ uint64_t lds[kFinishThreads / kWave + 1];
-  __shared__ uint32_t all_notes;
-  int64_t const first_offset = a.col.off(0), bytes = a.col.off(a.col.size) - first_offset;
-  bool const small     = bytes > 0 && bytes <= a.most_bytes;
-  int64_t const cbeg   = static_cast<int64_t>(reinterpret_cast<uintptr_t>(a.col.chars + first_offset) & 15u);
-  uint32_t const n     = small ? static_cast<uint32_t>((cbeg + bytes + tile - 1) / tile) : 0u;
-  uint32_t notes = 0;
-  uint64_t carry = 0;
-  if (threadIdx.x == 0) all_notes = 0;
-  constexpr uint32_t kEach = 4;
-  for (uint32_t base = 0; base < n; base += kEach * kFinishThreads) {
-    uint32_t const i = base + kEach * threadIdx.x;
-    uint64_t v[kEach], sum = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < kEach; ++k) {
-      v[k] = i + k < n ? a.range_tokens[i + k] : 0;
-      if (i + k < n) notes |= a.range_notes[i + k];
-      sum += v[k];
-    }
-    uint64_t total;
-    uint64_t run = carry + block_exclusive_scan64<kFinishThreads>(sum, lds, &total);
-#pragma unroll
-    for (uint32_t k = 0; k < kEach; ++k) {
-      if (i + k < n) bases[i + k] = static_cast<int64_t>(run);
-      run += v[k];
-    }
-    carry += total;
-  }
-  __syncthreads();
-  if (notes) atomicOr(&all_notes, notes);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    *again_count = 0;
-    dst[0]       = static_cast<uint64_t>(first_offset);
-    dst[1]       = static_cast<uint64_t>(first_offset + bytes);
-    dst[2]       = carry;
-    dst[3]       = all_notes;
-    post.send();
-  }
 }
 
 struct RangeTokensOf {
@@ -2632,24 +2668,24 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   // number of tokens is put on the stream at once, before the host knows how many bytes there are.  Where there are more
   // than were guessed, these kernels leave at once; up to small_most the same follows with the temporaries that the bytes
   // take (which is also done where a tile had not enough of them), beyond the call goes on as for a large column.
-  // (29 rows of 180 bytes: 87 us in eleven launches with two waits, 43 us in four with one; 32,768 rows of 120 bytes
-  // 145 -> 60 us)
-  bool const small    = scalars && sampling && rows <= kSmallRows && g_forced_range_tiles.load(std::memory_order_relaxed) == 0;
+  // (29 rows of 180 bytes: 87 us in eleven launches with two waits, 34 in four with one, 32 in two; 32,768 rows of 120 bytes
+  // 145, 50 and 47 us, 10 MB of those 84 and 77 with the last two)
+  Arrivals* const arrivals = scalars && sampling && rows <= kSmallRows && g_forced_range_tiles.load(std::memory_order_relaxed) == 0 ? thread_arrivals() : nullptr;
+  bool const small         = arrivals != nullptr;
   int64_t const small_most = std::min(std::max(rows * kSmallRowBytes, kSmallLeast), kSmallBytes);
   int64_t small_bytes      = small ? std::min(std::max(rows * kSmallGuess, kSmallSure), small_most) : 0;
   for (int attempt = 0; attempt < 2 && small_bytes > 0; ++attempt) {
     uint32_t const most_ranges  = static_cast<uint32_t>(small_bytes / kSmallTile + 2);
     uint32_t const slots        = most_ranges * (attempt == 0 ? kSmallLeastSlots : kSmallSlots);
     uint32_t const records      = most_ranges * (attempt == 0 ? kSmallLeastQueue : kSmallQueue);
-    size_t const temp_bytes[8]  = {static_cast<size_t>(slots) * sizeof(uint32_t),
+    size_t const temp_bytes[7]  = {static_cast<size_t>(slots) * sizeof(uint32_t),
                                    (static_cast<size_t>(most_ranges) + 1) * sizeof(uint32_t),
                                    static_cast<size_t>(most_ranges) * sizeof(uint32_t),
                                    static_cast<size_t>(most_ranges) * sizeof(uint32_t),
-                                   static_cast<size_t>(most_ranges) * sizeof(uint32_t),
-                                   (static_cast<size_t>(most_ranges) + 1) * sizeof(int64_t),
+                                   kSmallGrid * sizeof(uint64_t),
                                    (static_cast<size_t>(records) + 1) * sizeof(uint32_t),
                                    static_cast<size_t>(records) * sizeof(OovEntry)};
-    TempParts<8> const temps(mr, temp_bytes);
+    TempParts<7> const temps(mr, temp_bytes);
     if (!temps.ok()) break;  // (no room: as for a large column)
     TileArgs args{};
     args.col           = v;
@@ -2660,24 +2696,30 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     args.first_row_out = temps.part<uint32_t>(1);
     args.range_words   = temps.part<uint32_t>(2);
     args.range_tokens  = temps.part<uint32_t>(3);
-    args.range_notes   = temps.part<uint32_t>(4);
+    args.block_tokens  = temps.part<uint64_t>(4);
+    args.again_count   = temps.part<uint32_t>(5);
     args.offsets_out   = out->offsets;
-    args.queue         = temps.part<OovEntry>(7);
+    args.queue         = temps.part<OovEntry>(6);
     args.queue_cap     = records;
     args.most_bytes    = small_bytes;
-    int64_t* const bases        = temps.part<int64_t>(5);
-    uint32_t* const again_count = temps.part<uint32_t>(6);
+    args.arrivals      = arrivals;
+    args.host          = scalars;
+    args.post          = new_post();
+    uint32_t* const again_count = args.again_count;
+    unsigned const grid         = std::min((most_ranges + word_waves(true) - 1) / word_waves(true), kSmallGrid);
     void (*const kernel)(TileArgs) = is64 ? (limit ? wordpiece_word_kernel<kSmallTile, true, true, true> : wordpiece_word_kernel<kSmallTile, true, false, true>)
                                           : (limit ? wordpiece_word_kernel<kSmallTile, false, true, true> : wordpiece_word_kernel<kSmallTile, false, false, true>);
     {
       ProfileScope ps("wordpiece_word_kernel (small column)", stream);
-      hipLaunchKernelGGL(kernel, dim3(std::min((most_ranges + kTokWaves - 1) / kTokWaves, kSmallGrid)), dim3(kTokThreads), 0, stream, args);
+      hipLaunchKernelGGL(kernel, dim3(grid), dim3(word_waves(true) * kWave), 0, stream, args);
     }
-    HostPost const post = new_post();
-    hipLaunchKernelGGL(wordpiece_finish_kernel, dim3(1), dim3(kFinishThreads), 0, stream, args, kSmallTile, bases, again_count, scalars, post);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = wait_for_post(post, stream);
-    if (e != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
+    bool const launched = e == hipSuccess;
+    if (launched) e = wait_for_post(args.post, stream);
+    if (e != hipSuccess) {
+      if (launched) forsake_thread_arrivals();  // (nobody knows what it holds)
+      return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
+    }
     first_offset = static_cast<int64_t>(scalars[0]);
     last_offset  = static_cast<int64_t>(scalars[1]);
     int64_t const bytes = last_offset - first_offset;
@@ -2694,8 +2736,9 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
         if (!out->child) return give_up(NVTEXT_AMD_ALLOC_FAILED, "child allocation failed");
       }
       ProfileScope ps("wordpiece_emit_kernel", stream);
-      hipLaunchKernelGGL(wordpiece_emit_kernel, dim3((nranges + kTokWaves - 1) / kTokWaves), dim3(kTokThreads), 0, stream, nranges, args.arena,
-                         small_slots(slots, nranges), args.range_words, bases, args.first_row_out, args.queue, out->offsets,
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(wordpiece_emit_kernel<true>), dim3((nranges + kTokWaves - 1) / kTokWaves), dim3(kTokThreads), 0, stream, nranges,
+                         args.arena, small_slots(slots, nranges), args.range_words, static_cast<const int64_t*>(nullptr), args.block_tokens,
+                         args.range_tokens, small_block(nranges, grid), args.first_row_out, args.queue, out->offsets,
                          static_cast<int32_t*>(out->child), again_count + 1, again_count);
       if (scalars[3] & kNoteAgain)
         hipLaunchKernelGGL(wordpiece_retokenize_kernel, dim3(64), dim3(kRareThreads), 0, stream, vocabulary->table,
@@ -2798,7 +2841,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   unsigned const word_grid2 = grid_for(nranges - first_part);  // (0: the column is done in one part)
   unsigned const oov_grid  = static_cast<unsigned>(resident(reinterpret_cast<const void*>(wordpiece_oov_kernel), kOovThreads, 4));
   unsigned const emit_grid = static_cast<unsigned>(
-    std::min<int64_t>((static_cast<int64_t>(nranges) + kTokWaves - 1) / kTokWaves, resident(reinterpret_cast<const void*>(wordpiece_emit_kernel), kTokThreads, 5)));
+    std::min<int64_t>((static_cast<int64_t>(nranges) + kTokWaves - 1) / kTokWaves, resident(reinterpret_cast<const void*>(wordpiece_emit_kernel<false>), kTokThreads, 5)));
 
   TileArgs args{};
   args.col          = v;
@@ -2944,7 +2987,8 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     }
     {
       ProfileScope ps("wordpiece_emit_kernel", stream);
-      hipLaunchKernelGGL(wordpiece_emit_kernel, dim3(emit_grid), dim3(kTokThreads), 0, stream, nranges, arena, range_cap, words, bases, first_row, queue,
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(wordpiece_emit_kernel<false>), dim3(emit_grid), dim3(kTokThreads), 0, stream, nranges, arena, range_cap, words, bases,
+                         static_cast<const uint64_t*>(nullptr), static_cast<const uint32_t*>(nullptr), 1u, first_row, queue,
                          out->offsets, static_cast<int32_t*>(out->child), longer, flags + kFlagAgain);
       // (the list of longer words has served its purpose by now: its memory takes the list of words to do again, at most
       // one entry per queued word)

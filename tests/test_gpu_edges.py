@@ -396,6 +396,50 @@ def test_tokenize_small_columns_again(nv, orc, megabytes, dense, limit):
     assert nv.wordpiece_tokenize(dev(nv, host), vocabulary, limit).to_host().equals(orc.wordpiece_tokenize(host, reference, limit, nthreads=8))
 
 
+@pytest.mark.parametrize("tiles", [1, 7, 8, 9, 511, 4095, 4096, 4097, 4105, 8200])
+def test_tokenize_blocks_of_tiles(nv, orc, tiles):
+    """Columns of so many tiles of 1024 bytes: a block is eight of them, and more where 512 workgroups have more to do; the
+    last block is full, has one tile, or all but one.  A second call finds what the first left for it."""
+    rng = np.random.default_rng(tiles)
+    hv = HostStringsColumn.from_pylist(VOCABULARY)
+    vocabulary, reference = nv.WordPieceVocabulary(dev(nv, hv)), orc.Vocabulary(hv)
+    text = words_column(rng, [100_000], VOCABULARY, 0.1).chars
+    total = 1024 * tiles - 16  # (the first byte may lie up to 15 bytes into a tile)
+    chars = np.tile(text, total // text.size + 1)[:total].copy()
+    rows = max(total // 400, 1)
+    host = HostStringsColumn(chars, np.linspace(0, total, rows + 1).astype(np.int32), None, rows, 0, 0)
+    column, expected = dev(nv, host), orc.wordpiece_tokenize(host, reference, 60, nthreads=8)
+    for _ in range(2):
+        assert nv.wordpiece_tokenize(column, vocabulary, 60).to_host().equals(expected)
+
+
+def test_tokenize_from_threads_that_come_and_go(nv, orc):
+    """Forty host threads, eight at a time, tokenize small columns of different sizes: what a call adds up on the device is its thread's own,
+    and is there again for the threads that follow."""
+    import threading
+    import torch
+    rng = np.random.default_rng(3)
+    hv = HostStringsColumn.from_pylist(VOCABULARY)
+    vocabulary, reference = nv.WordPieceVocabulary(dev(nv, hv)), orc.Vocabulary(hv)
+    hosts = [words_column(rng, list(rng.integers(0, 300, 40 * 2 ** k)), VOCABULARY, 0.2) for k in range(8)]
+    columns, expected, wrong = [dev(nv, h) for h in hosts], [orc.wordpiece_tokenize(h, reference, 0) for h in hosts], []
+    torch.cuda.synchronize()
+
+    def work(k):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(3):
+                if not nv.wordpiece_tokenize(columns[k], vocabulary, 0).to_host().equals(expected[k]):
+                    wrong.append(k)
+
+    for _ in range(5):
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(8)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    assert not wrong
+
+
 @pytest.mark.parametrize("rows, each", [(4, 65_537), (4, 65_535), (131_072, 10), (131_073, 10), (9000, 3800)])
 def test_tokenize_where_small_columns_end(nv, orc, rows, each):
     """Around the bytes (256 KiB; 32 MiB) and the rows up to which a column is put on the stream before its size is known."""
