@@ -776,7 +776,12 @@ std::atomic<int> g_forced_range_tiles{0};
 std::atomic<int> g_sizing_sample{1};
 constexpr int kRangeTiles    = 8;     // tiles per range at most (a large column); a small column has fewer, so that every wavefront gets several ranges
 constexpr int kOverBlocks    = 16;   // 16-byte blocks staged past the tile: a word that starts in the tile ends in them, or is kMaxWord bytes or more
-constexpr uint32_t kQueueChunk = 512;  // queue entries a wavefront of the word pass reserves at a time
+// Queue entries that a wavefront of the word pass reserves at a time, in a large column and at least.  What a wavefront has
+// left in the end are records that the out-of-vocabulary pass reads to find nothing in them: where six thousand wavefronts
+// meet a few hundred unknown words each, chunks of 512 were mostly such (with the counters of QueueChunks, 128,000 rows of 500 bytes
+// 380 -> 303 us, 780,000 of 256 bytes 713 -> 570).
+constexpr uint32_t kQueueChunk      = 512;
+constexpr uint32_t kQueueLeastChunk = 64;
 // A word slot: the token id (0 .. 2^31-1, or -1 for an absent [UNK]), or kOovMark | index of the word's queue entry
 // (never 0xFFFFFFFF: the queue has fewer than 2^31 - 1 entries).
 constexpr uint32_t kOovMark = 0x80000000u;
@@ -858,7 +863,8 @@ struct TileArgs {
   int32_t* offsets_out;    // per row: words of its range before the row
   OovEntry* queue;
   uint32_t queue_cap;
-  uint32_t* queue_size;    // entries reserved so far
+  uint32_t queue_shift;    // a chunk of the queue is so many entries (a power of two)
+  uint32_t* queue_chunks;  // kCounterGroups counters of the chunks handed out (see QueueChunks)
   uint32_t* counter;       // next range to hand out
   uint32_t* overflow;      // set when a range has more words than range_cap
   // one launch for all (INLINE): the most bytes it is for, and what it leaves in place of the counters and flags
@@ -888,15 +894,17 @@ constexpr uint32_t kNoteAgain = 2u;  // a word of more tokens than a queue recor
 constexpr uint32_t kCounterGroups = 8;
 constexpr uint32_t kFlagLine      = 32;
 constexpr uint32_t kFlagOverflow  = 1;                                          // a range had more words than slots
-constexpr uint32_t kFlagQueueSize = 2;                                          // queue entries reserved
+constexpr uint32_t kFlagExtent    = 2;                                          // QueueChunks::extent(), where the host copies it
 constexpr uint32_t kFlagLonger    = 1 * kFlagLine;                              // words of more than 16 bytes
 constexpr uint32_t kFlagAgain     = 2 * kFlagLine;                              // words of more tokens than a queue record keeps
 constexpr uint32_t kFlagWordUnits = 3 * kFlagLine;                              // kCounterGroups work counters of the word pass, a line each
 constexpr uint32_t kFlagOovUnits  = kFlagWordUnits + kCounterGroups * kFlagLine;  // and of the out-of-vocabulary pass
 constexpr uint32_t kFlagWordUnits2 = kFlagOovUnits + kCounterGroups * kFlagLine;  // the same of the second launches, of a column that is done in two
 constexpr uint32_t kFlagOovUnits2  = kFlagWordUnits2 + kCounterGroups * kFlagLine;
-constexpr uint32_t kFlagMemo       = kFlagOovUnits2 + kCounterGroups * kFlagLine;  // words of the first ranges that the memo could take; keys that it took; queue entries of those ranges
-constexpr uint32_t kFlagWords      = kFlagMemo + kFlagLine;
+constexpr uint32_t kFlagMemo       = kFlagOovUnits2 + kCounterGroups * kFlagLine;  // words of the first ranges that the memo could take; keys that it took; from kMemoChunks on, the queue's chunks of those ranges
+constexpr uint32_t kMemoChunks     = 2;
+constexpr uint32_t kFlagQueue      = kFlagMemo + kFlagLine;                        // kCounterGroups counters of the queue's chunks, a line each
+constexpr uint32_t kFlagWords      = kFlagQueue + kCounterGroups * kFlagLine;
 
 // The next unit of work for a wavefront of a persistent kernel: its first one is its own number in the grid, the
 // following ones come from a counter.  Atomics on one address run at about 150 M/s: eight thousand wavefronts that all
@@ -917,6 +925,33 @@ __device__ __forceinline__ uint32_t next_unit(uint32_t* counters, bool first, ui
   if (lane == 0) n = atomicAdd(counters + g * kFlagLine, 1u);
   return wave_bcast(n, 0) * kCounterGroups + g;
 }
+
+// The queue is handed out in chunks of 2^shift entries by kCounterGroups counters, each in a line of its own: chunk n of group
+// g is the queue's chunk n * kCounterGroups + g.  A wavefront's group is that of the ranges it does, so that how many chunks
+// a group takes depends on the text, but for the last chunk of each wavefront.  (One counter, one atomic after the other at
+// 150 M/s, was a third of the word pass of 16 MB of text in chunks of 512, and most of it in chunks of 64.)
+struct QueueChunks {
+  const uint32_t* counts;
+  uint32_t shift;
+  __device__ __forceinline__ uint32_t of_group(uint32_t g) const { return counts[g * kFlagLine]; }
+  // Entries up to the end of the last chunk that has been handed out.
+  __device__ __forceinline__ uint64_t extent() const
+  {
+    uint32_t chunks = 0;
+#pragma unroll
+    for (uint32_t g = 0; g < kCounterGroups; ++g) {
+      uint32_t const n = of_group(g);
+      chunks           = max(chunks, n != 0 ? (n - 1u) * kCounterGroups + g + 1u : 0u);
+    }
+    return static_cast<uint64_t>(chunks) << shift;
+  }
+  // Entry q lies in a chunk that has been handed out.
+  __device__ __forceinline__ bool has(uint32_t q) const
+  {
+    uint32_t const chunk = q >> shift;
+    return chunk / kCounterGroups < of_group(chunk % kCounterGroups);
+  }
+};
 
 __device__ __forceinline__ void wave_lds_sync()
 {
@@ -1135,7 +1170,7 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
   uint32_t block_known = 0, block_notes = 0;  // INLINE: of the tiles of this wavefront
   bool const use_memo   = !INLINE && a.memo && memo_pays(a.memo_count[0], a.memo_count[1]);
 
-  uint32_t const my_number = blockIdx.x * kWaves + threadIdx.x / kWave;
+  uint32_t const my_number = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x * kWaves + threadIdx.x / kWave)));
   for (bool first = true;; first = false) {
     uint32_t range;
     if constexpr (INLINE) {
@@ -1426,11 +1461,7 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
         // lies behind the word it came from); what becomes of them, their slots and the records of those that go to the
         // queue follow afterwards, lanes <-> listed words.
         if (cursor + nwc > a.range_cap) spill = true;
-        uint32_t const room = q_lim - q_pos;  // left of the reserved entries: used up before the next ones are begun
-        uint32_t fresh      = 0;              // where the next ones begin, once they are needed
-        bool have_fresh     = false;
-        uint32_t listed     = 0;
-        auto queue_place = [&](uint32_t c) { return c < room ? q_pos + c : fresh + (c - room); };
+        uint32_t listed = 0;
         for (uint32_t k0 = 0; k0 < nwc; k0 += kWave) {
           uint32_t const k   = k0 + lane;
           bool const active  = k < nwc;
@@ -1492,7 +1523,6 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
         }
         wave_lds_sync();
         // the listed words: from the memo, or a queue record with the word's first 16 bytes, its length, its range and where it begins
-        uint32_t placed = 0;  // of them, in the queue
         for (uint32_t c0 = 0; c0 < listed; c0 += kWave) {
           uint32_t const c     = c0 + lane;
           uint32_t const entry = lds.word[c < listed ? c : 0u];
@@ -1521,16 +1551,20 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
           }
           uint64_t const qm = ballot64(queued);
           uint32_t const nq = static_cast<uint32_t>(__builtin_popcountll(qm));
-          if constexpr (INLINE) {
-            if (placed + nq > room) spill = true;
-          } else if (placed + nq > room && !have_fresh) {
-            if (lane == 0) fresh = atomicAdd(a.queue_size, kQueueChunk);
-            fresh      = wave_bcast(fresh, 0);
-            have_fresh = true;
+          uint32_t const room = q_lim - q_pos;  // left of the reserved entries: used up before the next ones are begun
+          uint32_t fresh      = 0;
+          if (nq > room) {
+            if constexpr (INLINE) {
+              spill = true;
+            } else {
+              // (a chunk has an entry for every lane)
+              uint32_t const group = my_number % kCounterGroups;
+              if (lane == 0) fresh = atomicAdd(a.queue_chunks + group * kFlagLine, 1u);
+              fresh = (wave_bcast(fresh, 0) * kCounterGroups + group) << a.queue_shift;
+            }
           }
-          uint32_t const place = placed + lanes_below(qm);
-          uint32_t const q     = queue_place(place);
-          placed += nq;
+          uint32_t const place = lanes_below(qm);
+          uint32_t const q     = place < room ? q_pos + place : fresh + (place - room);
           if (queued) value = kOovMark | q;
           if (c < listed && !spill) region[cursor + (entry >> 21)] = value;
           if (queued) {
@@ -1575,14 +1609,12 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
                                                static_cast<uint32_t>(static_cast<uint64_t>(at) >> 32)));
             }
           }
-        }
-        if (INLINE) {
-          q_pos += min(placed, room);
-        } else if (placed > room) {
-          q_pos = fresh + (placed - room);
-          q_lim = fresh + kQueueChunk;
-        } else {
-          q_pos += placed;
+          if (INLINE || nq <= room) {
+            q_pos += min(nq, room);
+          } else {
+            q_pos = fresh + (nq - room);
+            q_lim = fresh + (1u << a.queue_shift);
+          }
         }
         cursor += nwc;
         wave_lds_sync();
@@ -1634,11 +1666,10 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
 
 // ------------------------------------------------------------------ out-of-vocabulary pass
 // One lane per queued word, and a lane that finishes its word stores the result and takes the next one.  A wavefront
-// takes kOovBlock queue entries at a time (one atomic), brings them into LDS 64 at a time with whole-record reads (the
+// takes a chunk of the queue at a time (one atomic), brings them into LDS 64 at a time with whole-record reads (the
 // next 64 are requested while these are worked on) and lets its idle lanes take entries from there every trip.  Words
 // of up to 16 bytes, whole in their queue record, run in registers; the few longer ones are set aside and done, one
 // lane each, by the general state machine over the chars in memory, 64 and more at a time or at the end.
-constexpr uint32_t kOovBlock = 512;
 constexpr int kRefillAt      = 32;
 constexpr int kOovWaves      = 16;  // (two workgroups to a CU, 73 KB of LDS each, 8 wavefronts per SIMD)
 constexpr int kOovThreads    = kOovWaves * kWave;
@@ -1649,10 +1680,10 @@ struct OovLds {
 };
 
 __global__ void __launch_bounds__(kOovThreads, 8) wordpiece_oov_kernel(VocabTable table, const uint4* abase, OovEntry* __restrict__ queue,
-                                                                    const uint32_t* __restrict__ queue_size, uint32_t queue_cap,
+                                                                    QueueChunks chunks, uint32_t queue_cap,
                                                                     uint32_t* __restrict__ range_tokens, uint32_t* __restrict__ counter,
                                                                     uint32_t* __restrict__ longer, uint32_t* __restrict__ longer_count,
-                                                                    const uint32_t* __restrict__ queue_begin)
+                                                                    const uint32_t* __restrict__ begin_chunks)
 {
   __shared__ OovLds lds_all[kOovWaves];
   __shared__ int32_t first_ids[512];  // the ids of the one-byte keys of both key spaces: looked at whenever a piece of a word begins
@@ -1661,16 +1692,14 @@ __global__ void __launch_bounds__(kOovThreads, 8) wordpiece_oov_kernel(VocabTabl
   __shared__ uint4 trim[17];
   // an empty queue (a small call, text that is all in the vocabulary), or one that was too small (the host repeats the
   // passes with a larger one): nothing to do, and the tables need not be fetched
-  if (*queue_size == 0 || *queue_size > queue_cap) return;
+  uint64_t const extent = chunks.extent();
+  if (extent == 0 || extent > queue_cap) return;
   fill_trim_table(trim);
   for (int i = threadIdx.x; i < 512; i += kOovThreads) first_ids[i] = table.short_ids[2 * 65536 + i];
   for (uint32_t i = threadIdx.x; i < kLetters2; i += kOovThreads) pair_ids[i] = table.short_ids[65536 + ((i / 26u + 'a') | ((i % 26u + 'a') << 8))];
   for (uint32_t i = threadIdx.x; i < kLetters3 / 2; i += kOovThreads)
     reinterpret_cast<uint32_t*>(letters3)[i] = reinterpret_cast<const uint32_t*>(table.letters3)[i];
   __syncthreads();
-  uint32_t const total = *queue_size;
-  uint32_t const begin = queue_begin ? *queue_begin / kOovBlock : 0u;  // (whole blocks: what the word pass reserves at a time)
-  static_assert(kOovBlock == kQueueChunk, "the entries of a launch of the word pass are whole blocks");
   OovLds& lds          = lds_all[threadIdx.x / kWave];
   int const lane       = lane_id();
 
@@ -1711,23 +1740,26 @@ __global__ void __launch_bounds__(kOovThreads, 8) wordpiece_oov_kernel(VocabTabl
   };
   uint4 mine_tail = make_uint4(0u, 0u, 0u, 0u);  // the second half of my word's entry
 
-  // the queue entries being fetched: [f_base, f_base + f_n), one per lane; they come from the block [.., q_end) that
-  // this wavefront has taken, and a new block is taken when that one is used up
+  // the queue entries being fetched: [f_base, f_base + f_n), one per lane; they come from the chunk [.., q_end) that
+  // this wavefront has taken, and a new chunk of its group is taken when that one is used up
   uint32_t next_fetch = 0, q_end = 0, f_base = 0, f_n = 0;
-  bool no_more = false, first_block = true;
-  uint32_t const my_number = blockIdx.x * kOovWaves + threadIdx.x / kWave;
+  bool no_more = false, first_chunk = true;
+  // (neighbouring workgroups take neighbouring chunks: few are shared out over all CUs)
+  uint32_t const my_number = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave * gridDim.x + blockIdx.x)));
+  uint32_t const group     = my_number % kCounterGroups;
+  uint32_t const handed    = chunks.of_group(group);
+  uint32_t const begin     = begin_chunks ? begin_chunks[group] : 0u;
   uint4 pa = make_uint4(0u, 0u, 0u, 0u), pb = pa;
   auto start_fetch = [&] {
     f_n = 0;
     if (next_fetch >= q_end && !no_more) {
-      uint32_t const block   = begin + next_unit(counter, first_block, my_number, lane);
-      first_block            = false;
-      uint64_t const b_begin = static_cast<uint64_t>(block) * kOovBlock;
-      if (b_begin >= total) {
+      uint32_t const n = next_unit(counter, first_chunk, my_number, lane) / kCounterGroups;  // (of the group)
+      first_chunk      = false;
+      if (n >= handed - begin) {
         no_more = true;
       } else {
-        next_fetch = static_cast<uint32_t>(b_begin);
-        q_end      = static_cast<uint32_t>(min(b_begin + kOovBlock, static_cast<uint64_t>(total)));
+        next_fetch = ((begin + n) * kCounterGroups + group) << chunks.shift;
+        q_end      = next_fetch + (1u << chunks.shift);
       }
     }
     if (next_fetch < q_end) {
@@ -1849,12 +1881,12 @@ static_assert(RareWords::kRow % 2 == 1, "the rows begin in different banks");
 
 // The queued words of more than 16 bytes, which the kernel above has listed: one lane per word, the general state machine.
 __global__ void __launch_bounds__(kRareThreads) wordpiece_oov_long_kernel(VocabTable table, const uint4* abase, OovEntry* __restrict__ queue,
-                                                                         const uint32_t* __restrict__ queue_size, uint32_t queue_cap,
+                                                                         QueueChunks chunks, uint32_t queue_cap,
                                                                          const uint32_t* __restrict__ longer, const uint32_t* __restrict__ longer_count,
                                                                          uint32_t* __restrict__ range_tokens)
 {
   __shared__ RareWords words;
-  if (*queue_size > queue_cap) return;  // (see wordpiece_oov_kernel)
+  if (chunks.extent() > queue_cap) return;  // (see wordpiece_oov_kernel)
   uint32_t const n = *longer_count;
   for (uint32_t i = blockIdx.x * kRareThreads + threadIdx.x; i < n; i += gridDim.x * kRareThreads) {
     uint32_t const q   = longer[i];
@@ -1883,15 +1915,16 @@ __global__ void __launch_bounds__(kRareThreads) wordpiece_oov_long_kernel(VocabT
 // Between the word pass and the out-of-vocabulary pass of the first ranges: every queued word of up to kMemoWord bytes
 // puts itself in its place (owners[e] = 1 + its queue entry).
 constexpr int kMemoThreads = 1024;  // (few workgroups: one atomic each)
-__global__ void __launch_bounds__(kMemoThreads) wordpiece_memo_claim_kernel(const OovEntry* __restrict__ queue, const uint32_t* __restrict__ queue_size,
+__global__ void __launch_bounds__(kMemoThreads) wordpiece_memo_claim_kernel(const OovEntry* __restrict__ queue, QueueChunks chunks,
                                                                             uint32_t queue_cap, uint32_t* __restrict__ owners, uint32_t* __restrict__ counts)
 {
   __shared__ uint32_t all;
   if (threadIdx.x == 0) all = 0;
   __syncthreads();
-  uint32_t const total = min(*queue_size, queue_cap);
+  uint32_t const total = static_cast<uint32_t>(min(chunks.extent(), static_cast<uint64_t>(queue_cap)));
   uint32_t words       = 0;
   for (uint32_t q = blockIdx.x * kMemoThreads + threadIdx.x; q < total; q += gridDim.x * kMemoThreads) {
+    if (!chunks.has(q)) continue;
     const uint4* const e = reinterpret_cast<const uint4*>(queue + q);
     uint4 const h = e[0], n = e[1];
     uint32_t const wl = n.x & 0xFFu;
@@ -1905,7 +1938,8 @@ __global__ void __launch_bounds__(kMemoThreads) wordpiece_memo_claim_kernel(cons
   __syncthreads();
   if (threadIdx.x == 0) {
     if (all != 0) atomicAdd(&counts[0], all);
-    if (blockIdx.x == 0) counts[2] = *queue_size;
+    if (blockIdx.x == 0)
+      for (uint32_t g = 0; g < kCounterGroups; ++g) counts[kMemoChunks + g] = chunks.of_group(g);
   }
 }
 
@@ -2217,15 +2251,17 @@ __global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, Vo
 }
 
 // What the host needs to know before the emit pass: the number of tokens, whether a range ran out of word slots, the
-// queue entries reserved.
-__global__ void publish_state_kernel(const uint64_t* __restrict__ total, const uint32_t* __restrict__ flags, uint64_t* __restrict__ dst,
-                                     HostPost post)
+// queue entries that there ought to be.
+__global__ void publish_state_kernel(const uint64_t* __restrict__ total, const uint32_t* __restrict__ flags, QueueChunks chunks,
+                                     uint64_t* __restrict__ dst, HostPost post)
 {
   dst[0] = *total;
   dst[1] = flags[kFlagOverflow];
-  dst[2] = flags[kFlagQueueSize];
+  dst[2] = chunks.extent();
   post.send();
 }
+// ... where the host copies the flags.
+__global__ void extent_kernel(uint32_t* __restrict__ flags, QueueChunks chunks) { flags[kFlagExtent] = static_cast<uint32_t>(min(chunks.extent(), uint64_t{0xFFFFFFFFu})); }
 
 struct RangeTokensOf {
   const uint32_t* counts;
@@ -2821,10 +2857,12 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   int64_t const word_resident = resident(reinterpret_cast<const void*>(word_kernel), word_waves(false) * kWave, (is64 ? 2 : 0) + (limit ? 1 : 0));
   // A range is what a wavefront works through by itself, one tile after the other: kRangeTiles tiles when that still
   // leaves every wavefront of the word pass eight ranges or more (the last ones then end close together), fewer in a
-  // smaller column (2M rows of 120 bytes: 0.34 -> 0.30 ms for the word pass).
+  // smaller column (2M rows of 120 bytes: 0.34 -> 0.30 ms for the word pass); a single one only where there are not enough
+  // tiles for all wavefronts (780,000 rows of 256 bytes in ranges of 1: 570 us, 2: 530, 4: 541; 128,000 of 500 293, 279, 291).
   constexpr int kWordWaves = word_waves(false);
   int range_tiles = kRangeTiles;
-  while (range_tiles > 1 && ntiles / range_tiles < 8 * word_resident * kWordWaves) range_tiles >>= 1;
+  int const least_tiles = ntiles < word_resident * kWordWaves ? 1 : 2;
+  while (range_tiles > least_tiles && ntiles / range_tiles < 8 * word_resident * kWordWaves) range_tiles >>= 1;
   // A large column with unknown words is done in two parts, the first for the memo: shorter ranges, so that the first part has
   // enough of them to share out (tiles of 2 KB to a range: 1: 1388 us, 2: 1255, 4: 1243, 8: 1324).
   bool const with_memo = cend >= kMemoLeast && sample_queued * 50 > sample_words;
@@ -2861,8 +2899,16 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   // bytes and queues a word per 32 bytes.  A column with more (rows or words of a byte or two; text in another
   // language than the vocabulary's) makes the attempt fail, and the second has what the first found to be needed:
   // room for a word per byte, the exact number of queue entries.
-  uint32_t range_cap      = static_cast<uint32_t>(kRange * 5 / 16);
-  uint64_t queue_capacity = static_cast<uint64_t>((last_offset - first_offset) >> 5) + static_cast<uint64_t>(word_grid + word_grid2) * kWordWaves * kQueueChunk + 4096;
+  uint32_t range_cap    = static_cast<uint32_t>(kRange * 5 / 16);
+  uint32_t queue_chunk  = kQueueChunk;
+  uint64_t const word_pass_waves = static_cast<uint64_t>(word_grid + word_grid2) * kWordWaves;
+  if (sample_bytes > 0) {
+    // (a wavefront of the first launch reserves some four times)
+    double const each = sample_queued / sample_bytes * static_cast<double>(first_part) * static_cast<double>(kRange) / static_cast<double>(word_grid * kWordWaves);
+    while (queue_chunk > kQueueLeastChunk && static_cast<double>(queue_chunk) * 4 > each) queue_chunk /= 2;
+  }
+  args.queue_shift        = static_cast<uint32_t>(__builtin_ctz(queue_chunk));
+  uint64_t queue_capacity = static_cast<uint64_t>((last_offset - first_offset) >> 5) + word_pass_waves * queue_chunk + 4096;
   if (sample_bytes > 0) {
     // what the sample calls for, with half as much again for the ranges that are denser than the column as a whole
     // (never less than the sizes above: a sample can miss; the second attempt remains)
@@ -2871,7 +2917,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     range_cap = static_cast<uint32_t>(std::min<double>(static_cast<double>(kRange + 8), std::max<double>(range_cap, per_byte_words * 1.5 * static_cast<double>(kRange) + 256)));
     range_cap = (range_cap + 1u) & ~1u;  // (a range's slots begin at an even index)
     queue_capacity = std::max<uint64_t>(queue_capacity, static_cast<uint64_t>(per_byte_queued * 1.25 * static_cast<double>(last_offset - first_offset)) +
-                                                          static_cast<uint64_t>(word_grid + word_grid2) * kWordWaves * kQueueChunk + 4096);
+                                                          word_pass_waves * queue_chunk + 4096);
   }
   uint64_t total = 0;
   for (int attempt = 0;; ++attempt) {
@@ -2907,7 +2953,8 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     args.offsets_out     = out->offsets;
     args.queue           = queue;
     args.queue_cap       = qcap;
-    args.queue_size      = flags + kFlagQueueSize;
+    args.queue_chunks    = flags + kFlagQueue;
+    QueueChunks const chunks{flags + kFlagQueue, args.queue_shift};
     args.overflow        = flags + kFlagOverflow;
     uint4* const memo      = temps.part<uint4>(9);
     uint32_t* const owners = memo_entries ? reinterpret_cast<uint32_t*>(memo + kMemoEntries) : nullptr;
@@ -2924,15 +2971,15 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
         hipLaunchKernelGGL(word_kernel, dim3(part == 0 ? word_grid : word_grid2), dim3(kWordWaves * kWave), 0, stream, args);
       }
       if (part == 0 && owners) {
-        hipLaunchKernelGGL(wordpiece_memo_claim_kernel, dim3(static_cast<unsigned>(cus)), dim3(kMemoThreads), 0, stream, queue, flags + kFlagQueueSize, qcap,
+        hipLaunchKernelGGL(wordpiece_memo_claim_kernel, dim3(static_cast<unsigned>(cus)), dim3(kMemoThreads), 0, stream, queue, chunks, qcap,
                            owners, flags + kFlagMemo);
         hipLaunchKernelGGL(wordpiece_memo_keys_kernel, dim3(kMemoEntries / kMemoThreads), dim3(kMemoThreads), 0, stream, queue, owners, memo,
                            flags + kFlagMemo);
       }
       {
         ProfileScope ps("wordpiece_oov_kernel", stream);
-        hipLaunchKernelGGL(wordpiece_oov_kernel, dim3(oov_grid), dim3(kOovThreads), 0, stream, vocabulary->table, args.abase, queue, flags + kFlagQueueSize, qcap,
-                           tokens, flags + (part == 0 ? kFlagOovUnits : kFlagOovUnits2), longer, flags + kFlagLonger, part == 0 ? nullptr : flags + kFlagMemo + 2);
+        hipLaunchKernelGGL(wordpiece_oov_kernel, dim3(oov_grid), dim3(kOovThreads), 0, stream, vocabulary->table, args.abase, queue, chunks, qcap,
+                           tokens, flags + (part == 0 ? kFlagOovUnits : kFlagOovUnits2), longer, flags + kFlagLonger, part == 0 ? nullptr : flags + kFlagMemo + kMemoChunks);
       }
       if (part == 0 && owners)
         hipLaunchKernelGGL(wordpiece_memo_fill_kernel, dim3(kMemoEntries / kMemoThreads), dim3(kMemoThreads), 0, stream, queue, owners, memo, queue + qcap);
@@ -2940,42 +2987,45 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     {
       ProfileScope ps("wordpiece_oov_long_kernel", stream);
       hipLaunchKernelGGL(wordpiece_oov_long_kernel, dim3(static_cast<unsigned>(cus) * kRareGroups), dim3(kRareThreads), 0, stream, vocabulary->table, args.abase, queue,
-                         flags + kFlagQueueSize, qcap, longer, flags + kFlagLonger, tokens);
+                         chunks, qcap, longer, flags + kFlagLonger, tokens);
     }
     // where the tokens of each range go; the total decides the child size
     // (cpp/include/cudf/detail/sizes_to_offsets_iterator.cuh:302-339)
     device_exclusive_scan(RangeTokensOf{tokens}, static_cast<int64_t>(nranges), bases, scan_tmp, stream);
     // the total (the last word of the scan's temporaries) and the first flag words: written to the pinned words by a
     // kernel of one thread, or, without those, fetched in one copy (the flags lie right behind the scan's temporaries)
-    uint32_t state[3] = {0, 0, 0};
+    uint64_t state[3] = {0, 0, 0};  // (the first flag words: an overflow, the queue's extent)
     if (scalars) {
       HostPost const post = new_post();
-      hipLaunchKernelGGL(publish_state_kernel, dim3(1), dim3(1), 0, stream, scan_tmp + scan_tiles(nranges), flags, scalars + 2, post);
+      hipLaunchKernelGGL(publish_state_kernel, dim3(1), dim3(1), 0, stream, scan_tmp + scan_tiles(nranges), flags, chunks, scalars + 2, post);
       hipError_t e = hipGetLastError();
       if (e == hipSuccess) e = wait_for_post(post, stream);
       if (e != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
       total    = scalars[2];
-      state[1] = static_cast<uint32_t>(scalars[3]);
-      state[2] = static_cast<uint32_t>(scalars[4]);
+      state[1] = scalars[3];
+      state[2] = scalars[4];
     } else {
       const char* const from = reinterpret_cast<const char*>(scan_tmp + scan_tiles(nranges));
+      uint32_t words_of[3]   = {0, 0, 0};
       size_t const span      = static_cast<size_t>(reinterpret_cast<const char*>(flags + 3) - from);
-      alignas(8) char both[256 + 8 + sizeof(state)];
+      alignas(8) char both[256 + 8 + sizeof(words_of)];
       if (span > sizeof(both)) return give_up(NVTEXT_AMD_LOGIC_ERROR, "unexpected layout of the temporaries");
+      hipLaunchKernelGGL(extent_kernel, dim3(1), dim3(1), 0, stream, flags, chunks);
       hipError_t e = hipMemcpyAsync(both, from, span, hipMemcpyDeviceToHost, stream);
       if (e == hipSuccess) e = hipStreamSynchronize(stream);
       if (e != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
       std::memcpy(&total, both, sizeof(total));
-      std::memcpy(state, both + span - sizeof(state), sizeof(state));
+      std::memcpy(words_of, both + span - sizeof(words_of), sizeof(words_of));
+      for (int i = 1; i < 3; ++i) state[i] = words_of[i];
     }
     bool const words_over = state[1] != 0, queue_over = state[2] > qcap;
     if (words_over || queue_over) {
       if (attempt > 0 || state[2] > 0x7FFFFFF0u) return give_up(NVTEXT_AMD_LOGIC_ERROR, "words exceed internal limit");
       if (words_over) range_cap = static_cast<uint32_t>(kRange + 8);
-      // state[2] counts the chunks of kQueueChunk entries that the wavefronts reserved, the unused rest of each
-      // wavefront's last chunk included; which ranges a wavefront gets differs from one attempt to the next, and with it
-      // that rest: a chunk per wavefront on top of what this attempt reserved covers every assignment.
-      queue_capacity = std::max<uint64_t>(queue_capacity, static_cast<uint64_t>(state[2]) + static_cast<uint64_t>(word_grid + word_grid2) * kWordWaves * kQueueChunk);
+      // state[2] counts what the wavefronts reserved, the unused rest of each wavefront's last chunk included; which
+      // ranges of its group a wavefront gets differs from one attempt to the next, and with it that rest: a chunk per
+      // wavefront on top of what this attempt reserved covers every assignment.
+      queue_capacity = std::max<uint64_t>(queue_capacity, state[2] + word_pass_waves * queue_chunk);
       continue;
     }
     if (total > static_cast<uint64_t>(std::numeric_limits<int32_t>::max())) return give_up(NVTEXT_AMD_OVERFLOW, "Size of output exceeds the column size limit");

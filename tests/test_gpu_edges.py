@@ -413,6 +413,23 @@ def test_tokenize_blocks_of_tiles(nv, orc, tiles):
         assert nv.wordpiece_tokenize(column, vocabulary, 60).to_host().equals(expected)
 
 
+@pytest.mark.parametrize("rows", [140_000, 700_000])
+@pytest.mark.parametrize("oov", [0.0, 0.003, 0.1, 0.5, 1.0])
+def test_tokenize_chunks_of_the_queue(nv, orc, rows, oov):
+    """Columns beyond the small ones with no unknown word, a few for some of the wavefronts, a few for each, and so many that
+    the queue is handed out in larger chunks; some with words that overflow the first attempt's queue at one end of the column."""
+    rng = np.random.default_rng(rows + int(100 * oov))
+    hv = HostStringsColumn.from_pylist(VOCABULARY)
+    vocabulary, reference = nv.WordPieceVocabulary(dev(nv, hv)), orc.Vocabulary(hv)
+    text = words_column(rng, [300_000], VOCABULARY, oov).chars
+    total = rows * 60
+    chars = np.tile(text, total // text.size + 1)[:total].copy()
+    if oov == 0.1:
+        chars[total - total // 6:] = np.frombuffer(b"qz " * (total // 18 + 1), np.uint8)[: total // 6]
+    host = HostStringsColumn(chars, np.linspace(0, total, rows + 1).astype(np.int32), None, rows, 0, 0)
+    assert nv.wordpiece_tokenize(dev(nv, host), vocabulary, 0).to_host().equals(orc.wordpiece_tokenize(host, reference, 0, nthreads=8))
+
+
 def test_tokenize_from_threads_that_come_and_go(nv, orc):
     """Forty host threads, eight at a time, tokenize small columns of different sizes: what a call adds up on the device is its thread's own,
     and is there again for the threads that follow."""
