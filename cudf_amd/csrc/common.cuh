@@ -501,14 +501,12 @@ void device_exclusive_scan(F f, int64_t n, OutT* out, uint64_t* temp, hipStream_
 int device_cus();
 
 // ------------------------------------------------------------------ scalars for the host
-// A few KB of pinned host memory that kernels write and the host reads (a copy of a few bytes into ordinary host memory
-// goes through a staging buffer and costs ten microseconds and more): eight 64-bit words, behind them room for
-// kHostSampleWords 32-bit words, and a word in a cache line of its own that says what has been written.  One buffer per
-// host thread, allocated at the thread's first call and kept until the process ends; nullptr when the allocation failed
-// (the callers then copy).
-constexpr size_t kHostSampleWords = 3 * 512;
-constexpr size_t kHostPostedWord  = 8 + (kHostSampleWords / 2 + 7) / 8 * 8;  // (in 64-bit words)
-constexpr size_t kHostScalarBytes = (kHostPostedWord + 8) * sizeof(uint64_t);
+// A little pinned host memory that kernels write and the host reads (a copy of a few bytes into ordinary host memory
+// goes through a staging buffer and costs ten microseconds and more): eight 64-bit words, and a word in a cache line of its
+// own that says what has been written.  One buffer per host thread, allocated at the thread's first call and kept until the
+// process ends; nullptr when the allocation failed (the callers then copy).
+constexpr size_t kHostPostedWord  = 16;  // (in 64-bit words)
+constexpr size_t kHostScalarBytes = (kHostPostedWord + 16) * sizeof(uint64_t);
 uint64_t* host_scalars();
 
 // Word from a kernel that what it (and the kernels before it on its stream) wrote to the pinned words is there.  The host

@@ -2186,29 +2186,33 @@ __global__ void __launch_bounds__(kRareThreads) wordpiece_retokenize_kernel(Voca
 // first looks at kSampleWindows windows of kSampleBytes spread evenly over the column's bytes, one wavefront each:
 // words as maximal runs of bytes that are not spaces (rows and the word limit are left aside: an estimate), each
 // looked up whole.  It runs on the offsets alone, before the host knows where the bytes begin, and leaves the view's
-// first and last offset for the host as well: the call synchronises once for both.
+// first and last offset for the host as well: the call waits once for both, for the word of the last window to be done,
+// which learns the sums from what the atomic that adds its own answers.
 constexpr int kSampleWindows = 512;
 constexpr int kSampleBytes   = 512;
 constexpr int kSampleTail    = 208;  // bytes staged past a window: a word that starts in it ends there, or is kMaxWord bytes or more
-static_assert(3 * kSampleWindows <= kHostSampleWords, "a window's three counts fit the pinned words");
+// Arrivals::sum here: words, queued words, windows
+constexpr int kSampleQueuedAt = 24, kSampleWindowsAt = 48;
+static_assert(kSampleWindows * kSampleBytes < (1 << kSampleQueuedAt), "the sums stay apart");
+__host__ __device__ inline int64_t sample_windows(int64_t span)
+{
+  int64_t const windows = (span + kSampleBytes - 1) / kSampleBytes;
+  return windows < kSampleWindows ? windows : kSampleWindows;
+}
+__host__ __device__ inline int64_t sample_begin(int64_t span, int64_t window) { return span / sample_windows(span) * window; }
 
-__global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, VocabTable table, uint64_t* __restrict__ first_last,
-                                                               uint32_t* __restrict__ counts, uint32_t* __restrict__ hot)
+__global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, VocabTable table, uint64_t* __restrict__ host,
+                                                               uint32_t* __restrict__ hot, Arrivals* __restrict__ arrivals, HostPost post)
 {
   __shared__ uint32_t staged[(kSampleBytes + kSampleTail + 8) / 4 + 4];  // byte 4 + x of it: byte x of the window; byte 3: the one before
   int const lane      = lane_id();
   int64_t const first = col.off(0), last = col.off(col.size);
-  if (blockIdx.x == 0 && lane == 0) {
-    first_last[0] = static_cast<uint64_t>(first);
-    first_last[1] = static_cast<uint64_t>(last);
-  }
   int64_t const span    = last - first;
-  int64_t const windows = min(static_cast<int64_t>(kSampleWindows), (span + kSampleBytes - 1) / kSampleBytes);
-  uint32_t words = 0, queued = 0, bytes = 0;
+  int64_t const windows = span > 0 ? sample_windows(span) : 0;
+  uint32_t words = 0, queued = 0;
   if (static_cast<int64_t>(blockIdx.x) < windows) {
-    int64_t const begin = first + span / windows * blockIdx.x;
-    int64_t const end   = min(last, begin + kSampleBytes);
-    bytes               = static_cast<uint32_t>(end - begin);
+    int64_t const begin  = first + sample_begin(span, blockIdx.x);
+    uint32_t const bytes = static_cast<uint32_t>(min(last, begin + kSampleBytes) - begin);
     uint8_t* const sb   = reinterpret_cast<uint8_t*>(staged);
     for (int i = lane; i < 4 + kSampleBytes + kSampleTail + 8; i += kWave) {
       int64_t const g = begin + i - 4;
@@ -2243,10 +2247,15 @@ __global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, Vo
     }
   }
   uint32_t const w = wave_bcast(wave_inclusive_scan(words), kWave - 1), q = wave_bcast(wave_inclusive_scan(queued), kWave - 1);
-  if (lane == 0) {
-    counts[3 * blockIdx.x]     = w;
-    counts[3 * blockIdx.x + 1] = q;
-    counts[3 * blockIdx.x + 2] = bytes;
+  if (lane != 0) return;
+  unsigned long long const mine = w | static_cast<unsigned long long>(q) << kSampleQueuedAt | 1ull << kSampleWindowsAt;
+  unsigned long long const all  = atomicAdd(&arrivals->sum, mine) + mine;
+  if (all >> kSampleWindowsAt == kSampleWindows) {
+    atomicExch(&arrivals->sum, 0ull);  // (for the next)
+    host[0] = static_cast<uint64_t>(first);
+    host[1] = static_cast<uint64_t>(last);
+    host[2] = all;
+    post.send();
   }
 }
 
@@ -2696,7 +2705,8 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   size_t const ow = input->offsets_is_int64 ? 8 : 4;
   int64_t first_offset = 0, last_offset = 0;
   uint64_t* const scalars = host_scalars();  // pinned words that kernels write for the host (nullptr: copy instead)
-  bool const sampling     = g_sizing_sample.load(std::memory_order_relaxed) != 0;
+  Arrivals* const arrivals = scalars ? thread_arrivals() : nullptr;
+  bool const sampling      = arrivals && g_sizing_sample.load(std::memory_order_relaxed) != 0;
   double sample_words = 0, sample_queued = 0, sample_bytes = 0;  // what the sample found (nothing without the pinned words)
   bool const is64  = input->offsets_is_int64 != 0;
   bool const limit = max_words_per_row > 0;
@@ -2706,8 +2716,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   // take (which is also done where a tile had not enough of them), beyond the call goes on as for a large column.
   // (29 rows of 180 bytes: 87 us in eleven launches with two waits, 34 in four with one, 32 in two; 32,768 rows of 120 bytes
   // 145, 50 and 47 us, 10 MB of those 84 and 77 with the last two)
-  Arrivals* const arrivals = scalars && sampling && rows <= kSmallRows && g_forced_range_tiles.load(std::memory_order_relaxed) == 0 ? thread_arrivals() : nullptr;
-  bool const small         = arrivals != nullptr;
+  bool const small    = sampling && rows <= kSmallRows && g_forced_range_tiles.load(std::memory_order_relaxed) == 0;
   int64_t const small_most = std::min(std::max(rows * kSmallRowBytes, kSmallLeast), kSmallBytes);
   int64_t small_bytes      = small ? std::min(std::max(rows * kSmallGuess, kSmallSure), small_most) : 0;
   for (int attempt = 0; attempt < 2 && small_bytes > 0; ++attempt) {
@@ -2786,25 +2795,29 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     bool const full = bytes <= small_bytes && small_slots(slots, nranges) == kSmallSlots && small_queue(records, nranges) == kSmallQueue;
     small_bytes     = full ? 0 : bytes;
   }
-  Temp const hot(mr, scalars && sampling ? kHotWords * sizeof(uint32_t) : 0);
+  Temp const hot(mr, sampling ? kHotWords * sizeof(uint32_t) : 0);
   if (!hot.ok()) return give_up(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");
   if (scalars) {
-    uint32_t* const counts = reinterpret_cast<uint32_t*>(scalars + 8);
-    HostPost const post    = new_post();
+    HostPost const post = new_post();
     if (sampling)
-      hipLaunchKernelGGL(wordpiece_sample_kernel, dim3(kSampleWindows), dim3(kWave), 0, stream, v, vocabulary->table, scalars, counts,
-                         hot.as<uint32_t>());
+      hipLaunchKernelGGL(wordpiece_sample_kernel, dim3(kSampleWindows), dim3(kWave), 0, stream, v, vocabulary->table, scalars, hot.as<uint32_t>(),
+                         arrivals, post);
     else
       launch_read_two_offsets(input->offsets, input->offsets_is_int64 != 0, input->offset, static_cast<int64_t>(input->offset) + rows, scalars, post, stream);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = sampling ? hipStreamSynchronize(stream) : wait_for_post(post, stream);
-    if (e != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
+    bool const launched = e == hipSuccess;
+    if (launched) e = wait_for_post(post, stream);
+    if (e != hipSuccess) {
+      if (launched && sampling) forsake_thread_arrivals();
+      return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
+    }
     first_offset = static_cast<int64_t>(scalars[0]);
     last_offset  = static_cast<int64_t>(scalars[1]);
-    for (int i = 0; sampling && i < kSampleWindows; ++i) {
-      sample_words += counts[3 * i];
-      sample_queued += counts[3 * i + 1];
-      sample_bytes += counts[3 * i + 2];
+    if (sampling && last_offset > first_offset) {
+      int64_t const span = last_offset - first_offset;
+      sample_words       = static_cast<double>(scalars[2] & ((1u << kSampleQueuedAt) - 1u));
+      sample_queued      = static_cast<double>(scalars[2] >> kSampleQueuedAt & ((1u << (kSampleWindowsAt - kSampleQueuedAt)) - 1u));
+      for (int64_t i = 0; i < sample_windows(span); ++i) sample_bytes += static_cast<double>(std::min<int64_t>(span - sample_begin(span, i), kSampleBytes));
     }
   } else {
     unsigned char buf[16] = {0};
