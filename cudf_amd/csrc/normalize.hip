@@ -52,7 +52,7 @@ constexpr int kRawWords    = (kNormTile + kRawBefore + kRawAfter + 15 + 15) / 16
 constexpr int32_t kSmallRows     = 131072;  // a column of so many rows is worked on before its size is known (see nvtext_amd_normalize_characters)
 constexpr int64_t kSmallRowBytes = 4096;
 constexpr int64_t kSmallLeast    = 256 << 10;
-constexpr int64_t kSmallBytes    = 64 << 20;
+constexpr int64_t kSmallBytes    = 20 << 20;  // (40 MB of mixed text that way 130 us, as a large column 103; 18 MB 72 and 74)
 constexpr int kStageBytes  = 4 * kNormTile;  // output bytes of a tile that are assembled in LDS; a tile with more writes them one by one
 
 constexpr uint32_t kNotShort = 0x80000000u;  // beside the bytes of a string: there are more than eight, or it is the " [ " that may open a special token
@@ -720,11 +720,11 @@ __global__ void __launch_bounds__(kNormThreads, 8) normalize_count_kernel(const 
 // normalize_count_kernel does them.
 // What bounds it is instructions again: with a workgroup a tile half the time went on barriers, on starting, on staging
 // the table and on a list for every 512 bytes.  766 MB of mixed text 461 -> 255 to 266 us (traced); several tiles for a wavefront, with the bytes
-// of the next one on their way, no faster.  A small column has too few wavefronts this way: of 17 MB 73.5 us a call with a
-// workgroup a tile and 75.5 with this, of 34 MB 110 and 108, of 67 MB 180 and 172.
+// of the next one on their way, no faster.  A small column has too few wavefronts this way: with both passes by workgroups below 12,288
+// tiles, or by wavefronts from 4,096 on, 8.5 MB of mixed text take 43.9 and 46.9 us, 18 MB 75.6 and 71, of ASCII 40.9 and 38.8, 65 and 57.
 constexpr int kTileWaves          = kNormThreads / kWave;
 constexpr int kLaneWords          = kNormTile / kWave / 4;  // dwords of a tile per lane, two of every 512 bytes
-constexpr int64_t kManyTiles      = 12288;                  // a column of so many tiles
+constexpr int64_t kManyTiles      = 8192;                   // a column of so many tiles
 // Whether there is nothing for the end.  (Asked before the loop over the four: what the compiler gets ready for that loop it spills
 // to memory, 5 GB of HBM writes beside the 4.2 GB of a result.)
 __device__ __forceinline__ bool none_left(const uint32_t (&left)[kTileWaves])

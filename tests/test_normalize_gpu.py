@@ -337,3 +337,16 @@ def test_normalize_wavefront_a_tile_after_one_wait(nv, onorm, rows, tiles):
     host = HostStringsColumn(chars, offsets, None, rows, 0, 0)
     for tokens in ((), ("[SEP]",)):
         assert_same(run(nv, host, True, tokens), onorm.normalize_characters_native(host, True, [t.encode() for t in tokens], 8), f"{tokens}")
+
+
+@pytest.mark.parametrize("kind", ["plain", "tokens"])
+@pytest.mark.parametrize("rows, tiles", [(40_000, 8191), (40_000, 8192), (40_000, 10_240), (40_000, 10_241), (140_000, 8191), (140_000, 8193), (300, 2048 * 20 + 1)])
+def test_normalize_lines_between_the_ways(nv, onorm, kind, rows, tiles):
+    """Either side of the 8,192 tiles from which a wavefront does a tile alone, of the 20 MiB up to which a column of few rows is
+    counted before its size is known, and of scans of one, a few and many tiles of 2048 sums."""
+    rng = np.random.default_rng(tiles)
+    text = "Some [SEP] words, Été 漢字 Жи 각 and more plain words of text. "
+    chars = np.resize(np.frombuffer((text if kind == "tokens" else text.replace("[SEP]", "sep")).encode(), np.uint8), tiles * TILE - 5)
+    offsets = np.concatenate([[0], np.sort(rng.integers(0, chars.size, rows - 1)), [chars.size]]).astype(np.int32)
+    host = HostStringsColumn(chars, offsets, None, rows, 0, 0)
+    assert_same(run(nv, host, True, ("[SEP]",)), onorm.normalize_characters_native(host, True, [b"[SEP]"], 8), f"{rows} {tiles}")
