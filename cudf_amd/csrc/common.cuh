@@ -396,11 +396,19 @@ __device__ __forceinline__ uint64_t block_exclusive_scan64(uint64_t v, uint64_t*
 }
 
 // ------------------------------------------------------------------ device-wide exclusive scan
-// out[i] = sum_{j<i} f(j) for i in [0, n]  (n+1 entries; out[n] is the total).
-// Three launches: per-tile sums, scan of the tile sums (one workgroup), rescan + add; one launch for a few thousand values.
-constexpr int kScanThreads = 256;
-constexpr int kScanItems   = 8;
-constexpr int kScanTile    = kScanThreads * kScanItems;
+// out[i] = sum_{j<i} f(j) for i in [0, n]  (n+1 entries; out[n] is the total), and tell(total) by one thread as soon as the total
+// is known.
+// Two launches: the sums of the tiles; then every workgroup adds up the sums before its own, and the first all of them.  (With a
+// launch of its own for the scan of the sums, and another to tell the host, calls of 26 to 770 MB took 4 to 6 us more.)
+// Three where there are more than kScanDirect tiles, one for a few thousand values.
+constexpr int kScanThreads    = 256;
+constexpr int kScanItems      = 8;
+constexpr int kScanTile       = kScanThreads * kScanItems;
+constexpr int64_t kScanDirect = 1024;
+
+struct TellNobody {
+  __device__ void operator()(uint64_t) const {}
+};
 
 template <typename F>
 __global__ void __launch_bounds__(kScanThreads) scan_tile_sums_kernel(F f, int64_t n, uint64_t* tile_sums)
@@ -419,10 +427,29 @@ __global__ void __launch_bounds__(kScanThreads) scan_tile_sums_kernel(F f, int64
 }
 
 // exclusive scan of tile_sums in place; tile_sums[ntiles] = grand total
-__global__ void __launch_bounds__(kScanThreads) scan_tile_offsets_kernel(uint64_t* tile_sums, int64_t ntiles);
+template <typename Tell>
+__global__ void __launch_bounds__(kScanThreads) scan_tile_offsets_kernel(uint64_t* tile_sums, int64_t ntiles, Tell tell)
+{
+  __shared__ uint64_t lds[kScanThreads / kWave + 1];
+  uint64_t carry = 0;
+  for (int64_t base = 0; base < ntiles; base += kScanThreads) {
+    int64_t const i  = base + threadIdx.x;
+    uint64_t const v = (i < ntiles) ? tile_sums[i] : 0;
+    uint64_t total;
+    uint64_t const ex = block_exclusive_scan64<kScanThreads>(v, lds, &total);
+    if (i < ntiles) tile_sums[i] = carry + ex;
+    carry += total;
+  }
+  if (threadIdx.x == 0) {
+    tile_sums[ntiles] = carry;
+    tell(carry);
+  }
+}
 
-template <typename F, typename OutT>
-__global__ void __launch_bounds__(kScanThreads) scan_apply_kernel(F f, int64_t n, const uint64_t* tile_offsets, OutT* out)
+// SUMS: `tiles` holds the sums of the tiles as they are, and the first workgroup adds all of them up (tiles[number of tiles] = the
+// grand total); else what comes before each.
+template <bool SUMS, typename F, typename OutT, typename Tell>
+__global__ void __launch_bounds__(kScanThreads) scan_apply_kernel(F f, int64_t n, uint64_t* tiles, OutT* out, Tell tell)
 {
   __shared__ uint64_t lds[kScanThreads / kWave + 1];
   int64_t const base = static_cast<int64_t>(blockIdx.x) * kScanTile + static_cast<int64_t>(threadIdx.x) * kScanItems;
@@ -434,8 +461,27 @@ __global__ void __launch_bounds__(kScanThreads) scan_apply_kernel(F f, int64_t n
     vals[k]         = (i < n) ? static_cast<uint64_t>(f(i)) : 0;
     s += vals[k];
   }
-  uint64_t total;
-  uint64_t run = block_exclusive_scan64<kScanThreads>(s, lds, &total) + tile_offsets[blockIdx.x];
+  uint64_t total, before = 0;
+  if constexpr (SUMS) {
+    uint32_t const mine = blockIdx.x == 0 ? gridDim.x : blockIdx.x;  // (the first workgroup needs none before its own)
+    uint64_t part       = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < kScanDirect / kScanThreads; ++k) {
+      uint32_t const i = k * kScanThreads + threadIdx.x;
+      if (i < mine) part += tiles[i];
+    }
+    block_exclusive_scan64<kScanThreads>(part, lds, &before);
+    if (blockIdx.x == 0) {
+      if (threadIdx.x == 0) {
+        tiles[gridDim.x] = before;
+        tell(before);
+      }
+      before = 0;
+    }
+  } else {
+    before = tiles[blockIdx.x];
+  }
+  uint64_t run = block_exclusive_scan64<kScanThreads>(s, lds, &total) + before;
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k) {
     int64_t const i = base + k;
@@ -445,11 +491,11 @@ __global__ void __launch_bounds__(kScanThreads) scan_apply_kernel(F f, int64_t n
   }
 }
 
-// The whole scan by one workgroup, for the few thousand values of a small call: one launch instead of three.
-// tile_sums[tiles] receives the grand total, as scan_tile_offsets_kernel leaves it.
+// The whole scan by one workgroup, for the few thousand values of a small call: one launch.
+// tile_sums[tiles] receives the grand total, as the others leave it.
 constexpr int64_t kScanSmallTiles = 4;
-template <typename F, typename OutT>
-__global__ void __launch_bounds__(kScanThreads) scan_small_kernel(F f, int64_t n, uint64_t* total_out, OutT* out)
+template <typename F, typename OutT, typename Tell>
+__global__ void __launch_bounds__(kScanThreads) scan_small_kernel(F f, int64_t n, uint64_t* total_out, OutT* out, Tell tell)
 {
   __shared__ uint64_t lds[kScanThreads / kWave + 1];
   uint64_t carry = 0;
@@ -476,6 +522,7 @@ __global__ void __launch_bounds__(kScanThreads) scan_small_kernel(F f, int64_t n
   if (threadIdx.x == 0) {
     out[n]     = static_cast<OutT>(carry);
     *total_out = carry;
+    tell(carry);
   }
 }
 
@@ -484,17 +531,22 @@ inline size_t scan_temp_bytes(int64_t n) { return static_cast<size_t>(scan_tiles
 
 // `temp` holds scan_temp_bytes(n) bytes; temp[ntiles] receives the grand total (uint64).
 // n must be > 0.
-template <typename F, typename OutT>
-void device_exclusive_scan(F f, int64_t n, OutT* out, uint64_t* temp, hipStream_t stream)
+template <typename F, typename OutT, typename Tell>
+void device_exclusive_scan(F f, int64_t n, OutT* out, uint64_t* temp, hipStream_t stream, Tell tell)
 {
   int64_t const tiles = scan_tiles(n);
+  dim3 const grid(static_cast<unsigned>(tiles));
   if (tiles <= kScanSmallTiles) {
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(scan_small_kernel<F, OutT>), dim3(1), dim3(kScanThreads), 0, stream, f, n, temp + tiles, out);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(scan_small_kernel<F, OutT, Tell>), dim3(1), dim3(kScanThreads), 0, stream, f, n, temp + tiles, out, tell);
     return;
   }
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(scan_tile_sums_kernel<F>), dim3(static_cast<unsigned>(tiles)), dim3(kScanThreads), 0, stream, f, n, temp);
-  hipLaunchKernelGGL(scan_tile_offsets_kernel, dim3(1), dim3(kScanThreads), 0, stream, temp, tiles);
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(scan_apply_kernel<F, OutT>), dim3(static_cast<unsigned>(tiles)), dim3(kScanThreads), 0, stream, f, n, temp, out);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(scan_tile_sums_kernel<F>), grid, dim3(kScanThreads), 0, stream, f, n, temp);
+  if (tiles <= kScanDirect) {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(scan_apply_kernel<true, F, OutT, Tell>), grid, dim3(kScanThreads), 0, stream, f, n, temp, out, tell);
+    return;
+  }
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(scan_tile_offsets_kernel<Tell>), dim3(1), dim3(kScanThreads), 0, stream, temp, tiles, tell);
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(scan_apply_kernel<false, F, OutT, TellNobody>), grid, dim3(kScanThreads), 0, stream, f, n, temp, out, TellNobody{});
 }
 
 // Compute units of the current device (read once per device).
@@ -541,8 +593,6 @@ Arrivals* thread_arrivals();
 // After a failure it may hold anything: no thread gets it any more.
 void forsake_thread_arrivals();
 
-// *dst = *src
-void launch_publish(const uint64_t* src, uint64_t* dst, HostPost post, hipStream_t stream);
 // dst[0] = offsets[first_index], dst[1] = offsets[last_index] (offsets of 32 or 64 bits)
 void launch_read_two_offsets(const void* offsets, int is64, int64_t first_index, int64_t last_index, uint64_t* dst, HostPost post,
                              hipStream_t stream);

@@ -1,5 +1,5 @@
 // Host-side plumbing shared by the entry points: status text, allocator adaptor,
-// bitmask copy, fills, the middle stage of the device-wide scan and the small
+// bitmask copy, fills and the small
 // C-ABI utilities (version, last error, result release).
 #include "common.cuh"
 
@@ -109,21 +109,6 @@ void Mr::deallocate(void* p, size_t bytes) const
     return;
   }
   (void)hipFreeAsync(p, stream);
-}
-
-__global__ void __launch_bounds__(kScanThreads) scan_tile_offsets_kernel(uint64_t* tile_sums, int64_t ntiles)
-{
-  __shared__ uint64_t lds[kScanThreads / kWave + 1];
-  uint64_t carry = 0;
-  for (int64_t base = 0; base < ntiles; base += kScanThreads) {
-    int64_t const i  = base + threadIdx.x;
-    uint64_t const v = (i < ntiles) ? tile_sums[i] : 0;
-    uint64_t total;
-    uint64_t const ex = block_exclusive_scan64<kScanThreads>(v, lds, &total);
-    if (i < ntiles) tile_sums[i] = carry + ex;
-    carry += total;
-  }
-  if (threadIdx.x == 0) tile_sums[ntiles] = carry;
 }
 
 namespace {
@@ -288,19 +273,6 @@ hipError_t wait_for_post(HostPost const& post, hipStream_t stream)
     if (e != hipSuccess) return e;
     return sent() ? hipSuccess : hipErrorUnknown;
   }
-}
-
-namespace {
-__global__ void publish_kernel(const uint64_t* __restrict__ src, uint64_t* __restrict__ dst, HostPost post)
-{
-  *dst = *src;
-  post.send();
-}
-}  // namespace
-
-void launch_publish(const uint64_t* src, uint64_t* dst, HostPost post, hipStream_t stream)
-{
-  hipLaunchKernelGGL(publish_kernel, dim3(1), dim3(1), 0, stream, src, dst, post);
 }
 
 void launch_read_two_offsets(const void* offsets, int is64, int64_t first_index, int64_t last_index, uint64_t* dst, HostPost post, hipStream_t stream)

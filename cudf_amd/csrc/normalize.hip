@@ -1502,6 +1502,16 @@ struct TileBytes {
   const uint32_t* counts;
   __device__ uint64_t operator()(int64_t i) const { return counts[i]; }
 };
+// The bytes of the result, for the host.
+struct TellBytes {
+  uint64_t* host;
+  HostPost post;
+  __device__ void operator()(uint64_t total) const
+  {
+    host[0] = total;
+    post.send();
+  }
+};
 
 // ------------------------------------------------------------------ host: tables and tokens
 void append_utf8(std::string& s, uint32_t cp)
@@ -1816,13 +1826,13 @@ nvtext_amd_status nvtext_amd_normalize_characters(const nvtext_amd_strings_colum
     }
     hipLaunchKernelGGL(normalize_tile_rows_kernel, dim3(static_cast<unsigned>((tiles + 255) / 256)), dim3(256), 0, stream, view, first, tiles,
                        tile_row);
-    device_exclusive_scan(TileBytes{tile_bytes}, tiles, tile_offset, temps.part<uint64_t>(2), stream);
     if (scalars) {
       HostPost const post = new_post();
-      launch_publish(tile_offset + tiles, scalars, post, stream);
+      device_exclusive_scan(TileBytes{tile_bytes}, tiles, tile_offset, temps.part<uint64_t>(2), stream, TellBytes{scalars, post});
       e = hipGetLastError();
       if (e == hipSuccess) e = wait_for_post(post, stream);
     } else {
+      device_exclusive_scan(TileBytes{tile_bytes}, tiles, tile_offset, temps.part<uint64_t>(2), stream, TellNobody{});
       e = hipMemcpyAsync(&total, tile_offset + tiles, sizeof(total), hipMemcpyDeviceToHost, stream);
       if (e == hipSuccess) e = hipStreamSynchronize(stream);
     }

@@ -33,8 +33,8 @@
 //     of their own.  No chars-sized temporary is written: 2.4 bytes of temporaries per input byte.
 //   * a large column's first ranges go through the two passes by themselves; their unknown words, with the tokens found,
 //     are a table that the word pass of the other ranges looks into (see kMemoEntries).
-//   * a small column is put on the stream whole before its size is known: one launch that does everything per tile, one
-//     that finds the tiles' places, the emit pass, and one wait (see kSmallRows).
+//   * a small column is put on the stream whole before its size is known: one launch that does everything per tile and
+//     tells the host the number of tokens, the emit pass, and one wait (see kSmallRows).
 #include "common.cuh"
 
 #include <algorithm>
@@ -2261,14 +2261,19 @@ __global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, Vo
 
 // What the host needs to know before the emit pass: the number of tokens, whether a range ran out of word slots, the
 // queue entries that there ought to be.
-__global__ void publish_state_kernel(const uint64_t* __restrict__ total, const uint32_t* __restrict__ flags, QueueChunks chunks,
-                                     uint64_t* __restrict__ dst, HostPost post)
-{
-  dst[0] = *total;
-  dst[1] = flags[kFlagOverflow];
-  dst[2] = chunks.extent();
-  post.send();
-}
+struct TellState {
+  const uint32_t* flags;
+  QueueChunks chunks;
+  uint64_t* dst;
+  HostPost post;
+  __device__ void operator()(uint64_t total) const
+  {
+    dst[0] = total;
+    dst[1] = flags[kFlagOverflow];
+    dst[2] = chunks.extent();
+    post.send();
+  }
+};
 // ... where the host copies the flags.
 __global__ void extent_kernel(uint32_t* __restrict__ flags, QueueChunks chunks) { flags[kFlagExtent] = static_cast<uint32_t>(min(chunks.extent(), uint64_t{0xFFFFFFFFu})); }
 
@@ -3004,13 +3009,12 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     }
     // where the tokens of each range go; the total decides the child size
     // (cpp/include/cudf/detail/sizes_to_offsets_iterator.cuh:302-339)
-    device_exclusive_scan(RangeTokensOf{tokens}, static_cast<int64_t>(nranges), bases, scan_tmp, stream);
-    // the total (the last word of the scan's temporaries) and the first flag words: written to the pinned words by a
-    // kernel of one thread, or, without those, fetched in one copy (the flags lie right behind the scan's temporaries)
+    // the total (the last word of the scan's temporaries) and the first flag words: written to the pinned words as soon as
+    // the total is known, or, without those, fetched in one copy (the flags lie right behind the scan's temporaries)
     uint64_t state[3] = {0, 0, 0};  // (the first flag words: an overflow, the queue's extent)
     if (scalars) {
       HostPost const post = new_post();
-      hipLaunchKernelGGL(publish_state_kernel, dim3(1), dim3(1), 0, stream, scan_tmp + scan_tiles(nranges), flags, chunks, scalars + 2, post);
+      device_exclusive_scan(RangeTokensOf{tokens}, static_cast<int64_t>(nranges), bases, scan_tmp, stream, TellState{flags, chunks, scalars + 2, post});
       hipError_t e = hipGetLastError();
       if (e == hipSuccess) e = wait_for_post(post, stream);
       if (e != hipSuccess) return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
@@ -3019,6 +3023,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
       state[2] = scalars[4];
     } else {
       const char* const from = reinterpret_cast<const char*>(scan_tmp + scan_tiles(nranges));
+      device_exclusive_scan(RangeTokensOf{tokens}, static_cast<int64_t>(nranges), bases, scan_tmp, stream, TellNobody{});
       uint32_t words_of[3]   = {0, 0, 0};
       size_t const span      = static_cast<size_t>(reinterpret_cast<const char*>(flags + 3) - from);
       alignas(8) char both[256 + 8 + sizeof(words_of)];
