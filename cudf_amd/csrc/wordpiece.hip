@@ -26,7 +26,7 @@
 //   * out-of-vocabulary pass: one lane per queued word, lanes refilled from LDS as words finish.  Words of up to
 //     16 bytes are tokenized in registers, the greedy longest-match rule reduced to bit operations on a mask of
 //     candidate lengths, one table lookup per trip; the result (up to seven tokens and their number) takes the
-//     place of the queue record.  Longer words go through a general state machine in a second kernel.
+//     place of the queue record.  Longer words go through a second kernel, sixteen bytes of each in registers.
 //   * a device-wide scan of the ranges' token counts gives every range its place in the result; the emit pass
 //     (a wavefront per range) expands the word slots into the tokens and turns the rows' word counts into list
 //     offsets.  The few words with more pieces than a record keeps are tokenized again, into place, by a kernel
@@ -411,143 +411,9 @@ __device__ __forceinline__ uint32_t space_bytes(uint32_t x)
 __device__ __forceinline__ uint32_t gather_byte_flags(uint32_t z) { return (((z >> 7) * 0x00204081u) >> 21) & 0xFu; }
 
 // ------------------------------------------------------------------ out-of-vocabulary pass
-// Greedy longest-match-first tokenization (cpp/src/text/wordpiece_tokenize.cu:349-407) of a word whose
-// whole-word lookup has already failed, as a resumable state machine: every step() examines up to two
-// candidates (their table reads are in flight together) and the lanes of a wavefront, each somewhere
-// inside its own word, share the trips.  The state is the piece being searched, bytes [start, e): the
-// first piece (start 0) lives in the full key space, later ones in the "##" space.
-template <typename W>
-struct OovStepper {
-  uint32_t len, start, e, count;
-  uint32_t raw0, raw1;  // bytes [start, start+8) of the word
-  uint32_t lens;        // length filter word of the piece that starts at `start` (all ones when it is shorter than 3 bytes)
-  bool ascii;           // no byte of the word has bit 7 set: every position is a character boundary
-  bool fresh;           // [start, e) itself is still untried
-  bool done;
-
-  __device__ __forceinline__ bool inside_character(W const& w, uint32_t x) const { return !ascii && is_utf8_continuation(w.byte(x)); }
-
-  // wordpiece_tokenize.cu:307-317: the end after dropping the last UTF-8 character of [start, x); start if none is left
-  __device__ __forceinline__ uint32_t drop(W const& w, uint32_t x) const
-  {
-    if (x - start < 2) return start;
-    --x;
-    while (x > start && inside_character(w, x)) --x;
-    return x;
-  }
-
-  // The longest candidate end <= x (x on a character boundary, start < x < len or x == len) that the length
-  // filter does not rule out and that ends on a character boundary; start if there is none.  Only lengths
-  // without a key are skipped, so the candidates that can match are visited in the reference's order.
-  __device__ __forceinline__ uint32_t allowed_end(W const& w, uint32_t x) const
-  {
-    uint32_t l = x - start;
-    bool boundary = true;  // start + l is known to be a character boundary
-    while (l >= 3) {
-      if (l >= 34 && (lens >> 31)) break;
-      uint32_t const top = min(l - 3u, 30u);
-      uint32_t const m   = lens & (0xFFFFFFFFu >> (31u - top));
-      if (m == 0) {
-        l        = 2;
-        boundary = false;
-        break;
-      }
-      uint32_t const best = 34u - static_cast<uint32_t>(__builtin_clz(m));  // 3 + index of the highest set bit
-      boundary            = boundary && best == l;
-      l                   = best;
-      if (boundary || !inside_character(w, start + l)) {
-        boundary = true;
-        break;
-      }
-      --l;
-    }
-    if (!boundary)
-      while (l > 0 && inside_character(w, start + l)) --l;
-    return start + l;
-  }
-
-  __device__ __forceinline__ void load_filter(VocabTable const& t, uint32_t kind)
-  {
-    lens = len - start >= 3 ? piece_filter_word(t.lens[length_filter_index(kind, raw0 & 0x00FFFFFFu) & t.lens_mask], raw0) : 0xFFFFFFFFu;
-  }
-
-  // probed: the whole word has been looked up and is known to be absent
-  __device__ __forceinline__ void begin(VocabTable const& t, W const& w, uint32_t len_, bool ascii_, bool probed)
-  {
-    len = len_; start = 0; e = len_; count = 0;
-    ascii = ascii_;
-    fresh = !probed;  // a word known to be absent begins by being shortened
-    done  = false;
-    w.key8(0, min(len, 8u), &raw0, &raw1);
-    load_filter(t, 0);
-  }
-
-  template <typename Emit>
-  __device__ __forceinline__ void step(VocabTable const& t, W const& w, Emit&& emit)
-  {
-    uint32_t const kind = count ? 1u : 0u;
-    uint32_t const maxl = t.max_len[kind];
-    uint32_t ea         = fresh ? e : drop(w, e);
-    if (ea - start > maxl) {
-      // no key is this long: go straight to the longest candidate that can exist (on a character boundary)
-      ea = start + maxl;
-      while (ea > start && inside_character(w, ea)) --ea;
-    }
-    ea = allowed_end(w, ea);
-    if (ea == start) {
-      // no prefix of the word matched (375-379), or a later piece has no match and the word collapses
-      // (396-404): either way a single unknown token
-      emit(0u, t.unk_id);
-      count = 1;
-      done  = true;
-      return;
-    }
-    uint32_t const eb = allowed_end(w, drop(w, ea));
-    bool const has_b  = eb > start;
-    Probe const pa    = make_probe(t, kind, w, start, ea - start, raw0, raw1);
-    Probe const pb    = make_probe(t, kind, w, start, has_b ? eb - start : 1u, raw0, raw1);
-    uint4 const a0 = t.slots[2 * pa.bucket], a1 = t.slots[2 * pa.bucket + 1];
-    uint4 b0 = make_uint4(0, 0, 0, 0), b1 = b0;
-    if (has_b) {
-      b0 = t.slots[2 * pb.bucket];
-      b1 = t.slots[2 * pb.bucket + 1];
-    }
-    uint32_t hit_end = ea;
-    int32_t id       = finish_probe(t, pa, a0, a1, w, start, ea - start);
-    if (id == kNone && has_b) {
-      hit_end = eb;
-      id      = finish_probe(t, pb, b0, b1, w, start, eb - start);
-    }
-    if (id == kNone) {
-      e     = has_b ? eb : ea;
-      fresh = false;
-      return;
-    }
-    emit(count++, id);
-    if (hit_end == len) {
-      done = true;
-      return;
-    }
-    // next piece: the rest of the word (381-395)
-    start = hit_end;
-    e     = len;
-    fresh = true;
-    w.key8(start, min(len - start, 8u), &raw0, &raw1);
-    load_filter(t, 1);
-  }
-};
-
-// Runs one word, which has not been looked up whole, to completion (used where such words are rare).  Returns the
-// token count.
-template <typename W, typename Emit>
-__device__ __forceinline__ uint32_t tokenize_oov_word(VocabTable const& t, W const& w, uint32_t len, Emit emit)
-{
-  OovStepper<W> st;
-  st.begin(t, w, len, false, false);
-  while (!st.done) st.step(t, w, emit);
-  return st.count;
-}
-
+// Greedy longest-match-first tokenization (cpp/src/text/wordpiece_tokenize.cu:349-407) of words whose whole-word lookup has
+// failed, or which have not been looked up whole, as resumable state machines: every step() looks at the longest candidate left, and
+// the lanes of a wavefront, each somewhere inside its own word, share the trips.
 // Bit 7 of every byte of x that is a UTF-8 continuation byte (10xxxxxx); exact, no carries cross bytes.
 __device__ __forceinline__ uint32_t continuation_bytes(uint32_t x)
 {
@@ -706,8 +572,17 @@ struct ShortWord {
   // no lookup several to a trip, also with their openings coming from LDS: fewer trips, each slower by more, and the
   // registers it takes cost wavefronts per SIMD, which this loop needs: 1.03 ms with 8 of them, 1.07 with 6, 1.28 with 4.)
   // (next: the opening of the next piece, once the piece before it has been dropped)
+  // (go_on: what drops a matched piece and opens the next)
   template <typename Next, typename Emit>
   __device__ __forceinline__ void step(VocabTable const& t, const uint4* trim, Next&& next, Emit&& emit)
+  {
+    step_on(t, trim, emit, [&](uint32_t len) {
+      advance(len);  // next piece: the rest of the word (381-395)
+      open_piece(t, 1, next());
+    });
+  }
+  template <typename Emit, typename GoOn>
+  __device__ __forceinline__ void step_on(VocabTable const& t, const uint4* trim, Emit&& emit, GoOn&& go_on)
   {
     uint32_t const kind = count ? 1u : 0u;
     cand &= (lens << 2) | 3u;
@@ -753,12 +628,101 @@ struct ShortWord {
     count = unknown ? 1u : count + (hit ? 1u : 0u);
     done  = unknown || (hit && len == rem);
     cand  = longer_left | (cand & 3u);
-    if (hit && !done) {
-      advance(len);  // next piece: the rest of the word (381-395)
-      open_piece(t, 1, next());
-    }
+    if (hit && !done) go_on(len);
   }
 };
+
+// The same for a word of any length below kMaxWord that lies in LDS: the registers hold the sixteen bytes from the piece
+// being searched on and are filled anew with every piece.  Candidates of more than sixteen bytes, where the length filter
+// leaves any, come first, each with the general lookup.
+// (A state machine that asked LDS for its bytes one by one took the two kernels that go through such words, and words of more
+// tokens than a record keeps, 68 and 66 us of 1,200,001 rows of several scripts, now 47 and 46; 1.5 MB of such text 94 -> 71 us a call.)
+struct WindowWord : ShortWord {
+  TileWord w;       // from the piece being searched on
+  uint32_t longer;  // the longest candidate of more than sixteen bytes still to try (0: none), and the lengths that the filter leaves of those
+  uint32_t filter;
+
+  __device__ __forceinline__ bool boundary(uint32_t l) const { return l == rem || !is_utf8_continuation(w.byte(l)); }
+  // ... of up to l bytes
+  __device__ __forceinline__ uint32_t next_longer(uint32_t l) const
+  {
+    if ((filter >> 14) == 0) return 0;
+    for (; l > 16; --l)
+      if (((l == 17 ? filter >> 14 : filter >> 15) & 1u) != 0 && boundary(l)) return l;
+    return 0;
+  }
+  // The registers for the piece that begins at w.
+  __device__ __forceinline__ void fill(const uint4* trim)
+  {
+    w.head16(r);
+    uint32_t const in = min(rem, 16u);
+    uint4 const keep  = trim[in];
+    r[0] &= keep.x;
+    r[1] &= keep.y;
+    r[2] &= keep.z;
+    r[3] &= keep.w;
+    uint32_t const cont = gather_byte_flags(continuation_bytes(r[0])) | (gather_byte_flags(continuation_bytes(r[1])) << 4) |
+                          (gather_byte_flags(continuation_bytes(r[2])) << 8) | (gather_byte_flags(continuation_bytes(r[3])) << 12);
+    bnd = (~cont & ((1u << in) - 1u)) | (boundary(in) ? 1u << in : 0u);
+  }
+  __device__ __forceinline__ void open(VocabTable const& t, const int32_t* first_ids, uint32_t kind)
+  {
+    open_piece(t, kind, request(t, first_ids, kind, 0));
+    longer = 0;
+    if (rem > 16) {
+      filter = lens;
+      longer = next_longer(min(rem, t.max_len[kind]));
+    }
+  }
+  // probed: the whole word has been looked up and is known to be absent (up to 16 bytes)
+  __device__ __forceinline__ void begin(VocabTable const& t, const uint4* trim, const int32_t* first_ids, TileWord const& word, uint32_t len, bool probed)
+  {
+    w     = word;
+    rem   = len;
+    count = 0;
+    done  = false;
+    fill(trim);
+    open(t, first_ids, 0);
+    if (probed) cand &= ~(1u << (len - 1));
+  }
+  template <typename Emit>
+  __device__ __forceinline__ void step(VocabTable const& t, const uint4* trim, const int32_t* first_ids, Emit&& emit)
+  {
+    auto const go_on = [&](uint32_t len) {
+      if (rem > 16) {
+        w.start += len;
+        rem -= len;
+        fill(trim);
+      } else {
+        advance(len);  // (all that is left is in the registers; w is not looked at any more)
+      }
+      open(t, first_ids, 1);
+    };
+    if (longer != 0) {
+      int32_t const id = lookup_slow(t, count ? 1u : 0u, w, 0u, longer);
+      if (id == kNone) {
+        longer = next_longer(longer - 1u);
+        return;
+      }
+      emit(count++, id);
+      done = longer == rem;
+      if (!done) go_on(longer);
+      return;
+    }
+    step_on(t, trim, emit, go_on);
+  }
+};
+
+// Runs one word, which has not been looked up whole, to completion.  Returns the token count.
+template <typename Emit>
+__device__ __forceinline__ uint32_t tokenize_window_word(VocabTable const& t, const uint4* trim, TileWord const& w, uint32_t len, Emit emit)
+{
+  const int32_t* const first_ids = t.short_ids + 2 * 65536;
+  WindowWord word;
+  word.begin(t, trim, first_ids, w, len, false);
+  while (!word.done) word.step(t, trim, first_ids, emit);
+  return word.count;
+}
 
 // ------------------------------------------------------------------ the passes
 // The column's bytes, from the 16-byte aligned address at or below its first byte, are cut into tiles of TILE
@@ -1588,7 +1552,7 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
                 while (!sw.done) sw.step(table, trim, [&] { return sw.request(table, first_ids, 1u, 0u); }, keep_token);
                 count = sw.count;
               } else {
-                count = tokenize_oov_word(table, tw, wl, keep_token);
+                count = tokenize_window_word(table, trim, tw, wl, keep_token);
               }
               oov_tokens += count;
               if (count > kOovKeep) again = true;
@@ -1669,7 +1633,7 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
 // takes a chunk of the queue at a time (one atomic), brings them into LDS 64 at a time with whole-record reads (the
 // next 64 are requested while these are worked on) and lets its idle lanes take entries from there every trip.  Words
 // of up to 16 bytes, whole in their queue record, run in registers; the few longer ones are set aside and done, one
-// lane each, by the general state machine over the chars in memory, 64 and more at a time or at the end.
+// lane each, by the kernel after it.
 constexpr int kRefillAt      = 32;
 constexpr int kOovWaves      = 16;  // (two workgroups to a CU, 73 KB of LDS each, 8 wavefronts per SIMD)
 constexpr int kOovThreads    = kOovWaves * kWave;
@@ -1858,8 +1822,8 @@ __global__ void __launch_bounds__(kOovThreads, 8) wordpiece_oov_kernel(VocabTabl
   add_together(acc_count != 0);
 }
 
-// A word of up to kMaxWord bytes, copied into the lane's row of LDS: the general state machine asks for bytes and keys one
-// after the other, and out of memory each of them was a wait (words of 17 bytes and more of 1.2 M rows of mixed scripts:
+// A word of up to kMaxWord bytes, copied into the lane's row of LDS: it is asked for window by window, and out of memory
+// each of these was a wait (words of 17 bytes and more of 1.2 M rows of mixed scripts:
 // 82 us in the first of the two kernels below, 70 us from LDS).
 struct RareWords {
   static constexpr uint32_t kRow = kMaxWord / 4 + 5;  // + misalignment, + what a key read touches past the word; odd
@@ -1879,14 +1843,17 @@ struct RareWords {
 };
 static_assert(RareWords::kRow % 2 == 1, "the rows begin in different banks");
 
-// The queued words of more than 16 bytes, which the kernel above has listed: one lane per word, the general state machine.
+// The queued words of more than 16 bytes, which the kernel above has listed: one lane per word (see WindowWord).
 __global__ void __launch_bounds__(kRareThreads) wordpiece_oov_long_kernel(VocabTable table, const uint4* abase, OovEntry* __restrict__ queue,
                                                                          QueueChunks chunks, uint32_t queue_cap,
                                                                          const uint32_t* __restrict__ longer, const uint32_t* __restrict__ longer_count,
                                                                          uint32_t* __restrict__ range_tokens)
 {
   __shared__ RareWords words;
+  __shared__ uint4 trim[17];
   if (chunks.extent() > queue_cap) return;  // (see wordpiece_oov_kernel)
+  fill_trim_table(trim);
+  __syncthreads();
   uint32_t const n = *longer_count;
   for (uint32_t i = blockIdx.x * kRareThreads + threadIdx.x; i < n; i += gridDim.x * kRareThreads) {
     uint32_t const q   = longer[i];
@@ -1894,7 +1861,7 @@ __global__ void __launch_bounds__(kRareThreads) wordpiece_oov_long_kernel(VocabT
     uint32_t const wl  = e.len_flags & 0xFFu;
     int64_t const at   = static_cast<int64_t>((static_cast<uint64_t>(e.coord[1]) << 32) | e.coord[0]);
     int32_t tok[kOovKeep];
-    uint32_t const cnt = tokenize_oov_word(table, words.copy(abase, at, wl), wl, [&](uint32_t j, int32_t id) {
+    uint32_t const cnt = tokenize_window_word(table, trim, words.copy(abase, at, wl), wl, [&](uint32_t j, int32_t id) {
 #pragma unroll
       for (int k = 0; k < kOovKeep; ++k)
         if (j == static_cast<uint32_t>(k)) tok[k] = id;
@@ -2167,13 +2134,16 @@ __global__ void __launch_bounds__(kRareThreads) wordpiece_retokenize_kernel(Voca
                                                                            int32_t* __restrict__ child)
 {
   __shared__ RareWords words;
+  __shared__ uint4 trim[17];
+  fill_trim_table(trim);
+  __syncthreads();
   uint32_t const n = *again_count;
   for (uint32_t i = blockIdx.x * kRareThreads + threadIdx.x; i < n; i += gridDim.x * kRareThreads) {
     OovEntry const e   = queue[again[i]];  // head[0] = place in the child, head[3] = coord[1], len_flags, range, coord[0] as they were; coord[1] = the count
     uint32_t const cnt = e.coord[1];
     int64_t const at   = static_cast<int64_t>((static_cast<uint64_t>(e.head[3]) << 32) | e.coord[0]);
     int32_t* const d   = child + e.head[0];
-    tokenize_oov_word(table, words.copy(abase, at, e.len_flags & 0xFFu), e.len_flags & 0xFFu, [&](uint32_t j, int32_t id) {
+    tokenize_window_word(table, trim, words.copy(abase, at, e.len_flags & 0xFFu), e.len_flags & 0xFFu, [&](uint32_t j, int32_t id) {
       if (j < cnt) d[j] = id;
     });
   }

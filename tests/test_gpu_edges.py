@@ -430,6 +430,37 @@ def test_tokenize_chunks_of_the_queue(nv, orc, rows, oov):
     assert nv.wordpiece_tokenize(dev(nv, host), vocabulary, 0).to_host().equals(orc.wordpiece_tokenize(host, reference, 0, nthreads=8))
 
 
+@pytest.mark.parametrize("letters", ["ab", "aé", "漢字b", "a\U0001F600"])
+@pytest.mark.parametrize("rows", [900, 140_000])
+def test_tokenize_words_longer_than_a_window(nv, orc, letters, rows):
+    """Words of up to 199 bytes made of pieces of 1 to 60 bytes, some known, some one character off: candidates of 15 to 18 bytes
+    and of many more at the beginning of a word and behind other pieces, characters across the sixteenth byte, words of 7, 8,
+    14, 15 and more tokens; in a small column and in a large one."""
+    rng = np.random.default_rng(rows + len(letters))
+    def piece(nbytes):
+        out = ""
+        while len(out.encode()) < nbytes:
+            out += letters[int(rng.integers(0, len(letters)))]
+        return out
+    sizes = [1, 2, 3, 4, 5, 13, 14, 15, 16, 17, 18, 19, 20, 31, 33, 34, 35, 60]
+    keys = sorted({piece(n) for n in sizes for _ in range(4)})
+    vocab = ["[UNK]"] + [k for i, k in enumerate(keys) if i % 3 != 1] + ["##" + k for i, k in enumerate(keys) if i % 3 != 2]
+    vocab += [w for w in (c for c in letters[:1]) if w not in vocab] + ["##" + c for c in letters if "##" + c not in vocab]
+    words = []
+    for _ in range(1500):
+        parts = [keys[int(rng.integers(0, len(keys)))] for _ in range(int(rng.integers(1, 9)))]
+        if rng.random() < 0.3:
+            parts = [letters[int(rng.integers(0, len(letters)))] for _ in range(int(rng.choice([6, 7, 8, 13, 14, 15, 16, 30])))]
+        if rng.random() < 0.2:
+            parts.insert(int(rng.integers(0, len(parts) + 1)), "z")
+        words.append("".join(parts)[:199])
+    hv = HostStringsColumn.from_pylist(vocab)
+    vocabulary, reference = nv.WordPieceVocabulary(dev(nv, hv)), orc.Vocabulary(hv)
+    texts = [" ".join(words[int(i)] for i in rng.integers(0, len(words), 3)) for _ in range(900)]
+    host = HostStringsColumn.from_pylist([texts[i % 900] for i in range(rows)])
+    assert nv.wordpiece_tokenize(dev(nv, host), vocabulary, 0).to_host().equals(orc.wordpiece_tokenize(host, reference, 0, nthreads=8))
+
+
 def test_tokenize_from_threads_that_come_and_go(nv, orc):
     """Forty host threads, eight at a time, tokenize small columns of different sizes: what a call adds up on the device is its thread's own,
     and is there again for the threads that follow."""
