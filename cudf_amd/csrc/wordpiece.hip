@@ -1017,6 +1017,7 @@ constexpr uint32_t kSmallLeastSlots = kSmallTile / 4 + 8;  // (six bytes to a wo
 constexpr uint32_t kSmallQueue      = kSmallTile / 8;      // words of a tile that are not in the vocabulary (one in 37 bytes on the benchmark's rows)
 constexpr uint32_t kSmallLeastQueue = kSmallTile / 16;
 constexpr unsigned kSmallGrid       = 512;                 // workgroups at most (two to a CU): a wavefront then takes several tiles
+constexpr uint32_t kSmallSpread     = 256;                 // workgroups that have less than a tile for every wavefront
 // What every one of `tiles` tiles gets of the slots and of the queue's records (an even number of slots).
 __host__ __device__ inline uint32_t small_slots(uint32_t slots, uint32_t tiles)
 {
@@ -1042,11 +1043,13 @@ __device__ __forceinline__ void tell_host(TileArgs const& a, int64_t first_offse
 }
 
 // The tiles are shared out in blocks of neighbours, a workgroup's wavefronts taking theirs one after the other: how many
-// tiles a block has where `grid` workgroups were launched.
+// tiles a block has where `grid` workgroups were launched.  Few tiles go to as many CUs, where their wavefronts share nothing.
 __host__ __device__ inline uint32_t small_block(uint32_t tiles, uint32_t grid)
 {
-  uint32_t const each = (tiles + grid - 1) / grid;
-  return each > static_cast<uint32_t>(word_waves(true)) ? each : static_cast<uint32_t>(word_waves(true));
+  uint32_t const waves = static_cast<uint32_t>(word_waves(true));
+  uint32_t const each  = (tiles + kSmallSpread - 1) / kSmallSpread, least = (tiles + grid - 1) / grid;
+  uint32_t const block = each < waves ? each : waves;
+  return block > least ? block : least;
 }
 
 // One tile at a time per wavefront: stage its bytes (and the 256 after it) in LDS; mark the row starts in it; find
@@ -2726,7 +2729,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     args.host          = scalars;
     args.post          = new_post();
     uint32_t* const again_count = args.again_count;
-    unsigned const grid         = std::min((most_ranges + word_waves(true) - 1) / word_waves(true), kSmallGrid);
+    unsigned const grid         = std::min(most_ranges, kSmallGrid);
     void (*const kernel)(TileArgs) = is64 ? (limit ? wordpiece_word_kernel<kSmallTile, true, true, true> : wordpiece_word_kernel<kSmallTile, true, false, true>)
                                           : (limit ? wordpiece_word_kernel<kSmallTile, false, true, true> : wordpiece_word_kernel<kSmallTile, false, false, true>);
     {
