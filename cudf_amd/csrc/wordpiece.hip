@@ -839,7 +839,7 @@ struct TileArgs {
   const uint32_t* hot;     // slots of words that the sample found, kHotWords of them (nullptr: none)
   int64_t most_bytes;
   uint32_t* first_row_out; // as range_first_row
-  uint64_t* block_tokens;  // tokens of each workgroup's ranges
+  uint32_t* block_tokens;  // tokens of each workgroup's ranges
   uint32_t* again_count;   // words of more tokens than a queue record keeps (the emit pass counts them)
   Arrivals* arrivals;      // what the workgroups have added up between them, and where the last of them leaves it for the host
   uint64_t* host;
@@ -1964,12 +1964,12 @@ __global__ void __launch_bounds__(kMemoThreads) wordpiece_memo_fill_kernel(const
 // side in LDS first and written 64 at a time, the same tokens take a third of the instructions (0.69 -> 0.55 ms on
 // 3.2 GB of text with one word in seven from the queue).
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-// SMALL (after the launch for a small column): where a range's tokens go is added up here, by its wavefront, from the
-// tokens of the blocks of `block` ranges before its own and of the ranges before it in that.
+// SMALL (after the launch for a small column, a range a wavefront): where a range's tokens go is added up here, from the
+// tokens of the blocks of `block` ranges before the workgroup's first, and of the ranges from there on.
 template <bool SMALL>
 __global__ void __launch_bounds__(kTokThreads, 8) wordpiece_emit_kernel(uint32_t nranges, const uint32_t* __restrict__ arena, uint32_t range_cap,
                                                                      const uint32_t* __restrict__ range_words, const int64_t* __restrict__ range_base,
-                                                                     const uint64_t* __restrict__ block_tokens,
+                                                                     const uint32_t* __restrict__ block_tokens,
                                                                      const uint32_t* __restrict__ range_tokens, uint32_t block,
                                                                      const uint32_t* __restrict__ range_first_row, OovEntry* __restrict__ queue,
                                                                      int32_t* __restrict__ offsets, int32_t* __restrict__ child,
@@ -1981,6 +1981,24 @@ __global__ void __launch_bounds__(kTokThreads, 8) wordpiece_emit_kernel(uint32_t
   uint32_t* const stage     = stage_all[threadIdx.x / kWave];
   int const lane            = lane_id();
   uint32_t const my_number  = blockIdx.x * kTokWaves + threadIdx.x / kWave;
+  // SMALL: the workgroup's ranges begin in this block, its tokens there (32 bits: a small column has no more tokens than bytes)
+  uint32_t first_block = 0, first_place = 0;
+  if constexpr (SMALL) {
+    __shared__ uint32_t sums[kTokWaves];
+    first_block   = blockIdx.x * kTokWaves / block;
+    uint32_t part = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < (kSmallGrid + kTokThreads - 1) / kTokThreads; ++k) {
+      uint32_t const i = k * kTokThreads + threadIdx.x;
+      if (i < first_block) part += block_tokens[i];
+    }
+    part = wave_inclusive_scan(part);
+    if (lane == kWave - 1) sums[threadIdx.x / kWave] = part;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kTokWaves; ++w) first_place += sums[w];
+    first_place = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(first_place)));
+  }
   // The ranges cost this pass about the same, so every wavefront takes every W-th one (W wavefronts in the grid):
   // faster here than taking them from a counter as they go, as the other two passes do (0.71 against 0.77 ms on
   // 3.2 GB of text, 0.21 against 0.26 ms on two million short rows).
@@ -1992,11 +2010,9 @@ __global__ void __launch_bounds__(kTokThreads, 8) wordpiece_emit_kernel(uint32_t
     uint32_t const nwords       = range_words[range];
     int64_t base;
     if constexpr (SMALL) {
-      uint32_t const mine = range / block;
-      uint64_t before     = 0;
-      for (uint32_t i = lane; i < mine; i += kWave) before += block_tokens[i];
-      for (uint32_t i = mine * block + lane; i < range; i += kWave) before += range_tokens[i];
-      base = static_cast<int64_t>(wave_bcast64(wave_inclusive_scan64(before), kWave - 1));
+      uint32_t before = 0;
+      for (uint32_t i = first_block * block + lane; i < range; i += kWave) before += range_tokens[i];
+      base = static_cast<int64_t>(first_place + wave_bcast(wave_inclusive_scan(before), kWave - 1));
     } else {
       base = range_base[range];
     }
@@ -2705,7 +2721,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
                                    (static_cast<size_t>(most_ranges) + 1) * sizeof(uint32_t),
                                    static_cast<size_t>(most_ranges) * sizeof(uint32_t),
                                    static_cast<size_t>(most_ranges) * sizeof(uint32_t),
-                                   kSmallGrid * sizeof(uint64_t),
+                                   kSmallGrid * sizeof(uint32_t),
                                    (static_cast<size_t>(records) + 1) * sizeof(uint32_t),
                                    static_cast<size_t>(records) * sizeof(OovEntry)};
     TempParts<7> const temps(mr, temp_bytes);
@@ -2719,7 +2735,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     args.first_row_out = temps.part<uint32_t>(1);
     args.range_words   = temps.part<uint32_t>(2);
     args.range_tokens  = temps.part<uint32_t>(3);
-    args.block_tokens  = temps.part<uint64_t>(4);
+    args.block_tokens  = temps.part<uint32_t>(4);
     args.again_count   = temps.part<uint32_t>(5);
     args.offsets_out   = out->offsets;
     args.queue         = temps.part<OovEntry>(6);
@@ -3029,7 +3045,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     {
       ProfileScope ps("wordpiece_emit_kernel", stream);
       hipLaunchKernelGGL(HIP_KERNEL_NAME(wordpiece_emit_kernel<false>), dim3(emit_grid), dim3(kTokThreads), 0, stream, nranges, arena, range_cap, words, bases,
-                         static_cast<const uint64_t*>(nullptr), static_cast<const uint32_t*>(nullptr), 1u, first_row, queue,
+                         static_cast<const uint32_t*>(nullptr), static_cast<const uint32_t*>(nullptr), 1u, first_row, queue,
                          out->offsets, static_cast<int32_t*>(out->child), longer, flags + kFlagAgain);
       // (the list of longer words has served its purpose by now: its memory takes the list of words to do again, at most
       // one entry per queued word)
