@@ -176,6 +176,9 @@ constexpr int kTokThreads   = kTokWaves * kWave;
 constexpr int word_waves(bool small) { return small ? 8 : 12; }
 constexpr int32_t kNone     = std::numeric_limits<int32_t>::min();
 constexpr int kOovKeep      = 7;     // tokens of an out-of-vocabulary word that are kept while it is tokenized
+// ... in the launch for a small column, which gives a word of more than seven a second record (1.5 MB of text of several scripts in
+// rows of 500 bytes 70.7 -> 54.2 us, 10 MB 148 -> 118, without the launch that tokenizes such words again; of ASCII 84.8 -> 85.5)
+constexpr int kOovMore      = 14;
 // ------------------------------------------------------------------ where candidate keys live
 // Each source offers byte(k) and key8(p, len, &k0, &k1): bytes [p, p+8) as two dwords, zero padded past len.
 __device__ __forceinline__ void trim_key8(uint32_t len, uint32_t& lo, uint32_t& hi)
@@ -740,6 +743,8 @@ std::atomic<int> g_forced_range_tiles{0};
 std::atomic<int> g_sizing_sample{1};
 constexpr int kRangeTiles    = 8;     // tiles per range at most (a large column); a small column has fewer, so that every wavefront gets several ranges
 constexpr int kOverBlocks    = 16;   // 16-byte blocks staged past the tile: a word that starts in the tile ends in them, or is kMaxWord bytes or more
+// In the launch for a small column a word of 8 to kOovMore tokens has two records: tok[6] of the first says which the second is, whose
+// eight words are tokens 6, 7, ..
 // Queue entries that a wavefront of the word pass reserves at a time, in a large column and at least.  What a wavefront has
 // left in the end are records that the out-of-vocabulary pass reads to find nothing in them: where six thousand wavefronts
 // meet a few hundred unknown words each, chunks of 512 were mostly such (with the counters of QueueChunks, 128,000 rows of 500 bytes
@@ -1096,6 +1101,7 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
   __shared__ uint4 trim[17];
   __shared__ uint4 hot[INLINE ? 1 : kHotWords];  // the key (at most 8 bytes), its id, its length
   __shared__ uint32_t small_next, small_tokens, small_notes;  // INLINE: the next tile of the block; what its tiles have
+  __shared__ int32_t more_tokens[INLINE ? kWaves : 1][kOovMore - kOovKeep][INLINE ? kWave : 1];  // those that a lane's registers do not keep
   fill_trim_table(trim);
   if constexpr (INLINE) {
     if (threadIdx.x == 0) {
@@ -1531,6 +1537,7 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
             }
           }
           uint32_t const place = lanes_below(qm);
+          uint32_t seconds     = 0;  // INLINE: second records
           uint32_t const q     = place < room ? q_pos + place : fresh + (place - room);
           if (queued) value = kOovMark | q;
           if (c < listed && !spill) region[cursor + (entry >> 21)] = value;
@@ -1542,6 +1549,7 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
 #pragma unroll
                 for (int i = 0; i < kOovKeep; ++i)
                   if (j == static_cast<uint32_t>(i)) tok[i] = id;
+                if (j >= kOovKeep && j < kOovMore) more_tokens[threadIdx.x / kWave][j - kOovKeep][lane] = id;
               };
               uint32_t count;
               if (wl <= 16) {
@@ -1558,10 +1566,24 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
                 count = tokenize_window_word(table, trim, tw, wl, keep_token);
               }
               oov_tokens += count;
-              if (count > kOovKeep) again = true;
+              // (second records lie behind the round's first ones)
+              bool const two        = count > kOovKeep && count <= kOovMore;
+              uint64_t const twos   = ballot64(two);
+              uint32_t const second = nq + lanes_below(twos);
+              seconds               = static_cast<uint32_t>(__builtin_popcountll(twos));
+              if (count > kOovMore) again = true;
               if (place < room) {
                 uint4* const dst = reinterpret_cast<uint4*>(a.queue + q);
-                if (count <= kOovKeep) {
+                if (two) {
+                  auto const more = [&](int k) { return static_cast<uint32_t>(more_tokens[threadIdx.x / kWave][k][lane]); };
+                  dst[0] = make_uint4(static_cast<uint32_t>(tok[0]), static_cast<uint32_t>(tok[1]), static_cast<uint32_t>(tok[2]), static_cast<uint32_t>(tok[3]));
+                  dst[1] = make_uint4(static_cast<uint32_t>(tok[4]), static_cast<uint32_t>(tok[5]), q_pos + second, count);
+                  if (second < room) {
+                    uint4* const behind = reinterpret_cast<uint4*>(a.queue + q_pos + second);
+                    behind[0] = make_uint4(static_cast<uint32_t>(tok[6]), more(0), more(1), more(2));
+                    behind[1] = make_uint4(more(3), more(4), more(5), more(6));
+                  }
+                } else if (count <= kOovKeep) {
                   dst[0] = make_uint4(static_cast<uint32_t>(tok[0]), static_cast<uint32_t>(tok[1]), static_cast<uint32_t>(tok[2]), static_cast<uint32_t>(tok[3]));
                   dst[1] = make_uint4(static_cast<uint32_t>(tok[4]), static_cast<uint32_t>(tok[5]), static_cast<uint32_t>(tok[6]), count);
                 } else {  // (as the out-of-vocabulary pass leaves it)
@@ -1576,8 +1598,13 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
                                                static_cast<uint32_t>(static_cast<uint64_t>(at) >> 32)));
             }
           }
+          if constexpr (INLINE) {
+            // (any lane that had a word knows their number)
+            if (nq != 0) seconds = wave_bcast(seconds, __builtin_ctzll(qm));
+            if (nq + seconds > room) spill = true;
+          }
           if (INLINE || nq <= room) {
-            q_pos += min(nq, room);
+            q_pos += min(nq + seconds, room);
           } else {
             q_pos = fresh + (nq - room);
             q_lim = fresh + (1u << a.queue_shift);
@@ -1966,8 +1993,10 @@ __global__ void __launch_bounds__(kMemoThreads) wordpiece_memo_fill_kernel(const
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 // SMALL (after the launch for a small column, a range a wavefront): where a range's tokens go is added up here, from the
 // tokens of the blocks of `block` ranges before the workgroup's first, and of the ranges from there on.
+// (Six wavefronts per SIMD: with seven two registers are spilled and 10 MB in rows of 500 bytes take 14.1 instead of 13.1 us, with
+// eight sixteen and 21.7: wavefronts that live for one range pay for their scratch memory.)
 template <bool SMALL>
-__global__ void __launch_bounds__(kTokThreads, 8) wordpiece_emit_kernel(uint32_t nranges, const uint32_t* __restrict__ arena, uint32_t range_cap,
+__global__ void __launch_bounds__(kTokThreads, SMALL ? 6 : 8) wordpiece_emit_kernel(uint32_t nranges, const uint32_t* __restrict__ arena, uint32_t range_cap,
                                                                      const uint32_t* __restrict__ range_words, const int64_t* __restrict__ range_base,
                                                                      const uint32_t* __restrict__ block_tokens,
                                                                      const uint32_t* __restrict__ range_tokens, uint32_t block,
@@ -1976,6 +2005,7 @@ __global__ void __launch_bounds__(kTokThreads, 8) wordpiece_emit_kernel(uint32_t
                                                                      uint32_t* __restrict__ again, uint32_t* __restrict__ again_count)
 {
   constexpr uint32_t kRound = 2 * kWave;
+  constexpr uint32_t kMost  = SMALL ? kOovMore : kOovKeep;  // tokens of a word that its records keep
   constexpr uint32_t kStage = 768;  // tokens of a round that are put in order in LDS before they are written
   __shared__ uint32_t stage_all[kTokWaves][kStage];
   uint32_t* const stage     = stage_all[threadIdx.x / kWave];
@@ -2057,6 +2087,28 @@ __global__ void __launch_bounds__(kTokThreads, 8) wordpiece_emit_kernel(uint32_t
       uint32_t const ex   = incl - (c0 + c1);  // tokens of the round before my first word
       uint32_t const tot  = wave_bcast(incl, kWave - 1);
       int32_t* const dst  = dst0 + done + ex;
+      // SMALL: tokens 6, 7, .. of words with two records (seldom; what the first says instead of token 6 may have been staged: it is overwritten)
+      auto const second_records = [&](auto const& put) {
+        if constexpr (SMALL) {
+          auto const of_word = [&](bool queued, uint32_t cnt, uint32_t record, uint32_t at) {
+            bool const two = queued && cnt > kOovKeep && cnt <= kOovMore;
+            if (ballot64(two) == 0) return;
+            if (two) {
+              const uint4* const behind = reinterpret_cast<const uint4*>(queue + record);
+#pragma unroll 1
+              for (uint32_t k = 6; k < cnt; k += 4) {
+                uint4 const c = behind[(k - 6) / 4];
+                put(at, k, c.x);
+                if (k + 1 < cnt) put(at, k + 1, c.y);
+                if (k + 2 < cnt) put(at, k + 2, c.z);
+                if (k + 3 < cnt) put(at, k + 3, c.w);
+              }
+            }
+          };
+          of_word(q0, c0, rb0.z, ex);
+          of_word(q1, c1, rb1.z, ex + c0);
+        }
+      };
       if (ballot64(q0 || q1) == 0) {
         // no word of the round comes from the queue: a token each, the pair side by side
         if (act1) {
@@ -2068,7 +2120,7 @@ __global__ void __launch_bounds__(kTokThreads, 8) wordpiece_emit_kernel(uint32_t
       } else if (tot <= kStage) {
         // the tokens of the round side by side in LDS, then written 64 at a time
         auto stage_word = [&](bool active, bool queued, uint32_t slot, uint32_t cnt, uint4 const& ra, uint4 const& rb, uint32_t at) {
-          if (queued && cnt > kOovKeep) {
+          if (queued && cnt > kMost) {
             // more tokens than a record keeps (seldom): noted for wordpiece_retokenize_kernel, with the place of the
             // word's first token in the child left in its record (what is written there now is overwritten then)
             uint32_t const q                  = slot & ~kOovMark;
@@ -2091,12 +2143,13 @@ __global__ void __launch_bounds__(kTokThreads, 8) wordpiece_emit_kernel(uint32_t
         wave_lds_sync();  // (the writes of the round before have read their tokens)
         stage_word(act0, q0, v.x, c0, ra0, rb0, ex);
         stage_word(act1, q1, v.y, c1, ra1, rb1, ex + c0);
+        second_records([&](uint32_t at, uint32_t k, uint32_t id) { stage[at + k] = id; });
         wave_lds_sync();
         int32_t* const out = dst0 + done;
         for (uint32_t i = lane; i < tot; i += kWave) out[i] = static_cast<int32_t>(stage[i]);
       } else {
         auto write_word = [&](bool active, bool queued, uint32_t slot, uint32_t cnt, uint4 const& ra, uint4 const& rb, int32_t* d) {
-          if (queued && cnt > kOovKeep) {
+          if (queued && cnt > kMost) {
             // more tokens than a record keeps (seldom): noted for wordpiece_retokenize_kernel, with the place of the
             // word's first token in the child left in its record
             uint32_t const q                  = slot & ~kOovMark;
@@ -2111,13 +2164,14 @@ __global__ void __launch_bounds__(kTokThreads, 8) wordpiece_emit_kernel(uint32_t
                 if (queued && cnt > 3u) d[3] = static_cast<int32_t>(ra.w);
                 if (queued && cnt > 4u) d[4] = static_cast<int32_t>(rb.x);
                 if (queued && cnt > 5u) d[5] = static_cast<int32_t>(rb.y);
-                if (queued && cnt > 6u) d[6] = static_cast<int32_t>(rb.z);
+                if (queued && cnt == 7u) d[6] = static_cast<int32_t>(rb.z);
               }
             }
           }
         };
         write_word(act0, q0, v.x, c0, ra0, rb0, dst);
         write_word(act1, q1, v.y, c1, ra1, rb1, dst + c0);
+        second_records([&](uint32_t at, uint32_t k, uint32_t id) { dst0[done + at + k] = static_cast<int32_t>(id); });
       }
       // rows that begin at one of these words (or, in the last round, after the last word: the positions past it
       // hold the round's total)
