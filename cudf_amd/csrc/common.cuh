@@ -587,6 +587,7 @@ hipError_t wait_for_post(HostPost const& post, hipStream_t stream);
 struct alignas(128) Arrivals {
   unsigned long long sum;
   uint32_t notes;
+  alignas(128) uint32_t words[16];  // counters of the launch's own
 };
 constexpr int kMostArrivals = 1024;
 Arrivals* thread_arrivals();

@@ -503,13 +503,22 @@ __device__ __forceinline__ bool count_pair(ColView const& c1, ColView const& c2,
 constexpr uint32_t kOnceMore = 0x80000000u;  // (rows are fewer)
 
 // Work lists in `work`: a header of 16 words -- [i] = pairs on list i, [kLists] = null rows of the result,
-// [8..9] = the most bytes a pair of the global list has (64 bits) -- then four counters (|A|, |B|, |A n B|, parts done) for
-// every entry of the list of pairs in parts, and `rows` entries for each list.
+// [8..9] = the most bytes a pair of the global list has (64 bits), [kTotalParts] = parts of all pairs on the list of pairs in parts,
+// [kNextPiece] = pieces of work handed out
+// -- then four counters (|A|, |B|, |A n B|, parts done) for
+// every entry of the list of pairs in parts, and `rows` entries for each list; in a column of up to kLookRows pairs behind these a
+// list of the parts themselves (a pair's entry | its number << 16).
 constexpr int kListHeader = 16;
+constexpr int kTotalParts = 10;
+constexpr int kNextPiece  = 11;
 constexpr int32_t kLookRows = 32768;  // see nvtext_amd_jaccard_index
-__host__ __device__ __forceinline__ size_t work_words(int64_t rows) { return kListHeader + static_cast<size_t>(kLists + 4) * static_cast<size_t>(rows); }
+__host__ __device__ __forceinline__ size_t work_words(int64_t rows)
+{
+  return kListHeader + static_cast<size_t>(kLists + 4 + (rows <= kLookRows ? kMaxParts : 0)) * static_cast<size_t>(rows);
+}
 __device__ __forceinline__ uint32_t* list_entries(uint32_t* work, int list, int64_t rows) { return work + kListHeader + (4 + list) * rows; }
 __device__ __forceinline__ uint32_t* part_counters(uint32_t* work) { return work + kListHeader; }
+__device__ __forceinline__ uint32_t* single_parts(uint32_t* work, int64_t rows) { return work + kListHeader + (kLists + 4) * rows; }
 __device__ __forceinline__ void list_for_global(uint32_t* work, int64_t rows, int64_t r, int64_t bytes)
 {
   list_entries(work, kGlobalList, rows)[atomicAdd(&work[kGlobalList], 1u)] = static_cast<uint32_t>(r);
@@ -526,8 +535,15 @@ static_assert(kSlots[0] == PackedSet::kLeast, "every pair of a wavefront takes a
 // lists those that need more than a wavefront's own set for the later kernels with one atomic per list (atomics on one
 // cache line run at about 150 M/s: one per wavefront and list was most of this kernel's time), and its wavefronts do the
 // others, each taking the next one when it is done with one.  A column of few pairs is shared out over more workgroups.
+// told.arrivals (a column of up to kLookRows pairs, a workgroup for every group): the lists are counted there, and the workgroup that
+// is last to have listed its pairs tells the host the header, while all still have their own pairs to do.
+struct Told {
+  Arrivals* arrivals;
+  uint32_t* host;
+  HostPost post;
+};
 __global__ void __launch_bounds__(kThreads) jaccard_wave_kernel(ColView c1, ColView c2, int32_t width, float* __restrict__ out,
-                                                                uint32_t* __restrict__ work, int per_group)
+                                                                uint32_t* __restrict__ work, int per_group, Told told)
 {
   __shared__ WaveSetLds lds_all[kWaves];
   __shared__ uint32_t listed[kLists], place[kLists], solo[kThreads], solos, next;
@@ -535,6 +551,7 @@ __global__ void __launch_bounds__(kThreads) jaccard_wave_kernel(ColView c1, ColV
   int const wave     = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
   WaveSetLds& lds    = lds_all[wave];
   int64_t const rows = c1.size;
+  uint32_t* const counts = told.arrivals ? told.arrivals->words : work;
   auto wave_sync = [] {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -554,13 +571,40 @@ __global__ void __launch_bounds__(kThreads) jaccard_wave_kernel(ColView c1, ColV
     if (have && !later) solo[atomicAdd(&solos, 1u)] = static_cast<uint32_t>(r);
     if (later) at = atomicAdd(&listed[list], 1u);
     __syncthreads();
-    if (threadIdx.x < kLists && listed[threadIdx.x] != 0u) place[threadIdx.x] = atomicAdd(&work[threadIdx.x], listed[threadIdx.x]);
+    if (threadIdx.x < kLists && listed[threadIdx.x] != 0u) place[threadIdx.x] = atomicAdd(&counts[threadIdx.x], listed[threadIdx.x]);
     __syncthreads();
     if (later) {
       at += place[list];
       list_entries(work, list, rows)[at] = static_cast<uint32_t>(r);
-      if (list == kPartsList) reinterpret_cast<uint4*>(part_counters(work))[at] = make_uint4(0u, 0u, 0u, 0u);
-      if (list == kGlobalList) atomicMax(reinterpret_cast<unsigned long long*>(&work[8]), static_cast<unsigned long long>(all));
+      if (list == kPartsList) {
+        reinterpret_cast<uint4*>(part_counters(work))[at] = make_uint4(0u, 0u, 0u, 0u);
+        if (rows <= kLookRows) {
+          uint32_t const parts = static_cast<uint32_t>(parts_of(all)), first = atomicAdd(&counts[kTotalParts], parts);
+          for (uint32_t p = 0; p < parts; ++p) single_parts(work, rows)[first + p] = at | p << 16;
+        }
+      }
+      if (list == kGlobalList) {
+        atomicMax(reinterpret_cast<unsigned long long*>(&counts[8]), static_cast<unsigned long long>(all));
+        __threadfence();  // (there when the last workgroup has listed its pairs)
+      }
+    }
+    if (told.arrivals) {
+      __syncthreads();
+      if (wave == 0) {
+        uint32_t last = 0;
+        if (lane == 0) last = atomicAdd(&told.arrivals->sum, 1ull) + 1ull == gridDim.x;
+        if (wave_bcast(last, 0) != 0) {
+          // (all is left as it was found: zeros)
+          if (lane == 0) atomicExch(&told.arrivals->sum, 0ull);
+          if (lane < kListHeader) {
+            uint32_t const v = atomicExch(&told.arrivals->words[lane], 0u);
+            work[lane]       = v;
+            told.host[lane]  = v;
+          }
+          __threadfence_system();
+          if (lane == 0) told.post.send();
+        }
+      }
     }
     bool again = false;
     for (;;) {
@@ -653,7 +697,24 @@ __global__ void __launch_bounds__(kTierWaves[TIER] * kWave, kSimdWaves[TIER]) ja
   }
 }
 
-// The pairs in parts: workgroup (x, y) does part y of the pairs x, x + gridDim.x, ...  The last part to be done writes
+// By one thread: adds the counts of a part of pair r, which has this entry of its list.
+__device__ __forceinline__ void finish_part(uint32_t* work, int64_t rows, uint32_t r, int64_t bytes, uint32_t entry, uint32_t parts,
+                                            uint32_t const (&counts)[3], bool ok, float* out)
+{
+  uint32_t* const at = part_counters(work) + 4 * static_cast<int64_t>(entry);
+  for (int k = 0; k < 3; ++k) atomicAdd(&at[k], counts[k]);
+  __threadfence();
+  // a full set leaves a mark far above the number of parts
+  uint32_t const done = atomicAdd(&at[3], ok ? 1u : 1u + (1u << 16)) + (ok ? 1u : 1u + (1u << 16));
+  if ((done & 0xFFFFu) == parts) {
+    __threadfence();
+    if (done >> 16)
+      list_for_global(work, rows, r, bytes);
+    else
+      out[r] = index_of(atomicAdd(&at[0], 0u), atomicAdd(&at[1], 0u), atomicAdd(&at[2], 0u));
+  }
+}
+// The pairs in parts of a column of many pairs: workgroup (x, y) does part y of the pairs x, x + gridDim.x, ...  The last part to be done writes
 // the index.  A part whose set is full (its share of the hashes far above the average) has the pair done once more, by
 // the set in global memory.
 constexpr int kPartsTier = kTiers - 1;
@@ -676,20 +737,138 @@ __global__ void __launch_bounds__(kTierWaves[kPartsTier] * kWave) jaccard_parts_
     if (part.part >= part.parts) continue;
     uint32_t counts[3];
     bool const ok = count_pair<WAVES>(c1, c2, pair, width, part, slots, SLOTS, scratch, ++number, counts);
-    if (threadIdx.x == 0) {
-      uint32_t* const at = part_counters(work) + 4 * static_cast<int64_t>(i);
-      for (int k = 0; k < 3; ++k) atomicAdd(&at[k], counts[k]);
-      __threadfence();
-      // a full set leaves a mark far above the number of parts
-      uint32_t const done = atomicAdd(&at[3], ok ? 1u : 1u + (1u << 16)) + (ok ? 1u : 1u + (1u << 16));
-      if ((done & 0xFFFFu) == part.parts) {
-        __threadfence();
-        if (done >> 16)
-          list_for_global(work, rows, r, pair.bytes());
-        else
-          out[r] = index_of(atomicAdd(&at[0], 0u), atomicAdd(&at[1], 0u), atomicAdd(&at[2], 0u));
-      }
+    if (threadIdx.x == 0) finish_part(work, rows, r, pair.bytes(), i, part.parts, counts, ok, out);
+  }
+}
+
+// All lists but the last in one launch, where the host knows what is on them (columns of up to kLookRows pairs).  With a launch a
+// tier each waits for its slowest pair before the next begins.  A workgroup of sixteen wavefronts and the largest set takes
+// pieces of work until none is left: a part of a pair, a pair of the last two tiers, two pairs of tier 2 or four of tier 1,
+// each by a team of its wavefronts with its share of the set; the longest first.  The teams share the barriers.  Pairs of twice 1500
+// bytes, 166 of them 76 -> 33 us, 466 77 -> 33, 2,000 131 -> 80; of twice 6000, 1,666 330 -> 214, 3,333 418 -> 291, 16,666
+// 1526 -> 1120; 7,500 of twice 200 58 -> 51.  What bounds it is one piece: its bytes are hashed by one CU.
+// With more than kTeamPieces pieces of the first three tiers these have their own kernels, more of whose wavefronts fit a CU
+// (13,333 pairs of twice 1500 bytes in a launch 244 us, with their own kernels 230; 32,666 495 and 421; but 1,666 of twice 6000, 1,400
+// pieces, 213 and 267).
+struct Pieces {
+  uint32_t parts, tier4, tier3, tier2, tier1;  // where the pieces of each kind end
+  int waves2, waves1;                          // wavefronts of a team of the last two kinds
+};
+constexpr uint32_t kTeamPieces = 1536;  // of the first three tiers at most
+constexpr int kTeamWaves       = 16;
+constexpr uint32_t kTeamSlots  = kSlots[kTiers - 1];
+struct TeamScratch {
+  TileLds tile[kTeamWaves];
+  uint32_t sums[3][kTeamWaves];
+  uint32_t full[kTeamWaves];  // of a team's first wavefront: the set was full
+  uint32_t next;
+};
+__global__ void __launch_bounds__(kTeamWaves * kWave) jaccard_teams_kernel(ColView c1, ColView c2, int32_t width, float* __restrict__ out,
+                                                                           uint32_t* __restrict__ work, Pieces pieces)
+{
+  __shared__ alignas(16) uint32_t slots[kTeamSlots];
+  __shared__ TeamScratch scratch;
+  int64_t const rows = c1.size;
+  int const lane     = lane_id();
+  int const wave     = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
+  for (uint32_t i = threadIdx.x; i < kTeamSlots / 4; i += kTeamWaves * kWave) reinterpret_cast<uint4*>(slots)[i] = make_uint4(0u, 0u, 0u, 0u);
+  bool const more = pieces.tier1 > gridDim.x;
+  for (uint32_t piece = blockIdx.x; piece < pieces.tier1;) {
+    // the team's wavefronts, its share of the set, and the entry of its list that it has (none: `have` is false)
+    int waves = kTeamWaves, list = kPartsList;
+    uint32_t most = kTeamSlots, entry = piece;
+    if (piece >= pieces.tier2) {
+      waves = pieces.waves1, list = 0, most = kSlots[1];
+      entry = (piece - pieces.tier2) * (kTeamWaves / waves) + static_cast<uint32_t>(wave / waves);
+    } else if (piece >= pieces.tier3) {
+      waves = pieces.waves2, list = 1, most = kSlots[2];
+      entry = (piece - pieces.tier3) * (kTeamWaves / waves) + static_cast<uint32_t>(wave / waves);
+    } else if (piece >= pieces.tier4) {
+      list = 2, most = kSlots[3], entry = piece - pieces.tier4;
+    } else if (piece >= pieces.parts) {
+      list = 3, entry = piece - pieces.parts;
     }
+    int const team      = wave / waves, own = wave % waves;
+    uint32_t* const set = slots + static_cast<uint32_t>(team) * most;
+    Part part{0, 1};
+    uint32_t counter = 0;
+    bool have        = true;
+    if (list == kPartsList) {
+      uint32_t const e = single_parts(work, rows)[piece];
+      counter          = e & 0xFFFFu;
+      part.part        = e >> 16;
+      entry            = counter;
+    } else {
+      have = entry < work[list];
+    }
+    uint32_t r = 0;
+    Pair pair{0, 0, 0, 0};
+    if (have) {
+      r    = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(list_entries(work, list, rows)[entry])));
+      pair = uniform_pair_at(c1, c2, r);
+    }
+    if (list == kPartsList) part.parts = static_cast<uint32_t>(parts_of(pair.bytes()));
+    uint32_t const nslots = list == kPartsList ? most : slots_for(pair.bytes(), most);
+    if (own == 0 && lane == 0) scratch.full[wave] = 0u;
+    uint32_t next = pieces.tier1;
+    if (more && threadIdx.x == 0) next = atomicAdd(&work[kNextPiece], 1u) + gridDim.x;
+    __syncthreads();  // (the set is empty, the flags are down, the sums of the piece before have been read)
+    bool const ok = insert_pair(c1, c2, pair, width, PackedSet{set, nslots / 4}, part, scratch.tile[wave], own, waves, lane);
+    if (!ok) scratch.full[wave - own] = 1u;
+    if (threadIdx.x == 0) scratch.next = next;
+    __syncthreads();
+    bool const full = __builtin_amdgcn_readfirstlane(static_cast<int>(scratch.full[wave - own])) != 0;
+    next            = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(scratch.next)));
+    PackedSet::Count in;
+    for (uint32_t i = own * kWave + lane; i < nslots / 4; i += waves * kWave) {
+      uint4* const four = reinterpret_cast<uint4*>(set) + i;
+      in.add(*four);
+      *four = make_uint4(0u, 0u, 0u, 0u);
+    }
+    uint32_t u[3], total[3];
+    auto const add_team = [&] {
+      for (int k = 0; k < 3; ++k) u[k] = wave_inclusive_scan(u[k]);
+      if (lane == kWave - 1) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) scratch.sums[k][wave] = u[k];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        total[k] = 0;
+        for (int w = 0; w < waves; ++w) total[k] += scratch.sums[k][wave - own + w];
+      }
+    };
+    in.get(u);
+    add_team();
+    if (list != kPartsList && __syncthreads_or(full ? 1 : 0) != 0) {
+      // a value found no place in a packed set (none in text): such a pair once more with a plain one; every team comes along
+      PlainSet<true> const plain = plain_in(set, most);
+      Pair const again           = full ? pair : Pair{0, 0, 0, 0};
+      uint32_t const words       = plain.buckets / 8;
+      for (uint32_t i = own * kWave + lane; i < most; i += waves * kWave) set[i] = 0u;
+      __syncthreads();
+      insert_pair(c1, c2, again, width, plain, part, scratch.tile[wave], own, waves, lane);
+      __syncthreads();
+      u[0] = u[1] = u[2] = 0;
+      for (uint32_t i = own * kWave + lane; i < words; i += waves * kWave) {
+        u[0] += __builtin_popcount(plain.in1[i]);
+        u[1] += __builtin_popcount(plain.in2[i]);
+        u[2] += __builtin_popcount(plain.in1[i] & plain.in2[i]);
+      }
+      uint32_t const before[3] = {total[0], total[1], total[2]};
+      add_team();
+      if (!full)
+        for (int k = 0; k < 3; ++k) total[k] = before[k];
+      for (uint32_t i = own * kWave + lane; i < most; i += waves * kWave) set[i] = 0u;
+    }
+    if (have && own == 0 && lane == 0) {
+      if (list != kPartsList)
+        out[r] = index_of(total[0], total[1], total[2]);
+      else
+        finish_part(work, rows, r, pair.bytes(), counter, part.parts, total, !full, out);
+    }
+    piece = next;
   }
 }
 
@@ -791,29 +970,36 @@ nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* inpu
     return fail(NVTEXT_AMD_ALLOC_FAILED, "temporary allocation failed");
   }
   uint32_t* const lists = work.as<uint32_t>();
-  launch_fill_u32(lists, 0u, kListHeader, stream);
+  // In a column of few pairs the launches of the other kernels, most of which would find their lists empty, are more than
+  // the work: the host looks at the lists first and launches what has something to do (7 pairs of 300 bytes 48 -> 20 us).
+  // In a larger one the wait costs more than a few empty launches.
+  bool const look         = rows <= kLookRows;
+  uint64_t* const pinned  = host_scalars();
+  Arrivals* const own     = look && pinned ? thread_arrivals() : nullptr;  // (the lists are then counted there, and the first launch tells the host)
+  if (!own) launch_fill_u32(lists, 0u, kListHeader, stream);
 
   ColView const v1 = make_view(*input1);
   ColView const v2 = make_view(*input2);
   float* const values = static_cast<float*>(out->data);
   int const cus       = device_cus();
+  if (with_mask) {
+    int32_t const words = (rows + 31) / 32;
+    hipLaunchKernelGGL(and_bitmask_kernel, dim3((words + 255) / 256), dim3(256), 0, stream, out->null_mask,
+                       input1->null_count > 0 ? input1->null_mask : nullptr, input1->offset,
+                       input2->null_count > 0 ? input2->null_mask : nullptr, input2->offset, rows, words, own ? &own->words[kLists] : &lists[kLists]);
+  }
+  Told told{own, reinterpret_cast<uint32_t*>(pinned), HostPost{}};
+  if (own) told.post = new_post();
   {
     ProfileScope ps("jaccard_wave_kernel", stream);
     int per_group = kThreads;
     while (per_group > kWaves && rows / per_group < 4 * cus) per_group /= 2;
     int64_t const groups = (static_cast<int64_t>(rows) + per_group - 1) / per_group;
     unsigned const grid  = static_cast<unsigned>(std::min<int64_t>(groups, static_cast<int64_t>(cus) * 64));
-    hipLaunchKernelGGL(jaccard_wave_kernel, dim3(grid), dim3(kThreads), 0, stream, v1, v2, width, values, lists, per_group);
-  }
-  if (with_mask) {
-    int32_t const words = (rows + 31) / 32;
-    hipLaunchKernelGGL(and_bitmask_kernel, dim3((words + 255) / 256), dim3(256), 0, stream, out->null_mask,
-                       input1->null_count > 0 ? input1->null_mask : nullptr, input1->offset,
-                       input2->null_count > 0 ? input2->null_mask : nullptr, input2->offset, rows, words, &lists[kLists]);
+    hipLaunchKernelGGL(jaccard_wave_kernel, dim3(grid), dim3(kThreads), 0, stream, v1, v2, width, values, lists, per_group, told);
   }
   // what the host has to know: the header of the lists
   uint32_t copied[kListHeader] = {};
-  uint64_t* const pinned       = host_scalars();
   const uint32_t* const head   = pinned ? reinterpret_cast<const uint32_t*>(pinned) : copied;
   auto const read_header       = [&]() -> hipError_t {
     if (!pinned) {
@@ -825,31 +1011,58 @@ nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* inpu
     hipError_t const e = hipGetLastError();
     return e == hipSuccess ? wait_for_post(post, stream) : e;
   };
-  // In a column of few pairs the launches of the other kernels, most of which would find their lists empty, are more than
-  // the work: the host looks at the lists first and launches what has something to do (7 pairs of 300 bytes 48 -> 20 us).
-  // In a larger one the wait costs more than a few empty launches.
-  bool const look   = rows <= kLookRows;
-  hipError_t e      = look ? read_header() : hipSuccess;
+  hipError_t e = hipGetLastError();
+  if (own) {
+    if (e != hipSuccess) forsake_thread_arrivals();  // (nobody knows what it holds)
+    if (e == hipSuccess) {
+      e = wait_for_post(told.post, stream);
+      if (e != hipSuccess) forsake_thread_arrivals();
+    }
+  } else if (look && e == hipSuccess) {
+    e = read_header();
+  }
   auto const listed = [&](int list) { return look ? static_cast<int32_t>(head[list]) : rows; };
   auto const grid_of = [&](int list, int per_cu) { return dim3(static_cast<unsigned>(std::min<int64_t>(listed(list), static_cast<int64_t>(cus) * per_cu))); };
-  if (e == hipSuccess && listed(0) > 0) {
+  bool few = false;  // pairs on the first three lists
+  Pieces pieces{};
+  if (look && e == hipSuccess) {
+    pieces.parts = head[kTotalParts];
+    pieces.tier4 = pieces.parts + static_cast<uint32_t>(listed(3));
+    // (fewer pieces than CUs: a workgroup for every pair)
+    uint32_t const pairs = static_cast<uint32_t>(listed(2)) + static_cast<uint32_t>(listed(1)) + static_cast<uint32_t>(listed(0));
+    bool const alone     = pieces.tier4 + pairs <= static_cast<uint32_t>(cus);
+    pieces.waves2        = alone ? kTeamWaves : kTierWaves[2];
+    pieces.waves1        = alone ? kTeamWaves : kTierWaves[1];
+    auto const teams_of  = [&](int list, int waves) { return static_cast<uint32_t>((listed(list) + kTeamWaves / waves - 1) / (kTeamWaves / waves)); };
+    uint32_t const n3 = teams_of(2, kTeamWaves), n2 = teams_of(1, pieces.waves2), n1 = teams_of(0, pieces.waves1);
+    few          = n3 + n2 + n1 <= kTeamPieces;
+    pieces.tier3 = pieces.tier4 + (few ? n3 : 0u);
+    pieces.tier2 = pieces.tier3 + (few ? n2 : 0u);
+    pieces.tier1 = pieces.tier2 + (few ? n1 : 0u);
+    if (pieces.tier1 > 0) {
+      ProfileScope ps("jaccard_teams_kernel", stream);
+      hipLaunchKernelGGL(jaccard_teams_kernel, dim3(std::min<uint32_t>(pieces.tier1, static_cast<uint32_t>(cus))), dim3(kTeamWaves * kWave), 0, stream, v1, v2,
+                         width, values, lists, pieces);
+    }
+  }
+  if (!few && e == hipSuccess && listed(0) > 0) {
     ProfileScope ps("jaccard_listed_kernel<1>", stream);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(jaccard_listed_kernel<1>), grid_of(0, 28), dim3(kTierWaves[1] * kWave), 0, stream, v1, v2, width, values, lists);
   }
-  if (e == hipSuccess && listed(1) > 0) {
+  if (!few && e == hipSuccess && listed(1) > 0) {
     ProfileScope ps("jaccard_listed_kernel<2>", stream);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(jaccard_listed_kernel<2>), grid_of(1, 12), dim3(kTierWaves[2] * kWave), 0, stream, v1, v2, width, values, lists);
   }
-  if (e == hipSuccess && listed(2) > 0) {
+  if (!few && e == hipSuccess && listed(2) > 0) {
     ProfileScope ps("jaccard_listed_kernel<3>", stream);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(jaccard_listed_kernel<3>), grid_of(2, 8), dim3(kTierWaves[3] * kWave), 0, stream, v1, v2, width, values, lists);
   }
-  if (e == hipSuccess && listed(3) > 0) {
+  if (!look && e == hipSuccess) {
     ProfileScope ps("jaccard_listed_kernel<4>", stream);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(jaccard_listed_kernel<4>), grid_of(3, 4), dim3(kTierWaves[4] * kWave), 0, stream, v1, v2, width, values, lists);
   }
   bool const in_parts = listed(kPartsList) > 0;
-  if (e == hipSuccess && in_parts) {
+  if (!look && e == hipSuccess) {
     ProfileScope ps("jaccard_parts_kernel", stream);
     hipLaunchKernelGGL(jaccard_parts_kernel, dim3(grid_of(kPartsList, 1).x, static_cast<unsigned>(kMaxParts)), dim3(kTierWaves[kPartsTier] * kWave), 0, stream,
                        v1, v2, width, values, lists);

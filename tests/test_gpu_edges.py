@@ -106,6 +106,29 @@ def test_jaccard_values_of_neighbouring_buckets(nv, orc, count, slots, parts):
     assert np.array_equal(got.values.view(np.uint32), exp.values.view(np.uint32))
 
 
+@pytest.mark.parametrize("copies", [1, 20, 55, 400])
+def test_jaccard_lists_of_few_and_many_pairs(nv, orc, copies):
+    """Pairs for every set and in parts, side by side, some of which find no place in theirs: fewer than there are CUs, so many
+    that a workgroup has several of them at a time, and so many that the sets have kernels of their own."""
+    rng = np.random.default_rng(copies)
+    letters = np.concatenate([np.arange(65, 91), np.arange(97, 123)]).astype(np.uint32)
+    words = (letters[:, None, None, None] | letters[:, None, None] << 8 | letters[:, None] << 16 | letters << 24).astype(np.uint32).ravel()
+    rows = [random_text(rng, n).decode() for n in (10, 700, 900, 2500, 3276, 3277, 5000, 5606, 5607, 9000, 12_390, 12_391, 20_000)]
+    rows += [random_text(rng, n).decode() for n in (23_552, 23_553, 61_000)] if copies < 100 else []
+    for count, slots in ((600, 4096), (1000, 7008), (2000, 15488)):
+        home, step, _ = jaccard_places(words, slots // 4, 1)
+        from_there = np.flatnonzero((home >= 77) & (step == 1))
+        near = from_there[np.argsort(home[from_there], kind="stable")][:count]
+        rows.append(bytes(rng.permutation(words[near]).view(np.uint8)).decode())
+    left, right = [t[: len(t) // 3] for t in rows], [t[len(t) // 4:] for t in rows]
+    h1, h2 = (HostStringsColumn.from_pylist(side) for side in (left, right))
+    exp = orc.jaccard_index(h1, h2, 4, nthreads=8).values.view(np.uint32)
+    h1, h2 = (HostStringsColumn.from_pylist(side * copies) for side in (left, right))
+    for _ in range(2):
+        got = nv.jaccard_index(dev(nv, h1), dev(nv, h2), 4).to_host()
+        assert np.array_equal(got.values.view(np.uint32), np.tile(exp, copies))
+
+
 @pytest.mark.parametrize("width", [2, 7, 40])
 def test_jaccard_pair_sizes(nv, orc, width):
     """Pairs of the most bytes that each set takes (4/5 of its slots) and of one more, around one
