@@ -509,6 +509,7 @@ constexpr uint32_t kOnceMore = 0x80000000u;  // (rows are fewer)
 // every entry of the list of pairs in parts, and `rows` entries for each list; in a column of up to kLookRows pairs behind these a
 // list of the parts themselves (a pair's entry | its number << 16).
 constexpr int kListHeader = 16;
+constexpr int kMostBytes  = 8;
 constexpr int kTotalParts = 10;
 constexpr int kNextPiece  = 11;
 constexpr int32_t kLookRows = 32768;  // see nvtext_amd_jaccard_index
@@ -522,7 +523,7 @@ __device__ __forceinline__ uint32_t* single_parts(uint32_t* work, int64_t rows) 
 __device__ __forceinline__ void list_for_global(uint32_t* work, int64_t rows, int64_t r, int64_t bytes)
 {
   list_entries(work, kGlobalList, rows)[atomicAdd(&work[kGlobalList], 1u)] = static_cast<uint32_t>(r);
-  atomicMax(reinterpret_cast<unsigned long long*>(&work[8]), static_cast<unsigned long long>(bytes));
+  atomicMax(reinterpret_cast<unsigned long long*>(&work[kMostBytes]), static_cast<unsigned long long>(bytes));
 }
 
 struct WaveSetLds {
@@ -535,10 +536,13 @@ static_assert(kSlots[0] == PackedSet::kLeast, "every pair of a wavefront takes a
 // lists those that need more than a wavefront's own set for the later kernels with one atomic per list (atomics on one
 // cache line run at about 150 M/s: one per wavefront and list was most of this kernel's time), and its wavefronts do the
 // others, each taking the next one when it is done with one.  A column of few pairs is shared out over more workgroups.
-// told.arrivals (a column of up to kLookRows pairs, a workgroup for every group): the lists are counted there, and the workgroup that
-// is last to have listed its pairs tells the host the header, while all still have their own pairs to do.
+// told.arrivals (a column of up to kLookRows pairs): the first workgroups list 256 pairs each before they do their own, in counters
+// there, and the one that is last to have done so tells the host the header, while all have their own pairs yet to do.  (Were every
+// workgroup to list its own, of which there are 1,000 to 2,000 for the sake of those pairs, their atomics would be all of the
+// time: 3,333 pairs of twice 6000 bytes took 24 us to list, now 14, and 8,166 42, now 17; 7,500 of twice 200 bytes 36, now 24.)
 struct Told {
   Arrivals* arrivals;
+  uint32_t listers;
   uint32_t* host;
   HostPost post;
 };
@@ -551,12 +555,55 @@ __global__ void __launch_bounds__(kThreads) jaccard_wave_kernel(ColView c1, ColV
   int const wave     = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
   WaveSetLds& lds    = lds_all[wave];
   int64_t const rows = c1.size;
-  uint32_t* const counts = told.arrivals ? told.arrivals->words : work;
   auto wave_sync = [] {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
+  // lists the pairs r of this workgroup's threads in `counts`
+  auto const list_pairs = [&](bool later, int64_t r, int64_t bytes, uint32_t* counts, bool with_parts) {
+    int const list = list_of(bytes);
+    uint32_t at    = 0;
+    if (later) at = atomicAdd(&listed[list], 1u);
+    __syncthreads();
+    if (threadIdx.x < kLists && listed[threadIdx.x] != 0u) place[threadIdx.x] = atomicAdd(&counts[threadIdx.x], listed[threadIdx.x]);
+    __syncthreads();
+    if (!later) return;
+    at += place[list];
+    list_entries(work, list, rows)[at] = static_cast<uint32_t>(r);
+    if (list == kPartsList) {
+      reinterpret_cast<uint4*>(part_counters(work))[at] = make_uint4(0u, 0u, 0u, 0u);
+      if (with_parts) {
+        uint32_t const parts = static_cast<uint32_t>(parts_of(bytes)), first = atomicAdd(&counts[kTotalParts], parts);
+        for (uint32_t p = 0; p < parts; ++p) single_parts(work, rows)[first + p] = at | p << 16;
+      }
+    }
+    if (list == kGlobalList) atomicMax(reinterpret_cast<unsigned long long*>(&counts[kMostBytes]), static_cast<unsigned long long>(bytes));
+  };
+  if (told.arrivals && blockIdx.x < told.listers) {
+    if (threadIdx.x < kLists) listed[threadIdx.x] = 0u;
+    __syncthreads();
+    int64_t const r     = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    int64_t const bytes = r < rows ? pair_at(c1, c2, r).bytes() : 0;
+    list_pairs(bytes > most_bytes(kSlots[0]), r, bytes, told.arrivals->words, true);
+    __threadfence();  // (all that was added is there before this workgroup is seen to have arrived)
+    __syncthreads();
+    if (wave == 0) {
+      uint32_t last = 0;
+      if (lane == 0) last = atomicAdd(&told.arrivals->sum, 1ull) + 1ull == told.listers;
+      if (wave_bcast(last, 0) != 0) {
+        // (all is left as it was found: zeros)
+        if (lane == 0) atomicExch(&told.arrivals->sum, 0ull);
+        if (lane < kListHeader) {
+          uint32_t const v = atomicExch(&told.arrivals->words[lane], 0u);
+          work[lane]       = v;
+          told.host[lane]  = v;
+        }
+        __threadfence_system();
+        if (lane == 0) told.post.send();
+      }
+    }
+  }
   for (int64_t base = static_cast<int64_t>(blockIdx.x) * per_group; base < rows; base += static_cast<int64_t>(gridDim.x) * per_group) {
     __syncthreads();
     if (threadIdx.x < kLists) listed[threadIdx.x] = 0u;
@@ -566,46 +613,11 @@ __global__ void __launch_bounds__(kThreads) jaccard_wave_kernel(ColView c1, ColV
     bool const have   = r < rows && static_cast<int>(threadIdx.x) < per_group;
     int64_t const all = have ? pair_at(c1, c2, r).bytes() : 0;
     bool const later  = have && all > most_bytes(kSlots[0]);
-    int const list    = list_of(all);
-    uint32_t at       = 0;
     if (have && !later) solo[atomicAdd(&solos, 1u)] = static_cast<uint32_t>(r);
-    if (later) at = atomicAdd(&listed[list], 1u);
-    __syncthreads();
-    if (threadIdx.x < kLists && listed[threadIdx.x] != 0u) place[threadIdx.x] = atomicAdd(&counts[threadIdx.x], listed[threadIdx.x]);
-    __syncthreads();
-    if (later) {
-      at += place[list];
-      list_entries(work, list, rows)[at] = static_cast<uint32_t>(r);
-      if (list == kPartsList) {
-        reinterpret_cast<uint4*>(part_counters(work))[at] = make_uint4(0u, 0u, 0u, 0u);
-        if (rows <= kLookRows) {
-          uint32_t const parts = static_cast<uint32_t>(parts_of(all)), first = atomicAdd(&counts[kTotalParts], parts);
-          for (uint32_t p = 0; p < parts; ++p) single_parts(work, rows)[first + p] = at | p << 16;
-        }
-      }
-      if (list == kGlobalList) {
-        atomicMax(reinterpret_cast<unsigned long long*>(&counts[8]), static_cast<unsigned long long>(all));
-        __threadfence();  // (there when the last workgroup has listed its pairs)
-      }
-    }
-    if (told.arrivals) {
+    if (told.arrivals)
       __syncthreads();
-      if (wave == 0) {
-        uint32_t last = 0;
-        if (lane == 0) last = atomicAdd(&told.arrivals->sum, 1ull) + 1ull == gridDim.x;
-        if (wave_bcast(last, 0) != 0) {
-          // (all is left as it was found: zeros)
-          if (lane == 0) atomicExch(&told.arrivals->sum, 0ull);
-          if (lane < kListHeader) {
-            uint32_t const v = atomicExch(&told.arrivals->words[lane], 0u);
-            work[lane]       = v;
-            told.host[lane]  = v;
-          }
-          __threadfence_system();
-          if (lane == 0) told.post.send();
-        }
-      }
-    }
+    else
+      list_pairs(later, r, all, work, false);
     bool again = false;
     for (;;) {
       uint32_t t = 0;
@@ -973,9 +985,9 @@ nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* inpu
   // In a column of few pairs the launches of the other kernels, most of which would find their lists empty, are more than
   // the work: the host looks at the lists first and launches what has something to do (7 pairs of 300 bytes 48 -> 20 us).
   // In a larger one the wait costs more than a few empty launches.
-  bool const look         = rows <= kLookRows;
-  uint64_t* const pinned  = host_scalars();
-  Arrivals* const own     = look && pinned ? thread_arrivals() : nullptr;  // (the lists are then counted there, and the first launch tells the host)
+  uint64_t* const pinned = host_scalars();
+  Arrivals* const own    = rows <= kLookRows && pinned ? thread_arrivals() : nullptr;
+  bool const look        = own != nullptr;
   if (!own) launch_fill_u32(lists, 0u, kListHeader, stream);
 
   ColView const v1 = make_view(*input1);
@@ -988,7 +1000,7 @@ nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* inpu
                        input1->null_count > 0 ? input1->null_mask : nullptr, input1->offset,
                        input2->null_count > 0 ? input2->null_mask : nullptr, input2->offset, rows, words, own ? &own->words[kLists] : &lists[kLists]);
   }
-  Told told{own, reinterpret_cast<uint32_t*>(pinned), HostPost{}};
+  Told told{own, static_cast<uint32_t>((static_cast<int64_t>(rows) + kThreads - 1) / kThreads), reinterpret_cast<uint32_t*>(pinned), HostPost{}};
   if (own) told.post = new_post();
   {
     ProfileScope ps("jaccard_wave_kernel", stream);
@@ -1012,14 +1024,9 @@ nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* inpu
     return e == hipSuccess ? wait_for_post(post, stream) : e;
   };
   hipError_t e = hipGetLastError();
-  if (own) {
+  if (look) {
+    if (e == hipSuccess) e = wait_for_post(told.post, stream);
     if (e != hipSuccess) forsake_thread_arrivals();  // (nobody knows what it holds)
-    if (e == hipSuccess) {
-      e = wait_for_post(told.post, stream);
-      if (e != hipSuccess) forsake_thread_arrivals();
-    }
-  } else if (look && e == hipSuccess) {
-    e = read_header();
   }
   auto const listed = [&](int list) { return look ? static_cast<int32_t>(head[list]) : rows; };
   auto const grid_of = [&](int list, int per_cu) { return dim3(static_cast<unsigned>(std::min<int64_t>(listed(list), static_cast<int64_t>(cus) * per_cu))); };
