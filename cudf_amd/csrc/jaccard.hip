@@ -507,12 +507,12 @@ constexpr uint32_t kOnceMore = 0x80000000u;  // (rows are fewer)
 // [kNextPiece] = pieces of work handed out
 // -- then four counters (|A|, |B|, |A n B|, parts done) for
 // every entry of the list of pairs in parts, and `rows` entries for each list; in a column of up to kLookRows pairs behind these a
-// list of the parts themselves (a pair's entry | its number << 16).
+// list of the parts themselves (a pair's entry | its number << 28).
 constexpr int kListHeader = 16;
 constexpr int kMostBytes  = 8;
 constexpr int kTotalParts = 10;
 constexpr int kNextPiece  = 11;
-constexpr int32_t kLookRows = 32768;  // see nvtext_amd_jaccard_index
+constexpr int32_t kLookRows = 131072;  // see nvtext_amd_jaccard_index
 __host__ __device__ __forceinline__ size_t work_words(int64_t rows)
 {
   return kListHeader + static_cast<size_t>(kLists + 4 + (rows <= kLookRows ? kMaxParts : 0)) * static_cast<size_t>(rows);
@@ -575,7 +575,7 @@ __global__ void __launch_bounds__(kThreads) jaccard_wave_kernel(ColView c1, ColV
       reinterpret_cast<uint4*>(part_counters(work))[at] = make_uint4(0u, 0u, 0u, 0u);
       if (with_parts) {
         uint32_t const parts = static_cast<uint32_t>(parts_of(bytes)), first = atomicAdd(&counts[kTotalParts], parts);
-        for (uint32_t p = 0; p < parts; ++p) single_parts(work, rows)[first + p] = at | p << 16;
+        for (uint32_t p = 0; p < parts; ++p) single_parts(work, rows)[first + p] = at | p << 28;
       }
     }
     if (list == kGlobalList) atomicMax(reinterpret_cast<unsigned long long*>(&counts[kMostBytes]), static_cast<unsigned long long>(bytes));
@@ -807,8 +807,8 @@ __global__ void __launch_bounds__(kTeamWaves * kWave) jaccard_teams_kernel(ColVi
     bool have        = true;
     if (list == kPartsList) {
       uint32_t const e = single_parts(work, rows)[piece];
-      counter          = e & 0xFFFFu;
-      part.part        = e >> 16;
+      counter          = e & 0x0FFFFFFFu;
+      part.part        = e >> 28;
       entry            = counter;
     } else {
       have = entry < work[list];
@@ -983,8 +983,9 @@ nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* inpu
   }
   uint32_t* const lists = work.as<uint32_t>();
   // In a column of few pairs the launches of the other kernels, most of which would find their lists empty, are more than
-  // the work: the host looks at the lists first and launches what has something to do (7 pairs of 300 bytes 48 -> 20 us).
-  // In a larger one the wait costs more than a few empty launches.
+  // the work: the host looks at the lists first and launches what has something to do (35,000 pairs of twice 200 bytes 148 -> 127 us,
+  // 100,000 278 -> 264).  In a larger one its wait and the listing before all else cost more (245,000 527 -> 554, 250,001 of
+  // twice 2 KB 3500 -> 3605).
   uint64_t* const pinned = host_scalars();
   Arrivals* const own    = rows <= kLookRows && pinned ? thread_arrivals() : nullptr;
   bool const look        = own != nullptr;
