@@ -47,7 +47,10 @@ constexpr int kGlobalList = kTiers;
 constexpr int kLists      = kTiers + 1;
 
 constexpr int64_t kPartBytes = 20000;  // bytes of a pair per part: 0.68 of the largest set, room for an uneven cut
-constexpr int64_t kMaxParts  = 16;     // the hashing is done once per part
+// The hashing is done once per part, and the parts of a pair on as many CUs: a pair of 330 KB in 17 parts 0.22 ms, with one set in
+// global memory 3.7, and of 600 KB in 30 0.38 and 6.6; a thousand of them 13 and 42 ms, and 26 and 48 (with 64 parts many pairs
+// of more than 640 KB would take longer).
+constexpr int64_t kMaxParts  = 32;
 
 __device__ __host__ __forceinline__ int64_t parts_of(int64_t bytes) { return (bytes + kPartBytes - 1) / kPartBytes; }
 
@@ -214,9 +217,29 @@ __device__ __forceinline__ bool place(Set const& set, uint32_t value, typename S
   return false;
 }
 
-// A share of the hashes by value, for pairs that are cut into parts (other bits than the set's own multiplication uses).
+// A share of the hashes by value, for pairs that are cut into parts (other bits than the set's own multiplication uses).  A part
+// that its set has no room for is cut in two, as often as it takes (of 2^31 shares none has more than two values): nothing is left over for
+// another kernel, so that the host need not wait for the parts (41 pairs of twice 6000 bytes, some of them in parts, 62 -> 49 us).
 struct Part {
   uint32_t part, parts;
+  // The whole part, then what is left of it: `level` bits of `at` tell which share of it is next.
+  uint32_t level = 0, at = 0;
+  __device__ __forceinline__ Part share() const { return Part{(part << level) + at, parts << level}; }
+  // After a share: whether there is another one.
+  __device__ __forceinline__ bool more(bool full)
+  {
+    if (full) {
+      ++level;
+      at <<= 1;
+      return true;
+    }
+    ++at;
+    while (level != 0 && (at & 1u) == 0) {
+      at >>= 1;
+      --level;
+    }
+    return level != 0;
+  }
   __device__ __forceinline__ bool holds(uint32_t h) const
   {
     return parts == 1u || __umulhi((h ^ (h >> 15)) * 0x85EBCA6Bu, parts) == part;
@@ -506,26 +529,23 @@ constexpr uint32_t kOnceMore = 0x80000000u;  // (rows are fewer)
 // [8..9] = the most bytes a pair of the global list has (64 bits), [kTotalParts] = parts of all pairs on the list of pairs in parts,
 // [kNextPiece] = pieces of work handed out
 // -- then four counters (|A|, |B|, |A n B|, parts done) for
-// every entry of the list of pairs in parts, and `rows` entries for each list; in a column of up to kLookRows pairs behind these a
-// list of the parts themselves (a pair's entry | its number << 28).
+// every entry of the list of pairs in parts, `rows` entries for each list, and the first kMostParts of the parts themselves
+// (a pair's entry | its number << 27).
 constexpr int kListHeader = 16;
 constexpr int kMostBytes  = 8;
 constexpr int kTotalParts = 10;
 constexpr int kNextPiece  = 11;
 constexpr int32_t kLookRows = 131072;  // see nvtext_amd_jaccard_index
-__host__ __device__ __forceinline__ size_t work_words(int64_t rows)
+constexpr uint32_t kMostParts = 1u << 16;  // (of pairs of 0.8 GB and more)
+static_assert(kMostParts <= 1u << 27 && kMaxParts <= 32);
+__host__ __device__ __forceinline__ uint32_t most_parts(int64_t rows)
 {
-  return kListHeader + static_cast<size_t>(kLists + 4 + (rows <= kLookRows ? kMaxParts : 0)) * static_cast<size_t>(rows);
+  return rows < kMostParts / kMaxParts ? static_cast<uint32_t>(rows * kMaxParts) : kMostParts;
 }
+__host__ __device__ __forceinline__ size_t work_words(int64_t rows) { return kListHeader + static_cast<size_t>(kLists + 4) * static_cast<size_t>(rows) + most_parts(rows); }
 __device__ __forceinline__ uint32_t* list_entries(uint32_t* work, int list, int64_t rows) { return work + kListHeader + (4 + list) * rows; }
 __device__ __forceinline__ uint32_t* part_counters(uint32_t* work) { return work + kListHeader; }
 __device__ __forceinline__ uint32_t* single_parts(uint32_t* work, int64_t rows) { return work + kListHeader + (kLists + 4) * rows; }
-__device__ __forceinline__ void list_for_global(uint32_t* work, int64_t rows, int64_t r, int64_t bytes)
-{
-  list_entries(work, kGlobalList, rows)[atomicAdd(&work[kGlobalList], 1u)] = static_cast<uint32_t>(r);
-  atomicMax(reinterpret_cast<unsigned long long*>(&work[kMostBytes]), static_cast<unsigned long long>(bytes));
-}
-
 struct WaveSetLds {
   alignas(16) uint32_t slots[kSlots[0]];
   TileLds tile;
@@ -561,7 +581,7 @@ __global__ void __launch_bounds__(kThreads) jaccard_wave_kernel(ColView c1, ColV
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
   // lists the pairs r of this workgroup's threads in `counts`
-  auto const list_pairs = [&](bool later, int64_t r, int64_t bytes, uint32_t* counts, bool with_parts) {
+  auto const list_pairs = [&](bool later, int64_t r, int64_t bytes, uint32_t* counts) {
     int const list = list_of(bytes);
     uint32_t at    = 0;
     if (later) at = atomicAdd(&listed[list], 1u);
@@ -573,10 +593,8 @@ __global__ void __launch_bounds__(kThreads) jaccard_wave_kernel(ColView c1, ColV
     list_entries(work, list, rows)[at] = static_cast<uint32_t>(r);
     if (list == kPartsList) {
       reinterpret_cast<uint4*>(part_counters(work))[at] = make_uint4(0u, 0u, 0u, 0u);
-      if (with_parts) {
-        uint32_t const parts = static_cast<uint32_t>(parts_of(bytes)), first = atomicAdd(&counts[kTotalParts], parts);
-        for (uint32_t p = 0; p < parts; ++p) single_parts(work, rows)[first + p] = at | p << 28;
-      }
+      uint32_t const parts = static_cast<uint32_t>(parts_of(bytes)), first = atomicAdd(&counts[kTotalParts], parts);
+      for (uint32_t p = 0; p < parts && first + p < most_parts(rows); ++p) single_parts(work, rows)[first + p] = at | p << 27;
     }
     if (list == kGlobalList) atomicMax(reinterpret_cast<unsigned long long*>(&counts[kMostBytes]), static_cast<unsigned long long>(bytes));
   };
@@ -585,7 +603,7 @@ __global__ void __launch_bounds__(kThreads) jaccard_wave_kernel(ColView c1, ColV
     __syncthreads();
     int64_t const r     = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     int64_t const bytes = r < rows ? pair_at(c1, c2, r).bytes() : 0;
-    list_pairs(bytes > most_bytes(kSlots[0]), r, bytes, told.arrivals->words, true);
+    list_pairs(bytes > most_bytes(kSlots[0]), r, bytes, told.arrivals->words);
     __threadfence();  // (all that was added is there before this workgroup is seen to have arrived)
     __syncthreads();
     if (wave == 0) {
@@ -617,7 +635,7 @@ __global__ void __launch_bounds__(kThreads) jaccard_wave_kernel(ColView c1, ColV
     if (told.arrivals)
       __syncthreads();
     else
-      list_pairs(later, r, all, work, false);
+      list_pairs(later, r, all, work);
     bool again = false;
     for (;;) {
       uint32_t t = 0;
@@ -709,26 +727,19 @@ __global__ void __launch_bounds__(kTierWaves[TIER] * kWave, kSimdWaves[TIER]) ja
   }
 }
 
-// By one thread: adds the counts of a part of pair r, which has this entry of its list.
-__device__ __forceinline__ void finish_part(uint32_t* work, int64_t rows, uint32_t r, int64_t bytes, uint32_t entry, uint32_t parts,
-                                            uint32_t const (&counts)[3], bool ok, float* out)
+// By one thread: adds the counts of a part of pair r, which has this entry of its list.  The last part to be done writes the index.
+__device__ __forceinline__ void finish_part(uint32_t* work, uint32_t r, uint32_t entry, uint32_t parts, uint32_t const (&counts)[3], float* out)
 {
   uint32_t* const at = part_counters(work) + 4 * static_cast<int64_t>(entry);
   for (int k = 0; k < 3; ++k) atomicAdd(&at[k], counts[k]);
   __threadfence();
-  // a full set leaves a mark far above the number of parts
-  uint32_t const done = atomicAdd(&at[3], ok ? 1u : 1u + (1u << 16)) + (ok ? 1u : 1u + (1u << 16));
-  if ((done & 0xFFFFu) == parts) {
+  if (atomicAdd(&at[3], 1u) + 1u == parts) {
     __threadfence();
-    if (done >> 16)
-      list_for_global(work, rows, r, bytes);
-    else
-      out[r] = index_of(atomicAdd(&at[0], 0u), atomicAdd(&at[1], 0u), atomicAdd(&at[2], 0u));
+    out[r] = index_of(atomicAdd(&at[0], 0u), atomicAdd(&at[1], 0u), atomicAdd(&at[2], 0u));
   }
 }
-// The pairs in parts of a column of many pairs: workgroup (x, y) does part y of the pairs x, x + gridDim.x, ...  The last part to be done writes
-// the index.  A part whose set is full (its share of the hashes far above the average) has the pair done once more, by
-// the set in global memory.
+// The pairs in parts of a column whose lists the host does not look at, or where they have more than kMostParts: then all that the
+// pairs could have are gone through.
 constexpr int kPartsTier = kTiers - 1;
 __global__ void __launch_bounds__(kTierWaves[kPartsTier] * kWave) jaccard_parts_kernel(ColView c1, ColView c2, int32_t width, float* __restrict__ out,
                                                                                        uint32_t* __restrict__ work)
@@ -737,19 +748,36 @@ __global__ void __launch_bounds__(kTierWaves[kPartsTier] * kWave) jaccard_parts_
   constexpr int WAVES      = kTierWaves[kPartsTier];
   __shared__ alignas(16) uint32_t slots[SLOTS];
   __shared__ PairScratch<WAVES> scratch;
-  int64_t const rows   = c1.size;
-  uint32_t const count = work[kPartsList];
-  if (blockIdx.x >= count) return;
+  __shared__ uint32_t next;
+  int64_t const rows    = c1.size;
+  bool const known      = work[kTotalParts] <= most_parts(rows);
+  uint64_t const pieces = known ? work[kTotalParts] : static_cast<uint64_t>(work[kPartsList]) * kMaxParts;
+  if (blockIdx.x >= pieces) return;
   start_pairs(slots, SLOTS, scratch);
   uint32_t number = 0;
-  for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
-    uint32_t const r  = list_entries(work, kPartsList, rows)[i];
-    Pair const pair   = uniform_pair_at(c1, c2, r);
-    Part const part{blockIdx.y, static_cast<uint32_t>(parts_of(pair.bytes()))};
-    if (part.part >= part.parts) continue;
-    uint32_t counts[3];
-    bool const ok = count_pair<WAVES>(c1, c2, pair, width, part, slots, SLOTS, scratch, ++number, counts);
-    if (threadIdx.x == 0) finish_part(work, rows, r, pair.bytes(), i, part.parts, counts, ok, out);
+  for (uint32_t piece = blockIdx.x; piece < pieces;) {
+    uint32_t ahead = 0;
+    if (threadIdx.x == 0) ahead = atomicAdd(&work[kNextPiece], 1u) + gridDim.x;
+    uint32_t const e = known ? single_parts(work, rows)[piece] : 0u;
+    uint32_t const i = known ? e & 0x07FFFFFFu : piece / kMaxParts;
+    uint32_t const r = list_entries(work, kPartsList, rows)[i];
+    Pair const pair  = uniform_pair_at(c1, c2, r);
+    Part part{known ? e >> 27 : piece % static_cast<uint32_t>(kMaxParts), static_cast<uint32_t>(parts_of(pair.bytes()))};
+    if (part.part < part.parts) {
+      uint32_t sum[3] = {0, 0, 0};
+      for (bool more = true; more;) {
+        uint32_t counts[3];
+        bool const ok = count_pair<WAVES>(c1, c2, pair, width, part.share(), slots, SLOTS, scratch, ++number, counts);
+        if (ok)
+          for (int k = 0; k < 3; ++k) sum[k] += counts[k];
+        more = part.more(!ok);
+      }
+      if (threadIdx.x == 0) finish_part(work, r, i, part.parts, sum, out);
+    }
+    if (threadIdx.x == 0) next = ahead;
+    __syncthreads();
+    piece = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(next)));
+    __syncthreads();
   }
 }
 
@@ -807,8 +835,8 @@ __global__ void __launch_bounds__(kTeamWaves * kWave) jaccard_teams_kernel(ColVi
     bool have        = true;
     if (list == kPartsList) {
       uint32_t const e = single_parts(work, rows)[piece];
-      counter          = e & 0x0FFFFFFFu;
-      part.part        = e >> 28;
+      counter          = e & 0x07FFFFFFu;
+      part.part        = e >> 27;
       entry            = counter;
     } else {
       have = entry < work[list];
@@ -821,23 +849,9 @@ __global__ void __launch_bounds__(kTeamWaves * kWave) jaccard_teams_kernel(ColVi
     }
     if (list == kPartsList) part.parts = static_cast<uint32_t>(parts_of(pair.bytes()));
     uint32_t const nslots = list == kPartsList ? most : slots_for(pair.bytes(), most);
-    if (own == 0 && lane == 0) scratch.full[wave] = 0u;
     uint32_t next = pieces.tier1;
     if (more && threadIdx.x == 0) next = atomicAdd(&work[kNextPiece], 1u) + gridDim.x;
-    __syncthreads();  // (the set is empty, the flags are down, the sums of the piece before have been read)
-    bool const ok = insert_pair(c1, c2, pair, width, PackedSet{set, nslots / 4}, part, scratch.tile[wave], own, waves, lane);
-    if (!ok) scratch.full[wave - own] = 1u;
-    if (threadIdx.x == 0) scratch.next = next;
-    __syncthreads();
-    bool const full = __builtin_amdgcn_readfirstlane(static_cast<int>(scratch.full[wave - own])) != 0;
-    next            = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(scratch.next)));
-    PackedSet::Count in;
-    for (uint32_t i = own * kWave + lane; i < nslots / 4; i += waves * kWave) {
-      uint4* const four = reinterpret_cast<uint4*>(set) + i;
-      in.add(*four);
-      *four = make_uint4(0u, 0u, 0u, 0u);
-    }
-    uint32_t u[3], total[3];
+    uint32_t u[3], total[3], sum[3] = {0, 0, 0};
     auto const add_team = [&] {
       for (int k = 0; k < 3; ++k) u[k] = wave_inclusive_scan(u[k]);
       if (lane == kWave - 1) {
@@ -851,9 +865,32 @@ __global__ void __launch_bounds__(kTeamWaves * kWave) jaccard_teams_kernel(ColVi
         for (int w = 0; w < waves; ++w) total[k] += scratch.sums[k][wave - own + w];
       }
     };
-    in.get(u);
-    add_team();
-    if (list != kPartsList && __syncthreads_or(full ? 1 : 0) != 0) {
+    bool full, any;
+    for (;;) {
+      if (lane == 0) scratch.full[wave] = 0u;
+      __syncthreads();  // (the set is empty, the flags are down, the sums of the piece before have been read)
+      bool const ok = insert_pair(c1, c2, pair, width, PackedSet{set, nslots / 4}, part.share(), scratch.tile[wave], own, waves, lane);
+      if (!ok) scratch.full[wave - own] = 1u;
+      if (threadIdx.x == 0) scratch.next = next;
+      __syncthreads();
+      uint32_t const flag = lane < kTeamWaves ? scratch.full[lane] : 0u;
+      full                = wave_bcast(flag, wave - own) != 0;
+      any                 = ballot64(flag != 0) != 0;
+      PackedSet::Count in;
+      for (uint32_t i = own * kWave + lane; i < nslots / 4; i += waves * kWave) {
+        uint4* const four = reinterpret_cast<uint4*>(set) + i;
+        in.add(*four);
+        *four = make_uint4(0u, 0u, 0u, 0u);
+      }
+      in.get(u);
+      add_team();
+      if (list != kPartsList) break;
+      if (!full)
+        for (int k = 0; k < 3; ++k) sum[k] += total[k];
+      if (!part.more(full)) break;
+    }
+    next = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(scratch.next)));
+    if (list != kPartsList && any) {
       // a value found no place in a packed set (none in text): such a pair once more with a plain one; every team comes along
       PlainSet<true> const plain = plain_in(set, most);
       Pair const again           = full ? pair : Pair{0, 0, 0, 0};
@@ -878,7 +915,7 @@ __global__ void __launch_bounds__(kTeamWaves * kWave) jaccard_teams_kernel(ColVi
       if (list != kPartsList)
         out[r] = index_of(total[0], total[1], total[2]);
       else
-        finish_part(work, rows, r, pair.bytes(), counter, part.parts, total, !full, out);
+        finish_part(work, r, counter, part.parts, sum, out);
     }
     piece = next;
   }
@@ -1032,9 +1069,11 @@ nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* inpu
   auto const listed = [&](int list) { return look ? static_cast<int32_t>(head[list]) : rows; };
   auto const grid_of = [&](int list, int per_cu) { return dim3(static_cast<unsigned>(std::min<int64_t>(listed(list), static_cast<int64_t>(cus) * per_cu))); };
   bool few = false;  // pairs on the first three lists
+  bool in_pieces = false;  // the pairs in parts
   Pieces pieces{};
   if (look && e == hipSuccess) {
-    pieces.parts = head[kTotalParts];
+    in_pieces    = head[kTotalParts] <= most_parts(rows);
+    pieces.parts = in_pieces ? head[kTotalParts] : 0u;
     pieces.tier4 = pieces.parts + static_cast<uint32_t>(listed(3));
     // (fewer pieces than CUs: a workgroup for every pair)
     uint32_t const pairs = static_cast<uint32_t>(listed(2)) + static_cast<uint32_t>(listed(1)) + static_cast<uint32_t>(listed(0));
@@ -1069,13 +1108,12 @@ nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* inpu
     ProfileScope ps("jaccard_listed_kernel<4>", stream);
     hipLaunchKernelGGL(HIP_KERNEL_NAME(jaccard_listed_kernel<4>), grid_of(3, 4), dim3(kTierWaves[4] * kWave), 0, stream, v1, v2, width, values, lists);
   }
-  bool const in_parts = listed(kPartsList) > 0;
-  if (!look && e == hipSuccess) {
+  if (!in_pieces && e == hipSuccess) {
     ProfileScope ps("jaccard_parts_kernel", stream);
-    hipLaunchKernelGGL(jaccard_parts_kernel, dim3(grid_of(kPartsList, 1).x, static_cast<unsigned>(kMaxParts)), dim3(kTierWaves[kPartsTier] * kWave), 0, stream,
+    hipLaunchKernelGGL(jaccard_parts_kernel, dim3(static_cast<unsigned>(cus)), dim3(kTierWaves[kPartsTier] * kWave), 0, stream,
                        v1, v2, width, values, lists);
   }
-  if (e == hipSuccess && in_parts) e = read_header();  // (a part can turn out too full: its pair is then on the list of the last kernel)
+  if (e == hipSuccess && !look) e = read_header();
   if (e != hipSuccess) {
     nvtext_amd_fixed_column_free(out, stream_, mr_);
     return fail(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));

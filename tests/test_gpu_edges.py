@@ -148,6 +148,23 @@ def test_jaccard_pair_sizes(nv, orc, width):
     assert np.array_equal(got.values.view(np.uint32), exp.values.view(np.uint32))
 
 
+@pytest.mark.parametrize("copies, sizes", [(1, (320_001, 640_000, 640_001)), (30_000, (700,) * 4 + (23_600,)), (33_000, (23_600,)), (150_000, (20, 2000))])
+def test_jaccard_many_parts(nv, orc, copies, sizes):
+    """Pairs of 17 and of the most parts (32), and of more; columns whose lists the host does not look at (more than 131,072 pairs), and
+    more parts than have a place on their list (65,536)."""
+    rng = np.random.default_rng(copies)
+    sizes = list(sizes) + ([23_600, 50_000] if copies == 150_000 else [])
+    rows = [random_text(rng, n).decode() for n in sizes]
+    left, right = [t[: len(t) // 3] for t in rows], [t[len(t) // 4: len(t) // 4 * 3] for t in rows]
+    left[-1], right[-1] = rows[-1][: sizes[-1] // 2], rows[-1][sizes[-1] // 2:]
+    times = [copies] * len(rows) if copies < 150_000 else [copies, 100, 50, 20]
+    h1, h2 = (HostStringsColumn.from_pylist(side) for side in (left, right))
+    exp = orc.jaccard_index(h1, h2, 4, nthreads=8).values.view(np.uint32)
+    h1, h2 = (HostStringsColumn.from_pylist([t for t, n in zip(side, times) for _ in range(n)]) for side in (left, right))
+    got = nv.jaccard_index(dev(nv, h1), dev(nv, h2), 4).to_host()
+    assert np.array_equal(got.values.view(np.uint32), np.repeat(exp, times))
+
+
 def mixed_rows(rng, lens, nulls=()):
     """Rows of these lengths as a column; the rows named in `nulls` are null (and empty)."""
     lens = np.array(lens, np.int64)
