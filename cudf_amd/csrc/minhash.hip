@@ -252,7 +252,7 @@ struct MinimaAll {
   int lane;
 
   static constexpr int kLeast = 0;
-  __device__ __forceinline__ MinimaAll(Lds*, int lane_, bool) : lane(lane_) {}
+  __device__ __forceinline__ MinimaAll(Lds*, int lane_, int32_t) : lane(lane_) {}
   __device__ __forceinline__ int32_t stride() const { return kParams; }
   __device__ __forceinline__ int32_t slots() const { return kSlots; }
   __device__ __forceinline__ void load(Params<T> const& p, int32_t chunk)
@@ -336,16 +336,15 @@ struct Minima64 {
   };
   Params<T> params;
   int32_t base;    // first parameter of the chunk
-  int32_t groups;  // of the chunk: GROUPS or kLeast
+  int32_t groups;  // of the chunk: GROUPS, or fewer in a column with too few units of work for all wavefronts
   uint32_t warm;   // (see load)
   Lds* lds;
   int lane;
-  static constexpr int kLeast = GROUPS < 2 ? GROUPS : 2;  // groups of a chunk in a column with too few units of work for all wavefronts
+  static constexpr int kLeast = GROUPS < 2 ? GROUPS : 2;  // groups that a chunk has at least
 
-  __device__ __forceinline__ Minima64(Lds* lds_, int lane_, bool few) : groups(few ? kLeast : GROUPS), warm(0), lds(lds_), lane(lane_) {}
+  __device__ __forceinline__ Minima64(Lds* lds_, int lane_, int32_t groups_) : groups(groups_ != 0 ? groups_ : GROUPS), warm(0), lds(lds_), lane(lane_) {}
   __device__ __forceinline__ int32_t stride() const { return slots(); }  // parameters from a chunk to the next
   __device__ __forceinline__ int32_t slots() const { return groups * filter64::kGroup; }
-  static __device__ __forceinline__ int32_t chunks_of_least(int32_t count) { return (count + kLeast * filter64::kGroup - 1) / (kLeast * filter64::kGroup); }
   // What the first groups have in memory is asked for here, a cache line a lane, and waited for where it is used: the plan has
   // just written it, and a read then takes two microseconds.
   __device__ __forceinline__ void load(Params<T> const& p, int32_t chunk)
@@ -918,21 +917,27 @@ __global__ void __launch_bounds__(kThreads, (simd_waves<Source, Minima>())) minh
   bool one_counter;
   uint32_t const each   = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(parts.per_unit(total, min(params.count, Minima::kSlots), &one_counter))));
   uint32_t const units  = total / each + (total % each != 0 ? 1u : 0u);
-  // 64-bit hashes: chunks of two groups of parameters where the wavefronts suffice for that (the windows are hashed for each
-  // of them, by wavefronts that had nothing to do): 100 rows of 2000 bytes, 128 parameters 21 -> 18 us;
+  // 64-bit hashes: chunks of two groups of parameters where the wavefronts suffice for that, or else of four (the windows are hashed for each
+  // of them, by wavefronts that had nothing to do): 100 rows of 2000 bytes, 128 parameters 21 -> 18 us, 260 parameters, in fours,
+  // 32 -> 27; 700 of 300, 256 parameters 31 -> 27;
   // with twice or four times as many units as wavefronts it is no gain: 50 rows of 16 KB 33.2 us whole, 36.4 in chunks of two groups
-  bool few = false;
+  int32_t in_chunk_groups = 0;  // 0: as many as the minima are made for
   if constexpr (Minima::kLeast != 0) {
-    int32_t const least = Minima::chunks_of_least(params.count);
-    few                 = static_cast<uint64_t>(units) * static_cast<uint32_t>(least) <= static_cast<uint64_t>(parts.waves);
-    if (few) chunks = least;
+    if (units <= static_cast<uint32_t>(parts.waves)) {
+      uint32_t const waves = static_cast<uint32_t>(parts.waves), whole = static_cast<uint32_t>(chunks);
+      uint32_t const groups = static_cast<uint32_t>(params.count + filter64::kGroup - 1) / filter64::kGroup, twos = (groups + 1) / 2, fours = (groups + 3) / 4;
+      if (twos > whole && units * twos <= waves)
+        in_chunk_groups = 2, chunks = static_cast<int32_t>(twos);
+      else if (fours > whole && units * fours <= waves)
+        in_chunk_groups = 4, chunks = static_cast<int32_t>(fours);
+    }
   }
   uint64_t const all    = static_cast<uint64_t>(units) * static_cast<uint32_t>(chunks);
   int const lane        = lane_id();
   int const wave        = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
   uint32_t const me     = blockIdx.x * kWaves + static_cast<uint32_t>(wave);
   uint32_t chunk        = 0;
-  Minima minima(&minima_lds[wave], lane, few);
+  Minima minima(&minima_lds[wave], lane, in_chunk_groups);
   minima.load(params, 0);
   for (uint64_t unit = me; unit < all;) {
     while (unit >= static_cast<uint64_t>(chunk + 1u) * units) minima.load(params, static_cast<int32_t>(++chunk));  // (the next chunk of parameters)

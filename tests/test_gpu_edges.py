@@ -199,6 +199,16 @@ def test_minhash_parts_of_rows(nv, orc, bits, count):
         assert call(dev(nv, host), 5, a, b, 5).to_host().equals(ref(host, 5, a, b, 5, nthreads=8))
 
 
+@pytest.mark.parametrize("count", [96, 129, 256, 260, 520])
+@pytest.mark.parametrize("rows", [100, 450, 700, 1100, 2200])
+def test_minhash64_chunks_of_groups(nv, orc, rows, count):
+    """Columns in which the wavefronts suffice for two groups of 32 parameters each, for four, and for neither."""
+    rng = np.random.default_rng(rows + count)
+    a, b = params(rng, count, 64)
+    host = mixed_rows(rng, rng.integers(1, 600, rows), nulls=(3,))
+    assert nv.minhash64(dev(nv, host), 5, a, b, 5).to_host().equals(orc.minhash64(host, 5, a, b, 5, nthreads=8))
+
+
 @pytest.mark.parametrize("bits", [32, 64])
 @pytest.mark.parametrize("count", [1, 64, 130, 260])
 def test_minhash_rows_of_thousands_of_parts(nv, orc, bits, count):
