@@ -103,48 +103,47 @@ struct PackedSet {
     }
   };
 
+  // left: a bit a lane.
   template <int N>
-  __device__ __forceinline__ void place_at(bool (&left)[N], const uint32_t (&h)[N], const uint32_t (&bucket)[N], const uint32_t (&distance)[N], Mark mark,
-                                           bool (&taken)[N]) const
+  __device__ __forceinline__ void place_at(uint64_t (&left)[N], const uint32_t (&value)[N], const uint32_t (&bucket)[N], const uint32_t (&distance)[N], Mark mark,
+                                           uint64_t (&taken)[N]) const
   {
     uint4 v[N];
-    uint32_t id[N], s[N], full[N], old[N];
-    bool tried[N];
+    uint32_t id[N], s[N], old[N];
+    uint64_t tried[N];
 #pragma unroll
     for (int k = 0; k < N; ++k) v[k] = reinterpret_cast<const uint4*>(slots)[bucket[k]];
     __builtin_amdgcn_sched_barrier(0);  // (all reads on their way before the first is waited for)
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-      id[k] = (product(h[k]) & kValue) | distance[k] << kDistanceAt;
+      id[k] = (value[k] & kValue) | distance[k] << kDistanceAt;
       // 1 as long as the slots so far hold other values (0 where one is empty or holds this one)
       uint32_t const a0 = least(1u, v[k].x, (v[k].x ^ id[k]) & kSame);
       uint32_t const a1 = least(a0, v[k].y, (v[k].y ^ id[k]) & kSame);
       uint32_t const a2 = least(a1, v[k].z, (v[k].z ^ id[k]) & kSame);
-      full[k]           = least(a2, v[k].w, (v[k].w ^ id[k]) & kSame);
       s[k]              = 4u * bucket[k] + (a0 + a1 + a2);
-      taken[k]          = full[k] != 0u;
-      tried[k]          = left[k] & !taken[k];
+      taken[k]          = ballot64(least(a2, v[k].w, (v[k].w ^ id[k]) & kSame) != 0u);
+      tried[k]          = left[k] & ~taken[k];
     }
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-      old[k] = id[k] ^ 1u;  // (another one)
+      asm("" : "=v"(old[k]));  // (of the lanes that try nothing it does not matter)
       // (also where the slot holds the value already: cheaper than telling the two apart first)
-      if (tried[k]) old[k] = atomicCAS(&slots[s[k]], 0u, id[k] | mark);
+      if (__builtin_amdgcn_inverse_ballot_w64(tried[k])) old[k] = atomicCAS(&slots[s[k]], 0u, id[k] | mark);
     }
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-      bool const there = tried[k] & (((old[k] ^ id[k]) & kSame) == 0u);
-      if (there) atomicOr(&slots[s[k]], mark);
-      left[k] = left[k] & !(there | (tried[k] & (old[k] == 0u)));  // (else another value came first)
+      uint64_t const there = tried[k] & ballot64(((old[k] ^ id[k]) & kSame) == 0u);
+      if (__builtin_amdgcn_inverse_ballot_w64(there)) atomicOr(&slots[s[k]], mark);
+      left[k] &= ~(there | (tried[k] & ballot64(old[k] == 0u)));  // (else another value came first)
     }
   }
-  static __device__ __forceinline__ uint32_t product(uint32_t h) { return h * 0x9E3779B1u; }
-  __device__ __forceinline__ uint32_t home(uint32_t h) const { return __umulhi(product(h), buckets); }
+  __device__ __forceinline__ uint32_t home(uint32_t value) const { return __umulhi(value, buckets); }
   // Buckets from one that is full to the next to be looked at: an odd number up to 31 that the value tells (by bits that a slot
   // holds, so that a slot still tells its home).  With 1 for all the full buckets grow together: at a load of 0.8 the last of 64
   // values put aside had to look at 12 to 15 buckets, now at 6, and the furthest of a pair was 57 from home, now 16.  Random letters,
   // in which no window repeats: 30,000 pairs of 2803-byte rows 1431 -> 820 us, 15,000 of 6100 1565 -> 917, 250,001 of 2 KB words 3515 -> 3490.
-  static __device__ __forceinline__ uint32_t step(uint32_t h) { return (product(h) & 15u) * 2u + 1u; }
+  static __device__ __forceinline__ uint32_t step(uint32_t value) { return (value & 15u) * 2u + 1u; }
   // (written out: the compiler makes a comparison and a selection of the minimum with 1)
   static __device__ __forceinline__ uint32_t least(uint32_t a, uint32_t b, uint32_t c)
   {
@@ -172,49 +171,57 @@ struct PlainSet {
   uint32_t *in1, *in2;
 
   __device__ __forceinline__ Mark mark(bool second) const { return second ? in2 : in1; }
-  __device__ __forceinline__ uint32_t home(uint32_t h) const { return __umulhi(h * 0x9E3779B1u, buckets); }
+  __device__ __forceinline__ uint32_t home(uint32_t value) const { return __umulhi(value, buckets); }
   static __device__ __forceinline__ uint32_t step(uint32_t) { return 1u; }  // (every bucket is come by)
   template <int N>
-  __device__ __forceinline__ void place_at(bool (&left)[N], const uint32_t (&h)[N], const uint32_t (&bucket)[N], const uint32_t (&)[N], Mark in,
-                                           bool (&taken)[N]) const
+  __device__ __forceinline__ void place_at(uint64_t (&left)[N], const uint32_t (&value)[N], const uint32_t (&bucket)[N], const uint32_t (&)[N], Mark in,
+                                           uint64_t (&taken)[N]) const
   {
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-      taken[k] = false;
-      if (!left[k]) continue;
-      uint32_t s = 4u * bucket[k], v = 0;
-      for (int j = 0; j < 4; ++j, ++s) {
-        v = set_word<IN_LDS>(&slots[s]);
-        if (v == 0u) v = atomicCAS(&slots[s], 0u, h[k]);
-        if (v == 0u || v == h[k]) break;
+      bool full = false, in_set = false;
+      if (__builtin_amdgcn_inverse_ballot_w64(left[k])) {
+        uint32_t s = 4u * bucket[k], v = 0;
+        for (int j = 0; j < 4; ++j, ++s) {
+          v = set_word<IN_LDS>(&slots[s]);
+          if (v == 0u) v = atomicCAS(&slots[s], 0u, value[k]);
+          if (v == 0u || v == value[k]) break;
+        }
+        full = s == 4u * bucket[k] + 4u;
+        if (!full) {
+          atomicOr(&in[s >> 5], 1u << (s & 31u));
+          in_set = true;
+        }
       }
-      taken[k] = s == 4u * bucket[k] + 4u;
-      if (!taken[k]) {
-        atomicOr(&in[s >> 5], 1u << (s & 31u));
-        left[k] = false;
-      }
+      taken[k] = ballot64(full);
+      left[k] &= ~ballot64(in_set);
     }
   }
 };
 
-// From its home bucket on, until the value is in the set.  false: no place.
+// By all lanes: from its home bucket on, until the value is in the set, for the lanes of `left`; what is left found no place.
 template <typename Set>
-__device__ __forceinline__ bool place(Set const& set, uint32_t value, typename Set::Mark mark)
+__device__ __forceinline__ uint64_t place(Set const& set, uint64_t left, uint32_t value, typename Set::Mark mark)
 {
-  uint32_t const h[1]  = {value};
-  uint32_t bucket[1]   = {set.home(value)}, distance[1] = {0u};
-  uint32_t const most  = min(set.buckets, Set::kFar);
-  while (distance[0] < most) {
-    bool left[1] = {true}, taken[1];
-    set.template place_at<1>(left, h, bucket, distance, mark, taken);
-    if (!left[0]) return true;
-    if (taken[0]) {
+  uint32_t const values[1] = {value};
+  uint32_t bucket[1]       = {set.home(value)}, distance[1] = {0u};
+  uint32_t const most      = min(set.buckets, Set::kFar), step = Set::step(value);
+  uint64_t lost            = 0;
+  while (left != 0) {
+    uint64_t l[1] = {left}, taken[1];
+    set.template place_at<1>(l, values, bucket, distance, mark, taken);
+    left = l[0];
+    // on to the next bucket where this one is full (else another value came first: once more, at most until the bucket is full)
+    if (__builtin_amdgcn_inverse_ballot_w64(taken[0])) {
       ++distance[0];
-      bucket[0] += Set::step(value);
+      bucket[0] += step;
       if (bucket[0] >= set.buckets) bucket[0] -= set.buckets;
-    }  // (else another value came first: once more, at most until the bucket is full)
+    }
+    uint64_t const beyond = left & ballot64(distance[0] >= most);
+    lost |= beyond;
+    left &= ~beyond;
   }
-  return false;
+  return lost;
 }
 
 // A share of the hashes by value, for pairs that are cut into parts (other bits than the set's own multiplication uses).  A part
@@ -323,6 +330,48 @@ __device__ __host__ __forceinline__ uint64_t slots_for_global(int64_t bytes)
   return s;
 }
 
+// What a set holds for a hash: its product with an odd number (0 for 0, and no two alike).  The compiler does not see what it is,
+// or it multiplies once more for the 24 bits that a slot keeps.
+__device__ __forceinline__ uint32_t value_of(uint32_t h)
+{
+  uint32_t v = h * 0x9E3779B1u;
+  asm("" : "+v"(v));
+  return v;
+}
+
+// murmur3_x86_32_unmixed() with seed 0.  Windows in a tile of up to eleven bytes: no loop over their blocks, and every aligned
+// dword read once, from one address.
+template <int BLOCKS, int N>
+__device__ __forceinline__ void few_blocks(WordSrc const (&src)[N], uint32_t len, uint32_t (&h)[N])
+{
+  uint32_t const c1 = 0xcc9e2d51u, c2 = 0x1b873593u, rem = len & 3u;
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    h[n] = 0;
+#pragma unroll
+    for (int i = 0; i < BLOCKS; ++i) h[n] = rotl32(h[n] ^ (rotl32(src[n].dword(i) * c1, 15) * c2), 13) * 5u + 0xe6546b64u;
+    if (rem) h[n] ^= rotl32(keep_low_bytes(src[n].dword(BLOCKS), static_cast<int>(rem)) * c1, 15) * c2;
+    h[n] ^= len;
+  }
+}
+template <int N, typename Src>
+__device__ __forceinline__ void window_hashes(Src const (&src)[N], uint32_t len, uint32_t (&h)[N])
+{
+  murmur3_x86_32_unmixed(src, len, 0u, h);
+}
+template <int N>
+__device__ __forceinline__ void window_hashes(WordSrc const (&src)[N], uint32_t len, uint32_t (&h)[N])
+{
+  if (N == 1 || len >= 12)
+    murmur3_x86_32_unmixed(src, len, 0u, h);
+  else if (len >= 8)
+    few_blocks<2>(src, len, h);
+  else if (len >= 4)
+    few_blocks<1>(src, len, h);
+  else
+    few_blocks<0>(src, len, h);
+}
+
 // Hashes the windows of both rows (jaccard.cu:249-292) and inserts the non-zero hashes into the set.  The two rows, one list
 // of units of 64 window starts, are shared out evenly among `nwaves` wavefronts, which take up to kTile starts of a row at a
 // time.  (Whole tiles in turn left some of four wavefronts a tile more than the others: pairs of 0.8 to 3.3 KB 5 % slower.)
@@ -333,8 +382,8 @@ template <typename Set>
 __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2, Pair const& pair, int32_t width, Set const& set, Part part, TileLds& lds,
                                             int wave, int nwaves, int lane)
 {
-  auto const hash = [](auto const& src, uint32_t len, auto& h) { murmur3_x86_32_unmixed(src, len, 0u, h); };  // jaccard.cu:258: seed 0
-  bool ok         = true;
+  auto const hash = [](auto const& src, uint32_t len, auto& h) { window_hashes(src, len, h); };  // jaccard.cu:258: seed 0
+  uint64_t lost   = 0;  // (a bit a lane)
   if (static_cast<int64_t>(width) * 4 <= kHalo) {
     int32_t const n1 = static_cast<int32_t>(pair.n1), n2 = static_cast<int32_t>(pair.n2);  // (1.43 GB together at most)
     const uint8_t *const row1 = c1.chars + pair.o1, *const row2 = c2.chars + pair.o2;
@@ -344,7 +393,10 @@ __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2
     bool second    = false;
     auto const place_later = [&] {
       if (!second) later1 = later;
-      for (uint32_t i = lane; i < later; i += kWave) ok = place(set, lds.later[i], set.mark(i >= later1)) && ok;
+      for (uint32_t i = lane; i - lane < later; i += kWave) {
+        bool const have = i < later;
+        lost |= place(set, ballot64(have), have ? lds.later[i] : 0u, set.mark(i >= later1));
+      }
       later = later1 = 0;
     };
     struct At {
@@ -384,22 +436,23 @@ __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2
       };
       hash_tile_windows<uint32_t>(tile, next, a.row, a.n, 0, true, a.base, a.cnt, width, lds.bytes, lds.chars, lane, hash, [&](auto const& valid, auto const& hv) {
         constexpr int N = sizeof(hv) / sizeof(hv[0]);
-        bool left[N], taken[N];
-        uint32_t bucket[N], home[N];
+        uint64_t left[N], taken[N];
+        uint32_t value[N], bucket[N], home[N];
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-          left[k]   = valid[k] & (hv[k] != 0u) & part.holds(hv[k]);  // 282-286: zero hashes are dropped
-          bucket[k] = set.home(hv[k]);
+          left[k]   = ballot64(valid[k]) & ballot64(hv[k] != 0u) & ballot64(part.holds(hv[k]));  // 282-286: zero hashes are dropped
+          value[k]  = value_of(hv[k]);
+          bucket[k] = set.home(value[k]);
           home[k]   = 0u;
         }
-        set.template place_at<N>(left, hv, bucket, home, mark, taken);
+        set.template place_at<N>(left, value, bucket, home, mark, taken);
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-          uint64_t const which = ballot64(left[k]);
-          if (which != 0) {
-            if (later + static_cast<uint32_t>(__builtin_popcountll(which)) > kLater) place_later();
-            if (left[k]) lds.later[later + lanes_below(which)] = hv[k];
-            later += static_cast<uint32_t>(__builtin_popcountll(which));
+          if (left[k] != 0) {
+            uint32_t const more = static_cast<uint32_t>(__builtin_popcountll(left[k]));
+            if (later + more > kLater) place_later();
+            if (__builtin_amdgcn_inverse_ballot_w64(left[k])) lds.later[later + lanes_below(left[k])] = value[k];
+            later += more;
           }
         }
       });
@@ -407,26 +460,25 @@ __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2
       if (later >= kWave) place_later();
     }
     place_later();
-    return ok;
+    return lost == 0;
   }
   // very wide windows: bytes straight from global memory
 #pragma nounroll
   for (int row = 0; row < 2; ++row) {
     const uint8_t* const r = row == 0 ? c1.chars + pair.o1 : c2.chars + pair.o2;
     int64_t const n        = row == 0 ? pair.n1 : pair.n2;
-    for (int64_t gpos = static_cast<int64_t>(wave) * kWave + lane; gpos < n; gpos += nwaves * kWave) {
-      int64_t const remaining = n - gpos;
+    for (int64_t at = static_cast<int64_t>(wave) * kWave; at < n; at += nwaves * kWave) {
+      int64_t const gpos = at + lane, remaining = n - gpos;
       BoundedSrc const src[1] = {{r + gpos, remaining}};
-      uint32_t hlen;
-      uint32_t const readable = static_cast<uint32_t>(min(remaining, static_cast<int64_t>(width) * 4));
-      if (window_at(src[0], r + gpos, remaining, readable, gpos == 0, false, width, &hlen)) {
-        uint32_t hv[1];
-        hash(src, hlen, hv);
-        if (hv[0] != 0u && part.holds(hv[0])) ok = place(set, hv[0], set.mark(row != 0)) && ok;
+      uint32_t hv[1] = {0u}, hlen;
+      if (remaining > 0) {
+        uint32_t const readable = static_cast<uint32_t>(min(remaining, static_cast<int64_t>(width) * 4));
+        if (window_at(src[0], r + gpos, remaining, readable, gpos == 0, false, width, &hlen)) hash(src, hlen, hv);
       }
+      lost |= place(set, ballot64(hv[0] != 0u && part.holds(hv[0])), value_of(hv[0]), set.mark(row != 0));
     }
   }
-  return ok;
+  return lost == 0;
 }
 
 template <int WAVES>
