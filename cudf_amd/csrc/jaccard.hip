@@ -344,15 +344,26 @@ __device__ __forceinline__ uint32_t value_of(uint32_t h)
 template <int BLOCKS, int N>
 __device__ __forceinline__ void few_blocks(WordSrc const (&src)[N], uint32_t len, uint32_t (&h)[N])
 {
-  uint32_t const c1 = 0xcc9e2d51u, c2 = 0x1b873593u, rem = len & 3u;
+  auto const mixed = [](uint32_t k) { return rotl32(k * 0xcc9e2d51u, 15) * 0x1b873593u; };
+  uint32_t const rem = len & 3u;
+  uint32_t words[N][BLOCKS + 2];
 #pragma unroll
-  for (int n = 0; n < N; ++n) {
-    h[n] = 0;
+  for (int i = 0; i < BLOCKS + 2; ++i)
 #pragma unroll
-    for (int i = 0; i < BLOCKS; ++i) h[n] = rotl32(h[n] ^ (rotl32(src[n].dword(i) * c1, 15) * c2), 13) * 5u + 0xe6546b64u;
-    if (rem) h[n] ^= rotl32(keep_low_bytes(src[n].dword(BLOCKS), static_cast<int>(rem)) * c1, 15) * c2;
-    h[n] ^= len;
+    for (int n = 0; n < N; ++n) words[n][i] = src[n].at[i];
+  auto const dword = [&](int n, int i) { return __builtin_amdgcn_alignbit(words[n][i + 1], words[n][i], 8u * src[n].mis); };
+#pragma unroll
+  for (int n = 0; n < N; ++n) h[n] = 0;
+#pragma unroll
+  for (int i = 0; i < BLOCKS; ++i)
+#pragma unroll
+    for (int n = 0; n < N; ++n) h[n] = rotl32(h[n] ^ mixed(dword(n, i)), 13) * 5u + 0xe6546b64u;
+  if (rem) {
+#pragma unroll
+    for (int n = 0; n < N; ++n) h[n] ^= mixed(keep_low_bytes(dword(n, BLOCKS), static_cast<int>(rem)));
   }
+#pragma unroll
+  for (int n = 0; n < N; ++n) h[n] ^= len;
 }
 template <int N, typename Src>
 __device__ __forceinline__ void window_hashes(Src const (&src)[N], uint32_t len, uint32_t (&h)[N])

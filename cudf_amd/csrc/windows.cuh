@@ -237,20 +237,20 @@ __device__ __forceinline__ void hash_tile_windows(TileBytes& tile, Next&& next, 
   if (plain) {
     // (the last window of the row ends with it)
     uint32_t const starts_here = min(cnt, len - min(len, width_all - 1u));
-    uint32_t q = 0;
+    // (a lane beyond the last window hashes what lies there in the tile's LDS: no branch, and one address for both windows)
+    static_assert(kTile + kWave + kHalo / 4 + 32 <= 4 * kTileWords);
+    uint32_t const here = mis + lane;
+    uint32_t q          = 0;
     for (; q + kWave < starts_here; q += 2 * kWave) {
-      // (a lane beyond the last window hashes the bytes of that one: no branch)
-      uint32_t const p     = q + lane;
-      bool const valid[2]  = {true, p + kWave < starts_here};
-      WordSrc const src[2] = {WordSrc(bytes, mis + p), WordSrc(bytes, mis + min(p + kWave, starts_here - 1u))};
+      bool const valid[2]  = {true, q + kWave + lane < starts_here};
+      WordSrc const src[2] = {WordSrc(bytes + q / 4, here), WordSrc(bytes + q / 4 + kWave / 4, here)};
       T hv[2];
       hash(src, width_all, hv);
       sink(valid, hv);
     }
     if (q < starts_here) {
-      uint32_t const p     = q + lane;
-      bool const valid[1]  = {p < starts_here};
-      WordSrc const src[1] = {WordSrc(bytes, mis + min(p, starts_here - 1u))};
+      bool const valid[1]  = {q + lane < starts_here};
+      WordSrc const src[1] = {WordSrc(bytes + q / 4, here)};
       T hv[1];
       hash(src, width_all, hv);
       sink(valid, hv);
