@@ -103,6 +103,7 @@ struct PackedSet {
     }
   };
 
+  __device__ __forceinline__ uint32_t* at(uint32_t offset) const { return reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(slots) + offset); }
   // left: a bit a lane.
   template <int N>
   __device__ __forceinline__ void place_at(uint64_t (&left)[N], const uint32_t (&value)[N], const uint32_t (&bucket)[N], const uint32_t (&distance)[N], Mark mark,
@@ -121,7 +122,8 @@ struct PackedSet {
       uint32_t const a0 = least(1u, v[k].x, (v[k].x ^ id[k]) & kSame);
       uint32_t const a1 = least(a0, v[k].y, (v[k].y ^ id[k]) & kSame);
       uint32_t const a2 = least(a1, v[k].z, (v[k].z ^ id[k]) & kSame);
-      s[k]              = 4u * bucket[k] + (a0 + a1 + a2);
+      s[k]              = 16u * bucket[k] + 4u * (a0 + a1 + a2);
+      asm("" : "+v"(s[k]));  // (one address for both atomics)
       taken[k]          = ballot64(least(a2, v[k].w, (v[k].w ^ id[k]) & kSame) != 0u);
       tried[k]          = left[k] & ~taken[k];
     }
@@ -129,12 +131,12 @@ struct PackedSet {
     for (int k = 0; k < N; ++k) {
       asm("" : "=v"(old[k]));  // (of the lanes that try nothing it does not matter)
       // (also where the slot holds the value already: cheaper than telling the two apart first)
-      if (__builtin_amdgcn_inverse_ballot_w64(tried[k])) old[k] = atomicCAS(&slots[s[k]], 0u, id[k] | mark);
+      if (__builtin_amdgcn_inverse_ballot_w64(tried[k])) old[k] = atomicCAS(at(s[k]), 0u, id[k] | mark);
     }
 #pragma unroll
     for (int k = 0; k < N; ++k) {
       uint64_t const there = tried[k] & ballot64(((old[k] ^ id[k]) & kSame) == 0u);
-      if (__builtin_amdgcn_inverse_ballot_w64(there)) atomicOr(&slots[s[k]], mark);
+      if (__builtin_amdgcn_inverse_ballot_w64(there)) atomicOr(at(s[k]), mark);
       left[k] &= ~(there | (tried[k] & ballot64(old[k] == 0u)));  // (else another value came first)
     }
   }
@@ -373,6 +375,8 @@ __device__ __forceinline__ void window_hashes(Src const (&src)[N], uint32_t len,
 template <int N>
 __device__ __forceinline__ void window_hashes(WordSrc const (&src)[N], uint32_t len, uint32_t (&h)[N])
 {
+  // (one length for all windows; what is branched on is told from it anew: the compiler keeps the answers in lanes of vector registers)
+  if constexpr (N > 1) asm volatile("" : "+s"(len));
   if (N == 1 || len >= 12)
     murmur3_x86_32_unmixed(src, len, 0u, h);
   else if (len >= 8)
