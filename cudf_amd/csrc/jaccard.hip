@@ -391,9 +391,11 @@ __device__ __forceinline__ void window_hashes(WordSrc const (&src)[N], uint32_t 
 // of units of 64 window starts, are shared out evenly among `nwaves` wavefronts, which take up to kTile starts of a row at a
 // time.  (Whole tiles in turn left some of four wavefronts a tile more than the others: pairs of 0.8 to 3.3 KB 5 % slower.)
 // false: a value found no place.
+// FOUR: a lane hashes four windows of a whole tile at a time and not two, so that fewer waits for LDS are left where a SIMD has no more than
+// six wavefronts (43,934 pairs of 5.6 to 12.4 KB 1026 -> 978 us; with four wavefronts a pair and seven a SIMD 725 -> 757).
 // Nearly every hash finds its place with one look at one bucket, but in most rounds of 64 some lane does not: those are
 // put aside and placed 64 at a time, so that a round does not wait for its slowest lane.
-template <typename Set>
+template <bool FOUR = false, typename Set>
 __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2, Pair const& pair, int32_t width, Set const& set, Part part, TileLds& lds,
                                             int wave, int nwaves, int lane)
 {
@@ -449,7 +451,7 @@ __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2
           fetch(ahead);
         }
       };
-      hash_tile_windows<uint32_t>(tile, next, a.row, a.n, 0, true, a.base, a.cnt, width, lds.bytes, lds.chars, lane, hash, [&](auto const& valid, auto const& hv) {
+      hash_tile_windows<uint32_t, FOUR>(tile, next, a.row, a.n, 0, true, a.base, a.cnt, width, lds.bytes, lds.chars, lane, hash, [&](auto const& valid, auto const& hv) {
         constexpr int N = sizeof(hv) / sizeof(hv[0]);
         uint64_t left[N], taken[N];
         uint32_t value[N], bucket[N], home[N];
@@ -573,7 +575,7 @@ __device__ __forceinline__ bool count_pair(ColView const& c1, ColView const& c2,
 {
   int const lane = lane_id();
   int const wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
-  bool const ok  = insert_pair(c1, c2, pair, width, PackedSet{slots, nslots / 4}, part, scratch.tile[wave], wave, WAVES, lane);
+  bool const ok  = insert_pair<(WAVES >= 12)>(c1, c2, pair, width, PackedSet{slots, nslots / 4}, part, scratch.tile[wave], wave, WAVES, lane);
   if (!ok) scratch.full = number;
   __syncthreads();
   bool const full = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(scratch.full))) == number;
@@ -936,7 +938,7 @@ __global__ void __launch_bounds__(kTeamWaves * kWave) jaccard_teams_kernel(ColVi
     for (;;) {
       if (lane == 0) scratch.full[wave] = 0u;
       __syncthreads();  // (the set is empty, the flags are down, the sums of the piece before have been read)
-      bool const ok = insert_pair(c1, c2, pair, width, PackedSet{set, nslots / 4}, part.share(), scratch.tile[wave], own, waves, lane);
+      bool const ok = insert_pair<true>(c1, c2, pair, width, PackedSet{set, nslots / 4}, part.share(), scratch.tile[wave], own, waves, lane);
       if (!ok) scratch.full[wave - own] = 1u;
       if (threadIdx.x == 0) scratch.next = next;
       __syncthreads();

@@ -212,12 +212,13 @@ __device__ __forceinline__ bool window_at(Src const& src, const uint8_t* g, int6
 // lane of the wavefront calls together, with arrays of one window per lane or of two (two chains of LDS reads and multiplies
 // in flight instead of one).  `bytes` and `chars` are the wavefront's own LDS.  starts: `row` is the row's first byte.  Places
 // have 32 bits, which take half the scalar registers and instructions; `beyond` more bytes than n belong to a row that is
-// longer.  tile: the row's bytes from base on, tile_length() of them; when they are in LDS, next() may ask for others.
+// longer.  tile: the row's bytes from base on, tile_length() of them; when they are in LDS, next() may ask for others.  FOUR: sink()
+// takes four windows a lane as well, from whole tiles.
 __device__ __forceinline__ uint32_t tile_length(int32_t n, int32_t base, uint32_t cnt, int32_t width)
 {
   return min(static_cast<uint32_t>(n - base), cnt + static_cast<uint32_t>(width) * 4u);
 }
-template <typename T, typename Next, typename Hash, typename Sink>
+template <typename T, bool FOUR = false, typename Next, typename Hash, typename Sink>
 __device__ __forceinline__ void hash_tile_windows(TileBytes& tile, Next&& next, const uint8_t* row, int32_t n, int64_t beyond, bool starts, int32_t base, uint32_t cnt,
                                                   int32_t width, uint32_t* bytes, uint16_t* chars, int lane, Hash const& hash, Sink&& sink)
 {
@@ -241,6 +242,17 @@ __device__ __forceinline__ void hash_tile_windows(TileBytes& tile, Next&& next, 
     static_assert(kTile + kWave + kHalo / 4 + 32 <= 4 * kTileWords);
     uint32_t const here = mis + lane;
     uint32_t q          = 0;
+    if constexpr (FOUR) {
+      static_assert(kTile == 4 * kWave);
+      if (starts_here > 3u * kWave) {
+        bool const valid[4]  = {true, true, true, 3 * kWave + lane < starts_here};
+        WordSrc const src[4] = {WordSrc(bytes, here), WordSrc(bytes + kWave / 4, here), WordSrc(bytes + 2 * kWave / 4, here), WordSrc(bytes + 3 * kWave / 4, here)};
+        T hv[4];
+        hash(src, width_all, hv);
+        sink(valid, hv);
+        q = kTile;
+      }
+    }
     for (; q + kWave < starts_here; q += 2 * kWave) {
       bool const valid[2]  = {true, q + kWave + lane < starts_here};
       WordSrc const src[2] = {WordSrc(bytes + q / 4, here), WordSrc(bytes + q / 4 + kWave / 4, here)};
