@@ -321,7 +321,8 @@ __device__ __forceinline__ Pair uniform_pair_at(ColView const& c1, ColView const
 // Slots for a pair: room for twice its windows, which are at most its bytes, or what the tier has.
 __device__ __forceinline__ uint32_t slots_for(int64_t bytes, uint32_t most)
 {
-  return static_cast<uint32_t>(min(static_cast<int64_t>(most), max((2 * bytes + 63) / 32 * 32, static_cast<int64_t>(PackedSet::kLeast))));
+  uint32_t const few = static_cast<uint32_t>(min(bytes, static_cast<int64_t>(most)));
+  return min(most, max((2u * few + 63u) / 32u * 32u, PackedSet::kLeast));
 }
 
 // ... and in global memory: room for one and a half times its windows.
@@ -405,7 +406,8 @@ __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2
     int32_t const n1 = static_cast<int32_t>(pair.n1), n2 = static_cast<int32_t>(pair.n2);  // (1.43 GB together at most)
     const uint8_t *const row1 = c1.chars + pair.o1, *const row2 = c2.chars + pair.o2;
     int32_t const units1 = (n1 + kWave - 1) / kWave, units = units1 + (n2 + kWave - 1) / kWave;
-    int32_t const last   = static_cast<int32_t>(static_cast<int64_t>(units) * (wave + 1) / nwaves);
+    // (22 million units at most, times sixteen)
+    int32_t const last   = static_cast<int32_t>(static_cast<uint32_t>(units) * static_cast<uint32_t>(wave + 1) / static_cast<uint32_t>(nwaves));
     uint32_t later = 0, later1 = 0;  // hashes put aside, and how many of them (the first ones) are row 1's: the same in every lane
     bool second    = false;
     auto const place_later = [&] {
@@ -434,7 +436,7 @@ __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2
     };
     TileBytes tile;  // asked for a tile ahead
     auto const fetch = [&](At const& a) { tile.fetch(a.row + a.base, tile_length(a.n, a.base, a.cnt, width), lane); };
-    int32_t const first = static_cast<int32_t>(static_cast<int64_t>(units) * wave / nwaves);
+    int32_t const first = static_cast<int32_t>(static_cast<uint32_t>(units) * static_cast<uint32_t>(wave) / static_cast<uint32_t>(nwaves));
     At ahead{};
     if (first < last) {
       ahead = tile_at(first);
