@@ -7,8 +7,8 @@
 // Here a row pair needs no sort and no temporary: the window hashes of both rows go into ONE open-addressing set in
 // LDS whose slots also say "seen in row 1" and "seen in row 2".  |A|, |B| and |A n B| are then counts of these marks.
 //
-// What bounds it: vector instructions, some 100 per 64 windows, a third of them the hash, issued in three quarters of the
-// cycles, and LDS, busy for half of the time; HBM sees the chars once.  Hence
+// What bounds it: vector and scalar instructions, 70 and 62 per 64 windows, and LDS, each busy for 50 to 60 % of the time; HBM sees the
+// chars once.  Hence
 //   * buckets of four slots, read with one 16-byte LDS read: a probe seldom goes on to a second bucket, for which the whole
 //     wavefront would wait; what one look does not place is put aside and placed 64 at a time;
 //   * value and marks in one word (PackedSet): no address and no mask to be made for a mark;
@@ -22,7 +22,8 @@
 //     which hash the whole pair and keep their part (hashing is the cheap half); the counts of the parts add up.  Only
 //     pairs beyond that use a set in global memory, whose atomics run at a fiftieth of the rate (1,600 such pairs among
 //     250,000 of 2 KB rows: 3.7 of the call's 9.6 ms before the parts).
-// 250,001 pairs of 2 KB rows (1.02 GB): 4.08 ms with whole values, bits in arrays and tiles in turn, 3.5 ms now (290 GB/s).
+// 250,001 pairs of 2 KB rows (1.02 GB): 4.08 ms with whole values, bits in arrays and tiles in turn, 3.5 with a hundred vector instructions
+// per 64 windows, 2.95 ms now (347 GB/s).
 #include "common.cuh"
 #include "murmur.cuh"
 #include "windows.cuh"
@@ -62,16 +63,16 @@ __device__ __forceinline__ int list_of(int64_t bytes)
   return list < kPartsList ? list : parts_of(bytes) <= kMaxParts ? kPartsList : kGlobalList;
 }
 
-// Insert-only sets of non-zero uint32 values, in buckets of four slots that fill from the first to the last.  A value's home
-// bucket is what the top of its product with an odd number says.  place_at() has one look at bucket home + distance for each of
+// Insert-only sets of non-zero uint32 values (products of hashes, see value_of), in buckets of four slots that fill from the first to
+// the last.  A value's home bucket is what its top says.  place_at() has one look at bucket home + distance for each of
 // N values: `left` stays where the value is not in the set now, marked as its row's; `taken` tells whether the bucket is full
 // of others, so that the next one is to be looked at.
 //
-// The set of a pair whose windows LDS has room for.  A slot holds 24 bits of the value's product, which tell the values of one
+// The set of a pair whose windows LDS has room for.  A slot holds the low 24 bits of the value, which tell the values of one
 // home bucket apart where there are 256 buckets and more, how many steps from home it lies (6 bits), and two bits that say
 // which rows it occurs in: one compare-and-swap places a value and marks it, where that finds the value there already it is marked with
 // an or of a constant to the same address, and counting is a pass over the slots.  (With whole values and the bits in arrays
-// of their own a look took 65 vector instructions for 128 windows, beside 65 for their hashes; now 55.)
+// of their own a look took 65 vector instructions for 128 windows; now 50, beside 30 for the hashes of windows of five bytes.)
 struct PackedSet {
   static constexpr uint32_t kValue    = 0x00FFFFFFu;
   static constexpr uint32_t kFar      = 64;  // steps from home that can be told
