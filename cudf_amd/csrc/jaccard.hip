@@ -389,6 +389,14 @@ __device__ __forceinline__ void window_hashes(WordSrc const (&src)[N], uint32_t 
     few_blocks<0>(src, len, h);
 }
 
+// A number of wavefronts: known when this is compiled (an int), or a power of two.
+struct TeamOf {
+  int shift;
+  __device__ __forceinline__ operator int() const { return 1 << shift; }
+};
+__device__ __forceinline__ uint32_t share_of(uint32_t units, int waves) { return units / static_cast<uint32_t>(waves); }
+__device__ __forceinline__ uint32_t share_of(uint32_t units, TeamOf waves) { return units >> waves.shift; }
+
 // Hashes the windows of both rows (jaccard.cu:249-292) and inserts the non-zero hashes into the set.  The two rows, one list
 // of units of 64 window starts, are shared out evenly among `nwaves` wavefronts, which take up to kTile starts of a row at a
 // time.  (Whole tiles in turn left some of four wavefronts a tile more than the others: pairs of 0.8 to 3.3 KB 5 % slower.)
@@ -397,9 +405,9 @@ __device__ __forceinline__ void window_hashes(WordSrc const (&src)[N], uint32_t 
 // six wavefronts (43,934 pairs of 5.6 to 12.4 KB 1026 -> 978 us; with four wavefronts a pair and seven a SIMD 725 -> 757).
 // Nearly every hash finds its place with one look at one bucket, but in most rounds of 64 some lane does not: those are
 // put aside and placed 64 at a time, so that a round does not wait for its slowest lane.
-template <bool FOUR = false, typename Set>
+template <bool FOUR = false, typename Set, typename Waves>
 __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2, Pair const& pair, int32_t width, Set const& set, Part part, TileLds& lds,
-                                            int wave, int nwaves, int lane)
+                                            int wave, Waves nwaves, int lane)
 {
   auto const hash = [](auto const& src, uint32_t len, auto& h) { window_hashes(src, len, h); };  // jaccard.cu:258: seed 0
   uint64_t lost   = 0;  // (a bit a lane)
@@ -408,7 +416,7 @@ __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2
     const uint8_t *const row1 = c1.chars + pair.o1, *const row2 = c2.chars + pair.o2;
     int32_t const units1 = (n1 + kWave - 1) / kWave, units = units1 + (n2 + kWave - 1) / kWave;
     // (22 million units at most, times sixteen)
-    int32_t const last   = static_cast<int32_t>(static_cast<uint32_t>(units) * static_cast<uint32_t>(wave + 1) / static_cast<uint32_t>(nwaves));
+    int32_t const last   = static_cast<int32_t>(share_of(static_cast<uint32_t>(units) * static_cast<uint32_t>(wave + 1), nwaves));
     uint32_t later = 0, later1 = 0;  // hashes put aside, and how many of them (the first ones) are row 1's: the same in every lane
     bool second    = false;
     auto const place_later = [&] {
@@ -437,7 +445,7 @@ __device__ __forceinline__ bool insert_pair(ColView const& c1, ColView const& c2
     };
     TileBytes tile;  // asked for a tile ahead
     auto const fetch = [&](At const& a) { tile.fetch(a.row + a.base, tile_length(a.n, a.base, a.cnt, width), lane); };
-    int32_t const first = static_cast<int32_t>(static_cast<uint32_t>(units) * static_cast<uint32_t>(wave) / static_cast<uint32_t>(nwaves));
+    int32_t const first = static_cast<int32_t>(share_of(static_cast<uint32_t>(units) * static_cast<uint32_t>(wave), nwaves));
     At ahead{};
     if (first < last) {
       ahead = tile_at(first);
@@ -631,7 +639,7 @@ constexpr uint32_t kOnceMore = 0x80000000u;  // (rows are fewer)
 // and, on a cache line that nobody reads (63,333 pairs of twice 6000 bytes 3348 -> 3246 us), [kNextPiece] = pieces of work handed out
 // -- then four counters (|A|, |B|, |A n B|, parts done) for
 // every entry of the list of pairs in parts, `rows` entries for each list, and the first kMostParts of the parts themselves
-// (a pair's entry | its number << 27).
+// (a pair's entry | its number << 27, and the pair).
 constexpr int kListHeader = 64;
 constexpr int kToldWords  = 16;  // of the header, that the host is told
 constexpr int kMostBytes  = 8;
@@ -644,10 +652,12 @@ __host__ __device__ __forceinline__ uint32_t most_parts(int64_t rows)
 {
   return rows < kMostParts / kMaxParts ? static_cast<uint32_t>(rows * kMaxParts) : kMostParts;
 }
-__host__ __device__ __forceinline__ size_t work_words(int64_t rows) { return kListHeader + static_cast<size_t>(kLists + 4) * static_cast<size_t>(rows) + most_parts(rows); }
+__host__ __device__ __forceinline__ size_t work_words(int64_t rows) { return kListHeader + static_cast<size_t>(kLists + 4) * static_cast<size_t>(rows) + 2 * static_cast<size_t>(most_parts(rows)); }
 __device__ __forceinline__ uint32_t* list_entries(uint32_t* work, int list, int64_t rows) { return work + kListHeader + (4 + list) * rows; }
 __device__ __forceinline__ uint32_t* part_counters(uint32_t* work) { return work + kListHeader; }
-__device__ __forceinline__ uint32_t* single_parts(uint32_t* work, int64_t rows) { return work + kListHeader + (kLists + 4) * rows; }
+// (the lists are an even number of words: 8-byte records, aligned)
+static_assert((kLists + 4) % 2 == 0);
+__device__ __forceinline__ uint2* single_parts(uint32_t* work, int64_t rows) { return reinterpret_cast<uint2*>(work + kListHeader + (kLists + 4) * rows); }
 struct WaveSetLds {
   alignas(16) uint32_t slots[kSlots[0]];
   TileLds tile;
@@ -700,7 +710,7 @@ __global__ void __launch_bounds__(kThreads) jaccard_wave_kernel(ColView c1, ColV
     if (list == kPartsList) {
       reinterpret_cast<uint4*>(part_counters(work))[at] = make_uint4(0u, 0u, 0u, 0u);
       uint32_t const parts = static_cast<uint32_t>(parts_of(bytes)), first = atomicAdd(&counts[kTotalParts], parts);
-      for (uint32_t p = 0; p < parts && first + p < most_parts(rows); ++p) single_parts(work, rows)[first + p] = at | p << 27;
+      for (uint32_t p = 0; p < parts && first + p < most_parts(rows); ++p) single_parts(work, rows)[first + p] = make_uint2(at | p << 27, static_cast<uint32_t>(r));
     }
     if (list == kGlobalList) atomicMax(reinterpret_cast<unsigned long long*>(&counts[kMostBytes]), static_cast<unsigned long long>(bytes));
   };
@@ -870,11 +880,11 @@ __global__ void __launch_bounds__(kTierWaves[kPartsTier] * kWave) jaccard_parts_
   for (uint32_t piece = blockIdx.x; piece < pieces;) {
     uint32_t ahead = 0;
     if (threadIdx.x == 0) ahead = atomicAdd(&work[kNextPiece], 1u) + gridDim.x;
-    uint32_t const e = known ? single_parts(work, rows)[piece] : 0u;
-    uint32_t const i = known ? e & 0x07FFFFFFu : piece / kMaxParts;
-    uint32_t const r = list_entries(work, kPartsList, rows)[i];
+    uint2 const e    = known ? single_parts(work, rows)[piece] : make_uint2(0u, 0u);
+    uint32_t const i = known ? e.x & 0x07FFFFFFu : piece / kMaxParts;
+    uint32_t const r = known ? e.y : list_entries(work, kPartsList, rows)[i];
     Pair const pair  = uniform_pair_at(c1, c2, r);
-    Part part{known ? e >> 27 : piece % static_cast<uint32_t>(kMaxParts), static_cast<uint32_t>(parts_of(pair.bytes()))};
+    Part part{known ? e.x >> 27 : piece % static_cast<uint32_t>(kMaxParts), static_cast<uint32_t>(parts_of(pair.bytes()))};
     if (part.part < part.parts) {
       uint32_t sum[3] = {0, 0, 0};
       for (bool more = true; more;) {
@@ -904,10 +914,13 @@ __global__ void __launch_bounds__(kTierWaves[kPartsTier] * kWave) jaccard_parts_
 // pieces, 213 and 267).
 struct Pieces {
   uint32_t parts, tier4, tier3, tier2, tier1;  // where the pieces of each kind end
-  int waves2, waves1;                          // wavefronts of a team of the last two kinds
+  uint32_t pairs2, pairs1;                     // of the last two kinds
+  int shift2, shift1;                          // wavefronts of a team of these, their logarithm
 };
 constexpr uint32_t kTeamPieces = 1536;  // of the first three tiers at most
 constexpr int kTeamWaves       = kMostWaves;
+constexpr int kTeamShift       = 4;
+static_assert(kTeamWaves == 1 << kTeamShift);
 constexpr uint32_t kTeamSlots  = kSlots[kTiers - 1];
 struct TeamScratch {
   TileLds tile[kTeamWaves];
@@ -927,38 +940,38 @@ __global__ void __launch_bounds__(kTeamWaves * kWave) jaccard_teams_kernel(ColVi
   bool const more = pieces.tier1 > gridDim.x;
   for (uint32_t piece = blockIdx.x; piece < pieces.tier1;) {
     // the team's wavefronts, its share of the set, and the entry of its list that it has (none: `have` is false)
-    int waves = kTeamWaves, list = kPartsList;
+    int shift = kTeamShift, list = kPartsList;
     uint32_t most = kTeamSlots, entry = piece;
+    bool have     = true;
     if (piece >= pieces.tier2) {
-      waves = pieces.waves1, list = 0, most = kSlots[1];
-      entry = (piece - pieces.tier2) * (kTeamWaves / waves) + static_cast<uint32_t>(wave / waves);
+      shift = pieces.shift1, list = 0, most = kSlots[1];
+      entry = ((piece - pieces.tier2) << (kTeamShift - shift)) + (static_cast<uint32_t>(wave) >> shift);
+      have  = entry < pieces.pairs1;
     } else if (piece >= pieces.tier3) {
-      waves = pieces.waves2, list = 1, most = kSlots[2];
-      entry = (piece - pieces.tier3) * (kTeamWaves / waves) + static_cast<uint32_t>(wave / waves);
+      shift = pieces.shift2, list = 1, most = kSlots[2];
+      entry = ((piece - pieces.tier3) << (kTeamShift - shift)) + (static_cast<uint32_t>(wave) >> shift);
+      have  = entry < pieces.pairs2;
     } else if (piece >= pieces.tier4) {
       list = 2, most = kSlots[3], entry = piece - pieces.tier4;
     } else if (piece >= pieces.parts) {
       list = 3, entry = piece - pieces.parts;
     }
-    int const team      = wave / waves, own = wave % waves;
+    TeamOf const waves{shift};
+    int const team      = wave >> shift, own = wave & (waves - 1);
     uint32_t* const set = slots + static_cast<uint32_t>(team) * most;
     Part part{0, 1};
-    uint32_t counter = 0;
-    bool have        = true;
+    uint32_t counter = 0, r = 0;
     if (list == kPartsList) {
-      uint32_t const e = single_parts(work, rows)[piece];
-      counter          = e & 0x07FFFFFFu;
-      part.part        = e >> 27;
-      entry            = counter;
-    } else {
-      have = entry < work[list];
+      uint2 const e = single_parts(work, rows)[piece];
+      counter       = e.x & 0x07FFFFFFu;
+      part.part     = e.x >> 27;
+      r             = e.y;
+    } else if (have) {
+      r = list_entries(work, list, rows)[entry];
     }
-    uint32_t r = 0;
+    r = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(r)));
     Pair pair{0, 0, 0, 0};
-    if (have) {
-      r    = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(list_entries(work, list, rows)[entry])));
-      pair = uniform_pair_at(c1, c2, r);
-    }
+    if (have) pair = uniform_pair_at(c1, c2, r);
     if (list == kPartsList) part.parts = static_cast<uint32_t>(parts_of(pair.bytes()));
     uint32_t const nslots = list == kPartsList ? most : slots_for(pair.bytes(), most);
     uint32_t next = pieces.tier1;
@@ -1184,10 +1197,13 @@ nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* inpu
     // (fewer pieces than CUs: a workgroup for every pair)
     uint32_t const pairs = static_cast<uint32_t>(listed(2)) + static_cast<uint32_t>(listed(1)) + static_cast<uint32_t>(listed(0));
     bool const alone     = pieces.tier4 + pairs <= static_cast<uint32_t>(cus);
-    pieces.waves2        = alone ? kTeamWaves : kTierWaves[2];
-    pieces.waves1        = alone ? kTeamWaves : kTierWaves[1];
-    auto const teams_of  = [&](int list, int waves) { return static_cast<uint32_t>((listed(list) + kTeamWaves / waves - 1) / (kTeamWaves / waves)); };
-    uint32_t const n3 = teams_of(2, kTeamWaves), n2 = teams_of(1, pieces.waves2), n1 = teams_of(0, pieces.waves1);
+    static_assert(kTierWaves[2] == 8 && kTierWaves[1] == 4);
+    pieces.shift2        = alone ? kTeamShift : 3;
+    pieces.shift1        = alone ? kTeamShift : 2;
+    pieces.pairs2        = static_cast<uint32_t>(listed(1));
+    pieces.pairs1        = static_cast<uint32_t>(listed(0));
+    auto const teams_of  = [](uint32_t pairs, int shift) { return (pairs + (1u << (kTeamShift - shift)) - 1u) >> (kTeamShift - shift); };
+    uint32_t const n3 = static_cast<uint32_t>(listed(2)), n2 = teams_of(pieces.pairs2, pieces.shift2), n1 = teams_of(pieces.pairs1, pieces.shift1);
     few          = n3 + n2 + n1 <= kTeamPieces;
     pieces.tier3 = pieces.tier4 + (few ? n3 : 0u);
     pieces.tier2 = pieces.tier3 + (few ? n2 : 0u);
