@@ -2248,6 +2248,7 @@ __global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, Vo
                                                                uint32_t* __restrict__ hot, Arrivals* __restrict__ arrivals, HostPost post)
 {
   __shared__ uint32_t staged[(kSampleBytes + kSampleTail + 8) / 4 + 4];  // byte 4 + x of it: byte x of the window; byte 3: the one before
+  __shared__ uint16_t starts[kSampleBytes / 2];  // of its words
   int const lane      = lane_id();
   int64_t const first = col.off(0), last = col.off(col.size);
   int64_t const span    = last - first;
@@ -2257,15 +2258,27 @@ __global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, Vo
     int64_t const begin  = first + sample_begin(span, blockIdx.x);
     uint32_t const bytes = static_cast<uint32_t>(min(last, begin + kSampleBytes) - begin);
     uint8_t* const sb   = reinterpret_cast<uint8_t*>(staged);
+#pragma unroll
     for (int i = lane; i < 4 + kSampleBytes + kSampleTail + 8; i += kWave) {
       int64_t const g = begin + i - 4;
       sb[i]           = (g >= first && g < last) ? col.chars[g] : uint8_t{0x20};  // outside the view: a space
     }
     wave_lds_sync();
-    // a lane takes eight byte positions and the words that start there
+    // a lane finds the words that start at eight byte positions; then every lane takes one of them, and the next 64
     constexpr uint32_t kMine = kSampleBytes / kWave;
-    for (uint32_t p = kMine * lane; p < kMine * lane + kMine && p < bytes; ++p) {
-      if (sb[4 + p] == 0x20u || sb[3 + p] != 0x20u) continue;
+    uint32_t begins          = 0;
+    bool space               = sb[3 + kMine * lane] == 0x20u;
+#pragma unroll
+    for (uint32_t i = 0; i < kMine; ++i) {
+      bool const before = space;
+      space             = sb[4 + kMine * lane + i] == 0x20u;
+      if (before && !space && kMine * lane + i < bytes) begins |= 1u << i;
+    }
+    uint32_t const mine = __builtin_popcount(begins), upto = wave_inclusive_scan(mine), total = wave_bcast(upto, kWave - 1);
+    for (uint32_t at = upto - mine; begins != 0; begins &= begins - 1u) starts[at++] = static_cast<uint16_t>(kMine * lane + __builtin_ctz(begins));
+    wave_lds_sync();
+    for (uint32_t w = lane; w < total; w += kWave) {
+      uint32_t const p = starts[w];
       uint32_t len = 1;
       while (len < kMaxWord && sb[4 + p + len] != 0x20u) ++len;
       ++words;
