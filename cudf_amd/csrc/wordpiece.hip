@@ -2279,8 +2279,17 @@ __global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, Vo
     wave_lds_sync();
     for (uint32_t w = lane; w < total; w += kWave) {
       uint32_t const p = starts[w];
-      uint32_t len = 1;
-      while (len < kMaxWord && sb[4 + p + len] != 0x20u) ++len;
+      TileWord const tw{staged, 4u + p};
+      uint32_t k[4];
+      tw.head16(k);
+      // its length: the first space
+      uint32_t len = 16;
+#pragma unroll
+      for (int d = 3; d >= 0; --d) {
+        uint32_t const x = k[d] ^ 0x20202020u, spaces = (x - 0x01010101u) & ~x & 0x80808080u;
+        if (spaces != 0) len = 4u * d + (static_cast<uint32_t>(__builtin_ctz(spaces)) >> 3);
+      }
+      while (len >= 16 && len < kMaxWord && sb[4 + p + len] != 0x20u) ++len;
       ++words;
       if (len >= kMaxWord) continue;  // one unknown token, never queued
       if (len > 16) {
@@ -2288,9 +2297,6 @@ __global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, Vo
         continue;
       }
       // queued as the word pass queues: whatever the word's home bucket does not settle
-      TileWord const tw{staged, 4u + p};
-      uint32_t k[4];
-      tw.head16(k);
       trim_key8(min(len, 8u), k[0], k[1]);
       trim_key8(len > 8 ? len - 8u : 0u, k[2], k[3]);
       Probe const pr = make_probe(table, 0u, tw, 0u, len, k[0], k[1]);
