@@ -965,10 +965,13 @@ __device__ __forceinline__ uint32_t count_word_starts(const uint4* abase, int64_
   return total;
 }
 
-// range_first_row[g] = the first row (0..rows) that starts at or after the first byte of range g; [nranges] = rows.
+// range_first_row[g] = the first row (0..rows) that starts at or after the first byte of range g; [nranges] = rows.  Eight lanes
+// search for a range, an eighth of what is left each time (a lane a range reads twenty times, one after the other: 25 MB
+// in rows of 120 bytes 7.9 -> 5.3 us, 200 MB in rows of 500 9.3 -> 6.8, with sixteen lanes 8.9).
 // The first workgroup also sets the flag words of the call: zeros, but for the work counters, which start past the
 // units that the wavefronts take by their place in the grid (counter g serves the wavefronts g, g + kCounterGroups, ..
 // and hands out the units g, g + kCounterGroups, ..).
+constexpr int kSearchLanes = 8;
 __global__ void range_first_row_kernel(ColView col, int64_t first_offset, uint32_t cbeg, int64_t range_bytes, uint32_t nranges,
                                        uint32_t* __restrict__ range_first_row, uint32_t* __restrict__ flags, uint32_t word_waves,
                                        uint32_t oov_waves, uint32_t word_waves2, uint32_t* __restrict__ memo_owners)
@@ -987,16 +990,22 @@ __global__ void range_first_row_kernel(ColView col, int64_t first_offset, uint32
       flags[i] = v;
     }
   }
-  uint32_t const g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g > nranges) return;
+  uint32_t const g     = (blockIdx.x * blockDim.x + threadIdx.x) / kSearchLanes, member = threadIdx.x % kSearchLanes;
   int64_t const target = static_cast<int64_t>(g) * range_bytes;
-  uint32_t lo = 0, hi = static_cast<uint32_t>(col.size);
-  if (g == nranges) lo = hi;
-  while (lo < hi) {
-    uint32_t const mid = lo + ((hi - lo) >> 1);
-    if (col.off(mid) - first_offset + cbeg < target) lo = mid + 1;
-    else hi = mid;
+  uint32_t lo = 0, hi = g < nranges ? static_cast<uint32_t>(col.size) : 0u;  // the answer lies in [lo, hi]
+  while (ballot64(lo < hi) != 0) {
+    // row hi is at or after the byte; the group's rows lie evenly before it
+    uint32_t const length = hi - lo, at = lo + static_cast<uint32_t>(static_cast<uint64_t>(length) * member / kSearchLanes);
+    bool const before     = lo < hi && col.off(at) - first_offset + cbeg < target;
+    uint32_t const n      = __builtin_popcount(static_cast<uint32_t>(ballot64(before) >> (lane_id() & ~(kSearchLanes - 1))) & ((1u << kSearchLanes) - 1u));
+    if (lo >= hi) continue;
+    // (the first n of them are before it)
+    uint32_t const from = lo;
+    if (n > 0) lo = from + static_cast<uint32_t>(static_cast<uint64_t>(length) * (n - 1) / kSearchLanes) + 1u;
+    if (n < kSearchLanes) hi = from + static_cast<uint32_t>(static_cast<uint64_t>(length) * n / kSearchLanes);
   }
+  if (g == nranges) lo = static_cast<uint32_t>(col.size);
+  if (g > nranges || member != 0) return;
   range_first_row[g] = lo;
 }
 
@@ -3039,7 +3048,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     uint4* const memo      = temps.part<uint4>(9);
     uint32_t* const owners = memo_entries ? reinterpret_cast<uint32_t*>(memo + kMemoEntries) : nullptr;
     args.memo_count        = flags + kFlagMemo;
-    hipLaunchKernelGGL(range_first_row_kernel, dim3((nranges + 1 + 255) / 256), dim3(256), 0, stream, v, first_offset, cbeg, kRange, nranges, first_row,
+    hipLaunchKernelGGL(range_first_row_kernel, dim3((nranges + 1) / (256 / kSearchLanes) + 1), dim3(256), 0, stream, v, first_offset, cbeg, kRange, nranges, first_row,
                        flags, word_grid * kWordWaves, oov_grid * kOovWaves, word_grid2 * kWordWaves, owners);
     for (int part = 0; part < (word_grid2 > 0 ? 2 : 1); ++part) {
       args.unit_begin = part == 0 ? 0u : first_part;

@@ -480,6 +480,27 @@ def test_tokenize_chunks_of_the_queue(nv, orc, rows, oov):
     assert nv.wordpiece_tokenize(dev(nv, host), vocabulary, 0).to_host().equals(orc.wordpiece_tokenize(host, reference, 0, nthreads=8))
 
 
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("shape", ["first", "last", "middle", "empty between", "even", "short"])
+def test_tokenize_rows_of_ranges(nv, orc, shape, wide):
+    """Where the rows of every range begin: all bytes in one row of 140,003, runs of empty rows, ranges with no row's beginning and
+    ranges with thousands, of a column and of a slice of it."""
+    rng = np.random.default_rng(len(shape))
+    hv = HostStringsColumn.from_pylist(VOCABULARY)
+    vocabulary, reference = nv.WordPieceVocabulary(dev(nv, hv)), orc.Vocabulary(hv)
+    rows = 140_003
+    lens = {"even": np.full(rows, 9), "short": rng.integers(0, 3, rows), "empty between": np.where(np.arange(rows) % 10_000 < 9_990, 0, 997)}.get(shape)
+    if lens is None:
+        lens = np.zeros(rows, np.int64)
+        lens[{"first": 0, "last": rows - 1, "middle": 70_001}[shape]] = 300_000
+    offsets = np.concatenate([[0], np.cumsum(lens)])
+    chars = words_column(rng, [int(offsets[-1])], VOCABULARY, 0.1).chars[: int(offsets[-1])]
+    host = HostStringsColumn(chars, offsets.astype(np.int64 if wide else np.int32), None, rows, 0, 0)
+    for lo in (0, 3):
+        part = HostStringsColumn(host.chars, host.offsets, None, rows - lo, lo, 0)
+        assert nv.wordpiece_tokenize(dev(nv, host).slice(lo, rows, 0), vocabulary, 5).to_host().equals(orc.wordpiece_tokenize(part, reference, 5, nthreads=8))
+
+
 @pytest.mark.parametrize("letters", ["ab", "aé", "漢字b", "a\U0001F600"])
 @pytest.mark.parametrize("rows", [900, 140_000])
 def test_tokenize_words_longer_than_a_window(nv, orc, letters, rows):
