@@ -579,6 +579,24 @@ HostPost new_post();  // (only where host_scalars() gives memory)
 // Returns when it has been sent, or with the error that keeps it from being sent.
 hipError_t wait_for_post(HostPost const& post, hipStream_t stream);
 
+// By LANES neighbouring lanes (`member` is a lane's number among them; the whole wavefront comes along): the first of [lo, hi) that is not
+// before(i), or hi; all of them look at once, an even distance apart, and a LANES-th of what was left remains.
+template <int LANES, typename Before>
+__device__ __forceinline__ uint32_t search_by_lanes(uint32_t lo, uint32_t hi, uint32_t member, Before const& before)
+{
+  while (ballot64(lo < hi) != 0) {
+    auto const place     = [length = hi - lo, lo](uint32_t i) { return lo + static_cast<uint32_t>(static_cast<uint64_t>(length) * i / LANES); };
+    bool const yes       = lo < hi && before(place(member));
+    uint32_t const n     = __builtin_popcount(static_cast<uint32_t>(ballot64(yes) >> (lane_id() & ~(LANES - 1))) & ((1u << LANES) - 1u));  // the first n
+    uint32_t const first = n > 0 ? place(n - 1u) + 1u : lo, last = n < LANES ? place(n) : hi;
+    if (lo < hi) {
+      lo = first;
+      hi = last;
+    }
+  }
+  return lo;
+}
+
 // What the workgroups of one launch add up between them, so that the last to arrive knows the sum and need not be another
 // kernel: `sum` counts them in its upper bits.  Zeros between launches, which the last workgroup sees to.  Every host thread has
 // one of its own on every device (device memory of the library, no allocation; nullptr for more than kMostArrivals threads at a

@@ -993,17 +993,7 @@ __global__ void range_first_row_kernel(ColView col, int64_t first_offset, uint32
   uint32_t const g     = (blockIdx.x * blockDim.x + threadIdx.x) / kSearchLanes, member = threadIdx.x % kSearchLanes;
   int64_t const target = static_cast<int64_t>(g) * range_bytes;
   uint32_t lo = 0, hi = g < nranges ? static_cast<uint32_t>(col.size) : 0u;  // the answer lies in [lo, hi]
-  while (ballot64(lo < hi) != 0) {
-    // row hi is at or after the byte; the group's rows lie evenly before it
-    uint32_t const length = hi - lo, at = lo + static_cast<uint32_t>(static_cast<uint64_t>(length) * member / kSearchLanes);
-    bool const before     = lo < hi && col.off(at) - first_offset + cbeg < target;
-    uint32_t const n      = __builtin_popcount(static_cast<uint32_t>(ballot64(before) >> (lane_id() & ~(kSearchLanes - 1))) & ((1u << kSearchLanes) - 1u));
-    if (lo >= hi) continue;
-    // (the first n of them are before it)
-    uint32_t const from = lo;
-    if (n > 0) lo = from + static_cast<uint32_t>(static_cast<uint64_t>(length) * (n - 1) / kSearchLanes) + 1u;
-    if (n < kSearchLanes) hi = from + static_cast<uint32_t>(static_cast<uint64_t>(length) * n / kSearchLanes);
-  }
+  lo = search_by_lanes<kSearchLanes>(lo, hi, member, [&](uint32_t row) { return col.off(row) - first_offset + cbeg < target; });
   if (g == nranges) lo = static_cast<uint32_t>(col.size);
   if (g > nranges || member != 0) return;
   range_first_row[g] = lo;

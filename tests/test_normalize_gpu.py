@@ -350,3 +350,20 @@ def test_normalize_lines_between_the_ways(nv, onorm, kind, rows, tiles):
     offsets = np.concatenate([[0], np.sort(rng.integers(0, chars.size, rows - 1)), [chars.size]]).astype(np.int32)
     host = HostStringsColumn(chars, offsets, None, rows, 0, 0)
     assert_same(run(nv, host, True, ("[SEP]",)), onorm.normalize_characters_native(host, True, [b"[SEP]"], 8), f"{rows} {tiles}")
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("shape", ["first", "last", "middle", "empty between", "even", "short"])
+def test_normalize_rows_of_tiles(nv, onorm, shape, wide):
+    """Where the rows of every tile begin: all bytes in one row of 140,003, runs of empty rows, tiles with no row's beginning and
+    tiles with thousands."""
+    rng = np.random.default_rng(len(shape))
+    rows = 140_003
+    lens = {"even": np.full(rows, 9), "short": rng.integers(0, 3, rows), "empty between": np.where(np.arange(rows) % 10_000 < 9_990, 0, 997)}.get(shape)
+    if lens is None:
+        lens = np.zeros(rows, np.int64)
+        lens[{"first": 0, "last": rows - 1, "middle": 70_001}[shape]] = 300_000
+    offsets = np.concatenate([[0], np.cumsum(lens)])
+    chars = np.resize(np.frombuffer("Some words, and more of them. ".encode(), np.uint8), int(offsets[-1]))
+    host = HostStringsColumn(chars, offsets.astype(np.int64 if wide else np.int32), None, rows, 0, 0)
+    assert_same(run(nv, host, True, ()), onorm.normalize_characters_native(host, True, [], 8), shape)
