@@ -132,7 +132,7 @@ def test_jaccard_lists_of_few_and_many_pairs(nv, orc, copies):
 @pytest.mark.parametrize("width", [2, 7, 40])
 def test_jaccard_pair_sizes(nv, orc, width):
     """Pairs of the most bytes that each set takes (4/5 of its slots) and of one more, around one
-    and several parts of 20,000 bytes, and around the most parts (16); no window repeats, so the sets are as full as they get."""
+    and several parts of 20,000 bytes, and around sixteen parts; no window repeats, so the sets are as full as they get."""
     rng = np.random.default_rng(width)
     sizes = [n * 4 // 5 + d for n in JACCARD_SLOTS for d in (0, 1)]
     sizes += [40_000, 40_001, 60_001, 320_000, 320_001, 1, 2, 63, 64, 65]
@@ -597,7 +597,7 @@ def test_tokenize_words_met_before(nv, orc, different, limit, wide):
 @pytest.mark.parametrize("rows, each", [(1, 1), (3, 2047), (3, 2048), (61, 300), (4, 65_535), (4, 65_537), (131_072, 9), (131_073, 9), (30_000, 2300)])
 @pytest.mark.parametrize("brackets", [True, False])
 def test_normalize_where_small_columns_end(nv, rows, each, brackets):
-    """Tiles of 2048 bytes and their remainders, and the bytes (256 KiB; 64 MiB) and rows up to which a column is worked on
+    """Tiles of 2048 bytes and their remainders, and the bytes (256 KiB; 20 MiB) and rows up to which a column is worked on
     before its size is known; a view of it too.  With a special token in every tile, which is then written the long way, and
     without."""
     from oracle import normalize_py

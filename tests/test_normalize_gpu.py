@@ -329,8 +329,8 @@ def test_normalize_rows_of_a_wavefronts_tile(nv, onorm, per_tile):
 
 @pytest.mark.parametrize("rows, tiles", [(131_072, 12288), (131_072, 12287), (40_000, 16384)])
 def test_normalize_wavefront_a_tile_after_one_wait(nv, onorm, rows, tiles):
-    """Columns of few enough rows and bytes (64 MiB) to be worked on before their size is known, and of so many tiles that a
-    wavefront writes each; one tile less."""
+    """Columns of few enough rows to be worked on before their size is known, but of more than the 20 MiB up to which they are;
+    a wavefront does each of their tiles."""
     rng = np.random.default_rng(rows + tiles)
     chars = np.resize(np.frombuffer("Some [SEP] words, Été 漢字 Жи 각 and more plain words of text. ".encode(), np.uint8), tiles * TILE)
     offsets = np.concatenate([[0], np.sort(rng.integers(0, tiles * TILE, rows - 1)), [tiles * TILE]]).astype(np.int32)
