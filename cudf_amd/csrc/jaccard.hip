@@ -636,15 +636,17 @@ constexpr uint32_t kOnceMore = 0x80000000u;  // (rows are fewer)
 
 // Work lists in `work`: a header -- [i] = pairs on list i, [kLists] = null rows of the result,
 // [8..9] = the most bytes a pair of the global list has (64 bits), [kTotalParts] = parts of all pairs on the list of pairs in parts,
-// and, on a cache line that nobody reads (63,333 pairs of twice 6000 bytes 3348 -> 3246 us), [kNextPiece] = pieces of work handed out
-// -- then four counters (|A|, |B|, |A n B|, parts done) for
+// and, on a cache line that nobody reads (63,333 pairs of twice 6000 bytes 3348 -> 3246 us), pieces of work handed out by each of
+// the two kernels that hand some out ([kNextPiece], [kNextPart]: where there are more than kMostParts parts both of them run) -- then
+// four counters (|A|, |B|, |A n B|, parts done) for
 // every entry of the list of pairs in parts, `rows` entries for each list, and the first kMostParts of the parts themselves
 // (a pair's entry | its number << 27, and the pair).
 constexpr int kListHeader = 64;
 constexpr int kToldWords  = 16;  // of the header, that the host is told
 constexpr int kMostBytes  = 8;
 constexpr int kTotalParts = 10;
-constexpr int kNextPiece  = 32;
+constexpr int kNextPiece  = 32;  // jaccard_teams_kernel
+constexpr int kNextPart   = 48;  // jaccard_parts_kernel
 constexpr int32_t kLookRows = 131072;  // see nvtext_amd_jaccard_index
 constexpr uint32_t kMostParts = 1u << 16;  // (of pairs of 0.8 GB and more)
 static_assert(kMostParts <= 1u << 27 && kMaxParts <= 32);
@@ -879,7 +881,7 @@ __global__ void __launch_bounds__(kTierWaves[kPartsTier] * kWave) jaccard_parts_
   uint32_t number = 0;
   for (uint32_t piece = blockIdx.x; piece < pieces;) {
     uint32_t ahead = 0;
-    if (threadIdx.x == 0) ahead = atomicAdd(&work[kNextPiece], 1u) + gridDim.x;
+    if (threadIdx.x == 0) ahead = atomicAdd(&work[kNextPart], 1u) + gridDim.x;
     uint2 const e    = known ? single_parts(work, rows)[piece] : make_uint2(0u, 0u);
     uint32_t const i = known ? e.x & 0x07FFFFFFu : piece / kMaxParts;
     uint32_t const r = known ? e.y : list_entries(work, kPartsList, rows)[i];

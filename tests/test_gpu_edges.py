@@ -165,6 +165,33 @@ def test_jaccard_many_parts(nv, orc, copies, sizes):
     assert np.array_equal(got.values.view(np.uint32), np.repeat(exp, times))
 
 
+@pytest.fixture
+def filled_memory(monkeypatch):
+    """Results and temporaries hold ones in all bits (NaN) when a call gets them: what it leaves unwritten cannot pass for an answer."""
+    import torch
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *args, **kw: empty(*args, **kw).fill_(255) if kw.get("dtype") == torch.uint8 else empty(*args, **kw))
+
+
+@pytest.mark.parametrize("copies, others", [(33_000, {15_000: 300}), (33_000, {12_400: 2000, 21_000: 3000}),
+                                            (34_000, {500: 2000, 2000: 300, 4000: 300, 9000: 300, 15_000: 300, 61_000: 10, 640_001: 2}),
+                                            (33_000, {700: 1000, 2500: 9000, 5000: 2000, 9000: 2000, 12_391: 700})])
+def test_jaccard_more_parts_than_their_list_beside_other_pairs(nv, orc, filled_memory, copies, others):
+    """Columns of at most 131,072 pairs with more parts than have a place on their list (65,536), and more pieces of other work than
+    there are CUs: pairs of the largest set, pairs for every set and in global memory, and so many of the smaller ones that the sets have
+    kernels of their own."""
+    rng = np.random.default_rng(copies)
+    times = {23_600: copies, **others}
+    rows = [random_text(rng, n).decode() for n in times]
+    left, right = [t[: len(t) // 3] for t in rows], [t[len(t) // 4:] for t in rows]
+    left[0], right[0] = rows[0][:11_800], rows[0][11_800:]
+    exp = orc.jaccard_index(*(HostStringsColumn.from_pylist(side) for side in (left, right)), 4, nthreads=8).values.view(np.uint32)
+    order = rng.permutation(np.repeat(np.arange(len(rows)), list(times.values())))
+    h1, h2 = (HostStringsColumn.from_pylist([side[i] for i in order]) for side in (left, right))
+    got = nv.jaccard_index(dev(nv, h1), dev(nv, h2), 4).to_host()
+    assert np.array_equal(got.values.view(np.uint32), exp[order])
+
+
 def mixed_rows(rng, lens, nulls=()):
     """Rows of these lengths as a column; the rows named in `nulls` are null (and empty)."""
     lens = np.array(lens, np.int64)
