@@ -743,8 +743,10 @@ std::atomic<int> g_forced_range_tiles{0};
 std::atomic<int> g_sizing_sample{1};
 constexpr int kRangeTiles    = 8;     // tiles per range at most (a large column); a small column has fewer, so that every wavefront gets several ranges
 constexpr int kOverBlocks    = 16;   // 16-byte blocks staged past the tile: a word that starts in the tile ends in them, or is kMaxWord bytes or more
-// In the launch for a small column a word of 8 to kOovMore tokens has two records: tok[6] of the first says which the second is, whose
-// eight words are tokens 6, 7, ..
+// In the launch for a small column a word of 8 to kOovMore tokens has two records: the second, with tokens 7, 8, .., lies as far behind
+// the first as there are first ones, for every word a place.  (Were they taken from the places that a tile has for its unknown words,
+// a tile of many such words would have too few: 7.5 MB of 60 words of eight tokens a tile were done twice, 113 us instead of 59, of
+// 113 such words three times, 500 instead of 169, and 1 MB of those twice, 134 instead of 38.)
 // Queue entries that a wavefront of the word pass reserves at a time, in a large column and at least.  What a wavefront has
 // left in the end are records that the out-of-vocabulary pass reads to find nothing in them: where six thousand wavefronts
 // meet a few hundred unknown words each, chunks of 512 were mostly such (with the counters of QueueChunks, 128,000 rows of 500 bytes
@@ -832,6 +834,7 @@ struct TileArgs {
   int32_t* offsets_out;    // per row: words of its range before the row
   OovEntry* queue;
   uint32_t queue_cap;
+  uint32_t queue_seconds;  // INLINE: from a word's first record to its second
   uint32_t queue_shift;    // a chunk of the queue is so many entries (a power of two)
   uint32_t* queue_chunks;  // kCounterGroups counters of the chunks handed out (see QueueChunks)
   uint32_t* counter;       // next range to hand out
@@ -1004,11 +1007,12 @@ __global__ void range_first_row_kernel(ColView col, int64_t first_offset, uint32
 // 245 us, 32 MB 211 against 286, 48 MB 300 against 319, 60 MB 359 against 337), after which the passes' better use of the
 // lanes tells; it stops at 32 MB for its temporaries.
 // These are sized for the bytes that a column of so many rows is guessed to have at most, kSmallGuess a row (kSmallSure in
-// any case), and for kSmallLeastSlots and kSmallLeastQueue of every tile of that;
+// any case), and for kSmallLeastSlots and kSmallLeastQueue of every tile of that, with a second record for each first;
 // the tiles that there are share them out, up to kSmallSlots and kSmallQueue each.  A column of more bytes (up to
 // kSmallRowBytes a row and kSmallBytes in all), or with a tile that needs more, is done once more, in what its bytes take.  (32,768 rows of 120 bytes held 224 MB where room for 32 MB
 // of text with a word per two bytes was set aside, and 31 MB this way, 45 us both; 8,192 rows of 3000 bytes, done once more,
-// 182 MB instead of 241 and 162 us instead of 150; the passes of a large column take 197 MB and 258 us.)
+// 182 MB instead of 241 and 162 us instead of 150; the passes of a large column take 197 MB and 258 us.  With the second records
+// these two hold 48 and 266 MB.)
 constexpr int32_t kSmallRows        = 131072;
 constexpr int64_t kSmallRowBytes    = 4096;
 constexpr int64_t kSmallGuess       = 256;
@@ -1186,7 +1190,7 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
     uint32_t open_left  = 0;  // words the row that runs into the tile may still have (with a word limit)
     uint32_t* const region = a.arena + static_cast<int64_t>(range) * a.range_cap;
     bool spill             = false;
-    bool again             = false;  // INLINE: a word of more tokens than its record keeps
+    bool again             = false;  // INLINE: a word of more tokens than its records keep
     if constexpr (INLINE) {
       q_pos = range * a.queue_cap;
       q_lim = q_pos + a.queue_cap;
@@ -1536,7 +1540,6 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
             }
           }
           uint32_t const place = lanes_below(qm);
-          uint32_t seconds     = 0;  // INLINE: second records
           uint32_t const q     = place < room ? q_pos + place : fresh + (place - room);
           if (queued) value = kOovMark | q;
           if (c < listed && !spill) region[cursor + (entry >> 21)] = value;
@@ -1565,26 +1568,18 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
                 count = tokenize_window_word(table, trim, tw, wl, keep_token);
               }
               oov_tokens += count;
-              // (second records lie behind the round's first ones)
-              bool const two        = count > kOovKeep && count <= kOovMore;
-              uint64_t const twos   = ballot64(two);
-              uint32_t const second = nq + lanes_below(twos);
-              seconds               = static_cast<uint32_t>(__builtin_popcountll(twos));
               if (count > kOovMore) again = true;
               if (place < room) {
                 uint4* const dst = reinterpret_cast<uint4*>(a.queue + q);
-                if (two) {
-                  auto const more = [&](int k) { return static_cast<uint32_t>(more_tokens[threadIdx.x / kWave][k][lane]); };
-                  dst[0] = make_uint4(static_cast<uint32_t>(tok[0]), static_cast<uint32_t>(tok[1]), static_cast<uint32_t>(tok[2]), static_cast<uint32_t>(tok[3]));
-                  dst[1] = make_uint4(static_cast<uint32_t>(tok[4]), static_cast<uint32_t>(tok[5]), q_pos + second, count);
-                  if (second < room) {
-                    uint4* const behind = reinterpret_cast<uint4*>(a.queue + q_pos + second);
-                    behind[0] = make_uint4(static_cast<uint32_t>(tok[6]), more(0), more(1), more(2));
-                    behind[1] = make_uint4(more(3), more(4), more(5), more(6));
-                  }
-                } else if (count <= kOovKeep) {
+                if (count <= kOovMore) {
                   dst[0] = make_uint4(static_cast<uint32_t>(tok[0]), static_cast<uint32_t>(tok[1]), static_cast<uint32_t>(tok[2]), static_cast<uint32_t>(tok[3]));
                   dst[1] = make_uint4(static_cast<uint32_t>(tok[4]), static_cast<uint32_t>(tok[5]), static_cast<uint32_t>(tok[6]), count);
+                  if (count > kOovKeep) {
+                    auto const more     = [&](int k) { return static_cast<uint32_t>(more_tokens[threadIdx.x / kWave][k][lane]); };
+                    uint4* const behind = reinterpret_cast<uint4*>(a.queue + a.queue_seconds + q);
+                    behind[0] = make_uint4(more(0), more(1), more(2), more(3));
+                    behind[1] = make_uint4(more(4), more(5), more(6), 0u);
+                  }
                 } else {  // (as the out-of-vocabulary pass leaves it)
                   dst[0] = make_uint4(0u, 0u, 0u, static_cast<uint32_t>(static_cast<uint64_t>(at) >> 32));
                   dst[1] = make_uint4(wl | (defer == 2u ? kUnprobed : 0u), range, static_cast<uint32_t>(at), count);
@@ -1597,13 +1592,8 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
                                                static_cast<uint32_t>(static_cast<uint64_t>(at) >> 32)));
             }
           }
-          if constexpr (INLINE) {
-            // (any lane that had a word knows their number)
-            if (nq != 0) seconds = wave_bcast(seconds, __builtin_ctzll(qm));
-            if (nq + seconds > room) spill = true;
-          }
           if (INLINE || nq <= room) {
-            q_pos += min(nq + seconds, room);
+            q_pos += min(nq, room);
           } else {
             q_pos = fresh + (nq - room);
             q_lim = fresh + (1u << a.queue_shift);
@@ -1999,7 +1989,7 @@ __global__ void __launch_bounds__(kTokThreads, SMALL ? 6 : 8) wordpiece_emit_ker
                                                                      const uint32_t* __restrict__ range_words, const int64_t* __restrict__ range_base,
                                                                      const uint32_t* __restrict__ block_tokens,
                                                                      const uint32_t* __restrict__ range_tokens, uint32_t block,
-                                                                     const uint32_t* __restrict__ range_first_row, OovEntry* __restrict__ queue,
+                                                                     const uint32_t* __restrict__ range_first_row, OovEntry* __restrict__ queue, uint32_t queue_seconds,
                                                                      int32_t* __restrict__ offsets, int32_t* __restrict__ child,
                                                                      uint32_t* __restrict__ again, uint32_t* __restrict__ again_count)
 {
@@ -2086,17 +2076,17 @@ __global__ void __launch_bounds__(kTokThreads, SMALL ? 6 : 8) wordpiece_emit_ker
       uint32_t const ex   = incl - (c0 + c1);  // tokens of the round before my first word
       uint32_t const tot  = wave_bcast(incl, kWave - 1);
       int32_t* const dst  = dst0 + done + ex;
-      // SMALL: tokens 6, 7, .. of words with two records (seldom; what the first says instead of token 6 may have been staged: it is overwritten)
+      // SMALL: tokens 7, 8, .. of words with two records (seldom)
       auto const second_records = [&](auto const& put) {
         if constexpr (SMALL) {
-          auto const of_word = [&](bool queued, uint32_t cnt, uint32_t record, uint32_t at) {
+          auto const of_word = [&](bool queued, uint32_t cnt, uint32_t slot, uint32_t at) {
             bool const two = queued && cnt > kOovKeep && cnt <= kOovMore;
             if (ballot64(two) == 0) return;
             if (two) {
-              const uint4* const behind = reinterpret_cast<const uint4*>(queue + record);
+              const uint4* const behind = reinterpret_cast<const uint4*>(queue + queue_seconds + (slot & ~kOovMark));
 #pragma unroll 1
-              for (uint32_t k = 6; k < cnt; k += 4) {
-                uint4 const c = behind[(k - 6) / 4];
+              for (uint32_t k = kOovKeep; k < cnt; k += 4) {
+                uint4 const c = behind[(k - kOovKeep) / 4];
                 put(at, k, c.x);
                 if (k + 1 < cnt) put(at, k + 1, c.y);
                 if (k + 2 < cnt) put(at, k + 2, c.z);
@@ -2104,8 +2094,8 @@ __global__ void __launch_bounds__(kTokThreads, SMALL ? 6 : 8) wordpiece_emit_ker
               }
             }
           };
-          of_word(q0, c0, rb0.z, ex);
-          of_word(q1, c1, rb1.z, ex + c0);
+          of_word(q0, c0, v.x, ex);
+          of_word(q1, c1, v.y, ex + c0);
         }
       };
       if (ballot64(q0 || q1) == 0) {
@@ -2120,7 +2110,7 @@ __global__ void __launch_bounds__(kTokThreads, SMALL ? 6 : 8) wordpiece_emit_ker
         // the tokens of the round side by side in LDS, then written 64 at a time
         auto stage_word = [&](bool active, bool queued, uint32_t slot, uint32_t cnt, uint4 const& ra, uint4 const& rb, uint32_t at) {
           if (queued && cnt > kMost) {
-            // more tokens than a record keeps (seldom): noted for wordpiece_retokenize_kernel, with the place of the
+            // more tokens than its records keep (seldom): noted for wordpiece_retokenize_kernel, with the place of the
             // word's first token in the child left in its record (what is written there now is overwritten then)
             uint32_t const q                  = slot & ~kOovMark;
             again[atomicAdd(again_count, 1u)] = q;
@@ -2149,7 +2139,7 @@ __global__ void __launch_bounds__(kTokThreads, SMALL ? 6 : 8) wordpiece_emit_ker
       } else {
         auto write_word = [&](bool active, bool queued, uint32_t slot, uint32_t cnt, uint4 const& ra, uint4 const& rb, int32_t* d) {
           if (queued && cnt > kMost) {
-            // more tokens than a record keeps (seldom): noted for wordpiece_retokenize_kernel, with the place of the
+            // more tokens than its records keep (seldom): noted for wordpiece_retokenize_kernel, with the place of the
             // word's first token in the child left in its record
             uint32_t const q                  = slot & ~kOovMark;
             again[atomicAdd(again_count, 1u)] = q;
@@ -2163,7 +2153,7 @@ __global__ void __launch_bounds__(kTokThreads, SMALL ? 6 : 8) wordpiece_emit_ker
                 if (queued && cnt > 3u) d[3] = static_cast<int32_t>(ra.w);
                 if (queued && cnt > 4u) d[4] = static_cast<int32_t>(rb.x);
                 if (queued && cnt > 5u) d[5] = static_cast<int32_t>(rb.y);
-                if (queued && cnt == 7u) d[6] = static_cast<int32_t>(rb.z);
+                if (queued && cnt > 6u) d[6] = static_cast<int32_t>(rb.z);
               }
             }
           }
@@ -2795,7 +2785,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
                                    static_cast<size_t>(most_ranges) * sizeof(uint32_t),
                                    kSmallGrid * sizeof(uint32_t),
                                    (static_cast<size_t>(records) + 1) * sizeof(uint32_t),
-                                   static_cast<size_t>(records) * sizeof(OovEntry)};
+                                   static_cast<size_t>(records) * 2 * sizeof(OovEntry)};
     TempParts<7> const temps(mr, temp_bytes);
     if (!temps.ok()) break;  // (no room: as for a large column)
     TileArgs args{};
@@ -2812,6 +2802,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     args.offsets_out   = out->offsets;
     args.queue         = temps.part<OovEntry>(6);
     args.queue_cap     = records;
+    args.queue_seconds = records;
     args.most_bytes    = small_bytes;
     args.arrivals      = arrivals;
     args.host          = scalars;
@@ -2849,7 +2840,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
       ProfileScope ps("wordpiece_emit_kernel", stream);
       hipLaunchKernelGGL(HIP_KERNEL_NAME(wordpiece_emit_kernel<true>), dim3((nranges + kTokWaves - 1) / kTokWaves), dim3(kTokThreads), 0, stream, nranges,
                          args.arena, small_slots(slots, nranges), args.range_words, static_cast<const int64_t*>(nullptr), args.block_tokens,
-                         args.range_tokens, small_block(nranges, grid), args.first_row_out, args.queue, out->offsets,
+                         args.range_tokens, small_block(nranges, grid), args.first_row_out, args.queue, records, out->offsets,
                          static_cast<int32_t*>(out->child), again_count + 1, again_count);
       if (scalars[3] & kNoteAgain)
         hipLaunchKernelGGL(wordpiece_retokenize_kernel, dim3(64), dim3(kRareThreads), 0, stream, vocabulary->table,
@@ -3117,7 +3108,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     {
       ProfileScope ps("wordpiece_emit_kernel", stream);
       hipLaunchKernelGGL(HIP_KERNEL_NAME(wordpiece_emit_kernel<false>), dim3(emit_grid), dim3(kTokThreads), 0, stream, nranges, arena, range_cap, words, bases,
-                         static_cast<const uint32_t*>(nullptr), static_cast<const uint32_t*>(nullptr), 1u, first_row, queue,
+                         static_cast<const uint32_t*>(nullptr), static_cast<const uint32_t*>(nullptr), 1u, first_row, queue, 0u,
                          out->offsets, static_cast<int32_t*>(out->child), longer, flags + kFlagAgain);
       // (the list of longer words has served its purpose by now: its memory takes the list of words to do again, at most
       // one entry per queued word)

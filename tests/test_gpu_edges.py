@@ -473,6 +473,42 @@ def test_tokenize_small_columns_again(nv, orc, megabytes, dense, limit):
     assert nv.wordpiece_tokenize(dev(nv, host), vocabulary, limit).to_host().equals(orc.wordpiece_tokenize(host, reference, limit, nthreads=8))
 
 
+def kernel_launches(call):
+    """What call() gives, and the kernels that the library timed for it."""
+    import torch
+    from cudf_amd import _capi
+    _capi.profile_enable(True)
+    _capi.profile_read()
+    try:
+        out = call()
+        torch.cuda.synchronize()
+        return out, [name for name, _ in _capi.profile_read()]
+    finally:
+        _capi.profile_enable(False)
+
+
+@pytest.mark.parametrize("sizes, kilobytes, small, large", [((16,), 7500, 1, 0), ((32, 34), 1000, 1, 0), ((16, 28), 1000, 1, 0), ((8,), 1000, 1, 0),
+                                                            ((7, 8, 14, 15, 28), 1000, 1, 0), ((7, 8), 7500, 2, 0), ((2, 3), 1000, 1, 1)])
+def test_tokenize_small_columns_of_words_of_many_tokens(nv, orc, sizes, kilobytes, small, large):
+    """Columns all of whose words have about eight tokens, or fourteen, and one more: as many as a tile has second records for, more,
+    and several times as many; that takes no launch more than what their number takes (a tile of 1000 KB has records for 128 words, of
+    7500 KB for 64 in the first launch and for 128 in the second; beyond it is a large column's way)."""
+    rng = np.random.default_rng(kilobytes + len(sizes))
+    letters = "abcdefgh"
+    pairs = [a + b for a in letters for b in letters] if min(sizes) > 15 else []
+    hv = HostStringsColumn.from_pylist(["[UNK]"] + list(letters) + ["##" + c for c in letters] + pairs + ["##" + c for c in pairs])
+    vocabulary, reference = nv.WordPieceVocabulary(dev(nv, hv)), orc.Vocabulary(hv)
+    text = (" ".join("".join(rng.choice(list(letters), int(rng.choice(sizes)))) for _ in range(20_000)) + " ").encode()
+    total = kilobytes * 1000
+    chars = np.frombuffer(text * (total // len(text) + 1), np.uint8)[:total].copy()
+    host = HostStringsColumn(chars, np.linspace(0, total, 2001).astype(np.int32), None, 2000, 0, 0)
+    expected = orc.wordpiece_tokenize(host, reference, 0, nthreads=8)
+    for _ in range(2):
+        got, names = kernel_launches(lambda: nv.wordpiece_tokenize(dev(nv, host), vocabulary, 0))
+        assert got.to_host().equals(expected)
+        assert (names.count("wordpiece_word_kernel (small column)"), names.count("wordpiece_word_kernel")) == (small, large)
+
+
 @pytest.mark.parametrize("tiles", [1, 7, 8, 9, 511, 4095, 4096, 4097, 4105, 8200])
 def test_tokenize_blocks_of_tiles(nv, orc, tiles):
     """Columns of so many tiles of 1024 bytes: a block is eight of them, and more where 512 workgroups have more to do; the
