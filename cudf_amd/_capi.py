@@ -39,6 +39,7 @@ EXPORTS = [
     "nvtext_amd_profile_read",
     "nvtext_amd_profile_set_range_tiles",
     "nvtext_amd_profile_set_sizing_sample",
+    "nvtext_amd_profile_hold_arrivals",
 ]
 
 
@@ -246,6 +247,8 @@ def load():
     L.nvtext_amd_profile_set_range_tiles.argtypes = [C.c_int32]
     L.nvtext_amd_profile_set_sizing_sample.restype = None
     L.nvtext_amd_profile_set_sizing_sample.argtypes = [C.c_int32]
+    L.nvtext_amd_profile_hold_arrivals.restype = C.c_int32
+    L.nvtext_amd_profile_hold_arrivals.argtypes = [C.c_int32]
     _lib = L
     return L
 
@@ -262,6 +265,12 @@ def set_range_tiles(tiles: int) -> None:
 def set_sizing_sample(on: bool) -> None:
     """Test knob: whether wordpiece_tokenize sizes its first attempt from a sample of the column (the default)."""
     load().nvtext_amd_profile_set_sizing_sample(1 if on else 0)
+
+
+def hold_arrivals(count: int) -> int:
+    """Test knob: the calling thread's memory for what workgroups add up becomes unfit for use, `count` of the free pieces of such
+    memory are held back; how many are left."""
+    return load().nvtext_amd_profile_hold_arrivals(int(count))
 
 
 def profile_read(capacity: int = 4096):

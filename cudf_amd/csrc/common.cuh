@@ -599,18 +599,34 @@ __device__ __forceinline__ uint32_t search_by_lanes(uint32_t lo, uint32_t hi, ui
 
 // What the workgroups of one launch add up between them, so that the last to arrive knows the sum and need not be another
 // kernel: `sum` counts them in its upper bits.  Zeros between launches, which the last workgroup sees to.  Every host thread has
-// one of its own on every device (device memory of the library, no allocation; nullptr for more than kMostArrivals threads at a
-// time), given back when the thread ends.  For entry points that wait until the last workgroup has spoken: the thread's next call,
-// on whatever stream, then finds zeros.
+// one of its own on every device (device memory of the library, no allocation), given back when the thread ends.  For entry points
+// that wait until the last workgroup has spoken: the thread's next call, on whatever stream, then finds zeros.
 struct alignas(128) Arrivals {
   unsigned long long sum;
   uint32_t notes;
   alignas(128) uint32_t words[16];  // counters of the launch's own
 };
 constexpr int kMostArrivals = 1024;
-Arrivals* thread_arrivals();
-// After a failure it may hold anything: no thread gets it any more.
+Arrivals* thread_arrivals();  // (nullptr: as many threads as that have one)
+// After a failure it may hold anything: no thread gets it any more, and this one another at its next call.
 void forsake_thread_arrivals();
+void launch_fill_u32(uint32_t* dst, uint32_t value, int64_t count, hipStream_t stream);
+// What a call adds up in: the thread's, or, where there is none for it, memory of its own, zeroed first (a launch more).
+class CallArrivals {
+  Arrivals* const threads_;
+  Temp const own_;
+
+ public:
+  CallArrivals(Mr mr, bool wanted) : threads_(wanted ? thread_arrivals() : nullptr), own_(mr, wanted && !threads_ ? sizeof(Arrivals) : 0)
+  {
+    if (own_.ptr) launch_fill_u32(own_.as<uint32_t>(), 0u, sizeof(Arrivals) / sizeof(uint32_t), mr.stream);
+  }
+  Arrivals* get() const { return threads_ ? threads_ : own_.as<Arrivals>(); }  // (nullptr: not wanted, or no memory)
+  void failed() const
+  {
+    if (threads_) forsake_thread_arrivals();
+  }
+};
 
 // dst[0] = offsets[first_index], dst[1] = offsets[last_index] (offsets of 32 or 64 bits)
 void launch_read_two_offsets(const void* offsets, int is64, int64_t first_index, int64_t last_index, uint64_t* dst, HostPost post,
@@ -621,6 +637,5 @@ void launch_read_two_offsets(const void* offsets, int is64, int64_t first_index,
 // (cpp/src/bitmask/null_mask.cu:332-347).
 void launch_copy_bitmask(uint32_t* dst, const uint32_t* src, int32_t begin_bit, int32_t bits, hipStream_t stream);
 
-void launch_fill_u32(uint32_t* dst, uint32_t value, int64_t count, hipStream_t stream);
 
 }  // namespace nvtext_amd

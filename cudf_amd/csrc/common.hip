@@ -188,6 +188,7 @@ __device__ Arrivals g_arrivals[kMostArrivals];  // zeros when the library is loa
 struct FreeArrivals {
   std::mutex lock;
   std::vector<int> numbers;
+  std::vector<int> held;  // (see nvtext_amd_profile_hold_arrivals)
   FreeArrivals()
   {
     for (int i = kMostArrivals; i-- > 0;) numbers.push_back(i);
@@ -200,21 +201,21 @@ FreeArrivals& free_arrivals()
 }
 struct ThreadArrivals {
   static constexpr int kDevices = 64;
-  int number                    = -1;
-  bool forsaken                 = false;
+  int number                    = -1;  // (none)
   Arrivals* first[kDevices]     = {};  // of the device's array
-  ThreadArrivals()
+  bool take()
   {
+    if (number >= 0) return true;
     FreeArrivals& all = free_arrivals();
     std::lock_guard<std::mutex> const guard(all.lock);
-    if (!all.numbers.empty()) {
-      number = all.numbers.back();
-      all.numbers.pop_back();
-    }
+    if (all.numbers.empty()) return false;
+    number = all.numbers.back();
+    all.numbers.pop_back();
+    return true;
   }
   ~ThreadArrivals()
   {
-    if (number < 0 || forsaken) return;
+    if (number < 0) return;
     FreeArrivals& all = free_arrivals();
     std::lock_guard<std::mutex> const guard(all.lock);
     all.numbers.push_back(number);
@@ -231,7 +232,7 @@ Arrivals* thread_arrivals()
 {
   ThreadArrivals& mine = of_this_thread();
   int device           = 0;
-  if (mine.number < 0 || mine.forsaken || hipGetDevice(&device) != hipSuccess || device < 0 || device >= ThreadArrivals::kDevices) return nullptr;
+  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= ThreadArrivals::kDevices || !mine.take()) return nullptr;
   if (!mine.first[device]) {
     void* p = nullptr;
     if (hipGetSymbolAddress(&p, HIP_SYMBOL(g_arrivals)) != hipSuccess) {
@@ -243,7 +244,7 @@ Arrivals* thread_arrivals()
   return mine.first[device] + mine.number;
 }
 
-void forsake_thread_arrivals() { of_this_thread().forsaken = true; }
+void forsake_thread_arrivals() { of_this_thread().number = -1; }
 
 HostPost new_post()
 {
@@ -322,6 +323,20 @@ int32_t nvtext_amd_profile_read(const char** names, float* milliseconds, int32_t
   }
   nvtext_amd::g_profile.clear();
   return n;
+}
+
+int32_t nvtext_amd_profile_hold_arrivals(int32_t count)
+{
+  nvtext_amd::forsake_thread_arrivals();
+  auto& all = nvtext_amd::free_arrivals();
+  std::lock_guard<std::mutex> const guard(all.lock);
+  auto const move = [](std::vector<int>& from, std::vector<int>& to) {
+    to.push_back(from.back());
+    from.pop_back();
+  };
+  while (static_cast<int32_t>(all.held.size()) < count && !all.numbers.empty()) move(all.numbers, all.held);
+  while (static_cast<int32_t>(all.held.size()) > count && !all.held.empty()) move(all.held, all.numbers);
+  return static_cast<int32_t>(all.numbers.size());
 }
 
 const char* nvtext_amd_last_error(void) { return nvtext_amd::g_last_error.c_str(); }

@@ -1145,7 +1145,8 @@ nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* inpu
   // 100,000 278 -> 264).  In a larger one its wait and the listing before all else cost more (245,000 527 -> 554, 250,001 of
   // twice 2 KB 3500 -> 3605).
   uint64_t* const pinned = host_scalars();
-  Arrivals* const own    = rows <= kLookRows && pinned ? thread_arrivals() : nullptr;
+  CallArrivals const arrivals(mr, rows <= kLookRows && pinned);
+  Arrivals* const own    = arrivals.get();
   bool const look        = own != nullptr;
   if (!own) launch_fill_u32(lists, 0u, kListHeader, stream);
 
@@ -1185,7 +1186,7 @@ nvtext_amd_status nvtext_amd_jaccard_index(const nvtext_amd_strings_column* inpu
   hipError_t e = hipGetLastError();
   if (look) {
     if (e == hipSuccess) e = wait_for_post(told.post, stream);
-    if (e != hipSuccess) forsake_thread_arrivals();  // (nobody knows what it holds)
+    if (e != hipSuccess) arrivals.failed();  // (nobody knows what it holds)
   }
   auto const listed = [&](int list) { return look ? static_cast<int32_t>(head[list]) : rows; };
   auto const grid_of = [&](int list, int per_cu) { return dim3(static_cast<unsigned>(std::min<int64_t>(listed(list), static_cast<int64_t>(cus) * per_cu))); };

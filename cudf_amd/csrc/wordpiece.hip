@@ -2761,7 +2761,8 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
   size_t const ow = input->offsets_is_int64 ? 8 : 4;
   int64_t first_offset = 0, last_offset = 0;
   uint64_t* const scalars = host_scalars();  // pinned words that kernels write for the host (nullptr: copy instead)
-  Arrivals* const arrivals = scalars ? thread_arrivals() : nullptr;
+  CallArrivals const call_arrivals(mr, scalars != nullptr);
+  Arrivals* const arrivals = call_arrivals.get();
   bool const sampling      = arrivals && g_sizing_sample.load(std::memory_order_relaxed) != 0;
   double sample_words = 0, sample_queued = 0, sample_bytes = 0;  // what the sample found (nothing without the pinned words)
   bool const is64  = input->offsets_is_int64 != 0;
@@ -2819,7 +2820,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     bool const launched = e == hipSuccess;
     if (launched) e = wait_for_post(args.post, stream);
     if (e != hipSuccess) {
-      if (launched) forsake_thread_arrivals();  // (nobody knows what it holds)
+      if (launched) call_arrivals.failed();  // (nobody knows what it holds)
       return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
     }
     first_offset = static_cast<int64_t>(scalars[0]);
@@ -2865,7 +2866,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     bool const launched = e == hipSuccess;
     if (launched) e = wait_for_post(post, stream);
     if (e != hipSuccess) {
-      if (launched && sampling) forsake_thread_arrivals();
+      if (launched && sampling) call_arrivals.failed();
       return give_up(NVTEXT_AMD_DEVICE_ERROR, hipGetErrorString(e));
     }
     first_offset = static_cast<int64_t>(scalars[0]);

@@ -34,6 +34,12 @@ void    nvtext_amd_profile_set_range_tiles(int32_t tiles);
  * any other value switches it back on (the default).  Results do not depend on it. */
 void    nvtext_amd_profile_set_sizing_sample(int32_t on);
 
+/* Test knob.  What the workgroups of one launch add up between them lies in memory of the calling host thread, of which the
+ * library has 1,024 pieces: a call on a thread beyond those, or after a failed call has made a piece unfit for use, goes another
+ * way to the same result.  This call makes the calling thread's piece unfit, as a failed call does, and takes `count` of the
+ * pieces that no thread has out of use (0: none; those taken before are given back); it returns how many are left. */
+int32_t nvtext_amd_profile_hold_arrivals(int32_t count);
+
 #ifdef __cplusplus
 }
 #endif

@@ -622,6 +622,48 @@ def test_tokenize_from_threads_that_come_and_go(nv, orc):
     assert not wrong
 
 
+@pytest.fixture(params=["own", "another", "none"])
+def arrivals(request):
+    """Calls of a thread that has memory for what workgroups add up, of one whose memory a failed call has made unfit, and of one
+    beyond the 1,024 that the library has some for."""
+    from cudf_amd import _capi
+    if request.param != "own":
+        left = _capi.hold_arrivals(0)
+        assert (_capi.hold_arrivals(1 << 20) == 0) if request.param == "none" else left > 900
+    yield request.param
+    _capi.hold_arrivals(0)
+
+
+def test_a_thread_without_memory_of_its_own(nv, orc, arrivals):
+    """A small tokenizer column, one that is sampled and done in two parts, and jaccard_index of pairs that are listed go the
+    same way in all three."""
+    from cudf_amd import _capi
+    rng = np.random.default_rng(11)
+    hv = HostStringsColumn.from_pylist(VOCABULARY)
+    vocabulary, reference = nv.WordPieceVocabulary(dev(nv, hv)), orc.Vocabulary(hv)
+    small = words_column(rng, list(rng.integers(0, 90, 3000)), VOCABULARY, 0.2)
+    piece = words_column(rng, [100_000], VOCABULARY, 0.2).chars
+    total = 130 << 20
+    large = HostStringsColumn(np.tile(piece, total // piece.size + 1)[:total].copy(), np.linspace(0, total, 300_001).astype(np.int32), None, 300_000, 0, 0)
+    for host, kernel, launches in ((small, "wordpiece_word_kernel (small column)", 1), (large, "wordpiece_word_kernel", 2)):
+        column, expected = dev(nv, host), orc.wordpiece_tokenize(host, reference, 0, nthreads=8)
+        for _ in range(2):
+            got, names = kernel_launches(lambda: nv.wordpiece_tokenize(column, vocabulary, 0))
+            assert got.to_host().equals(expected)
+            assert [n for n in names if n.startswith("wordpiece_word_kernel")] == [kernel] * launches
+    rows = [random_text(rng, n).decode() for n in (10, 700, 2500, 5000, 9000, 15_000, 61_000)] * 9
+    h1, h2 = (HostStringsColumn.from_pylist(side) for side in ([t[: len(t) // 3] for t in rows], [t[len(t) // 4:] for t in rows]))
+    expected = orc.jaccard_index(h1, h2, 4, nthreads=8).values.view(np.uint32)
+    for _ in range(2):
+        got, names = kernel_launches(lambda: nv.jaccard_index(dev(nv, h1), dev(nv, h2), 4))
+        assert np.array_equal(got.to_host().values.view(np.uint32), expected)
+        assert names == ["jaccard_wave_kernel", "jaccard_teams_kernel"]
+    if arrivals == "another":
+        left = _capi.hold_arrivals(0)
+        nv.wordpiece_tokenize(dev(nv, small), vocabulary, 0)
+        assert _capi.hold_arrivals(0) == left - 1
+
+
 @pytest.mark.parametrize("rows, each", [(4, 65_537), (4, 65_535), (131_072, 10), (131_073, 10), (9000, 3800)])
 def test_tokenize_where_small_columns_end(nv, orc, rows, each):
     """Around the bytes (256 KiB; 32 MiB) and the rows up to which a column is put on the stream before its size is known."""
