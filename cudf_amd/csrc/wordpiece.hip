@@ -899,9 +899,12 @@ __device__ __forceinline__ uint32_t next_unit(uint32_t* counters, bool first, ui
 }
 
 // The queue is handed out in chunks of 2^shift entries by kCounterGroups counters, each in a line of its own: chunk n of group
-// g is the queue's chunk n * kCounterGroups + g.  A wavefront's group is that of the ranges it does, so that how many chunks
-// a group takes depends on the text, but for the last chunk of each wavefront.  (One counter, one atomic after the other at
-// 150 M/s, was a third of the word pass of 16 MB of text in chunks of 512, and most of it in chunks of 64.)
+// g is the queue's chunk n * kCounterGroups + g.  A wavefront asks the groups in turn, so that they hand out about as many
+// chunks each wherever the unknown words are: the queue has to reach to the end of the last chunk.  (With one group for all that a
+// wavefront asks for, that of its ranges, 64 MB with unknown words in every eighth range took eight times the queue that they fill, 0.99 GB
+// of memory in all, and a second attempt for it; both ways take the same time, 2 million rows of 256 bytes 1056 and 1054 us.  One
+// counter, one atomic after the other at 150 M/s, was a third of the word pass of 16 MB of text in chunks of 512, and most of it in
+// chunks of 64.)
 struct QueueChunks {
   const uint32_t* counts;
   uint32_t shift;
@@ -1534,7 +1537,8 @@ __global__ void __launch_bounds__(word_waves(INLINE) * kWave, INLINE ? 4 : 6) wo
               spill = true;
             } else {
               // (a chunk has an entry for every lane)
-              uint32_t const group = my_number % kCounterGroups;
+              // (the group after that of the chunk before)
+              uint32_t const group = (q_lim != 0 ? q_lim >> a.queue_shift : my_number) % kCounterGroups;
               if (lane == 0) fresh = atomicAdd(a.queue_chunks + group * kFlagLine, 1u);
               fresh = (wave_bcast(fresh, 0) * kCounterGroups + group) << a.queue_shift;
             }

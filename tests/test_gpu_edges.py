@@ -543,6 +543,37 @@ def test_tokenize_chunks_of_the_queue(nv, orc, rows, oov):
     assert nv.wordpiece_tokenize(dev(nv, host), vocabulary, 0).to_host().equals(orc.wordpiece_tokenize(host, reference, 0, nthreads=8))
 
 
+@pytest.mark.parametrize("every", [1, 8, 64])
+@pytest.mark.parametrize("megabytes", [64, 144])
+def test_tokenize_unknown_words_in_some_ranges(nv, orc, every, megabytes):
+    """Ranges of 2048 bytes of unknown words, every one, every eighth and every sixty-fourth, the others of known ones, in columns that
+    are done in one part and in two: the queue is handed out evenly, and not much longer than what they fill of it."""
+    import torch
+    from cudf_amd import _capi
+    hv = HostStringsColumn.from_pylist(VOCABULARY)
+    vocabulary, reference = nv.WordPieceVocabulary(dev(nv, hv)), orc.Vocabulary(hv)
+    tile = lambda text: np.frombuffer((text * (2048 // len(text) + 1)).encode(), np.uint8)[:2047].tolist() + [0x20]
+    rng = np.random.default_rng(every)
+    known, unknown = tile("hello world data frame "), [tile("".join("".join(rng.choice(LETTERS[:6], 2)) + " " for _ in range(683))) for _ in range(8)]
+    block = [unknown[i // every % 8] if i % every == min(3, every - 1) else known for i in range(512)]
+    chars = np.tile(np.array(block, np.uint8).reshape(-1), megabytes)
+    host = HostStringsColumn(chars, np.linspace(0, chars.size, 150_001).astype(np.int32), None, 150_000, 0, 0)
+    column, expected = dev(nv, host), orc.wordpiece_tokenize(host, reference, 0, nthreads=8)
+    _capi.set_range_tiles(1)
+    try:
+        nv.wordpiece_tokenize(column, vocabulary, 0)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        held = torch.cuda.memory_allocated()
+        got = nv.wordpiece_tokenize(column, vocabulary, 0)
+        # (2.5 bytes of temporaries for a byte and a chunk for a wavefront; what the queue takes of every unknown word; the result)
+        words = chars.size // every // 3
+        assert torch.cuda.max_memory_allocated() - held < 3 * chars.size + (300 << 20) + 48 * words + 4 * expected.child.size
+        assert got.to_host().equals(expected)
+    finally:
+        _capi.set_range_tiles(0)
+
+
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("shape", ["first", "last", "middle", "empty between", "even", "short"])
 def test_tokenize_rows_of_ranges(nv, orc, shape, wide):
