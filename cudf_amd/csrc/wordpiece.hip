@@ -2994,6 +2994,7 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     queue_capacity = std::max<uint64_t>(queue_capacity, static_cast<uint64_t>(per_byte_queued * 1.25 * static_cast<double>(last_offset - first_offset)) +
                                                           word_pass_waves * queue_chunk + 4096);
   }
+  constexpr int kMostAttempts = 4;  // (two wherever it has been seen)
   uint64_t total = 0;
   for (int attempt = 0;; ++attempt) {
     if (queue_capacity > 0x7FFFFFF0ull - kMemoResults) queue_capacity = 0x7FFFFFF0ull - kMemoResults;
@@ -3095,11 +3096,12 @@ nvtext_amd_status nvtext_amd_wordpiece_tokenize(const nvtext_amd_strings_column*
     }
     bool const words_over = state[1] != 0, queue_over = state[2] > qcap;
     if (words_over || queue_over) {
-      if (attempt > 0 || state[2] > 0x7FFFFFF0u) return give_up(NVTEXT_AMD_LOGIC_ERROR, "words exceed internal limit");
+      if (attempt + 1 == kMostAttempts || state[2] > 0x7FFFFFF0u) return give_up(NVTEXT_AMD_LOGIC_ERROR, "words exceed internal limit");
       if (words_over) range_cap = static_cast<uint32_t>(kRange + 8);
-      // state[2] counts what the wavefronts reserved, the unused rest of each wavefront's last chunk included; which
-      // ranges of its group a wavefront gets differs from one attempt to the next, and with it that rest: a chunk per
-      // wavefront on top of what this attempt reserved covers every assignment.
+      // state[2] tells how far what the wavefronts reserved reaches, the unused rest of each wavefront's last chunk included.
+      // Which ranges a wavefront gets and which words the memo has differ from one attempt to the next, and with them that rest and
+      // how evenly the groups are asked.  A chunk per wavefront on top covers the rests; all of it together has no bound that is worth
+      // its memory, so that an attempt which needs still more is followed by one that has it.
       queue_capacity = std::max<uint64_t>(queue_capacity, state[2] + word_pass_waves * queue_chunk);
       continue;
     }
