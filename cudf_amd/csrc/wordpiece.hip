@@ -677,8 +677,7 @@ struct WindowWord : ShortWord {
       longer = next_longer(min(rem, t.max_len[kind]));
     }
   }
-  // probed: the whole word has been looked up and is known to be absent (up to 16 bytes)
-  __device__ __forceinline__ void begin(VocabTable const& t, const uint4* trim, const int32_t* first_ids, TileWord const& word, uint32_t len, bool probed)
+  __device__ __forceinline__ void begin(VocabTable const& t, const uint4* trim, const int32_t* first_ids, TileWord const& word, uint32_t len)
   {
     w     = word;
     rem   = len;
@@ -686,7 +685,6 @@ struct WindowWord : ShortWord {
     done  = false;
     fill(trim);
     open(t, first_ids, 0);
-    if (probed) cand &= ~(1u << (len - 1));
   }
   template <typename Emit>
   __device__ __forceinline__ void step(VocabTable const& t, const uint4* trim, const int32_t* first_ids, Emit&& emit)
@@ -722,7 +720,7 @@ __device__ __forceinline__ uint32_t tokenize_window_word(VocabTable const& t, co
 {
   const int32_t* const first_ids = t.short_ids + 2 * 65536;
   WindowWord word;
-  word.begin(t, trim, first_ids, w, len, false);
+  word.begin(t, trim, first_ids, w, len);
   while (!word.done) word.step(t, trim, first_ids, emit);
   return word.count;
 }
