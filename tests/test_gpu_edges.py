@@ -86,8 +86,7 @@ def furthest_from_home(text, buckets, parts):
 def test_jaccard_values_of_neighbouring_buckets(nv, orc, count, slots, parts):
     """Words that belong in one bucket of their set, or in a few side by side, and take the same steps from there: 90 that find a
     place within the 64 buckets that a packed set looks at, and so many in sets of every size that some do not, so that the pair
-    is done once more with a plain set, or, where one of its parts has them all, with the one in global memory; among pairs that
-    are not."""
+    is done once more with a plain set, or, where one of its parts has them all, that part is cut in two; among pairs that are not."""
     rng = np.random.default_rng(count)
     assert jaccard_set(4 * count) == (slots, parts)
     letters = np.concatenate([np.arange(65, 91), np.arange(97, 123)]).astype(np.uint32)

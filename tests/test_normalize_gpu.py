@@ -281,8 +281,8 @@ def test_normalize_feeds_the_tokenizer(nv, onorm):
 @pytest.mark.parametrize("kind", ["plain", "tokens", "bytes", "wide"])
 @pytest.mark.parametrize("skip,extra", [(0, 0), (1, 1), (2, 2047), (3, 12345)])
 def test_normalize_wavefront_a_tile(nv, onorm, kind, skip, extra):
-    """Columns so large that a wavefront counts whole tiles, and just below that: the tiles' number is no multiple of the
-    workgroups', characters and special tokens lie across every border, the first byte has any alignment.  "wide":
+    """Columns so large that a wavefront does whole tiles (20 MiB and more: it counts them too), and just below that: the tiles' number
+    is no multiple of the workgroups', characters and special tokens lie across every border, the first byte has any alignment.  "wide":
     characters that turn into nine and twelve bytes, alone, side by side and in every place, few over-long brackets among them."""
     rng = np.random.default_rng(7 + skip)
     pieces = [b"word", b" ", b" a", b"Th", b"\xc3\xa9t\xc3\xa9", "漢字".encode(), "Жи".encode(), b".", b"),", b"\t", "\U0001F600".encode()]
@@ -299,7 +299,7 @@ def test_normalize_wavefront_a_tile(nv, onorm, kind, skip, extra):
     if kind == "tokens":
         which = np.where(rng.random(which.size) < 0.97, rng.integers(0, 11, which.size), which)
     part = np.frombuffer(b"".join(pieces[i] for i in which), np.uint8)
-    for tiles in (12288, 12287) if skip == 0 else (12288 + 64 * skip + 3,):
+    for tiles in (8192, 8191) if skip == 0 else (8192 + 64 * skip + 3,):
         n = tiles * TILE - (TILE - 1) + extra
         rows = 2500
         chars = np.resize(part, n + 40)
@@ -327,10 +327,10 @@ def test_normalize_rows_of_a_wavefronts_tile(nv, onorm, per_tile):
     assert_same(run(nv, host, True, ("[SEP]",)), onorm.normalize_characters_native(host, True, [b"[SEP]"], 8), f"{per_tile} rows")
 
 
-@pytest.mark.parametrize("rows, tiles", [(131_072, 12288), (131_072, 12287), (40_000, 16384)])
+@pytest.mark.parametrize("rows, tiles", [(131_072, 10_240), (131_072, 8192), (131_072, 8191), (40_000, 9001)])
 def test_normalize_wavefront_a_tile_after_one_wait(nv, onorm, rows, tiles):
-    """Columns of few enough rows to be worked on before their size is known, but of more than the 20 MiB up to which they are;
-    a wavefront does each of their tiles."""
+    """Columns of few enough rows and bytes (131,072; 20 MiB) to be counted before their size is known, whose tiles a wavefront
+    writes alone (from 8,192 on), and one of a tile less."""
     rng = np.random.default_rng(rows + tiles)
     chars = np.resize(np.frombuffer("Some [SEP] words, Été 漢字 Жи 각 and more plain words of text. ".encode(), np.uint8), tiles * TILE)
     offsets = np.concatenate([[0], np.sort(rng.integers(0, tiles * TILE, rows - 1)), [tiles * TILE]]).astype(np.int32)
@@ -340,10 +340,12 @@ def test_normalize_wavefront_a_tile_after_one_wait(nv, onorm, rows, tiles):
 
 
 @pytest.mark.parametrize("kind", ["plain", "tokens"])
-@pytest.mark.parametrize("rows, tiles", [(40_000, 8191), (40_000, 8192), (40_000, 10_240), (40_000, 10_241), (140_000, 8191), (140_000, 8193), (300, 2048 * 20 + 1)])
+@pytest.mark.parametrize("rows, tiles", [(40_000, 8191), (40_000, 8192), (40_000, 10_240), (40_000, 10_241), (140_000, 8191), (140_000, 8193), (300, 2048 * 20 + 1),
+                                         (140_000, 100_000), (140_000, 100_001)])
 def test_normalize_lines_between_the_ways(nv, onorm, kind, rows, tiles):
     """Either side of the 8,192 tiles from which a wavefront does a tile alone, of the 20 MiB up to which a column of few rows is
-    counted before its size is known, and of scans of one, a few and many tiles of 2048 sums."""
+    counted before its size is known, of the 8,192 sums up to which a scan is one launch and not two (three: see test_scan_gpu.py), and of
+    the 100,000 tiles up to which eight lanes search for a tile's first row."""
     rng = np.random.default_rng(tiles)
     text = "Some [SEP] words, Été 漢字 Жи 각 and more plain words of text. "
     chars = np.resize(np.frombuffer((text if kind == "tokens" else text.replace("[SEP]", "sep")).encode(), np.uint8), tiles * TILE - 5)
