@@ -909,11 +909,12 @@ __global__ void __launch_bounds__(kTierWaves[kPartsTier] * kWave) jaccard_parts_
 // tier each waits for its slowest pair before the next begins.  A workgroup of sixteen wavefronts and the largest set takes
 // pieces of work until none is left: a part of a pair, a pair of the last two tiers, two pairs of tier 2 or four of tier 1,
 // each by a team of its wavefronts with its share of the set; the longest first.  The teams share the barriers.  Pairs of twice 1500
-// bytes, 166 of them 76 -> 33 us, 466 77 -> 33, 2,000 131 -> 80; of twice 6000, 1,666 330 -> 214, 3,333 418 -> 291, 16,666
-// 1526 -> 1120; 7,500 of twice 200 58 -> 51.  What bounds it is one piece: its bytes are hashed by one CU.
-// With more than kTeamPieces pieces of the first three tiers these have their own kernels, more of whose wavefronts fit a CU
-// (13,333 pairs of twice 1500 bytes in a launch 244 us, with their own kernels 230; 32,666 495 and 421; but 1,666 of twice 6000, 1,400
-// pieces, 213 and 267).
+// bytes on average, lengths lognormal (0.8), with the first three tiers' own kernels and in this launch: 166 of them 59 and 27 us, 466 60 and 28,
+// 2,000 72 and 48; of twice 6000, 1,666 200 and 156; 7,500 of twice 200 41 and 35.  What bounds it is one piece: its bytes are hashed
+// by one CU.
+// With more than kTeamPieces pieces of the first three tiers these have their own kernels, more of whose wavefronts fit a CU (13,333
+// pairs of twice 1500 bytes 176 us with their own kernels and 205 in this launch, 32,666 341 and 469, 16,666 of twice 6000 868 and 945; between
+// them it depends on the lengths: 3,333 of twice 6000 219 and 188).
 struct Pieces {
   uint32_t parts, tier4, tier3, tier2, tier1;  // where the pieces of each kind end
   uint32_t pairs2, pairs1;                     // of the last two kinds

@@ -2249,7 +2249,6 @@ __global__ void __launch_bounds__(kWave) wordpiece_sample_kernel(ColView col, Vo
     int64_t const begin  = first + sample_begin(span, blockIdx.x);
     uint32_t const bytes = static_cast<uint32_t>(min(last, begin + kSampleBytes) - begin);
     uint8_t* const sb   = reinterpret_cast<uint8_t*>(staged);
-#pragma unroll
     for (int i = lane; i < 4 + kSampleBytes + kSampleTail + 8; i += kWave) {
       int64_t const g = begin + i - 4;
       sb[i]           = (g >= first && g < last) ? col.chars[g] : uint8_t{0x20};  // outside the view: a space
