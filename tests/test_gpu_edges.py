@@ -191,6 +191,29 @@ def test_jaccard_more_parts_than_their_list_beside_other_pairs(nv, orc, filled_m
     assert np.array_equal(got.values.view(np.uint32), exp[order])
 
 
+@pytest.mark.parametrize("times", [{9000: 1536}, {9000: 1537}, {2500: 4 * 1536}, {2500: 4 * 1536 + 1}, {23_600: 32_768, 15_000: 300, 2500: 10},
+                                   {20: 131_000, 2500: 30, 9000: 20, 15_000: 12, 61_000: 9, 640_001: 1}, {20: 131_000, 2500: 30, 9000: 21, 15_000: 12, 61_000: 9, 640_001: 1}])
+@pytest.mark.parametrize("nulls", [False, True])
+def test_jaccard_where_the_ways_part(nv, orc, filled_memory, times, nulls):
+    """Pieces of work up to which the sets share a launch (1,536) and one more, parts of which the last has the last place on their
+    list (65,536), pairs up to which the host looks at the lists (131,072) and one more; null rows in one column or the other, and a view."""
+    rng = np.random.default_rng(sum(times.values()))
+    rows = [random_text(rng, n).decode() for n in times]
+    left, right = [t[: len(t) // 3] for t in rows], [t[len(t) // 4:] for t in rows]
+    if 23_600 in times:
+        left[0], right[0] = rows[0][:11_800], rows[0][11_800:]
+    exp = orc.jaccard_index(*(HostStringsColumn.from_pylist(side) for side in (left, right)), 4, nthreads=8).values.view(np.uint32)
+    order = rng.permutation(np.repeat(np.arange(len(rows)), list(times.values())))
+    valid = np.ones((2, len(order)), bool)
+    if nulls:
+        valid[0, 3::7] = valid[1, 5::11] = False
+    h1, h2 = (HostStringsColumn.from_pylist(["skip", "these"] + [side[i] if v else None for i, v in zip(order, ok)]) for side, ok in zip((left, right), valid))
+    n, both = len(order), valid[0] & valid[1]
+    got = nv.jaccard_index(*(dev(nv, h).slice(2, n + 2, int((~ok).sum())) for h, ok in zip((h1, h2), valid)), 4).to_host()
+    assert got.null_count == int((~both).sum())
+    assert np.array_equal(got.values.view(np.uint32)[both], exp[order][both])
+
+
 def mixed_rows(rng, lens, nulls=()):
     """Rows of these lengths as a column; the rows named in `nulls` are null (and empty)."""
     lens = np.array(lens, np.int64)
