@@ -251,7 +251,7 @@ struct MinimaAll {
   Packing pk, tail_pk;
   int lane;
 
-  static constexpr int kLeast = 0;
+  static constexpr bool kCutUp = false;  // whether a chunk may have fewer parameters than it has room for (see minhash_parts_kernel)
   __device__ __forceinline__ MinimaAll(Lds*, int lane_, int32_t) : lane(lane_) {}
   __device__ __forceinline__ int32_t stride() const { return kParams; }
   __device__ __forceinline__ int32_t slots() const { return kSlots; }
@@ -340,9 +340,11 @@ struct Minima64 {
   uint32_t warm;   // (see load)
   Lds* lds;
   int lane;
-  static constexpr int kLeast = GROUPS < 2 ? GROUPS : 2;  // groups that a chunk has at least
+  static constexpr int kLeast  = GROUPS < 2 ? GROUPS : 2;  // groups that a chunk has at least
+  static constexpr bool kCutUp = GROUPS > kLeast;
 
-  __device__ __forceinline__ Minima64(Lds* lds_, int lane_, int32_t groups_) : groups(groups_ != 0 ? groups_ : GROUPS), warm(0), lds(lds_), lane(lane_) {}
+  // (with one group or two their number is known when this is compiled: 400,000 rows of several scripts, 64 parameters 2022 -> 2006 us)
+  __device__ __forceinline__ Minima64(Lds* lds_, int lane_, int32_t groups_) : groups(kCutUp && groups_ != 0 ? groups_ : GROUPS), warm(0), lds(lds_), lane(lane_) {}
   __device__ __forceinline__ int32_t stride() const { return slots(); }  // parameters from a chunk to the next
   __device__ __forceinline__ int32_t slots() const { return groups * filter64::kGroup; }
   // What the first groups have in memory is asked for here, a cache line a lane, and waited for where it is used: the plan has
@@ -513,7 +515,7 @@ struct Minima64 {
     uint32_t const rest = (0u - count) & 31u;
     if (static_cast<uint32_t>(lane) < rest) hashes[count + lane] = hashes[0];
     wave_lds_fence();
-    if (GROUPS > kLeast && AT_ONCE != kLeast && groups == kLeast) {
+    if (kCutUp && AT_ONCE != kLeast && groups == kLeast) {
       fold_groups<kLeast>(0, hashes, count + rest);
     } else {
 #pragma unroll 1
@@ -921,7 +923,7 @@ __global__ void __launch_bounds__(kThreads, (simd_waves<Source, Minima>())) minh
   // 32 -> 27; 700 of 300, 256 parameters 31 -> 27;
   // with twice or four times as many units as wavefronts it is no gain: 50 rows of 16 KB 33.2 us whole, 36.4 in chunks of two groups
   int32_t in_chunk_groups = 0;  // 0: as many as the minima are made for
-  if constexpr (Minima::kLeast != 0) {
+  if constexpr (Minima::kCutUp) {
     if (units <= static_cast<uint32_t>(parts.waves)) {
       uint32_t const waves = static_cast<uint32_t>(parts.waves), whole = static_cast<uint32_t>(chunks);
       uint32_t const groups = static_cast<uint32_t>(params.count + filter64::kGroup - 1) / filter64::kGroup, twos = (groups + 1) / 2, fours = (groups + 3) / 4;
